@@ -1,0 +1,861 @@
+"""What is timed: serving steps of the engine, driven as its own step loop
+drives them (LLMEngine.add_request / add_prefilled, Scheduler.schedule,
+ModelRunner.forward_logits and sample), with the logits of every step.
+
+A case is one of
+
+- "decode":  every request of a batch makes its next token over the context
+  that it holds (as on the decode instance of a disaggregated pair, whose
+  requests arrive with their pages). The requests are not advanced, so a pass
+  can be repeated.
+- "prefill": fresh prompts run to their first token.
+- "mixed":   a long prompt comes in chunk by chunk while a batch decodes.
+- "serve":   prompts run to their first token and then generate together
+  until every request is finished (models whose per-sequence state moves on
+  with every token).
+
+Models are the shapes of arks_amd.config.PRESET_CONFIGS cut to a few layers,
+each layer and the vocabulary at full size, with random weights whose greedy
+token is as clear as a trained model's (the output rows are the embedding
+rows of another token). Weights, prompts and cached pages come from the seed;
+lengths come from the case.
+"""
+
+from __future__ import annotations
+
+import contextlib
+import dataclasses
+import math
+import random
+import zlib
+
+import torch
+
+from arks_amd.config import EngineConfig, PRESET_CONFIGS
+from arks_amd.engine import LLMEngine, SamplingParams, SeqStatus
+
+PAGE = 16
+F64 = torch.float64
+
+# model of a case -> (preset, layers kept). "dense-fp8" is the dense model
+# with both low-precision options on (quantization, kv_cache_dtype).
+MODELS = {
+    "dense": ("qwen2.5-7b", 8),
+    "dense-fp8": ("qwen2.5-7b", 8),
+    "moe": ("qwen3-30b-a3b", 4),
+    "gagorax": ("gagorax-8b-slice", 8),
+    "pazilorn": ("pazilorn-8b-slice", 3),
+}
+
+
+# ------------------------------------------------------------------- cases
+def listed():
+    return [
+        # one user's stream: nothing but the latency of a step
+        dict(name="dense-decode-1", model="dense", kind="decode", batch=1,
+             low=700, high=700),
+        # the throughput benchmark of bench.py: 64 requests of 1024 tokens
+        dict(name="dense-decode-64", model="dense", kind="decode", batch=64,
+             low=1024, high=1024),
+        # a full server: many requests at every stage of their context
+        dict(name="dense-decode-200-ragged", model="dense", kind="decode",
+             batch=200, low=20, high=4000),
+        # both low-precision options, long contexts
+        dict(name="dense-decode-fp8", model="dense-fp8", kind="decode",
+             batch=48, low=900, high=5000),
+        # one long document
+        dict(name="dense-prefill-8192", model="dense", kind="prefill", batch=1,
+             low=8192, high=8192),
+        # a burst of chat prompts
+        dict(name="dense-prefill-ragged", model="dense", kind="prefill",
+             batch=24, low=20, high=400),
+        # a long prompt beside running requests, chunked
+        dict(name="dense-mixed", model="dense", kind="mixed", batch=31,
+             low=60, high=3000, prompt=6113, budget=2048),
+        # sparse experts: few and many requests, and prompts
+        dict(name="moe-decode-7", model="moe", kind="decode", batch=7, low=100,
+             high=2500),
+        dict(name="moe-decode-64", model="moe", kind="decode", batch=64,
+             low=1024, high=1024),
+        dict(name="moe-prefill-ragged", model="moe", kind="prefill", batch=6,
+             low=150, high=2500),
+        # layer-list models with per-sequence state: prompts and generation
+        dict(name="gagorax-serve", model="gagorax", kind="serve", batch=8,
+             low=200, high=1200, tokens=9),
+        dict(name="pazilorn-serve", model="pazilorn", kind="serve", batch=5,
+             low=150, high=1500, tokens=9),
+    ]
+
+
+def _spread(rng, low, high):
+    """A whole number between low and high, even over the logarithm."""
+    return int(round(math.exp(rng.uniform(math.log(low), math.log(high)))))
+
+
+def draw(rng):
+    """One more case: any model, any kind that it has, sizes over the ranges
+    of the listed cases."""
+    model = rng.choice(["dense", "dense", "dense-fp8", "moe", "moe", "gagorax",
+                        "pazilorn"])
+    if model in ("gagorax", "pazilorn"):
+        batch = _spread(rng, 1, 12)
+        high = min(_spread(rng, 30, 4000), 6000 // batch)
+        return dict(model=model, kind="serve", batch=batch,
+                    low=max(10, high // rng.randint(1, 8)), high=high,
+                    tokens=rng.randint(2, 7))
+    kind = rng.choice(["decode", "decode", "prefill", "mixed"])
+    if kind == "decode":
+        batch = _spread(rng, 1, 200)
+        high = min(_spread(rng, 40, 8000), 200000 // batch)
+        return dict(model=model, kind=kind, batch=batch,
+                    low=max(20, high // rng.randint(1, 40)), high=high)
+    if kind == "prefill":
+        batch = _spread(rng, 1, 24)
+        high = min(_spread(rng, 20, 8192), 8192 // batch)
+        return dict(model=model, kind=kind, batch=batch,
+                    low=max(10, high // rng.randint(1, 10)), high=high)
+    prompt = _spread(rng, 600, 6113)
+    budget = rng.choice([512, 1024, 2048, 4096])
+    return dict(model=model, kind=kind, batch=_spread(rng, 1, 60), low=40,
+                high=_spread(rng, 100, 3000), prompt=min(prompt, 3 * budget),
+                budget=budget)
+
+
+def _lengths(case):
+    """Tokens that every request of the case holds or brings."""
+    rng = random.Random(f"{case['batch']} {case['low']} {case['high']}")
+    return [_spread(rng, case["low"], case["high"])
+            for _ in range(case["batch"])]
+
+
+def _config(case):
+    preset, layers = MODELS[case["model"]]
+    cfg = PRESET_CONFIGS[preset]
+    if case["model"] in ("gagorax", "pazilorn"):
+        cfg = dataclasses.replace(cfg, layers=cfg.layers[:layers])
+        if case["model"] == "pazilorn":  # the table also gives the logits
+            cfg = dataclasses.replace(cfg, embed_scale=32.0)
+        return cfg
+    return dataclasses.replace(cfg, num_hidden_layers=layers)
+
+
+# ----------------------------------------------------------------- weights
+def _normal(seed, name, shape, std, dtype=torch.bfloat16, mean=0.0):
+    g = torch.Generator(device="cuda")
+    g.manual_seed((seed * 1000003 + zlib.crc32(name.encode())) % (2 ** 62))
+    return torch.randn(shape, generator=g, device="cuda").mul_(std).add_(
+        mean).to(dtype)
+
+
+def _llama_weights(cfg, seed):
+    """(name, tensor) of a llama-family model, in groups that load at once."""
+    W, I, D = cfg.hidden_size, cfg.intermediate_size, cfg.head_dim
+    nq, nkv = cfg.num_attention_heads * D, cfg.num_key_value_heads * D
+
+    def n(name, *shape, std=None, mean=0.0):
+        return _normal(seed, name, shape, shape[-1] ** -0.5 if std is None
+                       else std, mean=mean)
+
+    embed = n("embed", cfg.vocab_size, W, std=1.0)
+    yield {"model.embed_tokens.weight": embed,
+           "lm_head.weight": embed.roll(1, 0) * (2.0 * W ** -0.5),
+           "model.norm.weight": n("norm", W, std=0.1, mean=1.0)}
+    del embed
+    for i in range(cfg.num_hidden_layers):
+        p = f"model.layers.{i}."
+        a = p + "self_attn."
+        t = {p + "input_layernorm.weight": n(p + "n1", W, std=0.1, mean=1.0),
+             p + "post_attention_layernorm.weight":
+                 n(p + "n2", W, std=0.1, mean=1.0),
+             a + "q_proj.weight": n(a + "q", nq, W),
+             a + "k_proj.weight": n(a + "k", nkv, W, std=2.0 * W ** -0.5),
+             a + "v_proj.weight": n(a + "v", nkv, W),
+             a + "o_proj.weight": n(a + "o", W, nq)}
+        if cfg.attention_bias:
+            t.update({a + "q_proj.bias": n(a + "qb", nq, std=0.3),
+                      a + "k_proj.bias": n(a + "kb", nkv, std=0.3),
+                      a + "v_proj.bias": n(a + "vb", nkv, std=0.3)})
+        if cfg.qk_norm:
+            t.update({a + "q_norm.weight": n(a + "qn", D, std=0.1, mean=1.5),
+                      a + "k_norm.weight": n(a + "kn", D, std=0.1, mean=1.5)})
+        E = cfg.num_local_experts
+        if E:
+            F = cfg.moe_intermediate_size
+            t[p + "mlp.gate.weight"] = n(p + "gate", E, W, std=4.0 * W ** -0.5)
+            for part, shape in (("gate_proj", (E, F, W)), ("up_proj", (E, F, W)),
+                                ("down_proj", (E, W, F))):
+                full = n(p + part, *shape, std=(
+                    0.5 if part == "down_proj" else 1.0) * shape[-1] ** -0.5)
+                for e in range(E):
+                    t[p + f"mlp.experts.{e}.{part}.weight"] = full[e]
+        else:
+            t.update({p + "mlp.gate_proj.weight": n(p + "gate", I, W),
+                      p + "mlp.up_proj.weight": n(p + "up", I, W),
+                      p + "mlp.down_proj.weight": n(p + "down", W, I)})
+        yield t
+
+
+def _gagorax_weights(cfg, seed):
+    W = cfg.hidden_size
+
+    def n(name, *shape, std=None, mean=0.0):
+        return _normal(seed, name, shape, shape[-1] ** -0.5 if std is None
+                       else std, mean=mean)
+
+    embed = n("embed", cfg.vocab_size, W, std=1.0)
+    yield {"embed": embed, "head": embed.roll(1, 0) * (2.0 * W ** -0.5),
+           "final.norm": n("final", W, std=0.1, mean=1.0)}
+    for i, spec in enumerate(cfg.layers):
+        p, m = f"l{i}.", spec["mixer"]
+        x = p + "mix."
+        t = {p + "norm1": n(p + "norm1", W, std=0.1, mean=0.4),
+             p + "shift": n(p + "shift", W, std=0.2, mean=0.5),
+             p + "rg1": n(p + "rg1", W, W),
+             p + "rg1.b": n(p + "rg1.b", W, std=0.3)}
+        if spec["type"] == "attention":
+            H, G, D, V = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
+            shapes = {"q": (H * D, W), "k": (G * D, W), "v": (G * V, W),
+                      "o": (W, H * V)}
+            t.update({x + "q.norm": n(x + "qn", D, std=0.1, mean=1.5),
+                      x + "k.norm": n(x + "kn", D, std=0.1, mean=1.5)})
+        elif spec["type"] == "lightning":
+            H, D, V = m["heads"], m["dim"], m["vdim"]
+            shapes = {"q": (H * D, W), "k": (H * D, W), "v": (H * V, W),
+                      "g": (H * V, W), "o": (W, H * V)}
+            t[x + "norm"] = n(x + "norm", H * V, std=0.1, mean=1.0)
+        else:
+            C, N, R, K = m["inner"], m["state"], m["dt_rank"], m["conv"]
+            shapes = {"in": (2 * C, W), "conv": (C, K), "x": (R + 2 * N, C),
+                      "dt": (C, R), "o": (W, C)}
+            t.update({x + "conv.b": n(x + "conv.b", C, std=0.1),
+                      x + "dt.b": n(x + "dt.b", C, std=0.5, mean=-3.0),
+                      x + "A_log": n(x + "A_log", C, N, std=0.6, mean=1.2),
+                      x + "D": n(x + "D", C, std=0.3)})
+        t.update({x + k: n(x + k, *s) for k, s in shapes.items()})
+        if spec["mlp"] is not None:
+            F = spec["mlp"]["ff"]
+            t.update({p + "norm2": n(p + "norm2", W, std=0.1, mean=0.4),
+                      p + "mlp.up": n(p + "up", F, W),
+                      p + "mlp.down": n(p + "down", W, F),
+                      p + "rg2": n(p + "rg2", W, W),
+                      p + "rg2.b": n(p + "rg2.b", W, std=0.3)})
+        yield t
+
+
+def _pazilorn_weights(cfg, seed):
+    W = cfg.hidden_size
+
+    def n(name, *shape, std=None, mean=0.0):
+        return _normal(seed, name, shape, shape[-1] ** -0.5 if std is None
+                       else std, mean=mean)
+
+    yield {"embed": n("embed", cfg.vocab_size, W, std=1.0 / cfg.embed_scale),
+           "final.norm": n("final", W, std=0.1, mean=1.0)}
+    for i, spec in enumerate(cfg.layers):
+        p, m = f"l{i}.", spec["mixer"]
+        x = p + "mix."
+        t = {p + k: n(p + k, W, std=0.1, mean=1.0)
+             for k in ("norm1", "norm1b", "norm2", "norm2b")}
+        H, V = m["heads"], m["vdim"]
+        if spec["type"] == "channel_delta":
+            G, D, K = m["kv_heads"], m["dim"], m["conv"]
+            ra, rg = m["decay_rank"], m["gate_rank"]
+            shapes = {"q": (G * D, W), "k": (G * D, W), "v": (H * V, W),
+                      "b": (H, W), "a1": (ra, W), "a2": (H * D, ra),
+                      "g1": (rg, W), "g2": (H * V, rg), "o": (W, H * V)}
+            for leaf, rows in (("q", G * D), ("k", G * D), ("v", H * V)):
+                t[x + leaf + ".conv"] = n(x + leaf + ".conv", rows, K, std=0.5)
+            t.update({x + "A_log": n(x + "A_log", H, std=0.7),
+                      x + "dt_bias": n(x + "dt_bias", H * D, std=1.0, mean=-4.0),
+                      x + "norm": n(x + "norm", V, std=0.1, mean=1.0)})
+        else:
+            D, R, rk, rq = m["dim"], m["rot_dim"], m["kv_rank"], m["q_rank"]
+            shapes = {"dq": (rq, W), "uq": (H * (D + R), rq), "dkv": (rk + R, W),
+                      "uk": (H * D, rk), "uv": (H * V, rk), "g": (H, W),
+                      "o": (W, H * V)}
+            t.update({x + "dq.norm": n(x + "dq.norm", rq, std=0.1, mean=1.0),
+                      x + "dkv.norm": n(x + "dkv.norm", rk, std=0.1, mean=1.0)})
+        t.update({x + k: n(x + k, *s) for k, s in shapes.items()})
+        E, F = spec["mlp"]["router"]["experts"], spec["mlp"]["expert"]["ff"]
+        t[p + "mlp.router"] = n(p + "router", E, W, std=3.0 * W ** -0.5)
+        t[p + "mlp.router.b"] = n(p + "router.b", E, std=0.1)
+        for part, shape in (("gate", (E, F, W)), ("up", (E, F, W)),
+                            ("down", (E, W, F))):
+            full = n(p + part, *shape)
+            for e in range(E):
+                t[p + f"mlp.e{e}.{part}"] = full[e]
+        yield t
+
+
+def _weights(case, cfg, seed):
+    return {"gagorax": _gagorax_weights, "pazilorn": _pazilorn_weights}.get(
+        case["model"], _llama_weights)(cfg, seed)
+
+
+# ------------------------------------------------------------------ inputs
+def _prompts(case, cfg, seed):
+    g = torch.Generator().manual_seed(seed)
+    top = cfg.vocab_size - 2
+    out = [torch.randint(0, top, (n,), generator=g).tolist()
+           for n in _lengths(case)]
+    if case["kind"] == "mixed":
+        out.append(torch.randint(0, top, (case["prompt"],), generator=g).tolist())
+    return out
+
+
+def _cached_kv(case, cfg, seed, i, n):
+    """Pages of n tokens, [layers, 2, pages, kv heads, 16, dim]: what the
+    prefill instance hands over for request i (with fp8 pages: values that
+    such a page can hold)."""
+    pages = -(-n // PAGE)
+    kv = _normal(seed, f"kv{i}", (cfg.num_hidden_layers, 2, pages,
+                                  cfg.num_key_value_heads, PAGE, cfg.head_dim),
+                 1.0)
+    kv[:, 0] *= 2.0
+    if case["model"] == "dense-fp8":
+        kv = kv.to(torch.float8_e4m3fn).to(torch.bfloat16)
+    return kv
+
+
+@contextlib.contextmanager
+def _unset_embedding():
+    """An embedding is made without drawing values for it on the host, which
+    would take seconds: weights are loaded right after."""
+    reset = torch.nn.Embedding.reset_parameters
+    torch.nn.Embedding.reset_parameters = lambda self: None
+    try:
+        yield
+    finally:
+        torch.nn.Embedding.reset_parameters = reset
+
+
+def prepare(case, seed):
+    cfg = _config(case)
+    lens = _lengths(case)
+    pages = sum(-(-(n + 1 + case.get("tokens", 0)) // PAGE) for n in lens)
+    if case["kind"] == "mixed":
+        pages += -(-(case["prompt"] + 1) // PAGE)
+    low = case["model"] == "dense-fp8"
+    name = f"cases-{case['model']}"
+    PRESET_CONFIGS[name] = cfg
+    with _unset_embedding():
+        engine = LLMEngine(EngineConfig(
+            preset=name, seed=seed % (1 << 31), kv_cache_blocks=pages + 8,
+            max_num_seqs=max(case["batch"] + 1, 16),
+            max_num_batched_tokens=case.get("budget", 8192),
+            max_model_len=8192 + 16,  # a prompt of 8192 and its first token
+            kv_cache_dtype="fp8" if low else "auto",
+            # a repeated prompt has to run again
+            enable_prefix_caching=False))
+    for group in _weights(case, cfg, seed):
+        engine.runner.model.load_hf_state_dict(group)
+    if low:
+        engine.runner.model.quantize_fp8()
+    prompts = _prompts(case, cfg, seed)
+    state = {"engine": engine, "kind": case["kind"], "new": prompts,
+             "sampling": SamplingParams(max_tokens=case.get("tokens", 64),
+                                        ignore_eos=True)}
+    if case["kind"] in ("decode", "mixed"):
+        state["new"] = prompts[len(lens):]
+        for i, n in enumerate(lens):
+            engine.add_prefilled(prompts[i], prompts[i][0] ^ 1,
+                                 _cached_kv(case, cfg, seed, i, n),
+                                 state["sampling"], f"held-{i}")
+    run(state)  # captures the decode steps' graphs, as a server does at start
+    return state
+
+
+def run(state):
+    engine = state["engine"]
+    runner, scheduler = engine.runner, engine.scheduler
+    new = [engine.add_request(p, state["sampling"]) for p in state["new"]]
+    logits, tokens = [], []
+
+    def step():
+        batch = scheduler.schedule()
+        z = runner.forward_logits(batch)
+        ids = runner.sample(z, batch.seqs)
+        logits.append(z)
+        tokens.append(torch.tensor(ids))
+        return batch, ids
+
+    if state["kind"] == "serve":
+        while engine.has_work():
+            batch, ids = step()
+            logits[-1] = logits[-1].clone()  # the next step reuses the buffer
+            for seq, token in zip(batch.seqs, ids):
+                if seq.status is SeqStatus.RUNNING:
+                    seq.append_token(token)
+                    seq.check_finished(engine.model_cfg.eos_token_id)
+            scheduler.free_finished()
+        return {"logits": logits, "tokens": tokens}
+    step()
+    while scheduler.num_waiting:
+        step()
+    out = {"logits": logits, "tokens": tokens}
+    if new:
+        out["pages"] = [t for kv in runner.kv_caches for t in kv]
+    for seq in reversed(new):
+        scheduler.finish(seq)
+    return out
+
+
+# -------------------------------------------------------------------- work
+def _llama_counts(cfg):
+    """(attention weights, feed-forward weights of one expert, experts, of a
+    row) of one layer."""
+    W, D = cfg.hidden_size, cfg.head_dim
+    att = W * D * (2 * cfg.num_attention_heads + 2 * cfg.num_key_value_heads)
+    if cfg.num_local_experts:
+        return (att, 3 * W * cfg.moe_intermediate_size, cfg.num_local_experts,
+                cfg.num_experts_per_tok)
+    return att, 3 * W * cfg.intermediate_size, 1, 1
+
+
+def _layer_counts(spec, W):
+    """The same for a layer of a layer-list model, and the bytes of state
+    that a sequence's step reads and writes."""
+    m, state = spec["mixer"], 4 * W
+    if spec["type"] == "attention":
+        n = W * (m["heads"] * (m["dim"] + m["vdim"])
+                 + m["kv_heads"] * (m["dim"] + m["vdim"]))
+    elif spec["type"] == "lightning":
+        n = W * m["heads"] * (2 * m["dim"] + 3 * m["vdim"])
+        state += 4 * m["heads"] * m["dim"] * m["vdim"]
+    elif spec["type"] == "mamba1":
+        C, N, R = m["inner"], m["state"], m["dt_rank"]
+        n = 3 * C * W + C * (2 * R + 2 * N)
+        state += 4 * C * (N + m["conv"] - 1)
+    elif spec["type"] == "channel_delta":
+        H, G, D, V = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
+        ch = 2 * G * D + H * V
+        n = W * (ch + H + H * V) + (W + H * D) * m["decay_rank"] + (
+            W + H * V) * m["gate_rank"]
+        state = 4 * (H * D * V + (m["conv"] - 1) * ch)
+    else:
+        H, D, R, V = m["heads"], m["dim"], m["rot_dim"], m["vdim"]
+        n = W * (m["q_rank"] + m["kv_rank"] + R + H + H * V) + (
+            H * (D + R) * m["q_rank"] + H * (D + V) * m["kv_rank"])
+        state = 0
+    mlp = spec["mlp"]
+    if spec["type"] in ("attention", "lightning", "mamba1"):  # residual gates
+        n += W * W * (2 if mlp else 1)
+    if mlp is None:
+        return n, 0, 1, 1, state
+    if mlp.get("kind") == "moe":
+        r = mlp["router"]
+        return (n + W * r["experts"], 3 * W * mlp["expert"]["ff"], r["experts"],
+                r["top"], state)
+    return n, 2 * W * mlp["ff"], 1, 1, state
+
+
+def _touched(experts, per_row, rows):
+    """Experts that `rows` rows use, choices taken as even."""
+    return experts * (1.0 - (1.0 - per_row / experts) ** rows)
+
+
+def work(case):
+    cfg = _config(case)
+    W, V = cfg.hidden_size, cfg.vocab_size
+    lens = _lengths(case)
+    if case["kind"] == "decode":
+        steps = [[(n, 1) for n in lens]]
+    elif case["kind"] == "prefill":
+        steps = [[(0, n) for n in lens]]
+    elif case["kind"] == "mixed":
+        steps, at = [], 0
+        while at < case["prompt"]:
+            n = min(case["budget"] - len(lens), case["prompt"] - at)
+            steps.append([(c, 1) for c in lens] + [(at, n)])
+            at += n
+    else:
+        steps = [[(0, n) for n in lens]] + [
+            [(n + j, 1) for n in lens] for j in range(case["tokens"] - 1)]
+    low = case["model"] == "dense-fp8"
+    moved = flops = 0.0
+    for step in steps:
+        rows = sum(n for _, n in step)
+        # the logits: output rows once, one row of scores per sequence
+        moved += V * W * (1 if low else 2) + len(step) * V * (
+            4 if hasattr(cfg, "layers") else 2) + rows * W * 2
+        flops += 2.0 * len(step) * V * W
+        for i in range(cfg.num_hidden_layers):
+            if hasattr(cfg, "layers"):
+                spec = cfg.layers[i]
+                n, ff, E, k, state = _layer_counts(spec, W)
+                m = spec["mixer"]
+                moved += 2 * state * len(step)
+                flops += 4.0 * rows * (state / 4)
+                pairs = None
+                if spec["type"] == "attention":
+                    pairs = (m["heads"] * (m["dim"] + m["vdim"]),
+                             m["kv_heads"] * (m["dim"] + m["vdim"]))
+                elif spec["type"] == "latent_attention":
+                    pairs = (m["heads"] * (m["dim"] + m["rot_dim"] + m["vdim"]),
+                             m["kv_rank"] + m["rot_dim"])
+                window = (m.get("mask") or {}).get("size", 1 << 30)
+            else:
+                n, ff, E, k = _llama_counts(cfg)
+                pairs = (2 * cfg.num_attention_heads * cfg.head_dim,
+                         2 * cfg.num_key_value_heads * cfg.head_dim)
+                window = 1 << 30
+            touched = ff * (_touched(E, k, rows) if E > 1 else 1)
+            if low:
+                o = W * cfg.num_attention_heads * cfg.head_dim
+                moved += 2 * o + (n - o) + touched
+            else:
+                moved += 2 * (n + touched)
+            flops += 2.0 * rows * (n + k * ff)
+            if pairs:
+                seen = sum(min(c + t / 2, window) * t for c, t in step)
+                held = sum(min(c, window) + 2 * t for c, t in step)
+                moved += held * pairs[1] * (1 if low else 2)
+                flops += 2.0 * seen * pairs[0]
+    return {"bytes": moved, "flops": flops}
+
+
+def tolerance(case):
+    """bf16 rows through the layers of a slice: the present code is 0.006 to
+    0.013 off exact() (0.08 with fp8, whose rows have 3 bits of mantissa, so
+    that the last bit of a bf16 value can move one by a sixteenth), and
+    another order of the same sums can be about as far off the present code.
+    The largest single differences were 0.03 to 0.1 (fp8: 0.45)."""
+    return {"rel": 0.03, "max": 0.6, "differ": 0.005}
+
+
+# ------------------------------------------------- the same in 64 bits
+def _rms(x, w, eps):
+    return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + eps) * w
+
+
+def _silu(x):
+    return x * torch.sigmoid(x)
+
+
+def _attend(q, k, v, scale, start, window=1 << 30, sink=False):
+    """q [n, H, D] at positions start.., k [m, G, D], v [m, G, V] from
+    position 0: causal softmax attention, [n, H, V]."""
+    n, H, _ = q.shape
+    G = k.shape[1]
+    out = torch.empty(n, H, v.shape[2], dtype=F64, device=q.device)
+    kt, vt = k.permute(1, 2, 0), v.transpose(0, 1)
+    rows = max(1, min(n, (1 << 28) // (H * k.shape[0])))
+    j = torch.arange(k.shape[0], device=q.device)
+    for a in range(0, n, rows):
+        qa = q[a:a + rows].reshape(-1, G, H // G, q.shape[2])
+        r = qa.shape[0]
+        s = torch.matmul(qa.permute(1, 2, 0, 3).reshape(G, -1, q.shape[2])
+                         .contiguous(), kt.contiguous()) * scale
+        s = s.view(G, H // G, r, -1)
+        i = torch.arange(start + a, start + a + r, device=q.device)[:, None]
+        s.masked_fill_((j > i) | (i - j >= window), -math.inf)
+        top = s.amax(-1, keepdim=True)
+        if sink:
+            top = top.clamp(min=0.0)
+        p = torch.exp(s - top)
+        total = p.sum(-1, keepdim=True)
+        if sink:
+            total = total + torch.exp(-top)
+        p /= total
+        o = torch.matmul(p.view(G, -1, p.shape[-1]), vt.contiguous())
+        out[a:a + r] = o.view(G, H // G, r, -1).permute(2, 0, 1, 3).reshape(
+            r, H, -1)
+    return out
+
+
+def _angles(freqs, positions):
+    a = positions.to(F64)[:, None] * freqs
+    return torch.cos(a)[:, None], torch.sin(a)[:, None]
+
+
+def _turn_halves(x, cos, sin):
+    h = x.shape[-1] // 2
+    u, v = x[..., :h], x[..., h:]
+    return torch.cat([u * cos - v * sin, v * cos + u * sin], -1)
+
+
+def _turn_pairs(x, cos, sin):
+    out = torch.empty_like(x)
+    u, v = x[..., 0::2], x[..., 1::2]
+    out[..., 0::2], out[..., 1::2] = u * cos - v * sin, v * cos + u * sin
+    return out
+
+
+def _experts(h, weights, ids, expert):
+    """sum_j weights[t, j] expert(ids[t, j])(h[t])."""
+    out = torch.zeros_like(h)
+    for e in ids.unique().tolist():
+        t, j = (ids == e).nonzero(as_tuple=True)
+        out.index_add_(0, t, expert(e, h[t]) * weights[t, j][:, None])
+    return out
+
+
+def _fp8_rows(w):
+    """A weight as the fp8 option keeps it: e4m3 under one scale per row."""
+    scale = 448.0 / w.float().abs().amax(1, keepdim=True).clamp(min=1e-6)
+    return (w.float() * scale).to(torch.float8_e4m3fn).to(F64) / scale
+
+
+def _exact_llama(case, cfg, seed):
+    lens, prompts = _lengths(case), _prompts(case, cfg, seed)
+    D, G = cfg.head_dim, cfg.num_key_value_heads
+    freqs = cfg.rope_theta ** (-torch.arange(0, D, 2, dtype=F64, device="cuda") / D)
+    # requests as (tokens to run, tokens held); held keys and values by layer
+    if case["kind"] == "prefill":
+        reqs = [(p, 0) for p in prompts]
+    else:
+        reqs = [([p[0] ^ 1], n) for p, n in zip(prompts, lens)]
+        reqs += [(p, 0) for p in prompts[len(lens):]]
+    groups = _weights(case, cfg, seed)
+    first = next(groups)
+    x = torch.cat([first["model.embed_tokens.weight"][
+        torch.tensor(t, device="cuda")].to(F64) for t, _ in reqs])
+    pos = torch.cat([torch.arange(n, n + len(t), device="cuda") for t, n in reqs])
+    cos, sin = _angles(freqs, pos)
+    wide = case["model"] != "dense-fp8"
+    final, head = first["model.norm.weight"].to(F64), first["lm_head.weight"]
+    held = [_cached_kv(case, cfg, seed, r, n) if n else None
+            for r, (_, n) in enumerate(reqs)]
+    for i, t in enumerate(groups):
+        w = {k[len(f"model.layers.{i}."):]: v for k, v in t.items()}
+
+        def proj(h, name):
+            m = w[name + ".weight"]
+            y = h @ (m.to(F64) if wide or "o_proj" in name else _fp8_rows(m)).t()
+            return y + w[name + ".bias"].to(F64) if name + ".bias" in w else y
+
+        h = _rms(x, w["input_layernorm.weight"].to(F64), cfg.rms_norm_eps)
+        q = proj(h, "self_attn.q_proj").unflatten(-1, (-1, D))
+        k = proj(h, "self_attn.k_proj").unflatten(-1, (-1, D))
+        v = proj(h, "self_attn.v_proj").unflatten(-1, (-1, D))
+        if cfg.qk_norm:
+            q = _rms(q, w["self_attn.q_norm.weight"].to(F64), cfg.rms_norm_eps)
+            k = _rms(k, w["self_attn.k_norm.weight"].to(F64), cfg.rms_norm_eps)
+        q, k = _turn_halves(q, cos, sin), _turn_halves(k, cos, sin)
+        o, at = torch.empty_like(q), 0
+        for (toks, n), kv in zip(reqs, held):
+            s = slice(at, at + len(toks))
+            at += len(toks)
+            ks, vs = k[s], v[s]
+            if n:
+                old = kv[i].permute(0, 1, 3, 2, 4).reshape(2, -1, G, D)[:, :n]
+                ks = torch.cat([old[0].to(F64), ks])
+                vs = torch.cat([old[1].to(F64), vs])
+            o[s] = _attend(q[s], ks, vs, D ** -0.5, n)
+        x = x + proj(o.flatten(1), "self_attn.o_proj")
+        h = _rms(x, w["post_attention_layernorm.weight"].to(F64),
+                 cfg.rms_norm_eps)
+        if cfg.num_local_experts:
+            p = torch.softmax(h @ w["mlp.gate.weight"].to(F64).t(), -1)
+            p, ids = p.topk(cfg.num_experts_per_tok)
+            if cfg.norm_topk_prob:
+                p = p / p.sum(-1, keepdim=True)
+
+            def expert(e, r):
+                b = f"mlp.experts.{e}."
+                a = _silu(proj(r, b + "gate_proj")) * proj(r, b + "up_proj")
+                return proj(a, b + "down_proj")
+
+            x = x + _experts(h, p, ids, expert)
+        else:
+            x = x + proj(_silu(proj(h, "mlp.gate_proj"))
+                         * proj(h, "mlp.up_proj"), "mlp.down_proj")
+    x = _rms(x, final, cfg.rms_norm_eps)
+    if case["kind"] == "mixed":
+        # every step: the held requests' rows, then the chunk's last row
+        B, step, n = len(lens), case["budget"] - len(lens), case["prompt"]
+        picks = [list(range(B)) + [B + min(a + step, n) - 1]
+                 for a in range(0, n, step)]
+    else:
+        ends, at = [], -1
+        for t, _ in reqs:
+            at += len(t)
+            ends.append(at)
+        picks = [ends]
+    head = (head.to(F64) if wide else _fp8_rows(head)).t()
+    return {"logits": [x[torch.tensor(p, device="cuda")] @ head for p in picks],
+            "tokens": None, "pages": None}
+
+
+def _gagorax_mixer(spec, w, h, pos, st, eps):
+    m, n, dev = spec["mixer"], h.shape[0], h.device
+    if spec["type"] == "attention":
+        H, G, D, V = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
+        f = m["rot"]["base"] ** (-torch.arange(0, D, 2, dtype=F64, device=dev) / D)
+        cos, sin = _angles(f, pos)
+        q = _rms((h @ w["q"].t()).view(n, H, D), w["q.norm"], eps)
+        k = _rms((h @ w["k"].t()).view(n, G, D), w["k.norm"], eps)
+        v = _turn_pairs((h @ w["v"].t()).view(n, G, V), cos, sin)
+        k = _turn_pairs(k, cos, sin)
+        st["k"] = torch.cat([st["k"], k]) if "k" in st else k
+        st["v"] = torch.cat([st["v"], v]) if "v" in st else v
+        o = _attend(_turn_pairs(q, cos, sin), st["k"], st["v"], m["scale"],
+                    int(pos[0]), sink=True)
+        return _turn_pairs(o, cos, -sin).flatten(1) @ w["o"].t()
+    if spec["type"] == "lightning":
+        H, D, V = m["heads"], m["dim"], m["vdim"]
+        q, k, v = (_silu(h @ w[c].t()).view(n, H, -1) for c in "qkv")
+        decay = torch.tensor(m["decay"], dtype=F64, device=dev)[:, None, None]
+        S = st.get("S", torch.zeros(H, D, V, dtype=F64, device=dev))
+        o = torch.empty(n, H, V, dtype=F64, device=dev)
+        for t in range(n):
+            S = decay * S + k[t][:, :, None] * v[t][:, None, :]
+            o[t] = (q[t][:, None, :] @ S)[:, 0]
+        st["S"] = S
+        y = _rms(o.flatten(1), w["norm"], eps) * torch.sigmoid(h @ w["g"].t())
+        return y @ w["o"].t()
+    C, N, R, K = m["inner"], m["state"], m["dt_rank"], m["conv"]
+    x, z = (h @ w["in"].t()).split(C, -1)
+    past = st.get("conv", torch.zeros(K - 1, C, dtype=F64, device=dev))
+    x = torch.cat([past, x])
+    st["conv"] = x[-(K - 1):]
+    x = _silu(sum(x[j:j + n] * w["conv"][:, j] for j in range(K)) + w["conv.b"])
+    dt, B, Cm = (x @ w["x"].t()).split([R, N, N], -1)
+    dt = torch.nn.functional.softplus(dt @ w["dt"].t() + w["dt.b"])
+    A = -torch.exp(w["A_log"])
+    S = st.get("S", torch.zeros(C, N, dtype=F64, device=dev))
+    y = torch.empty_like(x)
+    u = dt * x
+    for t in range(n):
+        S = torch.exp(dt[t][:, None] * A) * S + u[t][:, None] * B[t]
+        y[t] = S @ Cm[t]
+    st["S"] = S
+    return ((y + w["D"] * x) * _silu(z)) @ w["o"].t()
+
+
+def _gagorax_layer(spec, w, x, pos, st, eps):
+    mix = {k[4:]: v for k, v in w.items() if k.startswith("mix.")}
+    prev = torch.cat([st.get("row", torch.zeros_like(x[:1])), x[:-1]])
+    st["row"] = x[-1:]
+    y = _gagorax_mixer(spec, mix, x + (prev - x) * w["shift"], pos,
+                       st.setdefault("mix", {}), eps)
+    y = y * torch.sigmoid(x @ w["rg1"].t() + w["rg1.b"])
+    x = x + _rms(y, w["norm1"], eps)
+    if spec["mlp"] is not None:
+        y = torch.nn.functional.gelu(x @ w["mlp.up"].t(), approximate="tanh")
+        y = (y @ w["mlp.down"].t()) * torch.sigmoid(
+            x @ w["rg2"].t() + w["rg2.b"])
+        x = x + _rms(y, w["norm2"], eps)
+    return x
+
+
+def _ramped_freqs(rot, dev):
+    n, sc = rot["dims"], rot["scaling"]
+    f = rot["base"] ** (-torch.arange(0, n, 2, dtype=F64, device=dev) / n)
+
+    def at(turns):
+        return n * math.log(sc["original"] / (2 * math.pi * turns)) / (
+            2 * math.log(rot["base"]))
+
+    lo = max(math.floor(at(sc["fast"])), 0)
+    hi = min(math.ceil(at(sc["slow"])), n - 1)
+    ramp = ((torch.arange(n // 2, dtype=F64, device=dev) - lo)
+            / max(hi - lo, 0.001)).clamp(0.0, 1.0)
+    return (f / sc["factor"] * ramp + f * (1.0 - ramp),
+            0.1 * math.log(sc["factor"]) + 1.0)
+
+
+def _pazilorn_mixer(spec, w, h, pos, st, eps):
+    m, n, dev = spec["mixer"], h.shape[0], h.device
+    H, D, V = m["heads"], m["dim"], m["vdim"]
+    if spec["type"] == "channel_delta":
+        K = m["conv"]
+
+        def conv(leaf):
+            u = h @ w[leaf].t()
+            past = st.get(leaf, torch.zeros(K - 1, u.shape[1], dtype=F64,
+                                            device=dev))
+            u = torch.cat([past, u])
+            st[leaf] = u[-(K - 1):]
+            return _silu(sum(u[j:j + n] * w[leaf + ".conv"][:, j]
+                             for j in range(K))).view(n, H, -1)
+
+        q, k, v = conv("q"), conv("k"), conv("v")
+        q, k = (t * torch.rsqrt((t * t).sum(-1, keepdim=True) + 1e-6)
+                for t in (q, k))
+        q = q * D ** -0.5
+        g = torch.nn.functional.softplus(
+            (h @ w["a1"].t()) @ w["a2"].t() + w["dt_bias"]).view(n, H, D)
+        g = torch.exp(-torch.exp(w["A_log"])[:, None] * g)
+        beta = torch.sigmoid(h @ w["b"].t())
+        S = st.get("S", torch.zeros(H, D, V, dtype=F64, device=dev))
+        o = torch.empty(n, H, V, dtype=F64, device=dev)
+        for t in range(n):
+            S = g[t][:, :, None] * S
+            u = beta[t][:, None] * (v[t] - (k[t][:, None, :] @ S)[:, 0])
+            S = S + k[t][:, :, None] * u[:, None, :]
+            o[t] = (q[t][:, None, :] @ S)[:, 0]
+        st["S"] = S
+        gate = torch.sigmoid((h @ w["g1"].t()) @ w["g2"].t()).view(n, H, V)
+        return (_rms(o, w["norm"], eps) * gate).flatten(1) @ w["o"].t()
+    R, rank = m["rot_dim"], m["kv_rank"]
+    f, mag = _ramped_freqs(m["rot"], dev)
+    cos, sin = (a * mag for a in _angles(f, pos))
+    q = (_rms(h @ w["dq"].t(), w["dq.norm"], eps) @ w["uq"].t()).view(n, H, D + R)
+    down = h @ w["dkv"].t()
+    c = _rms(down[:, :rank], w["dkv.norm"], eps)
+    kr = _turn_halves(down[:, None, rank:], cos, sin)
+    q = torch.cat([q[..., :D], _turn_halves(q[..., D:], cos, sin)], -1)
+    k = torch.cat([(c @ w["uk"].t()).view(n, H, D), kr.expand(n, H, R)], -1)
+    v = (c @ w["uv"].t()).view(n, H, V)
+    st["k"] = torch.cat([st["k"], k]) if "k" in st else k
+    st["v"] = torch.cat([st["v"], v]) if "v" in st else v
+    o = _attend(q, st["k"], st["v"], m["scale"], int(pos[0]), m["mask"]["size"])
+    o = o * torch.sigmoid(h @ w["g"].t())[:, :, None]
+    return o.flatten(1) @ w["o"].t()
+
+
+def _pazilorn_layer(spec, w, x, pos, st, eps, mult=0.5):
+    mix = {k[4:]: v for k, v in w.items() if k.startswith("mix.")}
+    y = _pazilorn_mixer(spec, mix, _rms(x, w["norm1"], eps), pos, st, eps)
+    x = x + mult * _rms(y, w["norm1b"], eps)
+    h = _rms(x, w["norm2"], eps)
+    z, ids = (h @ w["mlp.router"].t() + w["mlp.router.b"]).topk(
+        spec["mlp"]["router"]["top"])
+
+    def expert(e, r):
+        gate, up, down = (w[f"mlp.e{e}.{p}"].to(F64) for p in ("gate", "up", "down"))
+        return (_silu(r @ gate.t()) * (r @ up.t())) @ down.t()
+
+    y = _experts(h, torch.softmax(z, -1), ids, expert)
+    return x + mult * _rms(y, w["norm2b"], eps)
+
+
+def _exact_layers(case, cfg, seed):
+    """Layer-list models: every request's prompt, then token by token."""
+    groups = list(_weights(case, cfg, seed))
+    first = groups.pop(0)
+    embed = first["embed"]
+    head = first.get("head", embed).to(F64).t()
+    final = first["final.norm"].to(F64)
+    layer = _gagorax_layer if case["model"] == "gagorax" else _pazilorn_layer
+    weights = [{k.split(".", 1)[1]: v if ".mlp.e" in k else v.to(F64)
+                for k, v in t.items()} for t in groups]
+    eps = cfg.rms_norm_eps
+    prompts = _prompts(case, cfg, seed)
+    states = [[{} for _ in cfg.layers] for _ in prompts]
+    run_now, held = prompts, [0] * len(prompts)
+    logits = []
+    for _ in range(case["tokens"]):
+        last = []
+        for r, toks in enumerate(run_now):
+            x = embed[torch.tensor(toks, device="cuda")].to(F64) * cfg.embed_scale
+            pos = torch.arange(held[r], held[r] + len(toks), device="cuda")
+            for i, spec in enumerate(cfg.layers):
+                x = layer(spec, weights[i], x, pos, states[r][i], eps)
+            held[r] += len(toks)
+            last.append(x[-1])
+        z = _rms(torch.stack(last), final, eps) @ head * cfg.logit_scale
+        if cfg.logit_softcap:
+            z = cfg.logit_softcap * torch.tanh(z / cfg.logit_softcap)
+        logits.append(z)
+        run_now = [[t] for t in z.argmax(-1).tolist()]
+    return {"logits": logits, "tokens": None}
+
+
+def exact(case, seed):
+    cfg = _config(case)
+    with torch.no_grad():
+        if case["kind"] == "serve":
+            return _exact_layers(case, cfg, seed)
+        return _exact_llama(case, cfg, seed)
