@@ -63,11 +63,9 @@ void arks_skinny_gemm_v(void* part, void* out, const void* a, const void* w,
                         const void* bias, int m_rows, int n_total, int k_total,
                         int k_per_split, int nsplits, int64_t a_stride,
                         int variant, bool fuse_silu, hipStream_t stream);
-void arks_greedy_sample(void* out, const void* logits, int rows, int vocab,
-                        hipStream_t stream);
-void arks_gumbel_sample(void* out, const void* logits, const void* temperatures,
-                        const void* uniform, int rows, int vocab,
-                        hipStream_t stream);
+void arks_sample(void* out, void* part_val, void* part_idx, const void* logits,
+                 const void* temperatures, const void* uniform, int rows,
+                 int vocab, int parts, hipStream_t stream);
 void arks_ar_seq_inc(void* seq, hipStream_t stream);
 void arks_one_shot_allreduce(void* out, const void* src, void* mail_ptrs[8],
                              void* flag_ptrs[8], void* seq, int rank,
@@ -327,11 +325,28 @@ void quant_fp8_rows(torch::Tensor out, torch::Tensor inv_scale,
                       x.size(0), x.size(1), current_stream());
 }
 
+// Workgroups per row: ~1024 in all (4 per CU), each with at least 2048 values.
+void sample_rows(torch::Tensor out, torch::Tensor logits, const void* temps,
+                 const void* uniform) {
+  const int64_t rows = logits.size(0), vocab = logits.size(1);
+  const int64_t parts = std::max<int64_t>(
+      1, std::min<int64_t>({64, vocab / 2048,
+                            1024 / std::max<int64_t>(rows, 1)}));
+  torch::Tensor val, idx;
+  if (parts > 1) {
+    val = torch::empty({rows * parts}, logits.options().dtype(torch::kFloat32));
+    idx = torch::empty({rows * parts}, logits.options().dtype(torch::kInt32));
+  }
+  if (rows > 0)
+    arks_sample(out.data_ptr(), parts > 1 ? val.data_ptr() : nullptr,
+                parts > 1 ? idx.data_ptr() : nullptr, logits.data_ptr(), temps,
+                uniform, (int)rows, (int)vocab, (int)parts, current_stream());
+}
+
 void greedy_sample(torch::Tensor out, torch::Tensor logits) {
   check_bf16_contig(logits, "logits");
   TORCH_CHECK(out.scalar_type() == torch::kInt64);
-  arks_greedy_sample(out.data_ptr(), logits.data_ptr(), logits.size(0),
-                     logits.size(1), current_stream());
+  sample_rows(out, logits, nullptr, nullptr);
 }
 
 void gumbel_sample(torch::Tensor out, torch::Tensor logits,
@@ -340,9 +355,7 @@ void gumbel_sample(torch::Tensor out, torch::Tensor logits,
   TORCH_CHECK(out.scalar_type() == torch::kInt64);
   TORCH_CHECK(temperatures.scalar_type() == torch::kFloat32);
   TORCH_CHECK(uniform.scalar_type() == torch::kFloat32);
-  arks_gumbel_sample(out.data_ptr(), logits.data_ptr(), temperatures.data_ptr(),
-                     uniform.data_ptr(), logits.size(0), logits.size(1),
-                     current_stream());
+  sample_rows(out, logits, temperatures.data_ptr(), uniform.data_ptr());
 }
 
 // D[16,16] = A[16,32] @ B[32,16], all bf16 in / f32 out. Verifies the MFMA

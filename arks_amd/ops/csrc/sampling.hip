@@ -11,16 +11,24 @@
 
 namespace arks {
 
-// One workgroup (256 threads) per row; each thread scans a strided slice
-// keeping (best_val, best_idx); reduce via wave shuffles + LDS.
+// Latency bounds it at few rows: one workgroup walking a row of 152064 took
+// 55-60 us, 1 row or 64. So a row is cut over `parts` workgroups, as many
+// as give ~1024 in all but at least 2048 values each (one 16 B load per
+// thread), and a wave per row picks among their (value, index) pairs: 10 us at
+// 1 row, 14 us at 64, both launches together.
+//
+// Each thread scans a strided slice of its workgroup's part keeping
+// (best_val, best_idx); reduce via wave shuffles + LDS.
 template <bool GUMBEL>
-__global__ void sample_kernel(int64_t* __restrict__ out,
+__global__ void sample_kernel(int64_t* __restrict__ out,     // parts == 1
+                              float* __restrict__ part_val,  // [rows, parts]
+                              int* __restrict__ part_idx,
                               const bf16* __restrict__ logits,  // [rows, vocab]
                               const float* __restrict__ temperatures,  // null if !GUMBEL
                               const float* __restrict__ uniform,  // [rows, vocab]
-                              const int vocab) {
+                              const int vocab, const int parts) {
   constexpr int BLOCK = 256;
-  const int row = blockIdx.x;
+  const int row = blockIdx.x / parts, part = blockIdx.x % parts;
   const bf16* lrow = logits + (int64_t)row * vocab;
   float inv_t = 0.f;
   bool greedy = true;
@@ -36,7 +44,9 @@ __global__ void sample_kernel(int64_t* __restrict__ out,
   // Vectorized 8-wide scan. vocab need not be a multiple of 8: tail handled
   // scalar.
   const int nvec = vocab / 8;
-  for (int i = threadIdx.x; i < nvec; i += BLOCK) {
+  const int v_lo = (int)((int64_t)nvec * part / parts);
+  const int v_hi = (int)((int64_t)nvec * (part + 1) / parts);
+  for (int i = v_lo + threadIdx.x; i < v_hi; i += BLOCK) {
     ushort8 x = *reinterpret_cast<const ushort8*>(lrow + i * 8);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -55,7 +65,8 @@ __global__ void sample_kernel(int64_t* __restrict__ out,
       }
     }
   }
-  for (int idx = nvec * 8 + threadIdx.x; idx < vocab; idx += BLOCK) {
+  for (int idx = part + 1 == parts ? nvec * 8 + threadIdx.x : vocab; idx < vocab;
+       idx += BLOCK) {
     float v = bf16_bits_to_float(lrow[idx]);
     if constexpr (GUMBEL) {
       if (!greedy) {
@@ -97,8 +108,33 @@ __global__ void sample_kernel(int64_t* __restrict__ out,
         bi = sidx[w];
       }
     }
-    out[row] = bi;
+    if (parts == 1) {
+      out[row] = bi;
+    } else {
+      part_val[row * parts + part] = b;
+      part_idx[row * parts + part] = bi;
+    }
   }
+}
+
+// One wave per row over its parts' (value, index) pairs.
+__global__ __launch_bounds__(64) void sample_pick_kernel(
+    int64_t* __restrict__ out, const float* __restrict__ part_val,
+    const int* __restrict__ part_idx, const int parts) {
+  const int row = blockIdx.x, lane = threadIdx.x;
+  const int at = row * parts + min(lane, parts - 1);
+  float best = part_val[at];
+  int best_idx = part_idx[at];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    float ov = __shfl_xor(best, off, WAVE_SIZE);
+    int oi = __shfl_xor(best_idx, off, WAVE_SIZE);
+    if (ov > best || (ov == best && oi < best_idx)) {
+      best = ov;
+      best_idx = oi;
+    }
+  }
+  if (lane == 0) out[row] = best_idx;
 }
 
 }  // namespace arks
@@ -107,19 +143,25 @@ using namespace arks;
 
 extern "C" {
 
-void arks_greedy_sample(void* out, const void* logits, int rows, int vocab,
-                        hipStream_t stream) {
-  hipLaunchKernelGGL((sample_kernel<false>), dim3(rows), dim3(256), 0, stream,
-                     (int64_t*)out, (const bf16*)logits, nullptr, nullptr,
-                     vocab);
-}
-
-void arks_gumbel_sample(void* out, const void* logits, const void* temperatures,
-                        const void* uniform, int rows, int vocab,
-                        hipStream_t stream) {
-  hipLaunchKernelGGL((sample_kernel<true>), dim3(rows), dim3(256), 0, stream,
-                     (int64_t*)out, (const bf16*)logits,
-                     (const float*)temperatures, (const float*)uniform, vocab);
+// temperatures, uniform: null for greedy; part_val, part_idx: rows * parts
+// values each (unused for one part), parts <= 64
+void arks_sample(void* out, void* part_val, void* part_idx, const void* logits,
+                 const void* temperatures, const void* uniform, int rows,
+                 int vocab, int parts, hipStream_t stream) {
+  dim3 grid(rows * parts), block(256);
+  if (temperatures)
+    hipLaunchKernelGGL((sample_kernel<true>), grid, block, 0, stream,
+                       (int64_t*)out, (float*)part_val, (int*)part_idx,
+                       (const bf16*)logits, (const float*)temperatures,
+                       (const float*)uniform, vocab, parts);
+  else
+    hipLaunchKernelGGL((sample_kernel<false>), grid, block, 0, stream,
+                       (int64_t*)out, (float*)part_val, (int*)part_idx,
+                       (const bf16*)logits, nullptr, nullptr, vocab, parts);
+  if (parts > 1)
+    hipLaunchKernelGGL(sample_pick_kernel, dim3(rows), dim3(64), 0, stream,
+                       (int64_t*)out, (const float*)part_val,
+                       (const int*)part_idx, parts);
 }
 
 }  // extern "C"

@@ -195,6 +195,23 @@ def test_attention_decode_partitions_agree():
     torch.testing.assert_close(o8.float().cpu(), expect, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("rows,vocab", [(1, 5), (1, 4095), (1, 4096), (3, 20001),
+                                        (64, 152064), (600, 4099)])
+def test_greedy_sample_parts(rows, vocab):
+    """Rows cut over workgroups: the first of the largest values wins, also
+    where its equals lie in other parts."""
+    assert_native()
+    g = torch.Generator().manual_seed(vocab)
+    logits = torch.randint(-50, 50, (rows, vocab), generator=g).to(torch.bfloat16)
+    logits[0] = -1.0
+    logits[0, -1] = 3.0
+    if rows > 1:
+        logits[1] = float("-inf")
+        logits[1, vocab // 2] = logits[1, vocab // 2 + 1] = -7.0
+    out = ops.greedy_sample(logits.to(DEV)).cpu()
+    assert torch.equal(out, torch.from_numpy(logits.float().numpy().argmax(1)))
+
+
 def test_strided_qkv_views():
     """RoPE/cache/attention on strided views into a fused QKV buffer must
     match the contiguous path (the engine's no-copy hot path)."""
