@@ -40,6 +40,10 @@ class ForwardBatch:
     # them, keyed by head layout
     kv_lens_list: list[int] | None = None
     tile_cache: dict = field(default_factory=dict)
+    # what the layers of one forward pass share and derive on the device
+    # (emptied at its start: a captured pass has to hold the kernels that
+    # make it)
+    step_cache: dict = field(default_factory=dict)
 
     @property
     def num_tokens(self) -> int:

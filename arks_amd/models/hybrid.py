@@ -563,6 +563,7 @@ class HybridForCausalLM(nn.Module):
     # ------------------------------------------------------------ forward
     def forward(self, batch: ForwardBatch, caches: list) -> torch.Tensor:
         """fp32 logits for batch.logits_indices rows (all rows if None)."""
+        batch.step_cache = {}
         if self.arr.norm_place == "input":
             return self._forward_streams(batch, caches)
         if self.arr.norm_place == "shared":

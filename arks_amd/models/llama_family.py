@@ -116,6 +116,7 @@ class Attention(nn.Module):
                     q, k_cache, v_cache, batch.block_tables, batch.seq_lens,
                     batch.cu_seqlens, batch.seq_lens_list, self.scale,
                     window=self.window, tiles=batch.ext_tiles,
+                    step_cache=batch.step_cache,
                 )
             else:
                 out = ops.attention_prefill_varlen(
@@ -125,7 +126,9 @@ class Attention(nn.Module):
         else:
             out = ops.attention_decode_paged(
                 q, k_cache, v_cache, batch.block_tables, batch.seq_lens,
-                self.scale, window=self.window,
+                self.scale, window=self.window, plan=ops.step_decode_plan(
+                    batch.seq_lens, self.nkv_local, self.window,
+                    k_cache.dtype != torch.bfloat16, None, batch.step_cache),
             )
         return self.o_proj(out.view(T, -1))
 
@@ -456,6 +459,7 @@ class LlamaFamilyForCausalLM(nn.Module):
 
     def forward(self, batch: ForwardBatch, kv_caches: list) -> torch.Tensor:
         """Returns logits for batch.logits_indices rows."""
+        batch.step_cache = {}
         x = self.embed_tokens(batch.input_ids)
         residual = None
         for i, layer in enumerate(self.layers):

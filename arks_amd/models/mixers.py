@@ -291,7 +291,8 @@ class SinkRotaryAttention(nn.Module):
             q, cache["k"], cache["v"], batch.block_tables, batch.seq_lens,
             batch.cu_seqlens, batch.token_seq, self.scale, self.sink,
             self.inv_freq_v, self.interleaved, batch.max_q_len,
-            batch.positions, self._tiles(batch, q))
+            batch.positions, self._tiles(batch, q),
+            step_cache=batch.step_cache)
         if out_scale != 1.0:
             res = res * out_scale
         out.copy_(res.view(p.shape[0], H * V))
@@ -310,7 +311,8 @@ class SinkRotaryAttention(nn.Module):
             q, cache["k"], cache["v"], batch.block_tables, batch.seq_lens,
             batch.cu_seqlens, batch.token_seq, self.scale, self.sink,
             self.inv_freq_v, self.interleaved, batch.max_q_len,
-            batch.positions, self._tiles(batch, q))
+            batch.positions, self._tiles(batch, q),
+            step_cache=batch.step_cache)
         return linear(out.view(T, H * V), self.o)
 
 

@@ -235,7 +235,7 @@ def attention_extend_paged(
     q, k_cache, v_cache, block_tables, kv_lens, cu_seqlens_q,
     q_lens: list[int], scale: float, window: int = 0, tiles=None,
     sink: bool = False, native=None, maps: int = 1, sink_w=None, slopes=None,
-    out=None,
+    out=None, step_cache: dict | None = None,
 ):
     """Causal attention of packed NEW tokens over each sequence's full paged
     KV history (cached prefix + new tokens already written by
@@ -251,7 +251,9 @@ def attention_extend_paged(
     a sink's score per head, a distance bias slope[h] (i - j) off the scores
     (256-row tiles and single rows only: build_extend_tiles(min_ladder=1);
     the extension must be the layer-list models'). out: a contiguous
-    [Tq, Hq, D] tensor to write.
+    [Tq, Hq, D] tensor to write. step_cache: a dict of the calls of one
+    forward pass, which shares what they would each derive from the lengths
+    and tables of the single rows.
 
     Dispatch: big chunks run the 8-wave 32x32-MFMA ladder kernel
     (attn_extend2.hip, 256-row q tiles); small chunks and fp8-KV runs use
@@ -294,8 +296,9 @@ def attention_extend_paged(
         if drows is not None:
             assert maps == 1, "single rows of a two-map cache: no flash-decode"
             dq = q[drows].contiguous()
-            dtab = block_tables[dseqs].contiguous()
-            dlens = kv_lens[dseqs].contiguous()
+            dtab, dlens, plan = _single_rows(
+                block_tables, kv_lens, dseqs, k_cache.shape[1], window, kv_fp8,
+                sink_w is None and slopes is None, C, step_cache)
             if sink_w is not None or slopes is not None:
                 each = torch.arange(dq.shape[0] + 1, dtype=torch.int32,
                                     device=q.device)
@@ -306,7 +309,7 @@ def attention_extend_paged(
             else:
                 dout = attention_decode_paged(
                     dq, k_cache, v_cache, dtab, dlens, scale, window=window,
-                    sink=bool(sink), native=C,
+                    sink=bool(sink), native=C, plan=plan,
                 )
             out[drows] = dout
         return out
@@ -316,45 +319,88 @@ def attention_extend_paged(
     )
 
 
-def decode_num_partitions(num_seqs: int, num_kv_heads: int, max_blocks: int) -> int:
-    """Flash-decode split factor: fill the 256 CUs (target ~2 workgroups/CU)
-    when batch x kv_heads alone cannot. Each partition keeps >= 8 pages so
-    all 4 waves of a workgroup get a 2-page chunk and the K-prefetch
-    software pipeline has depth (bench_decode2: starved waves at <8
-    pages/partition cap short-seq shapes)."""
-    base = num_seqs * num_kv_heads
-    target = 512
-    nparts = max(1, -(-target // base))
-    nparts = min(nparts, max(1, max_blocks // 8), 64)
-    return nparts
+def _single_rows(block_tables, kv_lens, dseqs, num_kv_heads: int, window: int,
+                 kv_fp8: bool, planned: bool, native,
+                 step_cache: dict | None):
+    """(block tables, lengths, decode plan) of the single rows of a mixed
+    batch: the same for all layers of a forward pass (step_cache)."""
+    cache = {} if step_cache is None else step_cache
+    if "single_rows" not in cache:
+        cache["single_rows"] = (block_tables[dseqs].contiguous(),
+                                kv_lens[dseqs].contiguous())
+    dtab, dlens = cache["single_rows"]
+    plan = (step_decode_plan(dlens, num_kv_heads, window, kv_fp8, native, cache)
+            if planned else None)
+    return dtab, dlens, plan
+
+
+def step_decode_plan(seq_lens, num_kv_heads: int, window: int, kv_fp8: bool,
+                     native, step_cache: dict | None):
+    """attention_decode_plan, made once per forward pass (step_cache)."""
+    if step_cache is None:
+        return None
+    key = ("decode_plan", num_kv_heads, window, kv_fp8)
+    if key not in step_cache:
+        step_cache[key] = attention_decode_plan(seq_lens, num_kv_heads, window,
+                                                kv_fp8, native=native)
+    return step_cache[key]
+
+
+def decode_waves(num_seqs: int, num_kv_heads: int, kv_fp8: bool = False,
+                 num_partitions: int | None = None) -> int:
+    """Runs per key/value head that the decode kernel cuts all sequences'
+    pages into (attn_decode.hip). One workgroup of 4 waves per CU where a run
+    holds few sequences (64 x 1024: 31.4 us, with two 33.2; 16 x 8000: 55 and
+    64), two where waves often start on a new sequence and wait for its first
+    rows (256 sequences of 1..4000: 86 and 74 us) or where the rows are half
+    as long (48 fp8 ones: 36 and 33). num_partitions: that many runs per
+    sequence on average instead."""
+    if num_partitions is not None:
+        return max(1, num_partitions * num_seqs)
+    waves = 2048 if kv_fp8 or num_seqs > 64 else 1024
+    return max(1, waves // num_kv_heads)
+
+
+def attention_decode_plan(seq_lens, num_kv_heads: int, window: int = 0,
+                          kv_fp8: bool = False,
+                          num_partitions: int | None = None, native=None):
+    """What every wave of attention_decode_paged reads, for layers of this
+    window, number of key/value heads and kind of pages: made once per step
+    and handed to each of them (plan=). None on CPU tensors."""
+    if not seq_lens.is_cuda:
+        return None
+    C = native if native is not None else _native()
+    waves = decode_waves(seq_lens.shape[0], num_kv_heads, kv_fp8,
+                         num_partitions)
+    plan = torch.empty(4 * waves + 2 * seq_lens.shape[0], dtype=torch.int32,
+                       device=seq_lens.device)
+    C.attention_decode_plan(plan, seq_lens, waves, window)
+    return plan
 
 
 def attention_decode_paged(
     q, k_cache, v_cache, block_tables, seq_lens, scale: float,
     num_partitions: int | None = None, part_out=None, window: int = 0,
-    sink: bool = False, native=None,
+    sink: bool = False, native=None, plan=None,
 ):
+    """plan: attention_decode_plan's for these lengths, heads, window and
+    num_partitions (None: made here)."""
     if q.is_cuda:
         C = native if native is not None else _native()
-        out = torch.empty(
-            (q.shape[0], q.shape[1], q.shape[2]), dtype=q.dtype, device=q.device
-        )
-        num_kv_heads = k_cache.shape[1]
-        if num_partitions is None:
-            num_partitions = decode_num_partitions(
-                q.shape[0], num_kv_heads, block_tables.shape[1]
-            )
-        if num_partitions > 1 and part_out is None:
-            gq = q.shape[1] // num_kv_heads
-            part_out = torch.empty(
-                q.shape[0] * num_kv_heads * num_partitions * gq * (q.shape[2] + 2),
-                dtype=torch.float32, device=q.device,
-            )
-        elif part_out is None:
-            part_out = q.new_empty(0, dtype=torch.float32)
+        S, hq, hd = q.shape
+        hkv = k_cache.shape[1]
+        out = torch.empty((S, hq, hd), dtype=q.dtype, device=q.device)
+        kv_fp8 = k_cache.dtype != torch.bfloat16
+        if plan is None:
+            plan = attention_decode_plan(seq_lens, hkv, window, kv_fp8,
+                                         num_partitions, C)
+        waves = decode_waves(S, hkv, kv_fp8, num_partitions)
+        need = (waves + S) * (hq * hd + 16 * hkv)
+        if part_out is None or part_out.numel() < need:
+            part_out = torch.empty(need, dtype=torch.float32, device=q.device)
         C.attention_decode_paged(
             out, q, k_cache, v_cache, block_tables, seq_lens, scale,
-            part_out, num_partitions, window, 1 if sink else 0,
+            part_out, plan, waves, window, 1 if sink else 0,
         )
         return out
     return ref.attention_decode_paged(
@@ -697,7 +743,8 @@ def attention_sink_paged(q, k_cache, v_cache, block_tables, seq_lens,
                          inv_freq_v=None, interleaved=True, max_q_len=0,
                          positions=None, tiles=None, sink_w=None,
                          softcap=0.0, window=0, keep_first=0, out=None,
-                         out_scale=1.0, maps=1, slopes=None):
+                         out_scale=1.0, maps=1, slopes=None,
+                         step_cache: dict | None = None):
     """Causal attention of packed rows over paged keys with an optional
     sink (score 0, or sink_w per head), tanh-capped scores, a distance bias
     (slopes [H]: slope[h] (i - j) off the scores), a sliding
@@ -742,7 +789,8 @@ def attention_sink_paged(q, k_cache, v_cache, block_tables, seq_lens,
             # work list, so it also runs inside a captured decode graph
             out = attention_decode_paged(
                 q, k_cache, v_cache, block_tables, seq_lens, scale,
-                sink=sink, native=_native_seq())
+                sink=sink, native=_native_seq(), plan=step_decode_plan(
+                    seq_lens, G, 0, False, _native_seq(), step_cache))
             if inv_freq_v is not None:
                 _native_seq().unrotate_rows(out, positions, inv_freq_v,
                                             interleaved)
@@ -750,7 +798,8 @@ def attention_sink_paged(q, k_cache, v_cache, block_tables, seq_lens,
         if fast and tiles is not None and D in _MFMA_HEAD_DIMS:
             out = attention_extend_paged(
                 q, k_cache, v_cache, block_tables, seq_lens, cu_seqlens,
-                None, scale, tiles=tiles, sink=sink, native=_native_seq())
+                None, scale, tiles=tiles, sink=sink, native=_native_seq(),
+                step_cache=step_cache)
             if inv_freq_v is not None:
                 _native_seq().unrotate_rows(out, positions, inv_freq_v,
                                             interleaved)

@@ -14,10 +14,13 @@ extern "C" {
 void arks_attn_decode_paged(void* out, void* part_out, const void* q,
                             const void* k_cache, const void* v_cache,
                             const void* block_tables, const void* seq_lens,
-                            float scale, int num_seqs, int num_q_heads,
-                            int num_kv_heads, int head_dim, int max_blocks,
-                            int nparts, int64_t q_stride, int kv_fp8,
-                            int window, int sink, hipStream_t stream);
+                            const void* plan, float scale, int num_seqs,
+                            int num_q_heads, int num_kv_heads, int head_dim,
+                            int max_blocks, int waves, int64_t q_stride,
+                            int kv_fp8, int window, int sink,
+                            hipStream_t stream);
+void arks_attn_decode_plan(void* plan, const void* seq_lens, int num_seqs,
+                           int window, int waves, hipStream_t stream);
 void arks_attn_extend_paged(void* out, const void* q, const void* k_cache,
                             const void* v_cache, const void* block_tables,
                             const void* kv_lens, const void* cu_seqlens_q,
@@ -68,11 +71,31 @@ inline void check_bf16_rowstrided(const torch::Tensor& t, const char* name) {
     TORCH_CHECK(t.stride(1) == t.size(2), name, " inner dims must be dense");
   }
 }
+inline void check_decode_plan(const torch::Tensor& plan, int64_t waves,
+                              int64_t num_seqs) {
+  TORCH_CHECK(waves >= 1 && plan.is_cuda() && plan.is_contiguous() &&
+                  plan.scalar_type() == torch::kInt32 &&
+                  plan.numel() >= 4 * waves + 2 * num_seqs &&
+                  reinterpret_cast<uintptr_t>(plan.data_ptr()) % 16 == 0,
+              "plan must be int32 of 4 * waves + 2 * sequences");
+}
+// The runs of a decode step (attn_decode.hip), shared by all layers of the
+// same window and number of key/value heads.
+inline void attention_decode_plan(torch::Tensor plan, torch::Tensor seq_lens,
+                                  int64_t waves, int64_t window) {
+  TORCH_CHECK(seq_lens.is_cuda() && seq_lens.is_contiguous() &&
+              seq_lens.scalar_type() == torch::kInt32);
+  check_decode_plan(plan, waves, seq_lens.numel());
+  arks_attn_decode_plan(plan.data_ptr(), seq_lens.data_ptr(),
+                        (int)seq_lens.numel(), (int)window, (int)waves,
+                        attn_current_stream());
+}
 inline void attention_decode_paged(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_tables, torch::Tensor seq_lens,
                             double scale, torch::Tensor part_out,
-                            int64_t nparts, int64_t window, int64_t sink) {
+                            torch::Tensor plan, int64_t waves, int64_t window,
+                            int64_t sink) {
   check_bf16_contig(out, "out");
   check_bf16_rowstrided(q, "q");
   const bool kv_fp8 = check_kv_cache(k_cache, "k_cache");
@@ -89,19 +112,17 @@ inline void attention_decode_paged(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(gq >= 1 && gq <= 8 && gq * num_kv_heads == num_q_heads,
               "q/kv head ratio must be integral and <= 8");
   const int max_blocks = block_tables.size(1);
-  if (nparts > 1) {
-    TORCH_CHECK(part_out.scalar_type() == torch::kFloat32 &&
-                part_out.numel() >=
-                    (int64_t)num_seqs * num_kv_heads * nparts * gq *
-                        (head_dim + 2),
-                "part_out workspace too small");
-  }
-  arks_attn_decode_paged(out.data_ptr(),
-                         nparts > 1 ? part_out.data_ptr() : nullptr,
-                         q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+  check_decode_plan(plan, waves, num_seqs);
+  TORCH_CHECK(part_out.scalar_type() == torch::kFloat32 &&
+                  reinterpret_cast<uintptr_t>(part_out.data_ptr()) % 16 == 0 &&
+                  part_out.numel() >= (waves + num_seqs) *
+                                          (int64_t)num_kv_heads *
+                                          (gq * head_dim + 16),
+              "part_out workspace too small");
+  arks_attn_decode_paged(out.data_ptr(), part_out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                          block_tables.data_ptr(), seq_lens.data_ptr(),
-                         (float)scale, num_seqs, num_q_heads, num_kv_heads,
-                         head_dim, max_blocks, (int)nparts, q.stride(0),
+                         plan.data_ptr(), (float)scale, num_seqs, num_q_heads,
+                         num_kv_heads, head_dim, max_blocks, (int)waves, q.stride(0),
                          kv_fp8 ? 1 : 0, (int)window, (int)sink,
                          attn_current_stream());
 }
@@ -213,6 +234,7 @@ inline void attention_extend2_combine(torch::Tensor out, torch::Tensor part_ws,
 }
 
 inline void def_paged_attention(pybind11::module_& m) {
+  m.def("attention_decode_plan", &attention_decode_plan);
   m.def("attention_decode_paged", &attention_decode_paged);
   m.def("attention_extend_paged", &attention_extend_paged);
   using pybind11::arg;

@@ -39,11 +39,10 @@ def main():
             bt = torch.arange(1, total, dtype=torch.int32,
                               device="cuda").reshape(S, nb)
             sl = torch.full((S,), L, dtype=torch.int32, device="cuda")
-            nparts = ops.decode_num_partitions(S, hkv, nb)
             t = bench(lambda: ops.attention_decode_paged(
                 q, kc, vc, bt, sl, hd ** -0.5))
             kv_bytes = S * L * hkv * hd * 2 * 2
-            print(f"S={S:4d} L={L:6d} nparts={nparts:3d}  {t:8.1f}us  "
+            print(f"S={S:4d} L={L:6d} {t:8.1f}us  "
                   f"{kv_bytes / t / 1e6:5.2f} TB/s")
 
 

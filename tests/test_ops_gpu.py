@@ -195,6 +195,68 @@ def test_attention_decode_partitions_agree():
     torch.testing.assert_close(o8.float().cpu(), expect, atol=2e-2, rtol=2e-2)
 
 
+# lengths around a unit (32 tokens), its second page and a piece (32 units);
+# more sequences than a plan thread block; runs over many short sequences;
+# windows that start inside and on the edge of a unit (dropped pages: -1)
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize(
+    "hq,hkv,hd,lens,window,partitions",
+    [
+        (7, 1, 128, [1, 15, 16, 17, 31, 32, 33, 63, 65], 0, None),
+        (8, 2, 64, [1023, 1024, 1025, 2049], 0, None),
+        (2, 1, 64, [1 + (7 * i) % 90 for i in range(1100)], 0, None),
+        (4, 4, 128, [3000, 1, 40], 0, 3),
+        (8, 2, 128, [700, 123, 48, 2000, 31], 100, None),
+        (8, 2, 128, [96, 97, 400], 32, 2),
+    ],
+)
+def test_attention_decode_runs(hq, hkv, hd, lens, window, partitions, fp8):
+    """The runs that the decode kernel cuts the sequences into."""
+    assert_native()
+    torch.manual_seed(len(lens) + window)
+    S, pages = len(lens), [(n + 15) // 16 for n in lens]
+    total = sum(pages)
+    q = torch.randn(S, hq, hd, dtype=torch.bfloat16, device=DEV)
+    kc = torch.randn(total, hkv, 16, hd, device=DEV)
+    vc = torch.randn(total, hkv, 16, hd, device=DEV)
+    dtype = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    kc, vc = kc.to(dtype), vc.to(dtype)
+    bt = torch.zeros(S, max(pages) + 2, dtype=torch.int32)
+    order, at = torch.randperm(total, dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    full = bt.clone()
+    if window:
+        for i, n in enumerate(lens):
+            bt[i, :max(0, n - window) // 16] = -1
+    sl = torch.tensor(lens, dtype=torch.int32)
+    out = ops.attention_decode_paged(q, kc, vc, bt.to(DEV), sl.to(DEV),
+                                     hd ** -0.5, num_partitions=partitions,
+                                     window=window)
+    expect = ref.attention_decode_paged(
+        q.float().cpu(), kc.float().cpu(), vc.float().cpu(), full, sl,
+        hd ** -0.5, window)
+    # weights and result are rounded to bf16 (2^-9 each) under |v| < 6
+    torch.testing.assert_close(out.float().cpu(), expect, atol=2.4e-2, rtol=0)
+
+
+def test_attention_decode_fp8_codes():
+    """Every e4m3 code reads as its own value."""
+    assert_native()
+    codes = torch.arange(256, dtype=torch.uint8, device=DEV)
+    kc = torch.zeros(1, 2, 16, 128, device=DEV).to(torch.float8_e4m3fn)
+    vc = kc.clone()
+    vc[0, :, 0] = codes.view(torch.float8_e4m3fn).view(2, 128)
+    out = ops.attention_decode_paged(
+        torch.zeros(1, 2, 128, dtype=torch.bfloat16, device=DEV), kc, vc,
+        torch.zeros(1, 1, dtype=torch.int32, device=DEV),
+        torch.ones(1, dtype=torch.int32, device=DEV), 1.0)
+    expect = codes.view(torch.float8_e4m3fn).float().view(2, 128)
+    torch.testing.assert_close(out[0].float(), expect, atol=0, rtol=0,
+                               equal_nan=True)
+
+
 @pytest.mark.parametrize("rows,vocab", [(1, 5), (1, 4095), (1, 4096), (3, 20001),
                                         (64, 152064), (600, 4099)])
 def test_greedy_sample_parts(rows, vocab):
