@@ -152,22 +152,6 @@ class MLP(nn.Module):
         return self.down_proj(ops.silu_mul(gate_up))
 
 
-_ARANGE_CACHE: dict[tuple[int, int, str], torch.Tensor] = {}
-
-
-def _arange_interleave(T: int, k: int, device) -> torch.Tensor:
-    """Cached [0,0,..,1,1,..] token-index vector — identical for every MoE
-    layer of a forward, so build it once per (T, k) instead of 48 times."""
-    key = (T, k, str(device))
-    t = _ARANGE_CACHE.get(key)
-    if t is None:
-        if len(_ARANGE_CACHE) > 256:
-            _ARANGE_CACHE.clear()
-        t = torch.arange(T, device=device).repeat_interleave(k)
-        _ARANGE_CACHE[key] = t
-    return t
-
-
 class MoEMLP(nn.Module):
     """Mixtral-style sparse MoE block, expert-parallel over the TP group:
     each rank owns num_local_experts/tp whole experts (an expert's FFN is
@@ -193,17 +177,15 @@ class MoEMLP(nn.Module):
         self.gate = nn.Parameter(
             torch.empty(E, cfg.hidden_size, dtype=dtype), requires_grad=False
         )
-        # fused [gate|up] and down per local expert, stored PRE-TRANSPOSED
-        # ([in, out] per expert) so every MoE GEMM is an NN strided bmm /
-        # mm with contiguous operands: strided bmm with a transposed-VIEW B
-        # memory-faults on this ROCm stack at prefill shapes (contiguous B
-        # passes), and NN needs no per-call transpose copies.
-        self.w13 = nn.Parameter(
-            torch.empty(self.local_experts, self.hidden, 2 * self.inter,
+        # [gate rows | up rows] and down per local expert, in the
+        # checkpoint's own [out, in] layout: the expert kernels read weight
+        # rows along their input
+        self.w_up = nn.Parameter(
+            torch.empty(self.local_experts, 2 * self.inter, self.hidden,
                         dtype=dtype), requires_grad=False,
         )
-        self.w2 = nn.Parameter(
-            torch.empty(self.local_experts, self.inter, self.hidden,
+        self.w_down = nn.Parameter(
+            torch.empty(self.local_experts, self.hidden, self.inter,
                         dtype=dtype), requires_grad=False,
         )
         # Qwen2-MoE shared expert (dense, TP-sharded like a normal MLP) with
@@ -222,139 +204,27 @@ class MoEMLP(nn.Module):
                 requires_grad=False,
             )
 
-    # Below this many tokens the dense path wins: every expert's weights
-    # are streamed from HBM regardless (tokens scatter over all experts),
-    # so decode is weight-bandwidth-bound and the extra MFMA work of
-    # computing all tokens per expert stays at or under the HBM floor up
-    # to ~256 tokens (E*T*3*I*H*2 flops vs E*3*I*H*2 bytes: the crossover
-    # at ~1.5 PF effective and ~6 TB/s is T ~ 250). Data-independent
-    # shapes make every decode batch size hipGraph-capturable.
+    @property
+    def w13(self) -> torch.Tensor:
+        """w_up as the right operand of a product, [expert, in, 2 * inter]."""
+        return self.w_up.transpose(1, 2)
+
+    @property
+    def w2(self) -> torch.Tensor:
+        """w_down as the right operand of a product, [expert, inter, out]."""
+        return self.w_down.transpose(1, 2)
+
+    # rows up to which decode steps are captured as graphs (the expert kernels
+    # need no host read of the routing at any size)
     DENSE_TOKENS = 256
 
     def forward(self, x):
         from ..parallel.comm import tp_all_reduce
 
-        T = x.shape[0]
-        router_logits = torch.nn.functional.linear(x, self.gate).float()
-        # fused softmax+topk+renorm routing kernel (ops.moe_topk) replaces
-        # a 5-kernel torch chain per layer
-        weights, selected = ops.moe_topk(router_logits, self.top_k,
-                                         self.norm_topk)
-        out = torch.zeros_like(x)
-        if T <= self.DENSE_TOKENS:
-            # Batched over experts: two strided-batch GEMMs (bmm) instead of
-            # a per-expert loop — one launch pair regardless of E (Qwen3-MoE
-            # has 128 experts), and every expert's weights stream once. The
-            # weighted mix over experts is one gather kernel (ops.moe_mix).
-            E = self.local_experts
-            xb = x.unsqueeze(0).expand(E, T, self.hidden)
-            gu = torch.bmm(xb, self.w13)  # [E, T, 2I]
-            h = ops.silu_mul(gu.reshape(E * T, 2 * self.inter))
-            y = torch.bmm(h.view(E, T, self.inter), self.w2)  # [E, T, H]
-            out = ops.moe_mix(y, weights, selected, self.expert_base)
-            out = tp_all_reduce(out)
-            if self.shared is not None:
-                gate = torch.sigmoid(
-                    torch.nn.functional.linear(x, self.shared_gate).float()
-                ).to(x.dtype)
-                out = out + gate * self.shared(x)
-            return out
-        # Sparse path (prefill-sized T): sort token-expert pairs once so
-        # each expert sees a contiguous segment (one host sync per layer
-        # for the segment table), run the expert FFNs into ONE flat output
-        # buffer — a capacity-clamped grouped bmm plus large-M overflow
-        # GEMMs for heavily-routed experts — and combine with the
-        # moe_mix_rows gather kernel. No index_add_ scatters anywhere:
-        # torch's indexFuncLargeIndex was 36% of Qwen3-30B prefill GPU
-        # time (profiles/r02_final.md).
-        k = self.top_k
-        flat_sel = selected.reshape(-1).long()
-        flat_tok = _arange_interleave(T, k, x.device)
-        order = torch.argsort(flat_sel, stable=True)
-        tok_sorted = flat_tok[order]
-        counts = torch.bincount(flat_sel, minlength=self.num_experts)
-        offs = torch.cumsum(counts, 0)
-        seg = torch.stack((counts, offs)).cpu()  # ONE host sync per layer
-        counts_h = seg[0].tolist()
-        offs_h = seg[1].tolist()
-        El = self.local_experts
-        base = self.expert_base
-        local_counts_h = counts_h[base:base + El]
-        cap = max(local_counts_h or [0])
-        cap_lim = max(1, (512 * 1024 * 1024) // (El * 2 * self.inter * 2))
-        # clamp the grouped capacity near 2x the mean load: under skewed
-        # routing, padding the whole block to the heaviest expert wastes
-        # multiples of the useful FLOPs, while spilled experts finish in
-        # efficient large-M overflow GEMMs below
-        mean2 = 2 * ((sum(local_counts_h) + El - 1) // El) if El else 0
-        cap_eff = min(cap, cap_lim, max(128, mean2))
-        ovf = [(le, c - cap_eff) for le, c in enumerate(local_counts_h)
-               if c > cap_eff]
-        n_of = sum(o for _, o in ovf)
-        if cap_eff == 0:
-            out = tp_all_reduce(out)  # no pairs routed to this rank
-            if self.shared is not None:
-                gate = torch.sigmoid(
-                    torch.nn.functional.linear(x, self.shared_gate).float()
-                ).to(x.dtype)
-                out = out + gate * self.shared(x)
-            return out
-
-        y_all = x.new_empty(El * cap_eff + n_of, self.hidden)
-        # grouped part: pad each local expert's segment to cap_eff rows
-        # (two strided-batch GEMMs for the whole block; padding rows index
-        # row 0 and are never gathered)
-        local_counts = counts[base:base + El, None]        # [El, 1]
-        local_starts = (offs[base:base + El] -
-                        counts[base:base + El])[:, None]   # [El, 1]
-        capped = torch.clamp(local_counts, max=cap_eff)
-        ar = torch.arange(cap_eff, device=x.device)[None, :]  # [1, cap]
-        flat = torch.where(ar < capped, local_starts + ar,
-                           torch.zeros_like(ar)).reshape(-1)
-        # single fused gather x[tok_sorted[flat]] — materializing an
-        # intermediate x_g[T*k, H] costs a full extra round trip per layer
-        xp = x[tok_sorted[flat]].view(El, cap_eff, self.hidden)
-        gu = torch.bmm(xp, self.w13)
-        h = ops.silu_mul(gu.reshape(El * cap_eff, 2 * self.inter))
-        torch.bmm(h.view(El, cap_eff, self.inter), self.w2,
-                  out=y_all[:El * cap_eff].view(El, cap_eff, self.hidden))
-        # overflow part: experts past cap_eff finish with plain large-M
-        # GEMMs appended to the same buffer
-        p0 = El * cap_eff
-        of_base_h = []
-        acc = 0
-        for le, o in ovf:
-            of_base_h.append((le, acc))
-            ge = base + le
-            sl = slice(offs_h[ge] - counts_h[ge] + cap_eff, offs_h[ge])
-            h2 = ops.silu_mul(x[tok_sorted[sl]] @ self.w13[le])
-            torch.mm(h2, self.w2[le], out=y_all[p0 + acc:p0 + acc + o])
-            acc += o
-
-        # row map [T, k]: each pair's position in y_all
-        inv = torch.empty_like(order)
-        inv[order] = torch.arange(T * k, device=x.device)
-        inv = inv.view(T, k)
-        sel = selected.long().view(T, k)
-        sel_local = sel - base
-        mine = (sel_local >= 0) & (sel_local < El)
-        seg_start = offs - counts  # [E] global segment starts
-        local_idx = inv - seg_start[sel]
-        in_cap = local_idx < cap_eff
-        sl_safe = sel_local.clamp(0, El - 1)
-        if ovf:
-            of_base_t = torch.zeros(El, dtype=torch.long, device=x.device)
-            of_base_t[torch.tensor([le for le, _ in of_base_h],
-                                   device=x.device)] = torch.tensor(
-                [a for _, a in of_base_h], device=x.device)
-            rows_of = p0 + of_base_t[sl_safe] + (local_idx - cap_eff)
-        else:
-            rows_of = torch.zeros_like(local_idx)
-        rows = torch.where(in_cap, sl_safe * cap_eff + local_idx, rows_of)
-        rows = torch.where(mine, rows, torch.zeros_like(rows))
-        w_masked = torch.where(mine, weights,
-                               torch.zeros_like(weights))
-        out = ops.moe_mix_rows(y_all, w_masked, rows.to(torch.int32))
+        weights, selected = ops.moe_route(x, self.gate, self.top_k,
+                                          self.norm_topk)
+        out = ops.moe_experts(x, self.w_up, self.w_down, weights, selected,
+                              self.expert_base)
         out = tp_all_reduce(out)
         if self.shared is not None:
             gate = torch.sigmoid(
@@ -583,14 +453,13 @@ class LlamaFamilyForCausalLM(nn.Module):
                     which = sub.split(".")[3]
                     le = e - moe.expert_base
                     if 0 <= le < moe.local_experts:
-                        # HF [out, in] -> our pre-transposed [in, out]
                         I = moe.inter
                         if which == "gate_proj":
-                            moe.w13.data[le, :, :I].copy_(w.t().to(moe.w13.dtype))
+                            moe.w_up.data[le, :I].copy_(w.to(moe.w_up.dtype))
                         elif which == "up_proj":
-                            moe.w13.data[le, :, I:].copy_(w.t().to(moe.w13.dtype))
+                            moe.w_up.data[le, I:].copy_(w.to(moe.w_up.dtype))
                         elif which == "down_proj":
-                            moe.w2.data[le].copy_(w.t().to(moe.w2.dtype))
+                            moe.w_down.data[le].copy_(w.to(moe.w_down.dtype))
                 elif sub.startswith("block_sparse_moe.experts."):
                     # Mixtral expert naming: w1=gate, w3=up, w2=down.
                     # EP-sharded: only this rank's experts are kept.
@@ -599,14 +468,13 @@ class LlamaFamilyForCausalLM(nn.Module):
                     which = sub.split(".")[3]
                     le = e - moe.expert_base
                     if 0 <= le < moe.local_experts:
-                        # HF [out, in] -> our pre-transposed [in, out]
                         I = moe.inter
                         if which == "w1":
-                            moe.w13.data[le, :, :I].copy_(w.t().to(moe.w13.dtype))
+                            moe.w_up.data[le, :I].copy_(w.to(moe.w_up.dtype))
                         elif which == "w3":
-                            moe.w13.data[le, :, I:].copy_(w.t().to(moe.w13.dtype))
+                            moe.w_up.data[le, I:].copy_(w.to(moe.w_up.dtype))
                         elif which == "w2":
-                            moe.w2.data[le].copy_(w.t().to(moe.w2.dtype))
+                            moe.w_down.data[le].copy_(w.to(moe.w_down.dtype))
                 # rotary_emb.inv_freq etc. are ignored (recomputed)
 
     @torch.no_grad()

@@ -577,6 +577,56 @@ def moe_topk(router_logits, k: int, renorm: bool):
     return ref.moe_topk(router_logits, k, renorm)
 
 
+# Rows up to which one kernel does the whole routing (a workgroup per row reads
+# the router's weights, 0.5 MB from L2); beyond, a GEMM for all rows is faster.
+MOE_ROUTE_ROWS = 256
+
+
+def _rows_16b(x):
+    """x, or a copy whose rows start on 16 bytes."""
+    if x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
+        return x
+    return x.clone(memory_format=torch.contiguous_format)
+
+
+def moe_route(x, gate, k: int, renorm: bool):
+    """moe_topk of the router product x gate^T (fp32 logits up to
+    MOE_ROUTE_ROWS rows, rounded to x's type beyond)."""
+    if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= MOE_ROUTE_ROWS
+            and x.shape[1] % 64 == 0 and gate.is_contiguous()
+            and gate.data_ptr() % 16 == 0):
+        logits = torch.empty((x.shape[0], gate.shape[0]), dtype=torch.float32,
+                             device=x.device)
+        _native().stream_gemm(logits, _rows_16b(x), gate, None, 1, 16)
+        return moe_topk(logits, k, renorm)
+    import torch.nn.functional as F
+
+    return moe_topk(F.linear(x, gate).float(), k, renorm)
+
+
+def moe_tile(rows: int, top_k: int, experts: int) -> int:
+    """Pairs of one work item (moe_gemm.hip): weights streamed under 16 of them
+    up to 8 pairs per expert on the mean, 128 x 128 tiles beyond. 128 experts
+    of 2048 x 768, 8 per row, us: 7 rows 96 (tiles 134), 128 rows 241 (250),
+    200 rows 268 (252), 512 rows 493 (270)."""
+    return 16 if rows * top_k <= 8 * experts else 128
+
+
+def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0):
+    """sum_j weights[t, j] * expert(ids[t, j])(x[t]) over the silu-GLU experts
+    w13 [El, 2I, H] (gate rows, then up rows), w2 [El, H, I]; experts outside
+    [expert_base, expert_base + El) contribute nothing (another rank's)."""
+    El, H, I = w13.shape[0], w13.shape[2], w2.shape[2]
+    k = ids.shape[1]
+    if (x.is_cuda and x.dtype == torch.bfloat16 and H % 32 == 0
+            and I % 32 == 0 and El <= 1024 and k <= 16):
+        out = torch.empty((x.shape[0], H), dtype=x.dtype, device=x.device)
+        _native().moe_experts(out, _rows_16b(x), w13, w2, weights, ids,
+                              expert_base, moe_tile(x.shape[0], k, El))
+        return out
+    return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
+
+
 def moe_mix(y, weights, ids, expert_base: int = 0):
     """out[t] = sum_i weights[t,i] * y[ids[t,i]-expert_base, t] with
     out-of-slice experts contributing 0 (TP expert parallelism)."""

@@ -30,6 +30,8 @@ SOURCES = [
     os.path.join(CSRC, "skinny_gemm.hip"),
     os.path.join(CSRC, "sampling.hip"),
     os.path.join(CSRC, "moe.hip"),
+    os.path.join(CSRC, "moe_gemm.hip"),
+    os.path.join(CSRC, "stream_gemm.hip"),
     os.path.join(CSRC, "allreduce.hip"),
 ]
 

@@ -71,6 +71,12 @@ inline void check_bf16_rowstrided(const torch::Tensor& t, const char* name) {
     TORCH_CHECK(t.stride(1) == t.size(2), name, " inner dims must be dense");
   }
 }
+// rows of 16-byte loads
+inline void check_rows_16b(const torch::Tensor& t, const char* name) {
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
+                  t.stride(0) % 8 == 0,
+              name, " rows must start on 16 bytes");
+}
 inline void check_decode_plan(const torch::Tensor& plan, int64_t waves,
                               int64_t num_seqs) {
   TORCH_CHECK(waves >= 1 && plan.is_cuda() && plan.is_contiguous() &&

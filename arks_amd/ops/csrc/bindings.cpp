@@ -78,6 +78,18 @@ void arks_moe_mix(void* out, const void* y, const void* weights,
 void arks_moe_mix_rows(void* out, const void* y, const void* weights,
                        const void* rows, int T, int H, int k,
                        hipStream_t stream);
+void arks_stream_gemm(void* out, const void* a, const void* w, const void* bias,
+                      int m, int n, int k, int64_t a_stride, int nf, int wv,
+                      int f32, hipStream_t stream);
+void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
+                   void* n_items, const void* ids, const void* weights,
+                   int pairs, int expert_base, int n_local, int tile,
+                   int max_items, hipStream_t stream);
+void arks_moe_gemm(void* out, const void* a, const void* w, const void* perm,
+                   const void* items, const void* n_items, int64_t a_stride,
+                   int64_t w_expert, int64_t w_stride, int n_out, int k_total,
+                   int top_k, int max_items, int tile, int up,
+                   hipStream_t stream);
 void arks_mfma_probe(void* d, const void* a, const void* b, hipStream_t stream);
 void arks_mfma_probe32(void* d, const void* a, const void* b, hipStream_t stream);
 void arks_tr16_probe(void* out, int stride_bytes, hipStream_t stream);
@@ -495,6 +507,86 @@ void moe_mix_rows(torch::Tensor out, torch::Tensor y,
                     rows.data_ptr(), T, H, k, current_stream());
 }
 
+// weights [T, k] f32 and ids [T, k] of the rows x over the router gate [E, H]
+// out [M, N] (bf16 or fp32) = a [M, K] w [N, K]^T (+ bias [N])
+void stream_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
+                 c10::optional<torch::Tensor> bias, int64_t nf, int64_t wv) {
+  check_bf16_rowstrided(a, "a");
+  check_bf16_contig(w, "w");
+  check_rows_16b(a, "a");
+  check_rows_16b(w, "w");
+  TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && out.is_cuda() &&
+              out.is_contiguous());
+  const bool f32 = out.scalar_type() == torch::kFloat32;
+  TORCH_CHECK(f32 || out.scalar_type() == torch::kBFloat16);
+  const int64_t M = a.size(0), N = w.size(0), K = a.size(1);
+  TORCH_CHECK(w.size(1) == K && out.dim() == 2 && out.size(0) == M &&
+              out.size(1) == N);
+  TORCH_CHECK(K % 64 == 0 && M <= 16 * 65535 && N < (1 << 30), "need K % 64 == 0");
+  TORCH_CHECK((nf == 1 || nf == 2) && (wv == 8 || wv == 16));
+  if (bias.has_value()) {
+    check_bf16_contig(*bias, "bias");
+    TORCH_CHECK(bias->numel() == N);
+  }
+  if (M == 0 || N == 0) return;
+  arks_stream_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(),
+                   bias.has_value() ? bias->data_ptr() : nullptr, (int)M,
+                   (int)N, (int)K, a.stride(0), (int)nf, (int)wv, f32 ? 1 : 0,
+                   current_stream());
+}
+
+// The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
+// beyond this rank's El experts from expert_base on count as zero.
+void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
+                 torch::Tensor w2, torch::Tensor weights, torch::Tensor ids,
+                 int64_t expert_base, int64_t tile) {
+  check_bf16_contig(out, "out");
+  check_bf16_rowstrided(x, "x");
+  check_bf16_contig(w13, "w13");
+  check_bf16_contig(w2, "w2");
+  check_rows_16b(x, "x");
+  check_rows_16b(w13, "w13");
+  check_rows_16b(w2, "w2");
+  const int64_t T = x.size(0), H = x.size(1), El = w13.size(0);
+  const int64_t I = w2.size(2), k = weights.size(1), P = T * k;
+  TORCH_CHECK(x.dim() == 2 && out.size(0) == T && out.size(1) == H);
+  TORCH_CHECK(w13.size(1) == 2 * I && w13.size(2) == H && w2.size(0) == El &&
+                  w2.size(1) == H,
+              "expert weights do not fit");
+  TORCH_CHECK(H % 32 == 0 && I % 32 == 0 && El <= 1024 && k <= 16,
+              "need H % 32 == 0, I % 32 == 0, at most 1024 experts, k <= 16");
+  TORCH_CHECK(weights.scalar_type() == torch::kFloat32 &&
+              weights.is_contiguous() && ids.scalar_type() == torch::kInt32 &&
+              ids.is_contiguous() && ids.size(0) == T && ids.size(1) == k &&
+              weights.size(0) == T);
+  TORCH_CHECK(tile == 16 || tile == 128);
+  if (T == 0) return;
+  const int64_t max_items = std::min(P, El) + P / tile;
+  TORCH_CHECK(max_items <= 65535 || tile == 128, "too many rows for this tile");
+  auto ints = x.options().dtype(torch::kInt32);
+  // [items | perm | rows | count], the items on 16-byte places
+  torch::Tensor plan = torch::empty({4 * max_items + 2 * P + 1}, ints);
+  int* items = plan.data_ptr<int>();
+  int* perm = items + 4 * max_items;
+  int* rows = perm + P;
+  int* n_items = rows + P;
+  torch::Tensor w_pair = torch::empty_like(weights);
+  torch::Tensor h = torch::empty({P, I}, x.options());
+  torch::Tensor y = torch::empty({P, H}, x.options());
+  auto stream = current_stream();
+  arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, ids.data_ptr(),
+                weights.data_ptr(), (int)P, (int)expert_base, (int)El,
+                (int)tile, (int)max_items, stream);
+  arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
+                n_items, x.stride(0), 2 * I * H, H, (int)I, (int)H, (int)k,
+                (int)max_items, (int)tile, 1, stream);
+  arks_moe_gemm(y.data_ptr(), h.data_ptr(), w2.data_ptr(), perm, items, n_items,
+                I, H * I, I, (int)H, (int)I, (int)k, (int)max_items, (int)tile,
+                0, stream);
+  arks_moe_mix_rows(out.data_ptr(), y.data_ptr(), w_pair.data_ptr(), rows,
+                    (int)T, (int)H, (int)k, stream);
+}
+
 void mfma_probe(torch::Tensor d, torch::Tensor a, torch::Tensor b) {
   check_bf16_contig(a, "a");
   check_bf16_contig(b, "b");
@@ -532,6 +624,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_topk", &moe_topk);
   m.def("moe_mix", &moe_mix);
   m.def("moe_mix_rows", &moe_mix_rows);
+  m.def("stream_gemm", &stream_gemm);
+  m.def("moe_experts", &moe_experts);
   m.def("mfma_probe", &mfma_probe);
   m.def("mfma_probe32", &mfma_probe32);
   m.def("tr16_probe", &tr16_probe);

@@ -1,0 +1,408 @@
+// Sparse expert feed-forward (gfx950): the (row, expert) pairs of a step run
+// only the experts that they chose, without a host read of the routing.
+//
+//   moe_plan   pairs sorted by expert, cut into items of one expert and at
+//              most `tile` pairs; every pair's place in the sorted order
+//   moe_stream few pairs per expert: bound by the stream of the chosen
+//              experts' weights. Tiles of 16 weight rows (gate and up rows
+//              side by side), the waves of a workgroup splitting K, no LDS
+//              and no barrier before the final sum over the waves. 7 rows, 8
+//              of 128 experts each (2048 x 768): 90 us for 46 experts' 434 MB
+//              (4.8 TB/s); every expert as a batched product took 210 us.
+//   moe_tile   many pairs per expert: bound by the matrix cores. 128 pairs x
+//              128 weight rows, 64 of K per step through double-buffered LDS.
+//              5012 rows: 670 us (560 TFLOP/s); a padded batched product with
+//              its gathers, activation and overflow products took 1160 us.
+//
+// Both products exist as "up" (rows gathered by pair, silu(gate) * up in fp32
+// before the one rounding) and "down". Weights lie as in checkpoints,
+// [expert, out, in]: a lane reads 16 bytes along K, as the MFMA operands
+// want them. Items past the last one are empty, so grids depend on the shapes
+// alone and a decode step can be captured.
+#include "common.h"
+
+namespace arks {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+constexpr int MOE_MAX_E = 1024;
+
+__device__ __forceinline__ f32x4 moe_mfma(const ushort8& a, const ushort8& b,
+                                          f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+      *reinterpret_cast<const bf16x8*>(&a), *reinterpret_cast<const bf16x8*>(&b),
+      c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float moe_silu_mul(float g, float u) {
+  return g / (1.f + __expf(-g)) * u;
+}
+
+// One workgroup. perm[place] = pair, rows[pair] = place (0 where the expert
+// is another rank's), weights_out[pair] = the pair's weight (0 there),
+// items[i] = {local expert, first place, pairs, 0}, n_items.
+__global__ __launch_bounds__(1024) void moe_plan_kernel(
+    int* __restrict__ perm, int* __restrict__ rows,
+    float* __restrict__ weights_out, int4* __restrict__ items,
+    int* __restrict__ n_items, const int* __restrict__ ids,
+    const float* __restrict__ weights, const int pairs, const int expert_base,
+    const int n_local, const int tile, const int max_items) {
+  __shared__ int count[MOE_MAX_E], start[MOE_MAX_E], first_item[MOE_MAX_E];
+  __shared__ int total_items;
+  const int tid = threadIdx.x;
+  for (int e = tid; e < n_local; e += 1024) count[e] = 0;
+  __syncthreads();
+  constexpr int PB = 8;  // loads in flight per thread
+  for (int p0 = tid; p0 < pairs; p0 += 1024 * PB) {
+    int e[PB];
+#pragma unroll
+    for (int j = 0; j < PB; ++j)
+      e[j] = p0 + j * 1024 < pairs ? ids[p0 + j * 1024] - expert_base : -1;
+#pragma unroll
+    for (int j = 0; j < PB; ++j)
+      if (e[j] >= 0 && e[j] < n_local) atomicAdd(&count[e[j]], 1);
+  }
+  __syncthreads();
+  if (tid < WAVE_SIZE) {  // prefix sums, 64 experts at a time
+    int at = 0, item = 0;
+    for (int e0 = 0; e0 < n_local; e0 += WAVE_SIZE) {
+      const int e = e0 + tid;
+      const int c = e < n_local ? count[e] : 0;
+      const int n = (c + tile - 1) / tile;
+      int sc = c, sn = n;
+#pragma unroll
+      for (int off = 1; off < WAVE_SIZE; off <<= 1) {
+        const int vc = __shfl_up(sc, off, WAVE_SIZE);
+        const int vn = __shfl_up(sn, off, WAVE_SIZE);
+        if (tid >= off) {
+          sc += vc;
+          sn += vn;
+        }
+      }
+      if (e < n_local) {
+        start[e] = at + sc - c;
+        first_item[e] = item + sn - n;
+      }
+      at += __shfl(sc, WAVE_SIZE - 1, WAVE_SIZE);
+      item += __shfl(sn, WAVE_SIZE - 1, WAVE_SIZE);
+    }
+    if (tid == 0) {
+      total_items = item;
+      *n_items = item;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < n_local; e += 1024) {
+    const int c = count[e];
+    for (int i = 0; i * tile < c; ++i)
+      items[first_item[e] + i] =
+          make_int4(e, start[e] + i * tile, min(tile, c - i * tile), 0);
+    count[e] = 0;  // from here on: pairs placed
+  }
+  for (int i = total_items + tid; i < max_items; i += 1024)
+    items[i] = make_int4(0, 0, 0, 0);
+  __syncthreads();
+  for (int p0 = tid; p0 < pairs; p0 += 1024 * PB) {
+    int e[PB];
+    float w[PB];
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+      const int p = min(p0 + j * 1024, pairs - 1);
+      e[j] = ids[p] - expert_base;
+      w[j] = weights[p];
+    }
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+      const int p = p0 + j * 1024;
+      if (p >= pairs) break;
+      const bool mine = e[j] >= 0 && e[j] < n_local;
+      int place = 0;
+      if (mine) {
+        place = start[e[j]] + atomicAdd(&count[e[j]], 1);
+        perm[place] = p;
+      }
+      rows[p] = place;
+      weights_out[p] = mine ? w[j] : 0.f;
+    }
+  }
+}
+
+// Weight rows [n0, n0 + 16 * NF) of one item's expert (UP: 16 gate rows and
+// their 16 up rows) times its up to 16 pairs; a grid of (row tiles, items). Waves take the 64-wide chunks of K in turn, two chunks of loads in
+// flight each, and sum through LDS in a fixed order.
+template <int NF, int WV, bool UP>
+__global__ __launch_bounds__(WV * 64) void moe_stream_kernel(
+    bf16* __restrict__ out,        // [pairs, n_out]
+    const bf16* __restrict__ a,    // UP: [T, K] by pair / k; else [pairs, K]
+    const bf16* __restrict__ w,    // expert e's rows at w + e * w_expert
+    const int* __restrict__ perm, const int4* __restrict__ items,
+    const int64_t a_stride, const int64_t w_expert, const int64_t w_stride,
+    const int n_out, const int k_total, const int top_k) {
+  const int4 item = items[blockIdx.y];
+  const int cnt = item.z;
+  if (cnt == 0) return;
+  __shared__ f32x4 red[WV][NF][WAVE_SIZE];
+  const int lane = threadIdx.x % WAVE_SIZE, lq = lane % 16, la = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int n0 = blockIdx.x * (UP ? 16 : 16 * NF);
+  const int nch = k_total / 64;
+  f32x4 acc[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bf16* wp[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+    wp[f] = w + (int64_t)item.x * w_expert +
+            (int64_t)(UP ? f * n_out + n0 + lq : n0 + f * 16 + lq) * w_stride +
+            8 * la + wave * 64;
+  const int place = item.y + min(lq, cnt - 1);
+  const bf16* ap = a + (int64_t)(UP ? perm[place] / top_k : place) * a_stride +
+                   8 * la + wave * 64;
+  struct Chunk {
+    ushort8 w[NF][2], a[2];
+  };
+  auto load = [&](Chunk& c, int i, int halves) {
+    const int64_t o = (int64_t)i * WV * 64;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (h >= halves) break;
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        c.w[f][h] = *reinterpret_cast<const ushort8*>(wp[f] + o + 32 * h);
+      c.a[h] = *reinterpret_cast<const ushort8*>(ap + o + 32 * h);
+    }
+  };
+  auto mul = [&](Chunk& c, int halves) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (h >= halves) break;
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        acc[f] = moe_mfma(c.w[f][h], c.a[h], acc[f]);
+    }
+  };
+  const int own = (nch - wave + WV - 1) / WV;
+  if (own > 0) {
+    Chunk c0, c1;
+    load(c0, 0, 2);
+    if (own > 1) load(c1, 1, 2);
+    int i = 0;
+    for (; i + 3 < own; i += 2) {
+      mul(c0, 2);
+      load(c0, i + 2, 2);
+      mul(c1, 2);
+      load(c1, i + 3, 2);
+    }
+    const int left = own - i;
+    mul(c0, 2);
+    if (left > 2) load(c0, i + 2, 2);
+    if (left > 1) mul(c1, 2);
+    if (left > 2) mul(c0, 2);
+  }
+  if (k_total % 64 != 0 && wave == nch % WV) {  // half a chunk behind the last
+    Chunk c;
+    load(c, nch / WV, 1);
+    mul(c, 1);
+  }
+#pragma unroll
+  for (int f = 0; f < NF; ++f) red[wave][f][lane] = acc[f];
+  __syncthreads();
+  auto total = [&](int x) {
+    f32x4 s = red[0][x][lane];
+#pragma unroll
+    for (int v = 1; v < WV; ++v) s += red[v][x][lane];
+    return s;
+  };
+  for (int f = wave; f < (UP ? 1 : NF); f += WV) {
+    f32x4 s = total(f);
+    if (UP) {
+      const f32x4 u = total(1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[r] = moe_silu_mul(s[r], u[r]);
+    }
+    if (lq < cnt) {
+      ushort4v o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = float_to_bf16_bits(s[r]);
+      *reinterpret_cast<ushort4v*>(out + (int64_t)(item.y + lq) * n_out + n0 +
+                                   f * 16 + 4 * la) = o;
+    }
+  }
+}
+
+// 128 pairs of one expert x 128 weight rows (UP: 64 gate rows and their 64 up
+// rows). 4 waves of 64 x 64; the next 64 of K travel through registers while
+// the present ones are multiplied out of LDS (rows padded by 16 B: reads and
+// writes without conflicts). Workgroups go round the 8 XCDs in launch order:
+// each XCD takes a contiguous stretch of (item, row tile) so that its L2 holds
+// an item's rows and its expert's weights.
+constexpr int MT_BM = 128, MT_BN = 128, MT_BK = 64, MT_LS = MT_BK + 8;
+
+template <bool UP>
+__global__ __launch_bounds__(256, 2) void moe_tile_kernel(
+    bf16* __restrict__ out, const bf16* __restrict__ a,
+    const bf16* __restrict__ w, const int* __restrict__ perm,
+    const int4* __restrict__ items, const int* __restrict__ n_items,
+    const int64_t a_stride, const int64_t w_expert, const int64_t w_stride,
+    const int n_out, const int k_total, const int top_k, const int row_tiles) {
+  const int total = *n_items * row_tiles;
+  const int per = (total + 7) / 8;
+  const int slot = blockIdx.x / 8;
+  const int job = blockIdx.x % 8 * per + slot;
+  if (slot >= per || job >= total) return;
+  const int4 item = items[job / row_tiles];
+  const int cnt = item.z;
+  const int n0 = job % row_tiles * (UP ? MT_BN / 2 : MT_BN);
+  __shared__ __attribute__((aligned(16))) bf16 a_s[2][MT_BM][MT_LS];
+  __shared__ __attribute__((aligned(16))) bf16 w_s[2][MT_BN][MT_LS];
+  const int tid = threadIdx.x, lane = tid % WAVE_SIZE, lq = lane % 16,
+            la = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
+  const int wm = wave / 2, wn = wave % 2;
+  // staging: thread -> rows tid / 8 + 32 * j, columns (tid % 8) * 8
+  const int sr = tid / 8, sc = tid % 8 * 8;
+  const bf16* ap[4];
+  const bf16* wp[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int place = item.y + min(sr + 32 * j, cnt - 1);
+    ap[j] = a + (int64_t)(UP ? perm[place] / top_k : place) * a_stride + sc;
+    // UP: rows of a wave's half are 32 gate rows, then their 32 up rows
+    const int r = sr + 32 * j;
+    const int n = UP ? min(n0 + r / 64 * 32 + r % 32, n_out - 1) +
+                           (r / 32 % 2) * n_out
+                     : min(n0 + r, n_out - 1);
+    wp[j] = w + (int64_t)item.x * w_expert + (int64_t)n * w_stride + sc;
+  }
+  ushort8 ar[4], wr[4];
+  auto load = [&](int k0) {
+    const bool in = k0 + sc < k_total;  // the last 64 may be half there
+    const int o = in ? k0 : 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      ar[j] = *reinterpret_cast<const ushort8*>(ap[j] + o);
+      wr[j] = *reinterpret_cast<const ushort8*>(wp[j] + o);
+    }
+    if (!in) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ar[j] = wr[j] = ushort8{};
+    }
+  };
+  auto store = [&](int b) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      *reinterpret_cast<ushort8*>(&a_s[b][sr + 32 * j][sc]) = ar[j];
+      *reinterpret_cast<ushort8*>(&w_s[b][sr + 32 * j][sc]) = wr[j];
+    }
+  };
+  f32x4 acc[4][4];  // [weight rows][pairs]
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (k_total + MT_BK - 1) / MT_BK;
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int s = 0; s < steps; ++s) {
+    const int b = s & 1;
+    if (s + 1 < steps) load((s + 1) * MT_BK);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      ushort8 wf[4], af[4];
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+        wf[f] = *reinterpret_cast<const ushort8*>(
+            &w_s[b][wn * 64 + f * 16 + lq][q * 32 + 8 * la]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        af[t] = *reinterpret_cast<const ushort8*>(
+            &a_s[b][wm * 64 + t * 16 + lq][q * 32 + 8 * la]);
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          acc[f][t] = moe_mfma(wf[f], af[t], acc[f][t]);
+    }
+    if (s + 1 < steps) store(b ^ 1);
+    // (the loads of the step behind the next are not issued yet)
+    __syncthreads();
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int m = wm * 64 + t * 16 + lq;
+    if (m >= cnt) continue;
+    bf16* row = out + (int64_t)(item.y + m) * n_out;
+#pragma unroll
+    for (int f = 0; f < (UP ? 2 : 4); ++f) {
+      const int n = n0 + wn * (UP ? 32 : 64) + f * 16 + 4 * la;
+      if (n >= n_out) continue;
+      ushort4v o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[r] = float_to_bf16_bits(
+            UP ? moe_silu_mul(acc[f][t][r], acc[f + 2][t][r]) : acc[f][t][r]);
+      *reinterpret_cast<ushort4v*>(row + n) = o;
+    }
+  }
+}
+
+}  // namespace arks
+
+using namespace arks;
+
+extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
+                              void* items, void* n_items, const void* ids,
+                              const void* weights, int pairs, int expert_base,
+                              int n_local, int tile, int max_items,
+                              hipStream_t stream) {
+  hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, stream,
+                     (int*)perm, (int*)rows, (float*)weights_out, (int4*)items,
+                     (int*)n_items, (const int*)ids, (const float*)weights,
+                     pairs, expert_base, n_local, tile, max_items);
+}
+
+// tile: pairs of an item, 16 (streamed) or 128 (tiles through LDS).
+extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
+                              const void* perm, const void* items,
+                              const void* n_items, int64_t a_stride,
+                              int64_t w_expert, int64_t w_stride, int n_out,
+                              int k_total, int top_k, int max_items, int tile,
+                              int up, hipStream_t stream) {
+#define ARKS_STREAM(NF, WV, UP)                                               \
+  hipLaunchKernelGGL((moe_stream_kernel<NF, WV, UP>),                         \
+                     dim3(n_out / (UP ? 16 : 16 * NF), max_items),            \
+                     dim3(WV * 64), 0, stream, (bf16*)out, (const bf16*)a,    \
+                     (const bf16*)w, (const int*)perm, (const int4*)items,    \
+                     a_stride, w_expert, w_stride, n_out, k_total, top_k)
+  // waves that split K: enough to cover it in a few chunks each
+  if (tile == 16) {
+    if (up) {
+      if (k_total >= 1024) ARKS_STREAM(2, 8, true);
+      else ARKS_STREAM(2, 4, true);
+    } else if (n_out % 32 == 0) {
+      if (k_total >= 4096) ARKS_STREAM(2, 8, false);
+      else ARKS_STREAM(2, 4, false);
+    } else {
+      ARKS_STREAM(1, 4, false);
+    }
+  } else {
+    const int cols = up ? MT_BN / 2 : MT_BN;
+    const int row_tiles = (n_out + cols - 1) / cols;
+    const dim3 grid((max_items * row_tiles + 7) / 8 * 8), block(256);
+    if (up)
+      hipLaunchKernelGGL((moe_tile_kernel<true>), grid, block, 0, stream,
+                         (bf16*)out, (const bf16*)a, (const bf16*)w,
+                         (const int*)perm, (const int4*)items,
+                         (const int*)n_items, a_stride, w_expert, w_stride,
+                         n_out, k_total, top_k, row_tiles);
+    else
+      hipLaunchKernelGGL((moe_tile_kernel<false>), grid, block, 0, stream,
+                         (bf16*)out, (const bf16*)a, (const bf16*)w,
+                         (const int*)perm, (const int4*)items,
+                         (const int*)n_items, a_stride, w_expert, w_stride,
+                         n_out, k_total, top_k, row_tiles);
+  }
+#undef ARKS_STREAM
+}

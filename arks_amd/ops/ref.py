@@ -275,6 +275,19 @@ def moe_topk(router_logits: torch.Tensor, k: int, renorm: bool):
     return weights, selected.to(torch.int32)
 
 
+def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0):
+    """The chosen experts of every row, expert by expert; rows and products in
+    x's type, the weighted sum in fp32."""
+    out = torch.zeros(x.shape, dtype=torch.float32, device=x.device)
+    for e in range(w13.shape[0]):
+        t, j = (ids == e + expert_base).nonzero(as_tuple=True)
+        if t.numel():
+            h = silu_mul(torch.nn.functional.linear(x[t], w13[e]))
+            y = torch.nn.functional.linear(h, w2[e])
+            out.index_add_(0, t, y.float() * weights[t, j].float()[:, None])
+    return out.to(x.dtype)
+
+
 def moe_mix(y: torch.Tensor, weights: torch.Tensor, ids: torch.Tensor,
             expert_base: int = 0) -> torch.Tensor:
     """Weighted mix of per-(local-)expert dense outputs y [El, T, H]."""

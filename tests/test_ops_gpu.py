@@ -668,6 +668,103 @@ def test_moe_mix_matches_einsum():
                                atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("T,E,k,H,I,base,El,tile,skew", [
+    (1, 8, 2, 64, 32, 0, 8, 16, False),       # smallest product sizes
+    (7, 128, 8, 256, 96, 0, 128, 16, False),  # half chunks of K
+    (33, 64, 8, 2048, 768, 16, 16, 16, False),  # another rank's pairs
+    (5, 8, 1, 64, 32, 4, 4, 16, False),
+    (50, 8, 2, 256, 64, 0, 8, 16, True),      # many items of one expert
+    (300, 16, 4, 96, 224, 0, 16, 128, False),  # tiles over the ends of N
+    (500, 8, 2, 256, 64, 0, 8, 128, True),
+    (7, 128, 8, 256, 96, 8, 100, 128, False),
+    (65, 16, 8, 64, 32, 0, 16, None, False),  # either side of the rule
+    (16, 16, 8, 64, 32, 0, 16, None, False),
+    (17, 16, 8, 64, 32, 0, 16, None, False),
+])
+def test_moe_experts(T, E, k, H, I, base, El, tile, skew, monkeypatch):
+    """Routed experts vs fp64: both kernels, local slices, empty experts."""
+    assert_native()
+    torch.manual_seed(T + E)
+    x = torch.randn(T, 2 * H, device=DEV).bfloat16()[:, :H]
+    w13 = (torch.randn(El, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(El, H, I, device=DEV) * I ** -0.5).bfloat16()
+    ids = torch.rand(T, E, device=DEV).topk(k).indices.int()
+    if skew:  # one expert takes every row, its neighbour the second choice
+        ids = torch.arange(k, device=DEV, dtype=torch.int32).expand(T, k).contiguous()
+    w = torch.rand(T, k, device=DEV)
+    if tile:
+        monkeypatch.setattr(ops, "moe_tile", lambda *a: tile)
+    out = ops.moe_experts(x, w13, w2, w, ids, base)
+    expect = torch.zeros(T, H, dtype=torch.float64)
+    xd, wd = x.double().cpu(), w.double().cpu()
+    for e in range(El):
+        t, j = (ids.cpu() == e + base).nonzero(as_tuple=True)
+        gu = xd[t] @ w13[e].double().cpu().t()
+        h = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+        y = h @ w2[e].double().cpu().t()
+        expect.index_add_(0, t, y * wd[t, j][:, None])
+    # three roundings to bf16 (the hidden, an expert's row, the sum), each at
+    # most 2^-8 of its value
+    err = (out.double().cpu() - expect).norm()
+    assert err <= 3 * 2 ** -8 * expect.norm()
+
+
+@pytest.mark.parametrize("T,E,k,H", [(1, 128, 8, 2048), (17, 60, 4, 512),
+                                     (64, 130, 16, 64), (256, 1024, 2, 1088)])
+def test_moe_route(T, E, k, H):
+    """Router product and choice of few rows vs fp64."""
+    assert_native()
+    torch.manual_seed(E)
+    x = torch.randn(T, H, device=DEV).bfloat16()
+    gate = (torch.randn(E, H, device=DEV) * 4 * H ** -0.5).bfloat16()
+    w, ids = ops.moe_route(x, gate, k, True)
+    z = x.double().cpu() @ gate.double().cpu().t()
+    chosen = z.gather(1, ids.long().cpu())
+    # fp32 sums of H products: each within H * 2^-24 of sum |x g|
+    slack = H * 2 ** -24 * (x.double().abs().cpu() @ gate.double().abs().cpu().t()).max()
+    best = z.topk(k).values
+    assert (chosen - best).abs().max() <= 2 * slack
+    assert all(len(set(r)) == k for r in ids.tolist())
+    torch.testing.assert_close(w.double().cpu(), torch.softmax(chosen, -1),
+                               atol=1e-5, rtol=1e-4)
+
+
+def test_moe_topk_ties_and_nan():
+    """Equal logits go to the lower expert; -inf and NaN still give experts
+    of the table."""
+    assert_native()
+    logits = torch.zeros(4, 200, device=DEV)
+    logits[1, 130:] = 1.0
+    logits[2, 3:] = float("-inf")
+    logits[3, :] = float("nan")
+    w, ids = ops.moe_topk(logits, 5, True)
+    assert ids[0].tolist() == [0, 1, 2, 3, 4]
+    assert ids[1].tolist() == [130, 131, 132, 133, 134]
+    assert ids[2].tolist() == [0, 1, 2, 3, 4]
+    assert w[2, 3:].tolist() == [0.0, 0.0]
+    assert sorted(set(ids[3].tolist())) == sorted(ids[3].tolist())
+    assert 0 <= ids.min() and ids.max() < 200 and w[3].isnan().all()
+
+
+@pytest.mark.parametrize("H,k", [(2048, 8), (30, 3), (72, 16)])
+def test_moe_mix_rows_zero_weights(H, k):
+    """Rows of weight 0 count as nothing, whatever they hold."""
+    assert_native()
+    torch.manual_seed(H)
+    T, R = 19, 64
+    y = torch.randn(R, H, dtype=torch.bfloat16, device=DEV)
+    rows = torch.randint(1, R, (T, k), dtype=torch.int32, device=DEV)
+    w = torch.rand(T, k, device=DEV)
+    w[::2, -1] = 0.0
+    rows[::2, -1] = 0
+    expect = ref.moe_mix_rows(y.double().cpu(), w.double().cpu(), rows.cpu())
+    y[0] = float("nan")
+    out = ops.moe_mix_rows(y, w, rows)
+    # one rounding to bf16 after an fp32 sum
+    torch.testing.assert_close(out.double().cpu(), expect.double(),
+                               atol=1e-5, rtol=2 ** -8)
+
+
 def test_one_shot_allreduce_single_device():
     """p2p all-reduce data path on one GPU: world=1 is identity; a
     simulated world=2 (two mailbox sets on one device, flags pre-armed so
