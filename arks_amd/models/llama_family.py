@@ -85,18 +85,24 @@ class Attention(nn.Module):
         # Strided views into the fused QKV buffer — RoPE/cache/attention
         # kernels take row strides, so no .contiguous() copies on the hot path.
         q, k, v = self.qkv_proj.split_qkv(qkv)
-        if self.q_norm is not None:
+        k_cache, v_cache = kv_cache
+        norms = {}
+        if self.q_norm is not None and not (
+                self.use_rope and (not q.is_cuda
+                                   or self.head_dim in ops.HEAD_NORM_DIMS)):
             hd = self.head_dim
             q = self.q_norm(
                 q.contiguous().view(-1, hd)).view(T, self.nq_local * hd)
             k = self.k_norm(
                 k.contiguous().view(-1, hd)).view(T, self.nkv_local * hd)
             v = v.contiguous()  # reshape_and_cache wants one shared kv stride
-        k_cache, v_cache = kv_cache
+        elif self.q_norm is not None:
+            norms = dict(q_norm=self.q_norm.weight, k_norm=self.k_norm.weight,
+                         eps=self.q_norm.eps)
         if self.use_rope:
             q, k = ops.rope_and_cache(
                 batch.positions, q, k, v, k_cache, v_cache,
-                batch.slot_mapping, self._cos_sin, self.head_dim,
+                batch.slot_mapping, self._cos_sin, self.head_dim, **norms,
             )
         else:
             # NoPE layer: cache k/v as-is, q unrotated

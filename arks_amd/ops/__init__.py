@@ -83,17 +83,26 @@ def rope_apply_inplace(positions, q, k, cos_sin, head_dim: int):
     return ref.rope_apply(positions, q, k, cos_sin, head_dim)
 
 
+HEAD_NORM_DIMS = (32, 64, 128, 256)  # head sizes rope_and_cache norms
+
+
 def rope_and_cache(positions, q, k, v, k_cache, v_cache, slot_mapping,
-                   cos_sin, head_dim: int):
+                   cos_sin, head_dim: int, q_norm=None, k_norm=None,
+                   eps: float = 0.0):
     """Fused RoPE + paged-cache write (GPU): rotates q/k in place and
     scatters rotated k + v into the cache in one launch. CPU path runs the
-    two reference steps."""
+    reference steps. q_norm, k_norm [head_dim]: every head of q and k is
+    RMS-normed first (GPU: head_dim in HEAD_NORM_DIMS)."""
     if q.is_cuda:
         _native().rope_and_cache(positions, q, k, v, k_cache, v_cache,
-                                 slot_mapping, cos_sin, head_dim)
+                                 slot_mapping, cos_sin, head_dim, q_norm,
+                                 k_norm, eps)
         return q, k
-    q2, k2 = ref.rope_apply(positions, q, k, cos_sin, head_dim)
     T = q.shape[0]
+    if q_norm is not None:
+        q, k = (ref.rmsnorm(t.reshape(T, -1, head_dim), w, eps).view(T, -1)
+                for t, w in ((q, q_norm), (k, k_norm)))
+    q2, k2 = ref.rope_apply(positions, q, k, cos_sin, head_dim)
     nkv = k.numel() // max(T, 1) // head_dim
     ref.reshape_and_cache(
         k2.reshape(T, nkv, head_dim), v.reshape(T, nkv, head_dim),

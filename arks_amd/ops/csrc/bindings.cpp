@@ -41,7 +41,8 @@ void arks_rope_and_cache(const void* positions, void* q, void* k,
                          const void* slot_mapping, const void* cos_sin,
                          int num_tokens, int head_dim, int num_q_heads,
                          int num_kv_heads, int block_size, int64_t q_stride,
-                         int64_t k_stride, int kv_fp8, hipStream_t stream);
+                         int64_t k_stride, int kv_fp8, const void* q_norm,
+                         const void* k_norm, float eps, hipStream_t stream);
 void arks_attn_prefill_varlen(void* out, const void* q, const void* k,
                               const void* v, const void* cu_seqlens,
                               const void* tile_info, int ntiles, float scale,
@@ -182,9 +183,20 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
 void rope_and_cache(torch::Tensor positions, torch::Tensor q,
                     torch::Tensor k, torch::Tensor v, torch::Tensor k_cache,
                     torch::Tensor v_cache, torch::Tensor slot_mapping,
-                    torch::Tensor cos_sin, int64_t head_dim) {
+                    torch::Tensor cos_sin, int64_t head_dim,
+                    c10::optional<torch::Tensor> q_norm,
+                    c10::optional<torch::Tensor> k_norm, double eps) {
   TORCH_CHECK(positions.scalar_type() == torch::kInt64);
   TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
+  TORCH_CHECK(q_norm.has_value() == k_norm.has_value());
+  if (q_norm.has_value()) {
+    check_bf16_contig(*q_norm, "q_norm");
+    check_bf16_contig(*k_norm, "k_norm");
+    TORCH_CHECK(q_norm->numel() == head_dim && k_norm->numel() == head_dim);
+    TORCH_CHECK(head_dim == 32 || head_dim == 64 || head_dim == 128 ||
+                    head_dim == 256,
+                "head norms need head_dim 32, 64, 128 or 256");
+  }
   TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32 &&
               cos_sin.is_contiguous());
   check_bf16_rowstrided(q, "q");
@@ -201,7 +213,10 @@ void rope_and_cache(torch::Tensor positions, torch::Tensor q,
                       v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                       slot_mapping.data_ptr(), cos_sin.data_ptr(), T,
                       (int)head_dim, nq, nkv, block_size, q.stride(0),
-                      k.stride(0), kv_fp8 ? 1 : 0, current_stream());
+                      k.stride(0), kv_fp8 ? 1 : 0,
+                      q_norm.has_value() ? q_norm->data_ptr() : nullptr,
+                      k_norm.has_value() ? k_norm->data_ptr() : nullptr,
+                      (float)eps, current_stream());
 }
 
 
@@ -605,7 +620,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul", &silu_mul);
   m.def("rope_inplace", &rope_inplace);
   m.def("reshape_and_cache", &reshape_and_cache);
-  m.def("rope_and_cache", &rope_and_cache);
+  m.def("rope_and_cache", &rope_and_cache, pybind11::arg("positions"),
+        pybind11::arg("q"), pybind11::arg("k"), pybind11::arg("v"),
+        pybind11::arg("k_cache"), pybind11::arg("v_cache"),
+        pybind11::arg("slot_mapping"), pybind11::arg("cos_sin"),
+        pybind11::arg("head_dim"), pybind11::arg("q_norm") = pybind11::none(),
+        pybind11::arg("k_norm") = pybind11::none(), pybind11::arg("eps") = 0.0);
   m.def("attention_prefill_varlen", &attention_prefill_varlen);
   m.def("quant_fp8_rows", &quant_fp8_rows);
   m.def("rmsnorm_fp8", &rmsnorm_fp8);

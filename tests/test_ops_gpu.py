@@ -845,3 +845,37 @@ def test_rope_and_cache_fused_matches_two_step(fp8):
     torch.testing.assert_close(k, k2, atol=2e-2, rtol=2e-2)
     torch.testing.assert_close(kc_a.float(), kc_b.float(), atol=3e-2, rtol=3e-2)
     torch.testing.assert_close(vc_a.float(), vc_b.float(), atol=3e-2, rtol=3e-2)
+
+
+@pytest.mark.parametrize("hq,hkv,hd,fp8", [(32, 4, 128, False), (3, 1, 64, True),
+                                           (5, 5, 32, False), (2, 1, 256, True)])
+def test_rope_and_cache_head_norms(hq, hkv, hd, fp8):
+    """Head norms inside the rotation vs norm, rotation and cache in fp64."""
+    assert_native()
+    torch.manual_seed(hd)
+    T, bs, nblocks = 9, 16, 4
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    qkv = torch.randn(T, (hq + 2 * hkv) * hd, dtype=torch.bfloat16, device=DEV)
+    q, k, v = qkv.split([hq * hd, hkv * hd, hkv * hd], dim=-1)
+    qn, kn = (1 + torch.randn(2, hd, device=DEV) * 0.2).bfloat16()
+    cos_sin = ref.rope_cos_sin_cache(hd, 64, 10000.0).cuda()
+    pos = torch.randint(0, 64, (T,), dtype=torch.int64, device=DEV)
+    slots = torch.tensor([i * 3 if i != 4 else -1 for i in range(T)], device=DEV)
+    kc = torch.zeros(nblocks, hkv, bs, hd, dtype=dt, device=DEV)
+    vc = torch.zeros_like(kc)
+    qd, kd = (ref.rmsnorm(t.double().cpu().reshape(T, -1, hd), n.double().cpu(),
+                          1e-6).view(T, -1) for t, n in ((q, qn), (k, kn)))
+    qd, kd = ref.rope_apply(pos.cpu(), qd, kd, cos_sin.double().cpu(), hd)
+    ops.rope_and_cache(pos, q, k, v, kc, vc, slots, cos_sin, hd, qn, kn, 1e-6)
+    # one rounding to bf16 of values that the rotation may cancel (|x| < 8)
+    for got, want in ((q, qd), (k, kd)):
+        torch.testing.assert_close(got.double().cpu(), want.double(),
+                                   atol=1e-5, rtol=2 ** -8)
+    for t in range(T):
+        if t == 4:
+            continue
+        s = int(slots[t])
+        # e4m3 has 3 bits behind the point, and 2^-10 below its normal range
+        torch.testing.assert_close(
+            kc[s // bs, :, s % bs].double().cpu(), kd[t].view(hkv, hd).double(),
+            atol=2 ** -10 if fp8 else 1e-5, rtol=2 ** -3.9 if fp8 else 2 ** -8)
