@@ -152,10 +152,12 @@ class MLP(nn.Module):
     fp8 = False
 
     def forward(self, x):
-        gate_up = self.gate_up_proj(x)
         if self.fp8:
-            return self.down_proj(ops.silu_mul_fp8(gate_up))
-        return self.down_proj(ops.silu_mul(gate_up))
+            return self.down_proj(ops.silu_mul_fp8(self.gate_up_proj(x)))
+        if isinstance(x, tuple) or self.gate_up_proj.fp8:
+            return self.down_proj(ops.silu_mul(self.gate_up_proj(x)))
+        return self.down_proj(
+            ops.linear_silu_mul(x, self.gate_up_proj.weight))
 
 
 class MoEMLP(nn.Module):

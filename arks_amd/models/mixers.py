@@ -89,7 +89,7 @@ from ..engine.forward_batch import ForwardBatch
 
 def linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
     """x @ w^T (+ b) as a library GEMM (the decode-shaped bf16 cases go to
-    the split-K kernel when the main extension is built)."""
+    the streamed kernels when the main extension is built)."""
     if x.dtype == torch.bfloat16:
         return ops.linear_bf16(x, w, b)
     return F.linear(x, w, b)
@@ -103,6 +103,9 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     fp32 accumulate, no rounding of the result)."""
     if x.dtype == torch.float32:
         return F.linear(x, w)
+    out = ops.linear_f32_rows(x, w)
+    if out is not None:
+        return out
     if _MM_OUT_DTYPE.get(x.device.type, True):
         try:
             return torch.mm(x, w.t(), out_dtype=torch.float32)

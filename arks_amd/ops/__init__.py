@@ -429,9 +429,6 @@ def _extend_ws(need: int, device):
     return ws
 
 
-_SKINNY_WS: dict = {}
-
-
 def skinny_gemm(x, weight, bias=None):
     """C = x @ weight^T for decode-sized M (<=64) via the split-K streaming
     MFMA kernel. Beats hipBLASLt's ~19 us latency floor on the small
@@ -474,13 +471,7 @@ def skinny_gemm(x, weight, bias=None):
 
 def _skinny_ws(nsplits: int, N: int, M: int, device):
     mrows = ((M + 15) // 16) * 16
-    key = (device.index,)
-    need = nsplits * N * mrows
-    ws = _SKINNY_WS.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(need, dtype=torch.float32, device=device)
-        _SKINNY_WS[key] = ws
-    return ws
+    return torch.empty(nsplits * N * mrows, dtype=torch.float32, device=device)
 
 
 _USE_SKINNY = os.environ.get("ARKS_SKINNY_GEMM", "1") == "1"
@@ -497,9 +488,75 @@ _SKINNY_TALLK_MAX_ELEMS = 80_000_000
 _SKINNY_TALLK_VARIANT = int(os.environ.get("ARKS_SKINNY_TALLK_V", "7"))
 
 
+def _rows_16b(x):
+    """x, or a copy whose rows start on 16 bytes."""
+    if x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
+        return x
+    return x.clone(memory_format=torch.contiguous_format)
+
+
+def _stream_split(M: int, N: int):
+    """(row tiles, groups of 16 weight rows, waves) of a streamed product
+    (stream_gemm.hip). Up to 256 groups of weight rows one per workgroup, so
+    that most CUs have one, and up to 512 two: 3584 x 3584, 8 rows, us: 8.4
+    (two 11.6); 4608 x 3584: 11.9 (13.0). Waves that split K help while few
+    rows of x come with each weight. Beyond, one group of 4 waves for up to 4
+    rows (28672 x 4096, 4 rows: 47.7, two groups of 16 waves 51.7), two for
+    more (16384 x 4096, 8 rows: 30.1, one group 31.4)."""
+    mt = 1 if M <= 16 else 2
+    tiles = -(-N // 16)
+    if tiles <= 256:
+        return mt, 1, 16 if M <= 8 else 4
+    if tiles <= 512 or M > 16:
+        return mt, 2, 16
+    if tiles > 2048:
+        return mt, 2, 8
+    return (mt, 1, 4) if M <= 4 else (mt, 2, 16)
+
+
+def _streams(x, weight, silu: bool = False) -> bool:
+    """Whether x weight^T takes stream_gemm. A workgroup reads all of x's rows
+    beside its 16 or 32 weight rows, so the line lies where that traffic, and
+    the waves' tails, meet what the other path loses: us, here (other), the
+    other being the split kernel up to _SKINNY_MAX_ELEMS and the library
+    beyond. 3584 x 3584: 1 row 7.4 (14.1), 32 rows 12.5 (15.0). 4608 x 3584:
+    16 rows 13.2 (15.5), 32 rows 16.7 (16.2). 544 x 8192, too few workgroups
+    for its K: 8 rows 13.8 (10.4). Library: 18432 x 4096, 16 rows 42.6 (80.1);
+    32000 x 4096, 8 rows 54.5 (67.4), 16 rows 62.0 (62.5); 151936 x 2048, 16
+    rows 134 (206), 32 rows 167 (149); 37888 x 3584, 1 row 52.9 (53.2), 8 rows
+    58.7 (53.1), with the activation 57.8 (59); 3584 x 18944, 1 row 30.3
+    (32.5), 4 rows 33.4 (32.6)."""
+    M, (N, K) = x.shape[0], weight.shape
+    if not (_USE_SKINNY and x.is_cuda and x.dim() == 2 and 1 <= M <= 32
+            and x.dtype == weight.dtype == torch.bfloat16 and K % 32 == 0
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or weight.requires_grad))
+            and native_available()):
+        return False
+    if N * K <= _SKINNY_MAX_ELEMS:
+        return K <= 4096 or N >= 2048
+    if M <= 2 or (silu and M <= 8 and K <= 4096):
+        return True
+    return M <= 16 and (K <= 2048 or (K <= 4096 and N * K <= 1 << 27))
+
+
+def _stream_gemm(x, weight, bias=None, dtype=None, silu: bool = False):
+    M, N = x.shape[0], weight.shape[0] // (2 if silu else 1)
+    out = torch.empty((M, N), dtype=dtype or x.dtype, device=x.device)
+    mt, nf, wv = _stream_split(M, weight.shape[0])
+    if silu:  # a group of gate rows with their up rows
+        nf, wv = 2, 16 if weight.shape[0] <= 8192 else 8
+    _native().stream_gemm(out, _rows_16b(x), weight, bias, mt, nf, wv, silu)
+    return out
+
+
 def linear_bf16(x, weight, bias=None):
-    """Linear dispatch: the skinny split-K kernel for small decode-shaped
-    GEMMs on GPU, hipBLASLt (F.linear) otherwise."""
+    """Linear dispatch: the streamed product for few rows, the skinny split-K
+    kernel for other small decode-shaped GEMMs on GPU, hipBLASLt (F.linear)
+    otherwise."""
+    if x.dim() == 2 and _streams(x, weight):
+        return _stream_gemm(x, weight, bias)
     if (
         _USE_SKINNY
         and x.is_cuda
@@ -519,6 +576,21 @@ def linear_bf16(x, weight, bias=None):
     import torch.nn.functional as F
 
     return F.linear(x, weight, bias)
+
+
+def linear_f32_rows(x, weight):
+    """x weight^T in fp32 (bf16 operands) where the streamed product takes it,
+    else None."""
+    if x.dim() == 2 and _streams(x, weight):
+        return _stream_gemm(x, weight, dtype=torch.float32)
+    return None
+
+
+def linear_silu_mul(x, weight):
+    """silu_mul(x weight^T), weight [2N, K] the gate rows, then the up rows."""
+    if x.dim() == 2 and weight.shape[0] % 2 == 0 and _streams(x, weight, True):
+        return _stream_gemm(x, weight, silu=True)
+    return silu_mul(linear_bf16(x, weight))
 
 
 def rmsnorm_fp8(x, weight, eps: float = 1e-6):
@@ -591,22 +663,15 @@ def moe_topk(router_logits, k: int, renorm: bool):
 MOE_ROUTE_ROWS = 256
 
 
-def _rows_16b(x):
-    """x, or a copy whose rows start on 16 bytes."""
-    if x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
-        return x
-    return x.clone(memory_format=torch.contiguous_format)
-
-
 def moe_route(x, gate, k: int, renorm: bool):
     """moe_topk of the router product x gate^T (fp32 logits up to
     MOE_ROUTE_ROWS rows, rounded to x's type beyond)."""
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= MOE_ROUTE_ROWS
-            and x.shape[1] % 64 == 0 and gate.is_contiguous()
+            and x.shape[1] % 32 == 0 and gate.is_contiguous()
             and gate.data_ptr() % 16 == 0):
         logits = torch.empty((x.shape[0], gate.shape[0]), dtype=torch.float32,
                              device=x.device)
-        _native().stream_gemm(logits, _rows_16b(x), gate, None, 1, 16)
+        _native().stream_gemm(logits, _rows_16b(x), gate, None, 1, 1, 16, False)
         return moe_topk(logits, k, renorm)
     import torch.nn.functional as F
 

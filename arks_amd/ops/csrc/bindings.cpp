@@ -80,8 +80,8 @@ void arks_moe_mix_rows(void* out, const void* y, const void* weights,
                        const void* rows, int T, int H, int k,
                        hipStream_t stream);
 void arks_stream_gemm(void* out, const void* a, const void* w, const void* bias,
-                      int m, int n, int k, int64_t a_stride, int nf, int wv,
-                      int f32, hipStream_t stream);
+                      int m, int n, int k, int64_t a_stride, int mt, int nf,
+                      int wv, int f32, int silu, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, const void* ids, const void* weights,
                    int pairs, int expert_base, int n_local, int tile,
@@ -523,31 +523,39 @@ void moe_mix_rows(torch::Tensor out, torch::Tensor y,
 }
 
 // weights [T, k] f32 and ids [T, k] of the rows x over the router gate [E, H]
-// out [M, N] (bf16 or fp32) = a [M, K] w [N, K]^T (+ bias [N])
+// out [M, N] (bf16 or fp32) = a [M, K] w [N, K]^T (+ bias [N]); silu: w is
+// [2N, K] and out silu of the first N columns times the others
 void stream_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
-                 c10::optional<torch::Tensor> bias, int64_t nf, int64_t wv) {
+                 c10::optional<torch::Tensor> bias, int64_t mt, int64_t nf,
+                 int64_t wv, bool silu) {
   check_bf16_rowstrided(a, "a");
   check_bf16_contig(w, "w");
-  check_rows_16b(a, "a");
-  check_rows_16b(w, "w");
   TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && out.is_cuda() &&
               out.is_contiguous());
+  check_rows_16b(a, "a");
+  check_rows_16b(w, "w");
   const bool f32 = out.scalar_type() == torch::kFloat32;
-  TORCH_CHECK(f32 || out.scalar_type() == torch::kBFloat16);
-  const int64_t M = a.size(0), N = w.size(0), K = a.size(1);
-  TORCH_CHECK(w.size(1) == K && out.dim() == 2 && out.size(0) == M &&
-              out.size(1) == N);
-  TORCH_CHECK(K % 64 == 0 && M <= 16 * 65535 && N < (1 << 30), "need K % 64 == 0");
-  TORCH_CHECK((nf == 1 || nf == 2) && (wv == 8 || wv == 16));
+  TORCH_CHECK((f32 && !silu) || out.scalar_type() == torch::kBFloat16);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0);
+  const int64_t M = a.size(0), K = a.size(1);
+  const int64_t N = silu ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(w.size(1) == K && w.size(0) == (silu ? 2 * N : N) &&
+              out.dim() == 2 && out.size(0) == M && out.size(1) == N);
+  TORCH_CHECK(K % 32 == 0 && M <= 16 * 65535 && N < (1 << 30),
+              "need K % 32 == 0");
+  TORCH_CHECK(mt == 1 || mt == 2);
+  TORCH_CHECK(silu ? nf == 2 && (wv == 8 || wv == 16)
+                   : (nf == 1 && (wv == 4 || wv == 16)) ||
+                         (nf == 2 && (wv == 8 || wv == 16)));
   if (bias.has_value()) {
     check_bf16_contig(*bias, "bias");
-    TORCH_CHECK(bias->numel() == N);
+    TORCH_CHECK(bias->numel() == N && !silu);
   }
   if (M == 0 || N == 0) return;
   arks_stream_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(),
                    bias.has_value() ? bias->data_ptr() : nullptr, (int)M,
-                   (int)N, (int)K, a.stride(0), (int)nf, (int)wv, f32 ? 1 : 0,
-                   current_stream());
+                   (int)N, (int)K, a.stride(0), (int)mt, (int)nf, (int)wv,
+                   f32 ? 1 : 0, silu ? 1 : 0, current_stream());
 }
 
 // The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs

@@ -879,3 +879,67 @@ def test_rope_and_cache_head_norms(hq, hkv, hd, fp8):
         torch.testing.assert_close(
             kc[s // bs, :, s % bs].double().cpu(), kd[t].view(hkv, hd).double(),
             atol=2 ** -10 if fp8 else 1e-5, rtol=2 ** -3.9 if fp8 else 2 ** -8)
+
+
+@pytest.mark.parametrize("M,N,K,bias", [
+    (1, 1, 32, False), (3, 30, 96, True), (16, 64, 64, True), (9, 4608, 3584, True),
+    (17, 3584, 1056, False), (32, 4608, 512, True), (2, 544, 4096, False),
+    (1, 3584, 18944, False), (5, 16400, 4096, False), (4, 16400, 2048, False),
+    (16, 33000, 2048, False),
+])
+def test_stream_gemm(M, N, K, bias):
+    """Few-row product vs fp64: both outputs, half chunks, ends of tiles."""
+    assert_native()
+    torch.manual_seed(N + K)
+    x = torch.randn(M, 2 * K, dtype=torch.bfloat16, device=DEV)[:, :K]
+    w = torch.randn(N, K, dtype=torch.bfloat16, device=DEV)
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV) if bias else None
+    assert ops._streams(x, w)
+    xd, wd = x.double().cpu(), w.double().cpu()
+    expect = xd @ wd.t()
+    # fp32 sums of K products: within K * 2^-24 of sum |x w|
+    slack = K * 2 ** -24 * (xd.abs() @ wd.abs().t())
+    out = ops.linear_f32_rows(x, w)
+    assert ((out.double().cpu() - expect).abs() <= slack).all()
+    if b is not None:
+        expect = expect + b.double().cpu()
+    out = ops.linear_bf16(x, w, b).double().cpu()
+    assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs()).all()
+
+
+@pytest.mark.parametrize("M,I,K", [(1, 18944, 3584), (8, 40, 96), (16, 9216, 1024),
+                                   (31, 100, 64), (7, 4096, 2048)])
+def test_linear_silu_mul(M, I, K):
+    """Gate, up and activation in one product vs fp64."""
+    assert_native()
+    torch.manual_seed(I + K)
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = (torch.randn(2 * I, K, device=DEV) * K ** -0.5).bfloat16()
+    assert ops._streams(x, w, True)
+    out = ops.linear_silu_mul(x, w).double().cpu()
+    xd, wd = x.double().cpu(), w.double().cpu()
+    gu = xd @ wd.t()
+    g, u = gu[:, :I], gu[:, I:]
+    # |d silu| <= 1.1 |d g|; each sum within K * 2^-24 of sum |x w|, the
+    # exponential within 2^-20; one rounding to bf16
+    s = K * 2 ** -24 * (xd.abs() @ wd.abs().t())
+    expect = torch.nn.functional.silu(g) * u
+    slack = 1.1 * s[:, :I] * u.abs() + g.abs() * s[:, I:] + 2 ** -19 * expect.abs()
+    assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
+
+
+def test_streams_refuses():
+    """What the streamed product leaves to the other paths."""
+    assert_native()
+    x = torch.randn(4, 64, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(64, 64, dtype=torch.bfloat16, device=DEV)
+    assert ops._streams(x, w)
+    assert not ops._streams(x.float(), w)
+    assert not ops._streams(x[:, :40], w[:, :40].contiguous())  # K % 32
+    assert not ops._streams(x, w.t())
+    assert not ops._streams(x.expand(9, 4, 64).reshape(36, 64), w)
+    assert not ops._streams(x, torch.empty(65 * 64, dtype=x.dtype, device=DEV)[1:4097].view(64, 64))
+    buf = torch.randn(4, 70, dtype=torch.bfloat16, device=DEV)
+    odd = buf[:, 3:67]  # rows off 16 bytes are copied
+    torch.testing.assert_close(ops.linear_bf16(odd, w), torch.nn.functional.linear(odd, w),
+                               atol=5e-2, rtol=5e-2)
