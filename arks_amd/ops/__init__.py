@@ -151,6 +151,7 @@ E2_KVBLK = 64        # keys per LDS tile in the ladder kernel
 # kernel; shorter ones (decode-adjacent chunks, prefix-cache hits) stay on
 # the 64-row kernel where a mostly-empty 256-row tile would waste waves.
 EXTEND2_MIN_QLEN = 97
+EXTEND2_SHORT_KEYS = 256  # shorter portions with this many keys go there too
 
 
 def build_extend_tiles(q_lens: list[int], kv_lens: list[int] | None,
@@ -175,11 +176,23 @@ def build_extend_tiles(q_lens: list[int], kv_lens: list[int] | None,
     all layers."""
     t64, t256, dec = [], [], []
     kvl = kv_lens if kv_lens is not None else q_lens
+    # Few short portions behind a context leave the 64-row kernel a few
+    # workgroups that walk all keys alone; the 256-row kernel splits them.
+    # 28/4 heads, us, 64-row and split: 65 rows at 256 keys 18.4 and 17.0, at
+    # 512 keys 33 and 20, at 6113 keys 414 and 48; 4 x 33 rows at 1024 keys 76
+    # and 39, 8 x 33 rows 77 and 71, 16 x 33 rows (more than one workgroup per
+    # CU) 83 and 107.
+    short = [i for i, n in enumerate(q_lens)
+             if n < min_ladder and not (n == 1 and flash_decode)]
+    few = (ladder and not kv_fp8
+           and sum(-(-q_lens[i] // PREFILL_QTILE) for i in short) * num_q_heads
+           <= 256)
+    deep = {i for i in short if few and kvl[i] >= EXTEND2_SHORT_KEYS}
     for i, n in enumerate(q_lens):
         off = kvl[i] - n
         if n == 1 and flash_decode:
             dec.append(i)
-        elif kv_fp8 or n < min_ladder or not ladder:
+        elif kv_fp8 or (n < min_ladder and i not in deep) or not ladder:
             for q0 in range(0, n, PREFILL_QTILE):
                 t64.append((i, q0, min(kvl[i], off + q0 + PREFILL_QTILE)))
         else:
@@ -264,9 +277,9 @@ def attention_extend_paged(
     forward pass, which shares what they would each derive from the lengths
     and tables of the single rows.
 
-    Dispatch: big chunks run the 8-wave 32x32-MFMA ladder kernel
-    (attn_extend2.hip, 256-row q tiles); small chunks and fp8-KV runs use
-    the 4-wave 64-row kernel."""
+    Dispatch: big chunks, and a few small ones behind a context, run the
+    8-wave 32x32-MFMA ladder kernel (attn_extend2.hip, 256-row q tiles); other
+    small chunks and fp8-KV runs use the 4-wave 64-row kernel."""
     if q.is_cuda:
         C = native if native is not None else _native()
         sink = 1 if sink else 0

@@ -27,6 +27,10 @@
 // sequences of a few rows beside long ones, so a wave skips the tiles none of
 // its rows can see.
 //
+// SKIP: waves without rows only help to stage: 65 rows over 6113 keys in 8
+// parts 48 us, with their masked scores worked out 75. Launches without split
+// tiles go without that branch (whole prompts are mostly full tiles).
+//
 // This is the prefix-caching / chunked-prefill attention of the runtime
 // slot (the reference delegates it to vLLM/SGLang images
 // at arksapplication_controller.go:941-1002).
@@ -64,7 +68,7 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
 // conflicted) while the tr16 read pairs overlap by only 8 of 64 banks.
 constexpr int VBLK_ELEMS = 80;
 
-template <int HEAD_DIM, bool BIASED>
+template <int HEAD_DIM, bool BIASED, bool SKIP>
 __global__ __launch_bounds__(512) void attn_extend2_kernel(
     bf16* __restrict__ out,            // [Tq, Hq, D]
     const bf16* __restrict__ q,        // [Tq, Hq, D] (packed new tokens)
@@ -247,6 +251,7 @@ __global__ __launch_bounds__(512) void attn_extend2_kernel(
   }
   __syncthreads();
 
+  const bool has_rows = __builtin_amdgcn_readfirstlane(q0 + wave * 32) < q_len;
   int buf = 0;
   for (int j = j0; j < ntiles; ++j, buf ^= 1) {
     const int key_base = j * E2_KVBLK;
@@ -256,9 +261,10 @@ __global__ __launch_bounds__(512) void attn_extend2_kernel(
 
     const int wrow0 = q0 + wave * 32;  // this wave's first row
     const bool busy =
-        !BIASED || (wrow0 < q_len && key_base <= kv_off + wrow0 + 31 &&
-                    (window <= 0 ||
-                     key_base + E2_KVBLK > kv_off + wrow0 - window + 1));
+        (!SKIP || has_rows) &&
+        (!BIASED || (key_base <= kv_off + wrow0 + 31 &&
+                     (window <= 0 ||
+                      key_base + E2_KVBLK > kv_off + wrow0 - window + 1)));
     if (busy) {
       // ---- QK^T (swapped): A = K rows (32 keys), B = Q. C[key][qrow=col].
       // The two subtiles interleave so consecutive MFMAs hit independent
@@ -439,6 +445,7 @@ __global__ __launch_bounds__(512) void attn_extend2_kernel(
 #pragma unroll
     for (int r16 = 0; r16 < 16; ++r16) {
       const int row = 8 * (r16 >> 2) + 4 * half + (r16 & 3);
+      if (q0 + wave * 32 + row >= q_len) continue;
       float* wr = slab + (int64_t)(wave * 32 + row) * (HEAD_DIM + 2) + col;
 #pragma unroll
       for (int n = 0; n < DTILES; ++n) wr[32 * n] = oacc[n][r16];
@@ -467,18 +474,20 @@ __global__ __launch_bounds__(512) void attn_extend2_kernel(
   }
 }
 
-// Merge the flash partials of split tiles: grid (Hq, n_split, row-groups
-// of 8) — the row-group axis exists purely for parallelism (a single
-// (head, tile) block is latency-bound on the strided part reads);
-// combine_table rows = (first_y, nparts, seq, q0). Standard flash merge
+// Merge the flash partials of split tiles: grid (Hq, n_split, groups of 8
+// rows); combine_table rows = (first_y, nparts, seq, q0). Standard flash merge
 // in f32: m* = max m_p; out = sum_p exp(m_p - m*) O_p / sum_p
-// exp(m_p - m*) l_p (m is base-2: exp2).
+// exp(m_p - m*) l_p (m is base-2: exp2). Reading the slabs bounds it, so the
+// loads of up to 8 parts are in flight together, two dims a thread: 8 tiles of
+// 3 parts, 28 heads (90 MB) 31 us, one part and dim after the other 37.
 template <int HEAD_DIM>
 __global__ __launch_bounds__(256) void attn_extend2_combine_kernel(
     bf16* __restrict__ out, const float* __restrict__ part_ws,
     const int* __restrict__ combine_table,
     const int* __restrict__ cu_seqlens_q, const float scale,
     const int num_q_heads) {
+  constexpr int TPR = HEAD_DIM / 2;  // threads of a row
+  constexpr int PARTS = 8;           // loaded together
   const int h = blockIdx.x;
   const int ci = blockIdx.y;
   const int first_y = combine_table[ci * 4];
@@ -491,29 +500,43 @@ __global__ __launch_bounds__(256) void attn_extend2_combine_kernel(
   const int64_t slab_stride = (int64_t)num_q_heads * E2_QTILE * (HEAD_DIM + 2);
   const float* base = part_ws + (int64_t)first_y * slab_stride +
                       (int64_t)h * E2_QTILE * (HEAD_DIM + 2);
-  // this block's 8-row group; 256 threads = 256/HEAD_DIM rows per pass
+  const int d = threadIdx.x % TPR * 2;
   const int row0 = blockIdx.z * 8;
-  for (int row = row0 + threadIdx.x / HEAD_DIM; row < row0 + 8;
-       row += 256 / HEAD_DIM) {
+  for (int row = row0 + threadIdx.x / TPR; row < row0 + 8; row += 256 / TPR) {
     const int qrow = q0 + row;
     if (qrow >= q_len) continue;
-    const int d = threadIdx.x % HEAD_DIM;
     const float* r0 = base + (int64_t)row * (HEAD_DIM + 2);
-    float m_star = -1e30f;
-    for (int p = 0; p < nparts; ++p)
-      m_star = fmaxf(m_star, r0[p * slab_stride + HEAD_DIM]);
-    float l_tot = 0.f;
-    float acc = 0.f;
-    for (int p = 0; p < nparts; ++p) {
-      const float mp = r0[p * slab_stride + HEAD_DIM];
-      const float lp = r0[p * slab_stride + HEAD_DIM + 1];
-      const float a = __builtin_amdgcn_exp2f((mp - m_star) * scale2);
-      l_tot += a * lp;
-      acc += a * r0[p * slab_stride + d];
+    float m_star = -1e30f, l_tot = 0.f, acc0 = 0.f, acc1 = 0.f;
+    for (int p0 = 0; p0 < nparts; p0 += PARTS) {
+      float2 ml[PARTS], v[PARTS];
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) {
+        const float* r = r0 + (int64_t)min(p0 + p, nparts - 1) * slab_stride;
+        ml[p] = *reinterpret_cast<const float2*>(r + HEAD_DIM);
+        v[p] = *reinterpret_cast<const float2*>(r + d);
+      }
+      float m_new = m_star;
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) m_new = fmaxf(m_new, ml[p].x);
+      const float keep = __builtin_amdgcn_exp2f((m_star - m_new) * scale2);
+      l_tot *= keep;
+      acc0 *= keep;
+      acc1 *= keep;
+      m_star = m_new;
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) {
+        const float e = __builtin_amdgcn_exp2f((ml[p].x - m_star) * scale2);
+        const float a = p0 + p < nparts ? e : 0.f;
+        l_tot += a * ml[p].y;
+        acc0 += a * v[p].x;
+        acc1 += a * v[p].y;
+      }
     }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    out[((int64_t)(q_start + qrow) * num_q_heads + h) * HEAD_DIM + d] =
-        float_to_bf16_bits(acc * inv);
+    const uint32_t two = (uint32_t)float_to_bf16_bits(acc0 * inv) |
+                         ((uint32_t)float_to_bf16_bits(acc1 * inv) << 16);
+    *reinterpret_cast<uint32_t*>(
+        out + ((int64_t)(q_start + qrow) * num_q_heads + h) * HEAD_DIM + d) = two;
   }
 }
 
@@ -529,7 +552,7 @@ extern "C" void arks_attn_extend_paged2(
     int64_t q_stride, int window, int sink, int maps, const void* sink_w,
     const void* slopes, hipStream_t stream) {
   dim3 grid(num_q_heads, ntiles), block(512);
-  static bool attr_set[4] = {false, false, false, false};
+  static bool attr_set[6] = {};
   auto launch = [&](auto kern, int lds_bytes, int idx) {
     if (!attr_set[idx]) {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -548,12 +571,14 @@ extern "C" void arks_attn_extend_paged2(
   };
   if (head_dim == 128) {
     constexpr int LDS = (2 * 64 * 128 + 2 * 16 * 8 * VBLK_ELEMS) * 2;
-    if (sink_w || slopes) launch(attn_extend2_kernel<128, true>, LDS, 2);
-    else launch(attn_extend2_kernel<128, false>, LDS, 0);
+    if (sink_w || slopes) launch(attn_extend2_kernel<128, true, true>, LDS, 2);
+    else if (part_ws) launch(attn_extend2_kernel<128, false, true>, LDS, 4);
+    else launch(attn_extend2_kernel<128, false, false>, LDS, 0);
   } else if (head_dim == 64) {
     constexpr int LDS = (2 * 64 * 64 + 2 * 16 * 4 * VBLK_ELEMS) * 2;
-    if (sink_w || slopes) launch(attn_extend2_kernel<64, true>, LDS, 3);
-    else launch(attn_extend2_kernel<64, false>, LDS, 1);
+    if (sink_w || slopes) launch(attn_extend2_kernel<64, true, true>, LDS, 3);
+    else if (part_ws) launch(attn_extend2_kernel<64, false, true>, LDS, 5);
+    else launch(attn_extend2_kernel<64, false, false>, LDS, 1);
   }
 }
 

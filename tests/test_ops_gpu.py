@@ -943,3 +943,41 @@ def test_streams_refuses():
     odd = buf[:, 3:67]  # rows off 16 bytes are copied
     torch.testing.assert_close(ops.linear_bf16(odd, w), torch.nn.functional.linear(odd, w),
                                atol=5e-2, rtol=5e-2)
+
+
+@pytest.mark.parametrize("hd,hq,hkv,window", [(128, 7, 1, 0), (64, 8, 4, 0),
+                                              (128, 4, 2, 300)])
+def test_extend_short_portions(hd, hq, hkv, window):
+    """Few short portions behind a context: split over keys, beside a long
+    portion and single rows, vs the oracle."""
+    assert_native()
+    torch.manual_seed(hd + hq)
+    qlens, kvs = [2, 65, 1, 33, 96, 130], [256, 1501, 700, 33, 4000, 130]
+    pages = [-(-n // 16) for n in kvs]
+    kc = torch.randn(sum(pages) + 1, hkv, 16, hd, device=DEV).bfloat16()
+    vc = torch.randn_like(kc)
+    bt = torch.zeros(len(kvs), max(pages), dtype=torch.int32, device=DEV)
+    order, at = torch.randperm(sum(pages)).int() + 1, 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    q = torch.randn(sum(qlens), hq, hd, device=DEV).bfloat16()
+    lens = torch.tensor(kvs, dtype=torch.int32, device=DEV)
+    cu = torch.tensor([0] + qlens, device=DEV).cumsum(0).int()
+    tiles = ops.build_extend_tiles(qlens, kvs, False, q.device, num_q_heads=hq)
+    assert {r[0] for r in tiles[0].tolist()} == {3}  # the one without context
+    assert {r[0] for r in tiles[1].tolist()} == {0, 1, 4, 5}
+    assert tiles[4] > 0
+    out = ops.attention_extend_paged(q, kc, vc, bt, lens, cu, qlens, hd ** -0.5,
+                                     window=window, tiles=tiles)
+    expect = ref.attention_extend_paged(
+        q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt.cpu(),
+        lens.cpu(), cu.cpu(), hd ** -0.5, window)
+    # the weights and the sum are each rounded to bf16 once: 2^-8 of sum p |v|
+    bound = 2 ** -7 * vc.abs().max().item()
+    assert (out.float().cpu() - expect.float()).abs().max() <= bound
+    # many short portions keep the 64-row kernel
+    many = ops.build_extend_tiles([33] * 16, [3000] * 16, False, q.device,
+                                  num_q_heads=28)
+    assert many[1].numel() == 0 and many[0].shape[0] == 16
+    assert ops.build_extend_tiles([33], [3000], True, q.device)[1].numel() == 0
