@@ -38,6 +38,7 @@ class RMSNorm(nn.Module):
 
     def forward(self, x, residual=None):
         if self.fp8_out:
+            x = ops.parts_sum(x)
             if residual is None:
                 return ops.rmsnorm_fp8(x, self.weight, self.eps)
             q, s, res = ops.fused_add_rmsnorm_fp8(x, residual, self.weight, self.eps)
@@ -81,7 +82,26 @@ class Attention(nn.Module):
 
     def forward(self, x, batch: ForwardBatch, kv_cache) -> torch.Tensor:
         T = (x[0] if isinstance(x, tuple) else x).shape[0]
-        qkv = self.qkv_proj(x)
+        # in decode steps k and v are read from the cache alone, and the
+        # norms behind the two row-parallel products can add split sums
+        decode = not batch.is_prefill
+        if (decode and self.use_rope and not isinstance(x, tuple)
+                and not self.qkv_proj.fp8
+                and (self.q_norm is None
+                     or self.head_dim in ops.HEAD_NORM_DIMS)
+                and self.head_dim % 8 == 0):
+            qkv = ops.linear_parts(x, self.qkv_proj.weight, self.qkv_proj.bias)
+        else:
+            qkv = self.qkv_proj(x)
+        if isinstance(qkv, ops.Parts):
+            norms = {} if self.q_norm is None else dict(
+                q_norm=self.q_norm.weight, k_norm=self.k_norm.weight,
+                eps=self.q_norm.eps)
+            q = ops.rope_and_cache_parts(
+                batch.positions, qkv, kv_cache[0], kv_cache[1],
+                batch.slot_mapping, self._cos_sin, self.head_dim, **norms)
+            return self.o_proj(self._decode(q, batch, kv_cache).view(T, -1),
+                               parts=True)
         # Strided views into the fused QKV buffer — RoPE/cache/attention
         # kernels take row strides, so no .contiguous() copies on the hot path.
         q, k, v = self.qkv_proj.split_qkv(qkv)
@@ -130,13 +150,18 @@ class Attention(nn.Module):
                     window=self.window,
                 )
         else:
-            out = ops.attention_decode_paged(
-                q, k_cache, v_cache, batch.block_tables, batch.seq_lens,
-                self.scale, window=self.window, plan=ops.step_decode_plan(
-                    batch.seq_lens, self.nkv_local, self.window,
-                    k_cache.dtype != torch.bfloat16, None, batch.step_cache),
-            )
-        return self.o_proj(out.view(T, -1))
+            out = self._decode(q, batch, kv_cache)
+        return self.o_proj(out.view(T, -1), parts=decode)
+
+    def _decode(self, q, batch: ForwardBatch, kv_cache):
+        k_cache, v_cache = kv_cache
+        return ops.attention_decode_paged(
+            q.view(q.shape[0], self.nq_local, self.head_dim), k_cache, v_cache,
+            batch.block_tables, batch.seq_lens,
+            self.scale, window=self.window, plan=ops.step_decode_plan(
+                batch.seq_lens, self.nkv_local, self.window,
+                k_cache.dtype != torch.bfloat16, None, batch.step_cache),
+        )
 
 
 class MLP(nn.Module):
@@ -151,13 +176,14 @@ class MLP(nn.Module):
 
     fp8 = False
 
-    def forward(self, x):
+    def forward(self, x, parts: bool = False):
         if self.fp8:
             return self.down_proj(ops.silu_mul_fp8(self.gate_up_proj(x)))
         if isinstance(x, tuple) or self.gate_up_proj.fp8:
-            return self.down_proj(ops.silu_mul(self.gate_up_proj(x)))
-        return self.down_proj(
-            ops.linear_silu_mul(x, self.gate_up_proj.weight))
+            h = ops.silu_mul(self.gate_up_proj(x))
+        else:
+            h = ops.linear_silu_mul(x, self.gate_up_proj.weight)
+        return self.down_proj(h, parts=parts)
 
 
 class MoEMLP(nn.Module):
@@ -226,7 +252,7 @@ class MoEMLP(nn.Module):
     # need no host read of the routing at any size)
     DENSE_TOKENS = 256
 
-    def forward(self, x):
+    def forward(self, x, parts: bool = False):
         from ..parallel.comm import tp_all_reduce
 
         weights, selected = ops.moe_route(x, self.gate, self.top_k,
@@ -261,7 +287,7 @@ class DecoderLayer(nn.Module):
             x, residual = self.input_layernorm(x, residual)
         x = self.self_attn(x, batch, kv_cache)
         x, residual = self.post_attention_layernorm(x, residual)
-        x = self.mlp(x)
+        x = self.mlp(x, parts=not batch.is_prefill)
         return x, residual
 
 

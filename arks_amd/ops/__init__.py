@@ -58,6 +58,11 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.T
 
 def fused_add_rmsnorm(x, residual, weight, eps: float = 1e-6):
     """In-place on GPU: residual += x (written to residual), out = norm(residual)."""
+    if isinstance(x, Parts):
+        assert x.bias is None
+        out = torch.empty_like(residual)
+        _native().fused_add_rmsnorm_parts(out, x.sums, residual, weight, eps)
+        return out, residual
     if x.is_cuda:
         out = torch.empty_like(x)
         _native().fused_add_rmsnorm(out, x, residual, weight, eps)
@@ -109,6 +114,20 @@ def rope_and_cache(positions, q, k, v, k_cache, v_cache, slot_mapping,
         k_cache, v_cache, slot_mapping,
     )
     return q2, k2
+
+
+def rope_and_cache_parts(positions, qkv, k_cache, v_cache, slot_mapping,
+                         cos_sin, head_dim: int, q_norm=None, k_norm=None,
+                         eps: float = 0.0):
+    """rope_and_cache of a projection [q | k | v] that is still Parts: returns
+    q, and writes k and v to the cache alone."""
+    _, T, width = qkv.sums.shape
+    q = torch.empty((T, width - 2 * k_cache.shape[1] * head_dim),
+                    dtype=torch.bfloat16, device=qkv.sums.device)
+    _native().rope_and_cache_parts(positions, q, qkv.sums, qkv.bias, k_cache,
+                                   v_cache, slot_mapping, cos_sin, head_dim,
+                                   q_norm, k_norm, eps)
+    return q
 
 
 def reshape_and_cache(k, v, k_cache, v_cache, slot_mapping):
@@ -443,62 +462,19 @@ def _extend_ws(need: int, device):
 
 
 def skinny_gemm(x, weight, bias=None):
-    """C = x @ weight^T for decode-sized M (<=64) via the split-K streaming
-    MFMA kernel. Beats hipBLASLt's ~19 us latency floor on the small
-    qkv/o_proj shapes and its ~46 us in-graph down-proj algo (bench_skinny /
-    bench_down logs, r2); the dispatcher keeps the wide streaming shapes
-    (gate_up, lm_head: N >> K) on the tuned library algos. Deterministic
-    split-K (fixed-order combine, no atomics)."""
+    """x weight^T (+ bias) for decode-sized M (<= 64) with K split over
+    workgroups where it can be (stream_gemm.hip; fixed order of the sums, no
+    atomics)."""
     M, K = x.shape
-    N = weight.shape[0]
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    ntiles = N // 64
-    if K > N and ntiles < 128 and M > 48:
-        # tall-K (down-proj shape): few N tiles, parallelism comes from
-        # K-splits; the deeper-staged AB=3 variant at nsplits ~= 448/ntiles
-        # measured fastest (34.6 us vs hipBLASLt's 46.4 in-graph, r2).
-        # M-gated: the variant kernel is fixed at MT=4 (full 64-row cost)
-        # while hipBLASLt switches to a faster algo below M~48 — routing
-        # small-M down-proj here regressed b16x8k decode by 4% (r2)
-        nsplits = min(-(-448 // ntiles), -(-K // 256))
-        k_per_split = -(-(-(-K // nsplits)) // 32) * 32
-        nsplits = -(-K // k_per_split)
-        part = (_skinny_ws(nsplits, N, 64, x.device) if nsplits > 1
-                else x.new_empty(0, dtype=torch.float32))
-        _native().skinny_gemm_v(out, part, x, weight, bias, k_per_split,
-                                nsplits, _SKINNY_TALLK_VARIANT, False)
-        return out
-    if ntiles >= 384:
-        nsplits = 1
-    else:
-        nsplits = min(-(-512 // ntiles), -(-K // 256))
-    k_ceil = -(-K // nsplits)
-    k_per_split = -(-k_ceil // 32) * 32
-    nsplits = -(-K // k_per_split)
-    part = _skinny_ws(nsplits, N, M, x.device) if nsplits > 1 else x.new_empty(
-        0, dtype=torch.float32
-    )
-    _native().skinny_gemm(out, part, x, weight, bias, k_per_split, nsplits)
-    return out
-
-
-def _skinny_ws(nsplits: int, N: int, M: int, device):
-    mrows = ((M + 15) // 16) * 16
-    return torch.empty(nsplits * N * mrows, dtype=torch.float32, device=device)
+    if K % 64 or weight.shape[0] % 4:
+        return _stream_gemm(x, weight, bias)
+    return parts_sum(Parts(_stream_parts(x, weight), bias))
 
 
 _USE_SKINNY = os.environ.get("ARKS_SKINNY_GEMM", "1") == "1"
-# Weight-elements threshold: the split-K streaming kernel beats hipBLASLt's
-# ~19 us latency floor on the small decode shapes (qkv/o: 1.0-1.6x,
-# bench_skinny v3); the big streaming shapes (gate_up/down/lm_head) stay on
-# the tuned hipBLASLt algos which reach 5.4-6.4 TB/s there.
+# weights up to this many elements take the framework's kernels at any number
+# of rows up to 64, larger ones where the rules below say so
 _SKINNY_MAX_ELEMS = 34_000_000
-# tall-K decode shapes (down-proj: K > N) stream W near-HBM-rate through the
-# split-K kernel and beat the library's in-graph algo (r2); wide-N shapes
-# (gate_up/lm_head) stay on hipBLASLt which reaches ~6 TB/s there.
-_SKINNY_TALLK_MAX_ELEMS = 80_000_000
-# 7 = AB=3 deep-staged; 8 = same + non-temporal W loads
-_SKINNY_TALLK_VARIANT = int(os.environ.get("ARKS_SKINNY_TALLK_V", "7"))
 
 
 def _rows_16b(x):
@@ -527,31 +503,79 @@ def _stream_split(M: int, N: int):
     return (mt, 1, 4) if M <= 4 else (mt, 2, 16)
 
 
-def _streams(x, weight, silu: bool = False) -> bool:
-    """Whether x weight^T takes stream_gemm. A workgroup reads all of x's rows
-    beside its 16 or 32 weight rows, so the line lies where that traffic, and
-    the waves' tails, meet what the other path loses: us, here (other), the
-    other being the split kernel up to _SKINNY_MAX_ELEMS and the library
-    beyond. 3584 x 3584: 1 row 7.4 (14.1), 32 rows 12.5 (15.0). 4608 x 3584:
-    16 rows 13.2 (15.5), 32 rows 16.7 (16.2). 544 x 8192, too few workgroups
-    for its K: 8 rows 13.8 (10.4). Library: 18432 x 4096, 16 rows 42.6 (80.1);
-    32000 x 4096, 8 rows 54.5 (67.4), 16 rows 62.0 (62.5); 151936 x 2048, 16
-    rows 134 (206), 32 rows 167 (149); 37888 x 3584, 1 row 52.9 (53.2), 8 rows
-    58.7 (53.1), with the activation 57.8 (59); 3584 x 18944, 1 row 30.3
-    (32.5), 4 rows 33.4 (32.6)."""
-    M, (N, K) = x.shape[0], weight.shape
-    if not (_USE_SKINNY and x.is_cuda and x.dim() == 2 and 1 <= M <= 32
-            and x.dtype == weight.dtype == torch.bfloat16 and K % 32 == 0
+def _few_rows(x, weight) -> bool:
+    """Whether the kernels of stream_gemm.hip can take x weight^T."""
+    return (_USE_SKINNY and x.is_cuda and x.dim() == 2
+            and 1 <= x.shape[0] <= 64
+            and x.dtype == weight.dtype == torch.bfloat16
+            and weight.shape[1] % 32 == 0
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled()
                      and (x.requires_grad or weight.requires_grad))
-            and native_available()):
+            and native_available())
+
+
+def _streams(x, weight, silu: bool = False) -> bool:
+    """Whether x weight^T takes stream_gemm. A workgroup reads all of x's rows
+    beside its 16 or 32 weight rows, so the line lies where that traffic (rows
+    x K), and the waves' tails, meet what the other path loses: us, here
+    (other), the other being the split product with its sums up to
+    _SKINNY_MAX_ELEMS and the library beyond. 3584 x 3584: 1 row 7.4 (10.9),
+    16 rows 9.5 (11.3), 32 rows 12.5 (13.0). 5120 x 2048, 32 rows 10.4 (12.4);
+    6144 x 4096, 32 rows 20.1 (17.7); 544 x 8192, 8 rows 13.8 (10.4). Library:
+    18432 x 4096, 16 rows 42.6 (80.1); 32000 x 4096, 8 rows 54.5 (67.4), 16
+    rows 62.0 (62.5); 151936 x 2048, 16 rows 134 (206), 32 rows 167 (149);
+    37888 x 3584, 1 row 52.9 (53.2), 8 rows 58.7 (53.1), with the activation
+    57.8 (59); 3584 x 18944, 1 row 30.3 (32.5), 4 rows 33.4 (32.6)."""
+    if not _few_rows(x, weight):
         return False
+    M, (N, K) = x.shape[0], weight.shape
     if N * K <= _SKINNY_MAX_ELEMS:
-        return K <= 4096 or N >= 2048
+        return M * K <= 98304 and (K <= 4096 or N >= 2048) or K % 64 != 0
     if M <= 2 or (silu and M <= 8 and K <= 4096):
         return True
     return M <= 16 and (K <= 2048 or (K <= 4096 and N * K <= 1 << 27))
+
+
+def _splits(x, weight) -> bool:
+    """Whether x weight^T splits K over workgroups (asked after _streams):
+    weights up to _SKINNY_MAX_ELEMS, and larger ones that are tall. us with
+    the sums (library): 3584 x 18944, 4 rows 30.7 (32.6), 32 rows 31.7 (43.9),
+    64 rows 36.8 (49.6); 8192 x 28672, 8 rows 88.5 (91.8), 64 rows 108 (154);
+    wide ones, as 16384 x 4096 at 32 rows, 36 (34)."""
+    N, K = weight.shape
+    return (_few_rows(x, weight) and K % 64 == 0 and N % 4 == 0
+            and (N * K <= _SKINNY_MAX_ELEMS or K >= 2 * N))
+
+
+class Parts:
+    """A product whose sums over runs of K are not added yet: sums [splits,
+    M, N] fp32, and a bias [N] that belongs to their sum."""
+
+    def __init__(self, sums, bias=None):
+        self.sums, self.bias = sums, bias
+
+
+def _stream_parts(x, weight):
+    """Split sums; as many splits as give every CU a workgroup of 128 weight
+    rows (3584 x 3584, 64 rows, us without the sums: 4 splits 14.9, 8 11.4, 12
+    13.2), at most 16 and, where many rows make the sums long, 8."""
+    M, (N, K) = x.shape[0], weight.shape
+    splits = max(1, min(256 // -(-N // 128), 16 if M <= 32 else 8,
+                        K // (128 if K % 128 == 0 else 64)))
+    sums = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
+    _native().stream_split(sums, _rows_16b(x), weight)
+    return sums
+
+
+def parts_sum(x):
+    """The bf16 tensor that x, a Parts or already a tensor, stands for."""
+    if not isinstance(x, Parts):
+        return x
+    out = torch.empty(x.sums.shape[1:], dtype=torch.bfloat16,
+                      device=x.sums.device)
+    _native().stream_sum(out, x.sums, x.bias)
+    return out
 
 
 def _stream_gemm(x, weight, bias=None, dtype=None, silu: bool = False):
@@ -564,28 +588,21 @@ def _stream_gemm(x, weight, bias=None, dtype=None, silu: bool = False):
     return out
 
 
+def linear_parts(x, weight, bias=None):
+    """linear_bf16 for a consumer that takes Parts."""
+    if x.dim() == 2 and not _streams(x, weight) and _splits(x, weight):
+        return Parts(_stream_parts(x, weight), bias)
+    return linear_bf16(x, weight, bias)
+
+
 def linear_bf16(x, weight, bias=None):
-    """Linear dispatch: the streamed product for few rows, the skinny split-K
-    kernel for other small decode-shaped GEMMs on GPU, hipBLASLt (F.linear)
-    otherwise."""
+    """Linear dispatch: the streamed product for few rows, K split over
+    workgroups for other small decode-shaped and tall GEMMs on GPU, hipBLASLt
+    (F.linear) otherwise."""
     if x.dim() == 2 and _streams(x, weight):
         return _stream_gemm(x, weight, bias)
-    if (
-        _USE_SKINNY
-        and x.is_cuda
-        and x.dim() == 2
-        and 1 <= x.shape[0] <= 64
-        and x.dtype == torch.bfloat16
-        and weight.shape[0] % 64 == 0
-        and weight.shape[1] % 32 == 0
-        and (weight.numel() <= _SKINNY_MAX_ELEMS
-             or (weight.shape[1] > weight.shape[0]
-                 and x.shape[0] > 48
-                 and weight.numel() <= _SKINNY_TALLK_MAX_ELEMS))
-        and weight.is_contiguous()
-        and native_available()
-    ):
-        return skinny_gemm(x, weight, bias)
+    if x.dim() == 2 and _splits(x, weight):
+        return parts_sum(Parts(_stream_parts(x, weight), bias))
     import torch.nn.functional as F
 
     return F.linear(x, weight, bias)

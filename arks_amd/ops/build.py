@@ -27,7 +27,6 @@ SOURCES = [
     os.path.join(CSRC, "attn_extend.hip"),
     os.path.join(CSRC, "attn_extend2.hip"),
     os.path.join(CSRC, "quant_fp8.hip"),
-    os.path.join(CSRC, "skinny_gemm.hip"),
     os.path.join(CSRC, "sampling.hip"),
     os.path.join(CSRC, "moe.hip"),
     os.path.join(CSRC, "moe_gemm.hip"),

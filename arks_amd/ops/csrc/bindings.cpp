@@ -20,6 +20,17 @@ void arks_rmsnorm(void* out, const void* input, const void* weight, float eps,
 void arks_fused_add_rmsnorm(void* out, const void* input, void* residual,
                             const void* weight, float eps, int rows, int hidden,
                             hipStream_t stream);
+void arks_fused_add_rmsnorm_parts(void* out, const void* part, int splits,
+                                  void* residual, const void* weight, float eps,
+                                  int rows, int hidden, hipStream_t stream);
+void arks_rope_and_cache_parts(const void* positions, void* q, const void* part,
+                               const void* bias, int splits, void* k_cache,
+                               void* v_cache, const void* slot_mapping,
+                               const void* cos_sin, int num_tokens,
+                               int head_dim, int num_q_heads, int num_kv_heads,
+                               int block_size, int kv_fp8, const void* q_norm,
+                               const void* k_norm, float eps,
+                               hipStream_t stream);
 void arks_silu_mul(void* out, const void* gate_up, int64_t rows, int d,
                    hipStream_t stream);
 void arks_rope_inplace(const void* positions, void* q, void* k,
@@ -56,14 +67,6 @@ void arks_rmsnorm_fp8(void* out, void* inv_scale, const void* input,
                       int hidden, int fused_add, hipStream_t stream);
 void arks_silu_mul_fp8(void* out, void* inv_scale, const void* gate_up,
                        int rows, int d, hipStream_t stream);
-void arks_skinny_gemm(void* part, void* out, const void* a, const void* w,
-                      const void* bias, int m_rows, int n_total, int k_total,
-                      int k_per_split, int nsplits, int64_t a_stride,
-                      hipStream_t stream);
-void arks_skinny_gemm_v(void* part, void* out, const void* a, const void* w,
-                        const void* bias, int m_rows, int n_total, int k_total,
-                        int k_per_split, int nsplits, int64_t a_stride,
-                        int variant, bool fuse_silu, hipStream_t stream);
 void arks_sample(void* out, void* part_val, void* part_idx, const void* logits,
                  const void* temperatures, const void* uniform, int rows,
                  int vocab, int parts, hipStream_t stream);
@@ -82,6 +85,10 @@ void arks_moe_mix_rows(void* out, const void* y, const void* weights,
 void arks_stream_gemm(void* out, const void* a, const void* w, const void* bias,
                       int m, int n, int k, int64_t a_stride, int mt, int nf,
                       int wv, int f32, int silu, hipStream_t stream);
+void arks_stream_split(void* part, const void* a, const void* w, int m, int n,
+                       int k, int64_t a_stride, int splits, hipStream_t stream);
+void arks_stream_sum(void* out, const void* part, const void* bias, int64_t m,
+                     int n, int splits, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, const void* ids, const void* weights,
                    int pairs, int expert_base, int n_local, int tile,
@@ -108,6 +115,14 @@ hipStream_t current_stream() {
 // bf16 tensor whose trailing dims are contiguous; dim-0 rows may be strided
 // (a view into the fused QKV buffer).
 
+void check_parts(const torch::Tensor& part) {
+  TORCH_CHECK(part.is_cuda() && part.is_contiguous() && part.dim() == 3 &&
+                  part.scalar_type() == torch::kFloat32 && part.size(0) >= 1 &&
+                  part.size(2) % 4 == 0 &&
+                  reinterpret_cast<uintptr_t>(part.data_ptr()) % 16 == 0,
+              "parts must be fp32 [splits, rows, columns], columns % 4 == 0");
+}
+
 void rmsnorm(torch::Tensor out, torch::Tensor input, torch::Tensor weight,
              double eps) {
   check_bf16_contig(out, "out");
@@ -132,6 +147,22 @@ void fused_add_rmsnorm(torch::Tensor out, torch::Tensor input,
   arks_fused_add_rmsnorm(out.data_ptr(), input.data_ptr(), residual.data_ptr(),
                          weight.data_ptr(), (float)eps, rows, hidden,
                          current_stream());
+}
+
+// fused_add_rmsnorm of the sum of part's splits
+void fused_add_rmsnorm_parts(torch::Tensor out, torch::Tensor part,
+                             torch::Tensor residual, torch::Tensor weight,
+                             double eps) {
+  check_bf16_contig(out, "out");
+  check_bf16_contig(residual, "residual");
+  check_parts(part);
+  const int64_t hidden = part.size(2), rows = part.size(1);
+  TORCH_CHECK(hidden % 8 == 0 && out.numel() == rows * hidden &&
+              residual.numel() == rows * hidden && weight.numel() == hidden);
+  arks_fused_add_rmsnorm_parts(out.data_ptr(), part.data_ptr(),
+                               (int)part.size(0), residual.data_ptr(),
+                               weight.data_ptr(), (float)eps, (int)rows,
+                               (int)hidden, current_stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor gate_up) {
@@ -219,6 +250,54 @@ void rope_and_cache(torch::Tensor positions, torch::Tensor q,
                       (float)eps, current_stream());
 }
 
+// rope_and_cache of the projection's split sums part [splits, T, (q heads + 2
+// kv heads) * head_dim] (+ bias): rotated q to q, k and v to the cache only
+void rope_and_cache_parts(torch::Tensor positions, torch::Tensor q,
+                          torch::Tensor part, c10::optional<torch::Tensor> bias,
+                          torch::Tensor k_cache, torch::Tensor v_cache,
+                          torch::Tensor slot_mapping, torch::Tensor cos_sin,
+                          int64_t head_dim, c10::optional<torch::Tensor> q_norm,
+                          c10::optional<torch::Tensor> k_norm, double eps) {
+  TORCH_CHECK(positions.scalar_type() == torch::kInt64);
+  TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
+  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32);
+  check_bf16_contig(q, "q");
+  check_parts(part);
+  const int64_t T = part.size(1), width = part.size(2);
+  const int nkv = k_cache.size(1), block_size = k_cache.size(2);
+  TORCH_CHECK(head_dim % 8 == 0 && k_cache.size(3) == head_dim &&
+              k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              v_cache.sizes() == k_cache.sizes());
+  TORCH_CHECK(q.dim() == 2 && q.size(0) == T && q.size(1) % head_dim == 0 &&
+              width == q.size(1) + 2 * nkv * head_dim &&
+              positions.numel() == T && slot_mapping.numel() == T);
+  const bool kv_fp8 = k_cache.scalar_type() != torch::kBFloat16;
+  TORCH_CHECK(v_cache.scalar_type() == k_cache.scalar_type() &&
+              k_cache.element_size() == (kv_fp8 ? 1 : 2));
+  if (bias.has_value()) {
+    check_bf16_contig(*bias, "bias");
+    TORCH_CHECK(bias->numel() == width);
+  }
+  TORCH_CHECK(q_norm.has_value() == k_norm.has_value());
+  if (q_norm.has_value()) {
+    check_bf16_contig(*q_norm, "q_norm");
+    check_bf16_contig(*k_norm, "k_norm");
+    TORCH_CHECK(q_norm->numel() == head_dim && k_norm->numel() == head_dim);
+    TORCH_CHECK(head_dim == 32 || head_dim == 64 || head_dim == 128 ||
+                    head_dim == 256,
+                "head norms need head_dim 32, 64, 128 or 256");
+  }
+  arks_rope_and_cache_parts(
+      positions.data_ptr(), q.data_ptr(), part.data_ptr(),
+      bias.has_value() ? bias->data_ptr() : nullptr, (int)part.size(0),
+      k_cache.data_ptr(), v_cache.data_ptr(), slot_mapping.data_ptr(),
+      cos_sin.data_ptr(), (int)T, (int)head_dim, (int)(q.size(1) / head_dim),
+      nkv, block_size, kv_fp8 ? 1 : 0,
+      q_norm.has_value() ? q_norm->data_ptr() : nullptr,
+      k_norm.has_value() ? k_norm->data_ptr() : nullptr, (float)eps,
+      current_stream());
+}
+
 
 void attention_prefill_varlen(torch::Tensor out, torch::Tensor q,
                               torch::Tensor k, torch::Tensor v,
@@ -247,66 +326,6 @@ void attention_prefill_varlen(torch::Tensor out, torch::Tensor q,
 
 // 8-wave 32x32-MFMA ladder (attn_extend2.hip): 256-row q tiles, bf16 KV.
 
-
-void skinny_gemm(torch::Tensor out, torch::Tensor part, torch::Tensor a,
-                 torch::Tensor w, c10::optional<torch::Tensor> bias,
-                 int64_t k_per_split, int64_t nsplits) {
-  check_bf16_contig(out, "out");
-  check_bf16_rowstrided(a, "a");
-  check_bf16_contig(w, "w");
-  const int m = a.size(0), k = a.size(1), n = w.size(0);
-  TORCH_CHECK(m >= 1 && m <= 64, "skinny_gemm needs 1 <= M <= 64");
-  TORCH_CHECK(n % 64 == 0 && k % 32 == 0, "N%64==0 and K%32==0 required");
-  TORCH_CHECK(w.size(1) == k && out.size(0) == m && out.size(1) == n);
-  const void* bias_ptr = nullptr;
-  if (bias.has_value()) {
-    check_bf16_contig(*bias, "bias");
-    TORCH_CHECK(bias->numel() == n);
-    bias_ptr = bias->data_ptr();
-  }
-  const int mrows = ((m + 15) / 16) * 16;
-  if (nsplits > 1) {
-    TORCH_CHECK(part.scalar_type() == torch::kFloat32 &&
-                part.numel() >= (int64_t)nsplits * n * mrows,
-                "skinny_gemm workspace too small");
-  }
-  arks_skinny_gemm(nsplits > 1 ? part.data_ptr() : nullptr, out.data_ptr(),
-                   a.data_ptr(), w.data_ptr(), bias_ptr, m, n, k,
-                   (int)k_per_split, (int)nsplits, a.stride(0),
-                   current_stream());
-}
-
-// Variant/fused entry (MT fixed at 4, i.e. M <= 64). fuse_silu: `a` is the
-// gate_up output [M, >=2K] (gate cols [0,K), up cols [K,2K)).
-void skinny_gemm_v(torch::Tensor out, torch::Tensor part, torch::Tensor a,
-                   torch::Tensor w, c10::optional<torch::Tensor> bias,
-                   int64_t k_per_split, int64_t nsplits, int64_t variant,
-                   bool fuse_silu) {
-  check_bf16_contig(out, "out");
-  check_bf16_rowstrided(a, "a");
-  check_bf16_contig(w, "w");
-  const int m = a.size(0), k = w.size(1), n = w.size(0);
-  TORCH_CHECK(m >= 1 && m <= 64, "skinny_gemm_v needs 1 <= M <= 64");
-  TORCH_CHECK(n % 64 == 0 && k % 32 == 0, "N%64==0 and K%32==0 required");
-  TORCH_CHECK(a.size(1) >= (fuse_silu ? 2 * k : k), "A too narrow");
-  TORCH_CHECK(out.size(0) == m && out.size(1) == n);
-  TORCH_CHECK(0 <= variant && variant <= 8, "variant in 0..8");
-  const void* bias_ptr = nullptr;
-  if (bias.has_value()) {
-    check_bf16_contig(*bias, "bias");
-    TORCH_CHECK(bias->numel() == n);
-    bias_ptr = bias->data_ptr();
-  }
-  if (nsplits > 1) {
-    TORCH_CHECK(part.scalar_type() == torch::kFloat32 &&
-                part.numel() >= (int64_t)nsplits * n * 64,
-                "skinny_gemm_v workspace too small");
-  }
-  arks_skinny_gemm_v(nsplits > 1 ? part.data_ptr() : nullptr, out.data_ptr(),
-                     a.data_ptr(), w.data_ptr(), bias_ptr, m, n, k,
-                     (int)k_per_split, (int)nsplits, a.stride(0),
-                     (int)variant, fuse_silu, current_stream());
-}
 
 void rmsnorm_fp8(torch::Tensor out, torch::Tensor inv_scale,
                  torch::Tensor input, c10::optional<torch::Tensor> residual,
@@ -558,6 +577,38 @@ void stream_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
                    f32 ? 1 : 0, silu ? 1 : 0, current_stream());
 }
 
+// part [splits, M, N] fp32: the sums of a [M, K] w [N, K]^T over runs of K
+void stream_split(torch::Tensor part, torch::Tensor a, torch::Tensor w) {
+  check_bf16_rowstrided(a, "a");
+  check_bf16_contig(w, "w");
+  TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && part.dim() == 3);
+  check_rows_16b(a, "a");
+  check_rows_16b(w, "w");
+  check_parts(part);
+  const int64_t M = a.size(0), N = w.size(0), K = a.size(1);
+  TORCH_CHECK(w.size(1) == K && part.size(1) == M && part.size(2) == N);
+  TORCH_CHECK(M >= 1 && M <= 64 && K % 64 == 0 && N < (1 << 30),
+              "need at most 64 rows and K % 64 == 0");
+  TORCH_CHECK(part.size(0) <= K / 64, "more splits than chunks");
+  arks_stream_split(part.data_ptr(), a.data_ptr(), w.data_ptr(), (int)M, (int)N,
+                    (int)K, a.stride(0), (int)part.size(0), current_stream());
+}
+
+void stream_sum(torch::Tensor out, torch::Tensor part,
+                c10::optional<torch::Tensor> bias) {
+  check_bf16_contig(out, "out");
+  check_parts(part);
+  const int64_t M = part.size(1), N = part.size(2);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == N);
+  if (bias.has_value()) {
+    check_bf16_contig(*bias, "bias");
+    TORCH_CHECK(bias->numel() == N);
+  }
+  arks_stream_sum(out.data_ptr(), part.data_ptr(),
+                  bias.has_value() ? bias->data_ptr() : nullptr, M, (int)N,
+                  (int)part.size(0), current_stream());
+}
+
 // The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
 // beyond this rank's El experts from expert_base on count as zero.
 void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
@@ -638,8 +689,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quant_fp8_rows", &quant_fp8_rows);
   m.def("rmsnorm_fp8", &rmsnorm_fp8);
   m.def("silu_mul_fp8", &silu_mul_fp8);
-  m.def("skinny_gemm", &skinny_gemm);
-  m.def("skinny_gemm_v", &skinny_gemm_v);
   m.def("greedy_sample", &greedy_sample);
   m.def("gumbel_sample", &gumbel_sample);
   m.def("ipc_alloc", &ipc_alloc);
@@ -652,7 +701,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_topk", &moe_topk);
   m.def("moe_mix", &moe_mix);
   m.def("moe_mix_rows", &moe_mix_rows);
+  m.def("fused_add_rmsnorm_parts", &fused_add_rmsnorm_parts);
+  m.def("rope_and_cache_parts", &rope_and_cache_parts);
   m.def("stream_gemm", &stream_gemm);
+  m.def("stream_split", &stream_split);
+  m.def("stream_sum", &stream_sum);
   m.def("moe_experts", &moe_experts);
   m.def("mfma_probe", &mfma_probe);
   m.def("mfma_probe32", &mfma_probe32);

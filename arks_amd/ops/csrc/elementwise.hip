@@ -3,22 +3,32 @@
 // accumulation. Ops: rmsnorm, fused residual-add + rmsnorm, silu_mul (SwiGLU),
 // neox-style RoPE (in-place on q and k).
 #include "common.h"
+#include "parts.h"
 
 namespace arks {
 
 // ---------------------------------------------------------------------------
 // RMSNorm: one workgroup (256 threads = 4 waves) per row.
 // hidden must be a multiple of 8 (bf16x8 vector loads).
+// PARTS: the input is the sum of fp32 splits [splits, rows, hidden] of the
+// product before it; adding 8 of them here takes 1 us at 64 x 3584, a launch
+// of its own 5.
 // ---------------------------------------------------------------------------
-template <bool FUSED_ADD>
+template <bool FUSED_ADD, bool PARTS = false>
 __global__ void rmsnorm_kernel(bf16* __restrict__ out,
-                               const bf16* __restrict__ input,
+                               const void* __restrict__ input,
                                bf16* __restrict__ residual,  // null unless FUSED_ADD
                                const bf16* __restrict__ weight,
-                               const float eps, const int hidden) {
-  constexpr int BLOCK = 256;
+                               const float eps, const int hidden,
+                               const int splits = 0) {
+  // split sums come with few rows: more threads, so that a row is one pass
+  constexpr int BLOCK = PARTS ? 512 : 256;
   const int row = blockIdx.x;
-  const bf16* in_row = input + (int64_t)row * hidden;
+  const bf16* in_row =
+      reinterpret_cast<const bf16*>(input) + (int64_t)row * hidden;
+  const float* part_row =
+      reinterpret_cast<const float*>(input) + (int64_t)row * hidden;
+  const int64_t part_stride = (int64_t)gridDim.x * hidden;
   bf16* res_row = FUSED_ADD ? residual + (int64_t)row * hidden : nullptr;
   bf16* out_row = out + (int64_t)row * hidden;
 
@@ -26,13 +36,23 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
   float ss = 0.f;
   // Pass 1: (optionally add residual and store it), accumulate sum of squares.
   for (int i = threadIdx.x; i < nvec; i += BLOCK) {
-    ushort8 x = *reinterpret_cast<const ushort8*>(in_row + i * 8);
+    float x[8];
+    if constexpr (PARTS) {
+      const f32x4 lo = sum_parts4(part_row + i * 8, part_stride, splits);
+      const f32x4 hi = sum_parts4(part_row + i * 8 + 4, part_stride, splits);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = j < 4 ? lo[j % 4] : hi[j % 4];
+    } else {
+      const ushort8 u = *reinterpret_cast<const ushort8*>(in_row + i * 8);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = bf16_bits_to_float(u[j]);
+    }
     if constexpr (FUSED_ADD) {
       ushort8 r = *reinterpret_cast<const ushort8*>(res_row + i * 8);
       ushort8 s;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        float v = bf16_bits_to_float(x[j]) + bf16_bits_to_float(r[j]);
+        float v = x[j] + bf16_bits_to_float(r[j]);
         s[j] = float_to_bf16_bits(v);
         // Accumulate on the bf16-rounded value so pass 2's re-read matches.
         float vb = bf16_bits_to_float(s[j]);
@@ -41,10 +61,7 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
       *reinterpret_cast<ushort8*>(res_row + i * 8) = s;
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float v = bf16_bits_to_float(x[j]);
-        ss += v * v;
-      }
+      for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
     }
   }
 
@@ -147,7 +164,7 @@ void arks_rmsnorm(void* out, const void* input, const void* weight, float eps,
                   int rows, int hidden, hipStream_t stream) {
   dim3 grid(rows), block(256);
   hipLaunchKernelGGL((rmsnorm_kernel<false>), grid, block, 0, stream,
-                     (bf16*)out, (const bf16*)input, nullptr,
+                     (bf16*)out, input, nullptr,
                      (const bf16*)weight, eps, hidden);
 }
 
@@ -156,8 +173,15 @@ void arks_fused_add_rmsnorm(void* out, const void* input, void* residual,
                             hipStream_t stream) {
   dim3 grid(rows), block(256);
   hipLaunchKernelGGL((rmsnorm_kernel<true>), grid, block, 0, stream, (bf16*)out,
-                     (const bf16*)input, (bf16*)residual, (const bf16*)weight,
-                     eps, hidden);
+                     input, (bf16*)residual, (const bf16*)weight, eps, hidden, 0);
+}
+
+void arks_fused_add_rmsnorm_parts(void* out, const void* part, int splits,
+                                  void* residual, const void* weight, float eps,
+                                  int rows, int hidden, hipStream_t stream) {
+  hipLaunchKernelGGL((rmsnorm_kernel<true, true>), dim3(rows), dim3(512), 0,
+                     stream, (bf16*)out, part, (bf16*)residual,
+                     (const bf16*)weight, eps, hidden, splits);
 }
 
 void arks_silu_mul(void* out, const void* gate_up, int64_t rows, int d,

@@ -2,6 +2,7 @@
 // Cache layout: [num_blocks, num_kv_heads, block_size, head_dim] bf16
 // slot = block_id * block_size + offset  (flat, per token)
 #include "common.h"
+#include "parts.h"
 
 #include <hip/hip_fp8.h>
 
@@ -117,8 +118,11 @@ namespace arks {
 // until the rotated ones are rounded). As separate passes the two norms and
 // the contiguous copies that they need cost 14 us per layer at 7 rows and
 // 100 us at 5012 (32/4 heads x 128).
+// PARTS: q, k and v are the sums of fp32 splits [splits, T, q | k | v] of the
+// projection (+ bias); k and v go to the cache alone. Saves the launch that
+// would add them (5 us at 64 rows of 4608).
 // ---------------------------------------------------------------------------
-template <bool FP8, bool NORM>
+template <bool FP8, bool NORM, bool PARTS>
 __global__ void rope_cache_kernel(
     const int64_t* __restrict__ positions,
     bf16* __restrict__ q,        // [T, Hq*D] rows strided
@@ -131,8 +135,12 @@ __global__ void rope_cache_kernel(
     const int head_dim, const int num_q_heads, const int num_kv_heads,
     const int block_size, const int64_t q_stride, const int64_t k_stride,
     const bf16* __restrict__ q_norm, const bf16* __restrict__ k_norm,
-    const float eps) {
+    const float eps, const float* __restrict__ part,
+    const bf16* __restrict__ bias, const int splits) {
   const int token = blockIdx.x;
+  const int width = (num_q_heads + 2 * num_kv_heads) * head_dim;
+  const int64_t part_stride = (int64_t)gridDim.x * width;
+  const float* part_row = part + (int64_t)token * width;
   const int half = head_dim / 2;
   const int64_t pos = positions[token];
   const float* cs = cos_sin + pos * head_dim;
@@ -147,7 +155,9 @@ __global__ void rope_cache_kernel(
 
   const int total_heads = num_q_heads + num_kv_heads;
   const int pairs2 = half / 2;
-  for (int idx = threadIdx.x; idx < total_heads * pairs2; idx += blockDim.x) {
+  const int first = blockIdx.y * blockDim.x + threadIdx.x;
+  const int step = gridDim.y * blockDim.x;
+  for (int idx = first; idx < total_heads * pairs2; idx += step) {
     const int h = idx / pairs2;
     const int p2 = (idx % pairs2) * 2;
     const bool is_q = h < num_q_heads;
@@ -155,14 +165,28 @@ __global__ void rope_cache_kernel(
                      ? q + (int64_t)token * q_stride + (int64_t)h * head_dim
                      : k + (int64_t)token * k_stride +
                            (int64_t)(h - num_q_heads) * head_dim;
-    ushort2v x1 = *reinterpret_cast<const ushort2v*>(base + p2);
-    ushort2v x2 = *reinterpret_cast<const ushort2v*>(base + half + p2);
     ushort2v o1, o2;
     float a2[2], b2[2];
+    if constexpr (PARTS) {
+      const int c = h * head_dim + p2;
+      const float2 f1 = sum_parts2(part_row + c, part_stride, splits);
+      const float2 f2 = sum_parts2(part_row + c + half, part_stride, splits);
+      a2[0] = f1.x, a2[1] = f1.y, b2[0] = f2.x, b2[1] = f2.y;
+      if (bias) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      a2[j] = bf16_bits_to_float(x1[j]);
-      b2[j] = bf16_bits_to_float(x2[j]);
+        for (int j = 0; j < 2; ++j) {
+          a2[j] += bf16_bits_to_float(bias[c + j]);
+          b2[j] += bf16_bits_to_float(bias[c + half + j]);
+        }
+      }
+    } else {
+      const ushort2v x1 = *reinterpret_cast<const ushort2v*>(base + p2);
+      const ushort2v x2 = *reinterpret_cast<const ushort2v*>(base + half + p2);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        a2[j] = bf16_bits_to_float(x1[j]);
+        b2[j] = bf16_bits_to_float(x2[j]);
+      }
     }
     if constexpr (NORM) {
       float ss = a2[0] * a2[0] + a2[1] * a2[1] + b2[0] * b2[0] + b2[1] * b2[1];
@@ -185,8 +209,10 @@ __global__ void rope_cache_kernel(
       o1[j] = float_to_bf16_bits(a * c - b * s);
       o2[j] = float_to_bf16_bits(b * c + a * s);
     }
-    *reinterpret_cast<ushort2v*>(base + p2) = o1;
-    *reinterpret_cast<ushort2v*>(base + half + p2) = o2;
+    if (!PARTS || is_q) {
+      *reinterpret_cast<ushort2v*>(base + p2) = o1;
+      *reinterpret_cast<ushort2v*>(base + half + p2) = o2;
+    }
     if (!is_q && cache) {
       const int64_t dst = cbase + (int64_t)(h - num_q_heads) * hstride;
       if constexpr (FP8) {
@@ -211,11 +237,23 @@ __global__ void rope_cache_kernel(
   // v: plain copy into the page (vectorized 8)
   const bf16* v_src = v + (int64_t)token * k_stride;
   const int nvec = num_kv_heads * head_dim / 8;
-  for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
+  for (int i = first; i < nvec; i += step) {
     const int h = (i * 8) / head_dim;
     const int d = (i * 8) % head_dim;
     const int64_t dst = cbase + (int64_t)h * hstride + d;
-    ushort8 vv8 = *reinterpret_cast<const ushort8*>(v_src + i * 8);
+    ushort8 vv8;
+    if constexpr (PARTS) {
+      const int c = (num_q_heads + num_kv_heads) * head_dim + i * 8;
+      const f32x4 lo = sum_parts4(part_row + c, part_stride, splits);
+      const f32x4 hi = sum_parts4(part_row + c + 4, part_stride, splits);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float b = bias ? bf16_bits_to_float(bias[c + e]) : 0.f;
+        vv8[e] = float_to_bf16_bits((e < 4 ? lo[e % 4] : hi[e % 4]) + b);
+      }
+    } else {
+      vv8 = *reinterpret_cast<const ushort8*>(v_src + i * 8);
+    }
     if constexpr (FP8) {
       uchar8 vo;
 #pragma unroll
@@ -232,6 +270,13 @@ __global__ void rope_cache_kernel(
 
 }  // namespace arks
 
+// Workgroups per token: few tokens leave most CUs idle, so each thread gets one
+// couple of pairs. 64 tokens of 28/4 heads x 128, with 8 splits to add: 1 group
+// 12.2 us, 4 groups 7.1 us.
+static int rope_groups(int num_tokens, int heads, int head_dim) {
+  return num_tokens > 256 ? 1 : (heads * (head_dim / 4) + 255) / 256;
+}
+
 // q_norm, k_norm: null, or bf16 [head_dim] weights of the heads' RMS norms
 // (head_dim 32, 64, 128 or 256).
 extern "C" void arks_rope_and_cache(
@@ -241,15 +286,44 @@ extern "C" void arks_rope_and_cache(
     int block_size, int64_t q_stride, int64_t k_stride, int kv_fp8,
     const void* q_norm, const void* k_norm, float eps, hipStream_t stream) {
   if (num_tokens == 0) return;
-  dim3 grid(num_tokens), block(256);
+  dim3 grid(num_tokens,
+            rope_groups(num_tokens, num_q_heads + num_kv_heads, head_dim)),
+      block(256);
 #define ARKS_ROPE(FP8, NORM)                                                   \
-  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM>), grid, block, 0, stream,   \
+  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, false>), grid, block, 0,    \
+                     stream,                                                   \
                      (const int64_t*)positions, (bf16*)q, (bf16*)k,            \
                      (const bf16*)v, k_cache, v_cache,                         \
                      (const int64_t*)slot_mapping, (const float*)cos_sin,      \
                      head_dim, num_q_heads, num_kv_heads, block_size,          \
                      q_stride, k_stride, (const bf16*)q_norm,                  \
-                     (const bf16*)k_norm, eps)
+                     (const bf16*)k_norm, eps, nullptr, nullptr, 0)
+  if (kv_fp8) {
+    if (q_norm) ARKS_ROPE(true, true); else ARKS_ROPE(true, false);
+  } else {
+    if (q_norm) ARKS_ROPE(false, true); else ARKS_ROPE(false, false);
+  }
+#undef ARKS_ROPE
+}
+
+extern "C" void arks_rope_and_cache_parts(
+    const void* positions, void* q, const void* part, const void* bias,
+    int splits, void* k_cache, void* v_cache, const void* slot_mapping,
+    const void* cos_sin, int num_tokens, int head_dim, int num_q_heads,
+    int num_kv_heads, int block_size, int kv_fp8, const void* q_norm,
+    const void* k_norm, float eps, hipStream_t stream) {
+  dim3 grid(num_tokens,
+            rope_groups(num_tokens, num_q_heads + num_kv_heads, head_dim)),
+      block(256);
+#define ARKS_ROPE(FP8, NORM)                                                   \
+  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, true>), grid, block, 0,     \
+                     stream, (const int64_t*)positions, (bf16*)q, nullptr,     \
+                     nullptr, k_cache, v_cache, (const int64_t*)slot_mapping,  \
+                     (const float*)cos_sin, head_dim, num_q_heads,             \
+                     num_kv_heads, block_size,                                 \
+                     (int64_t)num_q_heads * head_dim, 0, (const bf16*)q_norm,  \
+                     (const bf16*)k_norm, eps, (const float*)part,             \
+                     (const bf16*)bias, splits)
   if (kv_fp8) {
     if (q_norm) ARKS_ROPE(true, true); else ARKS_ROPE(true, false);
   } else {

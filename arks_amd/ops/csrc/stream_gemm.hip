@@ -9,13 +9,13 @@
 // library product with its conversion 11 us. With more rows the loads of a,
 // one set per workgroup, take over: 151936 x 2048, 16 rows 134 us.
 #include "common.h"
+#include "parts.h"
 
 namespace arks {
 
 namespace {
 
 using bf16x8_sg = __attribute__((ext_vector_type(8))) __bf16;
-using f32x4 = __attribute__((ext_vector_type(4))) float;
 
 __device__ __forceinline__ f32x4 stream_mfma(const ushort8& w, const ushort8& a,
                                              const f32x4& c) {
@@ -161,6 +161,130 @@ __global__ __launch_bounds__(WV * 64) void stream_gemm_kernel(
   }
 }
 
+// For more rows than stream_gemm_kernel takes, and for few weight rows with
+// long K: K is split over blockIdx.y too, and the fp32 sums of a split go to
+// part [splits, M, N] for the consumer to add. 8 waves take 16 weight rows
+// each and share the rows of a: KC columns of them at a time through two LDS
+// buffers, fetched three chunks ahead, the weights PF chunks ahead in
+// registers. The barriers wait for LDS alone, so the loads stay in flight.
+// 3584 x 18944 (136 MB) in 8 splits: 8 rows 27 us, 64 rows 34 us, and 3 us
+// for the sums where no consumer adds them; with barriers that drain the loads
+// and 64 weight rows a workgroup 40 and 5 us, in the library 33 and 50 us.
+template <int MT, int KC, int PF>
+__global__ __launch_bounds__(512) void stream_split_kernel(
+    float* __restrict__ part, const bf16* __restrict__ a,
+    const bf16* __restrict__ w, const int m_rows, const int n_total,
+    const int k_total, const int64_t a_stride, const int splits) {
+  static_assert(PF % 2 == 0, "buffers alternate over a round");
+  constexpr int S = KC / 32, CPR = KC / 8, ITEMS = MT * 16 * CPR;
+  constexpr int AI = (ITEMS + 511) / 512;
+  __shared__ __attribute__((aligned(16))) bf16 lds[2][MT * 16][KC + 8];
+  const int tid = threadIdx.x, lane = tid % WAVE_SIZE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE_SIZE);
+  const int lq = lane % 16, la = lane / 16;
+  const int n0 = (blockIdx.x * 8 + wave) * 16;
+  const int chunks = k_total / KC;
+  const int first = (int)((int64_t)chunks * blockIdx.y / splits);
+  const int n = (int)((int64_t)chunks * (blockIdx.y + 1) / splits) - first;
+  f32x4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bf16* wp = w + (int64_t)min(n0 + lq, n_total - 1) * k_total + 8 * la +
+                   (int64_t)first * KC;
+  const bf16* ap[AI];
+#pragma unroll
+  for (int t = 0; t < AI; ++t) {
+    const int i = tid + t * 512;
+    ap[t] = a + (int64_t)min(i / CPR, m_rows - 1) * a_stride + i % CPR * 8 +
+            (int64_t)first * KC;
+  }
+  ushort8 wr[PF][S], ar[2][AI];
+  auto load_w = [&](ushort8 (&r)[S], const int i) {
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+      r[q] = *reinterpret_cast<const ushort8*>(wp + (int64_t)i * KC + q * 32);
+  };
+  auto load_a = [&](ushort8 (&r)[AI], const int i) {
+#pragma unroll
+    for (int t = 0; t < AI; ++t)
+      r[t] = *reinterpret_cast<const ushort8*>(ap[t] + (int64_t)i * KC);
+  };
+  auto store_a = [&](const ushort8 (&r)[AI], const int b) {
+#pragma unroll
+    for (int t = 0; t < AI; ++t) {
+      const int i = tid + t * 512;
+      if (ITEMS % 512 == 0 || i < ITEMS)
+        *reinterpret_cast<ushort8*>(&lds[b][i / CPR][i % CPR * 8]) = r[t];
+    }
+  };
+  auto mul = [&](const ushort8 (&r)[S], const int b) {
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t] = stream_mfma(r[q],
+                             *reinterpret_cast<const ushort8*>(
+                                 &lds[b][t * 16 + lq][q * 32 + 8 * la]),
+                             acc[t]);
+  };
+  auto meet = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  load_a(ar[0], 0);
+#pragma unroll
+  for (int j = 0; j < PF; ++j)
+    if (j < n) load_w(wr[j], j);
+  if (n > 1) load_a(ar[1], 1);
+  store_a(ar[0], 0);
+  if (n > 2) load_a(ar[0], 2);
+  meet();
+  int i = 0;
+  for (; i + 2 * PF <= n && i + PF + 2 < n; i += PF) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      store_a(ar[(j + 1) & 1], (j + 1) & 1);
+      load_a(ar[(j + 1) & 1], i + j + 3);
+      mul(wr[j], j & 1);
+      load_w(wr[j], i + j + PF);
+      meet();
+    }
+  }
+  for (; i < n; i += PF) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j)
+      if (i + j < n) {
+        if (i + j + 1 < n) store_a(ar[(j + 1) & 1], (j + 1) & 1);
+        if (i + j + 3 < n) load_a(ar[(j + 1) & 1], i + j + 3);
+        mul(wr[j], j & 1);
+        if (i + j + PF < n) load_w(wr[j], i + j + PF);
+        meet();
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int m = t * 16 + lq, col = n0 + 4 * la;
+    if (m < m_rows && col < n_total)  // n_total % 4 == 0
+      *reinterpret_cast<f32x4*>(
+          part + ((int64_t)blockIdx.y * m_rows + m) * n_total + col) = acc[t];
+  }
+}
+
+// out = the sum of the splits (+ bias), 4 columns a thread.
+__global__ __launch_bounds__(256) void stream_sum_kernel(
+    bf16* __restrict__ out, const float* __restrict__ part,
+    const bf16* __restrict__ bias, const int64_t total, const int n_total,
+    const int splits) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= total) return;
+  f32x4 s = sum_parts4(part + i, total, splits);
+  ushort4v o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    o[r] = float_to_bf16_bits(
+        s[r] + (bias ? bf16_bits_to_float(bias[i % n_total + r]) : 0.f));
+  *reinterpret_cast<ushort4v*>(out + i) = o;
+}
+
 }  // namespace arks
 
 using namespace arks;
@@ -203,4 +327,40 @@ extern "C" void arks_stream_gemm(void* out, const void* a, const void* w,
   }
 #undef ARKS_SG_O
 #undef ARKS_SG
+}
+
+// part [splits, m, n] fp32; m <= 64, n % 4 == 0, k % 64 == 0. Up to 32 rows
+// chunks of 128 columns where K has them: 3584 x 18944, 32 rows 28.9 us, 64 of
+// them 30.2.
+extern "C" void arks_stream_split(void* part, const void* a, const void* w,
+                                  int m, int n, int k, int64_t a_stride,
+                                  int splits, hipStream_t stream) {
+#define ARKS_SS(MT, KC, PF)                                                    \
+  hipLaunchKernelGGL((stream_split_kernel<MT, KC, PF>),                        \
+                     dim3((n + 127) / 128, splits), dim3(512), 0, stream,      \
+                     (float*)part, (const bf16*)a, (const bf16*)w, m, n, k,    \
+                     a_stride, splits)
+  const bool wide = k % 128 == 0 && splits <= k / 128;
+  switch ((m + 15) / 16) {
+    case 1:
+      if (wide) ARKS_SS(1, 128, 2);
+      else ARKS_SS(1, 64, 4);
+      break;
+    case 2:
+      if (wide) ARKS_SS(2, 128, 2);
+      else ARKS_SS(2, 64, 4);
+      break;
+    case 3: ARKS_SS(3, 64, 4); break;
+    default: ARKS_SS(4, 64, 4); break;
+  }
+#undef ARKS_SS
+}
+
+extern "C" void arks_stream_sum(void* out, const void* part, const void* bias,
+                                int64_t m, int n, int splits,
+                                hipStream_t stream) {
+  const int64_t total = m * n;
+  hipLaunchKernelGGL(stream_sum_kernel, dim3((total / 4 + 255) / 256),
+                     dim3(256), 0, stream, (bf16*)out, (const float*)part,
+                     (const bf16*)bias, total, n, splits);
 }

@@ -191,7 +191,8 @@ class RowParallelLinear(nn.Module):
 
     fp8 = False
 
-    def forward(self, x) -> torch.Tensor:
+    def forward(self, x, parts: bool = False):
+        """parts: the caller takes ops.Parts too (one rank, no bias)."""
         if isinstance(x, tuple) or self.fp8:
             bias = self.bias
             self.bias = None  # bias must be applied post-reduce, once
@@ -203,6 +204,8 @@ class RowParallelLinear(nn.Module):
         else:
             from .. import ops
 
+            if parts and get_tp_world_size() == 1 and self.bias is None:
+                return ops.linear_parts(x, self.weight)
             y = ops.linear_bf16(x, self.weight)
         y = tp_all_reduce(y)
         if self.bias is not None:

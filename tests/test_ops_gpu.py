@@ -885,7 +885,8 @@ def test_rope_and_cache_head_norms(hq, hkv, hd, fp8):
     (1, 1, 32, False), (3, 30, 96, True), (16, 64, 64, True), (9, 4608, 3584, True),
     (17, 3584, 1056, False), (32, 4608, 512, True), (2, 544, 4096, False),
     (1, 3584, 18944, False), (5, 16400, 4096, False), (4, 16400, 2048, False),
-    (16, 33000, 2048, False),
+    (16, 33000, 2048, False), (64, 1536, 1536, True), (33, 100, 2080, False),
+    (48, 8200, 1024, True),
 ])
 def test_stream_gemm(M, N, K, bias):
     """Few-row product vs fp64: both outputs, half chunks, ends of tiles."""
@@ -937,7 +938,7 @@ def test_streams_refuses():
     assert not ops._streams(x.float(), w)
     assert not ops._streams(x[:, :40], w[:, :40].contiguous())  # K % 32
     assert not ops._streams(x, w.t())
-    assert not ops._streams(x.expand(9, 4, 64).reshape(36, 64), w)
+    assert not ops._streams(x.expand(17, 4, 64).reshape(68, 64), w)
     assert not ops._streams(x, torch.empty(65 * 64, dtype=x.dtype, device=DEV)[1:4097].view(64, 64))
     buf = torch.randn(4, 70, dtype=torch.bfloat16, device=DEV)
     odd = buf[:, 3:67]  # rows off 16 bytes are copied
@@ -981,3 +982,90 @@ def test_extend_short_portions(hd, hq, hkv, window):
                                   num_q_heads=28)
     assert many[1].numel() == 0 and many[0].shape[0] == 16
     assert ops.build_extend_tiles([33], [3000], True, q.device)[1].numel() == 0
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 544, 8192), (16, 4, 64 * 1600 + 64), (17, 130 * 4, 8192), (40, 2048, 4096),
+    (49, 4608, 3584), (64, 3584, 18944), (33, 100, 3008), (9, 1000, 17 * 1024),
+])
+def test_split_product(M, N, K):
+    """K split over workgroups vs fp64: every row tile, ends of the columns,
+    chunks of 64 and 128, as many splits as chunks; the sums and the norm and
+    rotation that add them."""
+    assert_native()
+    torch.manual_seed(N + K)
+    x = torch.randn(M, 2 * K, dtype=torch.bfloat16, device=DEV)[:, :K]
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV)
+    assert not ops._streams(x, w) and ops._splits(x, w)
+    parts = ops.linear_parts(x, w, b)
+    xd, wd = x.double().cpu(), w.double().cpu()
+    expect = xd @ wd.t()
+    # fp32 sums of K products: within K * 2^-24 of sum |x w|
+    slack = K * 2 ** -24 * (xd.abs() @ wd.abs().t())
+    assert ((parts.sums.double().sum(0).cpu() - expect).abs() <= slack).all()
+    expect = expect + b.double().cpu()
+    out = ops.linear_bf16(x, w, b).double().cpu()
+    assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs()).all()
+    if N % 8:
+        return
+    res = torch.randn(M, N, dtype=torch.bfloat16, device=DEV)
+    nw = torch.randn(N, dtype=torch.bfloat16, device=DEV)
+    total = parts.sums.double().sum(0).cpu() + res.double().cpu()
+    normed, res = ops.fused_add_rmsnorm(ops.Parts(parts.sums), res, nw, 1e-6)
+    assert ((res.double().cpu() - total).abs()
+            <= 1e-5 + 2 ** -8 * total.abs()).all()
+    want = ref.rmsnorm(res.double().cpu(), nw.double().cpu(), 1e-6)
+    # one rounding, and the fp32 sum of squares
+    torch.testing.assert_close(normed.double().cpu(), want.double(), atol=1e-5,
+                               rtol=2 ** -7.9)
+
+
+@pytest.mark.parametrize("hq,hkv,hd,splits,fp8,norm,bias", [
+    (28, 4, 128, 8, False, False, True), (3, 1, 64, 1, True, True, False),
+    (5, 5, 32, 16, False, True, True), (2, 1, 256, 9, True, False, True),
+    (2, 2, 24, 3, False, False, False)])
+def test_rope_and_cache_parts(hq, hkv, hd, splits, fp8, norm, bias):
+    """Split sums of the projection vs the kernel behind their rounded sum."""
+    assert_native()
+    torch.manual_seed(hd)
+    T, bs, nblocks = 9, 16, 4
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    width = (hq + 2 * hkv) * hd
+    sums = torch.randn(splits, T, width, device=DEV)
+    # sums that bf16 holds, so that both paths see the same numbers
+    qkv = sums.sum(0).bfloat16()
+    sums[0] += qkv.float() - sums.sum(0)
+    b = torch.randn(width, device=DEV).bfloat16() if bias else None
+    both = qkv.float() + (b.float() if bias else 0.0)
+    qn = kn = None
+    if norm:
+        qn, kn = (1 + torch.randn(2, hd, device=DEV) * 0.2).bfloat16()
+    cos_sin = ref.rope_cos_sin_cache(hd, 64, 10000.0).cuda()
+    pos = torch.randint(0, 64, (T,), dtype=torch.int64, device=DEV)
+    slots = torch.tensor([i * 3 if i != 4 else -1 for i in range(T)], device=DEV)
+    kc, vc = torch.zeros(2, nblocks, hkv, bs, hd, dtype=dt, device=DEV)
+    out = ops.rope_and_cache_parts(pos, ops.Parts(sums, b), kc, vc, slots,
+                                   cos_sin, hd, qn, kn, 1e-6)
+    q, k, v = both.double().cpu().split([hq * hd, hkv * hd, hkv * hd], dim=-1)
+    if norm:
+        q, k = (ref.rmsnorm(t.reshape(T, -1, hd), n.double().cpu(), 1e-6).view(T, -1)
+                for t, n in ((q, qn), (k, kn)))
+    q, k = ref.rope_apply(pos.cpu(), q, k, cos_sin.double().cpu(), hd)
+    # fp32 sums of up to 17 terms below 2^5, one rounding to bf16
+    torch.testing.assert_close(out.double().cpu(), q.double(), atol=1e-4,
+                               rtol=2 ** -8)
+    for t in range(T):
+        if t == 4:
+            continue
+        s = int(slots[t])
+        for cache, want in ((kc, k), (vc, v)):
+            # e4m3 has 3 bits behind the point, 2^-10 below its normal range
+            torch.testing.assert_close(
+                cache[s // bs, :, s % bs].double().cpu(),
+                want[t].view(hkv, hd).double(),
+                atol=2 ** -10 if fp8 else 1e-4, rtol=2 ** -3.9 if fp8 else 2 ** -8)
+    free = torch.ones(nblocks * bs, dtype=torch.bool)
+    free[slots[slots >= 0].cpu()] = False
+    flat = kc.float().cpu().transpose(1, 2).reshape(nblocks * bs, -1)
+    assert (flat[free] == 0).all()
