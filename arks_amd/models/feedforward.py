@@ -12,12 +12,11 @@ constants as constructor parameters:
   highest single scores stay eligible; the chosen scores are renormalised.
   The gate|up matrices of all experts are stacked in ONE [experts * 2ff,
   width] matrix in the checkpoint's own [out, in] layout; the down matrices
-  are kept pre-transposed ([in, out] per expert) like the framework's other
-  sparse feed-forward (models/llama_family.py MoEMLP). Two execution paths
-  as there: up to DENSE_TOKENS rows every expert runs on every row — one
-  linear() for all gate|up projections (no per-expert copies of the rows),
-  one batched GEMM down — with data-independent shapes, so the step can be
-  captured; above it the (row, expert) pairs are sorted by expert and every
+  are kept pre-transposed ([in, out] per expert), the right operands of
+  batched products. Two execution paths: up to DENSE_TOKENS rows every expert
+  runs on every row — one linear() for all gate|up projections (no
+  per-expert copies of the rows), one batched GEMM down — with
+  data-independent shapes, so the step can be captured; above it the (row, expert) pairs are sorted by expert and every
   expert runs plain GEMMs on its own segment (its row block of the stacked
   matrix).
 - RoutedMoE: `experts` small silu-GLU feed-forwards of which every row
@@ -151,7 +150,7 @@ class SquaredReLU(nn.Module):
 
 
 class GroupedMoE(nn.Module):
-    DENSE_TOKENS = 256  # see models/llama_family.py MoEMLP.DENSE_TOKENS
+    DENSE_TOKENS = 256  # rows up to which a step may be captured as a graph
 
     def __init__(self, width: int, experts: int, ff: int, top: int,
                  groups: int, keep: int, dtype):
@@ -193,7 +192,7 @@ class GroupedMoE(nn.Module):
 
 
 class RoutedMoE(nn.Module):
-    DENSE_TOKENS = 256  # see models/llama_family.py MoEMLP.DENSE_TOKENS
+    DENSE_TOKENS = 256  # rows up to which a step may be captured as a graph
 
     def __init__(self, width: int, experts: int, ff: int, top: int, dtype,
                  shared_ff: int = 0, score: str = "sigmoid",

@@ -115,7 +115,8 @@ class Attention(nn.Module):
                 q.contiguous().view(-1, hd)).view(T, self.nq_local * hd)
             k = self.k_norm(
                 k.contiguous().view(-1, hd)).view(T, self.nkv_local * hd)
-            v = v.contiguous()  # reshape_and_cache wants one shared kv stride
+            # reshape_and_cache wants one shared kv stride (also of one row)
+            v = v.reshape(-1).view(T, -1)
         elif self.q_norm is not None:
             norms = dict(q_norm=self.q_norm.weight, k_norm=self.k_norm.weight,
                          eps=self.q_norm.eps)

@@ -728,6 +728,15 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0):
         _native().moe_experts(out, _rows_16b(x), w13, w2, weights, ids,
                               expert_base, moe_tile(x.shape[0], k, El))
         return out
+    if x.is_cuda and x.shape[0] <= MOE_ROUTE_ROWS:
+        # sizes the kernels do not take, in steps that may be captured: every
+        # expert over all rows, without a host read of the routing
+        out = torch.zeros(x.shape, dtype=torch.float32, device=x.device)
+        for e in range(El):
+            share = (weights * (ids == e + expert_base)).sum(-1, keepdim=True)
+            y = linear_bf16(silu_mul(linear_bf16(x, w13[e])), w2[e]).float()
+            out += torch.where(share != 0, y * share, 0.0)
+        return out.to(x.dtype)
     return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
 
 

@@ -709,6 +709,33 @@ def test_moe_experts(T, E, k, H, I, base, El, tile, skew, monkeypatch):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+def test_moe_experts_other_sizes_capture():
+    """Sizes without a kernel: few rows run without a host read, so that the
+    step can be captured; replays with other routing follow it."""
+    assert_native()
+    torch.manual_seed(3)
+    T, E, k, H, I = 5, 4, 2, 72, 40
+    x = torch.randn(T, H, device=DEV).bfloat16()
+    w13 = (torch.randn(E, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(E, H, I, device=DEV) * I ** -0.5).bfloat16()
+    ids = torch.rand(T, E, device=DEV).topk(k).indices.int()
+    w = torch.rand(T, k, device=DEV)
+    ops.moe_experts(x, w13, w2, w, ids)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.moe_experts(x, w13, w2, w, ids)
+    for _ in range(3):
+        ids.copy_(torch.rand(T, E, device=DEV).topk(k).indices)
+        graph.replay()
+        torch.cuda.synchronize()
+        expect = ref.moe_experts(x.double().cpu(), w13.double().cpu(),
+                                 w2.double().cpu(), w.cpu(), ids.cpu())
+        # three roundings to bf16 behind the activation's own two
+        err = (out.double().cpu() - expect.double()).norm()
+        assert err <= 5 * 2 ** -8 * expect.double().norm()
+
+
 @pytest.mark.parametrize("T,E,k,H", [(1, 128, 8, 2048), (17, 60, 4, 512),
                                      (64, 130, 16, 64), (256, 1024, 2, 1088)])
 def test_moe_route(T, E, k, H):
@@ -852,8 +879,13 @@ def test_rope_and_cache_fused_matches_two_step(fp8):
 def test_rope_and_cache_head_norms(hq, hkv, hd, fp8):
     """Head norms inside the rotation vs norm, rotation and cache in fp64."""
     assert_native()
+    for T in (9, 1):
+        check_head_norms(T, hq, hkv, hd, fp8)
+
+
+def check_head_norms(T, hq, hkv, hd, fp8):
     torch.manual_seed(hd)
-    T, bs, nblocks = 9, 16, 4
+    bs, nblocks = 16, 4
     dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
     qkv = torch.randn(T, (hq + 2 * hkv) * hd, dtype=torch.bfloat16, device=DEV)
     q, k, v = qkv.split([hq * hd, hkv * hd, hkv * hd], dim=-1)
