@@ -139,9 +139,10 @@ __global__ __launch_bounds__(256) void moe_mix_rows_kernel(
     base[threadIdx.x] = (int64_t)rows[(int64_t)t * k + j] * H;
   }
   __syncthreads();
-  // 8 rows' loads at a time; rows of weight 0 count as nothing (they may
-  // hold anything)
-  if (H % 8 == 0) {
+  // 8 rows' loads at a time, of 16 bytes where rows start there; rows of
+  // weight 0 count as nothing (they may hold anything)
+  if (H % 8 == 0 &&
+      (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out)) % 16 == 0) {
     for (int h = threadIdx.x * 8; h < H; h += 256 * 8) {
       float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       for (int j0 = 0; j0 < k; j0 += 8) {

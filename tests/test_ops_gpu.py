@@ -790,6 +790,10 @@ def test_moe_mix_rows_zero_weights(H, k):
     # one rounding to bf16 after an fp32 sum
     torch.testing.assert_close(out.double().cpu(), expect.double(),
                                atol=1e-5, rtol=2 ** -8)
+    # rows that start on 4 bytes only
+    buf = torch.empty(R * H + 2, dtype=torch.bfloat16, device=DEV)
+    shifted = buf[2:].view(R, H).copy_(y)
+    assert torch.equal(ops.moe_mix_rows(shifted, w, rows), out)
 
 
 def test_one_shot_allreduce_single_device():
