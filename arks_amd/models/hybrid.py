@@ -520,6 +520,8 @@ class HybridForCausalLM(nn.Module):
                 continue  # layer weight_owner(i)'s module and tensors
             for k, v in layer.weight_map().items():
                 self._wmap[f"l{i}.{k}"] = v
+        if cfg.num_local_experts:
+            ops.fix_sums((*self.parameters(), *self.buffers()))
         self._loaded: set = set()
         self.residual_tap = None  # tests/tools: called with (layer, x)
 

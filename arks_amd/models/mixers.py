@@ -91,6 +91,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
     """x @ w^T (+ b) as a library GEMM (the decode-shaped bf16 cases go to
     the streamed kernels when the main extension is built)."""
     if x.dtype == torch.bfloat16:
+        if getattr(w, "fixed_sums", False):
+            return ops.linear_fixed(x, w, b)
         return ops.linear_bf16(x, w, b)
     return F.linear(x, w, b)
 
@@ -103,9 +105,10 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     fp32 accumulate, no rounding of the result)."""
     if x.dtype == torch.float32:
         return F.linear(x, w)
-    out = ops.linear_f32_rows(x, w)
-    if out is not None:
-        return out
+    if not getattr(w, "fixed_sums", False):
+        out = ops.linear_f32_rows(x, w)
+        if out is not None:
+            return out
     if _MM_OUT_DTYPE.get(x.device.type, True):
         try:
             return torch.mm(x, w.t(), out_dtype=torch.float32)

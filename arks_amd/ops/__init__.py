@@ -608,6 +608,48 @@ def linear_bf16(x, weight, bias=None):
     return F.linear(x, weight, bias)
 
 
+def _fixed_run(M: int, N: int, K: int) -> int:
+    """Columns of K that one sum of a fixed product takes (0: a library
+    product): 512 sums of 64 weight rows in all, of at least 256 columns;
+    beyond 48 rows 448 where K > N, which takes tall weights too."""
+    if N % 64 or K % 32:
+        return 0
+    tiles, tall = N // 64, K > N and M > 48
+    if N * K > (80_000_000 if tall else _SKINNY_MAX_ELEMS):
+        return 0
+    if tall and tiles < 128:
+        splits = -(-448 // tiles)
+    else:
+        splits = 1 if tiles >= 384 else -(-512 // tiles)
+    splits = min(splits, -(-K // 256))
+    return -(-(-(-K // splits)) // 32) * 32
+
+
+def fix_sums(weights) -> None:
+    """Has linear_fixed take the products of these parameters."""
+    for w in weights:
+        w.fixed_sums = True
+
+
+def linear_fixed(x, weight, bias=None):
+    """x weight^T (+ bias) whose order of sums follows from the weight alone up
+    to 48 rows, for models that choose experts. Near a tie between two of them
+    the last bits of a row decide, and with the expert its logits move (up to
+    0.2 of their norm in 3 layers of 16 experts): the choice must not turn with
+    the number of rows that share a step. linear_bf16 picks its kernel, and so
+    the order, by the rows."""
+    M, (N, K) = x.shape[0], weight.shape
+    per = _fixed_run(M, N, K) if _few_rows(x, weight) else 0
+    if per:
+        sums = torch.empty((-(-K // per), M, N), dtype=torch.float32,
+                           device=x.device)
+        _native().stream_split(sums, _rows_16b(x), weight, per)
+        return parts_sum(Parts(sums, bias))
+    import torch.nn.functional as F
+
+    return F.linear(x, weight, bias)
+
+
 def linear_f32_rows(x, weight):
     """x weight^T in fp32 (bf16 operands) where the streamed product takes it,
     else None."""

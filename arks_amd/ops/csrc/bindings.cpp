@@ -86,7 +86,8 @@ void arks_stream_gemm(void* out, const void* a, const void* w, const void* bias,
                       int m, int n, int k, int64_t a_stride, int mt, int nf,
                       int wv, int f32, int silu, hipStream_t stream);
 void arks_stream_split(void* part, const void* a, const void* w, int m, int n,
-                       int k, int64_t a_stride, int splits, hipStream_t stream);
+                       int k, int64_t a_stride, int splits, int per,
+                       hipStream_t stream);
 void arks_stream_sum(void* out, const void* part, const void* bias, int64_t m,
                      int n, int splits, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
@@ -577,8 +578,10 @@ void stream_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
                    f32 ? 1 : 0, silu ? 1 : 0, current_stream());
 }
 
-// part [splits, M, N] fp32: the sums of a [M, K] w [N, K]^T over runs of K
-void stream_split(torch::Tensor part, torch::Tensor a, torch::Tensor w) {
+// part [splits, M, N] fp32: the sums of a [M, K] w [N, K]^T over runs of K,
+// even ones (per 0) or of per columns, the last of what is left
+void stream_split(torch::Tensor part, torch::Tensor a, torch::Tensor w,
+                  int64_t per) {
   check_bf16_rowstrided(a, "a");
   check_bf16_contig(w, "w");
   TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && part.dim() == 3);
@@ -586,12 +589,17 @@ void stream_split(torch::Tensor part, torch::Tensor a, torch::Tensor w) {
   check_rows_16b(w, "w");
   check_parts(part);
   const int64_t M = a.size(0), N = w.size(0), K = a.size(1);
+  const int64_t splits = part.size(0);
   TORCH_CHECK(w.size(1) == K && part.size(1) == M && part.size(2) == N);
-  TORCH_CHECK(M >= 1 && M <= 64 && K % 64 == 0 && N < (1 << 30),
-              "need at most 64 rows and K % 64 == 0");
-  TORCH_CHECK(part.size(0) <= K / 64, "more splits than chunks");
+  TORCH_CHECK(M >= 1 && M <= 64 && N < (1 << 30) && K < (1 << 30),
+              "need at most 64 rows");
+  TORCH_CHECK(per == 0 ? K % 64 == 0 && splits <= K / 64
+                       : per > 0 && per % 32 == 0 && K % 32 == 0 &&
+                             (splits - 1) * per < K && K <= splits * per,
+              "splits do not fit the columns");
   arks_stream_split(part.data_ptr(), a.data_ptr(), w.data_ptr(), (int)M, (int)N,
-                    (int)K, a.stride(0), (int)part.size(0), current_stream());
+                    (int)K, a.stride(0), (int)splits, (int)per,
+                    current_stream());
 }
 
 void stream_sum(torch::Tensor out, torch::Tensor part,
@@ -704,7 +712,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm_parts", &fused_add_rmsnorm_parts);
   m.def("rope_and_cache_parts", &rope_and_cache_parts);
   m.def("stream_gemm", &stream_gemm);
-  m.def("stream_split", &stream_split);
+  m.def("stream_split", &stream_split, pybind11::arg("part"),
+        pybind11::arg("a"), pybind11::arg("w"), pybind11::arg("per") = 0);
   m.def("stream_sum", &stream_sum);
   m.def("moe_experts", &moe_experts);
   m.def("mfma_probe", &mfma_probe);

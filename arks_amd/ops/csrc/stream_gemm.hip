@@ -170,11 +170,13 @@ __global__ __launch_bounds__(WV * 64) void stream_gemm_kernel(
 // 3584 x 18944 (136 MB) in 8 splits: 8 rows 27 us, 64 rows 34 us, and 3 us
 // for the sums where no consumer adds them; with barriers that drain the loads
 // and 64 weight rows a workgroup 40 and 5 us, in the library 33 and 50 us.
+// run: chunks of KC that a split takes, the last what is left; 0: even splits.
 template <int MT, int KC, int PF>
 __global__ __launch_bounds__(512) void stream_split_kernel(
     float* __restrict__ part, const bf16* __restrict__ a,
     const bf16* __restrict__ w, const int m_rows, const int n_total,
-    const int k_total, const int64_t a_stride, const int splits) {
+    const int k_total, const int64_t a_stride, const int splits,
+    const int run) {
   static_assert(PF % 2 == 0, "buffers alternate over a round");
   constexpr int S = KC / 32, CPR = KC / 8, ITEMS = MT * 16 * CPR;
   constexpr int AI = (ITEMS + 511) / 512;
@@ -184,8 +186,11 @@ __global__ __launch_bounds__(512) void stream_split_kernel(
   const int lq = lane % 16, la = lane / 16;
   const int n0 = (blockIdx.x * 8 + wave) * 16;
   const int chunks = k_total / KC;
-  const int first = (int)((int64_t)chunks * blockIdx.y / splits);
-  const int n = (int)((int64_t)chunks * (blockIdx.y + 1) / splits) - first;
+  const int first = run > 0 ? blockIdx.y * run
+                            : (int)((int64_t)chunks * blockIdx.y / splits);
+  const int n = run > 0 ? min(run, chunks - first)
+                        : (int)((int64_t)chunks * (blockIdx.y + 1) / splits) -
+                              first;
   f32x4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -329,30 +334,41 @@ extern "C" void arks_stream_gemm(void* out, const void* a, const void* w,
 #undef ARKS_SG
 }
 
-// part [splits, m, n] fp32; m <= 64, n % 4 == 0, k % 64 == 0. Up to 32 rows
-// chunks of 128 columns where K has them: 3584 x 18944, 32 rows 28.9 us, 64 of
-// them 30.2.
+// part [splits, m, n] fp32; m <= 64, n % 4 == 0. per 0: even splits, k % 64
+// == 0; else columns of a split, k % 32 == per % 32 == 0 and (splits - 1) * per
+// < k <= splits * per. Up to 32 rows chunks of 128 columns where K has them:
+// 3584 x 18944, 32 rows 28.9 us, 64 of them 30.2.
 extern "C" void arks_stream_split(void* part, const void* a, const void* w,
                                   int m, int n, int k, int64_t a_stride,
-                                  int splits, hipStream_t stream) {
+                                  int splits, int per, hipStream_t stream) {
 #define ARKS_SS(MT, KC, PF)                                                    \
   hipLaunchKernelGGL((stream_split_kernel<MT, KC, PF>),                        \
                      dim3((n + 127) / 128, splits), dim3(512), 0, stream,      \
                      (float*)part, (const bf16*)a, (const bf16*)w, m, n, k,    \
-                     a_stride, splits)
-  const bool wide = k % 128 == 0 && splits <= k / 128;
+                     a_stride, splits, per / KC)
+  const int kc = per == 0 ? (k % 128 == 0 && splits <= k / 128 ? 128 : 64)
+                 : (k | per) % 128 == 0 ? 128
+                 : (k | per) % 64 == 0  ? 64
+                                        : 32;
+#define ARKS_SS_M(MT)                                                          \
+  do {                                                                         \
+    if (kc == 32) ARKS_SS(MT, 32, 8);                                          \
+    else if (kc == 128) ARKS_SS(MT, 128, 2);                                   \
+    else ARKS_SS(MT, 64, 4);                                                   \
+  } while (0)
   switch ((m + 15) / 16) {
-    case 1:
-      if (wide) ARKS_SS(1, 128, 2);
-      else ARKS_SS(1, 64, 4);
+    case 1: ARKS_SS_M(1); break;
+    case 2: ARKS_SS_M(2); break;
+    case 3:
+      if (kc == 32) ARKS_SS(3, 32, 8);
+      else ARKS_SS(3, 64, 4);
       break;
-    case 2:
-      if (wide) ARKS_SS(2, 128, 2);
-      else ARKS_SS(2, 64, 4);
+    default:
+      if (kc == 32) ARKS_SS(4, 32, 8);
+      else ARKS_SS(4, 64, 4);
       break;
-    case 3: ARKS_SS(3, 64, 4); break;
-    default: ARKS_SS(4, 64, 4); break;
   }
+#undef ARKS_SS_M
 #undef ARKS_SS
 }
 

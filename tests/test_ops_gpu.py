@@ -1105,3 +1105,39 @@ def test_rope_and_cache_parts(hq, hkv, hd, splits, fp8, norm, bias):
     free[slots[slots >= 0].cpu()] = False
     flat = kc.float().cpu().transpose(1, 2).reshape(nblocks * bs, -1)
     assert (flat[free] == 0).all()
+
+
+@pytest.mark.parametrize("N,K", [(4096, 4096), (6144, 1536), (4096, 512),
+                                 (128, 1056), (512, 4160), (3072, 4096),
+                                 (2560, 3488), (32768, 96)])
+def test_fixed_products(N, K):
+    """Products of models that choose experts: a row's sums are the same bits
+    for any number of rows in the step, the runs of K added in order (run
+    lengths of 128, 64 and 32, short last ones), and right vs fp64."""
+    assert_native()
+    torch.manual_seed(N + K)
+    x = torch.randn(64, 2 * K, dtype=torch.bfloat16, device=DEV)[:, :K]
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV)
+    per = ops._fixed_run(48, N, K)
+    assert per and per == ops._fixed_run(1, N, K)
+    ends = [*range(per, K, per), K]
+    # each run alone, as one even split (columns past its end are zeros)
+    total = torch.zeros(64, N, device=DEV)
+    for end in ends:
+        lo = end - per if end % per == 0 else end - end % per
+        xs = torch.zeros(64, -(-per // 64) * 64, dtype=x.dtype, device=DEV)
+        ws = torch.zeros(N, xs.shape[1], dtype=x.dtype, device=DEV)
+        xs[:, :end - lo], ws[:, :end - lo] = x[:, lo:end], w[:, lo:end]
+        one = torch.empty(1, 64, N, device=DEV)
+        ops._native().stream_split(one, xs, ws)
+        total += one[0]
+    want = (total + b.float()).bfloat16()
+    exact = x.double().cpu() @ w.double().cpu().t() + b.double().cpu()
+    # fp32 sums of K products, one rounding to bf16
+    slack = K * 2 ** -24 * (x.double().abs().cpu() @ w.double().abs().cpu().t())
+    assert ((want.double().cpu() - exact).abs()
+            <= 2 * slack + 2 ** -8 * exact.abs()).all()
+    for m in (1, 2, 5, 16, 17, 25, 32, 33, 48, 49, 64):
+        if ops._fixed_run(m, N, K) == per:
+            assert torch.equal(ops.linear_fixed(x[:m], w, b), want[:m]), m

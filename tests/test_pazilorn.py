@@ -1005,3 +1005,46 @@ def test_captured_decode_steps_equal_eager_ones(tmp_path):
         got[eager] = replay(eng, tmp_path, steps)
     for c in ("a", "b"):
         assert rel_err(got[False][c], got[True][c]) < 2e-2
+
+
+@pytest.mark.parametrize("name,fixed", [("tiny-pazilorn", True),
+                                        ("tiny-fuzelorn", True),
+                                        ("tiny-gagorax", False)])
+def test_products_of_models_that_choose_experts(name, fixed, monkeypatch):
+    """Their order of sums must not turn with the rows of a step."""
+    from arks_amd import ops
+    from arks_amd.config import PRESET_CONFIGS
+    from arks_amd.models import mixers
+    from arks_amd.models.hybrid import HybridForCausalLM
+
+    model = HybridForCausalLM(PRESET_CONFIGS[name])
+    calls = []
+    monkeypatch.setattr(ops, "linear_fixed",
+                        lambda x, w, b=None: calls.append("fixed") or x)
+    monkeypatch.setattr(ops, "linear_bf16",
+                        lambda x, w, b=None: calls.append("rows") or x)
+    monkeypatch.setattr(ops, "linear_f32_rows",
+                        lambda x, w: calls.append("rows"))
+    weights = [p for p in (*model.parameters(), *model.buffers())
+               if p.dim() == 2 and p.dtype == torch.bfloat16]
+    for w in weights:
+        mixers.linear(torch.zeros(1, w.shape[1], dtype=w.dtype), w)
+        mixers.linear_f32(torch.zeros(1, w.shape[1], dtype=w.dtype), w)
+    if fixed:
+        assert calls == ["fixed"] * len(weights)
+    else:
+        assert calls == ["rows"] * 2 * len(weights)
+
+
+def test_fixed_runs():
+    """Runs of K of fixed products: as many for any rows of a decode step, and
+    none where they would not fit."""
+    from arks_amd import ops
+
+    for n, k, per in ((4096, 4096, 512), (6144, 1536, 256), (4096, 512, 256),
+                      (3072, 4096, 384), (32768, 96, 96)):
+        assert [ops._fixed_run(m, n, k) for m in (1, 16, 17, 48)] == [per] * 4
+    assert ops._fixed_run(64, 4096, 14336) == 2048  # tall, many rows
+    assert ops._fixed_run(48, 4096, 14336) == 0  # a library product
+    assert ops._fixed_run(1, 12576, 4096) == 0  # rows do not fill tiles of 64
+    assert ops._fixed_run(1, 4096, 4080) == 0
