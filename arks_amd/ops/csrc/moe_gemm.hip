@@ -239,6 +239,20 @@ __global__ __launch_bounds__(WV * 64) void moe_stream_kernel(
 // an item's rows and its expert's weights.
 constexpr int MT_BM = 128, MT_BN = 128, MT_BK = 64, MT_LS = MT_BK + 8;
 
+// First of the 8 columns of a row that a lane loads for the step at k0: its
+// own, or the row's first ones where K ends before them (they count as zero).
+__host__ __device__ constexpr int moe_stage_column(int k0, int sc, int k_total) {
+  return k0 + sc < k_total ? k0 + sc : 0;
+}
+constexpr bool moe_stage_columns_in_rows() {
+  for (int k = 8; k <= 4 * MT_BK; k += 8)
+    for (int k0 = 0; k0 < k; k0 += MT_BK)
+      for (int sc = 0; sc < MT_BK; sc += 8)
+        if (moe_stage_column(k0, sc, k) + 8 > k) return false;
+  return true;
+}
+static_assert(moe_stage_columns_in_rows(), "loads stay inside their rows");
+
 template <bool UP>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ a,
@@ -267,18 +281,18 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int place = item.y + min(sr + 32 * j, cnt - 1);
-    ap[j] = a + (int64_t)(UP ? perm[place] / top_k : place) * a_stride + sc;
+    ap[j] = a + (int64_t)(UP ? perm[place] / top_k : place) * a_stride;
     // UP: rows of a wave's half are 32 gate rows, then their 32 up rows
     const int r = sr + 32 * j;
     const int n = UP ? min(n0 + r / 64 * 32 + r % 32, n_out - 1) +
                            (r / 32 % 2) * n_out
                      : min(n0 + r, n_out - 1);
-    wp[j] = w + (int64_t)item.x * w_expert + (int64_t)n * w_stride + sc;
+    wp[j] = w + (int64_t)item.x * w_expert + (int64_t)n * w_stride;
   }
   ushort8 ar[4], wr[4];
   auto load = [&](int k0) {
     const bool in = k0 + sc < k_total;  // the last 64 may be half there
-    const int o = in ? k0 : 0;
+    const int o = moe_stage_column(k0, sc, k_total);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       ar[j] = *reinterpret_cast<const ushort8*>(ap[j] + o);

@@ -675,6 +675,7 @@ def test_moe_mix_matches_einsum():
     (5, 8, 1, 64, 32, 4, 4, 16, False),
     (50, 8, 2, 256, 64, 0, 8, 16, True),      # many items of one expert
     (300, 16, 4, 96, 224, 0, 16, 128, False),  # tiles over the ends of N
+    (40, 4, 2, 32, 32, 0, 4, 128, False),     # K below a step of 64
     (500, 8, 2, 256, 64, 0, 8, 128, True),
     (7, 128, 8, 256, 96, 8, 100, 128, False),
     (65, 16, 8, 64, 32, 0, 16, None, False),  # either side of the rule
