@@ -635,13 +635,14 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   TORCH_CHECK(w13.size(1) == 2 * I && w13.size(2) == H && w2.size(0) == El &&
                   w2.size(1) == H,
               "expert weights do not fit");
-  TORCH_CHECK(H % 32 == 0 && I % 32 == 0 && El <= 1024 && k <= 16,
-              "need H % 32 == 0, I % 32 == 0, at most 1024 experts, k <= 16");
+  TORCH_CHECK(tile == 16 || tile == 128);
+  TORCH_CHECK((H | I) % (tile == 16 ? 32 : 8) == 0 && El <= 1024 && k <= 16,
+              "need H and I % 8 == 0 (tile 16: % 32), at most 1024 experts, "
+              "k <= 16");
   TORCH_CHECK(weights.scalar_type() == torch::kFloat32 &&
               weights.is_contiguous() && ids.scalar_type() == torch::kInt32 &&
               ids.is_contiguous() && ids.size(0) == T && ids.size(1) == k &&
               weights.size(0) == T);
-  TORCH_CHECK(tile == 16 || tile == 128);
   if (T == 0) return;
   const int64_t max_items = std::min(P, El) + P / tile;
   TORCH_CHECK(max_items <= 65535 || tile == 128, "too many rows for this tile");

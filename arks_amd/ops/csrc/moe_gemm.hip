@@ -377,7 +377,8 @@ extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
                      pairs, expert_base, n_local, tile, max_items);
 }
 
-// tile: pairs of an item, 16 (streamed) or 128 (tiles through LDS).
+// tile: pairs of an item, 16 (streamed; n_out % 32 == k_total % 32 == 0) or 128
+// (tiles through LDS; n_out % 8 == k_total % 8 == 0).
 extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
                               const void* perm, const void* items,
                               const void* n_items, int64_t a_stride,
@@ -395,11 +396,9 @@ extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
     if (up) {
       if (k_total >= 1024) ARKS_STREAM(2, 8, true);
       else ARKS_STREAM(2, 4, true);
-    } else if (n_out % 32 == 0) {
+    } else {
       if (k_total >= 4096) ARKS_STREAM(2, 8, false);
       else ARKS_STREAM(2, 4, false);
-    } else {
-      ARKS_STREAM(1, 4, false);
     }
   } else {
     const int cols = up ? MT_BN / 2 : MT_BN;

@@ -676,6 +676,8 @@ def test_moe_mix_matches_einsum():
     (50, 8, 2, 256, 64, 0, 8, 16, True),      # many items of one expert
     (300, 16, 4, 96, 224, 0, 16, 128, False),  # tiles over the ends of N
     (40, 4, 2, 32, 32, 0, 4, 128, False),     # K below a step of 64
+    (3, 4, 2, 8, 8, 0, 4, None, False),       # other sizes: tiles at any T
+    (300, 12, 3, 200, 72, 4, 5, None, False),
     (500, 8, 2, 256, 64, 0, 8, 128, True),
     (7, 128, 8, 256, 96, 8, 100, 128, False),
     (65, 16, 8, 64, 32, 0, 16, None, False),  # either side of the rule
@@ -711,8 +713,8 @@ def test_moe_experts(T, E, k, H, I, base, El, tile, skew, monkeypatch):
 
 
 def test_moe_experts_other_sizes_capture():
-    """Sizes without a kernel: few rows run without a host read, so that the
-    step can be captured; replays with other routing follow it."""
+    """Sizes that the streamed kernel does not take, in a captured step (no
+    host read); replays with other routing follow it."""
     assert_native()
     torch.manual_seed(3)
     T, E, k, H, I = 5, 4, 2, 72, 40
