@@ -259,7 +259,7 @@ class MoEMLP(nn.Module):
         weights, selected = ops.moe_route(x, self.gate, self.top_k,
                                           self.norm_topk)
         out = ops.moe_experts(x, self.w_up, self.w_down, weights, selected,
-                              self.expert_base)
+                              self.expert_base, self.num_experts)
         out = tp_all_reduce(out)
         if self.shared is not None:
             gate = torch.sigmoid(

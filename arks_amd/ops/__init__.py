@@ -754,14 +754,18 @@ def moe_tile(rows: int, top_k: int, experts: int) -> int:
     """Pairs of one work item (moe_gemm.hip): weights streamed under 16 of them
     up to 8 pairs per expert on the mean, 128 x 128 tiles beyond. 128 experts
     of 2048 x 768, 8 per row, us: 7 rows 96 (tiles 134), 128 rows 241 (250),
-    200 rows 268 (252), 512 rows 493 (270)."""
+    200 rows 268 (252), 512 rows 493 (270). experts: those that the rows choose
+    from, of all ranks (16 of the 128 here: 17 rows 59 (75), 128 rows 70 (87),
+    512 rows 91 (90))."""
     return 16 if rows * top_k <= 8 * experts else 128
 
 
-def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0):
+def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
+                experts: int | None = None):
     """sum_j weights[t, j] * expert(ids[t, j])(x[t]) over the silu-GLU experts
     w13 [El, 2I, H] (gate rows, then up rows), w2 [El, H, I]; experts outside
-    [expert_base, expert_base + El) contribute nothing (another rank's)."""
+    [expert_base, expert_base + El) contribute nothing (another rank's).
+    experts: the number on all ranks (None: El)."""
     El, H, I = w13.shape[0], w13.shape[2], w2.shape[2]
     k = ids.shape[1]
     if (x.is_cuda and x.dtype == torch.bfloat16 and H % 8 == 0
@@ -770,7 +774,7 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0):
         # the streamed kernel takes whole matrix operands of 32 columns only
         # (16 experts of 2056 x 1416, 4 per row, 7 rows, with routing: 95 us
         # in tiles, 120 us as batched products)
-        tile = moe_tile(x.shape[0], k, El) if (H | I) % 32 == 0 else 128
+        tile = moe_tile(x.shape[0], k, experts or El) if (H | I) % 32 == 0 else 128
         _native().moe_experts(out, _rows_16b(x), w13, w2, weights, ids,
                               expert_base, tile)
         return out

@@ -712,6 +712,36 @@ def test_moe_experts(T, E, k, H, I, base, El, tile, skew, monkeypatch):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+def test_moe_tile_of_a_rank(monkeypatch):
+    """A rank's share of the experts takes the kernel that their total number
+    asks for: its share of the pairs is as small."""
+    assert_native()
+    import dataclasses
+
+    from arks_amd.config import PRESET_CONFIGS
+    from arks_amd.models import llama_family
+
+    cfg = dataclasses.replace(PRESET_CONFIGS["tiny-moe"], num_local_experts=128,
+                              num_experts_per_tok=8, hidden_size=64,
+                              moe_intermediate_size=32)
+    with monkeypatch.context() as m:
+        m.setattr(llama_family, "get_tp_world_size", lambda: 8)
+        moe = llama_family.MoEMLP(cfg).to(DEV)
+    assert moe.local_experts == 16
+    for p in moe.parameters():
+        p.data.normal_()
+    tiles, rule = [], ops.moe_tile
+
+    def record(*a):
+        tiles.append(rule(*a))
+        return tiles[-1]
+
+    monkeypatch.setattr(ops, "moe_tile", record)
+    for rows in (17, 128, 129):
+        moe(torch.randn(rows, 64, device=DEV).bfloat16())
+    assert tiles == [16, 16, 128]
+
+
 def test_moe_experts_other_sizes_capture():
     """Sizes that the streamed kernel does not take, in a captured step (no
     host read); replays with other routing follow it."""
