@@ -97,24 +97,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
     return F.linear(x, w, b)
 
 
-_MM_OUT_DTYPE = {}  # device type -> torch.mm(..., out_dtype=) available
-
-
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T with fp32 OUTPUT from rows of the model's dtype (bf16 inputs,
     fp32 accumulate, no rounding of the result)."""
-    if x.dtype == torch.float32:
-        return F.linear(x, w)
-    if not getattr(w, "fixed_sums", False):
+    if x.dtype != torch.float32 and not getattr(w, "fixed_sums", False):
         out = ops.linear_f32_rows(x, w)
         if out is not None:
             return out
-    if _MM_OUT_DTYPE.get(x.device.type, True):
-        try:
-            return torch.mm(x, w.t(), out_dtype=torch.float32)
-        except (TypeError, RuntimeError):
-            _MM_OUT_DTYPE[x.device.type] = False
-    return F.linear(x, w).float()
+    return ops.linear_f32_lib(x, w)
 
 
 def step_chunks(batch: ForwardBatch, device, chunk: int = 0):

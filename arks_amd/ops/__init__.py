@@ -658,6 +658,32 @@ def linear_f32_rows(x, weight):
     return None
 
 
+_MM_OUT_DTYPE = {}  # device type -> torch.mm(..., out_dtype=) available
+
+
+def _mm_out_dtype(x) -> bool:
+    ok = _MM_OUT_DTYPE.get(x.device.type)
+    if ok is None:
+        try:
+            one = x.new_zeros(16, 16)
+            torch.mm(one, one, out_dtype=torch.float32)
+            ok = True
+        except (TypeError, RuntimeError):
+            ok = False
+        _MM_OUT_DTYPE[x.device.type] = ok
+    return ok
+
+
+def linear_f32_lib(x, weight):
+    """x weight^T in fp32 as a library product: 16-bit operands, fp32 sums, no
+    rounding of the result where torch.mm has such a product."""
+    import torch.nn.functional as F
+
+    if x.dtype != torch.float32 and _mm_out_dtype(x):
+        return torch.mm(x, weight.t(), out_dtype=torch.float32)
+    return F.linear(x, weight).float()
+
+
 def linear_silu_mul(x, weight):
     """silu_mul(x weight^T), weight [2N, K] the gate rows, then the up rows."""
     if x.dim() == 2 and weight.shape[0] % 2 == 0 and _streams(x, weight, True):
@@ -730,14 +756,15 @@ def moe_topk(router_logits, k: int, renorm: bool):
     return ref.moe_topk(router_logits, k, renorm)
 
 
-# Rows up to which one kernel does the whole routing (a workgroup per row reads
-# the router's weights, 0.5 MB from L2); beyond, a GEMM for all rows is faster.
+# Rows up to which the router's logits come from the streamed product, which
+# reads 16 rows of the gate a workgroup; beyond, the library's is faster.
 MOE_ROUTE_ROWS = 256
 
 
 def moe_route(x, gate, k: int, renorm: bool):
-    """moe_topk of the router product x gate^T (fp32 logits up to
-    MOE_ROUTE_ROWS rows, rounded to x's type beyond)."""
+    """moe_topk of the router product x gate^T, its logits fp32 at any number
+    of rows: rounded ones tie, and the choice of a row must not turn with the
+    step that it runs in."""
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= MOE_ROUTE_ROWS
             and x.shape[1] % 32 == 0 and gate.is_contiguous()
             and gate.data_ptr() % 16 == 0):
@@ -745,9 +772,7 @@ def moe_route(x, gate, k: int, renorm: bool):
                              device=x.device)
         _native().stream_gemm(logits, _rows_16b(x), gate, None, 1, 1, 16, False)
         return moe_topk(logits, k, renorm)
-    import torch.nn.functional as F
-
-    return moe_topk(F.linear(x, gate).float(), k, renorm)
+    return moe_topk(linear_f32_lib(x, gate), k, renorm)
 
 
 def moe_tile(rows: int, top_k: int, experts: int) -> int:

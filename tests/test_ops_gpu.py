@@ -770,9 +770,11 @@ def test_moe_experts_other_sizes_capture():
 
 
 @pytest.mark.parametrize("T,E,k,H", [(1, 128, 8, 2048), (17, 60, 4, 512),
-                                     (64, 130, 16, 64), (256, 1024, 2, 1088)])
+                                     (64, 130, 16, 64), (256, 1024, 2, 1088),
+                                     (257, 128, 8, 2048), (3000, 60, 4, 512),
+                                     (5, 16, 4, 72)])
 def test_moe_route(T, E, k, H):
-    """Router product and choice of few rows vs fp64."""
+    """Router product and choice vs fp64, either side of the row limit."""
     assert_native()
     torch.manual_seed(E)
     x = torch.randn(T, H, device=DEV).bfloat16()
