@@ -21,10 +21,12 @@ from ..config import ModelConfig
 from ..engine.forward_batch import ForwardBatch
 from ..parallel.comm import get_tp_rank, get_tp_world_size
 from ..parallel.layers import (
+    ColumnParallelLinear,
     MergedColumnParallelLinear,
     ParallelLMHead,
     QKVParallelLinear,
     RowParallelLinear,
+    passable,
 )
 
 
@@ -80,16 +82,20 @@ class Attention(nn.Module):
             RMSNorm(cfg.head_dim, cfg.rms_norm_eps, dtype) if cfg.qk_norm else None
         )
 
-    def forward(self, x, batch: ForwardBatch, kv_cache) -> torch.Tensor:
+    def forward(self, x, batch: ForwardBatch, kv_cache, parts: bool = False):
+        """parts: the caller takes ops.Parts too."""
         T = (x[0] if isinstance(x, tuple) else x).shape[0]
-        # in decode steps k and v are read from the cache alone, and the
-        # norms behind the two row-parallel products can add split sums
-        decode = not batch.is_prefill
-        if (decode and self.use_rope and not isinstance(x, tuple)
+        # the rotation kernel can norm the heads of q and k
+        rope_norms = (self.use_rope and self.q_norm is not None
+                      and self.head_dim in ops.HEAD_NORM_DIMS
+                      and passable(self.q_norm, RMSNorm)
+                      and passable(self.k_norm, RMSNorm))
+        # in decode steps k and v are read from the cache alone
+        if (not batch.is_prefill and self.use_rope and not isinstance(x, tuple)
                 and not self.qkv_proj.fp8
-                and (self.q_norm is None
-                     or self.head_dim in ops.HEAD_NORM_DIMS)
-                and self.head_dim % 8 == 0):
+                and (self.q_norm is None or rope_norms)
+                and self.head_dim % 8 == 0
+                and passable(self.qkv_proj, ColumnParallelLinear)):
             qkv = ops.linear_parts(x, self.qkv_proj.weight, self.qkv_proj.bias)
         else:
             qkv = self.qkv_proj(x)
@@ -100,16 +106,13 @@ class Attention(nn.Module):
             q = ops.rope_and_cache_parts(
                 batch.positions, qkv, kv_cache[0], kv_cache[1],
                 batch.slot_mapping, self._cos_sin, self.head_dim, **norms)
-            return self.o_proj(self._decode(q, batch, kv_cache).view(T, -1),
-                               parts=True)
+            return self._out(self._decode(q, batch, kv_cache).view(T, -1), parts)
         # Strided views into the fused QKV buffer — RoPE/cache/attention
         # kernels take row strides, so no .contiguous() copies on the hot path.
         q, k, v = self.qkv_proj.split_qkv(qkv)
         k_cache, v_cache = kv_cache
         norms = {}
-        if self.q_norm is not None and not (
-                self.use_rope and (not q.is_cuda
-                                   or self.head_dim in ops.HEAD_NORM_DIMS)):
+        if self.q_norm is not None and not rope_norms:
             hd = self.head_dim
             q = self.q_norm(
                 q.contiguous().view(-1, hd)).view(T, self.nq_local * hd)
@@ -152,7 +155,10 @@ class Attention(nn.Module):
                 )
         else:
             out = self._decode(q, batch, kv_cache)
-        return self.o_proj(out.view(T, -1), parts=decode)
+        return self._out(out.view(T, -1), parts)
+
+    def _out(self, x, parts: bool):
+        return self.o_proj(x, parts=True) if parts else self.o_proj(x)
 
     def _decode(self, q, batch: ForwardBatch, kv_cache):
         k_cache, v_cache = kv_cache
@@ -180,11 +186,12 @@ class MLP(nn.Module):
     def forward(self, x, parts: bool = False):
         if self.fp8:
             return self.down_proj(ops.silu_mul_fp8(self.gate_up_proj(x)))
-        if isinstance(x, tuple) or self.gate_up_proj.fp8:
+        if (isinstance(x, tuple) or self.gate_up_proj.fp8
+                or not passable(self.gate_up_proj, ColumnParallelLinear)):
             h = ops.silu_mul(self.gate_up_proj(x))
         else:
             h = ops.linear_silu_mul(x, self.gate_up_proj.weight)
-        return self.down_proj(h, parts=parts)
+        return self.down_proj(h, parts=True) if parts else self.down_proj(h)
 
 
 class MoEMLP(nn.Module):
@@ -253,7 +260,7 @@ class MoEMLP(nn.Module):
     # need no host read of the routing at any size)
     DENSE_TOKENS = 256
 
-    def forward(self, x, parts: bool = False):
+    def forward(self, x):
         from ..parallel.comm import tp_all_reduce
 
         weights, selected = ops.moe_route(x, self.gate, self.top_k,
@@ -280,16 +287,27 @@ class DecoderLayer(nn.Module):
             MoEMLP(cfg, dtype) if cfg.num_local_experts > 0 else MLP(cfg, dtype)
         )
 
-    def forward(self, x, residual, batch: ForwardBatch, kv_cache):
+    def forward(self, x, residual, batch: ForwardBatch, kv_cache,
+                parts: bool = False):
+        """parts: the caller takes ops.Parts too."""
         if residual is None:
             residual = x
             x = self.input_layernorm(x)
         else:
             x, residual = self.input_layernorm(x, residual)
-        x = self.self_attn(x, batch, kv_cache)
+        # the norm behind a row-parallel product of a decode step can add its
+        # split sums; what a hook may look at stays a tensor
+        if (not batch.is_prefill and passable(self.self_attn, Attention)
+                and passable(self.self_attn.o_proj, RowParallelLinear)
+                and passable(self.post_attention_layernorm, RMSNorm)):
+            x = self.self_attn(x, batch, kv_cache, parts=True)
+        else:
+            x = self.self_attn(x, batch, kv_cache)
         x, residual = self.post_attention_layernorm(x, residual)
-        x = self.mlp(x, parts=not batch.is_prefill)
-        return x, residual
+        if (parts and passable(self.mlp, MLP)
+                and passable(self.mlp.down_proj, RowParallelLinear)):
+            return self.mlp(x, parts=True), residual
+        return self.mlp(x), residual
 
 
 class LlamaFamilyForCausalLM(nn.Module):
@@ -367,8 +385,18 @@ class LlamaFamilyForCausalLM(nn.Module):
         batch.step_cache = {}
         x = self.embed_tokens(batch.input_ids)
         residual = None
+        last = len(self.layers) - 1
         for i, layer in enumerate(self.layers):
-            x, residual = layer(x, residual, batch, kv_caches[i])
+            parts = not batch.is_prefill and passable(layer, DecoderLayer)
+            if parts and i < last:
+                after = self.layers[i + 1]
+                parts = (passable(after, DecoderLayer)
+                         and passable(after.input_layernorm, RMSNorm))
+            elif parts:
+                parts = passable(self.norm, RMSNorm)
+            x, residual = (layer(x, residual, batch, kv_caches[i], parts=True)
+                           if parts else
+                           layer(x, residual, batch, kv_caches[i]))
         x, _ = self.norm(x, residual)
         if isinstance(x, tuple):  # fp8: (values, per-token scales)
             q8, sc = x

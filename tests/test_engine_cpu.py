@@ -492,3 +492,64 @@ def test_smollm3_nope_engine_decode_matches_prefill():
     full = prompts[0] + out1[0][:-1]
     out3 = e2.generate([full], SamplingParams(max_tokens=1, ignore_eos=True))
     assert out3[0][0] == out1[0][-1]
+
+
+def hooked_calls(engine, prompts, params):
+    """(tokens, hooked modules that a decode step did not call), every module
+    under a forward hook that takes tensors alone."""
+    model = engine.runner.model
+    called = set()
+
+    def tensors(v):
+        if isinstance(v, (tuple, list)):
+            return all(tensors(e) for e in v)
+        return not type(v).__name__ == "Parts"
+
+    def see(name):
+        def hook(module, args, out):
+            assert tensors(args) and tensors(out), name
+            called.add(name)
+        return hook
+
+    names = [n for n, m in model.named_modules()
+             if not isinstance(m, torch.nn.ModuleList)]
+    for n in names:
+        model.get_submodule(n).register_forward_hook(see(n))
+    for p in prompts:
+        engine.add_request(p, params)
+    engine.step()  # prompts
+    called.clear()
+    tokens = [o.new_token_id for o in engine.step()]
+    return tokens, set(names) - called
+
+
+@pytest.mark.parametrize("preset,device", [
+    ("tiny", "cpu"), ("tiny-qwen3", "cpu"),
+    pytest.param("tiny-gpu", "cuda", marks=pytest.mark.gpu),
+    pytest.param("qwen3-gpu", "cuda", marks=pytest.mark.gpu)])
+def test_forward_hooks_see_every_module(preset, device, monkeypatch):
+    """Products that are fused with their neighbours run as the modules that
+    they are where a hook stands on them, with the same tokens."""
+    import dataclasses
+
+    from arks_amd import config
+
+    monkeypatch.setitem(config.PRESET_CONFIGS, "qwen3-gpu", dataclasses.replace(
+        config.PRESET_CONFIGS["tiny-gpu"], architecture="Qwen3ForCausalLM",
+        qk_norm=True, attention_bias=False))
+    prompts = [[1, 5, 9, 20], [3, 3, 7]]
+    sp = SamplingParams(max_tokens=8, ignore_eos=True)
+
+    def make():
+        return LLMEngine(EngineConfig(
+            preset=preset, device=device, kv_cache_blocks=64, max_model_len=512,
+            enforce_eager=True, seed=3))
+
+    plain = make()
+    for p in prompts:
+        plain.add_request(p, sp)
+    plain.step()
+    expect = [o.new_token_id for o in plain.step()]
+    got, missed = hooked_calls(make(), prompts, sp)
+    assert not missed
+    assert got == expect
