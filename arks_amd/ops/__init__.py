@@ -360,16 +360,26 @@ def attention_extend_paged(
     )
 
 
+def _of_step(step_cache: dict, key, inputs: tuple, make):
+    """What make() gives for these tensors: made once per forward pass
+    (step_cache), and again for other ones or after they were written."""
+    state = [0 if t.is_inference() else t._version for t in inputs]
+    held = step_cache.get(key)
+    if (held is None or held[1] != state
+            or any(a is not b for a, b in zip(held[0], inputs))):
+        held = step_cache[key] = (inputs, state, make())
+    return held[2]
+
+
 def _single_rows(block_tables, kv_lens, dseqs, num_kv_heads: int, window: int,
                  kv_fp8: bool, planned: bool, native,
                  step_cache: dict | None):
     """(block tables, lengths, decode plan) of the single rows of a mixed
-    batch: the same for all layers of a forward pass (step_cache)."""
+    batch: shared by the layers of a forward pass (step_cache)."""
     cache = {} if step_cache is None else step_cache
-    if "single_rows" not in cache:
-        cache["single_rows"] = (block_tables[dseqs].contiguous(),
-                                kv_lens[dseqs].contiguous())
-    dtab, dlens = cache["single_rows"]
+    dtab, dlens = _of_step(
+        cache, "single_rows", (block_tables, kv_lens, dseqs),
+        lambda: (block_tables[dseqs].contiguous(), kv_lens[dseqs].contiguous()))
     plan = (step_decode_plan(dlens, num_kv_heads, window, kv_fp8, native, cache)
             if planned else None)
     return dtab, dlens, plan
@@ -377,14 +387,14 @@ def _single_rows(block_tables, kv_lens, dseqs, num_kv_heads: int, window: int,
 
 def step_decode_plan(seq_lens, num_kv_heads: int, window: int, kv_fp8: bool,
                      native, step_cache: dict | None):
-    """attention_decode_plan, made once per forward pass (step_cache)."""
+    """attention_decode_plan, shared by the layers of a forward pass
+    (step_cache)."""
     if step_cache is None:
         return None
-    key = ("decode_plan", num_kv_heads, window, kv_fp8)
-    if key not in step_cache:
-        step_cache[key] = attention_decode_plan(seq_lens, num_kv_heads, window,
-                                                kv_fp8, native=native)
-    return step_cache[key]
+    return _of_step(
+        step_cache, ("decode_plan", num_kv_heads, window, kv_fp8), (seq_lens,),
+        lambda: attention_decode_plan(seq_lens, num_kv_heads, window, kv_fp8,
+                                      native=native))
 
 
 def decode_waves(num_seqs: int, num_kv_heads: int, kv_fp8: bool = False,

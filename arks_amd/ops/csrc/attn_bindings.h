@@ -81,7 +81,7 @@ inline void check_decode_plan(const torch::Tensor& plan, int64_t waves,
                               int64_t num_seqs) {
   TORCH_CHECK(waves >= 1 && plan.is_cuda() && plan.is_contiguous() &&
                   plan.scalar_type() == torch::kInt32 &&
-                  plan.numel() >= 4 * waves + 2 * num_seqs &&
+                  plan.numel() == 4 * waves + 2 * num_seqs &&
                   reinterpret_cast<uintptr_t>(plan.data_ptr()) % 16 == 0,
               "plan must be int32 of 4 * waves + 2 * sequences");
 }

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
     const int* __restrict__ seq_lens,      // [S]
     const int4* __restrict__ runs, const float scale, const int num_kv_heads,
     const int max_blocks, const int64_t q_stride, const int window,
-    const int sink, const int waves) {
+    const int sink, const int waves, const int num_seqs) {
   constexpr int NUM_WAVES = 4;
   constexpr int STEPS = HEAD_DIM / 32;   // QK^T contraction steps
   constexpr int CHUNKS = HEAD_DIM / 16;  // PV output dim chunks
@@ -414,8 +414,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
     left -= n;
     if (left == 0) return;
     off = 0;
-    do {  // the next sequence with a key
-      ++seq;
+    do {  // the next sequence with a key (the bound: a plan of other lengths)
+      if (++seq >= num_seqs) return;
       L = __builtin_amdgcn_readfirstlane(seq_lens[seq]);
     } while (L <= 0);
   }
@@ -497,12 +497,12 @@ void launch_decode_gq(bf16* out, float* part_out, const bf16* q,
       hipLaunchKernelGGL((attn_decode_kernel<HEAD_DIM, G, true>),             \
                          dim3(blocks), dim3(256), 0, stream, out, part_out,   \
                          q, kc, vc, bt, sl, runs, scale, num_kv_heads,        \
-                         max_blocks, q_stride, window, sink, waves);          \
+                         max_blocks, q_stride, window, sink, waves, num_seqs);\
     } else {                                                                  \
       hipLaunchKernelGGL((attn_decode_kernel<HEAD_DIM, G, false>),            \
                          dim3(blocks), dim3(256), 0, stream, out, part_out,   \
                          q, kc, vc, bt, sl, runs, scale, num_kv_heads,        \
-                         max_blocks, q_stride, window, sink, waves);          \
+                         max_blocks, q_stride, window, sink, waves, num_seqs);\
     }                                                                         \
     break;
   switch (gq) {

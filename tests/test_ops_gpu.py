@@ -241,6 +241,20 @@ def test_attention_decode_runs(hq, hkv, hd, lens, window, partitions, fp8):
     torch.testing.assert_close(out.float().cpu(), expect, atol=2.4e-2, rtol=0)
 
 
+def test_attention_decode_plan_size():
+    """A plan for another number of sequences or runs is refused."""
+    assert_native()
+    q = torch.zeros(3, 2, 64, dtype=torch.bfloat16, device=DEV)
+    kc = torch.zeros(4, 1, 16, 64, dtype=torch.bfloat16, device=DEV)
+    bt = torch.zeros(3, 1, dtype=torch.int32, device=DEV)
+    lens = torch.tensor([3, 1, 9], dtype=torch.int32, device=DEV)
+    for plan in (ops.attention_decode_plan(lens[:2].contiguous(), 1),
+                 ops.attention_decode_plan(torch.cat([lens, lens]), 1),
+                 ops.attention_decode_plan(lens, 1, num_partitions=2)):
+        with pytest.raises(RuntimeError, match="plan"):
+            ops.attention_decode_paged(q, kc, kc, bt, lens, 1.0, plan=plan)
+
+
 def test_attention_decode_fp8_codes():
     """Every e4m3 code reads as its own value."""
     assert_native()

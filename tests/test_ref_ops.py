@@ -94,3 +94,36 @@ def test_rope_scaling_matches_transformers():
     mine2, ms2 = _scaled_inv_freq(base2, yarn, 10000.0, 128)
     torch.testing.assert_close(mine2, inv_hf2.double(), rtol=1e-5, atol=0)
     assert abs(ms2 - att2) < 1e-9
+
+
+def test_step_results_follow_their_inputs(monkeypatch):
+    """What the layers of a pass share belongs to the lengths, tables and rows
+    that it was made from."""
+    import arks_amd.ops as ops
+
+    made = []
+
+    def plan(lens, *a, **kw):
+        made.append(lens.tolist())
+        return tuple(lens.tolist())
+
+    monkeypatch.setattr(ops, "attention_decode_plan", plan)
+    cache = {}
+    a, b = torch.tensor([5, 9]), torch.tensor([7, 1])
+    get = lambda lens: ops.step_decode_plan(lens, 4, 0, False, None, cache)
+    assert get(a) == get(a) == (5, 9) and len(made) == 1
+    assert get(b) == (7, 1) and get(a) == (5, 9)
+    a.add_(1)
+    assert get(a) == (6, 10)
+    with torch.inference_mode():
+        c = torch.tensor([3])
+        assert get(c) == (3,)
+    tables, lens = torch.arange(12).view(3, 4), torch.tensor([10, 20, 30])
+    rows = lambda pick: ops._single_rows(tables, lens, torch.tensor(pick), 4, 0,
+                                         False, True, None, cache)
+    for pick in ([0, 2], [1], [0, 2]):
+        tab, n, p = rows(pick)
+        assert torch.equal(tab, tables[pick]) and n.tolist() == list(p)
+        assert p == tuple(lens[pick].tolist())
+    lens.mul_(2)
+    assert rows([0, 2])[2] == (20, 60)
