@@ -202,7 +202,7 @@ def build_extend_tiles(q_lens: list[int], kv_lens: list[int] | None,
     # and 39, 8 x 33 rows 77 and 71, 16 x 33 rows (more than one workgroup per
     # CU) 83 and 107.
     short = [i for i, n in enumerate(q_lens)
-             if n < min_ladder and not (n == 1 and flash_decode)]
+             if 0 < n < min_ladder and not (n == 1 and flash_decode)]
     few = (ladder and not kv_fp8
            and sum(-(-q_lens[i] // PREFILL_QTILE) for i in short) * num_q_heads
            <= 256)
@@ -223,22 +223,31 @@ def build_extend_tiles(q_lens: list[int], kv_lens: list[int] | None,
         [x[:2] for x in t], dtype=torch.int32, device=device
     ).reshape(-1, 2)
 
-    # KV-split policy for the 256-row kernel: when tiles x heads cannot
-    # fill ~2 workgroups per CU, split the deepest tiles' key ranges.
-    base_wgs = len(t256) * max(num_q_heads, 1)
-    factor = 1
-    if t256 and base_wgs < 256:
+    # KV-split policy for the 256-row kernel: when the long portions' tiles x
+    # heads cannot fill ~2 workgroups per CU, split the deepest tiles' key
+    # ranges. Short portions are here to be split also beside enough others,
+    # unless those walk as many keys. 28/4 heads: 2560 rows beside 65 at 6113 keys 156 us
+    # (unsplit 364, in the 64-row kernel 530), beside 33 at 1000 keys 125 (117).
+    def parts(tiles: int) -> int:
         # truly starved launches only (256 CUs, 1 block/CU kernel): the
         # partial slabs + combine cost ~2x slab traffic, so marginal
         # shortfalls are better left unsplit
-        factor = min(8, -(-512 // base_wgs))
+        wgs = tiles * max(num_q_heads, 1)
+        return min(8, -(-512 // wgs)) if 0 < wgs < 256 else 1
+
+    long = [k for i, _, k in t256 if i not in deep]
+    factor = parts(len(long))
+    deep_factor = max(2, parts(len(t256) - len(long)))
+    longest = max(long, default=0)
     rows, combine = [], []
     ws_rows = 0
-    if factor > 1:
+    if factor > 1 or deep:
         split, plain = [], []
         for (i, q0, kmax) in t256:
             span = (kmax + E2_KVBLK - 1) // E2_KVBLK
-            p = min(factor, max(1, span // 4))
+            most = (deep_factor if i in deep and (factor > 1 or kmax > longest)
+                    else factor)
+            p = min(most, max(1, span // 4))
             (split if p > 1 else plain).append((i, q0, p))
         # cap the f32 partial workspace at ~512 MB
         slab = num_q_heads * EXTEND2_QTILE * 130 * 4

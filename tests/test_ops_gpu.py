@@ -1069,6 +1069,36 @@ def test_extend_short_portions(hd, hq, hkv, window):
     assert ops.build_extend_tiles([33], [3000], True, q.device)[1].numel() == 0
 
 
+def test_extend_short_portions_beside_long_ones():
+    """The cut of a short portion in a launch that long portions fill."""
+    assert_native()
+    torch.manual_seed(9)
+    hq, hkv, hd = 32, 2, 64
+    qlens, kvs = [2048, 40, 300], [2048, 3001, 700]
+    pages = [-(-n // 16) for n in kvs]
+    kc = torch.randn(sum(pages), hkv, 16, hd, device=DEV).bfloat16()
+    vc = torch.randn_like(kc)
+    bt = torch.zeros(len(kvs), max(pages), dtype=torch.int32)
+    for i, n in enumerate(pages):
+        bt[i, :n] = torch.arange(sum(pages[:i]), sum(pages[:i]) + n)
+    q = torch.randn(sum(qlens), hq, hd, device=DEV).bfloat16()
+    lens = torch.tensor(kvs, dtype=torch.int32)
+    cu = torch.tensor([0] + qlens).cumsum(0).int()
+    tiles = ops.build_extend_tiles(qlens, kvs, False, q.device, num_q_heads=hq)
+    assert tiles[3].tolist() == [[0, 8, 1, 0]]  # the short one's parts
+    out = ops.attention_extend_paged(q, kc, vc, bt.to(DEV), lens.to(DEV),
+                                     cu.to(DEV), qlens, hd ** -0.5, tiles=tiles)
+    args = (bt, lens, cu, hd ** -0.5)
+    expect = ref.attention_extend_paged(
+        q.float().cpu(), kc.float().cpu(), vc.float().cpu(), *args)
+    # the weights and the sum are each rounded to bf16 once, each by at most
+    # 2^-8 of itself (8 bits): 2^-8 of sum p |v| and of the sum
+    spread = ref.attention_extend_paged(
+        q.float().cpu(), kc.float().cpu(), vc.float().abs().cpu(), *args)
+    assert ((out.float().cpu() - expect).abs()
+            <= 2 ** -8 * (spread + expect.abs()) + 1e-5).all()
+
+
 @pytest.mark.parametrize("M,N,K", [
     (1, 544, 8192), (16, 4, 64 * 1600 + 64), (17, 130 * 4, 8192), (40, 2048, 4096),
     (49, 4608, 3584), (64, 3584, 18944), (33, 100, 3008), (9, 1000, 17 * 1024),

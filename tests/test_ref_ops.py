@@ -127,3 +127,29 @@ def test_step_results_follow_their_inputs(monkeypatch):
         assert p == tuple(lens[pick].tolist())
     lens.mul_(2)
     assert rows([0, 2])[2] == (20, 60)
+
+
+def test_short_portions_are_split_beside_long_ones():
+    """A short portion behind a deep context is cut over its keys also where
+    long portions fill the chip, and leaves their own cut as it was."""
+    from arks_amd.ops import build_extend_tiles
+
+    def split(q, kv, **kw):
+        t64, t256, _, combine, ws = build_extend_tiles(
+            q, kv, False, "cpu", num_q_heads=28, **kw)
+        rows = t256.tolist()
+        assert ws == sum(r[3] > 1 for r in rows)
+        for at, n, i, q0 in combine.tolist():
+            assert rows[at:at + n] == [[i, q0, p, n] for p in range(n)]
+        return {i: max(r[3] for r in rows if r[0] == i)
+                for i in {r[0] for r in rows}}, t64.shape[0]
+
+    assert split([2560, 65], [2560, 6113]) == ({0: 1, 1: 8}, 0)
+    assert split([2560, 65], [2560, 600]) == ({0: 1, 1: 1}, 0)  # none waits
+    assert split([2560, 65], [2560, 200]) == ({0: 1}, 2)  # 64-row kernel
+    assert split([2560], [2560]) == ({0: 1}, 0)
+    # 8 x 28 workgroups are cut in 3, also with 2 x 28 of short portions
+    assert split([2048], [2048])[0] == {0: 3}
+    assert split([2048, 33, 33], [2048, 3000, 3000])[0] == {0: 3, 1: 8, 2: 8}
+    assert split([65], [6113])[0] == {0: 8}
+    assert split([0, 65], [400, 6113], min_ladder=1)[0] == {1: 8}
