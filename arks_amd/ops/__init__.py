@@ -522,19 +522,32 @@ def _stream_split(M: int, N: int):
     return (mt, 1, 4) if M <= 4 else (mt, 2, 16)
 
 
-def _few_rows(x, weight) -> bool:
-    """Whether the kernels of stream_gemm.hip can take x weight^T."""
+def _plain(*tensors) -> bool:
+    """Whether kernels may take these past autograd: no gradient, tangent or
+    transform (vmap) of theirs is followed."""
+    if torch.autograd.forward_ad._current_level >= 0:
+        return False
+    grad = torch.is_grad_enabled()
+    return not any(
+        type(t) not in (torch.Tensor, torch.nn.Parameter)
+        or torch._C._functorch.is_functorch_wrapped_tensor(t)
+        or (grad and t.requires_grad) for t in tensors if t is not None)
+
+
+def _few_rows(x, weight, bias=None) -> bool:
+    """Whether the kernels of stream_gemm.hip can take x weight^T (+ bias)."""
     return (_USE_SKINNY and x.is_cuda and x.dim() == 2
             and 1 <= x.shape[0] <= 64
             and x.dtype == weight.dtype == torch.bfloat16
             and weight.shape[1] % 32 == 0
+            and _plain(x, weight, bias)
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0
-            and not (torch.is_grad_enabled()
-                     and (x.requires_grad or weight.requires_grad))
+            and (bias is None or (bias.dtype == x.dtype
+                                  and bias.is_contiguous()))
             and native_available())
 
 
-def _streams(x, weight, silu: bool = False) -> bool:
+def _streams(x, weight, silu: bool = False, bias=None) -> bool:
     """Whether x weight^T takes stream_gemm. A workgroup reads all of x's rows
     beside its 16 or 32 weight rows, so the line lies where that traffic (rows
     x K), and the waves' tails, meet what the other path loses: us, here
@@ -546,7 +559,7 @@ def _streams(x, weight, silu: bool = False) -> bool:
     rows 62.0 (62.5); 151936 x 2048, 16 rows 134 (206), 32 rows 167 (149);
     37888 x 3584, 1 row 52.9 (53.2), 8 rows 58.7 (53.1), with the activation
     57.8 (59); 3584 x 18944, 1 row 30.3 (32.5), 4 rows 33.4 (32.6)."""
-    if not _few_rows(x, weight):
+    if not _few_rows(x, weight, bias):
         return False
     M, (N, K) = x.shape[0], weight.shape
     if N * K <= _SKINNY_MAX_ELEMS:
@@ -556,14 +569,14 @@ def _streams(x, weight, silu: bool = False) -> bool:
     return M <= 16 and (K <= 2048 or (K <= 4096 and N * K <= 1 << 27))
 
 
-def _splits(x, weight) -> bool:
+def _splits(x, weight, bias=None) -> bool:
     """Whether x weight^T splits K over workgroups (asked after _streams):
     weights up to _SKINNY_MAX_ELEMS, and larger ones that are tall. us with
     the sums (library): 3584 x 18944, 4 rows 30.7 (32.6), 32 rows 31.7 (43.9),
     64 rows 36.8 (49.6); 8192 x 28672, 8 rows 88.5 (91.8), 64 rows 108 (154);
     wide ones, as 16384 x 4096 at 32 rows, 36 (34)."""
     N, K = weight.shape
-    return (_few_rows(x, weight) and K % 64 == 0 and N % 4 == 0
+    return (_few_rows(x, weight, bias) and K % 64 == 0 and N % 4 == 0
             and (N * K <= _SKINNY_MAX_ELEMS or K >= 2 * N))
 
 
@@ -609,7 +622,8 @@ def _stream_gemm(x, weight, bias=None, dtype=None, silu: bool = False):
 
 def linear_parts(x, weight, bias=None):
     """linear_bf16 for a consumer that takes Parts."""
-    if x.dim() == 2 and not _streams(x, weight) and _splits(x, weight):
+    if (x.dim() == 2 and not _streams(x, weight, bias=bias)
+            and _splits(x, weight, bias)):
         return Parts(_stream_parts(x, weight), bias)
     return linear_bf16(x, weight, bias)
 
@@ -618,9 +632,9 @@ def linear_bf16(x, weight, bias=None):
     """Linear dispatch: the streamed product for few rows, K split over
     workgroups for other small decode-shaped and tall GEMMs on GPU, hipBLASLt
     (F.linear) otherwise."""
-    if x.dim() == 2 and _streams(x, weight):
+    if x.dim() == 2 and _streams(x, weight, bias=bias):
         return _stream_gemm(x, weight, bias)
-    if x.dim() == 2 and _splits(x, weight):
+    if x.dim() == 2 and _splits(x, weight, bias):
         return parts_sum(Parts(_stream_parts(x, weight), bias))
     import torch.nn.functional as F
 
@@ -658,7 +672,7 @@ def linear_fixed(x, weight, bias=None):
     the number of rows that share a step. linear_bf16 picks its kernel, and so
     the order, by the rows."""
     M, (N, K) = x.shape[0], weight.shape
-    per = _fixed_run(M, N, K) if _few_rows(x, weight) else 0
+    per = _fixed_run(M, N, K) if _few_rows(x, weight, bias) else 0
     if per:
         sums = torch.empty((-(-K // per), M, N), dtype=torch.float32,
                            device=x.device)

@@ -1031,6 +1031,29 @@ def test_streams_refuses():
                                atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("N,K", [(40000, 1024), (4096, 9216)])
+def test_products_that_autograd_follows(N, K):
+    """Transforms, tangents, gradients and other biases of large weights go to
+    the library product (wide: streamed, tall: split)."""
+    assert_native()
+    torch.manual_seed(K)
+    F = torch.nn.functional
+    M = 16 if N > K else 40
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV)
+    assert ops._streams(x, w) if N > K else ops._splits(x, w)
+    close = lambda a, e: torch.testing.assert_close(a, e, atol=3e-2, rtol=3e-2)
+    close(torch.func.vmap(lambda t: ops.linear_bf16(t, w))(x[None]), F.linear(x[None], w))
+    _, t = torch.func.jvp(lambda t: ops.linear_bf16(t, w, b), (x,), (x,))
+    close(t, F.linear(x, w))
+    bias = b.clone().requires_grad_()
+    ops.linear_bf16(x, w, bias).sum().backward()
+    close(bias.grad, torch.full_like(b, M))
+    spread = torch.stack([b, b], 1)[:, 0]
+    close(ops.linear_bf16(x, w, spread), F.linear(x, w, b))
+
+
 @pytest.mark.parametrize("hd,hq,hkv,window", [(128, 7, 1, 0), (64, 8, 4, 0),
                                               (128, 4, 2, 300)])
 def test_extend_short_portions(hd, hq, hkv, window):
