@@ -156,6 +156,7 @@ void fused_add_rmsnorm_parts(torch::Tensor out, torch::Tensor part,
                              double eps) {
   check_bf16_contig(out, "out");
   check_bf16_contig(residual, "residual");
+  check_bf16_contig(weight, "weight");
   check_parts(part);
   const int64_t hidden = part.size(2), rows = part.size(1);
   TORCH_CHECK(hidden % 8 == 0 && out.numel() == rows * hidden &&
@@ -259,15 +260,20 @@ void rope_and_cache_parts(torch::Tensor positions, torch::Tensor q,
                           torch::Tensor slot_mapping, torch::Tensor cos_sin,
                           int64_t head_dim, c10::optional<torch::Tensor> q_norm,
                           c10::optional<torch::Tensor> k_norm, double eps) {
-  TORCH_CHECK(positions.scalar_type() == torch::kInt64);
-  TORCH_CHECK(slot_mapping.scalar_type() == torch::kInt64);
-  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32);
+  for (const auto& t : {positions, slot_mapping})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+                    t.scalar_type() == torch::kInt64,
+                "positions and slots must be int64 on GPU");
+  TORCH_CHECK(cos_sin.is_cuda() && cos_sin.is_contiguous() &&
+                  cos_sin.scalar_type() == torch::kFloat32 &&
+                  cos_sin.size(-1) == head_dim,
+              "cos_sin must be fp32 [positions, head_dim] on GPU");
   check_bf16_contig(q, "q");
   check_parts(part);
   const int64_t T = part.size(1), width = part.size(2);
   const int nkv = k_cache.size(1), block_size = k_cache.size(2);
   TORCH_CHECK(head_dim % 8 == 0 && k_cache.size(3) == head_dim &&
-              k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              k_cache.is_cuda() && v_cache.is_cuda() && k_cache.is_contiguous() && v_cache.is_contiguous() &&
               v_cache.sizes() == k_cache.sizes());
   TORCH_CHECK(q.dim() == 2 && q.size(0) == T && q.size(1) % head_dim == 0 &&
               width == q.size(1) + 2 * nkv * head_dim &&
@@ -639,7 +645,8 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   TORCH_CHECK((H | I) % (tile == 16 ? 32 : 8) == 0 && El <= 1024 && k <= 16,
               "need H and I % 8 == 0 (tile 16: % 32), at most 1024 experts, "
               "k <= 16");
-  TORCH_CHECK(weights.scalar_type() == torch::kFloat32 &&
+  TORCH_CHECK(weights.is_cuda() && ids.is_cuda() &&
+              weights.scalar_type() == torch::kFloat32 &&
               weights.is_contiguous() && ids.scalar_type() == torch::kInt32 &&
               ids.is_contiguous() && ids.size(0) == T && ids.size(1) == k &&
               weights.size(0) == T);

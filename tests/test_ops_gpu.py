@@ -1243,3 +1243,31 @@ def test_fixed_products(N, K):
     for m in (1, 2, 5, 16, 17, 25, 32, 33, 48, 49, 64):
         if ops._fixed_run(m, N, K) == per:
             assert torch.equal(ops.linear_fixed(x[:m], w, b), want[:m]), m
+
+
+def test_host_tensors_are_refused():
+    """Tensors on the host never reach a kernel."""
+    assert_native()
+    bf = lambda *s: torch.ones(*s, dtype=torch.bfloat16, device=DEV)
+    parts = ops.Parts(torch.ones(2, 3, 96, device=DEV))
+    with pytest.raises(RuntimeError):
+        ops.fused_add_rmsnorm(parts, bf(3, 96), bf(96).cpu(), 1e-6)
+    with pytest.raises(RuntimeError):
+        ops.fused_add_rmsnorm(parts, bf(3, 96), bf(96).float(), 1e-6)
+    kc = torch.zeros(2, 1, 16, 32, dtype=torch.bfloat16, device=DEV)
+    pos, slots = torch.arange(3, device=DEV), torch.arange(3, device=DEV)
+    cs = torch.ones(8, 32, device=DEV)
+    ops.rope_and_cache_parts(pos, parts, kc, kc.clone(), slots, cs, 32)
+    for bad in ((pos.cpu(), slots, cs, kc), (pos, slots.cpu(), cs, kc),
+                (pos, slots, cs.cpu(), kc), (pos, slots, cs, kc.cpu()),
+                (pos, slots, cs.t()[:8, :8], kc)):
+        with pytest.raises(RuntimeError):
+            ops.rope_and_cache_parts(bad[0], parts, bad[3], kc.clone(), bad[1],
+                                     bad[2], 32)
+    x, w13, w2 = bf(3, 32), bf(2, 64, 32), bf(2, 32, 32)
+    w, ids = torch.ones(3, 1, device=DEV), torch.zeros(3, 1, dtype=torch.int32, device=DEV)
+    for bad in ((w.cpu(), ids), (w, ids.cpu())):
+        with pytest.raises(RuntimeError):
+            ops.moe_experts(x, w13, w2, *bad)
+    with pytest.raises(RuntimeError):
+        ops.linear_bf16(x, bf(64, 32).cpu())
