@@ -214,31 +214,54 @@ def test_attention_decode_runs(hq, hkv, hd, lens, window, partitions, fp8):
     """The runs that the decode kernel cuts the sequences into."""
     assert_native()
     torch.manual_seed(len(lens) + window)
-    S, pages = len(lens), [(n + 15) // 16 for n in lens]
-    total = sum(pages)
-    q = torch.randn(S, hq, hd, dtype=torch.bfloat16, device=DEV)
-    kc = torch.randn(total, hkv, 16, hd, device=DEV)
-    vc = torch.randn(total, hkv, 16, hd, device=DEV)
+    # keys on both sides of every unit, of a sequence's ends and of its window
+    marks = [{0, n - 1, n - window, n - window - 1} | set(range(31, n, 32))
+             | set(range(32, n, 32)) for n in lens]
+    q, kc, vc, bt = marked_pages(len(lens), hq, hkv, hd, lens, marks)
     dtype = torch.float8_e4m3fn if fp8 else torch.bfloat16
     kc, vc = kc.to(dtype), vc.to(dtype)
-    bt = torch.zeros(S, max(pages) + 2, dtype=torch.int32)
-    order, at = torch.randperm(total, dtype=torch.int32), 0
-    for i, n in enumerate(pages):
-        bt[i, :n] = order[at:at + n]
-        at += n
-    full = bt.clone()
+    held = bt.clone()
     if window:
         for i, n in enumerate(lens):
-            bt[i, :max(0, n - window) // 16] = -1
+            held[i, :max(0, n - window) // 16] = -1
     sl = torch.tensor(lens, dtype=torch.int32)
-    out = ops.attention_decode_paged(q, kc, vc, bt.to(DEV), sl.to(DEV),
-                                     hd ** -0.5, num_partitions=partitions,
-                                     window=window)
-    expect = ref.attention_decode_paged(
-        q.float().cpu(), kc.float().cpu(), vc.float().cpu(), full, sl,
-        hd ** -0.5, window)
-    # weights and result are rounded to bf16 (2^-9 each) under |v| < 6
-    torch.testing.assert_close(out.float().cpu(), expect, atol=2.4e-2, rtol=0)
+    out = ops.attention_decode_paged(
+        q.to(DEV), kc.to(DEV), vc.to(DEV), held.to(DEV), sl.to(DEV), hd ** -0.5,
+        num_partitions=partitions, window=window)
+    check_attention(out, ref.attention_decode_paged, q, kc, vc, bt, sl,
+                    hd ** -0.5, window)
+
+
+def marked_pages(rows, hq, hkv, hd, lens, marks):
+    """(q [rows], key and value pages, block tables) of sequences whose marked
+    keys have about e^5 times the weight of others for every query, so that
+    each shows in the result; rows behind a sequence's end have e^20 times."""
+    pages = [-(-n // 16) for n in lens]
+    u = torch.randn(hkv, hd)
+    u *= hd ** 0.5 / u.norm(dim=-1, keepdim=True)
+    q = (torch.randn(rows, hkv, hq // hkv, hd) + u[:, None]).view(rows, hq, hd)
+    kc, vc = torch.randn(2, sum(pages), hkv, 16, hd)
+    bt = torch.zeros(len(lens), max(pages) + 2, dtype=torch.int32)
+    order, at = torch.randperm(sum(pages), dtype=torch.int32), 0
+    for i, (n, m) in enumerate(zip(lens, marks)):
+        bt[i, :pages[i]] = order[at:at + pages[i]]
+        at += pages[i]
+        for t in m:
+            if 0 <= t < n:
+                kc[bt[i, t // 16], :, t % 16] += 5 * hd ** -0.5 * u
+        if n % 16:
+            kc[bt[i, n // 16], :, n % 16:] += 20 * hd ** -0.5 * u[:, None]
+            vc[bt[i, n // 16], :, n % 16:] = 100.0
+    return q.bfloat16(), kc.bfloat16(), vc.bfloat16(), bt
+
+
+def check_attention(out, oracle, q, kc, vc, *args):
+    """Weights and result are rounded to bf16 once, each by at most 2^-8 of
+    itself: within 2^-8 of sum p |v| and of the result."""
+    expect = oracle(q.float(), kc.float(), vc.float(), *args)
+    spread = oracle(q.float(), kc.float(), vc.float().abs(), *args)
+    err = (out.float().cpu() - expect).abs()
+    assert (err <= 2 ** -8 * (spread + expect.abs()) + 1e-5).all()
 
 
 def test_attention_decode_plan_size():
@@ -286,6 +309,33 @@ def test_greedy_sample_parts(rows, vocab):
         logits[1, vocab // 2] = logits[1, vocab // 2 + 1] = -7.0
     out = ops.greedy_sample(logits.to(DEV)).cpu()
     assert torch.equal(out, torch.from_numpy(logits.float().numpy().argmax(1)))
+
+
+@pytest.mark.parametrize("rows,vocab", [(1, 4096), (3, 20001), (64, 152064)])
+def test_gumbel_sample_parts(rows, vocab):
+    """Rows cut over workgroups at temperatures above 0, beside greedy ones:
+    the largest logit / t - log(-log u) wins."""
+    assert_native()
+    torch.manual_seed(vocab)
+    logits = (torch.randn(rows, vocab, device=DEV) * 3).bfloat16()
+    temps = 0.3 + torch.rand(rows, device=DEV)
+    temps[1::3] = 0.0
+    u = torch.rand(rows, vocab, device=DEV)
+    out = ops.sample_tokens(logits, temps, u)
+    x, t = logits.double().cpu(), temps.double().cpu()[:, None]
+    noise = -torch.log(-torch.log(u.double().cpu().clamp(min=1e-20)))
+    score = torch.where(t > 0, x / t.clamp(min=1e-9) + noise, x)
+    # fp32: 2^-22 of scores below 2^6 in all, and the logarithm's error near
+    # u = 1, where -log u keeps 2^-24 / (1 - u) of its value
+    slack = torch.where(t > 0, 2 ** -15 + 2 ** -22 / (1 - u.double().cpu()), 0.0)
+    picked = out.cpu()[:, None]
+    best = score.amax(-1, keepdim=True)
+    assert (score.gather(1, picked) + slack.gather(1, picked)
+            + slack.gather(1, score.argmax(-1, keepdim=True)) >= best).all()
+    # greedy rows: the first of the largest
+    cold = temps.cpu() == 0
+    assert torch.equal(out.cpu()[cold], torch.from_numpy(
+        logits[temps == 0].float().cpu().numpy().argmax(1)))
 
 
 def test_strided_qkv_views():
@@ -972,6 +1022,9 @@ def check_head_norms(T, hq, hkv, hd, fp8):
     (1, 3584, 18944, False), (5, 16400, 4096, False), (4, 16400, 2048, False),
     (16, 33000, 2048, False), (64, 1536, 1536, True), (33, 100, 2080, False),
     (48, 8200, 1024, True),
+    # large weights at one and two rows: a down product's columns, a head
+    (1, 1024, 57344, False), (2, 600, 57344, True), (1, 152064, 512, True),
+    (8, 152064, 512, False),
 ])
 def test_stream_gemm(M, N, K, bias):
     """Few-row product vs fp64: both outputs, half chunks, ends of tiles."""
@@ -1062,34 +1115,28 @@ def test_extend_short_portions(hd, hq, hkv, window):
     assert_native()
     torch.manual_seed(hd + hq)
     qlens, kvs = [2, 65, 1, 33, 96, 130], [256, 1501, 700, 33, 4000, 130]
-    pages = [-(-n // 16) for n in kvs]
-    kc = torch.randn(sum(pages) + 1, hkv, 16, hd, device=DEV).bfloat16()
-    vc = torch.randn_like(kc)
-    bt = torch.zeros(len(kvs), max(pages), dtype=torch.int32, device=DEV)
-    order, at = torch.randperm(sum(pages)).int() + 1, 0
-    for i, n in enumerate(pages):
-        bt[i, :n] = order[at:at + n]
-        at += n
-    q = torch.randn(sum(qlens), hq, hd, device=DEV).bfloat16()
-    lens = torch.tensor(kvs, dtype=torch.int32, device=DEV)
-    cu = torch.tensor([0] + qlens, device=DEV).cumsum(0).int()
-    tiles = ops.build_extend_tiles(qlens, kvs, False, q.device, num_q_heads=hq)
+    # keys on both sides of every tile of 64, and those of the portions' own
+    # rows: each is the last that its row sees and past the end of the others
+    marks = [{0} | set(range(63, n, 64)) | set(range(64, n, 64))
+             | set(range(n - m, n)) for m, n in zip(qlens, kvs)]
+    q, kc, vc, bt = marked_pages(sum(qlens), hq, hkv, hd, kvs, marks)
+    lens = torch.tensor(kvs, dtype=torch.int32)
+    cu = torch.tensor([0] + qlens).cumsum(0).int()
+    tiles = ops.build_extend_tiles(qlens, kvs, False, torch.device(DEV),
+                                   num_q_heads=hq)
     assert {r[0] for r in tiles[0].tolist()} == {3}  # the one without context
     assert {r[0] for r in tiles[1].tolist()} == {0, 1, 4, 5}
     assert tiles[4] > 0
-    out = ops.attention_extend_paged(q, kc, vc, bt, lens, cu, qlens, hd ** -0.5,
-                                     window=window, tiles=tiles)
-    expect = ref.attention_extend_paged(
-        q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt.cpu(),
-        lens.cpu(), cu.cpu(), hd ** -0.5, window)
-    # the weights and the sum are each rounded to bf16 once: 2^-8 of sum p |v|
-    bound = 2 ** -7 * vc.abs().max().item()
-    assert (out.float().cpu() - expect.float()).abs().max() <= bound
+    out = ops.attention_extend_paged(
+        q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), lens.to(DEV), cu.to(DEV),
+        qlens, hd ** -0.5, window=window, tiles=tiles)
+    check_attention(out, ref.attention_extend_paged, q, kc, vc, bt, lens, cu,
+                    hd ** -0.5, window)
     # many short portions keep the 64-row kernel
-    many = ops.build_extend_tiles([33] * 16, [3000] * 16, False, q.device,
+    many = ops.build_extend_tiles([33] * 16, [3000] * 16, False, torch.device(DEV),
                                   num_q_heads=28)
     assert many[1].numel() == 0 and many[0].shape[0] == 16
-    assert ops.build_extend_tiles([33], [3000], True, q.device)[1].numel() == 0
+    assert ops.build_extend_tiles([33], [3000], True, torch.device(DEV))[1].numel() == 0
 
 
 def test_extend_short_portions_beside_long_ones():
@@ -1098,28 +1145,65 @@ def test_extend_short_portions_beside_long_ones():
     torch.manual_seed(9)
     hq, hkv, hd = 32, 2, 64
     qlens, kvs = [2048, 40, 300], [2048, 3001, 700]
-    pages = [-(-n // 16) for n in kvs]
-    kc = torch.randn(sum(pages), hkv, 16, hd, device=DEV).bfloat16()
-    vc = torch.randn_like(kc)
-    bt = torch.zeros(len(kvs), max(pages), dtype=torch.int32)
-    for i, n in enumerate(pages):
-        bt[i, :n] = torch.arange(sum(pages[:i]), sum(pages[:i]) + n)
-    q = torch.randn(sum(qlens), hq, hd, device=DEV).bfloat16()
+    marks = [{0} | set(range(63, n, 64)) | set(range(64, n, 64)) for n in kvs]
+    q, kc, vc, bt = marked_pages(sum(qlens), hq, hkv, hd, kvs, marks)
     lens = torch.tensor(kvs, dtype=torch.int32)
     cu = torch.tensor([0] + qlens).cumsum(0).int()
-    tiles = ops.build_extend_tiles(qlens, kvs, False, q.device, num_q_heads=hq)
+    tiles = ops.build_extend_tiles(qlens, kvs, False, torch.device(DEV),
+                                   num_q_heads=hq)
     assert tiles[3].tolist() == [[0, 8, 1, 0]]  # the short one's parts
-    out = ops.attention_extend_paged(q, kc, vc, bt.to(DEV), lens.to(DEV),
-                                     cu.to(DEV), qlens, hd ** -0.5, tiles=tiles)
-    args = (bt, lens, cu, hd ** -0.5)
-    expect = ref.attention_extend_paged(
-        q.float().cpu(), kc.float().cpu(), vc.float().cpu(), *args)
-    # the weights and the sum are each rounded to bf16 once, each by at most
-    # 2^-8 of itself (8 bits): 2^-8 of sum p |v| and of the sum
-    spread = ref.attention_extend_paged(
-        q.float().cpu(), kc.float().cpu(), vc.float().abs().cpu(), *args)
-    assert ((out.float().cpu() - expect).abs()
-            <= 2 ** -8 * (spread + expect.abs()) + 1e-5).all()
+    out = ops.attention_extend_paged(
+        q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), lens.to(DEV), cu.to(DEV),
+        qlens, hd ** -0.5, tiles=tiles)
+    check_attention(out, ref.attention_extend_paged, q, kc, vc, bt, lens, cu,
+                    hd ** -0.5)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("maps", [1, 2])
+@pytest.mark.parametrize("sink", [False, True])
+def test_extend_short_portions_of_layer_lists(hd, maps, sink):
+    """The same split with two keys per cache row, and with a key of score 0
+    beside the others."""
+    assert ops.seq_native_available()
+    torch.manual_seed(hd + maps)
+    G, R = 2, 2
+    qlens, kvs = [40, 7], [900, 333]
+    # a cache row's keys side by side: pages of G heads of maps * hd columns
+    marks = [{0} | set(range(63, n, 64)) | set(range(64, n, 64)) for n in kvs]
+    q, kc, _, bt = marked_pages(sum(qlens), G * R, G, maps * hd, kvs, marks)
+    q = (q.view(-1, G, R, maps, hd).transpose(2, 3).reshape(-1, G * maps * R, hd)
+         .contiguous())
+    vc = torch.randn(kc.shape[0], G, 16, hd).bfloat16()
+    scale = (maps * hd) ** -0.5 * maps ** 0.5
+    lens = torch.tensor(kvs, dtype=torch.int32)
+    cu = torch.tensor([0] + qlens).cumsum(0).int()
+    tiles = ops.build_extend_tiles(qlens, kvs, False, torch.device(DEV),
+                                   num_q_heads=q.shape[1])
+    assert tiles[0].numel() == 0 and tiles[4] > 0
+    out = ops.attention_extend_paged(
+        q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), lens.to(DEV), cu.to(DEV),
+        qlens, scale, tiles=tiles, sink=sink, native=ops.seq_extension(),
+        maps=maps)
+
+    def oracle(q, kc, vc):
+        res = []
+        for i, (m, n) in enumerate(zip(qlens, kvs)):
+            rows = [t[bt[i, :-(-n // 16)].long()].transpose(1, 2).flatten(0, 1)[:n]
+                    .double() for t in (kc, vc)]
+            k = rows[0].view(n, G, maps, hd)
+            x = q[cu[i]:cu[i + 1]].double().view(m, G, maps, R, hd)
+            z = torch.einsum("mgprd,ngpd->mgprn", x, k) * scale
+            hidden = torch.arange(n) > torch.arange(n - m, n)[:, None]
+            z = z.masked_fill(hidden[:, None, None, None], -torch.inf)
+            if sink:
+                z = torch.cat([z, torch.zeros_like(z[..., :1])], -1)
+            p = torch.softmax(z, -1)[..., :n]
+            res.append(torch.einsum("mgprn,ngd->mgprd", p, rows[1])
+                       .reshape(m, G * maps * R, hd))
+        return torch.cat(res).float()
+
+    check_attention(out, oracle, q, kc, vc)
 
 
 @pytest.mark.parametrize("M,N,K", [
