@@ -520,10 +520,18 @@ class HybridForCausalLM(nn.Module):
                 continue  # layer weight_owner(i)'s module and tensors
             for k, v in layer.weight_map().items():
                 self._wmap[f"l{i}.{k}"] = v
-        if cfg.num_local_experts:
-            ops.fix_sums((*self.parameters(), *self.buffers()))
+        self._fix_sums()
         self._loaded: set = set()
         self.residual_tap = None  # tests/tools: called with (layer, x)
+
+    def _fix_sums(self) -> None:
+        if self.cfg.num_local_experts:
+            ops.fix_sums((*self.parameters(), *self.buffers()))
+
+    def _apply(self, fn, recurse=True):
+        out = super()._apply(fn, recurse)  # makes new buffers
+        self._fix_sums()
+        return out
 
     # ------------------------------------------------------------ cache
     def cache_layout(self, block_size: int) -> list:

@@ -1009,15 +1009,22 @@ def test_captured_decode_steps_equal_eager_ones(tmp_path):
 
 @pytest.mark.parametrize("name,fixed", [("tiny-pazilorn", True),
                                         ("tiny-fuzelorn", True),
+                                        ("tiny-fusolix", True),
                                         ("tiny-gagorax", False)])
-def test_products_of_models_that_choose_experts(name, fixed, monkeypatch):
-    """Their order of sums must not turn with the rows of a step."""
+@pytest.mark.parametrize("moved", [False, True])
+def test_products_of_models_that_choose_experts(name, fixed, moved, monkeypatch):
+    """Their order of sums must not turn with the rows of a step, also once
+    the model was moved (its parameters and buffers made again)."""
     from arks_amd import ops
     from arks_amd.config import PRESET_CONFIGS
     from arks_amd.models import mixers
     from arks_amd.models.hybrid import HybridForCausalLM
 
     model = HybridForCausalLM(PRESET_CONFIGS[name])
+    if moved:
+        model._apply(torch.clone)
+    assert all(getattr(t, "fixed_sums", False) == fixed
+               for t in (*model.parameters(), *model.buffers()))
     calls = []
     monkeypatch.setattr(ops, "linear_fixed",
                         lambda x, w, b=None: calls.append("fixed") or x)
