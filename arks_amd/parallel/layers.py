@@ -75,6 +75,7 @@ def passable(module, cls) -> bool:
     return (type(module).forward is cls.forward
             and "forward" not in module.__dict__
             and not module._forward_hooks and not module._forward_pre_hooks
+            and not module._backward_hooks and not module._backward_pre_hooks
             and not _has_any_global_hook())
 
 

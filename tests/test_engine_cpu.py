@@ -553,3 +553,18 @@ def test_forward_hooks_see_every_module(preset, device, monkeypatch):
     got, missed = hooked_calls(make(), prompts, sp)
     assert not missed
     assert got == expect
+
+
+def test_backward_hooks_see_a_fused_product():
+    from arks_amd import config
+    from arks_amd.models.llama_family import MLP
+
+    mlp = MLP(config.PRESET_CONFIGS["tiny"], torch.float32)
+    for p in mlp.parameters():
+        p.data.normal_(0, 0.05)
+    seen = []
+    mlp.gate_up_proj.register_full_backward_hook(
+        lambda module, gin, gout: seen.append(gin[0].shape))
+    x = torch.randn(3, mlp.gate_up_proj.in_features, requires_grad=True)
+    mlp(x).sum().backward()
+    assert seen == [x.shape] and x.grad.abs().max() > 0
