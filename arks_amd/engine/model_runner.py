@@ -372,9 +372,8 @@ class ModelRunner:
 
     # ---------------- hipGraph decode ----------------
     def _init_graph_buffers(self) -> None:
-        # round max_num_seqs up to the nearest capture size (capped at 256;
-        # MoE decode uses the dense bmm path, capture-safe through the full
-        # 256-size graph ladder)
+        # round max_num_seqs up to the nearest capture size (capped at 256,
+        # with experts at the rows that their feed-forward names)
         cap = self.GRAPH_SIZES[-1]
         if self.model_cfg.num_local_experts > 0:
             from ..models.llama_family import MoEMLP

@@ -844,9 +844,12 @@ def moe_mix(y, weights, ids, expert_base: int = 0):
     out-of-slice experts contributing 0 (TP expert parallelism)."""
     if y.is_cuda:
         El, T, H = y.shape
-        out = torch.empty(T, H, dtype=y.dtype, device=y.device)
-        _native().moe_mix(out, y.contiguous(), weights, ids, expert_base, El)
-        return out
+        assert ids.shape == weights.shape and ids.shape[0] == T
+        le = ids - expert_base
+        mine = (le >= 0) & (le < El)
+        rows = le * T + torch.arange(T, dtype=torch.int32, device=y.device)[:, None]
+        return moe_mix_rows(y.reshape(El * T, H), weights.where(mine, 0.0),
+                            rows.where(mine, 0))
     return ref.moe_mix(y, weights, ids, expert_base)
 
 

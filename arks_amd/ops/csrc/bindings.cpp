@@ -76,9 +76,6 @@ void arks_one_shot_allreduce(void* out, const void* src, void* mail_ptrs[8],
                              int world, int64_t n, hipStream_t stream);
 void arks_moe_topk(void* weights, void* ids, const void* logits, int T,
                    int E, int k, int renorm, hipStream_t stream);
-void arks_moe_mix(void* out, const void* y, const void* weights,
-                  const void* ids, int T, int H, int k, int expert_base,
-                  int n_local, hipStream_t stream);
 void arks_moe_mix_rows(void* out, const void* y, const void* weights,
                        const void* rows, int T, int H, int k,
                        hipStream_t stream);
@@ -519,21 +516,6 @@ void moe_topk(torch::Tensor weights, torch::Tensor ids,
                 (int)k, (int)renorm, current_stream());
 }
 
-void moe_mix(torch::Tensor out, torch::Tensor y, torch::Tensor weights,
-             torch::Tensor ids, int64_t expert_base, int64_t n_local) {
-  check_bf16_contig(out, "out");
-  check_bf16_contig(y, "y");
-  TORCH_CHECK(weights.scalar_type() == torch::kFloat32 &&
-              ids.scalar_type() == torch::kInt32);
-  const int T = out.size(0), H = out.size(1);
-  const int k = weights.size(1);
-  TORCH_CHECK(k <= 16 && H % 2 == 0);
-  TORCH_CHECK(y.size(1) == T && y.size(2) == H && y.size(0) == n_local);
-  arks_moe_mix(out.data_ptr(), y.data_ptr(), weights.data_ptr(),
-               ids.data_ptr(), T, H, k, (int)expert_base, (int)n_local,
-               current_stream());
-}
-
 void moe_mix_rows(torch::Tensor out, torch::Tensor y,
                   torch::Tensor weights, torch::Tensor rows) {
   check_bf16_contig(out, "out");
@@ -548,7 +530,6 @@ void moe_mix_rows(torch::Tensor out, torch::Tensor y,
                     rows.data_ptr(), T, H, k, current_stream());
 }
 
-// weights [T, k] f32 and ids [T, k] of the rows x over the router gate [E, H]
 // out [M, N] (bf16 or fp32) = a [M, K] w [N, K]^T (+ bias [N]); silu: w is
 // [2N, K] and out silu of the first N columns times the others
 void stream_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
@@ -715,7 +696,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ipc_close", &ipc_close);
   m.def("one_shot_allreduce", &one_shot_allreduce);
   m.def("moe_topk", &moe_topk);
-  m.def("moe_mix", &moe_mix);
   m.def("moe_mix_rows", &moe_mix_rows);
   m.def("fused_add_rmsnorm_parts", &fused_add_rmsnorm_parts);
   m.def("rope_and_cache_parts", &rope_and_cache_parts);

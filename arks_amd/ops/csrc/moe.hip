@@ -1,19 +1,15 @@
-// MoE routing + mixing kernels (gfx950).
+// MoE routing + mixing kernels (gfx950), around the expert products of
+// moe_gemm.hip. In torch the same steps (softmax -> topk -> renorm, then float
+// casts and an einsum for the weighted mix) are about 10 small kernels a layer.
 //
-// The dense-decode MoE path (models/llama_family.py MoEMLP.forward) is
-// weight-HBM-bound in its two expert bmms, but the torch glue around them
-// (softmax -> topk -> renorm -> scatter, then float casts + einsum for the
-// weighted mix) costs ~10 small kernels per layer — several ms per decode
-// step at batch 64-256. These two kernels replace that glue:
+//   moe_topk:      probs = softmax(logits[T,E]); per row select top-k
+//                  (ties -> lower expert id, matching torch.topk), optional
+//                  renormalization; emits (weights[T,k] f32, ids[T,k] i32).
+//   moe_mix_rows:  out[t] = sum_j w[t,j] * y[rows[t,j]], the weighted mix over
+//                  the experts' rows y [R, H].
 //
-//   moe_topk:  probs = softmax(logits[T,E]); per row select top-k
-//              (ties -> lower expert id, matching torch.topk), optional
-//              renormalization; emits (weights[T,k] f32, ids[T,k] i32).
-//   moe_mix:   out[t,h] = sum_i w[t,i] * y[ids[t,i], t, h] — the weighted
-//              gather-mix over the dense per-expert outputs y[E,T,H].
-//
-// Reference parity note: the reference delegates MoE serving to external
-// images; these kernels are runtime-slot internals.
+// The reference delegates MoE serving to external images; these kernels are
+// internals of its runtime slot.
 #include "common.h"
 
 #include <cfloat>
@@ -83,47 +79,9 @@ __global__ __launch_bounds__(64) void moe_topk_kernel(
   }
 }
 
-// Weighted mix of per-expert dense outputs: one block per token, lanes
-// stride the hidden dim; k gathered rows from y[E,T,H].
-__global__ __launch_bounds__(256) void moe_mix_kernel(
-    bf16* __restrict__ out,          // [T, H]
-    const bf16* __restrict__ y,      // [E_local, T, H]
-    const float* __restrict__ weights,  // [T, k] (global expert ids)
-    const int* __restrict__ ids,        // [T, k]
-    const int T, const int H, const int k,
-    const int expert_base, const int n_local) {
-  const int t = blockIdx.x;
-  // k-indexed state in LDS (runtime-k register arrays would spill).
-  // Experts outside this rank's [expert_base, +n_local) slice contribute 0
-  // (their partial sums come from other TP ranks' all-reduce).
-  __shared__ float w[16];
-  __shared__ int64_t base[16];
-  if (threadIdx.x < k) {
-    const int j = threadIdx.x;
-    const int le = ids[(int64_t)t * k + j] - expert_base;
-    const bool mine = le >= 0 && le < n_local;
-    w[j] = mine ? weights[(int64_t)t * k + j] : 0.f;
-    base[j] = ((int64_t)(mine ? le : 0) * T + t) * H;
-  }
-  __syncthreads();
-  for (int h = threadIdx.x * 2; h < H; h += 256 * 2) {
-    float a0 = 0.f, a1 = 0.f;
-    for (int j = 0; j < k; ++j) {
-      const uint32_t u = *reinterpret_cast<const uint32_t*>(y + base[j] + h);
-      a0 += w[j] * bf16_bits_to_float((uint16_t)u);
-      a1 += w[j] * bf16_bits_to_float((uint16_t)(u >> 16));
-    }
-    uint32_t packed = (uint32_t)float_to_bf16_bits(a0) |
-                      ((uint32_t)float_to_bf16_bits(a1) << 16);
-    *reinterpret_cast<uint32_t*>(out + (int64_t)t * H + h) = packed;
-  }
-}
-
-// Row-indexed variant for the sparse/grouped prefill path: y is a flat
-// [R, H] buffer (padded grouped-bmm block + overflow segments); rows[t,k]
-// addresses each token's k expert outputs directly. Replaces torch
-// index_add_ scatters (36% of Qwen3-30B prefill GPU time) with one
-// bandwidth-bound gather; zero-weight slots point at row 0.
+// One block per token over a flat [R, H] buffer of expert rows, in any order;
+// rows[t,k] addresses each token's k of them. Reading them bounds it (no
+// scatter, no atomics); zero-weight slots point at row 0.
 __global__ __launch_bounds__(256) void moe_mix_rows_kernel(
     bf16* __restrict__ out,          // [T, H]
     const bf16* __restrict__ y,      // [R, H]
@@ -203,14 +161,4 @@ extern "C" void arks_moe_mix_rows(void* out, const void* y,
   hipLaunchKernelGGL(moe_mix_rows_kernel, grid, block, 0, stream, (bf16*)out,
                      (const bf16*)y, (const float*)weights, (const int*)rows,
                      T, H, k);
-}
-
-extern "C" void arks_moe_mix(void* out, const void* y, const void* weights,
-                             const void* ids, int T, int H, int k,
-                             int expert_base, int n_local,
-                             hipStream_t stream) {
-  dim3 grid(T), block(256);
-  hipLaunchKernelGGL(moe_mix_kernel, grid, block, 0, stream, (bf16*)out,
-                     (const bf16*)y, (const float*)weights, (const int*)ids,
-                     T, H, k, expert_base, n_local);
 }

@@ -299,7 +299,7 @@ def test_qwen2_moe_shared_expert_logits_match_transformers(tmp_path):
         str(tmp_path), config=hf_cfg, torch_dtype=torch.float32
     )
     hf.eval()
-    # both dense (<=64) and sparse (>64) dispatch paths
+    # few rows and a prompt's
     for ids in ([5, 77, 2, 30, 9], [(11 * i + 3) % 500 for i in range(80)]):
         logits = forward_ours(ours, cfg, ids)
         with torch.no_grad():
@@ -325,7 +325,7 @@ def test_wide_expert_grouped_dispatch_matches_naive():
     m = MoEMLP(cfg)
     for p in m.parameters():
         p.data.normal_(0, 0.05)
-    T = 100  # > DENSE_TOKENS -> sparse path; 40 experts -> grouped bmm
+    T = 100
     x = torch.randn(T, cfg.hidden_size, dtype=torch.bfloat16)
     y = m(x)
 
@@ -339,7 +339,7 @@ def test_wide_expert_grouped_dispatch_matches_naive():
     for t in range(T):
         for j in range(cfg.num_experts_per_tok):
             e = int(sel[t, j])
-            # w13/w2 are stored pre-transposed [in, out]
+            # w13/w2: the stored [out, in] weights seen as [in, out]
             gu = x[t].float() @ m.w13[e].float()
             g, u = gu.chunk(2)
             h = torch.nn.functional.silu(g) * u
