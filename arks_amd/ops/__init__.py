@@ -10,6 +10,7 @@ are unit-testable without a GPU.
 
 from __future__ import annotations
 
+import math
 import os
 
 import torch
@@ -717,10 +718,41 @@ def linear_f32_lib(x, weight):
     return F.linear(x, weight).float()
 
 
+def _tile_fill(M: int, N: int) -> float:
+    """Share of the chip that tiles of 256 (the last of 128) rows x 128 columns
+    keep busy with rows that are there: they run in rounds of 256."""
+    rows, left = divmod(M, 256)
+    cost = rows + (0 if left == 0 else 0.55 if left <= 128 else 1.0)
+    cols = -(-N // 128)
+    return M * N / (256 * 128 * 256 * math.ceil(cost * cols / 256))
+
+
+def _tiles(x, weight) -> bool:
+    """Whether silu_mul(x weight^T) takes the product of tile_gemm.hip, with
+    its activation inside, rather than the library's and a pass behind it: many
+    rows, and tiles that fill their rounds over the chip. 18944 x 3584, us,
+    here (library and activation): 384 rows 130 (122), 512 rows 158 (148), 600
+    rows 167 (173), 900 rows 235 (291), 1024 rows 245 (260), 2017 rows 409
+    (547), 2048 rows 406 (433), 3150 rows 623 (811), 8192 rows 1523 (1636):
+    round row counts have picked library kernels, others not."""
+    M, (N, K) = x.shape[0], weight.shape
+    return (M > 512 and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16
+            and K % 64 == 0 and 64 <= K < 1 << 22 and N % 16 == 0
+            and x.stride(0) < 1 << 22 and _tile_fill(M, N // 2) >= 0.65
+            and _plain(x, weight)
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and native_available())
+
+
 def linear_silu_mul(x, weight):
     """silu_mul(x weight^T), weight [2N, K] the gate rows, then the up rows."""
-    if x.dim() == 2 and weight.shape[0] % 2 == 0 and _streams(x, weight, True):
-        return _stream_gemm(x, weight, silu=True)
+    if x.dim() == 2 and weight.shape[0] % 2 == 0:
+        if _streams(x, weight, True):
+            return _stream_gemm(x, weight, silu=True)
+        if _tiles(x, weight):
+            out = x.new_empty((x.shape[0], weight.shape[0] // 2))
+            _native().tile_silu(out, _rows_16b(x), weight)
+            return out
     return silu_mul(linear_bf16(x, weight))
 
 

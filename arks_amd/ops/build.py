@@ -31,6 +31,7 @@ SOURCES = [
     os.path.join(CSRC, "moe.hip"),
     os.path.join(CSRC, "moe_gemm.hip"),
     os.path.join(CSRC, "stream_gemm.hip"),
+    os.path.join(CSRC, "tile_gemm.hip"),
     os.path.join(CSRC, "allreduce.hip"),
 ]
 

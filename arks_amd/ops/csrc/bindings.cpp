@@ -87,6 +87,8 @@ void arks_stream_split(void* part, const void* a, const void* w, int m, int n,
                        hipStream_t stream);
 void arks_stream_sum(void* out, const void* part, const void* bias, int64_t m,
                      int n, int splits, hipStream_t stream);
+void arks_tile_silu(void* out, const void* a, const void* w, int m, int n,
+                    int k, int64_t a_stride, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, const void* ids, const void* weights,
                    int pairs, int expert_base, int n_local, int tile,
@@ -604,6 +606,27 @@ void stream_sum(torch::Tensor out, torch::Tensor part,
                   (int)part.size(0), current_stream());
 }
 
+// out [M, N] = silu(a w_gate^T) * (a w_up^T), w [2N, K] (tile_gemm.hip)
+void tile_silu(torch::Tensor out, torch::Tensor a, torch::Tensor w) {
+  check_bf16_contig(out, "out");
+  check_bf16_rowstrided(a, "a");
+  check_bf16_contig(w, "w");
+  TORCH_CHECK(out.dim() == 2 && a.dim() == 2 && w.dim() == 2);
+  check_rows_16b(out, "out");
+  check_rows_16b(a, "a");
+  check_rows_16b(w, "w");
+  const int64_t M = a.size(0), K = a.size(1), N = w.size(0) / 2;
+  TORCH_CHECK(w.size(1) == K && w.size(0) == 2 * N && out.size(0) == M &&
+              out.size(1) == N);
+  TORCH_CHECK(K >= 64 && K % 64 == 0 && N % 8 == 0 && M < (1 << 30) &&
+                  N < (1 << 29) && K < (1 << 22) &&
+                  a.stride(0) < (1 << 22),
+              "need K % 64 == 0, N % 8 == 0");
+  if (M == 0 || N == 0) return;
+  arks_tile_silu(out.data_ptr(), a.data_ptr(), w.data_ptr(), (int)M, (int)N,
+                 (int)K, a.stride(0), current_stream());
+}
+
 // The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
 // beyond this rank's El experts from expert_base on count as zero.
 void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
@@ -703,6 +726,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("stream_split", &stream_split, pybind11::arg("part"),
         pybind11::arg("a"), pybind11::arg("w"), pybind11::arg("per") = 0);
   m.def("stream_sum", &stream_sum);
+  m.def("tile_silu", &tile_silu);
   m.def("moe_experts", &moe_experts);
   m.def("mfma_probe", &mfma_probe);
   m.def("mfma_probe32", &mfma_probe32);

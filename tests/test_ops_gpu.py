@@ -1067,6 +1067,51 @@ def test_linear_silu_mul(M, I, K):
     assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("M,I,K", [
+    (1, 8, 64), (128, 136, 128), (129, 128, 192), (256, 120, 320),
+    (257, 1000, 64), (385, 520, 256),
+    # workgroups that go from tile to tile, whole and last ones of few rows
+    (2404, 4000, 64), (2404, 4000, 192), (2304, 4104, 128),
+])
+def test_tile_silu(M, I, K):
+    """Gate, up and activation in tiles vs fp64: ends of tiles in both
+    directions, one to five steps of K, strided rows."""
+    assert_native()
+    torch.manual_seed(M + I + K)
+    x = torch.randn(M, 2 * K, dtype=torch.bfloat16, device=DEV)[:, :K]
+    w = (torch.randn(2 * I, K, device=DEV) * K ** -0.5).bfloat16()
+    buf = torch.full((M + 1, I), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._native().tile_silu(buf[:M], x, w)
+    assert (buf[M] == 7.0).all()
+    xd, wd = x.double().cpu(), w.double().cpu()
+    gu = xd @ wd.t()
+    g, u = gu[:, :I], gu[:, I:]
+    # as in test_linear_silu_mul, the reciprocal within 2^-22
+    s = K * 2 ** -24 * (xd.abs() @ wd.abs().t())
+    expect = torch.nn.functional.silu(g) * u
+    slack = 1.1 * s[:, :I] * u.abs() + g.abs() * s[:, I:] + 2 ** -19 * expect.abs()
+    out = buf[:M].double().cpu()
+    assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
+
+
+def test_tiles_rule():
+    """Rows that fill the chip's rounds take the tiles, others the library."""
+    assert_native()
+    w = torch.empty(2 * 18944, 64, dtype=torch.bfloat16, device=DEV)
+    x = torch.randn(2048, 64, dtype=torch.bfloat16, device=DEV)
+    assert [ops._tiles(x[:m], w) for m in (512, 520, 600, 2017)] == [
+        False, False, True, True]
+    assert not ops._tiles(x, w[:4096])
+    assert not ops._tiles(x.float(), w)
+    assert not ops._tiles(x[:, :32], w[:, :32].contiguous())
+    assert not ops._tiles(x, w.clone().requires_grad_())
+    w.normal_(std=0.1)
+    torch.testing.assert_close(
+        ops.linear_silu_mul(x, w).float(),
+        ops.silu_mul(torch.nn.functional.linear(x, w)).float(),
+        atol=2e-2, rtol=2e-2)  # both factors rounded to bf16 there
+
+
 def test_streams_refuses():
     """What the streamed product leaves to the other paths."""
     assert_native()
