@@ -842,12 +842,24 @@ def moe_route(x, gate, k: int, renorm: bool):
 
 def moe_tile(rows: int, top_k: int, experts: int) -> int:
     """Pairs of one work item (moe_gemm.hip): weights streamed under 16 of them
-    up to 8 pairs per expert on the mean, 128 x 128 tiles beyond. 128 experts
-    of 2048 x 768, 8 per row, us: 7 rows 96 (tiles 134), 128 rows 241 (250),
-    200 rows 268 (252), 512 rows 493 (270). experts: those that the rows choose
-    from, of all ranks (16 of the 128 here: 17 rows 59 (75), 128 rows 70 (87),
-    512 rows 91 (90))."""
+    up to 8 pairs per expert on the mean, tiles of 128 or more beyond
+    (moe_experts). us, streamed (tiles of 256): 128 experts of 2048 x 768, 8 per
+    row: 7 rows 89 (116), 64 rows 213 (223), 129 rows 240 (238), 200 rows 268
+    (242), 512 rows 485 (251); 16 experts of 2048 x 1408, 4 per row: 32 rows 63
+    (60), 64 rows 78 (61); 8 experts of 4096 x 1024, 2 per row: 32 rows 43 (73),
+    112 rows 84 (73). experts: those that the rows choose from, of all ranks."""
     return 16 if rows * top_k <= 8 * experts else 128
+
+
+def _moe_engine(x, H: int, I: int, pairs: int) -> bool:
+    """Whether experts that moe_tile gives tiles run in those of up to 256
+    pairs: whole steps of 64 columns, and what their 32-bit row offsets reach.
+    Tiles of 128 take the rest, and were never the faster ones: 128 experts of
+    2048 x 768, 8 per row, us, 256 (128): 200 rows 242 (265), 5012 rows 545
+    (742); 8 of 4096 x 14336, 2 per row: 200 rows 565 (611), 8192 rows 4527
+    (9434)."""
+    return ((H | I) % 64 == 0 and x.shape[0] * x.stride(0) < 1 << 31
+            and 2 * I * H < 1 << 31 and pairs < 1 << 23)
 
 
 def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
@@ -861,12 +873,14 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
     if (x.is_cuda and x.dtype == torch.bfloat16 and H % 8 == 0
             and I % 8 == 0 and El <= 1024 and k <= 16):
         out = torch.empty((x.shape[0], H), dtype=x.dtype, device=x.device)
+        x = _rows_16b(x)
         # the streamed kernel takes whole matrix operands of 32 columns only
         # (16 experts of 2056 x 1416, 4 per row, 7 rows, with routing: 95 us
         # in tiles, 120 us as batched products)
         tile = moe_tile(x.shape[0], k, experts or El) if (H | I) % 32 == 0 else 128
-        _native().moe_experts(out, _rows_16b(x), w13, w2, weights, ids,
-                              expert_base, tile)
+        if tile == 128 and _moe_engine(x, H, I, x.shape[0] * k):
+            tile = 256
+        _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, tile)
         return out
     return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
 

@@ -90,12 +90,13 @@ void arks_stream_sum(void* out, const void* part, const void* bias, int64_t m,
 void arks_tile_silu(void* out, const void* a, const void* w, int m, int n,
                     int k, int64_t a_stride, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
-                   void* n_items, const void* ids, const void* weights,
+                   void* n_items, void* claims, const void* ids,
+                   const void* weights,
                    int pairs, int expert_base, int n_local, int tile,
                    int max_items, hipStream_t stream);
 void arks_moe_gemm(void* out, const void* a, const void* w, const void* perm,
-                   const void* items, const void* n_items, int64_t a_stride,
-                   int64_t w_expert, int64_t w_stride, int n_out, int k_total,
+                   const void* items, const void* n_items, void* claims,
+                   int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out, int k_total,
                    int top_k, int max_items, int tile, int up,
                    hipStream_t stream);
 void arks_mfma_probe(void* d, const void* a, const void* b, hipStream_t stream);
@@ -645,10 +646,15 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   TORCH_CHECK(w13.size(1) == 2 * I && w13.size(2) == H && w2.size(0) == El &&
                   w2.size(1) == H,
               "expert weights do not fit");
-  TORCH_CHECK(tile == 16 || tile == 128);
-  TORCH_CHECK((H | I) % (tile == 16 ? 32 : 8) == 0 && El <= 1024 && k <= 16,
-              "need H and I % 8 == 0 (tile 16: % 32), at most 1024 experts, "
-              "k <= 16");
+  TORCH_CHECK(tile == 16 || tile == 128 || tile == 256);
+  TORCH_CHECK((H | I) % (tile == 16 ? 32 : tile == 128 ? 8 : 64) == 0 &&
+                  El <= 1024 && k <= 16,
+              "need H and I % 8 == 0 (tile 16: % 32, 256: % 64), at most 1024 "
+              "experts, k <= 16");
+  // the engine's row offsets are 32 bits wide, the items of one expert 16
+  TORCH_CHECK(tile != 256 || (T * x.stride(0) < (1ll << 31) &&
+                              2 * I * H < (1ll << 31) && P < (1 << 23)),
+              "too large for this tile");
   TORCH_CHECK(weights.is_cuda() && ids.is_cuda() &&
               weights.scalar_type() == torch::kFloat32 &&
               weights.is_contiguous() && ids.scalar_type() == torch::kInt32 &&
@@ -656,10 +662,10 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
               weights.size(0) == T);
   if (T == 0) return;
   const int64_t max_items = std::min(P, El) + P / tile;
-  TORCH_CHECK(max_items <= 65535 || tile == 128, "too many rows for this tile");
+  TORCH_CHECK(max_items <= 65535 || tile != 16, "too many rows for this tile");
   auto ints = x.options().dtype(torch::kInt32);
-  // [items | perm | rows | count], the items on 16-byte places
-  torch::Tensor plan = torch::empty({4 * max_items + 2 * P + 1}, ints);
+  // [items | perm | rows | count | claims], the items on 16-byte places
+  torch::Tensor plan = torch::empty({4 * max_items + 2 * P + 17}, ints);
   int* items = plan.data_ptr<int>();
   int* perm = items + 4 * max_items;
   int* rows = perm + P;
@@ -668,15 +674,16 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   torch::Tensor h = torch::empty({P, I}, x.options());
   torch::Tensor y = torch::empty({P, H}, x.options());
   auto stream = current_stream();
-  arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, ids.data_ptr(),
-                weights.data_ptr(), (int)P, (int)expert_base, (int)El,
-                (int)tile, (int)max_items, stream);
+  int* claims = n_items + 1;
+  arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
+                ids.data_ptr(), weights.data_ptr(), (int)P, (int)expert_base,
+                (int)El, (int)tile, (int)max_items, stream);
   arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
-                n_items, x.stride(0), 2 * I * H, H, (int)I, (int)H, (int)k,
-                (int)max_items, (int)tile, 1, stream);
+                n_items, claims, x.stride(0), 2 * I * H, H, (int)I, (int)H,
+                (int)k, (int)max_items, (int)tile, 1, stream);
   arks_moe_gemm(y.data_ptr(), h.data_ptr(), w2.data_ptr(), perm, items, n_items,
-                I, H * I, I, (int)H, (int)I, (int)k, (int)max_items, (int)tile,
-                0, stream);
+                claims, I, H * I, I, (int)H, (int)I, (int)k, (int)max_items,
+                (int)tile, 0, stream);
   arks_moe_mix_rows(out.data_ptr(), y.data_ptr(), w_pair.data_ptr(), rows,
                     (int)T, (int)H, (int)k, stream);
 }

@@ -9,17 +9,22 @@
 //              and no barrier before the final sum over the waves. 7 rows, 8
 //              of 128 experts each (2048 x 768): 90 us for 46 experts' 434 MB
 //              (4.8 TB/s); every expert as a batched product took 210 us.
-//   moe_tile   many pairs per expert: bound by the matrix cores. 128 pairs x
-//              128 weight rows, 64 of K per step through double-buffered LDS.
-//              5012 rows: 670 us (560 TFLOP/s); a padded batched product with
-//              its gathers, activation and overflow products took 1160 us.
+//   moe_engine many pairs per expert: bound by the matrix cores, and by the
+//              weights' one read while experts have few. Up to 256 pairs x 256
+//              weight rows per workgroup (tile_engine.h). 128 experts of 2048 x
+//              768, 8 per row, with plan and mix: 5012 rows 545 us (tiles of
+//              128: 742), 512 rows 251 us for 1.2 GB of weights (270); 8
+//              experts of 4096 x 14336, 2 per row, 8192 rows 4.5 ms (9.4).
+//   moe_tile   the same for sizes that are no multiple of 64: 128 pairs x 128
+//              weight rows, 64 of K per step through double-buffered LDS and
+//              registers, 560 TFLOP/s.
 //
 // Both products exist as "up" (rows gathered by pair, silu(gate) * up in fp32
 // before the one rounding) and "down". Weights lie as in checkpoints,
 // [expert, out, in]: a lane reads 16 bytes along K, as the MFMA operands
 // want them. Items past the last one are empty, so grids depend on the shapes
 // alone and a decode step can be captured.
-#include "common.h"
+#include "tile_engine.h"
 
 namespace arks {
 
@@ -41,17 +46,20 @@ __device__ __forceinline__ float moe_silu_mul(float g, float u) {
 
 // One workgroup. perm[place] = pair, rows[pair] = place (0 where the expert
 // is another rank's), weights_out[pair] = the pair's weight (0 there),
-// items[i] = {local expert, first place, pairs, 0}, n_items.
+// items[i] = {local expert, first place, pairs, number within the expert |
+// items of the expert << 16}, n_items; claims[16] = 0 (moe_engine's).
 __global__ __launch_bounds__(1024) void moe_plan_kernel(
     int* __restrict__ perm, int* __restrict__ rows,
     float* __restrict__ weights_out, int4* __restrict__ items,
-    int* __restrict__ n_items, const int* __restrict__ ids,
+    int* __restrict__ n_items, int* __restrict__ claims,
+    const int* __restrict__ ids,
     const float* __restrict__ weights, const int pairs, const int expert_base,
     const int n_local, const int tile, const int max_items) {
   __shared__ int count[MOE_MAX_E], start[MOE_MAX_E], first_item[MOE_MAX_E];
   __shared__ int total_items;
   const int tid = threadIdx.x;
   for (int e = tid; e < n_local; e += 1024) count[e] = 0;
+  if (tid < 16) claims[tid] = 0;
   __syncthreads();
   constexpr int PB = 8;  // loads in flight per thread
   for (int p0 = tid; p0 < pairs; p0 += 1024 * PB) {
@@ -95,9 +103,10 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
   __syncthreads();
   for (int e = tid; e < n_local; e += 1024) {
     const int c = count[e];
-    for (int i = 0; i * tile < c; ++i)
-      items[first_item[e] + i] =
-          make_int4(e, start[e] + i * tile, min(tile, c - i * tile), 0);
+    const int n = (c + tile - 1) / tile;
+    for (int i = 0; i < n; ++i)
+      items[first_item[e] + i] = make_int4(
+          e, start[e] + i * tile, min(tile, c - i * tile), i | n << 16);
     count[e] = 0;  // from here on: pairs placed
   }
   for (int i = total_items + tid; i < max_items; i += 1024)
@@ -362,27 +371,152 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
   }
 }
 
+// Up to 256 pairs of one expert x 256 weight rows (UP: 128 gate rows and their
+// 128 up rows) in the product engine of tile_engine.h. Each XCD takes a
+// contiguous stretch of (expert, row tile, item), so that an expert's items meet
+// the same weights in its L2; its workgroups claim tiles one by one, since
+// those of at most 128 pairs take about 0.55 of the others' time (dealt out in
+// turn, 5012 rows: 591 us, claimed 545). The claim is made a tile ahead, so that
+// neither it nor the pairs' rows are waited for. Its place in LDS belongs to the
+// tiles' array: a second one made the compiler drain the loads before every
+// read of the first.
+template <bool UP>
+__global__ __launch_bounds__(512, 2) void moe_engine_kernel(
+    bf16* __restrict__ out, const bf16* __restrict__ a,
+    const bf16* __restrict__ w, const int* __restrict__ perm,
+    const int4* __restrict__ items, const int* __restrict__ n_items,
+    int* __restrict__ claims, const int64_t a_stride, const int64_t w_expert,
+    const int n_out, const int k_total, const int top_k, const int row_tiles) {
+  __shared__ __attribute__((aligned(1024))) char lds[TILE_LDS + 16];
+  int& claimed = *reinterpret_cast<int*>(lds + TILE_LDS);
+  const int total = *n_items * row_tiles;
+  const int xcd = blockIdx.x % 8, slots = gridDim.x / 8;
+  const int j0 = (int)((int64_t)total * xcd / 8);
+  const int jn = (int)((int64_t)total * (xcd + 1) / 8) - j0;
+  int i = blockIdx.x / 8;
+  if (i >= jn) return;
+  const int steps = k_total / TILE_K;
+  Tile tile(lds);
+  struct Job {
+    int expert, first, pairs, n0;
+  };
+  auto job = [&](int i) {
+    const int j = j0 + i, q = j / row_tiles, w4 = items[q].w;
+    const int i0 = q - (w4 & 0xffff), r = j - i0 * row_tiles, n = w4 >> 16;
+    const int4 it = items[i0 + r % n];
+    return Job{it.x, it.y, it.z, r / n * (UP ? 128 : 256)};
+  };
+  auto places = [&](const Job& b, int (&p)[2][2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r = min(h * 128 + tile_row(tile.wave(), tile.lane(), j),
+                          b.pairs - 1);
+        p[h][j] = UP ? perm[b.first + r] : r;
+      }
+  };
+  auto rows = [&](const Job& b, const int (&p)[2][2]) {
+    TileRows t;
+    t.a = tile_buffer(a + (UP ? 0 : b.first * a_stride));
+    const bf16* we = w + b.expert * w_expert;
+    t.w[0] = tile_buffer(we);
+    t.w[1] = tile_buffer(we + (UP ? (int64_t)n_out * k_total : 0));
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r = tile_row(tile.wave(), tile.lane(), j);
+        const uint32_t row = UP ? p[h][j] / top_k : p[h][j];
+        t.ao[h][j] = row * (uint32_t)(a_stride * 2) +
+                     tile_piece_a(r, tile.lane());
+        t.wo[h][j] =
+            (uint32_t)min(b.n0 + (UP ? 0 : h * 128) + r, n_out - 1) *
+                (uint32_t)(k_total * 2) +
+            tile_piece_w(r, tile.lane());
+      }
+    return t;
+  };
+  Job now = job(i);
+  int p[2][2];
+  places(now, p);
+  TileRows t = rows(now, p);
+  tile.prologue(t, steps, now.pairs <= TILE_HALF);
+  // workgroups' first tiles are theirs, the others are claimed
+  if (threadIdx.x == 0) claimed = slots + atomicAdd(&claims[xcd], 1);
+  Tile::sync();
+  i = __builtin_amdgcn_readfirstlane(claimed);
+  tile.prologue_wait(steps, now.pairs <= TILE_HALF);
+  for (;;) {
+    const bool more = i < jn;
+    const Job next = more ? job(i) : now;
+    if (more) places(next, p);
+    tile.run(t, steps, now.pairs <= TILE_HALF);
+    int c;
+    if (more) {
+      if (threadIdx.x == 0) c = atomicAdd(&claims[xcd], 1);
+      // its loads travel while this tile is stored
+      t = rows(next, p);
+      tile.prologue(t, steps, next.pairs <= TILE_HALF);
+    }
+    ushort8 o[UP ? 8 : 16];
+    tile.each([&](int x, int, int, const float(&g)[8], const float(&u)[8]) {
+      if constexpr (UP) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = tile_silu_mul(g[j], u[j]);
+        o[x] = tile_round(v);
+      } else {
+        o[2 * x] = tile_round(g);
+        o[2 * x + 1] = tile_round(u);
+      }
+    });
+    if (more) {
+      if (threadIdx.x == 0) claimed = slots + c;
+      tile.prologue_wait(steps, next.pairs <= TILE_HALF);
+    }
+    tile.each([&](int x, int m, int n, const float(&)[8], const float(&)[8]) {
+      bf16* row = out + (int64_t)(now.first + m) * n_out;
+      const int col = now.n0 + n;  // n_out % 8 == 0
+      if (m >= now.pairs) return;
+      if constexpr (UP) {
+        if (col < n_out) *reinterpret_cast<ushort8*>(row + col) = o[x];
+      } else {
+        if (col < n_out) *reinterpret_cast<ushort8*>(row + col) = o[2 * x];
+        if (col + 128 < n_out)
+          *reinterpret_cast<ushort8*>(row + col + 128) = o[2 * x + 1];
+      }
+    });
+    if (!more) return;
+    now = next;
+    Tile::sync();
+    i = __builtin_amdgcn_readfirstlane(claimed);
+  }
+}
+
 }  // namespace arks
 
 using namespace arks;
 
 extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
-                              void* items, void* n_items, const void* ids,
-                              const void* weights, int pairs, int expert_base,
+                              void* items, void* n_items, void* claims,
+                              const void* ids, const void* weights, int pairs, int expert_base,
                               int n_local, int tile, int max_items,
                               hipStream_t stream) {
   hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, stream,
                      (int*)perm, (int*)rows, (float*)weights_out, (int4*)items,
-                     (int*)n_items, (const int*)ids, (const float*)weights,
-                     pairs, expert_base, n_local, tile, max_items);
+                     (int*)n_items, (int*)claims, (const int*)ids,
+                     (const float*)weights, pairs, expert_base, n_local, tile, max_items);
 }
 
 // tile: pairs of an item, 16 (streamed; n_out % 32 == k_total % 32 == 0) or 128
-// (tiles through LDS; n_out % 8 == k_total % 8 == 0).
+// (tiles through LDS; n_out % 8 == k_total % 8 == 0) or 256 (the engine;
+// n_out % 8 == k_total % 64 == 0, w_stride == k_total, an expert's weights and
+// (up) all rows of a under 4 GiB).
 extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
                               const void* perm, const void* items,
-                              const void* n_items, int64_t a_stride,
-                              int64_t w_expert, int64_t w_stride, int n_out,
+                              const void* n_items, void* claims,
+                              int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out,
                               int k_total, int top_k, int max_items, int tile,
                               int up, hipStream_t stream) {
 #define ARKS_STREAM(NF, WV, UP)                                               \
@@ -400,6 +534,19 @@ extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
       if (k_total >= 4096) ARKS_STREAM(2, 8, false);
       else ARKS_STREAM(2, 4, false);
     }
+  } else if (tile == 256) {
+    const int row_tiles = (n_out + (up ? 127 : 255)) / (up ? 128 : 256);
+    const int64_t jobs = (int64_t)max_items * row_tiles;
+    const dim3 grid(jobs < 256 ? (jobs + 7) / 8 * 8 : 256), block(512);
+#define ARKS_ENGINE(UP)                                                       \
+  hipLaunchKernelGGL((moe_engine_kernel<UP>), grid, block, 0, stream,         \
+                     (bf16*)out, (const bf16*)a, (const bf16*)w,              \
+                     (const int*)perm, (const int4*)items,                    \
+                     (const int*)n_items, (int*)claims + (up ? 0 : 8),        \
+                     a_stride, w_expert, n_out, k_total, top_k, row_tiles)
+    if (up) ARKS_ENGINE(true);
+    else ARKS_ENGINE(false);
+#undef ARKS_ENGINE
   } else {
     const int cols = up ? MT_BN / 2 : MT_BN;
     const int row_tiles = (n_out + cols - 1) / cols;

@@ -168,6 +168,9 @@ class Tile {
     if (wm_ == 0) barrier();
   }
 
+  // All waves' LDS writes before it can be read behind it; loads stay under way.
+  __device__ __forceinline__ static void sync() { meet_reads(); }
+
   // f(group of sums 0..7, row of the tile, column of the half, [half 0's 8
   // sums], [half 1's]); the group is known to the compiler
   template <typename F>

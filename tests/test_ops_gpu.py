@@ -745,6 +745,14 @@ def test_moe_mix_matches_einsum():
     (500, 8, 2, 256, 64, 0, 8, 128, True),
     (7, 128, 8, 256, 96, 8, 100, 128, False),
     (65, 16, 8, 64, 32, 0, 16, None, False),  # either side of the rule
+    # tiles of up to 256 pairs: whole and half ones and one pair behind, ends
+    # of N, one to 33 steps of K, more tiles than workgroups
+    (128, 4, 2, 64, 64, 0, 4, 128, True),
+    (129, 4, 2, 128, 192, 0, 4, 128, True),
+    (257, 4, 2, 192, 320, 0, 4, 128, True),
+    (300, 16, 4, 192, 320, 4, 8, 128, False),
+    (1, 4, 2, 64, 64, 0, 4, 128, False),
+    (3000, 4, 2, 64, 2112, 0, 4, 128, False),
     (16, 16, 8, 64, 32, 0, 16, None, False),
     (17, 16, 8, 64, 32, 0, 16, None, False),
 ])
