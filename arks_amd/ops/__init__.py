@@ -10,6 +10,7 @@ are unit-testable without a GPU.
 
 from __future__ import annotations
 
+import functools
 import math
 import os
 
@@ -549,7 +550,8 @@ def _few_rows(x, weight, bias=None) -> bool:
 
 
 def _streams(x, weight, silu: bool = False, bias=None) -> bool:
-    """Whether x weight^T takes stream_gemm. A workgroup reads all of x's rows
+    """Whether x weight^T takes stream_gemm (larger weights: if _mid does not
+    take them). A workgroup reads all of x's rows
     beside its 16 or 32 weight rows, so the line lies where that traffic (rows
     x K), and the waves' tails, meet what the other path loses: us, here
     (other), the other being the split product with its sums up to
@@ -571,14 +573,101 @@ def _streams(x, weight, silu: bool = False, bias=None) -> bool:
 
 
 def _splits(x, weight, bias=None) -> bool:
-    """Whether x weight^T splits K over workgroups (asked after _streams):
-    weights up to _SKINNY_MAX_ELEMS, and larger ones that are tall. us with
-    the sums (library): 3584 x 18944, 4 rows 30.7 (32.6), 32 rows 31.7 (43.9),
-    64 rows 36.8 (49.6); 8192 x 28672, 8 rows 88.5 (91.8), 64 rows 108 (154);
-    wide ones, as 16384 x 4096 at 32 rows, 36 (34)."""
+    """Whether x weight^T splits K over workgroups of stream_gemm.hip (asked
+    after _mid, which takes N % 8 == 0, and _streams): weights up to
+    _SKINNY_MAX_ELEMS, and larger ones that are tall. us with the sums
+    (library): 3584 x 18944, 4 rows 30.7 (32.6), 32 rows 31.7 (43.9), 64 rows
+    36.8 (49.6); 8192 x 28672, 8 rows 88.5 (91.8), 64 rows 108 (154); wide
+    ones, as 16384 x 4096 at 32 rows, 36 (34)."""
     N, K = weight.shape
     return (_few_rows(x, weight, bias) and K % 64 == 0 and N % 4 == 0
             and (N * K <= _SKINNY_MAX_ELEMS or K >= 2 * N))
+
+
+# us that a step of mid_gemm.hip (64 columns of 32 * qt weight rows) takes at up
+# to 64, 128, 192 and 256 rows, but for 0.155 qt: fits of what it measured
+_MID_STEP = (0.07, 0.13, 0.26, 0.32)
+
+
+@functools.lru_cache(maxsize=4096)
+def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool):
+    """(qt, splits, us) of a mid_gemm: weight rows of a tile (32 * qt) and runs
+    of K that keep 256 CUs busy in the fewest steps, 1.5 us being lost at the
+    start of a round; the fp32 sums of the runs are written and read at 5 TB/s,
+    and added by a launch of their own unless the consumer does (summed). us,
+    chosen (others): 3584 x 18944, 64 rows, 4, 9
+    26.1 (5, 9 28.1; 2, 4 29.8; 4, 6 33); 3584 x 3584, 200 rows, without the
+    sums, 2, 4 15.1 (4, 8 15.2); 37888 x 3584, 64 rows, 5, 1 44.8 (4, 1 64.7)."""
+    steps, step = K // 64, _MID_STEP[(M + 63) // 64 - 1]
+    best = None
+    for qt in (5, 4, 2):
+        tiles = -(-N // ((16 if silu else 32) * qt))
+        most = 1 if silu or tiles >= 180 else min(8, steps)
+        for splits in range(1, most + 1):
+            us = -(-tiles * splits // 256) * (
+                1.5 + -(-steps // splits) * (step + 0.155 * qt))
+            if splits > 1:
+                us += splits * M * N * 1.6e-6 + (0.0 if summed else 4.0)
+            if best is None or us < best[2]:
+                best = (qt, splits, us)
+    return best
+
+
+def _mid(x, weight, bias=None, silu: bool = False, summed: bool = False):
+    """(qt, splits) if x weight^T (or silu(gate) * up of it) takes mid_gemm,
+    else None. summed: the consumer adds the sums of splits. It takes up to 256
+    rows, but for what the streamed product (few rows of small weights, which
+    has no sums to add) or the library does as fast. us, here (other): 37888 x
+    3584 with the activation, 1 row 43.0 (48.1), 32 rows 43.1 (57.6), 128 rows
+    51.0 (71.2), 200 rows 65 (85); 152064 x 3584, 1 row 170 (182), 64 rows 201
+    (209), 200 rows 284 (325); 3584 x 18944, 1 row 22.7 and 0.3 of sums (27.4),
+    100 rows 30.3 and 3 (96.5). The others' side of the line: 3584 x 3584 and
+    its sums, 1 row 7.6 (6.2), 100 rows 15 (13.1); 57344 x 8192, whose tiles
+    fill the second round of CUs by 3/4, 200 rows 247 (228)."""
+    if not (_USE_SKINNY and x.is_cuda and x.dim() == 2
+            and 1 <= x.shape[0] <= 256
+            and x.dtype == weight.dtype == torch.bfloat16):
+        return None
+    M, (N, K) = x.shape[0], weight.shape
+    if silu:
+        N //= 2
+    if (K % 64 or N % 8 or not 64 <= K < 1 << 22 or not 0 < N < 1 << 24
+            or x.stride(0) >= 1 << 22 or (silu and 2 * N * K >= 1 << 31)):
+        return None
+    small = weight.shape[0] * K <= _SKINNY_MAX_ELEMS
+    if small and (M * K <= 16384 and N <= 4096 if summed
+                  else _streams(x, weight, silu, bias)):
+        return None
+    if not (_plain(x, weight, bias)
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == x.dtype
+                                  and bias.is_contiguous()))
+            and native_available()):
+        return None
+    qt, splits, _ = _mid_cut(M, N, K, silu, summed)
+    if splits == 1:
+        tiles = -(-N // ((16 if silu else 32) * qt))
+        fill = tiles / (256 * -(-tiles // 256))
+        if fill < (0.35 if silu and M <= 64 else 0.55 if M <= 64
+                   else 0.6 if M <= 128 or N * K <= 1 << 27 else 0.9):
+            return None
+    elif not summed:
+        if not (small or K >= 2 * N) or (M > 64 and N * K < 16_000_000):
+            return None
+    return qt, splits
+
+
+def _mid_gemm(x, weight, bias, cut, silu: bool = False):
+    """A product by mid_gemm: a tensor, or Parts where K is split."""
+    (qt, splits), M = cut, x.shape[0]
+    N = weight.shape[0] // (2 if silu else 1)
+    if splits > 1:
+        sums = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
+        _native().mid_gemm(sums, _rows_16b(x), weight, None, qt, False)
+        return Parts(sums, bias)
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    _native().mid_gemm(out, _rows_16b(x), weight, bias, qt, silu)
+    return out
 
 
 class Parts:
@@ -623,6 +712,9 @@ def _stream_gemm(x, weight, bias=None, dtype=None, silu: bool = False):
 
 def linear_parts(x, weight, bias=None):
     """linear_bf16 for a consumer that takes Parts."""
+    cut = _mid(x, weight, bias, summed=True)
+    if cut is not None:
+        return _mid_gemm(x, weight, bias, cut)
     if (x.dim() == 2 and not _streams(x, weight, bias=bias)
             and _splits(x, weight, bias)):
         return Parts(_stream_parts(x, weight), bias)
@@ -630,9 +722,12 @@ def linear_parts(x, weight, bias=None):
 
 
 def linear_bf16(x, weight, bias=None):
-    """Linear dispatch: the streamed product for few rows, K split over
-    workgroups for other small decode-shaped and tall GEMMs on GPU, hipBLASLt
-    (F.linear) otherwise."""
+    """Linear dispatch: the streamed product for few rows of small weights, the
+    tiles of mid_gemm.hip for up to 256 rows, K split over workgroups for sizes
+    that those do not take, hipBLASLt (F.linear) otherwise."""
+    cut = _mid(x, weight, bias)
+    if cut is not None:
+        return parts_sum(_mid_gemm(x, weight, bias, cut))
     if x.dim() == 2 and _streams(x, weight, bias=bias):
         return _stream_gemm(x, weight, bias)
     if x.dim() == 2 and _splits(x, weight, bias):
@@ -747,6 +842,9 @@ def _tiles(x, weight) -> bool:
 def linear_silu_mul(x, weight):
     """silu_mul(x weight^T), weight [2N, K] the gate rows, then the up rows."""
     if x.dim() == 2 and weight.shape[0] % 2 == 0:
+        cut = _mid(x, weight, silu=True)
+        if cut is not None:
+            return _mid_gemm(x, weight, None, cut, silu=True)
         if _streams(x, weight, True):
             return _stream_gemm(x, weight, silu=True)
         if _tiles(x, weight):

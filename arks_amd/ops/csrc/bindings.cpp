@@ -89,6 +89,9 @@ void arks_stream_sum(void* out, const void* part, const void* bias, int64_t m,
                      int n, int splits, hipStream_t stream);
 void arks_tile_silu(void* out, const void* a, const void* w, int m, int n,
                     int k, int64_t a_stride, hipStream_t stream);
+void arks_mid_gemm(void* out, const void* a, const void* w, const void* bias,
+                   int m, int n, int k, int64_t a_stride, int qt, int splits,
+                   int parts, int silu, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, void* claims, const void* ids,
                    const void* weights,
@@ -628,6 +631,46 @@ void tile_silu(torch::Tensor out, torch::Tensor a, torch::Tensor w) {
                  (int)K, a.stride(0), current_stream());
 }
 
+// out [M, N] = a w^T (+ bias), bf16, or fp32 [splits, M, N] its sums over runs
+// of K; silu: silu(gate) * up of w [2N, K] (mid_gemm.hip)
+void mid_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
+              c10::optional<torch::Tensor> bias, int64_t qt, bool silu) {
+  const bool parts = out.dim() == 3;
+  check_bf16_rowstrided(a, "a");
+  check_bf16_contig(w, "w");
+  if (parts) {
+    TORCH_CHECK(out.is_cuda() && out.scalar_type() == torch::kFloat32 &&
+                    out.is_contiguous() && !silu && !bias.has_value(),
+                "sums are contiguous fp32 on the GPU, without a bias");
+  } else {
+    check_bf16_contig(out, "out");
+  }
+  TORCH_CHECK((parts || out.dim() == 2) && a.dim() == 2 && w.dim() == 2);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0);
+  check_rows_16b(a, "a");
+  check_rows_16b(w, "w");
+  const int64_t M = a.size(0), K = a.size(1);
+  const int64_t N = silu ? w.size(0) / 2 : w.size(0);
+  const int64_t splits = parts ? out.size(0) : 1;
+  TORCH_CHECK(w.size(1) == K && w.size(0) == (silu ? 2 * N : N) &&
+              out.size(parts ? 1 : 0) == M && out.size(parts ? 2 : 1) == N);
+  TORCH_CHECK(qt == 2 || qt == 4 || qt == 5);
+  TORCH_CHECK(M <= 256 && K % 64 == 0 && N % 8 == 0 && splits >= 1 &&
+                  splits <= K / 64 && K < (1 << 22) && N < (1 << 24) &&
+                  a.stride(0) < (1 << 22) &&
+                  (!silu || 2 * N * K < (1ll << 31)),
+              "need M <= 256, K % 64 == 0, N % 8 == 0");
+  if (bias.has_value()) {
+    check_bf16_contig(*bias, "bias");
+    TORCH_CHECK(bias->numel() == N);
+  }
+  if (M == 0 || N == 0) return;
+  arks_mid_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(),
+                bias.has_value() ? bias->data_ptr() : nullptr, (int)M, (int)N,
+                (int)K, a.stride(0), (int)qt, (int)splits, parts, silu,
+                current_stream());
+}
+
 // The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
 // beyond this rank's El experts from expert_base on count as zero.
 void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
@@ -734,6 +777,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("a"), pybind11::arg("w"), pybind11::arg("per") = 0);
   m.def("stream_sum", &stream_sum);
   m.def("tile_silu", &tile_silu);
+  m.def("mid_gemm", &mid_gemm);
   m.def("moe_experts", &moe_experts);
   m.def("mfma_probe", &mfma_probe);
   m.def("mfma_probe32", &mfma_probe32);

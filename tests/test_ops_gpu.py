@@ -1102,6 +1102,76 @@ def test_tile_silu(M, I, K):
     assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("M,N,K,qt,splits", [
+    (1, 8, 64, 2, 1), (16, 72, 128, 5, 2), (17, 168, 192, 5, 1),
+    (64, 320, 1088, 4, 5), (65, 136, 256, 4, 1), (128, 152, 320, 2, 5),
+    (129, 64, 384, 2, 3), (192, 160, 448, 5, 2), (193, 1000, 576, 4, 9),
+    (256, 168, 640, 5, 3), (200, 128, 64, 4, 1),
+    # workgroups that go from tile to tile, of one step to more than the stages
+    (3, 41000, 64, 5, 1), (70, 20000, 192, 2, 1), (130, 9000, 384, 2, 2),
+    (250, 45000, 128, 5, 1),
+])
+@pytest.mark.parametrize("kind", ["bias", "sums", "silu"])
+def test_mid_gemm(M, N, K, qt, splits, kind):
+    """Up to 256 rows in tiles vs fp64: every tile, ends of tiles in both
+    directions, fewer steps than stages and more, runs of K, strided rows."""
+    assert_native()
+    torch.manual_seed(M + N + K)
+    silu = kind == "silu"
+    x = torch.randn(M, 2 * K, dtype=torch.bfloat16, device=DEV)[:, :K]
+    w = (torch.randn(2 * N if silu else N, K, device=DEV) * K ** -0.5).bfloat16()
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV) if kind == "bias" else None
+    if kind == "sums":
+        buf = torch.full((splits + 1, M, N), 7.0, device=DEV)
+        out = buf[:splits]
+    else:
+        buf = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
+        out = buf[:M]
+    ops._native().mid_gemm(out, x, w, b, qt, silu)
+    assert (buf[-1] == 7.0).all()
+    xd, wd = x.double(), w.double()
+    expect = xd @ wd.t()
+    # fp32 sums of K products: within K * 2^-24 of sum |x w|
+    slack = K * 2 ** -24 * (xd.abs() @ wd.abs().t())
+    if kind == "sums":
+        ends = [K // 64 * i // splits * 64 for i in range(splits + 1)]
+        for i, (lo, hi) in enumerate(zip(ends, ends[1:])):
+            run = xd[:, lo:hi] @ wd[:, lo:hi].t()
+            assert ((out[i].double() - run).abs() <= slack).all()
+        return
+    if silu:  # as in test_tile_silu
+        g, u, sg, su = expect[:, :N], expect[:, N:], slack[:, :N], slack[:, N:]
+        expect = torch.nn.functional.silu(g) * u
+        slack = 1.1 * sg * u.abs() + g.abs() * su + 2 ** -19 * expect.abs()
+    else:
+        expect = expect + b.double()
+    assert ((out.double() - expect).abs()
+            <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
+
+
+def test_mid_rule():
+    """Which products of up to 256 rows take the tiles, and that the runs of K
+    that are chosen fit."""
+    assert_native()
+    x = torch.randn(257, 4096, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(4608, 4096, dtype=torch.bfloat16, device=DEV) * 0.02
+    assert ops._mid(x[:1], w) is None  # streamed, nothing to add
+    assert ops._mid(x[:1], w, summed=True) and ops._mid(x[:64], w)
+    assert ops._mid(x[:256], w) and ops._mid(x, w) is None
+    assert ops._mid(x[:64].float(), w) is None
+    assert ops._mid(x[:64, :4000], w[:, :4000].contiguous()) is None
+    assert ops._mid(x[:64], w[:4604]) is None
+    assert ops._mid(x[:64], w.t()) is None
+    assert ops._mid(x[:64], w.clone().requires_grad_()) is None
+    for M in (1, 20, 100, 200, 256):
+        parts = ops.linear_parts(x[:M], w)
+        assert parts.sums.shape[0] <= 16
+        for out in (ops.parts_sum(parts), ops.linear_bf16(x[:M], w)):
+            torch.testing.assert_close(
+                out.float(), torch.nn.functional.linear(x[:M], w).float(),
+                atol=2e-2, rtol=2e-2)  # both rounded to bf16, values up to 6
+
+
 def test_tiles_rule():
     """Rows that fill the chip's rounds take the tiles, others the library."""
     assert_native()
