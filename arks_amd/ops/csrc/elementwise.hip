@@ -8,20 +8,24 @@
 namespace arks {
 
 // ---------------------------------------------------------------------------
-// RMSNorm: one workgroup (256 threads = 4 waves) per row.
+// RMSNorm: one workgroup per row, of 4 waves (8 where it adds split sums: such
+// rows are few, and a row is one pass then).
 // hidden must be a multiple of 8 (bf16x8 vector loads).
 // PARTS: the input is the sum of fp32 splits [splits, rows, hidden] of the
-// product before it; adding 8 of them here takes 1 us at 64 x 3584, a launch
+// product before it; adding 8 of them here takes 0.5 us at 64 x 3584, a launch
 // of its own 5.
+// NV: vectors of a thread that stay in registers, with the weights loaded
+// beside them: few rows are bound by the chain of loads, sum and store, many
+// by the bytes. Rows that are longer (NV 0) are read again from L2 behind the
+// sum, as all were before: 64 x 3584 and 4 splits 5.3 us, held 4.9.
 // ---------------------------------------------------------------------------
-template <bool FUSED_ADD, bool PARTS = false>
+template <bool FUSED_ADD, bool PARTS, int NV>
 __global__ void rmsnorm_kernel(bf16* __restrict__ out,
                                const void* __restrict__ input,
                                bf16* __restrict__ residual,  // null unless FUSED_ADD
                                const bf16* __restrict__ weight,
                                const float eps, const int hidden,
-                               const int splits = 0) {
-  // split sums come with few rows: more threads, so that a row is one pass
+                               const int splits) {
   constexpr int BLOCK = PARTS ? 512 : 256;
   const int row = blockIdx.x;
   const bf16* in_row =
@@ -34,53 +38,72 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
 
   const int nvec = hidden / 8;
   float ss = 0.f;
-  // Pass 1: (optionally add residual and store it), accumulate sum of squares.
-  for (int i = threadIdx.x; i < nvec; i += BLOCK) {
+  // the row's values at vector i (with the residual, stored back)
+  auto load = [&](const int i) {
     float x[8];
+    ushort8 r{}, s;
+    if constexpr (FUSED_ADD) r = *reinterpret_cast<const ushort8*>(res_row + i * 8);
     if constexpr (PARTS) {
-      const f32x4 lo = sum_parts4(part_row + i * 8, part_stride, splits);
-      const f32x4 hi = sum_parts4(part_row + i * 8 + 4, part_stride, splits);
+      f32x4 lo, hi;
+      sum_parts_pair(part_row + i * 8, part_row + i * 8 + 4, part_stride,
+                     splits, lo, hi);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = j < 4 ? lo[j % 4] : hi[j % 4];
     } else {
-      const ushort8 u = *reinterpret_cast<const ushort8*>(in_row + i * 8);
+      s = *reinterpret_cast<const ushort8*>(in_row + i * 8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = bf16_bits_to_float(u[j]);
+      for (int j = 0; j < 8; ++j) x[j] = bf16_bits_to_float(s[j]);
     }
     if constexpr (FUSED_ADD) {
-      ushort8 r = *reinterpret_cast<const ushort8*>(res_row + i * 8);
-      ushort8 s;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        float v = x[j] + bf16_bits_to_float(r[j]);
-        s[j] = float_to_bf16_bits(v);
-        // Accumulate on the bf16-rounded value so pass 2's re-read matches.
-        float vb = bf16_bits_to_float(s[j]);
-        ss += vb * vb;
+        s[j] = float_to_bf16_bits(x[j] + bf16_bits_to_float(r[j]));
+        // the sum of squares is that of the rounded values, which are normed
+        x[j] = bf16_bits_to_float(s[j]);
       }
       *reinterpret_cast<ushort8*>(res_row + i * 8) = s;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
     }
-  }
-
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+    return s;
+  };
   __shared__ float red[BLOCK / WAVE_SIZE];
-  float total = block_reduce_sum<BLOCK>(ss, red);
-  const float rrms = rsqrtf(total / (float)hidden + eps);
-
-  // Pass 2: normalize (re-read from L1/L2) and scale by weight.
-  const bf16* src_row = FUSED_ADD ? res_row : in_row;
-  for (int i = threadIdx.x; i < nvec; i += BLOCK) {
-    ushort8 x = *reinterpret_cast<const ushort8*>(src_row + i * 8);
-    ushort8 w = *reinterpret_cast<const ushort8*>(weight + i * 8);
+  float rrms;
+  auto store = [&](const int i, const ushort8& x, const ushort8& w) {
     ushort8 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float v = bf16_bits_to_float(x[j]) * rrms * bf16_bits_to_float(w[j]);
-      o[j] = float_to_bf16_bits(v);
-    }
+    for (int j = 0; j < 8; ++j)
+      o[j] = float_to_bf16_bits(bf16_bits_to_float(x[j]) * rrms *
+                                bf16_bits_to_float(w[j]));
     *reinterpret_cast<ushort8*>(out_row + i * 8) = o;
+  };
+  auto weights = [&](const int i) {
+    return *reinterpret_cast<const ushort8*>(weight + i * 8);
+  };
+  if constexpr (NV > 0) {
+    ushort8 x[NV], w[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = threadIdx.x + v * BLOCK;
+      if (i < nvec) w[v] = weights(i);
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = threadIdx.x + v * BLOCK;
+      if (i < nvec) x[v] = load(i);
+    }
+    rrms = rsqrtf(block_reduce_sum<BLOCK>(ss, red) / (float)hidden + eps);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = threadIdx.x + v * BLOCK;
+      if (i < nvec) store(i, x[v], w[v]);
+    }
+  } else {
+    for (int i = threadIdx.x; i < nvec; i += BLOCK) load(i);
+    rrms = rsqrtf(block_reduce_sum<BLOCK>(ss, red) / (float)hidden + eps);
+    const bf16* src_row = FUSED_ADD ? res_row : in_row;
+    for (int i = threadIdx.x; i < nvec; i += BLOCK)
+      store(i, *reinterpret_cast<const ushort8*>(src_row + i * 8), weights(i));
   }
 }
 
@@ -160,29 +183,40 @@ using namespace arks;
 
 extern "C" {
 
+#define ARKS_NORM(FUSED, PARTS, NV)                                            \
+  hipLaunchKernelGGL((rmsnorm_kernel<FUSED, PARTS, NV>), dim3(rows),           \
+                     dim3(PARTS ? 512 : 256), 0, stream, (bf16*)out, input,    \
+                     (bf16*)residual, (const bf16*)weight, eps, hidden, splits)
+#define ARKS_NORM_V(FUSED, PARTS)                                              \
+  do {                                                                         \
+    const int per = (hidden / 8 + (PARTS ? 511 : 255)) / (PARTS ? 512 : 256);  \
+    if (per <= 1) ARKS_NORM(FUSED, PARTS, 1);                                  \
+    else if (per <= 2) ARKS_NORM(FUSED, PARTS, 2);                             \
+    else if (per <= 4) ARKS_NORM(FUSED, PARTS, 4);                             \
+    else ARKS_NORM(FUSED, PARTS, 0);                                           \
+  } while (0)
+
 void arks_rmsnorm(void* out, const void* input, const void* weight, float eps,
                   int rows, int hidden, hipStream_t stream) {
-  dim3 grid(rows), block(256);
-  hipLaunchKernelGGL((rmsnorm_kernel<false>), grid, block, 0, stream,
-                     (bf16*)out, input, nullptr,
-                     (const bf16*)weight, eps, hidden);
+  void* const residual = nullptr;
+  const int splits = 0;
+  ARKS_NORM_V(false, false);
 }
 
 void arks_fused_add_rmsnorm(void* out, const void* input, void* residual,
                             const void* weight, float eps, int rows, int hidden,
                             hipStream_t stream) {
-  dim3 grid(rows), block(256);
-  hipLaunchKernelGGL((rmsnorm_kernel<true>), grid, block, 0, stream, (bf16*)out,
-                     input, (bf16*)residual, (const bf16*)weight, eps, hidden, 0);
+  const int splits = 0;
+  ARKS_NORM_V(true, false);
 }
 
-void arks_fused_add_rmsnorm_parts(void* out, const void* part, int splits,
+void arks_fused_add_rmsnorm_parts(void* out, const void* input, int splits,
                                   void* residual, const void* weight, float eps,
                                   int rows, int hidden, hipStream_t stream) {
-  hipLaunchKernelGGL((rmsnorm_kernel<true, true>), dim3(rows), dim3(512), 0,
-                     stream, (bf16*)out, part, (bf16*)residual,
-                     (const bf16*)weight, eps, hidden, splits);
+  ARKS_NORM_V(true, true);
 }
+#undef ARKS_NORM_V
+#undef ARKS_NORM
 
 void arks_silu_mul(void* out, const void* gate_up, int64_t rows, int d,
                    hipStream_t stream) {

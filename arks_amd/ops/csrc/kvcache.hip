@@ -146,8 +146,16 @@ __global__ void rope_cache_kernel(
   const float* cs = cos_sin + pos * head_dim;
   const int64_t slot = slot_mapping[token];
   const bool cache = slot >= 0;
-  const int64_t block_id = cache ? slot / block_size : 0;
-  const int offset = cache ? (int)(slot % block_size) : 0;
+  // (a division of 64 bits would be a long chain in front of the stores)
+  int64_t block_id = 0;
+  int offset = 0;
+  if (cache && slot <= 0x7fffffff) {
+    block_id = (uint32_t)slot / (uint32_t)block_size;
+    offset = (uint32_t)slot % (uint32_t)block_size;
+  } else if (cache) {
+    block_id = slot / block_size;
+    offset = (int)(slot % block_size);
+  }
   const int64_t cbase =
       (block_id * num_kv_heads) * (int64_t)block_size * head_dim +
       (int64_t)offset * head_dim;
@@ -169,8 +177,9 @@ __global__ void rope_cache_kernel(
     float a2[2], b2[2];
     if constexpr (PARTS) {
       const int c = h * head_dim + p2;
-      const float2 f1 = sum_parts2(part_row + c, part_stride, splits);
-      const float2 f2 = sum_parts2(part_row + c + half, part_stride, splits);
+      f32x2 f1, f2;
+      sum_parts_pair(part_row + c, part_row + c + half, part_stride, splits, f1,
+                     f2);
       a2[0] = f1.x, a2[1] = f1.y, b2[0] = f2.x, b2[1] = f2.y;
       if (bias) {
 #pragma unroll
@@ -244,8 +253,9 @@ __global__ void rope_cache_kernel(
     ushort8 vv8;
     if constexpr (PARTS) {
       const int c = (num_q_heads + num_kv_heads) * head_dim + i * 8;
-      const f32x4 lo = sum_parts4(part_row + c, part_stride, splits);
-      const f32x4 hi = sum_parts4(part_row + c + 4, part_stride, splits);
+      f32x4 lo, hi;
+      sum_parts_pair(part_row + c, part_row + c + 4, part_stride, splits, lo,
+                     hi);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float b = bias ? bf16_bits_to_float(bias[c + e]) : 0.f;

@@ -4,6 +4,7 @@
 
 namespace arks {
 
+using f32x2 = __attribute__((ext_vector_type(2))) float;
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 
 // 4 columns of all splits, `stride` floats apart; 8 loads in flight
@@ -24,24 +25,28 @@ __device__ __forceinline__ f32x4 sum_parts4(const float* p,
   return s;
 }
 
-__device__ __forceinline__ float2 sum_parts2(const float* p,
-                                             const int64_t stride,
-                                             const int splits) {
-  float2 s{0.f, 0.f};
+// The same at two places, 16 loads in flight (1 x 3584, 8 splits and their
+// norm 4.6 us; one place after the other 5.4).
+template <typename T>
+__device__ __forceinline__ void sum_parts_pair(const float* p, const float* q,
+                                               const int64_t stride,
+                                               const int splits, T& a, T& b) {
+  a = b = T{};
   for (int s0 = 0; s0 < splits; s0 += 8) {
-    float2 v[8];
+    T v[8], w[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      v[j] = *reinterpret_cast<const float2*>(
-          p + (int64_t)min(s0 + j, splits - 1) * stride);
+    for (int j = 0; j < 8; ++j) {
+      const int64_t at = (int64_t)min(s0 + j, splits - 1) * stride;
+      v[j] = *reinterpret_cast<const T*>(p + at);
+      w[j] = *reinterpret_cast<const T*>(q + at);
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       if (s0 + j < splits) {
-        s.x += v[j].x;
-        s.y += v[j].y;
+        a += v[j];
+        b += w[j];
       }
   }
-  return s;
 }
 
 }  // namespace arks

@@ -47,6 +47,33 @@ def test_fused_add_rmsnorm(rows, hidden):
     torch.testing.assert_close(out.float().cpu(), expect_out, atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("kind", ["plain", "fused", "sums"])
+@pytest.mark.parametrize("rows,hidden", [
+    (1, 8), (3, 2048), (2, 2056), (3, 4096), (1, 4104), (2, 8192), (2, 8200),
+    (1, 16384), (2, 16392)])
+def test_norm_widths(rows, hidden, kind):
+    """Rows held in 1, 2 or 4 vectors a thread and longer ones, vs fp64."""
+    assert_native()
+    torch.manual_seed(hidden)
+    x = torch.randn(rows, hidden, device=DEV).bfloat16()
+    w = torch.randn(hidden, device=DEV).bfloat16()
+    res = torch.randn(rows, hidden, device=DEV).bfloat16()
+    total = x.double() + (0 if kind == "plain" else res.double())
+    if kind == "plain":
+        out, res = ops.rmsnorm(x, w, 1e-6), x
+    elif kind == "fused":
+        out, res = ops.fused_add_rmsnorm(x, res, w, 1e-6)
+    else:
+        sums = torch.randn(9, rows, hidden, device=DEV)
+        sums[8] += x.float() - sums.sum(0)
+        out, res = ops.fused_add_rmsnorm(ops.Parts(sums), res, w, 1e-6)
+    # 1e-5: the order of 9 fp32 sums; one rounding
+    assert ((res.double() - total).abs() <= 1e-5 + 2 ** -8 * total.abs()).all()
+    want = ref.rmsnorm(res.double().cpu(), w.double().cpu(), 1e-6)
+    torch.testing.assert_close(out.double().cpu(), want.double(), atol=1e-5,
+                               rtol=2 ** -7.9)
+
+
 def test_silu_mul():
     assert_native()
     torch.manual_seed(2)
