@@ -938,26 +938,32 @@ def moe_route(x, gate, k: int, renorm: bool):
     return moe_topk(linear_f32_lib(x, gate), k, renorm)
 
 
-def moe_tile(rows: int, top_k: int, experts: int) -> int:
-    """Pairs of one work item (moe_gemm.hip): weights streamed under 16 of them
-    up to 8 pairs per expert on the mean, tiles of 128 or more beyond
-    (moe_experts). us, streamed (tiles of 256): 128 experts of 2048 x 768, 8 per
-    row: 7 rows 89 (116), 64 rows 213 (223), 129 rows 240 (238), 200 rows 268
-    (242), 512 rows 485 (251); 16 experts of 2048 x 1408, 4 per row: 32 rows 63
-    (60), 64 rows 78 (61); 8 experts of 4096 x 1024, 2 per row: 32 rows 43 (73),
-    112 rows 84 (73). experts: those that the rows choose from, of all ranks."""
+def moe_tile(rows: int, top_k: int, experts: int, whole: bool = False) -> int:
+    """Pairs of one work item: 16 where few experts have several (weights
+    streamed, moe_gemm.hip), 64 where they have 1 to 64 on the mean and the
+    sizes are whole steps (mid_gemm.hip, whose items of 128 take over at 32 on
+    the mean, as some experts have twice the mean), 128 or more beyond
+    (moe_experts). Other sizes are streamed up to 8 on the mean. us, 16 (64;
+    128 of mid_gemm; 256): 128 experts of 2048 x 768, 8 per row: 7 rows 83 (86),
+    16 rows 142 (142), 64 rows 208 (196; 215), 200 rows 268 (210; 228; 234), 600
+    rows (233; 251; 252), 1000 rows (346; 265; 269), 1300 rows (461; 280; 281);
+    8 experts of 4096 x 14336, 2 per row: 1 row 137 (169), 16 rows 509 (424;
+    429), 200 rows (463; 476; 590), 600 rows (1384; 1099; 726). experts: those
+    that the rows choose from, of all ranks."""
+    if whole and experts <= rows * top_k <= 64 * experts:
+        return 64
     return 16 if rows * top_k <= 8 * experts else 128
 
 
-def _moe_engine(x, H: int, I: int, pairs: int) -> bool:
-    """Whether experts that moe_tile gives tiles run in those of up to 256
-    pairs: whole steps of 64 columns, and what their 32-bit row offsets reach.
-    Tiles of 128 take the rest, and were never the faster ones: 128 experts of
-    2048 x 768, 8 per row, us, 256 (128): 200 rows 242 (265), 5012 rows 545
-    (742); 8 of 4096 x 14336, 2 per row: 200 rows 565 (611), 8192 rows 4527
-    (9434)."""
+def _moe_whole(x, H: int, I: int, pairs: int) -> bool:
+    """Whether experts can run in items of 64 and more pairs that load rows
+    straight into LDS (mid_gemm.hip, tile_engine.h): whole steps of 64 columns,
+    and what their 32-bit row offsets reach. Tiles of 128 take the rest, and
+    were never the faster ones: 128 experts of 2048 x 768, 8 per row, us, 256
+    (128): 200 rows 242 (265), 5012 rows 545 (742); 8 of 4096 x 14336, 2 per
+    row: 200 rows 565 (611), 8192 rows 4527 (9434)."""
     return ((H | I) % 64 == 0 and x.shape[0] * x.stride(0) < 1 << 31
-            and 2 * I * H < 1 << 31 and pairs < 1 << 23)
+            and 2 * I * H < 1 << 31 and pairs < (1 << 23) - 255)
 
 
 def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
@@ -975,10 +981,16 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
         # the streamed kernel takes whole matrix operands of 32 columns only
         # (16 experts of 2056 x 1416, 4 per row, 7 rows, with routing: 95 us
         # in tiles, 120 us as batched products)
-        tile = moe_tile(x.shape[0], k, experts or El) if (H | I) % 32 == 0 else 128
-        if tile == 128 and _moe_engine(x, H, I, x.shape[0] * k):
+        rows, experts = x.shape[0], experts or El
+        whole = _moe_whole(x, H, I, rows * k)
+        tile = (moe_tile(rows, k, experts, whole) if (H | I) % 32 == 0 else 128)
+        mid = tile == 64
+        if mid and rows * k > 32 * experts:
+            tile = 128
+        elif tile == 128 and whole:
             tile = 256
-        _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, tile)
+        _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, tile,
+                              mid)
         return out
     return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
 

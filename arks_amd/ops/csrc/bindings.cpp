@@ -92,6 +92,10 @@ void arks_tile_silu(void* out, const void* a, const void* w, int m, int n,
 void arks_mid_gemm(void* out, const void* a, const void* w, const void* bias,
                    int m, int n, int k, int64_t a_stride, int qt, int splits,
                    int parts, int silu, hipStream_t stream);
+void arks_mid_items(void* out, const void* a, const void* w, const void* perm,
+                    const void* items, const void* n_items, int64_t a_stride,
+                    int64_t w_expert, int n, int k, int top_k, int max_items,
+                    int ft, int silu, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, void* claims, const void* ids,
                    const void* weights,
@@ -672,10 +676,12 @@ void mid_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
 }
 
 // The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
-// beyond this rank's El experts from expert_base on count as zero.
+// beyond this rank's El experts from expert_base on count as zero. tile: pairs
+// of a work item; mid: of 64 or 128 pairs in mid_gemm.hip, else in
+// moe_gemm.hip (16, 128 or 256).
 void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
                  torch::Tensor w2, torch::Tensor weights, torch::Tensor ids,
-                 int64_t expert_base, int64_t tile) {
+                 int64_t expert_base, int64_t tile, bool mid) {
   check_bf16_contig(out, "out");
   check_bf16_rowstrided(x, "x");
   check_bf16_contig(w13, "w13");
@@ -689,14 +695,16 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   TORCH_CHECK(w13.size(1) == 2 * I && w13.size(2) == H && w2.size(0) == El &&
                   w2.size(1) == H,
               "expert weights do not fit");
-  TORCH_CHECK(tile == 16 || tile == 128 || tile == 256);
-  TORCH_CHECK((H | I) % (tile == 16 ? 32 : tile == 128 ? 8 : 64) == 0 &&
+  TORCH_CHECK(mid ? tile == 64 || tile == 128
+                  : tile == 16 || tile == 128 || tile == 256);
+  TORCH_CHECK((H | I) % (mid ? 64 : tile == 16 ? 32 : tile == 128 ? 8 : 64) == 0 &&
                   El <= 1024 && k <= 16,
-              "need H and I % 8 == 0 (tile 16: % 32, 256: % 64), at most 1024 "
-              "experts, k <= 16");
-  // the engine's row offsets are 32 bits wide, the items of one expert 16
-  TORCH_CHECK(tile != 256 || (T * x.stride(0) < (1ll << 31) &&
-                              2 * I * H < (1ll << 31) && P < (1 << 23)),
+              "need H and I % 8 == 0 (tile 16: % 32, 256 and mid: % 64), at "
+              "most 1024 experts, k <= 16");
+  // row offsets are 32 bits wide, the engine's items of one expert 15
+  TORCH_CHECK(!(mid || tile == 256) ||
+                  (T * x.stride(0) < (1ll << 31) && 2 * I * H < (1ll << 31) &&
+                   P < (1 << 23) - 255),
               "too large for this tile");
   TORCH_CHECK(weights.is_cuda() && ids.is_cuda() &&
               weights.scalar_type() == torch::kFloat32 &&
@@ -721,12 +729,22 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
                 ids.data_ptr(), weights.data_ptr(), (int)P, (int)expert_base,
                 (int)El, (int)tile, (int)max_items, stream);
-  arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
-                n_items, claims, x.stride(0), 2 * I * H, H, (int)I, (int)H,
-                (int)k, (int)max_items, (int)tile, 1, stream);
-  arks_moe_gemm(y.data_ptr(), h.data_ptr(), w2.data_ptr(), perm, items, n_items,
-                claims, I, H * I, I, (int)H, (int)I, (int)k, (int)max_items,
-                (int)tile, 0, stream);
+  if (mid) {
+    const int ft = (int)tile / 64;
+    arks_mid_items(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
+                   n_items, x.stride(0), 2 * I * H, (int)I, (int)H, (int)k,
+                   (int)max_items, ft, 1, stream);
+    arks_mid_items(y.data_ptr(), h.data_ptr(), w2.data_ptr(), nullptr, items,
+                   n_items, I, H * I, (int)H, (int)I, (int)k, (int)max_items,
+                   ft, 0, stream);
+  } else {
+    arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
+                  n_items, claims, x.stride(0), 2 * I * H, H, (int)I, (int)H,
+                  (int)k, (int)max_items, (int)tile, 1, stream);
+    arks_moe_gemm(y.data_ptr(), h.data_ptr(), w2.data_ptr(), perm, items,
+                  n_items, claims, I, H * I, I, (int)H, (int)I, (int)k,
+                  (int)max_items, (int)tile, 0, stream);
+  }
   arks_moe_mix_rows(out.data_ptr(), y.data_ptr(), w_pair.data_ptr(), rows,
                     (int)T, (int)H, (int)k, stream);
 }

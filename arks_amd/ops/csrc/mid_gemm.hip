@@ -23,12 +23,23 @@ namespace arks {
 
 constexpr int MID_LDS = 160 * 1024;
 
-// Stages of LDS: what fits, at most 5.
+// Stages of LDS: what fits, at most 5 (a workgroup's short run of K has not the
+// steps for more: 4608 x 3584, 64 rows, 8 stages 11.2 us, 5 10.6).
 constexpr int mid_stages(int qt, int ft) {
   return MID_LDS / ((32 * qt + 64 * ft) * 128) < 5
              ? MID_LDS / ((32 * qt + 64 * ft) * 128)
              : 5;
 }
+
+// Items of experts (moe_plan_kernel): {expert, first place, pairs, ..}; their
+// places' pairs, of which top_k share a row of a (null: rows are places).
+struct MidItems {
+  const int4* __restrict__ items;
+  const int* __restrict__ n_items;
+  const int* __restrict__ perm;
+  int64_t w_expert;
+  int top_k;
+};
 
 // 1 KB of 8 rows into LDS, 16 B a lane, from step s of its offset. The weights
 // are read once and pass the caches by (non-temporal): 64 rows x 37888 x 3584
@@ -51,13 +62,19 @@ __device__ __forceinline__ void mid_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int QT, int FT, bool SILU>
+// ITEMS: the experts that rows chose. Jobs are (item, tile), an item being up to
+// 64 * FT pairs of one expert, whose weights are so read once; workgroups go
+// through them in turn. With plan and mix, us, here (the best of moe_gemm.hip):
+// 128 experts of 2048 x 768, 8 per row: 16 rows 129 (133), 64 rows 197 (207),
+// 200 rows 211 (235), 600 rows 233 (250); 8 experts of 4096 x 14336, 2 per row:
+// 16 rows 425 (505), 200 rows 464 (591).
+template <int QT, int FT, bool SILU, bool ITEMS>
 __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
     void* __restrict__ out, const bf16* __restrict__ a,
     const bf16* __restrict__ w, const bf16* __restrict__ bias,
     const int m_rows, const int n_total, const int k_total,
     const int64_t a_stride, const int splits, const int parts,
-    const int rotate) {
+    const int rotate, const MidItems of) {
   constexpr int NS = mid_stages(QT, FT);
   constexpr int W_ROWS = 32 * QT, COLS = SILU ? W_ROWS / 2 : W_ROWS;
   constexpr int STAGE = (W_ROWS + 64 * FT) * 128;
@@ -69,7 +86,9 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int wm = wave / 4, wn = wave % 4;
   const int tiles = (n_total + COLS - 1) / COLS;
-  const int jobs = tiles * splits, all_steps = k_total / TILE_K;
+  const int jobs = tiles * (ITEMS ? *of.n_items : splits);
+  const int all_steps = k_total / TILE_K;
+  if (ITEMS && (int)blockIdx.x >= jobs) return;
   // where operand k of a fragment lies: 16 rows of 128 B, pieces permuted
   const int frag = lq * 128 + ((la ^ (lq & 7)) * 16);
   const int w_at = wm * QT * 2048 + frag;
@@ -95,25 +114,51 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   // us, x 57344 x 8192 164 -> 147).
   struct Job {
     int n0, split, s0, steps, turn;
+    int expert, first, rows;
   };
   auto job = [&](const int j) {
+    if constexpr (ITEMS) {
+      const int4 it = of.items[j / tiles];
+      return Job{j % tiles * COLS, 0, 0, all_steps,
+                 rotate ? (int)((unsigned)j % (unsigned)all_steps) : 0,
+                 it.x, it.y, it.z};
+    }
     const unsigned split = j / tiles, n = splits;  // all_steps * n < 2^32
     const int s0 = all_steps * split / n;
     const int steps = all_steps * (split + 1) / n - s0;
     return Job{(int)(j % tiles) * COLS, (int)split, s0, steps,
-               rotate ? (int)((unsigned)j % (unsigned)steps) : 0};
+               rotate ? (int)((unsigned)j % (unsigned)steps) : 0,
+               0, 0, m_rows};
   };
   __amdgpu_buffer_rsrc_t wb, ab;
   uint32_t wo[WL], ao[FT];
+  auto aim_rows = [&](const Job& b) {
 #pragma unroll
-  for (int j = 0; j < FT; ++j) {
-    const int row = (wave + 8 * j) * 8 + lane / 8;
-    ao[j] = (uint32_t)min(row, m_rows - 1) * (uint32_t)(a_stride * 2) +
-            tile_piece_a(row, lane);
-  }
+    for (int j = 0; j < FT; ++j) {
+      const int row = (wave + 8 * j) * 8 + lane / 8;
+      uint32_t from = min(row, b.rows - 1);
+      if (ITEMS && of.perm) {
+        // the 8 rows' pairs are scalar loads: a vector load would be waited
+        // for behind all of those that are under way (what lies up to 7 places
+        // behind the last one is the plan's too, and not taken)
+        const int base = min((wave + 8 * j) * 8, b.rows - 1);
+        const int* at = of.perm + b.first + base;
+        int pair = at[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i)
+          pair = (int)from - base == i ? at[i] : pair;
+        from = (uint32_t)pair / (uint32_t)of.top_k;
+      }
+      ao[j] = from * (uint32_t)(a_stride * 2) + tile_piece_a(row, lane);
+    }
+  };
+  if (!ITEMS) aim_rows(job(blockIdx.x));
   auto aim = [&](const Job& b) {  // the loads at a job
-    ab = tile_buffer(a + b.s0 * TILE_K);
-    wb = tile_buffer(w + (int64_t)b.n0 * k_total + b.s0 * TILE_K);
+    if (ITEMS) aim_rows(b);
+    ab = tile_buffer(a + b.s0 * TILE_K +
+                     (ITEMS && !of.perm ? b.first * a_stride : 0));
+    wb = tile_buffer(w + (ITEMS ? b.expert * of.w_expert : 0) +
+                     (int64_t)b.n0 * k_total + b.s0 * TILE_K);
 #pragma unroll
     for (int j = 0; j < WL; ++j) {
       const int row = (wave + 8 * j) * 8 + lane / 8;
@@ -237,8 +282,8 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
 #pragma unroll
     for (int f = 0; f < FT; ++f) {
       const int m = (wn * FT + f) * 16 + lq;
-      if (m >= m_rows) continue;
-      const int64_t row = (int64_t)m * n_total;
+      if (m >= now.rows) continue;
+      const int64_t row = (int64_t)(now.first + m) * n_total;
       if constexpr (SILU) {
         bf16* to_row = reinterpret_cast<bf16*>(out) + row;
 #pragma unroll
@@ -323,10 +368,10 @@ extern "C" void arks_mid_gemm(void* out, const void* a, const void* w,
   // 3584 x 18944 39 -> 48 us)
   const int rotate = (int64_t)m * k <= 1 << 20;
 #define ARKS_MID(QT, FT, SILU)                                                 \
-  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU>),                          \
+  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, false>),                   \
                      dim3(jobs < 256 ? jobs : 256), dim3(512), 0, stream, out, \
                      (const bf16*)a, (const bf16*)w, (const bf16*)bias, m, n,  \
-                     k, a_stride, splits, parts, rotate)
+                     k, a_stride, splits, parts, rotate, MidItems{})
 #define ARKS_MID_S(QT, FT)                                                     \
   do {                                                                         \
     if (silu) ARKS_MID(QT, FT, true);                                          \
@@ -344,5 +389,31 @@ extern "C" void arks_mid_gemm(void* out, const void* a, const void* w,
   else ARKS_MID_M(5);
 #undef ARKS_MID_M
 #undef ARKS_MID_S
+#undef ARKS_MID
+}
+
+// out [places, n]: the items' pairs (at most 64 * ft each) times their experts'
+// weights, silu: [2n, k] each; n_items of the max_items items are there. k % 64
+// == 0, n % 8 == 0; an expert's weights and (perm) all rows of a under 4 GiB; 7 ints
+// behind the last of perm are there.
+extern "C" void arks_mid_items(void* out, const void* a, const void* w,
+                               const void* perm, const void* items,
+                               const void* n_items, int64_t a_stride,
+                               int64_t w_expert, int n, int k, int top_k,
+                               int max_items, int ft, int silu,
+                               hipStream_t stream) {
+  const MidItems of{(const int4*)items, (const int*)n_items, (const int*)perm,
+                    w_expert, top_k};
+  const int cols = silu ? 64 : 128;
+  const int64_t jobs = (int64_t)((n + cols - 1) / cols) * max_items;
+  const int grid = (int)(jobs < 256 ? jobs : 256);
+#define ARKS_MID(QT, FT, SILU)                                                 \
+  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, true>), dim3(grid),        \
+                     dim3(512), 0, stream, out, (const bf16*)a,                \
+                     (const bf16*)w, nullptr, 0, n, k, a_stride, 1, 0, 1, of)
+  if (ft == 1 && silu) ARKS_MID(4, 1, true);
+  else if (ft == 1) ARKS_MID(4, 1, false);
+  else if (silu) ARKS_MID(4, 2, true);
+  else ARKS_MID(4, 2, false);
 #undef ARKS_MID
 }

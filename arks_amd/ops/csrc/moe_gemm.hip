@@ -3,13 +3,14 @@
 //
 //   moe_plan   pairs sorted by expert, cut into items of one expert and at
 //              most `tile` pairs; every pair's place in the sorted order
-//   moe_stream few pairs per expert: bound by the stream of the chosen
-//              experts' weights. Tiles of 16 weight rows (gate and up rows
+//   moe_stream few experts with a pair or two (from one pair per expert on the
+//              mean mid_gemm.hip takes them, and where sizes are whole steps
+//              of 64): bound by the stream of the chosen experts' weights. Tiles of 16 weight rows (gate and up rows
 //              side by side), the waves of a workgroup splitting K, no LDS
 //              and no barrier before the final sum over the waves. 7 rows, 8
 //              of 128 experts each (2048 x 768): 90 us for 46 experts' 434 MB
 //              (4.8 TB/s); every expert as a batched product took 210 us.
-//   moe_engine many pairs per expert: bound by the matrix cores, and by the
+//   moe_engine more than 64 pairs per expert on the mean: bound by the matrix cores, and by the
 //              weights' one read while experts have few. Up to 256 pairs x 256
 //              weight rows per workgroup (tile_engine.h). 128 experts of 2048 x
 //              768, 8 per row, with plan and mix: 5012 rows 545 us (tiles of

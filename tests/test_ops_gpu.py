@@ -811,6 +811,51 @@ def test_moe_experts(T, E, k, H, I, base, El, tile, skew, monkeypatch):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("T,E,k,H,I,base,El,tile,skew", [
+    (1, 4, 2, 64, 64, 0, 4, 64, False), (7, 128, 8, 256, 192, 0, 128, 64, False),
+    (33, 64, 8, 2048, 768, 16, 16, 64, False),  # another rank's pairs
+    (3, 8, 2, 64, 64, 6, 2, 64, True),          # none of this rank's
+    (64, 4, 2, 320, 576, 0, 4, 64, True), (65, 4, 2, 384, 128, 0, 4, 64, True),
+    (200, 4, 2, 128, 1088, 0, 4, 64, True), (128, 4, 2, 192, 320, 0, 4, 128, True),
+    (129, 4, 2, 64, 448, 0, 4, 128, True), (300, 16, 4, 576, 320, 4, 8, 128, False),
+    # more tiles than workgroups: of one step, of as many as there are stages,
+    # and of more
+    (60, 64, 4, 1088, 64, 0, 64, 64, False), (90, 64, 4, 320, 2112, 0, 64, 128, False),
+    (40, 64, 4, 2112, 256, 0, 64, 64, False),
+])
+def test_moe_items(T, E, k, H, I, base, El, tile, skew):
+    """Routed experts in items of 64 and 128 pairs vs fp64: ends of items and of
+    N, steps of K either side of the stages, empty experts."""
+    assert_native()
+    torch.manual_seed(T + E)
+    x = torch.randn(T, 2 * H, device=DEV).bfloat16()[:, :H]
+    w13 = (torch.randn(El, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(El, H, I, device=DEV) * I ** -0.5).bfloat16()
+    ids = torch.rand(T, E, device=DEV).topk(k).indices.int()
+    if skew:  # one expert takes every row, its neighbour the second choice
+        ids = torch.arange(k, device=DEV, dtype=torch.int32).expand(T, k).contiguous()
+    w = torch.rand(T, k, device=DEV)
+    out = torch.empty(T, H, device=DEV, dtype=torch.bfloat16)
+    ops._native().moe_experts(out, x, w13, w2, w, ids, base, tile, True)
+    expect = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for e in range(El):
+        t, j = (ids == e + base).nonzero(as_tuple=True)
+        gu = x[t].double() @ w13[e].double().t()
+        h = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+        expect.index_add_(0, t, h @ w2[e].double().t() * w[t, j, None].double())
+    # as in test_moe_experts
+    err = (out.double() - expect).norm()
+    assert err <= 3 * 2 ** -8 * expect.norm()
+
+
+def test_moe_tile_rule():
+    """The kernel that the number of pairs per expert asks for."""
+    sizes = (1, 7, 16, 17, 1024, 1025)
+    assert [ops.moe_tile(n, 8, 128, True) for n in sizes] == [
+        16, 16, 64, 64, 64, 128]
+    assert [ops.moe_tile(n, 8, 128) for n in (16, 128, 129)] == [16, 16, 128]
+
+
 def test_moe_tile_of_a_rank(monkeypatch):
     """A rank's share of the experts takes the kernel that their total number
     asks for: its share of the pairs is as small."""
