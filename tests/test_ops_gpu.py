@@ -659,6 +659,43 @@ def test_attention_extend2_big_tiles(hq, hkv, hd, spec):
     torch.testing.assert_close(out.float().cpu(), expect, atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("hq,hkv,hd", [
+    (7, 1, 128), (4, 2, 64), (6, 3, 128), (8, 4, 128), (8, 8, 64), (16, 16, 128),
+    (24, 24, 64)])
+@pytest.mark.parametrize("window", [0, 150])
+def test_extend_tiles_and_heads(hq, hkv, hd, window):
+    """The 256-row kernel vs fp64: one to seven key tiles (fewer than are staged
+    and more), whole last ones and ones of 1, 63 and other numbers of keys, every
+    way that heads go round the XCDs; what stands behind the last key of a
+    page is not read as numbers."""
+    assert_native()
+    spec = [(97, 97), (128, 127), (191, 100), (192, 192), (193, 97), (256, 256),
+            (257, 130), (321, 300), (385, 97), (448, 257)]
+    q, kc, vc, bt, kvl, cu_q, q_lens = _mk_paged(spec, hq, hkv, hd, seed=hq)
+    for i, (n, _) in enumerate(spec):
+        if n % 16:
+            kc[bt[i, n // 16].long(), :, n % 16:] = float("nan")
+            vc[bt[i, n // 16].long(), :, n % 16:] = float("inf")
+    scale = hd ** -0.5
+    out = ops.attention_extend_paged(q, kc, vc, bt, kvl, cu_q, q_lens, scale,
+                                     window=window)
+    expect = torch.zeros_like(out, dtype=torch.float64)
+    for i, (n, m) in enumerate(spec):
+        pages, at = bt[i, :-(-n // 16)].long(), int(cu_q[i])
+        k, v = (c[pages].transpose(1, 2).reshape(-1, hkv, hd)[:n].double()
+                .repeat_interleave(hq // hkv, 1) for c in (kc, vc))
+        x = q[at:at + m].double()
+        s = (x.transpose(0, 1) @ k.permute(1, 2, 0).contiguous()) * scale
+        pos = torch.arange(n - m, n, device=DEV)[:, None]
+        key = torch.arange(n, device=DEV)[None]
+        seen = (key <= pos) & ((key > pos - window) if window else key >= 0)
+        p = s.masked_fill(~seen, -math.inf).softmax(-1)
+        expect[at:at + m] = (p @ v.transpose(0, 1).contiguous()).transpose(0, 1)
+    # probabilities and the result are rounded to bf16: each within 2^-9 of the
+    # values' sizes, of which none is above 5
+    torch.testing.assert_close(out.double(), expect, atol=5 * 2 ** -8, rtol=2 ** -8)
+
+
 @pytest.mark.parametrize(
     "hq,hkv,hd,spec,window",
     [
