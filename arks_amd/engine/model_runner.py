@@ -239,32 +239,26 @@ class ModelRunner:
             # exercised for fresh prefills.
             use_extend = (self.device.type == "cuda" or self.seq_state
                           or any(s.num_cached_tokens > 0 for s in sb.seqs))
-            input_ids: list = []  # np.int64 arrays, one per seq
-            positions: list = []
-            slot_mapping: list = []
+            starts = [seq.num_cached_tokens for seq in sb.seqs]
+            # chunked prefill: run exactly the scheduled token count
+            # (== everything remaining unless the budget split it)
+            q_lens: list[int] = list(sb.num_new_tokens)
             cu = [0]
-            q_lens: list[int] = []
             kv_lens: list[int] = []
             logits_idx: list[int] = []
             lp_meta: list[tuple[int, int, int, int]] = []
             self._lp_prefill = None
-            import numpy as np
-
+            max_blocks = max(len(s.block_table) for s in sb.seqs)
+            bt = torch.zeros((len(sb.seqs), max_blocks), dtype=torch.int32)
+            input_ids, positions, slot_mapping = torch.empty(
+                (3, sum(q_lens)), dtype=torch.int64)
+            seq_lens = torch.empty(len(sb.seqs), dtype=torch.int32)
+            self._stage_rows(sb.seqs, starts, q_lens, input_ids, positions,
+                             slot_mapping, seq_lens, bt)
             for i, seq in enumerate(sb.seqs):
-                toks = seq.all_token_ids
-                c = seq.num_cached_tokens
-                # chunked prefill: run exactly the scheduled token count
-                # (== everything remaining unless the budget split it)
-                n = c + sb.num_new_tokens[i]
-                input_ids.append(np.asarray(toks[c:n], dtype=np.int64))
-                pos = np.arange(c, n, dtype=np.int64)
-                positions.append(pos)
-                # vectorized slot mapping (a per-token Python loop here cost
-                # ~2.8 ms of GPU idle per 8k-token chunk)
-                btn = np.asarray(seq.block_table, dtype=np.int64)
-                slot_mapping.append(btn[pos // bs] * bs + pos % bs)
+                c = starts[i]
+                n = c + q_lens[i]
                 cu.append(cu[-1] + (n - c))
-                q_lens.append(n - c)
                 kv_lens.append(n)
                 if seq.sampling.prompt_logprobs and c < seq.num_prompt_tokens:
                     # echo/prompt-scoring: lm_head on EVERY row of this seq
@@ -290,38 +284,34 @@ class ModelRunner:
                         sample_pos.append(g)
                         g += 1
                 self._lp_prefill = (lp_meta, sample_pos)
-            dev = self.device
-            block_tables = None
-            seq_lens = None
             ext_tiles = None
-            if use_extend:
-                max_blocks = max(len(s.block_table) for s in sb.seqs)
-                bt = torch.zeros((len(sb.seqs), max_blocks), dtype=torch.int32)
-                for i, seq in enumerate(sb.seqs):
-                    bt[i, : len(seq.block_table)] = torch.tensor(
-                        seq.block_table, dtype=torch.int32
-                    )
-                block_tables = bt.to(dev)
-                seq_lens = torch.tensor(kv_lens, dtype=torch.int32, device=dev)
             if use_extend and not self.seq_state:
                 ext_tiles = ops.build_extend_tiles(
-                    q_lens, kv_lens,
-                    self.cfg.kv_cache_dtype == "fp8", dev,
+                    q_lens, kv_lens, self.cfg.kv_cache_dtype == "fp8", "cpu",
                     num_q_heads=max(
                         self.model_cfg.num_attention_heads
                         // get_tp_world_size(), 1),
                 )
+            t64, t256, singles, ctab, ws_rows = (
+                ext_tiles or (None, None, (None, None), None, 0))
+            (input_ids, positions, slot_mapping, cu_seqlens, seq_lens, bt,
+             logits_indices, t64, t256, ctab, drows, dseqs) = ops.upload(
+                [input_ids, positions, slot_mapping,
+                 torch.tensor(cu, dtype=torch.int32), seq_lens, bt,
+                 torch.tensor(logits_idx, dtype=torch.int64), t64, t256, ctab,
+                 *singles], self.device)
             return ForwardBatch(
                 is_prefill=True,
-                input_ids=torch.from_numpy(np.concatenate(input_ids)).to(dev),
-                positions=torch.from_numpy(np.concatenate(positions)).to(dev),
-                slot_mapping=torch.from_numpy(np.concatenate(slot_mapping)).to(dev),
-                cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=dev),
+                input_ids=input_ids,
+                positions=positions,
+                slot_mapping=slot_mapping,
+                cu_seqlens=cu_seqlens,
                 seq_lens_list=q_lens,
-                block_tables=block_tables,
-                seq_lens=seq_lens,
-                ext_tiles=ext_tiles,
-                logits_indices=torch.tensor(logits_idx, dtype=torch.int64, device=dev),
+                block_tables=bt if use_extend else None,
+                seq_lens=seq_lens if use_extend else None,
+                ext_tiles=(ext_tiles and
+                           (t64, t256, (drows, dseqs), ctab, ws_rows)),
+                logits_indices=logits_indices,
                 **self._state_fields(sb.seqs, q_lens),
             )
         # decode
@@ -354,6 +344,26 @@ class ModelRunner:
                if self.seq_state else {}),
         )
 
+    def _stage_rows(self, seqs, starts, counts, ids, pos, slots, lens, bt) -> None:
+        """What the rows of a prefill step read, into host tensors; row i of bt
+        (zeros) gets sequence i's pages."""
+        if self.device.type == "cuda":
+            return ops.stage_rows(
+                [s.prompt_token_ids for s in seqs],
+                [s.output_token_ids for s in seqs],
+                [s.block_table for s in seqs], starts, counts, ids, pos, slots,
+                lens, bt, self.cfg.block_size)
+        bs, at = self.cfg.block_size, 0
+        for i, (seq, c, n) in enumerate(zip(seqs, starts, counts)):
+            p = torch.arange(c, c + n)
+            table = torch.tensor(seq.block_table, dtype=torch.int64)
+            ids[at:at + n] = torch.tensor(seq.all_token_ids[c:c + n])
+            pos[at:at + n] = p
+            slots[at:at + n] = table[p // bs] * bs + p % bs
+            lens[i] = c + n
+            bt[i, :len(table)] = table
+            at += n
+
     def _state_fields(self, seqs: list[Sequence], q_lens: list[int]) -> dict:
         """ForwardBatch fields of models with per-sequence state."""
         if not self.seq_state:
@@ -383,30 +393,29 @@ class ModelRunner:
         self._bmax = next(s for s in self.GRAPH_SIZES if s >= bmax)
         mb = (self.cfg.max_model_len + self.cfg.block_size - 1) // self.cfg.block_size
         dev = self.device
-        self._graph_bufs = {
-            "input_ids": torch.zeros(self._bmax, dtype=torch.int64, device=dev),
-            "positions": torch.zeros(self._bmax, dtype=torch.int64, device=dev),
-            "slot_mapping": torch.full((self._bmax,), -1, dtype=torch.int64, device=dev),
-            "block_tables": torch.zeros(self._bmax, mb, dtype=torch.int32, device=dev),
-            "seq_lens": torch.ones(self._bmax, dtype=torch.int32, device=dev),
-            # pinned host staging
-            "h_input_ids": torch.zeros(self._bmax, dtype=torch.int64, pin_memory=True),
-            "h_positions": torch.zeros(self._bmax, dtype=torch.int64, pin_memory=True),
-            "h_slot_mapping": torch.full((self._bmax,), -1, dtype=torch.int64, pin_memory=True),
-            "h_block_tables": torch.zeros(self._bmax, mb, dtype=torch.int32, pin_memory=True),
-            "h_seq_lens": torch.ones(self._bmax, dtype=torch.int32, pin_memory=True),
-        }
+        # what a captured step reads lies together and is moved as one: a step
+        # of bs rows takes the small fields and bs rows of page numbers
+        fields = [("input_ids", torch.int64), ("positions", torch.int64),
+                  ("slot_mapping", torch.int64), ("seq_lens", torch.int32)]
         if self.seq_state:
-            self._graph_bufs.update({
-                "state_slots": torch.full((self._bmax,), -1, dtype=torch.int32, device=dev),
-                "h_state_slots": torch.full((self._bmax,), -1, dtype=torch.int32, pin_memory=True),
-                # constants: one row per sequence
-                "cu_seqlens": torch.arange(self._bmax + 1, dtype=torch.int32, device=dev),
-                "token_seq": torch.arange(self._bmax, dtype=torch.int32, device=dev),
-            })
-        for name in ("input_ids", "positions", "slot_mapping", "block_tables",
-                     "seq_lens") + (("state_slots",) if self.seq_state else ()):
-            self._graph_bufs["np_" + name] = self._graph_bufs["h_" + name].numpy()
+            fields.append(("state_slots", torch.int32))
+        small = sum(-(-self._bmax * t.itemsize // 16) * 16 for _, t in fields)
+        b = self._graph_bufs = {"small": small, "row": 4 * mb}
+        room = small + self._bmax * 4 * mb
+        for pre, buf in (
+                ("", torch.zeros(room, dtype=torch.uint8, device=dev)),
+                ("h_", torch.zeros(room, dtype=torch.uint8, pin_memory=True))):
+            at = 0
+            for name, dtype in fields:
+                n = self._bmax * dtype.itemsize
+                b[pre + name] = buf[at:at + n].view(dtype)
+                at += -(-n // 16) * 16
+            b[pre + "block_tables"] = buf[small:].view(torch.int32).view(
+                self._bmax, mb)
+            b[pre + "all"] = buf
+        if self.seq_state:  # constants: one row per sequence
+            b["cu_seqlens"] = torch.arange(self._bmax + 1, dtype=torch.int32, device=dev)
+            b["token_seq"] = torch.arange(self._bmax, dtype=torch.int32, device=dev)
 
     def _capture(self, bs: int) -> "_DecodeGraph":
         b = self._graph_bufs
@@ -418,13 +427,13 @@ class ModelRunner:
             block_tables=b["block_tables"][:bs],
             seq_lens=b["seq_lens"][:bs],
         )
+        # warmup and capture run the model for real: every row is made a
+        # padding row first (no cache write, no state slot), or live
+        # sequences' pages and recurrent state would change
+        b["slot_mapping"][:bs].fill_(-1)
+        b["seq_lens"][:bs].fill_(1)
         if self.seq_state:
-            # warmup and capture run the model for real: every row is made a
-            # padding row first (no cache write, no state slot), or live
-            # sequences' recurrent state would advance
-            b["slot_mapping"][:bs].fill_(-1)
             b["state_slots"][:bs].fill_(-1)
-            b["seq_lens"][:bs].fill_(1)
             fb.state_slots = b["state_slots"][:bs]
             fb.cu_seqlens = b["cu_seqlens"][:bs + 1]
             fb.token_seq = b["token_seq"][:bs]
@@ -452,44 +461,33 @@ class ModelRunner:
         if bs not in self._graphs:
             self._graphs[bs] = self._capture(bs)
         b = self._graph_bufs
-        bsz = self.cfg.block_size
-        # numpy views of the pinned staging buffers: scalar stores are ~50x
-        # cheaper than torch indexed assignment on the decode hot path
-        # the pinned staging buffers are reused every step: the previous
-        # step's async uploads must have left them before they are rewritten
+        # the pinned staging buffer is reused every step: the previous
+        # step's async upload must have left it before it is rewritten
         # (a caller that does not read that step's logits never syncs)
-        if self._staging_event is not None:
-            self._staging_event.synchronize()
-        np_ids = b["np_input_ids"]
-        np_pos = b["np_positions"]
-        np_slot = b["np_slot_mapping"]
-        np_len = b["np_seq_lens"]
-        np_bt = b["np_block_tables"]
-        for i, seq in enumerate(sb.seqs):
-            pos = seq.num_tokens - 1
-            np_ids[i] = seq.output_token_ids[-1] if seq.output_token_ids else seq.prompt_token_ids[-1]
-            np_pos[i] = pos
-            np_slot[i] = seq.block_table[pos // bsz] * bsz + pos % bsz
-            np_len[i] = seq.num_tokens
-            bt = seq.block_table
-            np_bt[i, : len(bt)] = bt
-            seq.num_cached_tokens = seq.num_tokens
-            if self.seq_state:
-                b["np_state_slots"][i] = seq.state_slot
-        if self.seq_state:
-            b["np_state_slots"][B:bs] = -1
-            b["state_slots"][:bs].copy_(b["h_state_slots"][:bs], non_blocking=True)
-        if B < bs:  # neutralize padding rows
-            np_ids[B:bs] = 0
-            np_pos[B:bs] = 0
-            np_slot[B:bs] = -1
-            np_len[B:bs] = 1
-            np_bt[B:bs, 0] = 0
-        for name in ("input_ids", "positions", "slot_mapping", "seq_lens"):
-            b[name][:bs].copy_(b["h_" + name][:bs], non_blocking=True)
-        b["block_tables"][:bs].copy_(b["h_block_tables"][:bs], non_blocking=True)
         if self._staging_event is None:
             self._staging_event = torch.cuda.Event()
+        else:
+            self._staging_event.synchronize()
+        ops.stage_rows([s.prompt_token_ids for s in sb.seqs],
+                       [s.output_token_ids for s in sb.seqs],
+                       [s.block_table for s in sb.seqs], None, None,
+                       b["h_input_ids"], b["h_positions"], b["h_slot_mapping"],
+                       b["h_seq_lens"], b["h_block_tables"],
+                       self.cfg.block_size)
+        for seq in sb.seqs:
+            seq.num_cached_tokens = seq.num_tokens
+        if self.seq_state:
+            b["h_state_slots"][:B] = torch.tensor(
+                [s.state_slot for s in sb.seqs], dtype=torch.int32)
+            b["h_state_slots"][B:bs] = -1
+        if B < bs:  # neutralize padding rows
+            b["h_input_ids"][B:bs] = 0
+            b["h_positions"][B:bs] = 0
+            b["h_slot_mapping"][B:bs] = -1
+            b["h_seq_lens"][B:bs] = 1
+            b["h_block_tables"][B:bs, 0] = 0
+        n = b["small"] + bs * b["row"]
+        b["all"][:n].copy_(b["h_all"][:n], non_blocking=True)
         self._staging_event.record()
         gr = self._graphs[bs]
         gr.graph.replay()

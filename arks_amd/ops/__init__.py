@@ -166,6 +166,34 @@ def attention_prefill_varlen(q, k, v, cu_seqlens, seq_lens: list[int],
     return ref.attention_prefill_varlen(q, k, v, cu_seqlens, scale, window)
 
 
+def stage_rows(prompts: list, outputs: list, tables: list, starts, counts, ids,
+               pos, slots, lens, block_tables, block_size: int) -> None:
+    """What a step's rows read, into host tensors (see bindings.cpp)."""
+    _native().stage_rows(prompts, outputs, tables, starts, counts, ids, pos,
+                         slots, lens, block_tables, block_size)
+
+
+def upload(tensors: list, device) -> list:
+    """Host tensors (or None) on a device: moved as one, since a step waits for
+    every copy of its own (a dozen took 300 us)."""
+    device = torch.device(device)
+    if device.type != "cuda":
+        return [t if t is None else t.to(device) for t in tensors]
+    at, total = [], 0
+    for t in tensors:
+        at.append(total)
+        total += 0 if t is None else -(-t.numel() * t.element_size() // 16) * 16
+    host = torch.empty(total, dtype=torch.uint8, pin_memory=True)
+    whole = lambda buf, t, o: buf[o:o + t.numel() * t.element_size()].view(
+        t.dtype).view(t.shape)
+    for t, o in zip(tensors, at):
+        if t is not None:
+            whole(host, t, o).copy_(t)
+    moved = host.to(device, non_blocking=True)
+    return [None if t is None else whole(moved, t, o)
+            for t, o in zip(tensors, at)]
+
+
 EXTEND2_QTILE = 256  # q rows per workgroup in the 8-wave ladder kernel
 E2_KVBLK = 64        # keys per LDS tile in the ladder kernel
 # Sequences with at least this many new q tokens go to the 256-row ladder
@@ -221,9 +249,7 @@ def build_extend_tiles(q_lens: list[int], kv_lens: list[int] | None,
                 t256.append((i, q0, min(kvl[i], off + q0 + EXTEND2_QTILE)))
     t64.sort(key=lambda t: -t[2])
     t256.sort(key=lambda t: -t[2])
-    mk64 = lambda t: torch.tensor(
-        [x[:2] for x in t], dtype=torch.int32, device=device
-    ).reshape(-1, 2)
+    t64_t = torch.tensor([x[:2] for x in t64], dtype=torch.int32).reshape(-1, 2)
 
     # KV-split policy for the 256-row kernel: when the long portions' tiles x
     # heads cannot fill ~2 workgroups per CU, split the deepest tiles' key
@@ -264,23 +290,21 @@ def build_extend_tiles(q_lens: list[int], kv_lens: list[int] | None,
             rows.append((i, q0, 0, 1))
     else:
         rows = [(i, q0, 0, 1) for (i, q0, _) in t256]
-    t256_t = torch.tensor(rows, dtype=torch.int32,
-                          device=device).reshape(-1, 4)
-    ctab = torch.tensor(combine, dtype=torch.int32,
-                        device=device).reshape(-1, 4)
+    t256_t = torch.tensor(rows, dtype=torch.int32).reshape(-1, 4)
+    ctab = torch.tensor(combine, dtype=torch.int32).reshape(-1, 4)
 
+    drows = dseqs = None
     if dec:
         # gather indices: the single q row of each decode seq sits at
         # cu_seqlens_q[i]; seq-level metadata indexes with `dec` itself
         cu = [0]
         for n in q_lens:
             cu.append(cu[-1] + n)
-        drows = torch.tensor([cu[i] for i in dec], dtype=torch.long,
-                             device=device)
-        dseqs = torch.tensor(dec, dtype=torch.long, device=device)
-    else:
-        drows = dseqs = None
-    return mk64(t64), t256_t, (drows, dseqs), ctab, ws_rows
+        drows = torch.tensor([cu[i] for i in dec], dtype=torch.long)
+        dseqs = torch.tensor(dec, dtype=torch.long)
+    t64_t, t256_t, ctab, drows, dseqs = upload(
+        [t64_t, t256_t, ctab, drows, dseqs], device)
+    return t64_t, t256_t, (drows, dseqs), ctab, ws_rows
 
 
 def attention_extend_paged(

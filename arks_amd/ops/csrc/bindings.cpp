@@ -675,6 +675,79 @@ void mid_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
                 current_stream());
 }
 
+// What a step's rows read, into host tensors: sequence i's tokens (prompt, then
+// output) from starts[i] on, counts[i] of them (none given: its last one), their
+// positions and cache slots, packed; its length behind them into lens[i], its
+// page numbers into row i of block_tables (what stands behind them stays). Lists
+// are walked here because a step waits for it: 200 requests with 8700 pages take
+// 400 us in Python, 30 here.
+void stage_rows(pybind11::list prompts, pybind11::list outputs,
+                pybind11::list tables, pybind11::object starts,
+                pybind11::object counts, torch::Tensor ids, torch::Tensor pos,
+                torch::Tensor slots, torch::Tensor lens,
+                torch::Tensor block_tables, int64_t block_size) {
+  const Py_ssize_t n = PyList_GET_SIZE(prompts.ptr());
+  auto host = [](const torch::Tensor& t, torch::ScalarType type, int64_t least) {
+    TORCH_CHECK(!t.is_cuda() && t.scalar_type() == type && t.is_contiguous() &&
+                    t.numel() >= least,
+                "stage_rows: a host tensor is missing or too small");
+  };
+  const bool last = starts.is_none();
+  TORCH_CHECK(counts.is_none() == last && block_size > 0);
+  pybind11::list from, many;
+  if (!last) from = starts, many = counts;
+  TORCH_CHECK(PyList_GET_SIZE(outputs.ptr()) == n &&
+              PyList_GET_SIZE(tables.ptr()) == n &&
+              (last || (PyList_GET_SIZE(from.ptr()) == n &&
+                        PyList_GET_SIZE(many.ptr()) == n)));
+  host(lens, torch::kInt32, n);
+  host(block_tables, torch::kInt32, 0);
+  TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) >= n);
+  host(ids, torch::kInt64, last ? n : 0);
+  host(pos, torch::kInt64, last ? n : 0);
+  host(slots, torch::kInt64, last ? n : 0);
+  const int64_t room =
+      std::min({ids.numel(), pos.numel(), slots.numel()});
+  const int64_t width = block_tables.size(1);
+  auto* to_ids = ids.data_ptr<int64_t>();
+  auto* to_pos = pos.data_ptr<int64_t>();
+  auto* to_slots = slots.data_ptr<int64_t>();
+  auto* to_lens = lens.data_ptr<int32_t>();
+  auto* to_table = block_tables.data_ptr<int32_t>();
+  auto whole = [](PyObject* o) {
+    const long long v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) throw pybind11::error_already_set();
+    return (int64_t)v;
+  };
+  auto list_of = [](PyObject* o) {
+    TORCH_CHECK(PyList_Check(o), "stage_rows: lists of lists");
+    return o;
+  };
+  int64_t at = 0;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* p = list_of(PyList_GET_ITEM(prompts.ptr(), i));
+    PyObject* o = list_of(PyList_GET_ITEM(outputs.ptr(), i));
+    PyObject* t = list_of(PyList_GET_ITEM(tables.ptr(), i));
+    const int64_t np = PyList_GET_SIZE(p), all = np + PyList_GET_SIZE(o);
+    const int64_t pages = PyList_GET_SIZE(t);
+    const int64_t s = last ? all - 1 : whole(PyList_GET_ITEM(from.ptr(), i));
+    const int64_t c = last ? 1 : whole(PyList_GET_ITEM(many.ptr(), i));
+    TORCH_CHECK(s >= 0 && c >= 0 && s + c <= all && at + c <= room &&
+                    pages <= width && s + c <= pages * block_size,
+                "stage_rows: tokens, pages or room missing");
+    int32_t* row = to_table + i * width;
+    for (int64_t j = 0; j < pages; ++j)
+      row[j] = (int32_t)whole(PyList_GET_ITEM(t, j));
+    for (int64_t j = s; j < s + c; ++j, ++at) {
+      to_ids[at] = whole(j < np ? PyList_GET_ITEM(p, j)
+                                : PyList_GET_ITEM(o, j - np));
+      to_pos[at] = j;
+      to_slots[at] = (int64_t)row[j / block_size] * block_size + j % block_size;
+    }
+    to_lens[i] = (int32_t)(s + c);
+  }
+}
+
 // The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
 // beyond this rank's El experts from expert_base on count as zero. tile: pairs
 // of a work item; mid: of 64 or 128 pairs in mid_gemm.hip, else in
@@ -796,6 +869,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("stream_sum", &stream_sum);
   m.def("tile_silu", &tile_silu);
   m.def("mid_gemm", &mid_gemm);
+  m.def("stage_rows", &stage_rows);
   m.def("moe_experts", &moe_experts);
   m.def("mfma_probe", &mfma_probe);
   m.def("mfma_probe32", &mfma_probe32);

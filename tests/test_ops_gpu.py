@@ -1281,6 +1281,18 @@ def test_mid_rule():
                 atol=2e-2, rtol=2e-2)  # both rounded to bf16, values up to 6
 
 
+def test_upload():
+    """Host tensors that travel together keep types, shapes and values."""
+    host = [torch.arange(7), None, torch.rand(3, 5), torch.empty(0, 4, dtype=torch.int32),
+            torch.tensor([[1], [2]], dtype=torch.int32), torch.arange(9).view(3, 3).t()]
+    for _ in range(3):  # the staging buffer comes back
+        moved = ops.upload(host, DEV)
+        for h, m in zip(host, moved):
+            assert (m is None) if h is None else (
+                m.is_cuda and m.dtype == h.dtype and m.is_contiguous()
+                and torch.equal(m.cpu(), h))
+
+
 def test_tiles_rule():
     """Rows that fill the chip's rounds take the tiles, others the library."""
     assert_native()

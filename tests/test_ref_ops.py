@@ -153,3 +153,56 @@ def test_short_portions_are_split_beside_long_ones():
     assert split([2048, 33, 33], [2048, 3000, 3000])[0] == {0: 3, 1: 8, 2: 8}
     assert split([65], [6113])[0] == {0: 8}
     assert split([0, 65], [400, 6113], min_ladder=1)[0] == {1: 8}
+
+
+def test_stage_rows():
+    """What a step's rows read: spans that begin in the prompt or in the output,
+    last tokens, pages; missing tokens, pages or room are refused."""
+    import random
+
+    import pytest
+
+    import arks_amd.ops as ops
+
+    if not ops.native_available():
+        pytest.skip("needs the built extension")
+    rng, bs = random.Random(5), 16
+    prompts = [[rng.randrange(1 << 20) for _ in range(n)] for n in (40, 1, 16, 33)]
+    outputs = [[rng.randrange(1 << 20) for _ in range(n)] for n in (0, 5, 1, 15)]
+    tables = [rng.sample(range(1 << 30), n) for n in (3, 1, 2, 4)]
+    starts, counts = [3, 0, 16, 30], [37, 6, 1, 17]
+
+    def host(rows, width=5):
+        return (torch.full((rows,), -7), torch.full((rows,), -7),
+                torch.full((rows,), -7), torch.full((6,), -7, dtype=torch.int32),
+                torch.full((6, width), -7, dtype=torch.int32))
+
+    def check(first, many, bufs):
+        ids, pos, slots, lens, bt = bufs
+        at = 0
+        for i, (p, o, t, c, n) in enumerate(zip(prompts, outputs, tables, first, many)):
+            for j in range(c, c + n):
+                assert ids[at] == (p + o)[j] and pos[at] == j
+                assert slots[at] == t[j // bs] * bs + j % bs
+                at += 1
+            assert lens[i] == c + n
+            assert bt[i].tolist() == t + [-7] * (5 - len(t))
+        assert (ids[at:] == -7).all() and (pos[at:] == -7).all()
+        assert (lens[4:] == -7).all() and (bt[4:] == -7).all()
+
+    bufs = host(64)
+    ops.stage_rows(prompts, outputs, tables, starts, counts, *bufs, bs)
+    check(starts, counts, bufs)
+    bufs = host(5)
+    ops.stage_rows(prompts, outputs, tables, None, None, *bufs, bs)
+    last = [len(p) + len(o) - 1 for p, o in zip(prompts, outputs)]
+    check(last, [1] * 4, bufs)
+    for bad in (dict(counts=[38, 6, 1, 17]), dict(starts=[-1, 0, 16, 30]),
+                dict(tables=[[1, 2], *tables[1:]]), dict(bufs=host(60)),
+                dict(bufs=host(64, 3)), dict(counts=[37, 6, 1]),
+                dict(outputs=[()] * 4), dict(starts=None)):
+        a = dict(starts=starts, counts=counts, tables=tables, outputs=outputs,
+                 bufs=host(64)) | bad
+        with pytest.raises((RuntimeError, TypeError)):
+            ops.stage_rows(prompts, a["outputs"], a["tables"], a["starts"],
+                           a["counts"], *a["bufs"], bs)
