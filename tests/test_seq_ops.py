@@ -314,3 +314,70 @@ def test_lightning_matrix_core_prefill_equals_general_kernel(D, V):
     assert (res[True][0] - res[False][0]).abs().max() < 1e-2 * scale
     sscale = res[False][1].abs().max()
     assert (res[True][1] - res[False][1]).abs().max() < 1e-2 * sscale
+
+
+def _scan64(u, dbc, z, dt_w, dt_b, A, Dp, st, R):
+    """One sequence, row by row in float64; (y, state, bound of |y|)."""
+    u, dbc, z, dt_w, dt_b, A, Dp, st = (
+        t.double().cpu() for t in (u, dbc, z, dt_w, dt_b, A, Dp, st))
+    N = A.shape[1]
+    dt = torch.nn.functional.softplus(dbc[:, :R] @ dt_w.t() + dt_b, threshold=1e9)
+    ys, mag, sm = [], [], st.abs()
+    for t in range(len(u)):
+        e = torch.exp(dt[t][:, None] * A)
+        dx = (dt[t] * u[t])[:, None] * dbc[t, R:R + N]
+        st, sm = e * st + dx, e * sm + dx.abs()
+        c = dbc[t, R + N:]
+        g = z[t] * torch.sigmoid(z[t])
+        ys.append(((st * c).sum(1) + Dp * u[t]) * g)
+        mag.append(((sm * c.abs()).sum(1) + (Dp * u[t]).abs()) * g.abs())
+    return torch.stack(ys), st, torch.stack(mag), sm
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C,N,lens", [
+    (8, 16, [1]),               # whole states, one row
+    (257, 16, [1, 64, 3]),      # a second workgroup with one channel
+    (300, 8, [65, 129]),        # chunks with a last row of one
+    (256, 32, [70]), (40, 64, [66]),
+    (129, 12, [1, 67]),         # fewer states than lanes hold
+    (33, 5, [64, 2])])
+def test_selective_scan_lanes_against_64_bits(C, N, lens, dtype):
+    """dt from a product, old states, and dt arguments from far below zero to
+    far above. A row's decay and step have a relative error of some 2^-23
+    (|argument of exp| < 88 at most counts, times 2^-24), and the rows add
+    theirs up; bf16 outputs are rounded once more."""
+    dev = "cuda"
+    torch.manual_seed(C + N)
+    T, S, R = sum(lens), len(lens), 4
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    meta = (i32(cu, dev), i32([n + 5 for n in lens], dev),
+            i32(list(range(S))[::-1], dev))
+    u = torch.randn(T, C, device=dev).to(dtype)
+    dbc = torch.randn(T, R + 2 * N, device=dev).to(dtype)
+    z = (torch.randn(T, C, device=dev) * 4).to(dtype)
+    z[0, :4] = torch.tensor([-200.0, 200.0, -90.0, 0.0], device=dev).to(dtype)
+    dt_w = torch.randn(C, R, device=dev) * 0.3
+    dt_b = torch.linspace(-120.0, 6.0, C, device=dev)
+    dt_b[1::2] = torch.linspace(-3.0, 3.0, C, device=dev)[1::2]
+    A = -torch.rand(C, N, device=dev) * 2
+    Dp = torch.randn(C, device=dev)
+    st0 = torch.randn(S + 1, C, N, device=dev)
+    dt_pre = (dbc[:, :R].double() @ dt_w.double().t()).float()
+    st = st0.clone()
+    y = ops.selective_scan(u, dbc, z, dt_w, dt_b, A, Dp, st, *meta,
+                           max_q_len=max(lens), dt_pre=dt_pre,
+                           chunks=ops.scan_chunks(lens, torch.device(dev)))
+    assert torch.equal(st[S], st0[S])
+    for i, n in enumerate(lens):
+        a, b, slot = cu[i], cu[i + 1], S - 1 - i
+        want, wst, mag, sm = _scan64(u[a:b], dbc[a:b], z[a:b], dt_w, dt_b, A, Dp,
+                                     st0[slot], R)
+        # a step's argument carries dt_pre + dt_b's rounding: up to 2^-24 * 120
+        rel = 2.0 ** -24 * (160 + 16 * n)
+        assert bool(((st[slot].double().cpu() - wst).abs() <= rel * sm + 1e-30).all())
+        tol = (rel + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) * mag + 1e-30
+        assert bool(((y[a:b].double().cpu() - want).abs() <= tol).all())
