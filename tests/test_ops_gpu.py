@@ -885,6 +885,37 @@ def test_moe_items(T, E, k, H, I, base, El, tile, skew):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("T,E,k,base,El", [
+    (1024, 8, 8, 0, 8), (1025, 8, 8, 0, 8),     # either side of one workgroup
+    (1280, 100, 8, 0, 100), (5012, 128, 8, 0, 128),  # ends of the runs
+    (8193, 2, 1, 0, 1), (4100, 64, 4, 48, 16),  # another rank's pairs
+    (9000, 1024, 16, 0, 1024),                  # more runs than workgroups
+])
+def test_moe_plan_many_pairs(T, E, k, base, El):
+    """Every pair finds its expert's row: experts that give sign and size of one
+    value, so that the mix is known exactly (small whole numbers)."""
+    assert_native()
+    torch.manual_seed(T)
+    x = torch.zeros(T, 8, device=DEV, dtype=torch.bfloat16)
+    x[:, 0] = 32.0
+    at = torch.arange(El, device=DEV) % 64
+    w13 = torch.zeros(El, 16, 8, device=DEV)
+    w13[:, 0, 0] = 1.0   # silu(32) is 32 in bf16
+    w13[:, 8, 0] = 1 / 32
+    w2 = torch.zeros(El, 8, 8, device=DEV)
+    w2[:, 0, 0] = (at + 1) / 32
+    w2[:, 1, 0] = (torch.arange(El, device=DEV) // 64 + 1) / 32
+    ids = torch.rand(T, E, device=DEV).topk(k).indices.int()
+    w = torch.randint(0, 2, (T, k), device=DEV).float()
+    out = ops.moe_experts(x, w13.bfloat16(), w2.bfloat16(), w, ids, base)
+    mine = ((ids >= base) & (ids < base + El)).float() * w
+    e = (ids - base).clamp(0, El - 1)
+    for col, val in ((0, e % 64 + 1), (1, e // 64 + 1)):
+        want = (mine * val).sum(1).bfloat16()  # sums below 2^24: one rounding
+        assert torch.equal(out[:, col], want)
+    assert not out[:, 2:].any()
+
+
 def test_moe_tile_rule():
     """The kernel that the number of pairs per expert asks for."""
     sizes = (1, 7, 16, 17, 1024, 1025)
