@@ -121,8 +121,14 @@ namespace arks {
 // PARTS: q, k and v are the sums of fp32 splits [splits, T, q | k | v] of the
 // projection (+ bias); k and v go to the cache alone. Saves the launch that
 // would add them (5 us at 64 rows of 4608).
+// W: pairs of a thread. Many tokens take 8 where rows and bases lie on 16 bytes:
+// one access of 16 bytes per half of a head instead of four, and a workgroup of
+// as many threads as a token has work. 5012 rows of 32/4 heads x 128 with norms
+// 35.3 -> 28.4 us, 8192 of 28/4 without 35 -> 30.6 (of about 27 for the bytes).
+// Few tokens and split sums keep 2: a thread's chain of loads is what they wait
+// for.
 // ---------------------------------------------------------------------------
-template <bool FP8, bool NORM, bool PARTS>
+template <bool FP8, bool NORM, bool PARTS, int W>
 __global__ void rope_cache_kernel(
     const int64_t* __restrict__ positions,
     bf16* __restrict__ q,        // [T, Hq*D] rows strided
@@ -162,20 +168,22 @@ __global__ void rope_cache_kernel(
   const int64_t hstride = (int64_t)block_size * head_dim;
 
   const int total_heads = num_q_heads + num_kv_heads;
-  const int pairs2 = half / 2;
+  typedef __attribute__((ext_vector_type(W))) unsigned short bits;
+  const int lanes = half / W;  // threads of a head
   const int first = blockIdx.y * blockDim.x + threadIdx.x;
   const int step = gridDim.y * blockDim.x;
-  for (int idx = first; idx < total_heads * pairs2; idx += step) {
-    const int h = idx / pairs2;
-    const int p2 = (idx % pairs2) * 2;
+  for (int idx = first; idx < total_heads * lanes; idx += step) {
+    const int h = idx / lanes;
+    const int p2 = (idx % lanes) * W;
     const bool is_q = h < num_q_heads;
     bf16* base = is_q
                      ? q + (int64_t)token * q_stride + (int64_t)h * head_dim
                      : k + (int64_t)token * k_stride +
                            (int64_t)(h - num_q_heads) * head_dim;
-    ushort2v o1, o2;
-    float a2[2], b2[2];
+    bits o1, o2;
+    float a2[W], b2[W];
     if constexpr (PARTS) {
+      static_assert(W == 2);
       const int c = h * head_dim + p2;
       f32x2 f1, f2;
       sum_parts_pair(part_row + c, part_row + c + half, part_stride, splits, f1,
@@ -189,28 +197,34 @@ __global__ void rope_cache_kernel(
         }
       }
     } else {
-      const ushort2v x1 = *reinterpret_cast<const ushort2v*>(base + p2);
-      const ushort2v x2 = *reinterpret_cast<const ushort2v*>(base + half + p2);
+      const bits x1 = *reinterpret_cast<const bits*>(base + p2);
+      const bits x2 = *reinterpret_cast<const bits*>(base + half + p2);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < W; ++j) {
         a2[j] = bf16_bits_to_float(x1[j]);
         b2[j] = bf16_bits_to_float(x2[j]);
       }
     }
     if constexpr (NORM) {
-      float ss = a2[0] * a2[0] + a2[1] * a2[1] + b2[0] * b2[0] + b2[1] * b2[1];
-      for (int off = pairs2 / 2; off > 0; off >>= 1)
+      float sa = 0.f, sb = 0.f;
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        sa += a2[j] * a2[j];
+        sb += b2[j] * b2[j];
+      }
+      float ss = sa + sb;
+      for (int off = lanes / 2; off > 0; off >>= 1)
         ss += __shfl_xor(ss, off, WAVE_SIZE);
       const float r = rsqrtf(ss / (float)head_dim + eps);
       const bf16* nw = is_q ? q_norm : k_norm;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < W; ++j) {
         a2[j] *= r * bf16_bits_to_float(nw[p2 + j]);
         b2[j] *= r * bf16_bits_to_float(nw[half + p2 + j]);
       }
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < W; ++j) {
       const float c = cs[p2 + j];
       const float s = cs[half + p2 + j];
       const float a = a2[j];
@@ -219,26 +233,30 @@ __global__ void rope_cache_kernel(
       o2[j] = float_to_bf16_bits(b * c + a * s);
     }
     if (!PARTS || is_q) {
-      *reinterpret_cast<ushort2v*>(base + p2) = o1;
-      *reinterpret_cast<ushort2v*>(base + half + p2) = o2;
+      *reinterpret_cast<bits*>(base + p2) = o1;
+      *reinterpret_cast<bits*>(base + half + p2) = o2;
     }
     if (!is_q && cache) {
       const int64_t dst = cbase + (int64_t)(h - num_q_heads) * hstride;
       if constexpr (FP8) {
         uint8_t* kc = reinterpret_cast<uint8_t*>(k_cache);
+        typedef __attribute__((ext_vector_type(W))) unsigned char bytes;
+        bytes y1, y2;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < W; ++j) {
           // convert from the bf16-ROUNDED values so the cache is
           // bit-identical to the separate rope + reshape_and_cache path
           __hip_fp8_e4m3 a(bf16_bits_to_float(o1[j]));
           __hip_fp8_e4m3 b(bf16_bits_to_float(o2[j]));
-          kc[dst + p2 + j] = a.__x;
-          kc[dst + half + p2 + j] = b.__x;
+          y1[j] = a.__x;
+          y2[j] = b.__x;
         }
+        *reinterpret_cast<bytes*>(kc + dst + p2) = y1;
+        *reinterpret_cast<bytes*>(kc + dst + half + p2) = y2;
       } else {
         bf16* kc = reinterpret_cast<bf16*>(k_cache);
-        *reinterpret_cast<ushort2v*>(kc + dst + p2) = o1;
-        *reinterpret_cast<ushort2v*>(kc + dst + half + p2) = o2;
+        *reinterpret_cast<bits*>(kc + dst + p2) = o1;
+        *reinterpret_cast<bits*>(kc + dst + half + p2) = o2;
       }
     }
   }
@@ -296,11 +314,18 @@ extern "C" void arks_rope_and_cache(
     int block_size, int64_t q_stride, int64_t k_stride, int kv_fp8,
     const void* q_norm, const void* k_norm, float eps, hipStream_t stream) {
   if (num_tokens == 0) return;
-  dim3 grid(num_tokens,
-            rope_groups(num_tokens, num_q_heads + num_kv_heads, head_dim)),
-      block(256);
+  const int heads = num_q_heads + num_kv_heads;
+  const bool wide =
+      num_tokens > 256 && head_dim % 16 == 0 && q_stride % 8 == 0 &&
+      k_stride % 8 == 0 &&
+      (((uintptr_t)q | (uintptr_t)k | (uintptr_t)k_cache | (uintptr_t)cos_sin |
+        (uintptr_t)q_norm | (uintptr_t)k_norm) & 15) == 0;
+  dim3 grid(num_tokens, rope_groups(num_tokens, heads, head_dim)), block(256);
+  if (wide) block.x = std::min(512, (heads * (head_dim / 16) + 63) / 64 * 64);
 #define ARKS_ROPE(FP8, NORM)                                                   \
-  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, false>), grid, block, 0,    \
+  if (wide) ARKS_ROPE_W(FP8, NORM, 8); else ARKS_ROPE_W(FP8, NORM, 2)
+#define ARKS_ROPE_W(FP8, NORM, W)                                              \
+  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, false, W>), grid, block, 0, \
                      stream,                                                   \
                      (const int64_t*)positions, (bf16*)q, (bf16*)k,            \
                      (const bf16*)v, k_cache, v_cache,                         \
@@ -308,11 +333,16 @@ extern "C" void arks_rope_and_cache(
                      head_dim, num_q_heads, num_kv_heads, block_size,          \
                      q_stride, k_stride, (const bf16*)q_norm,                  \
                      (const bf16*)k_norm, eps, nullptr, nullptr, 0)
-  if (kv_fp8) {
-    if (q_norm) ARKS_ROPE(true, true); else ARKS_ROPE(true, false);
+  if (kv_fp8 && q_norm) {
+    ARKS_ROPE(true, true);
+  } else if (kv_fp8) {
+    ARKS_ROPE(true, false);
+  } else if (q_norm) {
+    ARKS_ROPE(false, true);
   } else {
-    if (q_norm) ARKS_ROPE(false, true); else ARKS_ROPE(false, false);
+    ARKS_ROPE(false, false);
   }
+#undef ARKS_ROPE_W
 #undef ARKS_ROPE
 }
 
@@ -326,7 +356,7 @@ extern "C" void arks_rope_and_cache_parts(
             rope_groups(num_tokens, num_q_heads + num_kv_heads, head_dim)),
       block(256);
 #define ARKS_ROPE(FP8, NORM)                                                   \
-  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, true>), grid, block, 0,     \
+  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, true, 2>), grid, block, 0,  \
                      stream, (const int64_t*)positions, (bf16*)q, nullptr,     \
                      nullptr, k_cache, v_cache, (const int64_t*)slot_mapping,  \
                      (const float*)cos_sin, head_dim, num_q_heads,             \

@@ -916,6 +916,60 @@ def test_moe_plan_many_pairs(T, E, k, base, El):
     assert not out[:, 2:].any()
 
 
+@pytest.mark.parametrize("hq,hkv,hd,T,fp8,norm", [
+    (28, 4, 128, 257, False, False), (32, 4, 128, 300, False, True),
+    (3, 1, 64, 257, True, True), (5, 5, 32, 400, False, True),
+    (2, 1, 256, 260, True, False), (70, 8, 128, 258, False, True),
+    (4, 2, 16, 270, False, False), (4, 2, 24, 270, False, False)])
+def test_rope_and_cache_many_tokens(hq, hkv, hd, T, fp8, norm):
+    """Eight pairs a thread against two (up to 256 tokens): the same bits
+    without norms; with them a sum of squares in another order, 2^-24 each
+    step, so results round to neighbours at most. Rows off 16 bytes too."""
+    assert_native()
+    torch.manual_seed(hd + T)
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    width = (hq + 2 * hkv) * hd
+    nw = (1 + torch.randn(2, hd, device=DEV) * 0.2).bfloat16()
+    args = (nw[0], nw[1].contiguous(), 1e-6) if norm else ()
+    cos_sin = ref.rope_cos_sin_cache(hd, 64, 10000.0).cuda()
+    pos = torch.randint(0, 64, (T,), dtype=torch.int64, device=DEV)
+    slots = torch.randperm(40 * 16, device=DEV)[:T]
+    slots[7] = -1
+    data = torch.randn(T, width, device=DEV).bfloat16()
+    res = []
+    for pad, off, cut in ((8, 0, T), (0, 0, 100), (4, 0, T), (8, 2, T)):
+        if off and hd % 8:
+            continue
+        buf = torch.empty(T, width + pad, device=DEV, dtype=torch.bfloat16)
+        q, k, v = buf[:, :width].split([hq * hd, hkv * hd, hkv * hd], dim=-1)
+        if pad == 4:  # v is read 16 bytes at a time at any number of tokens
+            buf = torch.empty(T, 2 * width + 8, device=DEV, dtype=torch.bfloat16)
+            k, v = buf[:, :2 * hkv * hd].split([hkv * hd, hkv * hd], dim=-1)
+            q = torch.empty(T, hq * hd + 4, device=DEV,
+                            dtype=torch.bfloat16)[:, :hq * hd]
+        elif off:
+            q = torch.empty(T * hq * hd + 8, device=DEV, dtype=torch.bfloat16)[
+                off:off + T * hq * hd].view(T, hq * hd)
+        for t, d in zip((q, k, v), data.split([hq * hd, hkv * hd, hkv * hd], dim=-1)):
+            t.copy_(d)
+        kc = torch.zeros(40, hkv, 16, hd, device=DEV).to(dt)
+        vc = torch.zeros_like(kc)
+        for a in range(0, T, cut):
+            b = min(T, a + cut)
+            ops.rope_and_cache(pos[a:b], q[a:b], k[a:b], v[a:b], kc, vc,
+                               slots[a:b], cos_sin, hd, *args)
+        res.append((q.float(), k.float(), kc.float(), vc.float()))
+    for other in res[1:]:
+        assert torch.equal(res[0][3], other[3])
+        for a, b in zip(res[0][:3], other[:3]):
+            if norm:  # neighbours: 2^-7 of a bf16 value, 2^-3 of an e4m3 one
+                rel = 2 ** -3 if fp8 and a is res[0][2] else 2 ** -7
+                torch.testing.assert_close(a, b, rtol=rel, atol=2 ** -9 if fp8
+                                           else 1e-5)
+            else:
+                assert torch.equal(a, b)
+
+
 def test_moe_tile_rule():
     """The kernel that the number of pairs per expert asks for."""
     sizes = (1, 7, 16, 17, 1024, 1025)
