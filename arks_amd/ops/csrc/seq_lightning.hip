@@ -31,7 +31,10 @@ __device__ __forceinline__ float rotated_ld(const AT* row, int d, float pos,
   return first ? x * cs - y * sn : x * cs + y * sn;
 }
 
-template <typename AT, int DMAX, int MODE>
+// WHOLE: D == DMAX and V % 64 == 0. A row is bound by its state's read and write;
+// with a test per value the loads waited for each other (8 single rows of 32
+// heads x 128 x 128: 30.4 -> 10.9 us).
+template <typename AT, int DMAX, int MODE, bool WHOLE>
 __global__ __launch_bounds__(64) void lightning_scan_kernel(
     float* __restrict__ out, const AT* __restrict__ q, const AT* __restrict__ k,
     const AT* __restrict__ v, int64_t ldq, int64_t ldk, int64_t ldv,
@@ -48,14 +51,19 @@ __global__ __launch_bounds__(64) void lightning_scan_kernel(
   if (rows == 0) return;
   const int start = seq_lens[s] - rows;
   const int slot = slots[s];
-  const bool live = col < V;
+  const bool live = WHOLE || col < V;
   const float lam = decay[h];
   float S[DMAX];
   float* sp = state + (((int64_t)(slot < 0 ? 0 : slot) * H + h) * D) * V + col;
   const bool has_state = start > 0 && slot >= 0 && live;
+  if (WHOLE && !has_state) {
 #pragma unroll
-  for (int d = 0; d < DMAX; ++d)
-    S[d] = (has_state && d < D) ? sp[(int64_t)d * V] : 0.f;
+    for (int d = 0; d < DMAX; ++d) S[d] = 0.f;
+  } else {
+#pragma unroll
+    for (int d = 0; d < DMAX; ++d)
+      S[d] = WHOLE || (has_state && d < D) ? sp[(int64_t)d * V] : 0.f;
+  }
   for (int r = 0; r < rows; ++r) {
     const int t = a + r;
     const int buf = r & 1;  // double buffer: one barrier per row
@@ -82,7 +90,7 @@ __global__ __launch_bounds__(64) void lightning_scan_kernel(
     float o = 0.f;
 #pragma unroll
     for (int d = 0; d < DMAX; ++d) {
-      if (d < D) {
+      if (WHOLE || d < D) {
         S[d] = lam * S[d] + k_s[buf][d] * vv;
         o += S[d] * q_s[buf][d];
       }
@@ -92,7 +100,7 @@ __global__ __launch_bounds__(64) void lightning_scan_kernel(
   if (slot >= 0 && live) {
 #pragma unroll
     for (int d = 0; d < DMAX; ++d)
-      if (d < D) sp[(int64_t)d * V] = S[d];
+      if (WHOLE || d < D) sp[(int64_t)d * V] = S[d];
   }
 }
 
@@ -175,11 +183,16 @@ static int launch_lightning(float* out, const void* q, const void* k,
                             int n_rot, int interleaved, float k_scale,
                             hipStream_t stream) {
   dim3 grid(S, H, (V + 63) / 64), block(64);
-#define LL(DM)                                                                 \
-  hipLaunchKernelGGL((lightning_scan_kernel<AT, DM, MODE>), grid, block, 0,    \
+#define LL_W(DM, W)                                                            \
+  hipLaunchKernelGGL((lightning_scan_kernel<AT, DM, MODE, W>), grid, block, 0, \
                      stream, out, (const AT*)q, (const AT*)k, (const AT*)v,    \
                      ldq, ldk, ldv, decay, state, cu, seq_lens, slots, H, D,   \
                      V, positions, freq, n_rot, interleaved, k_scale)
+#define LL(DM)                                                                 \
+  do {                                                                         \
+    if (D == DM && V % 64 == 0) LL_W(DM, true);                                \
+    else LL_W(DM, false);                                                      \
+  } while (0)
   if (D <= 16) LL(16);
   else if (D <= 32) LL(32);
   else if (D <= 64) LL(64);
@@ -187,6 +200,7 @@ static int launch_lightning(float* out, const void* q, const void* k,
   else if (D <= 256) LL(256);
   else return 1;
 #undef LL
+#undef LL_W
   return 0;
 }
 

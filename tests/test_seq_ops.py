@@ -381,3 +381,40 @@ def test_selective_scan_lanes_against_64_bits(C, N, lens, dtype):
         assert bool(((st[slot].double().cpu() - wst).abs() <= rel * sm + 1e-30).all())
         tol = (rel + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) * mag + 1e-30
         assert bool(((y[a:b].double().cpu() - want).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,V", [(16, 64), (128, 128), (256, 64),  # whole
+                                 (128, 72), (100, 64), (17, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_lightning_rows_against_64_bits(D, V, dtype):
+    """Rows walked one by one: states whole in a wave's registers and not, an
+    old state, a fresh one and a padding row. A state value takes two
+    operations a row and a sum of D terms: 2^-23 of the terms' size each."""
+    dev = "cuda"
+    torch.manual_seed(D + V)
+    H, lens = 3, [1, 5, 1]
+    T = sum(lens)
+    q, k, v = (torch.randn(T, H, n, device=dev).to(dtype) for n in (D, D, V))
+    decay = torch.tensor([1.0, 0.9, 0.0], device=dev)
+    st0 = torch.randn(4, H, D, V, device=dev)
+    st = st0.clone()
+    o = ops.lightning_scan(q, k, v, decay, st, i32([0, 1, 6, 7], dev),
+                           i32([9, 5, 4], dev), i32([2, 0, -1], dev), max_q_len=5)
+    silu = lambda t: torch.nn.functional.silu(t.double())
+    a, b, c, lam = silu(q), silu(k), silu(v), decay.double()[:, None, None]
+    at = 0
+    for n, slot, old in zip(lens, (2, 0, -1), (True, False, False)):
+        S = st0[slot].double() if old else torch.zeros_like(st0[0]).double()
+        M = S.abs()
+        for t in range(at, at + n):
+            kv = b[t][:, :, None] * c[t][:, None, :]
+            S, M = lam * S + kv, lam * M + kv.abs()
+            want = (S * a[t][:, :, None]).sum(1)
+            tol = (M * a[t].abs()[:, :, None]).sum(1) * 2.0 ** -23 * (D + 16)
+            assert bool(((o[t].double() - want).abs() <= tol + 1e-12).all())
+        if slot >= 0:
+            assert bool(((st[slot].double() - S).abs()
+                         <= 2.0 ** -23 * 16 * M + 1e-12).all())
+        at += n
+    assert torch.equal(st[1], st0[1]) and torch.equal(st[3], st0[3])
