@@ -418,3 +418,58 @@ def test_lightning_rows_against_64_bits(D, V, dtype):
                          <= 2.0 ** -23 * 16 * M + 1e-12).all())
         at += n
     assert torch.equal(st[1], st0[1]) and torch.equal(st[3], st0[3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W", [4, 1024, 1028, 2052, 4096, 8192, 8196, 1030])
+@pytest.mark.parametrize("gated", [False, True])
+def test_rms_norm_of_float_rows_against_64_bits(W, gated):
+    """Rows of every width class to bf16, plain and times a gate's sigmoid from
+    strided rows, on 8 bytes and off them: one rounding (2^-9 either way) of a
+    value with a relative error of some 2^-22."""
+    dev, T = "cuda", 3
+    torch.manual_seed(W)
+    x = torch.randn(T, W, device=dev) * 5
+    w = torch.randn(W, device=dev)
+    want = x.double() * torch.rsqrt(x.double().pow(2).mean(1, keepdim=True) + 1e-5)
+    want = want * w.double()
+    if not gated:
+        got = [ops.rms_norm_f32(x, w, 1e-5, torch.bfloat16)]
+    else:
+        buf = torch.randn(T, 2 * W + 9, device=dev).bfloat16()
+        got, wants = [], []
+        for gate in (buf[:, :W], buf[:, 1:W + 1], buf[:, :W].contiguous()):
+            out = torch.empty(T, W, device=dev, dtype=torch.bfloat16)
+            ops._native_seq().gated_rmsnorm(out, x, w, gate, 1e-5)
+            got.append(out)
+            wants.append(want * torch.sigmoid(gate.double()))
+    for i, g in enumerate(got):
+        ref = wants[i] if gated else want
+        assert bool(((g.double() - ref).abs() <= (2.0 ** -8) * ref.abs() + 1e-30).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_head_norm_rotation_of_few_and_many_rows(dtype):
+    """The same bits whether a row's heads are shared by several workgroups (up
+    to 256 rows) or walked by one; turned values, a row without a page."""
+    dev, T, H, G, D, V = "cuda", 300, 5, 3, 24, 40
+    torch.manual_seed(1)
+    q, k, v = (torch.randn(T, h, d, device=dev).to(dtype)
+               for h, d in ((H, D), (G, D), (G, V)))
+    qw, kw = torch.randn(2, D, device=dev)
+    f, fv = torch.rand(10, device=dev), torch.rand(V // 2, device=dev)
+    pos = torch.randint(0, 5000, (T,), device=dev)
+    slots = torch.randperm(320, device=dev)[:T]
+    slots[5] = -1
+    res = []
+    for cut in (T, 37):
+        kc = torch.zeros(20, G, 16, D, device=dev, dtype=dtype)
+        vc = torch.zeros(20, G, 16, V, device=dev, dtype=dtype)
+        qo = torch.cat([ops.qk_norm_rope_cache(
+            *(t[a:a + cut] for t in (q, k, v)), qw, kw.contiguous(), 1e-5,
+            pos[a:a + cut], f, fv, kc, vc, slots[a:a + cut])
+            for a in range(0, T, cut)])
+        res.append((qo, kc, vc))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
