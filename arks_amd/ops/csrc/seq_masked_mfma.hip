@@ -394,23 +394,49 @@ void attn_masked_tile_kernel(
   }
 }
 
-// Merge the key-split partials of one (row, head): ws [T, H, ks, V + 2].
-__global__ __launch_bounds__(64) void attn_masked_combine_kernel(
+// Merge the key-split partials of one (row, head): ws [T, H, ks, V + 2]. Bound
+// by its chain of loads at few rows, so the splits are loaded 16 at a time and
+// a thread has one or two values: 8 rows of 32 heads x 512 in 16 splits 6.2 us
+// (40.3 with one wave and a load per term). The order of the sums is that of
+// the splits.
+__global__ __launch_bounds__(256) void attn_masked_combine_kernel(
     bf16* __restrict__ out, int64_t ldo, const float* __restrict__ ws, int H,
     int V, int ks, float out_scale) {
+  constexpr int PB = 16;
   const int t = blockIdx.x, h = blockIdx.y;
   const float* wp = ws + ((int64_t)t * H + h) * ks * (V + 2);
   float m = -FLT_MAX;
-  for (int z = 0; z < ks; ++z) m = fmaxf(m, wp[z * (V + 2) + V]);
-  float l = 0.f;
-  for (int z = 0; z < ks; ++z)
-    l += wp[z * (V + 2) + V + 1] * __expf(wp[z * (V + 2) + V] - m);
-  const float inv = l > 0.f ? out_scale / l : 0.f;
-  for (int d = threadIdx.x; d < V; d += 64) {
-    float acc = 0.f;
-    for (int z = 0; z < ks; ++z)
-      acc += wp[z * (V + 2) + d] * __expf(wp[z * (V + 2) + V] - m);
-    out[(int64_t)t * ldo + (int64_t)h * V + d] = float_to_bf16_bits(acc * inv);
+  for (int z0 = 0; z0 < ks; z0 += PB) {
+    float mz[PB];
+#pragma unroll
+    for (int j = 0; j < PB; ++j) mz[j] = wp[min(z0 + j, ks - 1) * (V + 2) + V];
+#pragma unroll
+    for (int j = 0; j < PB; ++j) m = fmaxf(m, mz[j]);
+  }
+  for (int d0 = 0; d0 < V; d0 += blockDim.x) {
+    const int d = min(d0 + (int)threadIdx.x, V - 1);
+    float l = 0.f, acc = 0.f;
+    for (int z0 = 0; z0 < ks; z0 += PB) {
+      float mz[PB], lz[PB], a[PB];
+#pragma unroll
+      for (int j = 0; j < PB; ++j) {
+        const float* zp = wp + min(z0 + j, ks - 1) * (V + 2);
+        mz[j] = zp[V];
+        lz[j] = zp[V + 1];
+        a[j] = zp[d];
+      }
+#pragma unroll
+      for (int j = 0; j < PB; ++j) {
+        if (z0 + j < ks) {
+          const float f = __expf(mz[j] - m);
+          l += lz[j] * f;
+          acc += a[j] * f;
+        }
+      }
+    }
+    const float inv = l > 0.f ? out_scale / l : 0.f;
+    if (d0 + (int)threadIdx.x < V)
+      out[(int64_t)t * ldo + (int64_t)h * V + d] = float_to_bf16_bits(acc * inv);
   }
 }
 
@@ -700,9 +726,9 @@ int launch_masked_tile(dim3 grid, hipStream_t stream, bf16* out, int64_t ldo,
                      kv_lens, cu, token_seq, sink_w, num_seqs, a, G, H,
                      hpt_shift, max_blocks, ws);
   if (grid.z > 1)
-    hipLaunchKernelGGL(attn_masked_combine_kernel, dim3(grid.y, H), dim3(64),
-                       0, stream, out, ldo, ws, H, V, (int)grid.z,
-                       a.out_scale);
+    hipLaunchKernelGGL(attn_masked_combine_kernel, dim3(grid.y, H),
+                       dim3(std::min(256, (V + 63) / 64 * 64)), 0, stream, out,
+                       ldo, ws, H, V, (int)grid.z, a.out_scale);
   return 0;
 }
 

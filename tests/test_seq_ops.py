@@ -449,6 +449,34 @@ def test_rms_norm_of_float_rows_against_64_bits(W, gated):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,V", [(64, 64), (128, 128)])
+@pytest.mark.parametrize("n", [33, 65, 200, 700, 1100])
+def test_masked_rows_merge_their_key_splits(D, V, n):
+    """A row behind contexts that are cut in 1 to 16 runs, a full one among
+    sequences of other lengths. The weights are rounded to bf16 (2^-9 of
+    each term) and the result once more."""
+    dev, G, H = "cuda", 2, 8
+    torch.manual_seed(n)
+    lens = [n, 1, n // 2 + 1]
+    pages = -(-n // 16)
+    kc = torch.randn(3 * pages, G, 16, D, device=dev).bfloat16()
+    vc = torch.randn(3 * pages, G, 16, V, device=dev).bfloat16()
+    table = torch.randperm(3 * pages).view(3, pages)
+    q = torch.randn(3, H, D, device=dev).bfloat16()
+    out = torch.empty(3, H, V, dtype=torch.bfloat16, device=dev)
+    assert ops._native_seq().attention_masked_mfma(
+        out, q, kc, vc, table.int().to(dev), i32(lens, dev), i32([0, 1, 2, 3], dev),
+        i32([0, 1, 2], dev), D ** -0.5, None, 0.0, 0, 0, 1.0, False, 1)
+    for i, L in enumerate(lens):
+        k, v = (c[table[i].to(dev)].transpose(1, 2).reshape(-1, G, c.shape[3])[:L]
+                .double().repeat_interleave(H // G, 1) for c in (kc, vc))
+        p = torch.softmax((k * q[i].double()).sum(2) * D ** -0.5, 0)
+        want = (p[:, :, None] * v).sum(0)
+        tol = 2.0 ** -7 * (p[:, :, None] * v.abs()).sum(0)
+        assert bool(((out[i].double() - want).abs() <= tol).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_head_norm_rotation_of_few_and_many_rows(dtype):
     """The same bits whether a row's heads are shared by several workgroups (up
