@@ -21,7 +21,15 @@
 // D[m][n] = sum_k a[m][k] b[n][k]; a lane holds row (lane % 16) and k =
 // 8 (lane / 16) .. +7 of each 32-wide k step; the result lane holds column
 // n = lane % 16, rows m = 4 (lane / 16) + r. So every operand sits in LDS
-// with k contiguous: V, decayed K and the state are staged transposed.
+// with k contiguous: V and decayed K are staged transposed.
+//
+// Bound by the bytes (the states above all) and, before them, by the staging:
+// with a load of 2 bytes at a time, one 2-byte write across LDS rows each, and
+// every wave reading the whole state in the product's loop the passes took 142
+// and 216 us for 3853 rows of 32 heads x 128 x 128. VEC (MODE 0, rows on 16
+// bytes): all loads of a thread are issued first, 16 bytes each, the transposed
+// operands written as words of two rows; pass 2 loads its state before all
+// else: 56 and 85 us, the same bits.
 #include "seq_common.h"
 
 namespace arks {
@@ -96,6 +104,7 @@ __device__ __forceinline__ lm_f32x4 lm_mfma_r(const bf16* a, ushort8 ub,
 }
 
 __device__ __forceinline__ void split_bf16(float x, bf16& hi, bf16& lo) {
+#pragma clang fp contract(off)  // x may be a product: the rounded one, everywhere
   hi = float_to_bf16_bits(x);
   lo = float_to_bf16_bits(x - bf16_bits_to_float(hi));
 }
@@ -105,8 +114,51 @@ __device__ __forceinline__ float decay_pow(float log2_decay, int e) {
   return e == 0 ? 1.f : __builtin_amdgcn_exp2f(log2_decay * (float)e);
 }
 
+// 8 neighbouring values of a row, zeros beyond the chunk's rows.
+__device__ __forceinline__ ushort8 lm_row8(const bf16* p, bool live) {
+  return live ? *reinterpret_cast<const ushort8*>(p) : ushort8{};
+}
+
+__device__ __forceinline__ float lm_silu(bf16 x) {
+  return silu_f(bf16_bits_to_float(x));
+}
+
+// VEC staging of a transposed operand: item i of 32 * (W / 8) is 8 dims of two
+// neighbouring rows, so that the 32 lanes of a dim write 32 words side by side.
+// Loads of all a thread's items, then their conversion.
+template <int W>
+struct LmPairs {
+  static constexpr int ITEMS = 4 * W, N = (ITEMS + 255) / 256;
+  ushort8 a[N], b[N];
+  __device__ __forceinline__ void load(const bf16* rows, int64_t ld, int n,
+                                       int tid) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int i = tid + 256 * u, j = 2 * (i % 32), d = i / 32 * 8;
+      const bool in = ITEMS % 256 == 0 || i < ITEMS;
+      a[u] = lm_row8(rows + (int64_t)j * ld + d, in && j < n);
+      b[u] = lm_row8(rows + (int64_t)(j + 1) * ld + d, in && j + 1 < n);
+    }
+  }
+};
+
+template <int V>
+__device__ __forceinline__ void lm_stage_values(bf16* vt, int ld,
+                                                const LmPairs<V>& vp, int tid) {
+#pragma unroll
+  for (int u = 0; u < LmPairs<V>::N; ++u) {
+    const int i = tid + 256 * u, j = 2 * (i % 32), c = i / 32 * 8;
+    if (i >= LmPairs<V>::ITEMS) break;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      *reinterpret_cast<uint32_t*>(&vt[(c + e) * ld + j]) =
+          float_to_bf16_bits(lm_silu(vp.a[u][e])) |
+          (uint32_t)float_to_bf16_bits(lm_silu(vp.b[u][e])) << 16;
+  }
+}
+
 // ---- pass 1: end state of each chunk scanned from zero
-template <int D, int V, int MODE>
+template <int D, int V, int MODE, bool VEC>
 __global__ __launch_bounds__(256) void lightning_state_mfma_kernel(
     float* __restrict__ part,  // [chunks, H, V, D] (transposed states)
     const bf16* __restrict__ k, const bf16* __restrict__ v, int64_t ldk,
@@ -121,7 +173,30 @@ __global__ __launch_bounds__(256) void lightning_state_mfma_kernel(
   const int row0 = cu[ch], n = cu[ch + 1] - row0;
   const float l2 = log2f(decay[h]);
   const int tid = threadIdx.x;
-  if (MODE == 0) {
+  if constexpr (VEC) {
+    LmPairs<D> kp;
+    LmPairs<V> vp;
+    kp.load(k + (int64_t)row0 * ldk + (int64_t)h * D, ldk, n, tid);
+    vp.load(v + (int64_t)row0 * ldv + (int64_t)h * V, ldv, n, tid);
+#pragma unroll
+    for (int u = 0; u < LmPairs<D>::N; ++u) {
+      const int i = tid + 256 * u, j = 2 * (i % 32), d = i / 32 * 8;
+      if (i >= LmPairs<D>::ITEMS) break;
+      const float f0 = decay_pow(l2, max(n - 1 - j, 0));
+      const float f1 = decay_pow(l2, max(n - 2 - j, 0));
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        bf16 h0, l0, h1, l1;
+        split_bf16(lm_silu(kp.a[u][e]) * f0, h0, l0);
+        split_bf16(lm_silu(kp.b[u][e]) * f1, h1, l1);
+        *reinterpret_cast<uint32_t*>(&kt_hi[(d + e) * LK + j]) =
+            h0 | (uint32_t)h1 << 16;
+        *reinterpret_cast<uint32_t*>(&kt_lo[(d + e) * LK + j]) =
+            l0 | (uint32_t)l1 << 16;
+      }
+    }
+    lm_stage_values<V>(vt, LK, vp, tid);
+  } else if (MODE == 0) {
     for (int i = tid; i < LM_ROWS * D; i += 256) {
       const int j = i / D, d = i - j * D;
       float x = 0.f;
@@ -150,7 +225,7 @@ __global__ __launch_bounds__(256) void lightning_state_mfma_kernel(
       split_bf16(x1, kt_hi[d1 * LK + j], kt_lo[d1 * LK + j]);
     }
   }
-  for (int i = tid; i < LM_ROWS * V; i += 256) {
+  for (int i = tid; !VEC && i < LM_ROWS * V; i += 256) {
     const int j = i / V, c = i - j * V;
     float x = 0.f;
     if (j < n) {
@@ -175,21 +250,20 @@ __global__ __launch_bounds__(256) void lightning_state_mfma_kernel(
 #pragma unroll
       for (int c = 0; c < VT; ++c) {
         const bf16* a = vt + (c * 16 + lq) * LK + ko;  // rows = value dims
-        acc[c] = lm_mfma(a, bh, acc[c]);
-        acc[c] = lm_mfma(a, bl, acc[c]);
+        acc[c] = lm_mfma(bh, a, acc[c]);
+        acc[c] = lm_mfma(bl, a, acc[c]);
       }
     }
-    // result rows m = value dim, column n = key dim: out[v][d]
+    // result rows m = key dim, column n = value dim: out[v][d]
 #pragma unroll
     for (int c = 0; c < VT; ++c)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        out[(int64_t)(c * 16 + 4 * la + r) * D + dt * 16 + lq] = acc[c][r];
+      *reinterpret_cast<lm_f32x4*>(
+          &out[(int64_t)(c * 16 + lq) * D + dt * 16 + 4 * la]) = acc[c];
   }
 }
 
 // ---- pass 2: outputs of each chunk from its start state
-template <int D, int V, int MODE>
+template <int D, int V, int MODE, bool VEC>
 __global__ __launch_bounds__(256) void lightning_out_mfma_kernel(
     float* __restrict__ out,         // [T, H, V] fp32
     const float* __restrict__ part,  // [chunks, H, V, D] start states^T
@@ -209,7 +283,48 @@ __global__ __launch_bounds__(256) void lightning_out_mfma_kernel(
   const int row0 = cu[ch], n = cu[ch + 1] - row0;
   const float l2 = log2f(decay[h]);
   const int tid = threadIdx.x;
-  if (MODE == 0) {
+  const int wave = tid / 64, lane = tid % 64, lq = lane % 16, la = lane / 16;
+  // The second products' tiles: a wave has CT tiles of the values and RT of the
+  // rows, so that a value of the state is read and split by one wave (two of
+  // them at V = 32). Its loads are the first that are issued.
+  constexpr int VT = V / 16;
+  constexpr int WC = VT < 4 ? VT : 4, CT = VT / WC, RT = WC;
+  const int c0 = wave % WC * CT, r0 = wave / WC * RT;
+  const float* sp = part + ((int64_t)ch * H + h) * D * V;  // [V][D]
+  float4v sr[D / 32][CT][2];
+#pragma unroll
+  for (int st = 0; st < D / 32; ++st)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const float* p = sp + (int64_t)((c0 + c) * 16 + lq) * D + st * 32 + 8 * la;
+      sr[st][c][0] = *reinterpret_cast<const float4v*>(p);
+      sr[st][c][1] = *reinterpret_cast<const float4v*>(p + 4);
+    }
+  if constexpr (VEC) {
+    constexpr int NR = LM_ROWS * D / 8 / 256;
+    ushort8 q8[NR], k8[NR];
+    LmPairs<V> vp;
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      const int i = tid + 256 * u, j = i / (D / 8), d = i % (D / 8) * 8;
+      q8[u] = lm_row8(q + (int64_t)(row0 + j) * ldq + (int64_t)h * D + d, j < n);
+      k8[u] = lm_row8(k + (int64_t)(row0 + j) * ldk + (int64_t)h * D + d, j < n);
+    }
+    vp.load(v + (int64_t)row0 * ldv + (int64_t)h * V, ldv, n, tid);
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      const int i = tid + 256 * u, j = i / (D / 8), d = i % (D / 8) * 8;
+      ushort8 oq, ok;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        oq[e] = float_to_bf16_bits(lm_silu(q8[u][e]));
+        ok[e] = float_to_bf16_bits(lm_silu(k8[u][e]));
+      }
+      *reinterpret_cast<ushort8*>(&qs[j * LD + d]) = oq;
+      *reinterpret_cast<ushort8*>(&ks[j * LD + d]) = ok;
+    }
+    lm_stage_values<V>(vt, LK, vp, tid);
+  } else if (MODE == 0) {
     for (int i = tid; i < LM_ROWS * D; i += 256) {
       const int j = i / D, d = i - j * D;
       float xq = 0.f, xk = 0.f;
@@ -245,7 +360,7 @@ __global__ __launch_bounds__(256) void lightning_out_mfma_kernel(
       ks[j * LD + d1] = float_to_bf16_bits(k1);
     }
   }
-  for (int i = tid; i < LM_ROWS * V; i += 256) {
+  for (int i = tid; !VEC && i < LM_ROWS * V; i += 256) {
     const int j = i / V, c = i - j * V;
     float x = 0.f;
     if (j < n) {
@@ -254,9 +369,7 @@ __global__ __launch_bounds__(256) void lightning_out_mfma_kernel(
     }
     vt[c * LK + j] = float_to_bf16_bits(x);
   }
-  const float* sp = part + ((int64_t)ch * H + h) * D * V;  // [V][D]
   __syncthreads();
-  const int wave = tid / 64, lane = tid % 64, lq = lane % 16, la = lane / 16;
   // scores of this wave's 16 rows against all 64 keys, decayed and masked,
   // into a_hi/a_lo[i][j] (each wave writes only its own rows)
   const int irow = wave * 16 + lq;  // the row this lane's score column is
@@ -276,61 +389,69 @@ __global__ __launch_bounds__(256) void lightning_out_mfma_kernel(
     }
   }
   __syncthreads();
-  constexpr int VT = V / 16;
-  lm_f32x4 acc[VT], acs[VT];
+  lm_f32x4 acc[RT][CT], acs[RT][CT];
 #pragma unroll
-  for (int c = 0; c < VT; ++c) {
-    acc[c] = {0.f, 0.f, 0.f, 0.f};
-    acs[c] = {0.f, 0.f, 0.f, 0.f};
-  }
-  const int arow = wave * 16 + lq;  // A-operand row of this lane
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      acc[t][c] = {0.f, 0.f, 0.f, 0.f};
+      acs[t][c] = {0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
   for (int st = 0; st < LM_ROWS / 32; ++st) {
     const int ko = st * 32 + 8 * la;
 #pragma unroll
-    for (int c = 0; c < VT; ++c) {
-      const bf16* b = vt + (c * 16 + lq) * LK + ko;
-      acc[c] = lm_mfma(a_hi + arow * LK + ko, b, acc[c]);
-      acc[c] = lm_mfma(a_lo + arow * LK + ko, b, acc[c]);
+    for (int c = 0; c < CT; ++c) {
+      const bf16* b = vt + ((c0 + c) * 16 + lq) * LK + ko;
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int arow = (r0 + t) * 16 + lq;  // A-operand row of this lane
+        acc[t][c] = lm_mfma(a_hi + arow * LK + ko, b, acc[t][c]);
+        acc[t][c] = lm_mfma(a_lo + arow * LK + ko, b, acc[t][c]);
+      }
     }
   }
 #pragma unroll
   for (int st = 0; st < D / 32; ++st) {
     const int ko = st * 32 + 8 * la;
 #pragma unroll
-    for (int c = 0; c < VT; ++c) {
-      // 8 consecutive key dims of state row v = 16 c + lq, fp32 -> hi + lo
-      const float* sr = sp + (int64_t)(c * 16 + lq) * D + ko;
-      const float4v s0 = *reinterpret_cast<const float4v*>(sr);
-      const float4v s1 = *reinterpret_cast<const float4v*>(sr + 4);
+    for (int c = 0; c < CT; ++c) {
+      // 8 consecutive key dims of a state row v, fp32 -> hi + lo
       ushort8 bh, bl;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         bf16 h0, l0, h1, l1;
-        split_bf16(s0[e], h0, l0);
-        split_bf16(s1[e], h1, l1);
+        split_bf16(sr[st][c][0][e], h0, l0);
+        split_bf16(sr[st][c][1][e], h1, l1);
         bh[e] = h0; bl[e] = l0; bh[4 + e] = h1; bl[4 + e] = l1;
       }
-      acs[c] = lm_mfma_r(qs + arow * LD + ko, bh, acs[c]);
-      acs[c] = lm_mfma_r(qs + arow * LD + ko, bl, acs[c]);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const bf16* qr = qs + ((r0 + t) * 16 + lq) * LD + ko;
+        acs[t][c] = lm_mfma_r(qr, bh, acs[t][c]);
+        acs[t][c] = lm_mfma_r(qr, bl, acs[t][c]);
+      }
     }
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = wave * 16 + 4 * la + r;
-    if (i >= n) continue;
-    const float carry = decay_pow(l2, i + 1);
-    float* orow = out + ((int64_t)(row0 + i) * H + h) * V;
+  for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int c = 0; c < VT; ++c) orow[c * 16 + lq] = acc[c][r] + carry * acs[c][r];
-  }
+    for (int r = 0; r < 4; ++r) {
+      const int i = (r0 + t) * 16 + 4 * la + r;
+      if (i >= n) continue;
+      const float carry = decay_pow(l2, i + 1);
+      float* orow = out + ((int64_t)(row0 + i) * H + h) * V;
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        orow[(c0 + c) * 16 + lq] = acc[t][c][r] + carry * acs[t][c][r];
+    }
 }
 
 }  // namespace arks
 
 using namespace arks;
 
-template <int D, int V, int MODE>
+template <int D, int V, int MODE, bool VEC>
 static void launch_lm(float* out, float* part, const void* q, const void* k,
                       const void* v, int64_t ldq, int64_t ldk, int64_t ldv,
                       const float* decay, const int* cu, int chunks, int H,
@@ -342,11 +463,11 @@ static void launch_lm(float* out, float* part, const void* q, const void* k,
     static bool set = false;
     if (!set) {
       (void)hipFuncSetAttribute(
-          reinterpret_cast<const void*>(lightning_state_mfma_kernel<D, V, MODE>),
+          reinterpret_cast<const void*>(lightning_state_mfma_kernel<D, V, MODE, VEC>),
           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       set = true;
     }
-    hipLaunchKernelGGL((lightning_state_mfma_kernel<D, V, MODE>), grid, block, lds,
+    hipLaunchKernelGGL((lightning_state_mfma_kernel<D, V, MODE, VEC>), grid, block, lds,
                        stream, part, (const bf16*)k, (const bf16*)v, ldk, ldv,
                        decay, cu, H, rot);
   } else {
@@ -354,11 +475,11 @@ static void launch_lm(float* out, float* part, const void* q, const void* k,
     static bool set = false;
     if (!set) {
       (void)hipFuncSetAttribute(
-          reinterpret_cast<const void*>(lightning_out_mfma_kernel<D, V, MODE>),
+          reinterpret_cast<const void*>(lightning_out_mfma_kernel<D, V, MODE, VEC>),
           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       set = true;
     }
-    hipLaunchKernelGGL((lightning_out_mfma_kernel<D, V, MODE>), grid, block, lds,
+    hipLaunchKernelGGL((lightning_out_mfma_kernel<D, V, MODE, VEC>), grid, block, lds,
                        stream, out, part, (const bf16*)q, (const bf16*)k,
                        (const bf16*)v, ldq, ldk, ldv, decay, cu, H, rot);
   }
@@ -378,16 +499,19 @@ extern "C" int arks_seq_lightning_mfma(void* out, void* part, const void* q,
   if (chunks == 0) return 0;
   const LmRot rot{(const int64_t*)positions, (const float*)freq, n_rot,
                   interleaved, k_scale};
+  // pass 1 has no q
+  const bool vec =
+      ((pass == 1 ? 0 : ldq) | ldk | ldv) % 8 == 0 &&
+      (((pass == 1 ? 0 : (uintptr_t)q) | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+#define LM_GO(DD, VV, M, VEC)                                                 \
+  launch_lm<DD, VV, M, VEC>((float*)out, (float*)part, q, k, v, ldq, ldk, ldv, \
+                            (const float*)decay, (const int*)cu, chunks, H,   \
+                            pass, rot, stream)
 #define LM(DD, VV)                                                            \
   if (D == DD && V == VV) {                                                   \
-    if (mode == 0)                                                            \
-      launch_lm<DD, VV, 0>((float*)out, (float*)part, q, k, v, ldq, ldk, ldv, \
-                           (const float*)decay, (const int*)cu, chunks, H,    \
-                           pass, rot, stream);                                \
-    else                                                                      \
-      launch_lm<DD, VV, 1>((float*)out, (float*)part, q, k, v, ldq, ldk, ldv, \
-                           (const float*)decay, (const int*)cu, chunks, H,    \
-                           pass, rot, stream);                                \
+    if (mode == 1) LM_GO(DD, VV, 1, false);                                   \
+    else if (vec) LM_GO(DD, VV, 0, true);                                     \
+    else LM_GO(DD, VV, 0, false);                                             \
     return 0;                                                                 \
   }
   LM(32, 32)
@@ -398,5 +522,6 @@ extern "C" int arks_seq_lightning_mfma(void* out, void* part, const void* q,
   LM(64, 32)
   LM(128, 32)
 #undef LM
+#undef LM_GO
   return 1;
 }

@@ -501,3 +501,35 @@ def test_head_norm_rotation_of_few_and_many_rows(dtype):
         res.append((qo, kc, vc))
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,V", [(32, 32), (64, 64), (64, 128), (128, 64),
+                                 (128, 128), (64, 32), (128, 32)])
+def test_lightning_chunks_off_16_bytes(D, V):
+    """Rows on 16 bytes are staged by wide loads, others one value at a time:
+    the same bits. Chunk ends of one to 64 rows, odd ones among them."""
+    dev, H, lens = "cuda", 3, [1, 64, 130, 35, 99]
+    torch.manual_seed(D + V)
+    T, cu = sum(lens), [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    meta = (i32(cu, dev), i32([n + 3 for n in lens], dev), i32([4, 1, 0, 2, 3], dev))
+    chunks = ops.scan_chunks(lens, torch.device(dev))
+    data = [torch.randn(T, H * n, device=dev).bfloat16() * 4 for n in (D, D, V)]
+    decay = torch.tensor([1.0, 0.0, 0.98], device=dev)
+    st0 = torch.randn(5, H, D, V, device=dev)
+    res = []
+    for pads in ((0, 0, 0), (8, 8, 8), (2, 0, 0), (0, 4, 0), (0, 0, 1)):
+        rows = []
+        for t, n, pad in zip(data, (D, D, V), pads):
+            buf = torch.empty(T, H * n + pad, device=dev, dtype=torch.bfloat16)
+            buf[:, :H * n] = t
+            rows.append(buf[:, :H * n].view(T, H, n) if not pad
+                        else buf.as_strided((T, H, n), (H * n + pad, n, 1)))
+        st = st0.clone()
+        o = ops.lightning_scan(*rows, decay, st, *meta, max_q_len=max(lens),
+                               chunks=chunks)
+        res.append((o, st))
+    for o, st in res[1:]:
+        assert torch.equal(o, res[0][0]) and torch.equal(st, res[0][1])
