@@ -174,24 +174,25 @@ def stage_rows(prompts: list, outputs: list, tables: list, starts, counts, ids,
 
 
 def upload(tensors: list, device) -> list:
-    """Host tensors (or None) on a device: moved as one, since a step waits for
-    every copy of its own (a dozen took 300 us)."""
+    """Host tensors (or what stays on the host) on a device: moved as one, since
+    a step waits for every copy of its own (a dozen took 300 us)."""
     device = torch.device(device)
+    held = [isinstance(t, torch.Tensor) for t in tensors]
     if device.type != "cuda":
-        return [t if t is None else t.to(device) for t in tensors]
+        return [t.to(device) if h else t for t, h in zip(tensors, held)]
     at, total = [], 0
-    for t in tensors:
+    for t, h in zip(tensors, held):
         at.append(total)
-        total += 0 if t is None else -(-t.numel() * t.element_size() // 16) * 16
+        total += -(-t.numel() * t.element_size() // 16) * 16 if h else 0
     host = torch.empty(total, dtype=torch.uint8, pin_memory=True)
     whole = lambda buf, t, o: buf[o:o + t.numel() * t.element_size()].view(
         t.dtype).view(t.shape)
-    for t, o in zip(tensors, at):
-        if t is not None:
+    for t, o, h in zip(tensors, at, held):
+        if h:
             whole(host, t, o).copy_(t)
     moved = host.to(device, non_blocking=True)
-    return [None if t is None else whole(moved, t, o)
-            for t, o in zip(tensors, at)]
+    return [whole(moved, t, o) if h else t
+            for t, o, h in zip(tensors, at, held)]
 
 
 EXTEND2_QTILE = 256  # q rows per workgroup in the 8-wave ladder kernel
@@ -295,12 +296,17 @@ def build_extend_tiles(q_lens: list[int], kv_lens: list[int] | None,
 
     drows = dseqs = None
     if dec:
-        # gather indices: the single q row of each decode seq sits at
-        # cu_seqlens_q[i]; seq-level metadata indexes with `dec` itself
+        # the single q row of each decode seq sits at cu_seqlens_q[i]; seq-level
+        # metadata indexes with `dec` itself. Rows side by side (a scheduler
+        # puts running sequences together) are a slice, which needs no gather
+        # and no scatter: two launches, 10 us a layer.
         cu = [0]
         for n in q_lens:
             cu.append(cu[-1] + n)
-        drows = torch.tensor([cu[i] for i in dec], dtype=torch.long)
+        at = [cu[i] for i in dec]
+        drows = (slice(at[0], at[0] + len(at))
+                 if at[-1] - at[0] == len(at) - 1
+                 else torch.tensor(at, dtype=torch.long))
         dseqs = torch.tensor(dec, dtype=torch.long)
     t64_t, t256_t, ctab, drows, dseqs = upload(
         [t64_t, t256_t, ctab, drows, dseqs], device)
@@ -371,7 +377,10 @@ def attention_extend_paged(
             )
         if drows is not None:
             assert maps == 1, "single rows of a two-map cache: no flash-decode"
-            dq = q[drows].contiguous()
+            dq = q[drows]
+            if (dq.stride()[1:] != (dq.shape[2], 1) or dq.stride(0) % 8
+                    or dq.data_ptr() % 16):
+                dq = dq.clone(memory_format=torch.contiguous_format)
             dtab, dlens, plan = _single_rows(
                 block_tables, kv_lens, dseqs, k_cache.shape[1], window, kv_fp8,
                 sink_w is None and slopes is None, C, step_cache)
@@ -386,7 +395,10 @@ def attention_extend_paged(
                 dout = attention_decode_paged(
                     dq, k_cache, v_cache, dtab, dlens, scale, window=window,
                     sink=bool(sink), native=C, plan=plan,
+                    out=out[drows] if isinstance(drows, slice) else None,
                 )
+                if isinstance(drows, slice):
+                    return out
             out[drows] = dout
         return out
     return ref.attention_extend_paged(
@@ -467,15 +479,16 @@ def attention_decode_plan(seq_lens, num_kv_heads: int, window: int = 0,
 def attention_decode_paged(
     q, k_cache, v_cache, block_tables, seq_lens, scale: float,
     num_partitions: int | None = None, part_out=None, window: int = 0,
-    sink: bool = False, native=None, plan=None,
+    sink: bool = False, native=None, plan=None, out=None,
 ):
     """plan: attention_decode_plan's for these lengths, heads, window and
-    num_partitions (None: made here)."""
+    num_partitions (None: made here). out: a contiguous tensor to write."""
     if q.is_cuda:
         C = native if native is not None else _native()
         S, hq, hd = q.shape
         hkv = k_cache.shape[1]
-        out = torch.empty((S, hq, hd), dtype=q.dtype, device=q.device)
+        if out is None:
+            out = torch.empty((S, hq, hd), dtype=q.dtype, device=q.device)
         kv_fp8 = k_cache.dtype != torch.bfloat16
         if plan is None:
             plan = attention_decode_plan(seq_lens, hkv, window, kv_fp8,

@@ -1378,6 +1378,29 @@ def test_upload():
                 and torch.equal(m.cpu(), h))
 
 
+@pytest.mark.parametrize("pad", [0, 8, 4])
+def test_single_rows_side_by_side(pad):
+    """Single rows that lie together are read and written in place: the same
+    bits as by index; q rows with gaps, on 16 bytes and off them."""
+    assert_native()
+    torch.manual_seed(pad)
+    qlens, kvs, hq, hkv, hd = [70, 1, 1, 1, 150], [70, 40, 900, 17, 400], 8, 2, 128
+    q, kc, vc, bt = marked_pages(sum(qlens), hq, hkv, hd, kvs, [{0}] * 5)
+    buf = torch.zeros(sum(qlens), hq * hd + pad, dtype=torch.bfloat16, device=DEV)
+    buf[:, :hq * hd] = q.to(DEV).reshape(len(q), -1)
+    rows = buf[:, :hq * hd].unflatten(1, (hq, hd))
+    lens = torch.tensor(kvs, dtype=torch.int32, device=DEV)
+    cu = torch.tensor([0] + qlens).cumsum(0).int().to(DEV)
+    tiles = ops.build_extend_tiles(qlens, kvs, False, torch.device(DEV), num_q_heads=hq)
+    assert tiles[2][0] == slice(70, 73)
+    apart = ops.build_extend_tiles([1, 2, 1], [9, 9, 9], False, torch.device(DEV))[2][0]
+    assert apart.tolist() == [0, 3]
+    run = lambda x, t: ops.attention_extend_paged(
+        x, kc.to(DEV), vc.to(DEV), bt.to(DEV), lens, cu, qlens, hd ** -0.5, tiles=t)
+    index = (*tiles[:2], (torch.arange(70, 73, device=DEV), tiles[2][1]), *tiles[3:])
+    assert torch.equal(run(rows, tiles), run(rows.contiguous(), index))
+
+
 def test_tiles_rule():
     """Rows that fill the chip's rounds take the tiles, others the library."""
     assert_native()
