@@ -1378,6 +1378,44 @@ def test_upload():
                 and torch.equal(m.cpu(), h))
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+def test_extend_parts_merge(hd):
+    """Tiles of 1 to 8 parts in one table, a short one among them, a part that
+    saw no key: the merge in fp64 and one rounding to bf16 (fp32 exponents of
+    up to some 2^4 cost 2^-19)."""
+    assert_native()
+    torch.manual_seed(hd)
+    counts, H, scale = [1, 2, 3, 4, 5, 8], 3, hd ** -0.5
+    q_lens = [256, 256, 300, 100, 256, 7]
+    cu = torch.tensor([0] + q_lens).cumsum(0).int().to(DEV)
+    table, at = [], 0
+    for i, n in enumerate(counts):
+        table.append([at, n, i, 256 if i == 2 else 0])
+        at += n
+    ws = torch.randn(at, H, 256, hd + 2, device=DEV)
+    ws[..., hd] *= 8
+    ws[..., hd + 1] = ws[..., hd + 1].abs() + 0.1
+    ws[4, :, ::3, :hd] = 0.0  # a part of the third tile without a key
+    ws[4, :, ::3, hd] = -1e30
+    ws[4, :, ::3, hd + 1] = 0.0
+    out = torch.zeros(sum(q_lens), H, hd, dtype=torch.bfloat16, device=DEV)
+    ops._native().attention_extend2_combine(
+        out, ws.view(-1), torch.tensor(table, dtype=torch.int32, device=DEV), cu, scale)
+    seen = torch.zeros(sum(q_lens), dtype=torch.bool, device=DEV)
+    for first, n, i, q0 in table:
+        rows = min(256, q_lens[i] - q0)
+        p = ws[first:first + n, :, :rows].double()
+        m = p[..., hd] * scale
+        e = torch.exp(m - m.amax(0))
+        want = (e[..., None] * p[..., :hd]).sum(0) / (e * p[..., hd + 1]).sum(0)[..., None]
+        size = (e[..., None] * p[..., :hd].abs()).sum(0) / (e * p[..., hd + 1]).sum(0)[..., None]
+        a = int(cu[i]) + q0
+        got = out[a:a + rows].transpose(0, 1).double()
+        assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 2 ** -18 * size).all())
+        seen[a:a + rows] = True
+    assert not out[~seen].any()
+
+
 @pytest.mark.parametrize("pad", [0, 8, 4])
 def test_single_rows_side_by_side(pad):
     """Single rows that lie together are read and written in place: the same
