@@ -5,7 +5,7 @@ head_dim] cache tensors (one pair per layer). The allocator is pure
 bookkeeping — tensors live in the model runner.
 
 PrefixCachingAllocator adds content-addressed block reuse (the radix-cache
-capability SGLang brings to the reference's runtime slot — SURVEY.md §2.4):
+capability SGLang brings to the reference's runtime slot):
 full blocks are keyed by blake2b(parent_digest + token_ids); freed blocks
 keep their contents and sit in an LRU pool until evicted, so a later request
 sharing a prompt prefix re-references them instead of recomputing the KV.

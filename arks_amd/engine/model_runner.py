@@ -189,7 +189,7 @@ class ModelRunner:
     def extract_kv(self, block_table: list[int]) -> torch.Tensor:
         """Gather a sequence's KV pages to one host tensor
         [layers, 2(k/v), nblocks, num_kv_heads, block_size, head_dim] for
-        transfer to a decode instance (SURVEY.md §2.2: the reference's PD
+        transfer to a decode instance (the reference's PD
         split delegates this to SGLang's disaggregation-mode, reference
         arksdisaggregatedapplication_controller.go:1672-1724)."""
         if self.seq_state:

@@ -1,5 +1,5 @@
 """Continuous-batching scheduler (the subset of vLLM's engineering the
-runtime slot needs — SURVEY.md §7 'hard parts' #2).
+runtime slot needs).
 
 Policy (v0, vLLM-v0-like):
 - Prefill-priority: if waiting requests fit the token budget and KV blocks,

@@ -1,6 +1,6 @@
 """Safetensors weight loading with pinned-host staging.
 
-Cold-start time is a headline metric (BASELINE.md): weights stream PVC ->
+Cold-start time is a headline metric: weights stream PVC ->
 page cache -> pinned staging buffer -> HBM with hipMemcpyAsync on a side
 stream, double-buffered so disk reads overlap H2D copies. TP sharding happens
 on the host slice before upload, so only this rank's bytes cross PCIe.
@@ -92,8 +92,7 @@ def load_model_weights(model, model_path: str, device: torch.device,
     other buffer. Pinned memory is allocated exactly twice for the whole
     load: the previous per-tensor `pin_memory()` scheme spent most of the
     cold start page-locking fresh allocations (0.59 GB/s loader vs
-    3.5 GB/s raw disk on the same box — cold start is a headline metric,
-    BASELINE.md).
+    3.5 GB/s raw disk on the same box — cold start is a headline metric).
     """
     model.to(device)
     if device.type != "cuda":

@@ -1,7 +1,7 @@
 """In-tree build of the arks_amd HIP extension for gfx950.
 
 The extension builds into arks_amd/ops/_build (IN the repo tree, so the .so
-travels with gpurun snapshots) via torch.utils.cpp_extension, which drives
+travels with copies of the tree) via torch.utils.cpp_extension, which drives
 hipcc for the .hip sources. Cross-compiles fine on a GPU-less box.
 
 Usage: python -m arks_amd.ops.build [-v]

@@ -2,7 +2,7 @@
 //
 // RCCL's ring all-reduce is per-link bound on MI355X (7 p2p xGMI links
 // x ~153 GB/s, no switch) and latency-heavy for the small per-token
-// tensors of tensor-parallel decode (SURVEY.md §5). For payloads <= ~1 MiB
+// tensors of tensor-parallel decode. For payloads <= ~1 MiB
 // this kernel does the classic small-message one-shot instead: every rank
 // PUSHES its contribution into a slot of every peer's mailbox (p2p stores
 // over xGMI), signals per-block flags with system-scope release, and each

@@ -4,7 +4,7 @@
 // to their pages before this kernel runs on the same stream).
 //
 // This is the prefix-caching / chunked-prefill half of the runtime-slot
-// contract (SURVEY.md §2.4: SGLang's radix-cache "extend" phase, delegated
+// contract (SGLang's radix-cache "extend" phase, delegated
 // by the reference to external images at arksapplication_controller.go:956-969).
 //
 // Structure matches attn_prefill.hip: one workgroup = 4 waves = a 64-row

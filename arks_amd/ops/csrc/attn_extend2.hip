@@ -40,7 +40,7 @@
 // split tiles go without that branch (whole prompts are mostly full tiles).
 //
 // This is the prefix-caching / chunked-prefill attention of the runtime
-// slot (SURVEY.md §2.4; the reference delegates it to vLLM/SGLang images
+// slot (the reference delegates it to vLLM/SGLang images
 // at arksapplication_controller.go:941-1002).
 #include "common.h"
 

@@ -12,8 +12,7 @@
 // (guide common-mistake #6). P is staged through a per-wave padded LDS buffer
 // to re-shape for the PV A-fragment.
 //
-// This kernel is the prefill half of the runtime-slot contract described in
-// SURVEY.md §2.4 (vLLM's flash prefill at reference
+// This kernel is the prefill half of the runtime-slot contract (vLLM's flash prefill at reference
 // arksapplication_controller.go:941-955 delegated it to an external image).
 #include "common.h"
 
@@ -78,7 +77,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(
   // V tile as a tr16 image: [d-chunk cb][key-block kb][4 key x 16 col]
   // blocks of 64 bf16 padded to 96 so the two 16-lane regions of one
   // 32-lane ds_read_b64_tr_b16 group land on disjoint bank halves
-  // (stride 192 B = 48 dwords; probe: gpurun_out/probe_layouts.log).
+  // (stride 192 B = 48 dwords).
   // Each lane then receives the 4 keys of its column — B-fragment shape —
   // and V staging becomes two b128 stores instead of 16 scalar b16 writes.
   __shared__ __attribute__((aligned(16))) bf16 vt_img[2][HEAD_DIM / 16][8][96];

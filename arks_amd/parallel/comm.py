@@ -3,9 +3,8 @@
 One process per GPU; torch.distributed backend "nccl" IS RCCL on ROCm. The
 TP group is the whole world for a single serving instance (the LWS
 leader/worker topology of the reference maps each inference group to one
-node's xGMI-connected GPUs — SURVEY.md §5 'Distributed communication
-backend'). Falls back to gloo on CPU so the distributed path is testable
-without hardware.
+node's xGMI-connected GPUs). Falls back to gloo on CPU so the distributed path
+is testable without hardware.
 """
 
 from __future__ import annotations

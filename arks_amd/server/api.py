@@ -1,7 +1,7 @@
 """OpenAI-compatible HTTP server (FastAPI/ASGI).
 
 Implements the runtime-slot HTTP contract the reference delegates to
-vLLM/SGLang images (SURVEY.md §2.4): /v1/chat/completions and
+vLLM/SGLang images: /v1/chat/completions and
 /v1/completions with SSE streaming whose FINAL chunk carries `usage`
 (the gateway's accounting depends on it — reference
 handle_response.go:113-133), /v1/models, a readiness probe on the serving

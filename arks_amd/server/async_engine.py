@@ -140,7 +140,7 @@ class AsyncEngine:
 
     # ---- prefill/decode disaggregation (reference delegates this to
     # SGLang's --disaggregation-mode; here it is first-party over a TCP KV
-    # page transfer — SURVEY.md §2.2) ----
+    # page transfer) ----
     async def disagg_prefill(self, request_id: str, token_ids: list[int],
                              sampling: SamplingParams):
         """Prefill-instance side: run the prompt, sample the first token,
