@@ -94,8 +94,8 @@ void arks_mid_gemm(void* out, const void* a, const void* w, const void* bias,
                    int parts, int silu, hipStream_t stream);
 void arks_mid_items(void* out, const void* a, const void* w, const void* perm,
                     const void* items, const void* n_items, int64_t a_stride,
-                    int64_t w_expert, int n, int k, int top_k, int max_items,
-                    int ft, int silu, hipStream_t stream);
+                    int64_t w_expert, int n, int k, int top_k, int expert_base,
+                    int max_items, int ft, int silu, hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, void* claims, void* counts, const void* ids,
                    const void* weights, int pairs, int expert_base, int n_local,
@@ -811,10 +811,10 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
     const int ft = (int)tile / 64;
     arks_mid_items(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
                    n_items, x.stride(0), 2 * I * H, (int)I, (int)H, (int)k,
-                   (int)max_items, ft, 1, stream);
+                   (int)expert_base, (int)max_items, ft, 1, stream);
     arks_mid_items(y.data_ptr(), h.data_ptr(), w2.data_ptr(), nullptr, items,
-                   n_items, I, H * I, (int)H, (int)I, (int)k, (int)max_items,
-                   ft, 0, stream);
+                   n_items, I, H * I, (int)H, (int)I, (int)k,
+                   (int)expert_base, (int)max_items, ft, 0, stream);
   } else {
     arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
                   n_items, claims, x.stride(0), 2 * I * H, H, (int)I, (int)H,

@@ -39,6 +39,7 @@ struct MidItems {
   const int* __restrict__ perm;
   int64_t w_expert;
   int top_k;
+  int expert_base;  // number of the first of these experts among all ranks'
 };
 
 // 1 KB of 8 rows into LDS, 16 B a lane, from step s of its offset. The weights
@@ -111,7 +112,9 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   // turn: the step that a job begins with (then on to the last, and from the
   // first): workgroups that read the same columns of rows a power of two apart
   // would all meet on a few memory channels (16 rows x 151936 x 2048 127 -> 102
-  // us, x 57344 x 8192 164 -> 147).
+  // us, x 57344 x 8192 164 -> 147). An expert's follows from its number and
+  // the tile alone, not from the item: which item a pair is in depends on the
+  // other rows of the step, and its order of sums must not.
   struct Job {
     int n0, split, s0, steps, turn;
     int expert, first, rows;
@@ -119,8 +122,10 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   auto job = [&](const int j) {
     if constexpr (ITEMS) {
       const int4 it = of.items[j / tiles];
-      return Job{j % tiles * COLS, 0, 0, all_steps,
-                 rotate ? (int)((unsigned)j % (unsigned)all_steps) : 0,
+      const unsigned tile = j % tiles;
+      const unsigned at = (unsigned)(of.expert_base + it.x) * tiles + tile;
+      return Job{(int)tile * COLS, 0, 0, all_steps,
+                 rotate ? (int)(at % (unsigned)all_steps) : 0,
                  it.x, it.y, it.z};
     }
     const unsigned split = j / tiles, n = splits;  // all_steps * n < 2^32
@@ -400,10 +405,10 @@ extern "C" void arks_mid_items(void* out, const void* a, const void* w,
                                const void* perm, const void* items,
                                const void* n_items, int64_t a_stride,
                                int64_t w_expert, int n, int k, int top_k,
-                               int max_items, int ft, int silu,
+                               int expert_base, int max_items, int ft, int silu,
                                hipStream_t stream) {
   const MidItems of{(const int4*)items, (const int*)n_items, (const int*)perm,
-                    w_expert, top_k};
+                    w_expert, top_k, expert_base};
   const int cols = silu ? 64 : 128;
   const int64_t jobs = (int64_t)((n + cols - 1) / cols) * max_items;
   const int grid = (int)(jobs < 256 ? jobs : 256);

@@ -885,6 +885,37 @@ def test_moe_items(T, E, k, H, I, base, El, tile, skew):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("base,El", [(0, 8), (2, 5)])
+@pytest.mark.parametrize("tile", [64, 128])
+def test_moe_items_order_of_sums(tile, base, El):
+    """A row's result does not turn with the rows that share its step, nor from
+    call to call: an expert of several items, beside neighbours that send other
+    numbers of pairs to the experts in front of it."""
+    assert_native()
+    torch.manual_seed(tile + base)
+    T, E, k, H, I, same = 420, 8, 2, 576, 320, 300
+    w13 = (torch.randn(E, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(E, H, I, device=DEV) * I ** -0.5).bfloat16()
+    rows = torch.randn(same, H, device=DEV).bfloat16()
+    pairs = torch.stack([torch.full((same,), 4), torch.arange(same) % 3 + 5], 1).int()
+    weights = torch.rand(same, k, device=DEV)
+    seen = []
+    for seed in range(8):
+        g = torch.Generator().manual_seed(seed % 4)  # every batch twice
+        at = torch.randperm(T, generator=g)
+        other = torch.rand(T - same, E, generator=g)
+        other[:, : seed % 4] += 1  # these experts above all
+        ids = torch.cat([pairs, other.topk(k).indices.int()])
+        x = torch.cat([rows, torch.randn(T - same, H, generator=g).to(DEV).bfloat16()])
+        w = torch.cat([weights, torch.rand(T - same, k, generator=g).to(DEV)])
+        out = torch.empty(T, H, device=DEV, dtype=torch.bfloat16)
+        ops._native().moe_experts(
+            out, x[at], w13[base:base + El].contiguous(),
+            w2[base:base + El].contiguous(), w[at], ids[at].to(DEV), base, tile, True)
+        seen.append(out[at.argsort()[:same]])
+    assert all(torch.equal(o, seen[0]) for o in seen)
+
+
 @pytest.mark.parametrize("T,E,k,base,El", [
     (1024, 8, 8, 0, 8), (1025, 8, 8, 0, 8),     # either side of one workgroup
     (1280, 100, 8, 0, 100), (5012, 128, 8, 0, 128),  # ends of the runs
