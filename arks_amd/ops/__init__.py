@@ -378,13 +378,16 @@ def attention_extend_paged(
         if drows is not None:
             assert maps == 1, "single rows of a two-map cache: no flash-decode"
             dq = q[drows]
+            biased = sink_w is not None or slopes is not None
+            # attention_sink_paged takes contiguous rows, the other one gaps
             if (dq.stride()[1:] != (dq.shape[2], 1) or dq.stride(0) % 8
-                    or dq.data_ptr() % 16):
+                    or dq.data_ptr() % 16
+                    or (biased and not dq.is_contiguous())):
                 dq = dq.clone(memory_format=torch.contiguous_format)
             dtab, dlens, plan = _single_rows(
                 block_tables, kv_lens, dseqs, k_cache.shape[1], window, kv_fp8,
-                sink_w is None and slopes is None, C, step_cache)
-            if sink_w is not None or slopes is not None:
+                not biased, C, step_cache)
+            if biased:
                 each = torch.arange(dq.shape[0] + 1, dtype=torch.int32,
                                     device=q.device)
                 dout = attention_sink_paged(

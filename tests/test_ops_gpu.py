@@ -1470,6 +1470,31 @@ def test_single_rows_side_by_side(pad):
     assert torch.equal(run(rows, tiles), run(rows.contiguous(), index))
 
 
+@pytest.mark.parametrize("sink,bias", [(True, False), (False, True), (True, True)])
+def test_single_rows_side_by_side_biased(sink, bias):
+    """The same with a sink's score per head or a distance bias: rows of q with
+    gaps give what packed ones do."""
+    assert_native()
+    torch.manual_seed(3)
+    qlens, kvs, hq, hkv, hd = [70, 1, 1, 1, 300], [70, 40, 900, 17, 400], 8, 2, 128
+    q, kc, vc, bt = marked_pages(sum(qlens), hq, hkv, hd, kvs, [{0}] * 5)
+    buf = torch.zeros(sum(qlens), hq * hd + 8, dtype=torch.bfloat16, device=DEV)
+    buf[:, :hq * hd] = q.to(DEV).reshape(len(q), -1)
+    rows = buf[:, :hq * hd].unflatten(1, (hq, hd))
+    lens = torch.tensor(kvs, dtype=torch.int32, device=DEV)
+    cu = torch.tensor([0] + qlens).cumsum(0).int().to(DEV)
+    tiles = ops.build_extend_tiles(qlens, kvs, False, torch.device(DEV),
+                                   num_q_heads=hq, min_ladder=1)
+    assert tiles[2][0] == slice(70, 73)
+    run = lambda x, t: ops.attention_extend_paged(
+        x, kc.to(DEV), vc.to(DEV), bt.to(DEV), lens, cu, qlens, hd ** -0.5,
+        tiles=t, native=ops.seq_extension(),
+        sink_w=torch.linspace(-1, 1, hq, device=DEV) if sink else None,
+        slopes=torch.linspace(.01, .1, hq, device=DEV) if bias else None)
+    index = (*tiles[:2], (torch.arange(70, 73, device=DEV), tiles[2][1]), *tiles[3:])
+    assert torch.equal(run(rows, tiles), run(rows.contiguous(), index))
+
+
 def test_tiles_rule():
     """Rows that fill the chip's rounds take the tiles, others the library."""
     assert_native()
