@@ -288,9 +288,10 @@ __global__ __launch_bounds__(64) void selective_scan_kernel(
 // exponentials a row, so nothing else may cost much. WHOLE (N == NMAX) goes
 // without a test of every state (each was a branch that kept the loop's
 // operations in order) and moves states and A 16 bytes at a time; bf16 rows
-// take the softplus and the gate's sigmoid from the hardware's exp2 and
-// reciprocal. 3853 rows of 8192 channels x 16 states in chunks of 64, both
-// passes and the combination 590 -> 326 us; 8 single rows 13.0 -> 7.5.
+// take the softplus and the gate's exponential from the hardware's exp2, with
+// what rounding its argument loses carried along. 3853 rows of 8192 channels x
+// 16 states in chunks of 64, both passes and the combination 590 -> 332 us; 8
+// single rows 13.0 -> 8.
 constexpr int SCAN_ROWS = 32;
 
 // log(1 + e^x) = max(x, 0) + log(1 + t), t = e^-|x|, by log(1 + t) = 2 atanh(q),
@@ -322,13 +323,30 @@ __device__ __forceinline__ float softplus_fast(float x) {
       2.f * __builtin_fmaf(q * w, p, q_lo));
   return x > 0.f ? x + __builtin_fmaf(2.f, q, lo) : __builtin_fmaf(2.f, q, lo);
 }
+// x / (1 + e^-x); what rounding loses of the exponent is carried along (an
+// exponent of 130 or more is an infinity, one below -150 a zero)
 __device__ __forceinline__ float silu_fast(float x) {
-  return x * __builtin_amdgcn_rcpf(
-                 1.f + __builtin_amdgcn_exp2f(x * -1.44269504088896341f));
+  constexpr float LOG2E = 1.44269504088896341f, LOG2E_LO = 1.92596299e-8f;
+  constexpr float LN2 = 0.693147180559945309f;
+  const float n = -__builtin_amdgcn_fmed3f(x, -90.5f, 104.f);
+  const float h = n * LOG2E;
+  const float l = __builtin_fmaf(n, LOG2E_LO, __builtin_fmaf(n, LOG2E, -h));
+  const float e = __builtin_amdgcn_exp2f(h) * __builtin_fmaf(l, LN2, 1.f);
+  return x / (1.f + e);
+}
+
+// Waves per SIMD that the registers of a row's states allow: one register more
+// than that fits (2400 rows of 8192 channels in chunks: 5 waves of 96 registers
+// 196 us, 4 of 97 227).
+template <typename AT, int NMAX, bool WITH_Y, bool WHOLE>
+constexpr int scan_waves() {
+  if (!(sizeof(AT) == 2 && WITH_Y && WHOLE)) return 1;
+  return NMAX <= 8 ? 8 : NMAX <= 16 ? 5 : NMAX <= 32 ? 4 : 2;
 }
 
 template <typename AT, int NMAX, bool WITH_Y, bool WHOLE>
-__global__ __launch_bounds__(256) void selective_scan_lane_kernel(
+__global__ __launch_bounds__(256, (scan_waves<AT, NMAX, WITH_Y, WHOLE>()))
+void selective_scan_lane_kernel(
     AT* __restrict__ out, const AT* __restrict__ u, const AT* __restrict__ dbc,
     int64_t ldd, const AT* __restrict__ z, int64_t ldz,
     const float* __restrict__ dt_b, const float* __restrict__ A,
@@ -395,7 +413,8 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
         if (WHOLE || n < N) {
           const float e = FAST ? __builtin_amdgcn_exp2f(dt * Av[n])
                                : expf(dt * Av[n]);
-          S[n] = e * S[n] + dx * bc_s[rr][n];
+          // (the larger term is the one that goes unrounded)
+          S[n] = __builtin_fmaf(e, S[n], dx * bc_s[rr][n]);
           if (WITH_Y) y += S[n] * bc_s[rr][NMAX + n];
         }
       }

@@ -384,6 +384,32 @@ def test_selective_scan_lanes_against_64_bits(C, N, lens, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("C,N", [(4096, 16), (4097, 5)])
+def test_selective_scan_gate_of_bf16_rows(C, N):
+    """The gate of bf16 rows is fp32 work, seen in how often its rounding to bf16
+    is another one than that of the fp64 value. With C = 0 the output is D u
+    silu(z): exp to 1 ulp, a sum, a quotient and two products, at most 3 * 2^-23
+    of it in all, fall on the other side of a rounding border (2^-8 apart, or
+    more) for at most 2 * 3 * 2^-23 / 2^-8 of the values. An argument of exp2
+    that is rounded, at 64 and more by 2^-18, would do so for three times that."""
+    dev = "cuda"
+    torch.manual_seed(N)
+    T, R = 128, 4
+    z = -torch.linspace(45.0, 87.0, T, device=dev)[:, None].expand(T, C).bfloat16()
+    u = torch.ones(T, C, device=dev).bfloat16()
+    dbc = torch.zeros(T, R + 2 * N, device=dev).bfloat16()
+    Dp = torch.rand(C, device=dev) + 1
+    y = ops.selective_scan(
+        u, dbc, z.contiguous(), torch.zeros(C, R, device=dev), torch.zeros(C, device=dev),
+        -torch.rand(C, N, device=dev), Dp, torch.zeros(1, C, N, device=dev),
+        i32([0, T], dev), i32([T], dev), i32([0], dev), max_q_len=T,
+        dt_pre=torch.zeros(T, C, device=dev))
+    want = (Dp.double() * torch.nn.functional.silu(z.double())).bfloat16()
+    share = (y != want).double().mean().item()
+    assert share <= 2 * 3 * 2.0 ** -23 / 2.0 ** -8, share
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,V", [(16, 64), (128, 128), (256, 64),  # whole
                                  (128, 72), (100, 64), (17, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
