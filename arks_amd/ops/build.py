@@ -77,6 +77,16 @@ def built_so_path(name: str = EXT_NAME) -> str | None:
     return matches[0] if matches else None
 
 
+def drop_older(out_dir: str, src_dir: str = CSRC) -> None:
+    """Objects from before the last change of a header go: torch's ninja rule
+    for hipcc knows the .hip file that it compiles, not what that includes."""
+    headers = glob.glob(os.path.join(src_dir, "*.h"))
+    newest = max(map(os.path.getmtime, headers), default=0.0)
+    for obj in glob.glob(os.path.join(out_dir, "*.o")):
+        if os.path.getmtime(obj) <= newest:
+            os.remove(obj)
+
+
 def build(verbose: bool = False, name: str | None = None):
     """Compile one extension (or all of them) in-tree; returns the path of
     the last library built."""
@@ -89,6 +99,7 @@ def build(verbose: bool = False, name: str | None = None):
             continue
         out_dir = os.path.join(BUILD_DIR, ext)
         os.makedirs(out_dir, exist_ok=True)
+        drop_older(out_dir)
         cpp_extension.load(
             name=ext,
             sources=sources,

@@ -206,3 +206,20 @@ def test_stage_rows():
         with pytest.raises((RuntimeError, TypeError)):
             ops.stage_rows(prompts, a["outputs"], a["tables"], a["starts"],
                            a["counts"], *a["bufs"], bs)
+
+
+def test_objects_older_than_a_header_are_built_again(tmp_path):
+    import os
+
+    from arks_amd.ops.build import drop_older
+
+    src, out = tmp_path / "src", tmp_path / "out"
+    for d in (src, out):
+        d.mkdir()
+    for path, at in ((src / "a.h", 100), (src / "b.h", 200), (src / "c.hip", 900),
+                     (out / "old.o", 150), (out / "same.o", 200), (out / "new.o", 201),
+                     (out / "lib.so", 150)):
+        path.touch()
+        os.utime(path, (at, at))
+    drop_older(str(out), str(src))
+    assert sorted(p.name for p in out.iterdir()) == ["lib.so", "new.o"]
