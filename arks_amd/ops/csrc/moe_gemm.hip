@@ -41,10 +41,6 @@ __device__ __forceinline__ f32x4 moe_mfma(const ushort8& a, const ushort8& b,
       c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float moe_silu_mul(float g, float u) {
-  return g / (1.f + __expf(-g)) * u;
-}
-
 // perm[place] = pair, rows[pair] = place (0 where the expert is another
 // rank's), weights_out[pair] = the pair's weight (0 there), items[i] = {local
 // expert, first place, pairs, number within the expert | items of the expert
@@ -268,7 +264,7 @@ __global__ __launch_bounds__(WV * 64) void moe_stream_kernel(
     if (UP) {
       const f32x4 u = total(1);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s[r] = moe_silu_mul(s[r], u[r]);
+      for (int r = 0; r < 4; ++r) s[r] = tile_silu_mul(s[r], u[r]);
     }
     if (lq < cnt) {
       ushort4v o;
@@ -405,7 +401,7 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         o[r] = float_to_bf16_bits(
-            UP ? moe_silu_mul(acc[f][t][r], acc[f + 2][t][r]) : acc[f][t][r]);
+            UP ? tile_silu_mul(acc[f][t][r], acc[f + 2][t][r]) : acc[f][t][r]);
       *reinterpret_cast<ushort4v*>(row + n) = o;
     }
   }

@@ -885,6 +885,40 @@ def test_moe_items(T, E, k, H, I, base, El, tile, skew):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("way", [
+    "mid 5", "mid 100", "tiles", "items 64", "items 128", "engine", "stream"])
+def test_fused_silu_far_out(way):
+    """silu(gate) * up inside the products, at gates where the sigmoid's
+    denominator is near the end of fp32: no flush to zero. The exponential's
+    argument is rounded (2^-18 at 88), the result to bf16."""
+    assert_native()
+    g = torch.cat([torch.linspace(-88.5, -80, 40), torch.linspace(-80, 200, 59),
+                   torch.tensor([-200.0])])
+    g = g.to(DEV).bfloat16()
+    rows = 5 if way == "mid 5" else 100
+    x = torch.zeros(rows, 64, device=DEV, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = g[:rows], 1
+    n = 64
+    w = torch.zeros(2 * n, 64, device=DEV, dtype=torch.bfloat16)
+    w[:n, 0] = 1
+    w[n:, 1] = torch.linspace(1, 2, n, device=DEV)
+    want = (torch.nn.functional.silu(x[:, :1].double()) * w[n:, 1].double())
+    out = torch.empty(rows, n, device=DEV, dtype=torch.bfloat16)
+    if way[:3] == "mid":
+        ops._native().mid_gemm(out, x, w, None, 2, True)
+    elif way == "tiles":
+        ops._native().tile_silu(out, x, w)
+    else:
+        eye = torch.eye(64, n, device=DEV, dtype=torch.bfloat16)[None]
+        ops._native().moe_experts(
+            out, x, w[None], eye, torch.ones(rows, 1, device=DEV),
+            torch.zeros(rows, 1, device=DEV, dtype=torch.int32), 0,
+            {"items 64": 64, "engine": 256, "stream": 16}.get(way, 128), way[:5] == "items")
+    err = (out.double() - want).abs()
+    # experts round twice, the second time to the same value; 1e-40: no bf16
+    assert bool((err <= (2 ** -8 + 2 ** -16) * want.abs() + 1e-40).all())
+
+
 @pytest.mark.parametrize("base,El", [(0, 8), (2, 5)])
 @pytest.mark.parametrize("tile", [64, 128])
 def test_moe_items_order_of_sums(tile, base, El):
