@@ -206,7 +206,14 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
       }
   };
 
-  f32x4 acc[QT][FT];
+  // Up to 64 rows a chain of sums is 4 steps long, and those of 4 steps are added
+  // up apart: the streamed products, which are the other choice there, add up
+  // the shorter chains of several waves. 64 rows of 4608 x 3584 in 3 runs of K
+  // err by 1.0e-7, in a chain per run by 2.0e-7 (streamed, 7 runs: 1.4e-7); it
+  // takes 1.4 % longer over 60 sizes, in front of the multiplications (2.2 %
+  // behind them). Library products, the other choice beyond, are one chain too.
+  constexpr bool SETTLE = FT == 1;
+  f32x4 acc[QT][FT], settled[SETTLE ? QT : 1];
   ushort8 wf[QT][2], af[FT][2];
   auto read = [&](const int b) {
 #pragma unroll
@@ -221,7 +228,16 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
             lds + (b * STAGE + (a_at ^ (k * 64)) + f * 2048));
     }
   };
-  auto mul = [&] {
+  auto mul = [&](const int s) {
+    if constexpr (SETTLE) {
+      if ((s & 3) == 0) {
+#pragma unroll
+        for (int q = 0; q < QT; ++q) {
+          settled[q] += acc[q][0];
+          acc[q][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+    }
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -264,12 +280,15 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
     for (int q = 0; q < QT; ++q)
 #pragma unroll
       for (int f = 0; f < FT; ++f) acc[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < (SETTLE ? QT : 1); ++q)
+      settled[q] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int whole = max(0, now.steps - (NS - 1));
     for (int s = 0; s < whole; ++s) {
       read(at);
       load(now, s + NS - 1);  // into the stage that the last step read
       end_read(true);
-      mul();
+      mul(s);
       next_stage();
     }
     j += gridDim.x;
@@ -280,8 +299,12 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
       read(at);
       if (ahead) load(next, s - whole);
       end_read(ahead);
-      mul();
+      mul(s);
       next_stage();
+    }
+    if constexpr (SETTLE) {
+#pragma unroll
+      for (int q = 0; q < QT; ++q) acc[q][0] += settled[q];
     }
     const int n0 = now.n0 + wm * (COLS / 2);
 #pragma unroll

@@ -885,6 +885,24 @@ def test_moe_items(T, E, k, H, I, base, El, tile, skew):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("rows", [1, 17, 64])
+@pytest.mark.parametrize("qt", [2, 4, 5])
+def test_mid_gemm_short_chains(rows, qt):
+    """Sums of up to 64 rows are no single chain: 2^24 and 256 ones that a chain
+    would drop one by one. At most the 8 matrix operations of 4 steps meet the
+    large value, and each of 32 later sums is rounded once, by 1."""
+    assert_native()
+    K, N = 8192, 328
+    x = torch.zeros(rows, K, device=DEV, dtype=torch.bfloat16)
+    x[:, 5::32] = 1
+    w = torch.zeros(N, K, device=DEV, dtype=torch.bfloat16)
+    w[:, 5::32] = 1
+    x[:, 0] = w[:, 0] = 2.0 ** 12
+    out = torch.empty(1, rows, N, device=DEV)
+    ops._native().mid_gemm(out, x, w, None, qt, False)
+    assert (out.double() - (2 ** 24 + 256)).abs().max() <= 8 + 32
+
+
 @pytest.mark.parametrize("way", [
     "mid 5", "mid 100", "tiles", "items 64", "items 128", "engine", "stream"])
 def test_fused_silu_far_out(way):
