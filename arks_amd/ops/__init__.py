@@ -591,7 +591,13 @@ def _few_rows(x, weight, bias=None) -> bool:
 
 def _streams(x, weight, silu: bool = False, bias=None) -> bool:
     """Whether x weight^T takes stream_gemm (larger weights: if _mid does not
-    take them). A workgroup reads all of x's rows
+    take them)."""
+    return (_few_rows(x, weight, bias)
+            and _stream_sizes(x.shape[0], *weight.shape, silu))
+
+
+def _stream_sizes(M: int, N: int, K: int, silu: bool = False) -> bool:
+    """_streams, by the sizes. A workgroup reads all of x's rows
     beside its 16 or 32 weight rows, so the line lies where that traffic (rows
     x K), and the waves' tails, meet what the other path loses: us, here
     (other), the other being the split product with its sums up to
@@ -602,9 +608,8 @@ def _streams(x, weight, silu: bool = False, bias=None) -> bool:
     rows 62.0 (62.5); 151936 x 2048, 16 rows 134 (206), 32 rows 167 (149);
     37888 x 3584, 1 row 52.9 (53.2), 8 rows 58.7 (53.1), with the activation
     57.8 (59); 3584 x 18944, 1 row 30.3 (32.5), 4 rows 33.4 (32.6)."""
-    if not _few_rows(x, weight, bias):
+    if M > 64 or K % 32:
         return False
-    M, (N, K) = x.shape[0], weight.shape
     if N * K <= _SKINNY_MAX_ELEMS:
         return M * K <= 98304 and (K <= 4096 or N >= 2048) or K % 64 != 0
     if M <= 2 or (silu and M <= 8 and K <= 4096):
@@ -629,15 +634,16 @@ def _splits(x, weight, bias=None) -> bool:
 _MID_STEP = (0.07, 0.13, 0.26, 0.32)
 
 
-@functools.lru_cache(maxsize=4096)
 def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool):
-    """(qt, splits, us) of a mid_gemm: weight rows of a tile (32 * qt) and runs
+    """(qt, splits) of a mid_gemm: weight rows of a tile (32 * qt) and runs
     of K that keep 256 CUs busy in the fewest steps, 1.5 us being lost at the
     start of a round; the fp32 sums of the runs are written and read at 5 TB/s,
-    and added by a launch of their own unless the consumer does (summed). us,
-    chosen (others): 3584 x 18944, 64 rows, 4, 9
-    26.1 (5, 9 28.1; 2, 4 29.8; 4, 6 33); 3584 x 3584, 200 rows, without the
-    sums, 2, 4 15.1 (4, 8 15.2); 37888 x 3584, 64 rows, 5, 1 44.8 (4, 1 64.7)."""
+    and added by a launch of their own unless the consumer does (summed). At
+    most 8 runs, as the consumer's time grows with them. us with the norm that
+    adds the sums, weights cold, chosen (others): 3584 x 18944, 64 rows, 4, 8
+    33.0 (4, 9 33.3; without the norm 29.3 and 27.5; 5, 9 35.1; 2, 4 35.3; 4, 6
+    36.8); 3584 x 3584, 100 rows, 2, 4 16.8 (2, 2 19.9; 4, 8 19.1); 37888 x
+    3584 with the activation, 64 rows, 5, 1 48.6 (4, 1 66.2)."""
     steps, step = K // 64, _MID_STEP[(M + 63) // 64 - 1]
     best = None
     for qt in (5, 4, 2):
@@ -648,52 +654,87 @@ def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool):
                 1.5 + -(-steps // splits) * (step + 0.155 * qt))
             if splits > 1:
                 us += splits * M * N * 1.6e-6 + (0.0 if summed else 4.0)
-            if best is None or us < best[2]:
-                best = (qt, splits, us)
-    return best
+            if best is None or us < best[0]:
+                best = (us, qt, splits)
+    return best[1:]
 
 
 def _mid(x, weight, bias=None, silu: bool = False, summed: bool = False):
     """(qt, splits) if x weight^T (or silu(gate) * up of it) takes mid_gemm,
     else None. summed: the consumer adds the sums of splits. It takes up to 256
     rows, but for what the streamed product (few rows of small weights, which
-    has no sums to add) or the library does as fast. us, here (other): 37888 x
-    3584 with the activation, 1 row 43.0 (48.1), 32 rows 43.1 (57.6), 128 rows
-    51.0 (71.2), 200 rows 65 (85); 152064 x 3584, 1 row 170 (182), 64 rows 201
-    (209), 200 rows 284 (325); 3584 x 18944, 1 row 22.7 and 0.3 of sums (27.4),
-    100 rows 30.3 and 3 (96.5). The others' side of the line: 3584 x 3584 and
-    its sums, 1 row 7.6 (6.2), 100 rows 15 (13.1); 57344 x 8192, whose tiles
-    fill the second round of CUs by 3/4, 200 rows 247 (228)."""
+    has no sums to add) or the library does as fast (_mid_sizes). us, here
+    (other): 37888 x 3584 with the activation, 1 row 42.2 (48.1), 32 rows 42.9
+    (57.6), 128 rows 51.0 (71.2), 200 rows 65 (85); 152064 x 3584, 1 row 168
+    (182), 64 rows 201 (209), 200 rows 284 (325); 3584 x 18944, 1 row 23.0 and
+    0.3 of sums (27.4), 100 rows 30.3 and 3 (96.5)."""
     if not (_USE_SKINNY and x.is_cuda and x.dim() == 2
             and 1 <= x.shape[0] <= 256
             and x.dtype == weight.dtype == torch.bfloat16):
         return None
-    M, (N, K) = x.shape[0], weight.shape
-    if silu:
-        N //= 2
-    if (K % 64 or N % 8 or not 64 <= K < 1 << 22 or not 0 < N < 1 << 24
-            or x.stride(0) >= 1 << 22 or (silu and 2 * N * K >= 1 << 31)):
-        return None
-    small = weight.shape[0] * K <= _SKINNY_MAX_ELEMS
-    if small and (M * K <= 16384 and N <= 4096 if summed
-                  else _streams(x, weight, silu, bias)):
-        return None
     if not (_plain(x, weight, bias)
+            and x.stride(0) < 1 << 22
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and (bias is None or (bias.dtype == x.dtype
                                   and bias.is_contiguous()))
             and native_available()):
         return None
-    qt, splits, _ = _mid_cut(M, N, K, silu, summed)
+    N, K = weight.shape
+    return _mid_sizes(x.shape[0], N // 2 if silu else N, K, silu, summed)
+
+
+@functools.lru_cache(maxsize=4096)
+def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
+    """_mid, by the sizes (N columns of the result). The others' side of the
+    lines, us, here (other), sums with their consumer:
+    - streamed: 5120 x 2048, 1 row 12.1 (10.2), 16 rows 13.4 (11.7); 3072 x
+      2048, 16 rows 11 (10); 1152 x 896, 24 rows 8.5 (7.2), 64 rows 10 (8);
+      3584 x 3584, 8 rows 12.0 (11.4), 4096 x 4096 13.5 (12.2); with the
+      activation 16384 x 4096, 1 row 32.3 (27.6), 8 rows 32.0 (30.3), whose
+      tiles of 64 rows fill all CUs, 11008 x 4096 (2/3 of them) 0.85 of it;
+    - library, sums: 3584 x 3584, 256 rows 23.9 (22.2), 100 rows 15 (20); 2048
+      x 4096, 200 rows 18.9 (17.2), 176 rows the same; 3072 x 2048, 250 rows 20
+      (16); 1152 x 896, 192 rows 13.3 (12); without a consumer 8192 x 2048, 96
+      rows 16.3 (14.5), 208 rows 24.0 (17.4), 64 rows 0.85 of it;
+    - library, whole: 57344 x 8192, whose tiles fill the second round of CUs by
+      3/4, 200 rows 247 (228); 50304 x 1024, 1 row 23.2 (21.0), 96 rows 28.7
+      (25.5), 50304 x 2048, 250 rows 69 (66), 128 rows 0.91; 4096 x 4096, 200 rows 23.2 (21.9), 12288 x 4096,
+      240 rows 45 (40), 256 rows, as other multiples of 32, 0.93 of it; 64128 x 8192, 192 rows 247 (209), 128 rows 0.86
+      of it, 32064 x 8192 0.91; gate and up 55296 x 5120, 0.84 full, 96 rows
+      128.6 (121.4), 57344 x 8192, 0.875 full, 0.87 of it."""
+    if (K % 64 or N % 8 or not 64 <= K < 1 << 22 or not 0 < N < 1 << 24
+            or (silu and 2 * N * K >= 1 << 31)):
+        return None
+    rows = 2 * N if silu else N
+    small = rows * K <= _SKINNY_MAX_ELEMS
+    if small and (M * K <= 16384 and N <= 4096
+                  or M * K <= 32768 and (K <= 2048 or 3072 <= N <= 4096)
+                  or M <= 64 and K <= 1024
+                  if summed else _stream_sizes(M, rows, K, silu)):
+        return None
+    if (M > 192 and M % 32 and 2048 < K <= 4096 and N * K <= 1 << 26
+            and not silu and not summed):
+        return None
+    qt, splits = _mid_cut(M, N, K, silu, summed)
     if splits == 1:
         tiles = -(-N // ((16 if silu else 32) * qt))
         fill = tiles / (256 * -(-tiles // 256))
-        if fill < (0.35 if silu and M <= 64 else 0.55 if M <= 64
-                   else 0.6 if M <= 128 or N * K <= 1 << 27 else 0.9):
+        least = (0.35 if silu and M <= 64 else 0.55 if M <= 64
+                 else 0.9 if M > 128 and N * K > 1 << 27
+                 else 0.86 if silu and N * K > 1 << 27 else 0.6)
+        if (fill < least or (M > 128 and K >= 8192 and tiles > 256)
+                or (tiles > 256 and fill < 0.8
+                    and (K <= 1024 or (K <= 2048 and M > 192)))
+                or (silu and qt == 2 and fill > 0.9
+                    and M <= 8 and K <= 4096)):
             return None
-    elif not summed:
-        if not (small or K >= 2 * N) or (M > 64 and N * K < 16_000_000):
+    elif summed:
+        if N * K < 13_000_000 and K <= 4096 and M > (
+                128 if K <= 1024 or (K <= 2048 and M % 32) else 192):
             return None
+    elif (not (small or K >= 2 * N)
+          or (M > 64 and (K <= 2048 or N * K < 16_000_000))):
+        return None
     return qt, splits
 
 

@@ -1449,6 +1449,32 @@ def test_mid_rule():
                 atol=2e-2, rtol=2e-2)  # both rounded to bf16, values up to 6
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (65, 8, 64), (200, 8, 128), (65, 5752, 128), (129, 5768, 64),  # 180 tiles of 32
+    (70, 22976, 192), (256, 328, 512), (9, 8192, 4096), (100, 1152, 896)])
+def test_products_around_the_cuts(M, N, K):
+    """Short K, narrow weights and either side of 180 tiles through the entry
+    points vs fp64, whatever kernel takes them: one rounding of each product
+    (three with an activation behind it), fp32 sums before."""
+    assert_native()
+    torch.manual_seed(N + K)
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    want = x.double() @ w.double().t()
+    size = x.double().abs() @ w.double().abs().t()  # fp32 sums err by some of it
+    for out in (ops.linear_bf16(x, w), ops.parts_sum(ops.linear_parts(x, w))):
+        assert bool(((out.double() - want).abs()
+                     <= 2 ** -8 * want.abs() + 2 ** -20 * size).all())
+    if N % 16:
+        return
+    g, u = want.chunk(2, 1)
+    want = torch.nn.functional.silu(g) * u
+    out = ops.linear_silu_mul(x, w).double()
+    # gate and up may be rounded in front of the activation (slope below 1.1)
+    tol = 2 ** -8 * (2 * want.abs() + 1.1 * g.abs() * u.abs()) + 2 ** -17 * (1 + u.abs())
+    assert bool(((out - want).abs() <= tol).all())
+
+
 def test_upload():
     """Host tensors that travel together keep types, shapes and values."""
     host = [torch.arange(7), None, torch.rand(3, 5), torch.empty(0, 4, dtype=torch.int32),

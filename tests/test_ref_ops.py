@@ -223,3 +223,59 @@ def test_objects_older_than_a_header_are_built_again(tmp_path):
         os.utime(path, (at, at))
     drop_older(str(out), str(src))
     assert sorted(p.name for p in out.iterdir()) == ["lib.so", "new.o"]
+
+
+def test_mid_sizes_are_whole_cuts():
+    """Over a grid of sizes, what mid_gemm is given is a cut that its kernel has:
+    16 * 2, 4 or 5 weight rows a wave, at least a step of 64 columns a run of K,
+    one run with the activation."""
+    from arks_amd import ops
+
+    taken = set()
+    for M in (1, 2, 8, 17, 64, 65, 128, 129, 192, 193, 256):
+        for N in (8, 64, 328, 1024, 4608, 5752, 5760, 5768, 11520, 11528, 22976,
+                  28672, 57344, 151936):
+            for K in (64, 128, 192, 320, 512, 896, 2048, 3584, 8192, 18944):
+                for silu, summed in ((False, False), (False, True), (True, False)):
+                    cut = ops._mid_sizes(M, N, K, silu, summed)
+                    if cut is None:
+                        continue
+                    qt, splits = cut
+                    assert qt in (2, 4, 5)
+                    assert 1 <= splits <= min(8, K // 64)
+                    assert not silu or splits == 1
+                    taken.add((qt, splits > 1, silu))
+    assert taken == {(qt, many, silu) for qt in (2, 4, 5) for many in (False, True)
+                     for silu in (False, True) if not (many and silu)}
+    for bad in ((1, 8, 96), (1, 12, 64), (1, 8, 32), (1, 0, 64), (1, 1 << 24, 64),
+                (1, 8, 1 << 22)):
+        assert ops._mid_sizes(*bad, False, True) is None
+
+
+def test_mid_sizes_leave_what_others_do_faster():
+    """Both sides of the measured lines."""
+    from arks_amd import ops
+
+    takes = lambda *size, **kind: ops._mid_sizes(
+        *size, kind.get("silu", False), kind.get("summed", False)) is not None
+    summed = [  # M, N, K: streamed or the library's; beside it, taken
+        ((16, 5120, 2048), (24, 5120, 2048)), ((16, 3072, 2048), (48, 3072, 2048)),
+        ((64, 1152, 896), (65, 1152, 896)), ((129, 1152, 896), (128, 1152, 896)),
+        ((8, 4096, 4096), (16, 4096, 4096)), ((8, 3584, 3584), (16, 3584, 3584)),
+        ((8, 4096, 4096), (8, 4608, 3584)), ((8, 4096, 4096), (8, 2048, 4096)),
+        ((200, 2048, 4096), (192, 2048, 4096)), ((256, 3584, 3584), (256, 4608, 3584)),
+        ((176, 5120, 2048), (160, 5120, 2048)), ((250, 896, 896), (250, 896, 4864))]
+    for left, taken in summed:
+        assert not takes(*left, summed=True) and takes(*taken, summed=True)
+    plain = [
+        ((96, 8192, 2048), (64, 8192, 2048)), ((129, 64128, 8192), (128, 64128, 8192)),
+        ((129, 64128, 8192), (129, 32064, 8192)), ((200, 4096, 4096), (192, 4096, 4096)),
+        ((96, 50304, 1024), (96, 50304, 2048)), ((250, 50304, 2048), (192, 50304, 2048)),
+        ((240, 12288, 4096), (256, 12288, 4096)), ((240, 12288, 4096), (240, 24576, 4096))]
+    for left, taken in plain:
+        assert not takes(*left) and takes(*taken)
+    gated = [  # N: gate columns
+        ((8, 8192, 4096), (9, 8192, 4096)), ((8, 8192, 4096), (8, 5504, 4096)),
+        ((96, 27648, 5120), (64, 27648, 5120)), ((96, 27648, 5120), (96, 28672, 8192))]
+    for left, taken in gated:
+        assert not takes(*left, silu=True) and takes(*taken, silu=True)
