@@ -894,27 +894,44 @@ def linear_f32_lib(x, weight):
     return F.linear(x, weight).float()
 
 
+@functools.lru_cache(maxsize=4096)
 def _tile_fill(M: int, N: int) -> float:
     """Share of the chip that tiles of 256 (the last of 128) rows x 128 columns
-    keep busy with rows that are there: they run in rounds of 256."""
+    keep busy with rows that are there: workgroups of an XCD take its tiles in
+    turn, those of the last rows, 0.55 of a whole one's time, behind the others
+    (tile_gemm.hip). 600 rows x 96 columns of tiles are 24 and 12 on each of 8
+    XCDs of 32 workgroups, so that some have one of each."""
     rows, left = divmod(M, 256)
-    cost = rows + (0 if left == 0 else 0.55 if left <= 128 else 1.0)
+    rows, tail = rows + (left > 128), 0 < left <= 128
     cols = -(-N // 128)
-    return M * N / (256 * 128 * 256 * math.ceil(cost * cols / 256))
+    slots = min(256, -(-(rows + tail) * cols // 8) * 8) // 8
+    longest = 0.0
+    for xcd in range(8):
+        whole = rows * cols * (xcd + 1) // 8 - rows * cols * xcd // 8
+        every = whole + tail * (cols * (xcd + 1) // 8 - cols * xcd // 8)
+        for at in (0, whole % slots, every % slots):  # where the counts drop
+            n = -(-max(0, whole - at) // slots)
+            longest = max(longest, n + 0.55 * (-(-max(0, every - at) // slots) - n))
+    return M * N / (256 * 128 * 256 * longest)
 
 
 def _tiles(x, weight) -> bool:
     """Whether silu_mul(x weight^T) takes the product of tile_gemm.hip, with
     its activation inside, rather than the library's and a pass behind it: many
-    rows, and tiles that fill their rounds over the chip. 18944 x 3584, us,
-    here (library and activation): 384 rows 130 (122), 512 rows 158 (148), 600
-    rows 167 (173), 900 rows 235 (291), 1024 rows 245 (260), 2017 rows 409
-    (547), 2048 rows 406 (433), 3150 rows 623 (811), 8192 rows 1523 (1636):
-    round row counts have picked library kernels, others not."""
+    rows, and tiles that fill their rounds over the chip, the more so the longer
+    K is, as the library's loop is faster and the activation's pass counts for
+    less. us, here (library and activation): 18944 x 3584, 384 rows 130 (122),
+    512 rows 158 (148), 600 rows 167 (173), 900 rows 235 (291), 1024 rows 245
+    (260), 2017 rows 409 (547), 3150 rows 623 (811), 8192 rows 1540 (1636);
+    12288 x 4096, 600 rows (0.57 full) 1.26 of the library's time, 900 rows
+    (0.66) 1.11, 1200 rows (0.88) 0.96; 14336 x 8192, 640 rows (0.71) 1.15, 900
+    rows (0.77) 0.96; 13824 x 5120, 1300 rows (0.71) 1.07, 900 rows (0.74)
+    0.78: the library's kernels turn with the row count too."""
     M, (N, K) = x.shape[0], weight.shape
+    least = 0.67 if K < 4096 else 0.72 if K < 8192 else 0.75
     return (M > 512 and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16
             and K % 64 == 0 and 64 <= K < 1 << 22 and N % 16 == 0
-            and x.stride(0) < 1 << 22 and _tile_fill(M, N // 2) >= 0.65
+            and x.stride(0) < 1 << 22 and _tile_fill(M, N // 2) >= least
             and _plain(x, weight)
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and native_available())

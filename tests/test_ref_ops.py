@@ -279,3 +279,22 @@ def test_mid_sizes_leave_what_others_do_faster():
         ((96, 27648, 5120), (64, 27648, 5120)), ((96, 27648, 5120), (96, 28672, 8192))]
     for left, taken in gated:
         assert not takes(*left, silu=True) and takes(*taken, silu=True)
+
+
+def test_tile_fill_is_what_the_schedule_takes():
+    """The share against the schedule walked out: every workgroup's tiles of its
+    XCD in turn, 1 for a whole one and 0.55 for those of the last 128 rows."""
+    from arks_amd import ops
+
+    for M in (1, 128, 129, 256, 257, 513, 600, 640, 900, 1024, 2017, 3150, 8192):
+        for N in (8, 128, 1000, 4096, 9472, 12288, 14336, 18944, 28672):
+            left, cols = M % 256, -(-N // 128)
+            rows, tail = M // 256 + (left > 128), 0 < left <= 128
+            slots = min(256, -(-(rows + tail) * cols // 8) * 8) // 8
+            longest = 0
+            for xcd in range(8):
+                part = lambda n: n * (xcd + 1) // 8 - n * xcd // 8
+                cost = [1.0] * part(rows * cols) + [0.55] * (tail * part(cols))
+                longest = max([longest] + [sum(cost[s::slots]) for s in range(slots)])
+            want = M * N / (256 * 128 * 256 * longest)
+            assert abs(ops._tile_fill(M, N) / want - 1) < 1e-9, (M, N)
