@@ -1064,6 +1064,30 @@ def _moe_whole(x, H: int, I: int, pairs: int) -> bool:
             and 2 * I * H < 1 << 31 and pairs < (1 << 23) - 255)
 
 
+def _moe_way(rows: int, top_k: int, El: int, experts: int, H: int, I: int,
+             whole: bool):
+    """(pairs of an item, whether in mid_gemm.hip) for El experts here of
+    `experts` in all: moe_tile's, and 256 (tile_engine.h) in place of 128 where
+    whole. Experts whose columns leave most CUs without a tile keep the kernels
+    with more of them, us, 16 (64 of mid_gemm), 128 (256): 4 experts of 512 x
+    256, 2 per row, 16 rows 13 (21), 64 rows 24 (21) in tiles of 128, 1000 rows
+    29 (36), 5000 rows 47 (45); 16 experts of 4096 x 1024, 4 per row, 256 tiles
+    of 64 columns, 16 rows 88 (86), 400 rows 132 (131)."""
+    pairs = rows * top_k
+    few = El * -(-I // 64) < 64 and pairs <= 8 * experts
+    # the streamed kernel takes whole matrix operands of 32 columns only (16
+    # experts of 2056 x 1416, 4 per row, 7 rows, with routing: 95 us in tiles,
+    # 120 us as batched products)
+    tile = (moe_tile(rows, top_k, experts, whole and not few)
+            if (H | I) % 32 == 0 else 128)
+    if tile == 64:
+        return (128 if pairs > 32 * experts else 64), True
+    if (tile == 128 and whole
+            and (El + pairs // 256) * -(-I // 128) >= 64):
+        tile = 256
+    return tile, False
+
+
 def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
                 experts: int | None = None):
     """sum_j weights[t, j] * expert(ids[t, j])(x[t]) over the silu-GLU experts
@@ -1076,19 +1100,11 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
             and I % 8 == 0 and El <= 1024 and k <= 16):
         out = torch.empty((x.shape[0], H), dtype=x.dtype, device=x.device)
         x = _rows_16b(x)
-        # the streamed kernel takes whole matrix operands of 32 columns only
-        # (16 experts of 2056 x 1416, 4 per row, 7 rows, with routing: 95 us
-        # in tiles, 120 us as batched products)
-        rows, experts = x.shape[0], experts or El
-        whole = _moe_whole(x, H, I, rows * k)
-        tile = (moe_tile(rows, k, experts, whole) if (H | I) % 32 == 0 else 128)
-        mid = tile == 64
-        if mid and rows * k > 32 * experts:
-            tile = 128
-        elif tile == 128 and whole:
-            tile = 256
-        _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, tile,
-                              mid)
+        rows = x.shape[0]
+        _native().moe_experts(
+            out, x, w13, w2, weights, ids, expert_base,
+            *_moe_way(rows, k, El, experts or El, H, I,
+                      _moe_whole(x, H, I, rows * k)))
         return out
     return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
 

@@ -298,3 +298,23 @@ def test_tile_fill_is_what_the_schedule_takes():
                 longest = max([longest] + [sum(cost[s::slots]) for s in range(slots)])
             want = M * N / (256 * 128 * 256 * longest)
             assert abs(ops._tile_fill(M, N) / want - 1) < 1e-9, (M, N)
+
+
+def test_moe_way():
+    """Pairs of an item and their kernel: by pairs per expert, and for experts
+    so small that larger items leave most of the chip idle."""
+    from arks_amd import ops
+
+    big = lambda rows, whole=True: ops._moe_way(rows, 8, 128, 128, 2048, 768, whole)
+    assert [big(n) for n in (15, 16, 512, 513, 1024, 1025)] == [
+        (16, False), (64, True), (64, True), (128, True), (128, True), (256, False)]
+    assert [big(n, False) for n in (16, 128, 129, 5000)] == [
+        (16, False), (16, False), (128, False), (128, False)]
+    # a rank's 16 of 128 experts
+    assert ops._moe_way(64, 8, 16, 128, 2048, 768, True) == (64, True)
+    tiny = lambda rows: ops._moe_way(rows, 2, 4, 4, 512, 256, True)
+    assert [tiny(n) for n in (1, 16, 17, 64, 65, 128, 129, 2000, 5000)] == [
+        (16, False), (16, False), (64, True), (64, True), (128, True), (128, True),
+        (128, False), (128, False), (256, False)]
+    # no whole steps of 32: tiles of 128
+    assert ops._moe_way(7, 4, 16, 16, 2056, 1416, False) == (128, False)
