@@ -532,6 +532,9 @@ def skinny_gemm(x, weight, bias=None):
     return parts_sum(Parts(_stream_parts(x, weight), bias))
 
 
+# 0: products take the library's kernels (up to 256 rows, and gate and up
+# products of any number), experts the kernels of moe_gemm.hip without the
+# engine: for comparisons
 _USE_SKINNY = os.environ.get("ARKS_SKINNY_GEMM", "1") == "1"
 # weights up to this many elements take the framework's kernels at any number
 # of rows up to 64, larger ones where the rules below say so
@@ -929,8 +932,9 @@ def _tiles(x, weight) -> bool:
     0.78: the library's kernels turn with the row count too."""
     M, (N, K) = x.shape[0], weight.shape
     least = 0.67 if K < 4096 else 0.72 if K < 8192 else 0.75
-    return (M > 512 and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16
-            and K % 64 == 0 and 64 <= K < 1 << 22 and N % 16 == 0
+    return (_USE_SKINNY and M > 512 and x.is_cuda
+            and x.dtype == weight.dtype == torch.bfloat16 and K % 64 == 0
+            and 64 <= K < 1 << 22 and N % 16 == 0
             and x.stride(0) < 1 << 22 and _tile_fill(M, N // 2) >= least
             and _plain(x, weight)
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0
@@ -1060,7 +1064,8 @@ def _moe_whole(x, H: int, I: int, pairs: int) -> bool:
     were never the faster ones: 128 experts of 2048 x 768, 8 per row, us, 256
     (128): 200 rows 242 (265), 5012 rows 545 (742); 8 of 4096 x 14336, 2 per
     row: 200 rows 565 (611), 8192 rows 4527 (9434)."""
-    return ((H | I) % 64 == 0 and x.shape[0] * x.stride(0) < 1 << 31
+    return (_USE_SKINNY and (H | I) % 64 == 0
+            and x.shape[0] * x.stride(0) < 1 << 31
             and 2 * I * H < 1 << 31 and pairs < (1 << 23) - 255)
 
 

@@ -1591,6 +1591,21 @@ def test_tiles_rule():
         atol=2e-2, rtol=2e-2)  # both factors rounded to bf16 there
 
 
+def test_switch_to_the_library(monkeypatch):
+    """ARKS_SKINNY_GEMM=0: every product of linear_* is the library's, experts
+    keep to moe_gemm.hip's own tiles."""
+    assert_native()
+    w = torch.empty(2 * 18944, 64, dtype=torch.bfloat16, device=DEV)
+    x = torch.randn(2017, 64, dtype=torch.bfloat16, device=DEV)
+    routes = lambda: [bool(r) for r in (
+        ops._streams(x[:1], w[:64]), ops._splits(x[:1], w[:64]),
+        ops._mid(x[:128], w), ops._tiles(x, w),
+        ops._moe_whole(x, 64, 64, 100))]
+    assert routes() == [True] * 5
+    monkeypatch.setattr(ops, "_USE_SKINNY", False)
+    assert routes() == [False] * 5
+
+
 def test_streams_refuses():
     """What the streamed product leaves to the other paths."""
     assert_native()
