@@ -679,6 +679,7 @@ def _mid(x, weight, bias=None, silu: bool = False, summed: bool = False):
             and x.stride(0) < 1 << 22
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and (bias is None or (bias.dtype == x.dtype
+                                  and bias.shape == weight.shape[:1]
                                   and bias.is_contiguous()))
             and native_available()):
         return None

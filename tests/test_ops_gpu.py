@@ -1591,6 +1591,20 @@ def test_tiles_rule():
         atol=2e-2, rtol=2e-2)  # both factors rounded to bf16 there
 
 
+def test_products_that_broadcast():
+    """What the library takes beside a matrix and its bias stays accepted beyond
+    the few rows that the streamed products look at: one bias for all columns,
+    or a row of them."""
+    assert_native()
+    x = torch.randn(100, 256, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(16384, 256, dtype=torch.bfloat16, device=DEV)
+    one = torch.ones(1, dtype=torch.bfloat16, device=DEV)
+    assert ops._mid(x, w) and ops._mid(x, w, torch.zeros_like(w[:, 0]))
+    for bias in (one, torch.ones_like(w[:1, 0]).expand(1, 16384)):
+        for out in (ops.linear_bf16(x, w, bias), ops.linear_parts(x, w, bias)):
+            assert torch.equal(ops.parts_sum(out), torch.nn.functional.linear(x, w, bias))
+
+
 def test_switch_to_the_library(monkeypatch):
     """ARKS_SKINNY_GEMM=0: every product of linear_* is the library's, experts
     keep to moe_gemm.hip's own tiles."""
