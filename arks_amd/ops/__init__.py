@@ -367,7 +367,7 @@ def attention_extend_paged(
             )
             if ctab.numel():
                 C.attention_extend2_combine(
-                    out, ws, ctab, cu_seqlens_q, scale,
+                    out, ws, ctab, cu_seqlens_q, scale, k_cache.shape[1] * maps,
                 )
         if t64.numel():
             assert sink_w is None and slopes is None

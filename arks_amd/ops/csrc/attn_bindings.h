@@ -41,8 +41,8 @@ void arks_attn_extend_paged2(void* out, const void* q, const void* k_cache,
 void arks_attn_extend2_combine(void* out, const void* part_ws,
                                const void* combine_table,
                                const void* cu_seqlens_q, int n_split,
-                               float scale, int num_q_heads, int head_dim,
-                               hipStream_t stream);
+                               float scale, int num_q_heads, int num_kv_heads,
+                               int head_dim, hipStream_t stream);
 }
 
 namespace {
@@ -226,17 +226,21 @@ inline void attention_extend_paged2(torch::Tensor out, torch::Tensor q,
 }
 inline void attention_extend2_combine(torch::Tensor out, torch::Tensor part_ws,
                                torch::Tensor combine_table,
-                               torch::Tensor cu_seqlens_q, double scale) {
+                               torch::Tensor cu_seqlens_q, double scale,
+                               int64_t num_kv_heads) {
   check_bf16_rowstrided(out, "out");
   TORCH_CHECK(part_ws.scalar_type() == torch::kFloat32);
   TORCH_CHECK(combine_table.scalar_type() == torch::kInt32 &&
               combine_table.dim() == 2 && combine_table.size(1) == 4);
   const int num_q_heads = out.size(1);
   const int head_dim = out.size(2);
+  // (which XCD reads what follows from it, the result does not)
+  if (num_kv_heads <= 0) num_kv_heads = num_q_heads;
+  TORCH_CHECK(num_q_heads % num_kv_heads == 0);
   arks_attn_extend2_combine(out.data_ptr(), part_ws.data_ptr(),
                             combine_table.data_ptr(), cu_seqlens_q.data_ptr(),
                             combine_table.size(0), (float)scale, num_q_heads,
-                            head_dim, attn_current_stream());
+                            (int)num_kv_heads, head_dim, attn_current_stream());
 }
 
 inline void def_paged_attention(pybind11::module_& m) {
@@ -249,7 +253,9 @@ inline void def_paged_attention(pybind11::module_& m) {
         arg("kv_lens"), arg("cu_seqlens_q"), arg("tile_info"), arg("part_ws"),
         arg("scale"), arg("window"), arg("sink"), arg("maps"),
         arg("sink_w") = pybind11::none(), arg("slopes") = pybind11::none());
-  m.def("attention_extend2_combine", &attention_extend2_combine);
+  m.def("attention_extend2_combine", &attention_extend2_combine, arg("out"),
+        arg("part_ws"), arg("combine_table"), arg("cu_seqlens_q"), arg("scale"),
+        arg("num_kv_heads") = 0);
 }
 
 }  // namespace

@@ -143,6 +143,42 @@ __device__ __forceinline__ float e2_halves_sum(const float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The head and tile of a workgroup. Workgroups go round the XCDs in launch
+// order. An XCD keeps to as few key/value heads as it can, so that their tiles
+// meet in its L2: heads that 8 is a multiple of take 8 / heads XCDs each,
+// multiples of 8 go round.
+struct E2Place {
+  int h, y;
+};
+__device__ __forceinline__ E2Place e2_place(const int num_q_heads,
+                                            const int num_kv_heads) {
+  const int gq = num_q_heads / num_kv_heads, xcd = blockIdx.x % 8;
+  int at = blockIdx.x / 8, kvh;
+  if (8 % num_kv_heads == 0) {
+    const int per = 8 / num_kv_heads;
+    kvh = xcd / per;
+    at = at * per + xcd % per;
+  } else if (num_kv_heads % 8 == 0) {
+    const int per = num_kv_heads / 8;
+    kvh = xcd * per + at / gq % per;
+    at = at / (gq * per) * gq + at % gq;
+  } else {
+    const int all = blockIdx.x % num_q_heads;
+    kvh = all / gq;
+    at = blockIdx.x / num_q_heads * gq + all % gq;
+  }
+  return E2Place{kvh * gq + at % gq, at / gq};
+}
+// Workgroups for so many tiles of every head: where heads share XCDs, 8 times
+// those of the fullest one (the places behind the last tile return).
+static inline int e2_grid(const int num_q_heads, const int num_kv_heads,
+                          const int tiles) {
+  const int per_head = num_q_heads / num_kv_heads * tiles;
+  return 8 % num_kv_heads == 0
+             ? 8 * ((per_head + 8 / num_kv_heads - 1) / (8 / num_kv_heads))
+             : num_q_heads * tiles;
+}
+
 template <int HEAD_DIM, bool BIASED, bool SKIP>
 __global__ __launch_bounds__(512, 2) void attn_extend2_kernel(
     bf16* __restrict__ out,            // [Tq, Hq, D]
@@ -184,30 +220,9 @@ __global__ __launch_bounds__(512, 2) void attn_extend2_kernel(
     return HEAD_DIM == 128 ? (r & 3) << 2 : (r & 2) << 1;
   };
 
-  // Workgroups go round the XCDs in launch order. An XCD keeps to as few
-  // key/value heads as it can, so that their tiles meet in its L2: heads that
-  // 8 is a multiple of take 8 / heads XCDs each, multiples of 8 go round.
-  int h, y;
-  {
-    const int gq = num_q_heads / num_kv_heads, xcd = blockIdx.x % 8;
-    int at = blockIdx.x / 8, kvh;
-    if (8 % num_kv_heads == 0) {
-      const int per = 8 / num_kv_heads;
-      kvh = xcd / per;
-      at = at * per + xcd % per;
-    } else if (num_kv_heads % 8 == 0) {
-      const int per = num_kv_heads / 8;
-      kvh = xcd * per + at / gq % per;
-      at = at / (gq * per) * gq + at % gq;
-    } else {
-      const int all = blockIdx.x % num_q_heads;
-      kvh = all / gq;
-      at = blockIdx.x / num_q_heads * gq + all % gq;
-    }
-    y = at / gq;
-    h = kvh * gq + at % gq;
-    if (y >= num_tiles) return;
-  }
+  const E2Place place = e2_place(num_q_heads, num_kv_heads);
+  const int h = place.h, y = place.y;
+  if (y >= num_tiles) return;
   const int kvh = h / (num_q_heads / num_kv_heads);
   const int seq_idx = tile_info[y * 4];
   const int q0 = tile_info[y * 4 + 1];
@@ -628,13 +643,17 @@ __global__ __launch_bounds__(512, 2) void attn_extend2_kernel(
   }
 }
 
-// Merge the flash partials of split tiles: grid (Hq, n_split, groups of 8
-// rows); combine_table rows = (first_y, nparts, seq, q0). Standard flash merge
+// Merge the flash partials of split tiles: heads as in the kernel above x
+// (n_split, groups of 8 rows); combine_table rows = (first_y, nparts, seq, q0). Standard flash merge
 // in f32: m* = max m_p; out = sum_p exp(m_p - m*) O_p / sum_p
 // exp(m_p - m*) l_p (m is base-2: exp2). Reading the slabs bounds it, so the
 // loads of 2, 4 or 8 parts, as many as there are, are in flight together, two
 // dims a thread. Tiles of 3 parts, 28 heads, chunks of up to 2048 rows: 14.2 us
 // on the mean (90 MB at the most; with 8 loads for any number of parts 23.2).
+// A head's workgroups are on the XCD (or one of the XCDs) that wrote its slabs:
+// read on another one, their next writing was slower too (32/8 heads, 256 rows
+// behind 5000 keys in 8 parts: 22.4 + 7.3 us with a window of 1024, now 19.8 +
+// 7.0; of 128, 19.6 + 7.2, now 15.4 + 7.1).
 template <int HEAD_DIM, int PARTS>
 __device__ __forceinline__ void e2_combine_rows(
     bf16* __restrict__ to, const float* __restrict__ base,
@@ -684,9 +703,12 @@ __global__ __launch_bounds__(256) void attn_extend2_combine_kernel(
     bf16* __restrict__ out, const float* __restrict__ part_ws,
     const int* __restrict__ combine_table,
     const int* __restrict__ cu_seqlens_q, const float scale,
-    const int num_q_heads) {
-  const int h = blockIdx.x;
-  const int* entry = combine_table + blockIdx.y * 4;
+    const int num_q_heads, const int num_kv_heads, const int n_split) {
+  constexpr int GROUPS = E2_QTILE / 8;
+  const E2Place place = e2_place(num_q_heads, num_kv_heads);
+  const int h = place.h;
+  if (place.y >= n_split * GROUPS) return;
+  const int* entry = combine_table + place.y / GROUPS * 4;
   const int nparts = entry[1], seq_idx = entry[2], q0 = entry[3];
   const int q_start = cu_seqlens_q[seq_idx];
   const int q_len = cu_seqlens_q[seq_idx + 1] - q_start;
@@ -695,7 +717,7 @@ __global__ __launch_bounds__(256) void attn_extend2_combine_kernel(
                       (int64_t)h * E2_QTILE * (HEAD_DIM + 2);
   const int64_t out_stride = (int64_t)num_q_heads * HEAD_DIM;
   bf16* to = out + (q_start + q0) * out_stride + (int64_t)h * HEAD_DIM;
-  const int row0 = blockIdx.z * 8, rows = q_len - q0;
+  const int row0 = place.y % GROUPS * 8, rows = q_len - q0;
   const float scale2 = scale * E2_LOG2E;
 #define ARKS_ROWS(P)                                                         \
   e2_combine_rows<HEAD_DIM, P>(to, base, slab_stride, out_stride, row0, rows, \
@@ -717,12 +739,7 @@ extern "C" void arks_attn_extend_paged2(
     int num_q_heads, int num_kv_heads, int head_dim, int max_blocks,
     int64_t q_stride, int window, int sink, int maps, const void* sink_w,
     const void* slopes, hipStream_t stream) {
-  // 8 XCDs with as many workgroups each as the fullest one needs
-  const int per_head = num_q_heads / num_kv_heads * ntiles;
-  const int grid =
-      8 % num_kv_heads == 0
-          ? 8 * ((per_head + 8 / num_kv_heads - 1) / (8 / num_kv_heads))
-          : num_q_heads * ntiles;
+  const int grid = e2_grid(num_q_heads, num_kv_heads, ntiles);
   const dim3 block(512);
   static bool attr_set[6] = {};
   auto launch = [&](auto kern, int lds_bytes, int idx) {
@@ -757,17 +774,15 @@ extern "C" void arks_attn_extend_paged2(
 extern "C" void arks_attn_extend2_combine(
     void* out, const void* part_ws, const void* combine_table,
     const void* cu_seqlens_q, int n_split, float scale, int num_q_heads,
-    int head_dim, hipStream_t stream) {
-  dim3 grid(num_q_heads, n_split, E2_QTILE / 8), block(256);
-  if (head_dim == 128) {
-    hipLaunchKernelGGL((attn_extend2_combine_kernel<128>), grid, block, 0,
-                       stream, (bf16*)out, (const float*)part_ws,
-                       (const int*)combine_table, (const int*)cu_seqlens_q,
-                       scale, num_q_heads);
-  } else if (head_dim == 64) {
-    hipLaunchKernelGGL((attn_extend2_combine_kernel<64>), grid, block, 0,
-                       stream, (bf16*)out, (const float*)part_ws,
-                       (const int*)combine_table, (const int*)cu_seqlens_q,
-                       scale, num_q_heads);
-  }
+    int num_kv_heads, int head_dim, hipStream_t stream) {
+  if (n_split == 0) return;
+  const dim3 grid(e2_grid(num_q_heads, num_kv_heads, n_split * (E2_QTILE / 8)));
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, (bf16*)out,
+                       (const float*)part_ws, (const int*)combine_table,
+                       (const int*)cu_seqlens_q, scale, num_q_heads,
+                       num_kv_heads, n_split);
+  };
+  if (head_dim == 128) launch(attn_extend2_combine_kernel<128>);
+  else if (head_dim == 64) launch(attn_extend2_combine_kernel<64>);
 }
