@@ -5,9 +5,10 @@ different rope_theta/vocab). HF-config-driven (arks_amd.config.ModelConfig);
 weight names follow the HF checkpoint layout so safetensors load directly.
 
 Compute path: arks_amd.ops HIP kernels for the products of up to 256 rows, the
-gate and up products and experts of any number, RMSNorm / RoPE / paged attention
-/ SwiGLU; F.linear (hipBLASLt) for the other products of many rows; TP via column/row-parallel shards
-with one RCCL all-reduce per attention and per MLP block.
+gate and up products of many and experts of any number, RMSNorm / RoPE / paged
+attention / SwiGLU; F.linear (hipBLASLt) for the other products; TP via
+column/row-parallel shards with one RCCL all-reduce per attention and per MLP
+block.
 """
 
 from __future__ import annotations

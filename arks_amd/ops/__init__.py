@@ -600,10 +600,9 @@ def _streams(x, weight, silu: bool = False, bias=None) -> bool:
 
 
 def _stream_sizes(M: int, N: int, K: int, silu: bool = False) -> bool:
-    """_streams, by the sizes. A workgroup reads all of x's rows
-    beside its 16 or 32 weight rows, so the line lies where that traffic (rows
-    x K), and the waves' tails, meet what the other path loses: us, here
-    (other), the other being the split product with its sums up to
+    """_streams, by the sizes. A workgroup reads all of x's rows beside its 16
+    or 32 weight rows, so the line lies where that traffic (rows x K), and the
+    waves' tails, meet what the other path loses: us, here (other), the other being the split product with its sums up to
     _SKINNY_MAX_ELEMS and the library beyond. 3584 x 3584: 1 row 7.4 (10.9),
     16 rows 9.5 (11.3), 32 rows 12.5 (13.0). 5120 x 2048, 32 rows 10.4 (12.4);
     6144 x 4096, 32 rows 20.1 (17.7); 544 x 8192, 8 rows 13.8 (10.4). Library:
@@ -702,10 +701,11 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
       rows 16.3 (14.5), 208 rows 24.0 (17.4), 64 rows 0.85 of it;
     - library, whole: 57344 x 8192, whose tiles fill the second round of CUs by
       3/4, 200 rows 247 (228); 50304 x 1024, 1 row 23.2 (21.0), 96 rows 28.7
-      (25.5), 50304 x 2048, 250 rows 69 (66), 128 rows 0.91; 4096 x 4096, 200 rows 23.2 (21.9), 12288 x 4096,
-      240 rows 45 (40), 256 rows, as other multiples of 32, 0.93 of it; 64128 x 8192, 192 rows 247 (209), 128 rows 0.86
-      of it, 32064 x 8192 0.91; gate and up 55296 x 5120, 0.84 full, 96 rows
-      128.6 (121.4), 57344 x 8192, 0.875 full, 0.87 of it."""
+      (25.5), 50304 x 2048, 250 rows 69 (66), 128 rows 0.91 of it; 4096 x 4096,
+      200 rows 23.2 (21.9), 12288 x 4096, 240 rows 45 (40), 256 rows, as other
+      multiples of 32, 0.93 of it; 64128 x 8192, 192 rows 247 (209), 128 rows
+      0.86 of it, 32064 x 8192 0.91; gate and up 55296 x 5120, 0.84 full, 96
+      rows 128.6 (121.4), 57344 x 8192, 0.875 full, 0.87 of it."""
     if (K % 64 or N % 8 or not 64 <= K < 1 << 22 or not 0 < N < 1 << 24
             or (silu and 2 * N * K >= 1 << 31)):
         return None

@@ -644,8 +644,8 @@ __global__ __launch_bounds__(512, 2) void attn_extend2_kernel(
 }
 
 // Merge the flash partials of split tiles: heads as in the kernel above x
-// (n_split, groups of 8 rows); combine_table rows = (first_y, nparts, seq, q0). Standard flash merge
-// in f32: m* = max m_p; out = sum_p exp(m_p - m*) O_p / sum_p
+// (n_split, groups of 8 rows); combine_table rows = (first_y, nparts, seq, q0).
+// Standard flash merge in f32: m* = max m_p; out = sum_p exp(m_p - m*) O_p / sum_p
 // exp(m_p - m*) l_p (m is base-2: exp2). Reading the slabs bounds it, so the
 // loads of 2, 4 or 8 parts, as many as there are, are in flight together, two
 // dims a thread. Tiles of 3 parts, 28 heads, chunks of up to 2048 rows: 14.2 us

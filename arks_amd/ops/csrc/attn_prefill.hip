@@ -12,8 +12,9 @@
 // (guide common-mistake #6). P is staged through a per-wave padded LDS buffer
 // to re-shape for the PV A-fragment.
 //
-// This kernel is the prefill half of the runtime-slot contract (vLLM's flash prefill at reference
-// arksapplication_controller.go:941-955 delegated it to an external image).
+// This kernel is the prefill half of the runtime-slot contract (vLLM's flash
+// prefill at reference arksapplication_controller.go:941-955 delegated it to an
+// external image).
 #include "common.h"
 
 #include <cfloat>

@@ -1,21 +1,24 @@
 // out[M, N] = a[M, K] . w[N, K]^T (+ bias), or silu(gate) * up of two such
-// products, for 17 to 256 rows: steps that decode many requests, short prompts.
+// products, for up to 256 rows: steps that decode, short prompts.
 //
-// Between the products that the weights' stream alone bounds (stream_gemm.hip)
-// and those that the matrix cores bound (tile_engine.h) both take about the
-// same time: 200 rows x 37888 x 3584 are 45 us of weights and 39 us of matrix
-// operations. So all rows of a meet a weight row at once (it is read once), the
+// A few rows are bound by the weights' stream, 200 by both it and the matrix
+// cores (200 rows x 37888 x 3584 are 45 us of weights and 39 us of matrix
+// operations; tile_engine.h is for those that the cores alone bound, and
+// stream_gemm.hip takes few rows of small weights, without sums for anyone to
+// add). So all rows of a meet a weight row at once (it is read once), the
 // weights' rows are cut as finely as gives every CU one tile of them (or, for
 // small products, one run of K: fp32 sums of the runs for the consumer to
 // add), and loads run NS - 1 steps of 64 columns ahead.
 //
 // 8 waves, 2 along the weights x 4 along the rows of a: a wave holds 16 * QT
-// weight rows x 16 * FT rows of a. The two groups of four take turns, one reads
-// its operands of half a step from LDS while the other multiplies; rows go from
-// memory straight into LDS, their 16-byte pieces permuted by the row's number
-// (as in tile_engine.h, whose rules for waits hold here too: what a phase read
-// may be overwritten from the next phase on, and what a phase waited for may
-// be read from the next phase on).
+// weight rows x 16 * FT rows of a. The two groups of four take turns: in a slot
+// between two barriers one reads a whole step's operands from LDS (64 columns),
+// asks for the rows of step s + NS - 1 and waits, while the other multiplies the
+// step that it read in the slot before. Rows go from memory straight into LDS,
+// their 16-byte pieces permuted by the row's number (as in tile_engine.h, whose
+// rules for waits hold here too, a phase being such a step: what it read may be
+// overwritten from the next one on, and what it waited for may be read from the
+// next one on).
 #include "parts.h"
 #include "tile_engine.h"
 

@@ -3,22 +3,25 @@
 //
 //   moe_plan   pairs sorted by expert, cut into items of one expert and at
 //              most `tile` pairs; every pair's place in the sorted order
-//   moe_stream few experts with a pair or two (from one pair per expert on the
-//              mean mid_gemm.hip takes them, and where sizes are whole steps
-//              of 64): bound by the stream of the chosen experts' weights. Tiles of 16 weight rows (gate and up rows
-//              side by side), the waves of a workgroup splitting K, no LDS
-//              and no barrier before the final sum over the waves. 7 rows, 8
-//              of 128 experts each (2048 x 768): 90 us for 46 experts' 434 MB
+//   moe_stream less than one pair per expert on the mean (from there on
+//              mid_gemm.hip takes sizes of whole steps of 64 with columns for
+//              the chip; others are streamed up to 8): bound by the stream of
+//              the chosen experts' weights. Tiles of 16 weight rows (gate and
+//              up rows side by side), the waves of a workgroup splitting K, no
+//              LDS and no barrier before the final sum over the waves. 7 rows,
+//              8 of 128 experts each (2048 x 768): 90 us for 46 experts' 434 MB
 //              (4.8 TB/s); every expert as a batched product took 210 us.
-//   moe_engine more than 64 pairs per expert on the mean: bound by the matrix cores, and by the
-//              weights' one read while experts have few. Up to 256 pairs x 256
-//              weight rows per workgroup (tile_engine.h). 128 experts of 2048 x
-//              768, 8 per row, with plan and mix: 5012 rows 545 us (tiles of
-//              128: 742), 512 rows 251 us for 1.2 GB of weights (270); 8
-//              experts of 4096 x 14336, 2 per row, 8192 rows 4.5 ms (9.4).
-//   moe_tile   the same for sizes that are no multiple of 64: 128 pairs x 128
-//              weight rows, 64 of K per step through double-buffered LDS and
-//              registers, 560 TFLOP/s.
+//   moe_engine more than 64 pairs per expert on the mean: bound by the matrix
+//              cores, and by the weights' one read while experts have few. Up
+//              to 256 pairs x 256 weight rows per workgroup (tile_engine.h).
+//              128 experts of 2048 x 768, 8 per row, with plan and mix: 5012
+//              rows 545 us (tiles of 128: 742), 512 rows 251 us for 1.2 GB of
+//              weights (270); 8 experts of 4096 x 14336, 2 per row, 8192 rows
+//              4.5 ms (9.4).
+//   moe_tile   the same for sizes that are no multiple of 64, or leave the
+//              engine without work for the chip: 128 pairs x 128 weight rows, 64
+//              of K per step through double-buffered LDS and registers, 560
+//              TFLOP/s.
 //
 // Both products exist as "up" (rows gathered by pair, silu(gate) * up in fp32
 // before the one rounding) and "down". Weights lie as in checkpoints,
@@ -564,9 +567,10 @@ extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
 extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
                               const void* perm, const void* items,
                               const void* n_items, void* claims,
-                              int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out,
-                              int k_total, int top_k, int max_items, int tile,
-                              int up, hipStream_t stream) {
+                              int64_t a_stride, int64_t w_expert,
+                              int64_t w_stride, int n_out, int k_total,
+                              int top_k, int max_items, int tile, int up,
+                              hipStream_t stream) {
 #define ARKS_STREAM(NF, WV, UP)                                               \
   hipLaunchKernelGGL((moe_stream_kernel<NF, WV, UP>),                         \
                      dim3(n_out / (UP ? 16 : 16 * NF), max_items),            \

@@ -28,8 +28,6 @@
 //    that all but the newest n are there; stores in between only make it wait
 //    longer.
 #pragma once
-#include <type_traits>
-
 #include "common.h"
 
 namespace arks {
@@ -37,7 +35,7 @@ namespace arks {
 typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float tile_f32x4;
 
-constexpr int TILE_M = 256, TILE_HALF = 128, TILE_N = 256, TILE_K = 64;
+constexpr int TILE_M = 256, TILE_HALF = 128, TILE_K = 64;
 // full: 2 stages of 4 halves of 16 KB; half: 3 stages of 3
 constexpr int TILE_LDS = 3 * 3 * 16384;
 

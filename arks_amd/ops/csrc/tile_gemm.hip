@@ -2,11 +2,12 @@
 // rows, then the up rows: the product of tile_engine.h with a tile's two
 // halves of w as 128 gate rows and their up rows, so that the activation is
 // taken on the fp32 sums and neither product travels through memory. 18944 x
-// 3584: 8192 rows 1523 us (1461 TFLOP/s; a library product and the activation
-// behind it 1636), 3150 rows 623 us (1374 TFLOP/s; 812), 2048 rows 406 us
-// (433). One workgroup per CU goes from tile to tile, the next one's first
+// 3584: 8192 rows 1511 us (1473 TFLOP/s; a library product and the activation
+// behind it 1633), 3150 rows 612 us (1398 TFLOP/s; 798), 2048 rows 397 us
+// (420). One workgroup per CU goes from tile to tile, the next one's first
 // loads under way while the sums are stored: launched tile by tile 8192 rows
-// took 1548 us, 3150 rows (with the last 78 of them as a tile of 256) 655.
+// took 1.016 of the time, 3150 rows (with the last 78 of them as a tile of 256)
+// 1.05.
 #include "tile_engine.h"
 
 namespace arks {

@@ -2,9 +2,9 @@
 
 MI355X has no switch: 7 point-to-point xGMI links per GPU, so RCCL's ring
 all-reduce pays (world-1) serialized link hops — painful for the small
-per-token tensors of tensor-parallel decode, below ~1 MiB. OneShotAllReduce implements the classic
-small-message scheme (every rank pushes into every peer's mailbox, then
-reduces locally — see ops/csrc/allreduce.hip) with:
+per-token tensors of tensor-parallel decode, below ~1 MiB. OneShotAllReduce
+implements the classic small-message scheme (every rank pushes into every
+peer's mailbox, then reduces locally — see ops/csrc/allreduce.hip) with:
 
   * IPC-mapped mailboxes (hipIpcGetMemHandle/hipIpcOpenMemHandle,
     exchanged once over the existing torch.distributed group);

@@ -1458,7 +1458,7 @@ def test_mid_rule():
     assert ops._mid(x[:64], w.clone().requires_grad_()) is None
     for M in (1, 20, 100, 200, 256):
         parts = ops.linear_parts(x[:M], w)
-        assert parts.sums.shape[0] <= 16
+        assert isinstance(parts, ops.Parts) and 1 < parts.sums.shape[0] <= 8
         for out in (ops.parts_sum(parts), ops.linear_bf16(x[:M], w)):
             torch.testing.assert_close(
                 out.float(), torch.nn.functional.linear(x[:M], w).float(),
