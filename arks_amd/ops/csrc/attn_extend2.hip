@@ -643,14 +643,14 @@ __global__ __launch_bounds__(512, 2) void attn_extend2_kernel(
   }
 }
 
-// Merge the flash partials of split tiles: heads as in the kernel above x
-// (n_split, groups of 8 rows); combine_table rows = (first_y, nparts, seq, q0).
+// Merge the flash partials of split tiles: a workgroup has a head, a split tile
+// and 8 of its rows (LOCAL: heads as in the kernel above); combine_table rows = (first_y, nparts, seq, q0).
 // Standard flash merge in f32: m* = max m_p; out = sum_p exp(m_p - m*) O_p / sum_p
 // exp(m_p - m*) l_p (m is base-2: exp2). Reading the slabs bounds it, so the
 // loads of 2, 4 or 8 parts, as many as there are, are in flight together, two
 // dims a thread. Tiles of 3 parts, 28 heads, chunks of up to 2048 rows: 14.2 us
 // on the mean (90 MB at the most; with 8 loads for any number of parts 23.2).
-// A head's workgroups are on the XCD (or one of the XCDs) that wrote its slabs:
+// A head's workgroups are on the XCD that wrote its slabs, where one did:
 // read on another one, their next writing was slower too (32/8 heads, 256 rows
 // behind 5000 keys in 8 parts: 22.4 + 7.3 us with a window of 1024, now 19.8 +
 // 7.0; of 128, 19.6 + 7.2, now 15.4 + 7.1).
@@ -698,17 +698,19 @@ __device__ __forceinline__ void e2_combine_rows(
   }
 }
 
-template <int HEAD_DIM>
+template <int HEAD_DIM, bool LOCAL>
 __global__ __launch_bounds__(256) void attn_extend2_combine_kernel(
     bf16* __restrict__ out, const float* __restrict__ part_ws,
     const int* __restrict__ combine_table,
     const int* __restrict__ cu_seqlens_q, const float scale,
     const int num_q_heads, const int num_kv_heads, const int n_split) {
-  constexpr int GROUPS = E2_QTILE / 8;
-  const E2Place place = e2_place(num_q_heads, num_kv_heads);
-  const int h = place.h;
-  if (place.y >= n_split * GROUPS) return;
-  const int* entry = combine_table + place.y / GROUPS * 4;
+  int h = blockIdx.x, tile = blockIdx.y, group = blockIdx.z;
+  if constexpr (LOCAL) {
+    const E2Place place = e2_place(num_q_heads, num_kv_heads);
+    h = place.h, tile = place.y % n_split, group = place.y / n_split;
+    if (group >= E2_QTILE / 8) return;
+  }
+  const int* entry = combine_table + tile * 4;
   const int nparts = entry[1], seq_idx = entry[2], q0 = entry[3];
   const int q_start = cu_seqlens_q[seq_idx];
   const int q_len = cu_seqlens_q[seq_idx + 1] - q_start;
@@ -717,7 +719,7 @@ __global__ __launch_bounds__(256) void attn_extend2_combine_kernel(
                       (int64_t)h * E2_QTILE * (HEAD_DIM + 2);
   const int64_t out_stride = (int64_t)num_q_heads * HEAD_DIM;
   bf16* to = out + (q_start + q0) * out_stride + (int64_t)h * HEAD_DIM;
-  const int row0 = place.y % GROUPS * 8, rows = q_len - q0;
+  const int row0 = group * 8, rows = q_len - q0;
   const float scale2 = scale * E2_LOG2E;
 #define ARKS_ROWS(P)                                                         \
   e2_combine_rows<HEAD_DIM, P>(to, base, slab_stride, out_stride, row0, rows, \
@@ -776,13 +778,25 @@ extern "C" void arks_attn_extend2_combine(
     const void* cu_seqlens_q, int n_split, float scale, int num_q_heads,
     int num_kv_heads, int head_dim, hipStream_t stream) {
   if (n_split == 0) return;
-  const dim3 grid(e2_grid(num_q_heads, num_kv_heads, n_split * (E2_QTILE / 8)));
+  constexpr int GROUPS = E2_QTILE / 8;
+  // heads whose slabs one XCD wrote (where a group of them goes unevenly over
+  // XCDs, every other slab of a head is on another one, and launch order without
+  // the divisions is as fast: 28/4 heads, 2017 rows in 3 parts 15.3 us and 15.6)
+  const bool local =
+      num_kv_heads % 8 == 0 ||
+      (8 % num_kv_heads == 0 &&
+       num_q_heads / num_kv_heads % (8 / num_kv_heads) == 0);
+  const dim3 grid = local ? dim3(e2_grid(num_q_heads, num_kv_heads,
+                                         n_split * GROUPS))
+                          : dim3(num_q_heads, n_split, GROUPS);
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, (bf16*)out,
                        (const float*)part_ws, (const int*)combine_table,
                        (const int*)cu_seqlens_q, scale, num_q_heads,
                        num_kv_heads, n_split);
   };
-  if (head_dim == 128) launch(attn_extend2_combine_kernel<128>);
-  else if (head_dim == 64) launch(attn_extend2_combine_kernel<64>);
+  if (head_dim == 128 && local) launch(attn_extend2_combine_kernel<128, true>);
+  else if (head_dim == 128) launch(attn_extend2_combine_kernel<128, false>);
+  else if (head_dim == 64 && local) launch(attn_extend2_combine_kernel<64, true>);
+  else if (head_dim == 64) launch(attn_extend2_combine_kernel<64, false>);
 }
