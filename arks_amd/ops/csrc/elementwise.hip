@@ -187,19 +187,10 @@ extern "C" {
   hipLaunchKernelGGL((rmsnorm_kernel<FUSED, PARTS, NV>), dim3(rows),           \
                      dim3(PARTS ? 512 : 256), 0, stream, (bf16*)out, input,    \
                      (bf16*)residual, (const bf16*)weight, eps, hidden, splits)
-// Tensors that the XCDs' 32 MB of L2 hold beside the result are read twice for
-// nothing, and more rows fit a CU without the registers: 2048 x 4096 6.4 us, held
-// 7.2 (with the residual 9.7, 10.4), 1024 x 8192 6.5, 7.4; 4096 x 4096 12.8, held
-// 12.3, 8192 x 8192 55, 41; 512 x 4096 both 3.5.
-static bool norm_in_l2(int rows, int hidden) {
-  const int64_t all = (int64_t)rows * hidden;
-  return all >= 5000000 && all < 10500000;
-}
 #define ARKS_NORM_V(FUSED, PARTS)                                              \
   do {                                                                         \
     const int per = (hidden / 8 + (PARTS ? 511 : 255)) / (PARTS ? 512 : 256);  \
     if (per <= 1) ARKS_NORM(FUSED, PARTS, 1);                                  \
-    else if (!PARTS && norm_in_l2(rows, hidden)) ARKS_NORM(FUSED, PARTS, 0);   \
     else if (per <= 2) ARKS_NORM(FUSED, PARTS, 2);                             \
     else if (per <= 4) ARKS_NORM(FUSED, PARTS, 4);                             \
     else ARKS_NORM(FUSED, PARTS, 0);                                           \

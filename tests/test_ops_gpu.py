@@ -74,22 +74,6 @@ def test_norm_widths(rows, hidden, kind):
                                rtol=2 ** -7.9)
 
 
-@pytest.mark.parametrize("rows,hidden", [(1219, 4104), (1221, 4096), (2563, 4096),
-                                         (2564, 4096)])
-def test_norm_rows_either_side_of_l2(rows, hidden):
-    """Rows held in registers and read twice give the same bits as one by one."""
-    assert_native()
-    torch.manual_seed(rows)
-    x = torch.randn(rows, hidden, device=DEV).bfloat16()
-    res = torch.randn(rows, hidden, device=DEV).bfloat16()
-    w = torch.randn(hidden, device=DEV).bfloat16()
-    few = [0, 7, rows - 1]
-    assert torch.equal(ops.rmsnorm(x, w, 1e-6)[few], ops.rmsnorm(x[few], w, 1e-6))
-    want = ops.fused_add_rmsnorm(x[few], res[few], w, 1e-6)
-    got = ops.fused_add_rmsnorm(x, res, w, 1e-6)
-    assert all(torch.equal(a[few], b) for a, b in zip(got, want))
-
-
 def test_silu_mul():
     assert_native()
     torch.manual_seed(2)
