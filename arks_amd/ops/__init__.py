@@ -692,16 +692,20 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
     lines, us, here (other), sums with their consumer:
     - streamed: 5120 x 2048, 1 row 12.1 (10.2), 16 rows 13.4 (11.7); 3072 x
       2048, 16 rows 11 (10); 1152 x 896, 24 rows 8.5 (7.2), 64 rows 10 (8);
-      3584 x 3584, 8 rows 12.0 (11.4), 4096 x 4096 13.5 (12.2); with the
-      activation 16384 x 4096, 1 row 32.3 (27.6), 8 rows 32.0 (30.3), whose
-      tiles of 64 rows fill all CUs, 11008 x 4096 (2/3 of them) 0.85 of it;
+      3584 x 3584, 8 rows 12.0 (11.4), 4096 x 4096 13.5 (12.2); 7680 x 2560, 1
+      row 15 (14); with the activation 16384 x 4096, 1 row 32.3 (27.6), 8 rows
+      32.0 (30.3), whose tiles of 64 rows fill all CUs, 11008 x 4096 (2/3 of
+      them) 0.85 of it;
+    - few tiles with the activation: 8192 x 5120 (half of the CUs), 1 row 24
+      (18), 32 rows 29 (23), 6144 x 4096 (3/8) 20.5 (18), 6144 x 2048 0.72;
     - library, sums: 3584 x 3584, 256 rows 23.9 (22.2), 100 rows 15 (20); 2048
       x 4096, 200 rows 18.9 (17.2), 176 rows the same; 3072 x 2048, 250 rows 20
       (16); 1152 x 896, 192 rows 13.3 (12); without a consumer 8192 x 2048, 96
       rows 16.3 (14.5), 208 rows 24.0 (17.4), 64 rows 0.85 of it;
     - library, whole: 57344 x 8192, whose tiles fill the second round of CUs by
       3/4, 200 rows 247 (228); 50304 x 1024, 1 row 23.2 (21.0), 96 rows 28.7
-      (25.5), 50304 x 2048, 250 rows 69 (66), 128 rows 0.91 of it; 4096 x 4096,
+      (25.5), 50304 x 2048, 250 rows 69 (66), 128 rows 0.91 of it, 50304 x 2560
+      1.10 (64 rows 1.02); 9216 x 3072, 144 rows 28 (24), 72 rows 0.78; 4096 x 4096,
       200 rows 23.2 (21.9), 12288 x 4096, 240 rows 45 (40), 256 rows, as other
       multiples of 32, 0.93 of it; 64128 x 8192, 192 rows 247 (209), 128 rows
       0.86 of it, 32064 x 8192 0.91; gate and up 55296 x 5120, 0.84 full, 96
@@ -713,6 +717,7 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
     small = rows * K <= _SKINNY_MAX_ELEMS
     if small and (M * K <= 16384 and N <= 4096
                   or M * K <= 32768 and (K <= 2048 or 3072 <= N <= 4096)
+                  or M * K <= 24576 and K <= 3072
                   or M <= 64 and K <= 1024
                   if summed else _stream_sizes(M, rows, K, silu)):
         return None
@@ -723,12 +728,14 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
     if splits == 1:
         tiles = -(-N // ((16 if silu else 32) * qt))
         fill = tiles / (256 * -(-tiles // 256))
-        least = (0.35 if silu and M <= 64 else 0.55 if M <= 64
+        least = (0.35 if silu and M <= 64 and K < 4096
+                 else 0.6 if silu and M <= 64 else 0.55 if M <= 64
                  else 0.9 if M > 128 and N * K > 1 << 27
                  else 0.86 if silu and N * K > 1 << 27 else 0.6)
         if (fill < least or (M > 128 and K >= 8192 and tiles > 256)
                 or (tiles > 256 and fill < 0.8
-                    and (K <= 1024 or (K <= 2048 and M > 192)))
+                    and (K <= 1024 or (K <= 2048 and M > 192)
+                         or (2048 < K <= 3072 and M > 64)))
                 or (silu and qt == 2 and fill > 0.9
                     and M <= 8 and K <= 4096)):
             return None
@@ -737,7 +744,8 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
                 128 if K <= 1024 or (K <= 2048 and M % 32) else 192):
             return None
     elif (not (small or K >= 2 * N)
-          or (M > 64 and (K <= 2048 or N * K < 16_000_000))):
+          or (M > 64 and (K <= 2048 or N * K < 16_000_000))
+          or (M > 96 and K <= 3072)):
         return None
     return qt, splits
 

@@ -264,18 +264,20 @@ def test_mid_sizes_leave_what_others_do_faster():
         ((8, 4096, 4096), (16, 4096, 4096)), ((8, 3584, 3584), (16, 3584, 3584)),
         ((8, 4096, 4096), (8, 4608, 3584)), ((8, 4096, 4096), (8, 2048, 4096)),
         ((200, 2048, 4096), (192, 2048, 4096)), ((256, 3584, 3584), (256, 4608, 3584)),
-        ((176, 5120, 2048), (160, 5120, 2048)), ((250, 896, 896), (250, 896, 4864))]
+        ((8, 7680, 2560), (16, 7680, 2560)), ((176, 5120, 2048), (160, 5120, 2048)), ((250, 896, 896), (250, 896, 4864))]
     for left, taken in summed:
         assert not takes(*left, summed=True) and takes(*taken, summed=True)
     plain = [
         ((96, 8192, 2048), (64, 8192, 2048)), ((129, 64128, 8192), (128, 64128, 8192)),
         ((129, 64128, 8192), (129, 32064, 8192)), ((200, 4096, 4096), (192, 4096, 4096)),
         ((96, 50304, 1024), (96, 50304, 2048)), ((250, 50304, 2048), (192, 50304, 2048)),
+        ((96, 50304, 2560), (64, 50304, 2560)), ((144, 9216, 3072), (72, 9216, 3072)),
         ((240, 12288, 4096), (256, 12288, 4096)), ((240, 12288, 4096), (240, 24576, 4096))]
     for left, taken in plain:
         assert not takes(*left) and takes(*taken)
     gated = [  # N: gate columns
         ((8, 8192, 4096), (9, 8192, 4096)), ((8, 8192, 4096), (8, 5504, 4096)),
+        ((32, 4096, 5120), (32, 5120, 4096)), ((32, 3072, 4096), (64, 3072, 2048)),
         ((96, 27648, 5120), (64, 27648, 5120)), ((96, 27648, 5120), (96, 28672, 8192))]
     for left, taken in gated:
         assert not takes(*left, silu=True) and takes(*taken, silu=True)
