@@ -1,37 +1,52 @@
 // out[M, N] = a[M, K] . w[N, K]^T (+ bias), or silu(gate) * up of two such
 // products, for up to 256 rows: steps that decode, short prompts.
 //
-// A few rows are bound by the weights' stream, 200 by both it and the matrix
-// cores (200 rows x 37888 x 3584 are 45 us of weights and 39 us of matrix
-// operations; tile_engine.h is for those that the cores alone bound, and
-// stream_gemm.hip takes few rows of small weights, without sums for anyone to
-// add). So all rows of a meet a weight row at once (it is read once), the
-// weights' rows are cut as finely as gives every CU one tile of them (or, for
-// small products, one run of K: fp32 sums of the runs for the consumer to
-// add), and loads run NS - 1 steps of 64 columns ahead.
+// A few rows are bound by the weights' stream, 200 by it, the rows of a that
+// every workgroup reads beside it, and the matrix cores (200 rows x 37888 x 3584
+// are 40 us of weights at 6.8 TB/s and 39 us of matrix operations;
+// tile_engine.h is for those that the cores alone bound, and stream_gemm.hip
+// takes few rows of small weights, without sums for anyone to add). So all rows
+// of a meet a weight row at once (it is read once), and the weights' rows are
+// cut as finely as gives every CU one tile of them (or, for small products, one
+// run of K: fp32 sums of the runs for the consumer to add).
 //
-// 8 waves, 2 along the weights x 4 along the rows of a: a wave holds 16 * QT
-// weight rows x 16 * FT rows of a. The two groups of four take turns: in a slot
-// between two barriers one reads a whole step's operands from LDS (64 columns),
-// asks for the rows of step s + NS - 1 and waits, while the other multiplies the
-// step that it read in the slot before. Rows go from memory straight into LDS,
-// their 16-byte pieces permuted by the row's number (as in tile_engine.h, whose
-// rules for waits hold here too, a phase being such a step: what it read may be
-// overwritten from the next one on, and what it waited for may be read from the
-// next one on).
+// 4 waves multiply, one a SIMD, 2 along the weights x 2 along the rows of a: a
+// wave holds 16 * QT weight rows x 16 * FT rows of a. 4 more waves only load:
+// they go through the steps (64 columns) of all of the workgroup's jobs, NS
+// ahead, whatever the others do, so that the end of a job (its stores, which the
+// waits of a wave that also loads would count) does not hold up the stream. Rows
+// go from memory straight into LDS, their 16-byte pieces permuted by the row's
+// number (as in tile_engine.h). Rows of a are asked for in front of the weights:
+// hits in L2 behind misses come as late as those do (200 rows x 37888 x 3584
+// 61.8 -> 58.5 us), and 4 waves' loads are faster than 8 waves' (loads of 32 KB
+// of a and 24 KB of weights a step, nothing else: 58 and 70 us in 56 steps).
+//
+// One barrier a step. In front of the barrier of step s the waves that load wait
+// for their loads of step s + 1, and the others for their reads of step s:
+// behind it step s + 1 may be read and the stage of step s be loaded anew (with
+// step s + NS).
+//
+// us against the kernel before this one (8 waves that load and multiply in
+// turns), weights cold: 37888 x 3584 with the activation, 8 rows 43.4 -> 42.3,
+// 200 rows 63.5 -> 59.5; 3584 x 18944 in 8 runs of K, 64 rows 26.1 -> 25.3, 200
+// rows 41.2 -> 37.5; 4608 x 3584 in 4, 8 rows 12.7 -> 9.7, 64 rows 14.5 -> 13.1;
+// 152064 x 3584, 64 rows 201 -> 180, 208 rows 270 -> 251.
+#include <type_traits>
 #include "parts.h"
 #include "tile_engine.h"
 
 namespace arks {
 
+using u32x2 = __attribute__((ext_vector_type(2))) uint32_t;
+using u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
 constexpr int MID_LDS = 160 * 1024;
 
-// Stages of LDS: what fits, at most 5 (a workgroup's short run of K has not the
-// steps for more: 4608 x 3584, 64 rows, 8 stages 11.2 us, 5 10.6).
+// Stages of LDS: what fits, at most 6 (a workgroup's short run of K has not the
+// steps for more).
 constexpr int mid_stages(int qt, int ft) {
-  return MID_LDS / ((32 * qt + 64 * ft) * 128) < 5
-             ? MID_LDS / ((32 * qt + 64 * ft) * 128)
-             : 5;
+  return MID_LDS / ((32 * qt + 32 * ft) * 128) < 6
+             ? MID_LDS / ((32 * qt + 32 * ft) * 128)
+             : 6;
 }
 
 // Items of experts (moe_plan_kernel): {expert, first place, pairs, ..}; their
@@ -56,6 +71,37 @@ __device__ __forceinline__ void mid_load(const __amdgpu_buffer_rsrc_t& b,
       b, (__attribute__((address_space(3))) char*)to, 16, offset,
       s * (TILE_K * 2), 0, ONCE ? 2 : 0);
 }
+// Lanes of neighbouring rows swap x of the odd row against y of the even one:
+// a store then covers twice the columns of half the rows, whole lines.
+template <typename V>
+__device__ __forceinline__ void mid_swap(V& x, V& y, const bool odd) {
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(V) / 4); ++i) {
+    const uint32_t give = odd ? x[i] : y[i];
+    const uint32_t got = __builtin_amdgcn_mov_dpp(give, 0xB1, 0xF, 0xF, true);
+    if (odd) x[i] = got;
+    else y[i] = got;
+  }
+}
+
+// Where stores go that begin below 2 GiB of p; those beyond are dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mid_out(void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, 0x80000000, 0x00027000);
+}
+// once: past the caches (non-temporal)
+__device__ __forceinline__ void mid_store(const __amdgpu_buffer_rsrc_t& to,
+                                          const uint32_t offset, const u32x4& v,
+                                          const bool once) {
+  if (once) __builtin_amdgcn_raw_buffer_store_b128(v, to, offset, 0, 2);
+  else __builtin_amdgcn_raw_buffer_store_b128(v, to, offset, 0, 0);
+}
+__device__ __forceinline__ void mid_store(const __amdgpu_buffer_rsrc_t& to,
+                                          const uint32_t offset, const u32x2& v,
+                                          const bool once) {
+  if (once) __builtin_amdgcn_raw_buffer_store_b64(v, to, offset, 0, 2);
+  else __builtin_amdgcn_raw_buffer_store_b64(v, to, offset, 0, 0);
+}
+
 template <int N>
 __device__ __forceinline__ void mid_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -67,8 +113,9 @@ __device__ __forceinline__ void mid_barrier() {
 }
 
 // ITEMS: the experts that rows chose. Jobs are (item, tile), an item being up to
-// 64 * FT pairs of one expert, whose weights are so read once; workgroups go
-// through them in turn. With plan and mix, us, here (the best of moe_gemm.hip):
+// 32 * FT pairs of one expert, whose weights are so read once; workgroups go
+// through them in turn (64 rows of 128 experts of 2048 x 768, 8 per row: gate and
+// up 126 -> 123 us, down 71 -> 67 against the kernel before). With plan and mix, us, here (the best of moe_gemm.hip):
 // 128 experts of 2048 x 768, 8 per row: 16 rows 129 (133), 64 rows 197 (207),
 // 200 rows 211 (235), 600 rows 233 (250); 8 experts of 4096 x 14336, 2 per row:
 // 16 rows 425 (505), 200 rows 464 (591).
@@ -81,22 +128,16 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
     const int rotate, const MidItems of) {
   constexpr int NS = mid_stages(QT, FT);
   constexpr int W_ROWS = 32 * QT, COLS = SILU ? W_ROWS / 2 : W_ROWS;
-  constexpr int STAGE = (W_ROWS + 64 * FT) * 128;
-  constexpr int WL = (QT + 1) / 2;  // loads of weights a step, of waves 0 to 3
-  constexpr bool ODD = QT % 2 != 0;  // waves 4 to 7 take one less
-  static_assert(NS >= 3 && (NS - 2) * (WL + FT) < 64, "waits count to 63");
+  constexpr int W_STAGE = W_ROWS * 128, STAGE = W_STAGE + 32 * FT * 128;
+  constexpr int LOADS = QT + FT;  // of a step, of a wave that loads
+  static_assert(NS >= 3 && (NS - 1) * LOADS < 64, "waits count to 63");
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
   const int lane = threadIdx.x % WAVE_SIZE, lq = lane % 16, la = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
-  const int wm = wave / 4, wn = wave % 4;
   const int tiles = (n_total + COLS - 1) / COLS;
   const int jobs = tiles * (ITEMS ? *of.n_items : splits);
   const int all_steps = k_total / TILE_K;
   if (ITEMS && (int)blockIdx.x >= jobs) return;
-  // where operand k of a fragment lies: 16 rows of 128 B, pieces permuted
-  const int frag = lq * 128 + ((la ^ (lq & 7)) * 16);
-  const int w_at = wm * QT * 2048 + frag;
-  const int a_at = W_ROWS * 128 + wn * FT * 2048 + frag;
 
   // The column (of those of the tile) whose weight row stands at row `at` of a
   // wave's, so that a lane's sums are neighbours in the output: two fragments
@@ -109,7 +150,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
       return paired ? q / 2 * 16 + 4 * g + 2 * (q & 1) + r / 2
                     : 8 * q + 2 * g + r / 2;
     else
-      return paired ? q / 2 * 32 + 8 * g + 4 * (q & 1) + r : at;
+      return paired && !parts ? q / 2 * 32 + 8 * g + 4 * (q & 1) + r : at;
   };
 
   // turn: the step that a job begins with (then on to the last, and from the
@@ -138,185 +179,198 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
                rotate ? (int)((unsigned)j % (unsigned)steps) : 0,
                0, 0, m_rows};
   };
-  __amdgpu_buffer_rsrc_t wb, ab;
-  uint32_t wo[WL], ao[FT];
-  auto aim_rows = [&](const Job& b) {
+  if (wave >= 4) {
+    const int own = wave % 4;
+    __amdgpu_buffer_rsrc_t wb, ab;
+    uint32_t wo[QT], ao[FT];
+    auto aim = [&](const Job& b) {
+      wb = tile_buffer(w + (ITEMS ? b.expert * of.w_expert : 0) +
+                       (int64_t)b.n0 * k_total + b.s0 * TILE_K);
+      ab = tile_buffer(a + b.s0 * TILE_K +
+                       (ITEMS && !of.perm ? b.first * a_stride : 0));
 #pragma unroll
-    for (int j = 0; j < FT; ++j) {
-      const int row = (wave + 8 * j) * 8 + lane / 8;
-      uint32_t from = min(row, b.rows - 1);
-      if (ITEMS && of.perm) {
-        // the 8 rows' pairs are scalar loads: a vector load would be waited
-        // for behind all of those that are under way (what lies up to 7 places
-        // behind the last one is the plan's too, and not taken)
-        const int base = min((wave + 8 * j) * 8, b.rows - 1);
-        const int* at = of.perm + b.first + base;
-        int pair = at[0];
-#pragma unroll
-        for (int i = 1; i < 8; ++i)
-          pair = (int)from - base == i ? at[i] : pair;
-        from = (uint32_t)pair / (uint32_t)of.top_k;
+      for (int i = 0; i < QT; ++i) {
+        const int row = (own + 4 * i) * 8 + lane / 8;
+        const int side = row / (16 * QT), at = row % (16 * QT);
+        const int col = min(side * (COLS / 2) + column(at), n_total - 1 - b.n0);
+        wo[i] = (uint32_t)(col + (SILU && (at & 1) ? n_total : 0)) *
+                    (uint32_t)(k_total * 2) +
+                tile_piece_a(row, lane);
       }
-      ao[j] = from * (uint32_t)(a_stride * 2) + tile_piece_a(row, lane);
-    }
-  };
-  if (!ITEMS) aim_rows(job(blockIdx.x));
-  auto aim = [&](const Job& b) {  // the loads at a job
-    if (ITEMS) aim_rows(b);
-    ab = tile_buffer(a + b.s0 * TILE_K +
-                     (ITEMS && !of.perm ? b.first * a_stride : 0));
-    wb = tile_buffer(w + (ITEMS ? b.expert * of.w_expert : 0) +
-                     (int64_t)b.n0 * k_total + b.s0 * TILE_K);
 #pragma unroll
-    for (int j = 0; j < WL; ++j) {
-      const int row = (wave + 8 * j) * 8 + lane / 8;
-      const int half = row / (16 * QT), at = row % (16 * QT);
-      const int col =
-          min(half * (COLS / 2) + column(at), n_total - 1 - b.n0);
-      wo[j] = (uint32_t)(col + (SILU && (at & 1) ? n_total : 0)) *
-                  (uint32_t)(k_total * 2) +
-              tile_piece_a(row, lane);
-    }
-  };
-  auto column_step = [](const Job& b, const int s) {
-    return s + b.turn < b.steps ? s + b.turn : s + b.turn - b.steps;
-  };
-  auto load_w = [&](const int b, const int s) {
+      for (int i = 0; i < FT; ++i) {
+        const int row = (own + 4 * i) * 8 + lane / 8;
+        uint32_t r = min(row, b.rows - 1);
+        if (ITEMS && of.perm) {
+          // the 8 rows' pairs are scalar loads: a vector load would be waited
+          // for behind all of those that are under way (what lies up to 7 places
+          // behind the last one is the plan's too, and not taken)
+          const int base = min((own + 4 * i) * 8, b.rows - 1);
+          const int* at = of.perm + b.first + base;
+          int pair = at[0];
 #pragma unroll
-    for (int j = 0; j < WL; ++j)
-      if (!ODD || j + 1 < WL || wm == 0)
-        mid_load<true>(wb, lds + b * STAGE + (wave + 8 * j) * 1024, wo[j], s);
-  };
-  auto load_a = [&](const int b, const int s) {
-#pragma unroll
-    for (int j = 0; j < FT; ++j)
-      mid_load<false>(
-          ab, lds + b * STAGE + W_ROWS * 128 + (wave + 8 * j) * 1024, ao[j], s);
-  };
-  // the loads of the next step are there: those of NS - 2 steps may be under
-  // way behind them (`more`: so many were asked for)
-  auto arrived = [&](const bool more) {
-    if (!more) mid_wait<0>();
-    else if (!ODD || wm == 0) mid_wait<(NS - 2) * (WL + FT)>();
-    else mid_wait<(NS - 2) * (WL - 1 + FT)>();
-  };
-  auto prologue = [&](const Job& b) {
-#pragma unroll
-    for (int s = 0; s < NS - 1; ++s)
-      if (s < b.steps) {
-        load_w(s, column_step(b, s));
-        load_a(s, column_step(b, s));
+          for (int k = 1; k < 8; ++k) pair = (int)r - base == k ? at[k] : pair;
+          r = (uint32_t)pair / (uint32_t)of.top_k;
+        }
+        ao[i] = r * (uint32_t)(a_stride * 2) + tile_piece_a(row, lane);
       }
-  };
+    };
+    int total = 0;  // steps of all of this workgroup's jobs
+    if (ITEMS || splits == 1)
+      total = ((jobs - 1 - (int)blockIdx.x) / (int)gridDim.x + 1) * all_steps;
+    else
+      for (int j = blockIdx.x; j < jobs; j += gridDim.x) total += job(j).steps;
+    int j = blockIdx.x, s = 0, stage = 0;
+    Job b = job(j);
+    aim(b);
+    auto load = [&] {
+      const int at = s + b.turn < b.steps ? s + b.turn : s + b.turn - b.steps;
+      char* to = lds + stage * STAGE + own * 1024;
+#pragma unroll
+      for (int i = 0; i < FT; ++i)
+        mid_load<false>(ab, to + W_STAGE + i * 4096, ao[i], at);
+#pragma unroll
+      for (int i = 0; i < QT; ++i) mid_load<true>(wb, to + i * 4096, wo[i], at);
+      stage = stage == NS - 1 ? 0 : stage + 1;
+      if (++s == b.steps) {
+        s = 0;
+        j += gridDim.x;
+        if (j < jobs) {
+          b = job(j);
+          aim(b);
+        }
+      }
+    };
+    // the loads of all but the newest n steps are there
+    auto wait = [&](const int n) {
+      if (n >= NS - 1) mid_wait<(NS - 1) * LOADS>();
+      else if (n == 4) mid_wait<(NS > 5 ? 4 : 0) * LOADS>();
+      else if (n == 3) mid_wait<(NS > 4 ? 3 : 0) * LOADS>();
+      else if (n == 2) mid_wait<(NS > 3 ? 2 : 0) * LOADS>();
+      else if (n == 1) mid_wait<LOADS>();
+      else mid_wait<0>();
+    };
+    const int first = min(NS, total);
+    for (int t = 0; t < first; ++t) load();
+    wait(first - 1);
+    mid_barrier();
+    int t = 0;
+    for (; t + NS < total; ++t) {
+      mid_wait<(NS - 2) * LOADS>();
+      mid_barrier();
+      load();
+    }
+    for (; t < total; ++t) {
+      wait(max(0, total - 2 - t));
+      mid_barrier();
+    }
+    return;
+  }
 
+  const int wm = wave / 2, wn = wave % 2;
+  // where operand k of a fragment lies: 16 rows of 128 B, pieces permuted
+  const int frag = lq * 128 + ((la ^ (lq & 7)) * 16);
+  const int w_at = wm * QT * 2048 + frag;
+  const int a_at = W_STAGE + wn * FT * 2048 + frag;
   // Up to 64 rows a chain of sums is 4 steps long, and those of 4 steps are added
   // up apart: the streamed products, which are the other choice there, add up
   // the shorter chains of several waves. 64 rows of 4608 x 3584 in 3 runs of K
   // err by 1.0e-7, in a chain per run by 2.0e-7 (streamed, 7 runs: 1.4e-7); it
   // takes 1.4 % longer over 60 sizes, in front of the multiplications (2.2 %
   // behind them). Library products, the other choice beyond, are one chain too.
-  constexpr bool SETTLE = FT == 1;
-  f32x4 acc[QT][FT], settled[SETTLE ? QT : 1];
-  ushort8 wf[QT][2], af[FT][2];
-  auto read = [&](const int b) {
+  constexpr bool SETTLE = FT <= 2;
+  f32x4 acc[QT][FT], settled[SETTLE ? QT : 1][FT];
+  // The fragments of the next half step are read while this one's are
+  // multiplied: those of w and the last two of a into a second set of
+  // registers, the others into the same once they have been used.
+  constexpr int TWO = FT < 2 ? FT : 2;
+  ushort8 wf[2][QT], af[FT], al[2][TWO];
+  int at = 0;  // the stage that is read
+  auto read_w = [&](const int half, const int q) {
+    wf[half][q] = *reinterpret_cast<const ushort8*>(
+        lds + (at * STAGE + (w_at ^ (half * 64)) + q * 2048));
+  };
+  auto read_a = [&](const int half, const int f) {
+    const ushort8 v = *reinterpret_cast<const ushort8*>(
+        lds + (at * STAGE + (a_at ^ (half * 64)) + f * 2048));
+    if (f >= FT - TWO) al[half][f - (FT - TWO)] = v;
+    else af[f] = v;
+  };
+  auto half_step = [&](auto which) {
+    constexpr int H = decltype(which)::value;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int q = 0; q < QT; ++q) read_w(H ^ 1, q);
+#pragma unroll
+    for (int f = FT - TWO; f < FT; ++f) read_a(H ^ 1, f);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < FT; ++f) {
 #pragma unroll
       for (int q = 0; q < QT; ++q)
-        wf[q][k] = *reinterpret_cast<const ushort8*>(
-            lds + (b * STAGE + (w_at ^ (k * 64)) + q * 2048));
-#pragma unroll
-      for (int f = 0; f < FT; ++f)
-        af[f][k] = *reinterpret_cast<const ushort8*>(
-            lds + (b * STAGE + (a_at ^ (k * 64)) + f * 2048));
-    }
-  };
-  auto mul = [&](const int s) {
-    if constexpr (SETTLE) {
-      if ((s & 3) == 0) {
-#pragma unroll
-        for (int q = 0; q < QT; ++q) {
-          settled[q] += acc[q][0];
-          acc[q][0] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+        acc[q][f] = tile_mfma(
+            wf[H][q], f >= FT - TWO ? al[H][f - (FT - TWO)] : af[f], acc[q][f]);
+      if (f < FT - TWO) {
+        __builtin_amdgcn_sched_barrier(0);
+        read_a(H ^ 1, f);
       }
     }
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-      for (int q = 0; q < QT; ++q)
-#pragma unroll
-        for (int f = 0; f < FT; ++f)
-          acc[q][f] = tile_mfma(wf[q][k], af[f][k], acc[q][f]);
-    __builtin_amdgcn_s_setprio(0);
-    mid_barrier();
-  };
-
-  int at = 0, to = NS - 1;  // the stages that are read and loaded
-  auto load = [&](const Job& b, const int s) {
-    load_w(to, column_step(b, s));
-    load_a(to, column_step(b, s));
-  };
-  auto end_read = [&](const bool more) {
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    arrived(more);
-    mid_barrier();
   };
-  auto next_stage = [&] {
-    at = at == NS - 1 ? 0 : at + 1;
-    to = to == NS - 1 ? 0 : to + 1;
-  };
-  // The last steps of a job load the next job's first ones, where every job
-  // has that many (16 rows x 151936 x 2048 in tiles of 64 134 -> 121 us).
-  const bool chained = all_steps / splits >= NS - 1;
   int j = blockIdx.x;  // grid <= jobs
   Job now = job(j);
-  aim(now);
-  prologue(now);
-  arrived(now.steps >= NS - 1);
   mid_barrier();
-  if (wm == 1) mid_barrier();  // the second group runs one slot behind
   for (;;) {
+#pragma unroll
+  for (int q = 0; q < QT; ++q) read_w(0, q);
+#pragma unroll
+  for (int f = 0; f < FT; ++f) read_a(0, f);
 #pragma unroll
     for (int q = 0; q < QT; ++q)
 #pragma unroll
-      for (int f = 0; f < FT; ++f) acc[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int f = 0; f < FT; ++f) {
+        acc[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (SETTLE) settled[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    for (int s = 0; s < now.steps; ++s) {
+      if constexpr (SETTLE) {
+        if ((s & 3) == 0) {
 #pragma unroll
-    for (int q = 0; q < (SETTLE ? QT : 1); ++q)
-      settled[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int whole = max(0, now.steps - (NS - 1));
-    for (int s = 0; s < whole; ++s) {
-      read(at);
-      load(now, s + NS - 1);  // into the stage that the last step read
-      end_read(true);
-      mul(s);
-      next_stage();
+          for (int q = 0; q < QT; ++q)
+#pragma unroll
+            for (int f = 0; f < FT; ++f) {
+              settled[q][f] += acc[q][f];
+              acc[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+      }
+      half_step(std::integral_constant<int, 0>{});
+      // this step has been read, the next one is there
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      mid_barrier();
+      at = at == NS - 1 ? 0 : at + 1;
+      half_step(std::integral_constant<int, 1>{});
     }
     j += gridDim.x;
-    const bool more = j < jobs, ahead = more && chained;
-    const Job next = more ? job(j) : now;
-    if (ahead) aim(next);
-    for (int s = whole; s < now.steps; ++s) {
-      read(at);
-      if (ahead) load(next, s - whole);
-      end_read(ahead);
-      mul(s);
-      next_stage();
-    }
+    const bool more = j < jobs;
     if constexpr (SETTLE) {
 #pragma unroll
-      for (int q = 0; q < QT; ++q) acc[q][0] += settled[q];
+      for (int q = 0; q < QT; ++q)
+#pragma unroll
+        for (int f = 0; f < FT; ++f) acc[q][f] += settled[q][f];
     }
     const int n0 = now.n0 + wm * (COLS / 2);
 #pragma unroll
     for (int f = 0; f < FT; ++f) {
-      const int m = (wn * FT + f) * 16 + lq;
-      if (m >= now.rows) continue;
-      const int64_t row = (int64_t)(now.first + m) * n_total;
+      const int m0 = (wn * FT + f) * 16;
+      if (m0 >= now.rows) break;
+      // (worked out anew for each f, or they would fill the registers)
+      int lq = lane % 16, la = lane / 16;
+      asm volatile("" : "+v"(lq), "+v"(la));
+      const bool odd = lq & 1;
+      const int64_t row0 = (int64_t)(now.first + m0) * n_total + n0;
       if constexpr (SILU) {
-        bf16* to_row = reinterpret_cast<bf16*>(out) + row;
+        if (m0 + lq >= now.rows) continue;
+        bf16* to_row = reinterpret_cast<bf16*>(out) + row0 + lq * n_total - n0;
 #pragma unroll
         for (int q = 0; q < QT; q += 2) {
           bf16 o[4];
@@ -335,50 +389,82 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
               *reinterpret_cast<ushort2v*>(to_row + n) = ushort2v{o[0], o[1]};
           }
         }
-      } else if (parts) {
-        float* to_row = reinterpret_cast<float*>(out) +
-                        (int64_t)now.split * m_rows * n_total + row;
-#pragma unroll
-        for (int q = 0; q < QT; ++q) {
-          const int n = (q | 1) < QT ? n0 + q / 2 * 32 + 8 * la + 4 * (q & 1)
-                                     : n0 + q * 16 + 4 * la;
-          if (n < n_total) *reinterpret_cast<f32x4*>(to_row + n) = acc[q][f];
-        }
       } else {
-        bf16* to_row = reinterpret_cast<bf16*>(out) + row;
+        // Pieces of 16 bytes, of two rows at a time: stores that begin at `none`
+        // are not made. n_total % 8 == 0.
+        constexpr uint32_t none = 1u << 31;
+        // Past the caches beside the loads of other jobs, from 17 rows on: the
+        // output's lines do not push out those of a (152064 x 3584, 64 rows 197
+        // -> 178 us, 32 rows 179 -> 171; 8 rows 163 -> 166). Not sums: whoever
+        // adds them would read them from memory (64 rows x 3584 and their norm
+        // 5.0 -> 5.4 us, 200 rows 7.4 -> 8.5).
+        const bool once = jobs > (int)gridDim.x && now.rows > 16;
+        const uint32_t size = parts ? 4 : 2;
+        const uint32_t even = m0 + (lq & ~1) < now.rows
+                                  ? (lq & ~1) * n_total * size : none;
+        const uint32_t odds = m0 + (lq | 1) < now.rows
+                                  ? (lq | 1) * n_total * size : none;
+        const uint32_t own = odd ? odds : even;
+        auto at = [&](const uint32_t row, const int n) {
+          return n0 + n < n_total && row != none ? row + n * size : none;
+        };
+        if (parts) {
+          const auto to = mid_out(reinterpret_cast<float*>(out) +
+                                  (int64_t)now.split * m_rows * n_total + row0);
 #pragma unroll
-        for (int q = 0; q < QT; q += 2) {
-          const int width = q + 1 < QT ? 8 : 4;
-          const int n = n0 + q * 16 + width * la;
-          if (n >= n_total) continue;  // n_total % 8 == 0
-          bf16 o[8];
+          for (int q = 0; q + 1 < QT; q += 2) {
+            u32x4 x = *reinterpret_cast<const u32x4*>(&acc[q][f]);
+            u32x4 y = *reinterpret_cast<const u32x4*>(&acc[q + 1][f]);
+            mid_swap(x, y, odd);
+            const int n = q * 16 + 4 * la + (odd ? 16 : 0);
+            mid_store(to, at(even, n), x, false);
+            mid_store(to, at(odds, n), y, false);
+          }
+          if constexpr (QT % 2)
+            mid_store(to, at(own, (QT - 1) * 16 + 4 * la),
+                      *reinterpret_cast<const u32x4*>(&acc[QT - 1][f]), false);
+        } else {
+          const auto to = mid_out(reinterpret_cast<bf16*>(out) + row0);
+          const bf16* add = bias;
+          asm volatile("" : "+s"(add));  // its values are not kept in registers
+          auto value = [&](const int q, const int n) {
+            const bf16* b = add + min(n0 + n, n_total - 8);
+            bf16 o[8];
 #pragma unroll
-          for (int x = 0; x < width; ++x)
-            o[x] = float_to_bf16_bits(
-                acc[q + x / 4][f][x % 4] +
-                (bias ? bf16_bits_to_float(bias[n + x]) : 0.f));
-          if (q + 1 < QT)
-            *reinterpret_cast<ushort8*>(to_row + n) =
-                *reinterpret_cast<const ushort8*>(o);
-          else
-            *reinterpret_cast<ushort4v*>(to_row + n) =
-                ushort4v{o[0], o[1], o[2], o[3]};
+            for (int x = 0; x < 8; ++x)
+              o[x] = float_to_bf16_bits(acc[q + x / 4][f][x % 4] +
+                                        (add ? bf16_bits_to_float(b[x]) : 0.f));
+            return *reinterpret_cast<const u32x4*>(o);
+          };
+#pragma unroll
+          for (int q = 0; q + 3 < QT; q += 4) {
+            const int n = q * 16 + 8 * la;
+            u32x4 x = value(q, n), y = value(q + 2, n + 32);
+            mid_swap(x, y, odd);
+            mid_store(to, at(even, n + (odd ? 32 : 0)), x, once);
+            mid_store(to, at(odds, n + (odd ? 32 : 0)), y, once);
+          }
+#pragma unroll
+          for (int q = QT / 4 * 4; q + 1 < QT; q += 2)
+            mid_store(to, at(own, q * 16 + 8 * la), value(q, q * 16 + 8 * la),
+                      once);
+          if constexpr (QT % 2) {
+            const int n = (QT - 1) * 16 + 4 * la;
+            bf16 o[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              o[x] = float_to_bf16_bits(
+                  acc[QT - 1][f][x] +
+                  (add ? bf16_bits_to_float(add[min(n0 + n, n_total - 4) + x])
+                       : 0.f));
+            mid_store(to, at(own, n), *reinterpret_cast<const u32x2*>(o), once);
+          }
         }
       }
     }
     if (!more) break;
-    now = next;
-    if (!ahead) {
-      if (wm == 0) mid_barrier();  // all reads are over
-      at = 0, to = NS - 1;
-      aim(now);
-      prologue(now);
-      arrived(now.steps >= NS - 1);
-      mid_barrier();
-      if (wm == 1) mid_barrier();
-    }
+    now = job(j);
   }
-  if (wm == 0) mid_barrier();
 }
 
 }  // namespace arks
@@ -410,10 +496,14 @@ extern "C" void arks_mid_gemm(void* out, const void* a, const void* w,
   } while (0)
 #define ARKS_MID_M(QT)                                                         \
   do {                                                                         \
-    if (m <= 64) ARKS_MID_S(QT, 1);                                            \
-    else if (m <= 128) ARKS_MID_S(QT, 2);                                      \
-    else if (m <= 192) ARKS_MID_S(QT, 3);                                      \
-    else ARKS_MID_S(QT, 4);                                                    \
+    if (m <= 32) ARKS_MID_S(QT, 1);                                            \
+    else if (m <= 64) ARKS_MID_S(QT, 2);                                       \
+    else if (m <= 96) ARKS_MID_S(QT, 3);                                      \
+    else if (m <= 128) ARKS_MID_S(QT, 4);                                      \
+    else if (m <= 160) ARKS_MID_S(QT, 5);                                      \
+    else if (m <= 192) ARKS_MID_S(QT, 6);                                      \
+    else if (m <= 224) ARKS_MID_S(QT, 7);                                      \
+    else ARKS_MID_S(QT, 8);                                                    \
   } while (0)
   if (qt == 2) ARKS_MID_M(2);
   else if (qt == 4) ARKS_MID_M(4);
@@ -442,9 +532,9 @@ extern "C" void arks_mid_items(void* out, const void* a, const void* w,
   hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, true>), dim3(grid),        \
                      dim3(512), 0, stream, out, (const bf16*)a,                \
                      (const bf16*)w, nullptr, 0, n, k, a_stride, 1, 0, 1, of)
-  if (ft == 1 && silu) ARKS_MID(4, 1, true);
-  else if (ft == 1) ARKS_MID(4, 1, false);
-  else if (silu) ARKS_MID(4, 2, true);
-  else ARKS_MID(4, 2, false);
+  if (ft == 1 && silu) ARKS_MID(4, 2, true);
+  else if (ft == 1) ARKS_MID(4, 2, false);
+  else if (silu) ARKS_MID(4, 4, true);
+  else ARKS_MID(4, 4, false);
 #undef ARKS_MID
 }

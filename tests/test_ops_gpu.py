@@ -1426,6 +1426,29 @@ def test_mid_gemm(M, N, K, qt, splits, kind):
             <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("M", [16, 17, 32, 33, 96, 97, 160, 161, 224, 225])
+@pytest.mark.parametrize("qt", [2, 4, 5])
+@pytest.mark.parametrize("N", [88, 42008])
+def test_mid_gemm_row_edges(M, qt, N):
+    """A group of 32 rows full, and one row more; one job a workgroup, and
+    several, whose results pass the caches by from 17 rows on: every column,
+    nothing behind the last row."""
+    assert_native()
+    torch.manual_seed(M + qt + N)
+    K = 128
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV)
+    buf = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._native().mid_gemm(buf[:M], x, w, b, qt, False)
+    assert (buf[M] == 7.0).all()
+    expect = x.double() @ w.double().t() + b.double()
+    # as in test_mid_gemm
+    slack = K * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert ((buf[:M].double() - expect).abs()
+            <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
+
+
 def test_mid_rule():
     """Which products of up to 256 rows take the tiles, and that the runs of K
     that are chosen fit."""
