@@ -631,31 +631,28 @@ def _splits(x, weight, bias=None) -> bool:
             and (N * K <= _SKINNY_MAX_ELEMS or K >= 2 * N))
 
 
-# us that a step of mid_gemm.hip (64 columns of 32 * qt weight rows) takes at up
-# to 64, 128, 192 and 256 rows, but for 0.155 qt: fits of what it measured
-_MID_STEP = (0.07, 0.13, 0.26, 0.32)
-
-
 def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool):
     """(qt, splits) of a mid_gemm: weight rows of a tile (32 * qt) and runs
-    of K that keep 256 CUs busy in the fewest steps, 1.5 us being lost at the
-    start of a round; the fp32 sums of the runs are written and read at 5 TB/s,
-    and added by a launch of their own unless the consumer does (summed). At
-    most 8 runs, as the consumer's time grows with them. us with the norm that
-    adds the sums, weights cold, chosen (others): 3584 x 18944, 64 rows, 4, 8
-    33.0 (4, 9 33.3; without the norm 29.3 and 27.5; 5, 9 35.1; 2, 4 35.3; 4, 6
-    36.8); 3584 x 3584, 100 rows, 2, 4 16.8 (2, 2 19.9; 4, 8 19.1); 37888 x
-    3584 with the activation, 64 rows, 5, 1 48.6 (4, 1 66.2)."""
-    steps, step = K // 64, _MID_STEP[(M + 63) // 64 - 1]
+    of K that finish first, by a fit of what 52 sizes took at 1 to 256 rows with
+    all of their cuts (the chosen ones are 0.7 % from the best on average): a
+    step of 64 columns takes what its loads and matrix operations do, or the
+    weights' stream where all CUs share it; the fp32 sums of the runs are written
+    and read at 5 TB/s, and added by a launch of their own unless the consumer
+    does (summed). At most 8 runs, as the consumer's time grows with them."""
+    steps, groups = K // 64, -(-M // 32)
     best = None
     for qt in (5, 4, 2):
         tiles = -(-N // ((16 if silu else 32) * qt))
-        most = 1 if silu or tiles >= 180 else min(8, steps)
+        most = 1 if silu or tiles > 256 else min(8, steps)
         for splits in range(1, most + 1):
-            us = -(-tiles * splits // 256) * (
-                1.5 + -(-steps // splits) * (step + 0.155 * qt))
+            rounds, last = divmod(tiles * splits, 256)
+            alone = 0.02 + 0.095 * qt + 0.06 * groups
+            run = -(-steps // splits)
+            us = rounds * (0.6 + run * max(alone, 0.15 * qt))
+            if last:
+                us += 0.6 + run * max(alone, 0.15 * qt * last / 256)
             if splits > 1:
-                us += splits * M * N * 1.6e-6 + (0.0 if summed else 4.0)
+                us += splits * (0.1 + M * N * 1.6e-6) + (0.0 if summed else 4.0)
             if best is None or us < best[0]:
                 best = (us, qt, splits)
     return best[1:]
@@ -690,71 +687,70 @@ def _mid(x, weight, bias=None, silu: bool = False, summed: bool = False):
 def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
     """_mid, by the sizes (N columns of the result). The others' side of the
     lines, us, here (other), sums with their consumer:
-    - streamed: 5120 x 2048, 1 row 12.1 (10.2), 16 rows 13.4 (11.7); 3072 x
-      2048, 16 rows 11 (10); 1152 x 896, 24 rows 8.5 (7.2), 64 rows 10 (8);
-      3584 x 3584, 8 rows 12.0 (11.4), 4096 x 4096 13.5 (12.2); 7680 x 2560, 1
-      row 15 (14); with the activation 16384 x 4096, 1 row 32.3 (27.6), 8 rows
-      32.0 (30.3), whose tiles of 64 rows fill all CUs, 11008 x 4096 (2/3 of
-      them) 0.85 of it;
-    - few tiles with the activation: 8192 x 5120 (half of the CUs), 1 row 24
-      (18), 32 rows 29 (23), 6144 x 4096 (3/8) 20.5 (18), 6144 x 2048 0.72;
-    - library, sums: 3584 x 3584, 256 rows 23.9 (22.2), 100 rows 15 (20); 2048
-      x 4096, 200 rows 18.9 (17.2), 176 rows the same; 3072 x 2048, 250 rows 20
-      (16); 1152 x 896, 192 rows 13.3 (12); without a consumer 8192 x 2048, 96
-      rows 16.3 (14.5), 208 rows 24.0 (17.4), 64 rows 0.85 of it;
-    - library, whole: 57344 x 8192, whose tiles fill the second round of CUs by
-      3/4, 200 rows 247 (228); 50304 x 1024, 1 row 23.2 (21.0), 96 rows 28.7
-      (25.5), 50304 x 2048, 250 rows 69 (66), 128 rows 0.91 of it, 50304 x 2560
-      1.10 (64 rows 1.02); 9216 x 3072, 144 rows 28 (24), 72 rows 0.78; 4096 x 4096,
-      200 rows 23.2 (21.9), 12288 x 4096, 240 rows 45 (40), 256 rows, as other
-      multiples of 32, 0.93 of it; 64128 x 8192, 192 rows 247 (209), 128 rows
-      0.86 of it, 32064 x 8192 0.91; gate and up 55296 x 5120, 0.84 full, 96
-      rows 128.6 (121.4), 57344 x 8192, 0.875 full, 0.87 of it."""
+    - streamed, which has no sums to add: 1536 x 1536, 1 row 7.9 (7.3); 4096 x
+      4096, 4 rows 11.7 (11.2); 3584 x 3584, 1 row the same, 8 rows 0.89 of it;
+      5120 x 2048, 8 rows 0.88; without a consumer 4096 x 4096, 8 rows 1.18, 32
+      rows 0.82, 8192 x 2048, 16 rows 1.11, 48 rows 0.71; with the activation
+      1920 x 1088 (60 tiles), 5 rows 6.0 (5.6), 4096 x 5120 (half of the CUs)
+      the same;
+    - library, sums: 4096 x 2048, 208 rows 1.13 of it; 3584 x 3584, 256 rows
+      1.05; 1152 x 896, 208 rows 1.07; without a consumer 8192 x 2048, 96 rows
+      1.07, 208 rows 1.29, 64 rows 0.85, 4096 x 4096, 208 rows 1.02, 2192 x 896
+      (35 tiles), 100 rows 9.4 (8.3); with the activation 2256 x 2048 (71 tiles),
+      250 rows 24.5 (19.4);
+    - library, whole: 50304 x 2560, whose tiles fill the second round of CUs by
+      a quarter, 96 rows 1.15, 64 rows 1.04; gate and up 55296 x 5120, 0.84 full,
+      96 rows 1.06, 57344 x 8192, 0.875 full, 0.86."""
     if (K % 64 or N % 8 or not 64 <= K < 1 << 22 or not 0 < N < 1 << 24
             or (silu and 2 * N * K >= 1 << 31)):
         return None
-    rows = 2 * N if silu else N
-    small = rows * K <= _SKINNY_MAX_ELEMS
-    if small and (M * K <= 16384 and N <= 4096
-                  or M * K <= 32768 and (K <= 2048 or 3072 <= N <= 4096)
-                  or M * K <= 24576 and K <= 3072
-                  or M <= 64 and K <= 1024
-                  if summed else _stream_sizes(M, rows, K, silu)):
-        return None
-    if (M > 192 and M % 32 and 2048 < K <= 4096 and N * K <= 1 << 26
-            and not silu and not summed):
-        return None
+    small = N * K <= _SKINNY_MAX_ELEMS
     qt, splits = _mid_cut(M, N, K, silu, summed)
-    if splits == 1:
-        tiles = -(-N // ((16 if silu else 32) * qt))
-        fill = tiles / (256 * -(-tiles // 256))
-        least = (0.35 if silu and M <= 64 and K < 4096
-                 else 0.6 if silu and M <= 64 else 0.55 if M <= 64
-                 else 0.9 if M > 128 and N * K > 1 << 27
-                 else 0.86 if silu and N * K > 1 << 27 else 0.6)
-        if (fill < least or (M > 128 and K >= 8192 and tiles > 256)
-                or (tiles > 256 and fill < 0.8
-                    and (K <= 1024 or (K <= 2048 and M > 192)
-                         or (2048 < K <= 3072 and M > 64)))
-                or (silu and qt == 2 and fill > 0.9
-                    and M <= 8 and K <= 4096)):
+    tiles = -(-N // ((16 if silu else 32) * qt))
+    fill = tiles * splits / (256 * -(-tiles * splits // 256))
+    if summed:
+        if small and (M * K <= 32768 and (
+                          1024 < K <= 2048 or (K <= 4096 and 3072 <= N <= 4096))
+                      or M * K <= 24576 and 1024 < K <= 3072
+                      or K <= 1024 and M <= (64 if N <= 8192 else 8)):
             return None
-    elif summed:
         if N * K < 13_000_000 and K <= 4096 and M > (
                 128 if K <= 1024 or (K <= 2048 and M % 32) else 192):
             return None
-    elif (not (small or K >= 2 * N)
-          or (M > 64 and (K <= 2048 or N * K < 16_000_000))
-          or (M > 96 and K <= 3072)):
-        return None
+    elif silu:
+        if (fill < 0.6 and K >= 4096 and M <= 64
+                or fill < 0.3 and (M <= 32 or M > 192)
+                or qt == 2 and fill > 0.9 and M <= 8 and K <= 4096
+                or N * K > 1 << 27 and fill < 0.86 and 64 < M <= 160
+                or N * K > 1 << 27 and fill < 0.9 and M > 128 and K >= 8192):
+            return None
+    else:
+        few = splits > 1 or fill <= 0.5
+        if (small and few and N <= 8192
+                and M <= (16 if K <= 256 and N > 2048 else 64)
+                and (K <= 1536 or M * K <= (65536 if N > 2048 else 32768))):
+            return None
+        if few and M > 64 and (
+                K <= 1024 or (M > 160 and N * K < 16_000_000)
+                or (N > 2048 and (K <= 2048 or N * K < 16_000_000))
+                or (splits > 1 and M > 96 and K <= 3072)):
+            return None
+        if M > 192 and M % 32 and 2048 < K <= 4096 and N * K <= 1 << 26:
+            return None
+        if splits == 1 and tiles > 256 and (
+                (fill < 0.8 and M > 64 and (
+                    K <= 1024 or (K <= 2048 and M > 192) or 2048 < K <= 3072))
+                or (M > 128 and K >= 8192)):
+            return None
     return qt, splits
 
 
-def _mid_gemm(x, weight, bias, cut, silu: bool = False):
-    """A product by mid_gemm: a tensor, or Parts where K is split."""
+def _mid_gemm(x, weight, bias, cut, silu: bool = False, summed: bool = False):
+    """A product by mid_gemm: a tensor, or Parts where K is split or the
+    consumer adds sums (summed; one run of K then reaches it in fp32 too)."""
     (qt, splits), M = cut, x.shape[0]
     N = weight.shape[0] // (2 if silu else 1)
-    if splits > 1:
+    if splits > 1 or summed:
         sums = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
         _native().mid_gemm(sums, _rows_16b(x), weight, None, qt, False)
         return Parts(sums, bias)
@@ -807,7 +803,7 @@ def linear_parts(x, weight, bias=None):
     """linear_bf16 for a consumer that takes Parts."""
     cut = _mid(x, weight, bias, summed=True)
     if cut is not None:
-        return _mid_gemm(x, weight, bias, cut)
+        return _mid_gemm(x, weight, bias, cut, summed=True)
     if (x.dim() == 2 and not _streams(x, weight, bias=bias)
             and _splits(x, weight, bias)):
         return Parts(_stream_parts(x, weight), bias)
