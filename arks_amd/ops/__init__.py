@@ -694,7 +694,7 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
       1920 x 1088 (60 tiles), 5 rows 6.0 (5.6), 4096 x 5120 (half of the CUs)
       the same;
     - library, sums: 4096 x 2048, 208 rows 1.13 of it; 3584 x 3584, 256 rows
-      1.05; 1152 x 896, 208 rows 1.07; without a consumer 8192 x 2048, 96 rows
+      1.05, 224 rows 22.3 (23.8); 1152 x 896, 208 rows 1.07; without a consumer 8192 x 2048, 96 rows
       1.07, 208 rows 1.29, 64 rows 0.85, 4096 x 4096, 208 rows 1.02, 2192 x 896
       (35 tiles), 100 rows 9.4 (8.3); with the activation 2256 x 2048 (71 tiles),
       250 rows 24.5 (19.4);
@@ -715,7 +715,8 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
                       or K <= 1024 and M <= (64 if N <= 8192 else 8)):
             return None
         if N * K < 13_000_000 and K <= 4096 and M > (
-                128 if K <= 1024 or (K <= 2048 and M % 32) else 192):
+                128 if K <= 1024 or (K <= 2048 and M % 32)
+                else 224 if min(N, K) >= 3072 else 192):
             return None
     elif silu:
         if (fill < 0.6 and K >= 4096 and M <= 64
