@@ -631,19 +631,21 @@ def _splits(x, weight, bias=None) -> bool:
             and (N * K <= _SKINNY_MAX_ELEMS or K >= 2 * N))
 
 
-def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool):
+def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool,
+             whole: bool = False):
     """(qt, splits) of a mid_gemm: weight rows of a tile (32 * qt) and runs
     of K that finish first, by a fit of what 52 sizes took at 1 to 256 rows with
     all of their cuts (the chosen ones are 0.7 % from the best on average): a
     step of 64 columns takes what its loads and matrix operations do, or the
     weights' stream where all CUs share it; the fp32 sums of the runs are written
     and read at 5 TB/s, and added by a launch of their own unless the consumer
-    does (summed). At most 8 runs, as the consumer's time grows with them."""
+    does (summed). At most 8 runs, as the consumer's time grows with them.
+    whole: one run."""
     steps, groups = K // 64, -(-M // 32)
     best = None
-    for qt in (5, 4, 2):
+    for qt in (4, 5, 2):
         tiles = -(-N // ((16 if silu else 32) * qt))
-        most = 1 if silu or tiles > 256 else min(8, steps)
+        most = 1 if silu or whole or tiles > 256 else min(8, steps)
         for splits in range(1, most + 1):
             rounds, last = divmod(tiles * splits, 256)
             alone = 0.02 + 0.095 * qt + 0.06 * groups
@@ -658,6 +660,20 @@ def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool):
     return best[1:]
 
 
+def _mid_takes(x, weight, bias=None) -> bool:
+    """Whether mid_gemm can take these tensors, at sizes that it has."""
+    return (_USE_SKINNY and x.is_cuda and x.dim() == 2
+            and 1 <= x.shape[0] <= 256
+            and x.dtype == weight.dtype == torch.bfloat16
+            and _plain(x, weight, bias)
+            and x.stride(0) < 1 << 22
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == x.dtype
+                                  and bias.shape == weight.shape[:1]
+                                  and bias.is_contiguous()))
+            and native_available())
+
+
 def _mid(x, weight, bias=None, silu: bool = False, summed: bool = False):
     """(qt, splits) if x weight^T (or silu(gate) * up of it) takes mid_gemm,
     else None. summed: the consumer adds the sums of splits. It takes up to 256
@@ -667,17 +683,7 @@ def _mid(x, weight, bias=None, silu: bool = False, summed: bool = False):
     (57.6), 128 rows 51.0 (71.2), 200 rows 65 (85); 152064 x 3584, 1 row 168
     (182), 64 rows 201 (209), 200 rows 284 (325); 3584 x 18944, 1 row 23.0 and
     0.3 of sums (27.4), 100 rows 30.3 and 3 (96.5)."""
-    if not (_USE_SKINNY and x.is_cuda and x.dim() == 2
-            and 1 <= x.shape[0] <= 256
-            and x.dtype == weight.dtype == torch.bfloat16):
-        return None
-    if not (_plain(x, weight, bias)
-            and x.stride(0) < 1 << 22
-            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
-            and (bias is None or (bias.dtype == x.dtype
-                                  and bias.shape == weight.shape[:1]
-                                  and bias.is_contiguous()))
-            and native_available()):
+    if not _mid_takes(x, weight, bias):
         return None
     N, K = weight.shape
     return _mid_sizes(x.shape[0], N // 2 if silu else N, K, silu, summed)
@@ -869,9 +875,33 @@ def linear_fixed(x, weight, bias=None):
     return F.linear(x, weight, bias)
 
 
+def _mid_f32_tile(M: int, N: int, K: int):
+    """qt of a whole mid_gemm with an fp32 result, or None where another product
+    takes x weight^T: weights above _SKINNY_MAX_ELEMS at up to 64 rows, whose sums
+    are short chains, of K from 2560 on: 32000 x 4096 errs by 1.15e-7 at any
+    number of rows, streamed by 1.9e-7 up to 4 rows and 1.15e-7 up to 16, a
+    library product by 3.9e-7 (K 2048 1.02e-7, streamed 0.97e-7). us, here
+    (streamed to 16 rows, then library): 32000 x 4096, 1 row 43.6 (49.5), 8 rows
+    43.1 (55.0), 32 rows 44.1 (60.1), 64 rows 46.0 (61.9); 128256 x 4096, 64
+    rows 188 (223); 50304 x 2560, whose tiles fill their rounds to 0.77, 16 rows
+    50.0 (67.8), 48 rows 58.0 (54.3)."""
+    if (M > 64 or N * K <= _SKINNY_MAX_ELEMS or K < 2560 or K % 64 or N % 8
+            or K >= 1 << 22 or N >= 1 << 24):
+        return None
+    qt, _ = _mid_cut(M, N, K, False, False, whole=True)
+    tiles = -(-N // (32 * qt))
+    if tiles < (0.6 if M <= 16 else 0.8) * 256 * -(-tiles // 256):
+        return None
+    return qt
+
+
 def linear_f32_rows(x, weight):
-    """x weight^T in fp32 (bf16 operands) where the streamed product takes it,
-    else None."""
+    """x weight^T in fp32 (bf16 operands) where the tiles of mid_gemm or the
+    streamed product take it, else None."""
+    if x.dim() == 2 and _mid_takes(x, weight):
+        qt = _mid_f32_tile(x.shape[0], *weight.shape)
+        if qt is not None:
+            return _mid_gemm(x, weight, None, (qt, 1), summed=True).sums[0]
     if x.dim() == 2 and _streams(x, weight):
         return _stream_gemm(x, weight, dtype=torch.float32)
     return None

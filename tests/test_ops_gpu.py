@@ -1331,6 +1331,25 @@ def test_stream_gemm(M, N, K, bias):
     assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs()).all()
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 64])
+@pytest.mark.parametrize("N", [13320, 32000])
+def test_linear_f32_tiles(M, N):
+    """fp32 results of large weights vs fp64, strided rows: short chains of sums,
+    no rounding of the result."""
+    assert_native()
+    torch.manual_seed(M + N)
+    K = 2560
+    x = torch.randn(M, 2 * K, dtype=torch.bfloat16, device=DEV)[:, :K]
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    assert ops._mid_f32_tile(M, N, K) and ops._mid_f32_tile(65, N, K) is None
+    out = ops.linear_f32_rows(x, w)
+    assert out.dtype == torch.float32 and out.shape == (M, N)
+    expect = x.double() @ w.double().t()
+    # 40 steps of 64: chains of at most 8 + 10 sums of 32, within 50 * 2^-24
+    slack = 50 * 2 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert ((out.double() - expect).abs() <= slack).all()
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 18944, 3584), (8, 40, 96), (16, 9216, 1024),
                                    (31, 100, 64), (7, 4096, 2048)])
 def test_linear_silu_mul(M, I, K):
