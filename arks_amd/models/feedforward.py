@@ -34,7 +34,9 @@ constants as constructor parameters:
   the step is three GEMMs with data-independent shapes: all gate|up
   projections, an activation whose factor is 0 for the experts a row does
   not use (so their columns are exactly 0), and ONE down GEMM over all
-  columns, which sums the chosen experts and the shared one. Above it the
+  columns, which sums the chosen experts and the shared one (up to 16 rows
+  without a shared expert ops.routed_experts gives the same, and reads the
+  chosen experts alone). Above it the
   (row, expert) pairs are sorted by expert as in GroupedMoE. Experts may also
   be chosen in groups, by scores with a correction per expert that the
   weights do not see, and a group ranked by its best or its two best;
@@ -254,6 +256,10 @@ class RoutedMoE(nn.Module):
         if T <= self.DENSE_TOKENS:
             _, _, scale = ops.moe_route_grouped(
                 z, k, self.groups, self.keep, matrix=True, **route)
+            if not sff and ops.routed_takes(h, self.w_gu, self.w_down, E, ff):
+                return ops.routed_experts(h, self.w_gu, self.w_down, scale,
+                                          self.weigh_input, self.act,
+                                          self.limit, self.alpha)
             gu = linear(h, self.w_gu)
             return linear(ops.moe_glu_scaled(
                 gu, scale, E, ff, sff, self.weigh_input, self.act, self.limit,

@@ -1942,6 +1942,51 @@ def moe_glu_scaled(gu, scale, experts, ff, shared_ff, scale_input=True,
                               act, limit, shared_limit, alpha, shared_scale)
 
 
+def routed_takes(h, w_gu, w_down, experts: int, ff: int) -> bool:
+    """Whether routed_experts has kernels for these rows and weights: up to 16
+    rows of bf16, no shared expert, sizes in whole chunks of K."""
+    T, W = h.shape
+    return (_USE_SKINNY and h.is_cuda and 1 <= T <= 16
+            and h.dtype == w_gu.dtype == w_down.dtype == torch.bfloat16
+            and experts <= 64 and ff % 256 == 0 and experts * ff % 1024 == 0
+            and W % 512 == 0 and experts * ff < 1 << 22
+            and 4 * ff * W < 1 << 32 and h.stride(0) < 1 << 22
+            and w_gu.shape == (2 * experts * ff, W)
+            and w_down.shape == (W, experts * ff)
+            and all(w.is_contiguous() and w.data_ptr() % 16 == 0
+                    for w in (w_gu, w_down))
+            and _plain(h, w_gu, w_down) and seq_native_available())
+
+
+def routed_chunk(rows: int, down: bool) -> int:
+    """Columns of K after which the 4 chains of sums of a routed product move on
+    together. Which rows take which follows the library's products, whose places
+    these took and whose sums they are, bit for bit: 114688 x 4096 and 4096 x
+    57344 at 1 to 16 rows."""
+    if rows in (1, 8):
+        return 1024 if down else 512
+    return 512 if down else 128
+
+
+def routed_experts(h, w_gu, w_down, scale, scale_input=True, act="swiglu",
+                   limit=0.0, alpha=1.0):
+    """The weighted sum of the experts that rows chose (scale [T, E] fp32: their
+    weights, 0 elsewhere), for what routed_takes takes: linear, moe_glu_scaled and
+    linear over all experts, without those that nobody chose. us, here (those
+    three), 16 experts of ff 3584 on 4096 columns, 4 per row, weights cold: 1 row
+    (4 of them chosen) 67 (244), 2 rows (8) 124 (287), 8 rows (11) 167 (245), 16
+    rows (all) 248 (308)."""
+    T, E = scale.shape
+    C = _native_seq()
+    x = _rows_16b(h)
+    a = torch.empty((T, w_down.shape[1]), dtype=h.dtype, device=h.device)
+    C.routed_up(a, x, w_gu, scale, routed_chunk(T, False), bool(scale_input),
+                act == "clamped", float(limit), float(alpha))
+    y = torch.empty((T, w_down.shape[0]), dtype=h.dtype, device=h.device)
+    C.routed_down(y, a, w_down, scale, routed_chunk(T, True))
+    return y
+
+
 # ----------------------------------------------------------------------
 # Sandwich-norm blocks, per-head output gate, capped logits, channel-decay
 # delta rule (same extension, same rule).

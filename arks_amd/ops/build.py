@@ -55,6 +55,7 @@ SEQ_SOURCES = [
     os.path.join(CSRC, "seq_window.hip"),
     os.path.join(CSRC, "seq_window_mfma.hip"),
     os.path.join(CSRC, "seq_moe.hip"),
+    os.path.join(CSRC, "seq_routed.hip"),
     os.path.join(CSRC, "seq_shared.hip"),
     os.path.join(CSRC, "seq_mamba2.hip"),
     os.path.join(CSRC, "seq_masked_mfma.hip"),

@@ -197,6 +197,15 @@ int arks_seq_diff_head_norm_gate(void* out, int64_t ldo, const void* a,
                                  const void* gate, int64_t ldg, float lam,
                                  float eps, float mult, int T, int H, int G,
                                  int V, int act_f32, hipStream_t stream);
+void arks_seq_routed_up(void* out, const void* x, int64_t x_stride,
+                        const void* w, const void* scale, int64_t scale_stride,
+                        int m, int k, int chunk, int experts, int ff,
+                        int scale_in, int clamped, float limit, float alpha,
+                        hipStream_t stream);
+void arks_seq_routed_down(void* out, const void* x, int64_t x_stride,
+                          const void* w, const void* scale,
+                          int64_t scale_stride, int m, int n, int chunk,
+                          int experts, int ff, hipStream_t stream);
 void arks_seq_moe_glu_scaled(void* out, const void* gu, int64_t ldg,
                              const void* scale, int64_t lds, int64_t T, int E,
                              int ff, int sff, int scale_in, int clamped,
@@ -1197,6 +1206,62 @@ void diff_head_norm_gate(Tensor out, Tensor a, Tensor gate, double lam,
   TORCH_CHECK(rc == 0, "value size beyond the kernel's limit (", V, ")");
 }
 
+// bf16 rows that start on 16 bytes
+void check_routed_rows(const Tensor& t, const char* name) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 && t.dim() == 2 &&
+                  t.stride(1) == 1 && t.stride(0) % 8 == 0 &&
+                  t.stride(0) < (1 << 22) &&
+                  reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+              name, " must be bf16 rows on the GPU that start on 16 bytes");
+}
+
+void check_routed(const Tensor& x, const Tensor& w, const Tensor& scale,
+                  const Tensor& out, int64_t chunk, int64_t ff) {
+  check_routed_rows(x, "rows");
+  check_routed_rows(w, "weights");
+  check_routed_rows(out, "out");
+  TORCH_CHECK(w.is_contiguous() && out.is_contiguous());
+  TORCH_CHECK(scale.is_cuda() && scale.scalar_type() == torch::kFloat32 &&
+              scale.dim() == 2 && scale.stride(1) == 1 &&
+              scale.size(0) == x.size(0));
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(M >= 1 && M <= 16 && out.size(0) == M && scale.size(1) >= 1 &&
+                  scale.size(1) <= 64 && w.size(1) == K && ff % 16 == 0 && ff > 0,
+              "at most 16 rows and 64 experts");
+  TORCH_CHECK((chunk == 128 || (chunk > 0 && chunk % 256 == 0)) &&
+                  K % chunk == 0 && K % 256 == 0 && K < (1 << 22),
+              "K must be whole chunks");
+}
+
+// Activated gate and up products of the experts that rows chose (scale [M, E]:
+// not 0), 0 for those that only others chose; what nobody chose stays as it was.
+void routed_up(Tensor out, Tensor x, Tensor w, Tensor scale, int64_t chunk,
+               bool scale_input, bool clamped, double limit, double alpha) {
+  const int64_t E = scale.size(1), ff = w.size(0) / (2 * E);
+  check_routed(x, w, scale, out, chunk, ff);
+  TORCH_CHECK(w.size(0) == E * 2 * ff && out.size(1) == E * ff &&
+              2 * ff * w.size(1) * 2 < (1ll << 32));
+  arks_seq_routed_up(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(),
+                     scale.data_ptr(), scale.stride(0), (int)x.size(0),
+                     (int)x.size(1), (int)chunk, (int)E, (int)ff,
+                     scale_input ? 1 : 0, clamped ? 1 : 0, (float)limit,
+                     (float)alpha, current_stream());
+}
+
+// x [M, E * ff] . w [N, E * ff]^T over the columns of the experts that rows chose.
+void routed_down(Tensor out, Tensor x, Tensor w, Tensor scale, int64_t chunk) {
+  const int64_t E = scale.size(1), ff = w.size(1) / E;
+  check_routed(x, w, scale, out, chunk, ff);
+  TORCH_CHECK(w.size(1) == E * ff && out.size(1) == w.size(0) &&
+                  w.size(0) % 16 == 0 && w.size(0) < (1 << 24) &&
+                  chunk % 256 == 0 && ff % (chunk / 4) == 0,
+              "an expert's columns must be whole quarters of chunks");
+  arks_seq_routed_down(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(),
+                       scale.data_ptr(), scale.stride(0), (int)x.size(0),
+                       (int)w.size(0), (int)chunk, (int)E, (int)ff,
+                       current_stream());
+}
+
 void moe_glu_scaled(Tensor out, Tensor gu, Tensor scale, int64_t experts,
                     int64_t ff, int64_t shared_ff, bool scale_input,
                     bool clamped, bool shared_scale, double limit,
@@ -1743,6 +1808,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("conv_qkv_cache", &conv_qkv_cache);
   m.def("diff_head_norm_gate", &diff_head_norm_gate);
   m.def("moe_glu_scaled", &moe_glu_scaled);
+  m.def("routed_up", &routed_up);
+  m.def("routed_down", &routed_down);
   m.def("attention_masked_mfma", &attention_masked_mfma,
         py::arg("out"), py::arg("q"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("block_tables"), py::arg("seq_lens"),

@@ -559,3 +559,55 @@ def test_lightning_chunks_off_16_bytes(D, V):
         res.append((o, st))
     for o, st in res[1:]:
         assert torch.equal(o, res[0][0]) and torch.equal(st, res[0][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2, 8, 9, 16])
+@pytest.mark.parametrize("E,top,ff,W", [(16, 4, 256, 512), (4, 1, 512, 1024),
+                                        (64, 2, 256, 1536), (12, 12, 1024, 512)])
+@pytest.mark.parametrize("act", ["product", "input", "clamped"])
+def test_routed_experts_read_the_chosen_alone(rows, E, top, ff, W, act):
+    """The chosen experts' weighted sum against float64, strided rows; the
+    weights of experts that nobody chose are NaN, and no weight at all gives
+    zeros. Projections, activation and result are each rounded to bf16, the
+    activation turning 2^-8 of the gate into up to 4 of its own."""
+    torch.manual_seed(rows + E)
+    dev = "cuda"
+    h = torch.randn(rows, 2 * W, device=dev).bfloat16()[:, :W]
+    w_gu = (torch.randn(2 * E * ff, W, device=dev) * W ** -0.5).bfloat16()
+    w_down = (torch.randn(W, E * ff, device=dev) * ff ** -0.5).bfloat16()
+    scale = torch.zeros(rows, E, device=dev)
+    ids = torch.randn(rows, E, device=dev).topk(top).indices
+    scale.scatter_(1, ids, torch.rand(rows, top, device=dev) + 0.1)
+    unused = (scale == 0).all(0)
+    w_gu.view(E, 2 * ff, W)[unused] = math.nan
+    w_down.view(W, E, ff)[:, unused] = math.nan
+    assert ops.routed_takes(h, w_gu, w_down, E, ff)
+    limit, alpha = 1.5, 1.7
+    out = ops.routed_experts(
+        h, w_gu, w_down, scale, act == "input",
+        "clamped" if act == "clamped" else "swiglu", limit, alpha).double()
+    expect = torch.zeros(rows, W, dtype=torch.float64, device=dev)
+    slack = torch.zeros_like(expect)
+    for e in range(E):
+        if unused[e]:
+            continue
+        t = (scale[:, e] != 0).nonzero()[:, 0]
+        s = scale[t, e].double()[:, None]
+        g, u = (h[t].double() @ w_gu.view(E, 2, ff, W)[e].double().flatten(0, 1).t()
+                ).split(ff, 1)
+        if act == "clamped":
+            g, u = g.clamp(max=limit), u.clamp(-limit, limit) + 1
+            a = s * g * torch.sigmoid(alpha * g) * u
+        elif act == "input":
+            a = torch.nn.functional.silu(s * g) * s * u
+        else:
+            a = torch.nn.functional.silu(g) * s * u
+        d = w_down.view(W, E, ff)[:, e].double()
+        expect[t] += a @ d.t()
+        near = a.abs() + s * (g.abs() + 1) * 2 ** -8  # where a factor is near 0
+        slack[t] += 6 * 2 ** -8 * near @ d.abs().t()
+    assert bool(((out - expect).abs() <= slack + 2 ** -8 * expect.abs()).all())
+    scale.zero_()
+    w_gu.nan_to_num_(0.5), w_down.nan_to_num_(0.5)
+    assert not ops.routed_experts(h, w_gu, w_down, scale).any()
