@@ -1129,6 +1129,42 @@ def _moe_way(rows: int, top_k: int, El: int, experts: int, H: int, I: int,
     return tile, False
 
 
+@functools.lru_cache(maxsize=4096)
+def _moe_few(rows: int, top_k: int, El: int, experts: int, H: int, I: int,
+             streamed: bool):
+    """Up to 32 rows: (weight rows a wave / 16 of the gate and up tiles, of the
+    down tiles) for items of 32 pairs in mid_gemm.hip, or None where the streamed
+    kernel is expected to take less (streamed: it is the other choice, else items
+    of 64 are). Counted are the tiles of the experts that so many rows touch if
+    they choose evenly, in rounds over 256 CUs, a step as in _mid_cut, 1.5 us a
+    round; the streamed kernel at 4 us and 5 TB/s. us with plan and mix, items of 32 as
+    cut here (streamed; items of 64): 128 experts of 2048 x 768, 8 per row: 1 row
+    23.2 (25.7; 30.7), 7 rows 86 (92; 93), 16 rows 142 (146; 146); 8 of 4096 x
+    14336, 2 per row: 1 row 132 (132; 164), 4 rows 285 (333; 303), 8 rows 381
+    (435; 383); 16 of 4096 x 2048, 2 per row: 1 row 34.6 (30.9; 49), 8 rows 106
+    (100; 112). Over 6 sizes at 1 to 32 rows this choice is 1.7 % from the best,
+    streaming 9.2 %."""
+    n = max(1, round(El * (1 - (1 - top_k / experts) ** rows)))
+    best = [4 + 6 * H * I * n / 5e6] if streamed else [math.inf]
+    best.append(None)
+    cost = {}
+    for up in (True, False):
+        N, K = (I, H) if up else (H, I)
+        for qt in (2, 4):
+            jobs = n * -(-N // ((16 if up else 32) * qt))
+            rounds, last = divmod(jobs, 256)
+            alone = 0.08 + 0.095 * qt
+            us = rounds * (1.5 + K // 64 * max(alone, 0.15 * qt))
+            if last:
+                us += 1.5 + K // 64 * max(alone, 0.15 * qt * last / 256)
+            cost[up, qt] = us
+    for cut in ((4, 4), (2, 4), (4, 2), (2, 2)):
+        us = cost[True, cut[0]] + cost[False, cut[1]]
+        if us < best[0]:
+            best = [us, cut]
+    return best[1]
+
+
 def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
                 experts: int | None = None):
     """sum_j weights[t, j] * expert(ids[t, j])(x[t]) over the silu-GLU experts
@@ -1142,10 +1178,15 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
         out = torch.empty((x.shape[0], H), dtype=x.dtype, device=x.device)
         x = _rows_16b(x)
         rows = x.shape[0]
-        _native().moe_experts(
-            out, x, w13, w2, weights, ids, expert_base,
-            *_moe_way(rows, k, El, experts or El, H, I,
-                      _moe_whole(x, H, I, rows * k)))
+        whole = _moe_whole(x, H, I, rows * k)
+        way = _moe_way(rows, k, El, experts or El, H, I, whole)
+        # experts of 2 MB and more: below, launches are what counts
+        if (rows <= 32 and whole and way in ((16, False), (64, True))
+                and H * I >= 1 << 19):
+            cut = _moe_few(rows, k, El, experts or El, H, I, way[0] == 16)
+            if cut is not None:
+                way = (32, True, *cut)
+        _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, *way)
         return out
     return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
 

@@ -95,7 +95,8 @@ void arks_mid_gemm(void* out, const void* a, const void* w, const void* bias,
 void arks_mid_items(void* out, const void* a, const void* w, const void* perm,
                     const void* items, const void* n_items, int64_t a_stride,
                     int64_t w_expert, int n, int k, int top_k, int expert_base,
-                    int max_items, int ft, int silu, hipStream_t stream);
+                    int max_items, int ft, int qt, int silu,
+                    hipStream_t stream);
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, void* claims, void* counts, const void* ids,
                    const void* weights, int pairs, int expert_base, int n_local,
@@ -749,11 +750,13 @@ void stage_rows(pybind11::list prompts, pybind11::list outputs,
 
 // The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
 // beyond this rank's El experts from expert_base on count as zero. tile: pairs
-// of a work item; mid: of 64 or 128 pairs in mid_gemm.hip, else in
-// moe_gemm.hip (16, 128 or 256).
+// of a work item; mid: of 32, 64 or 128 pairs in mid_gemm.hip (32: qt_up and
+// qt_down, weight rows a wave / 16, may be 2), else in moe_gemm.hip (16, 128 or
+// 256).
 void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
                  torch::Tensor w2, torch::Tensor weights, torch::Tensor ids,
-                 int64_t expert_base, int64_t tile, bool mid) {
+                 int64_t expert_base, int64_t tile, bool mid, int64_t qt_up,
+                 int64_t qt_down) {
   check_bf16_contig(out, "out");
   check_bf16_rowstrided(x, "x");
   check_bf16_contig(w13, "w13");
@@ -767,7 +770,9 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   TORCH_CHECK(w13.size(1) == 2 * I && w13.size(2) == H && w2.size(0) == El &&
                   w2.size(1) == H,
               "expert weights do not fit");
-  TORCH_CHECK(mid ? tile == 64 || tile == 128
+  for (const int64_t qt : {qt_up, qt_down})
+    TORCH_CHECK(qt == 4 || (qt == 2 && tile == 32 && mid), "4, or 2 in items of 32");
+  TORCH_CHECK(mid ? tile == 32 || tile == 64 || tile == 128
                   : tile == 16 || tile == 128 || tile == 256);
   TORCH_CHECK((H | I) % (mid ? 64 : tile == 16 ? 32 : tile == 128 ? 8 : 64) == 0 &&
                   El <= 1024 && k <= 16,
@@ -808,13 +813,13 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
                 (int)expert_base, (int)El, (int)tile, (int)max_items,
                 (int)groups, stream);
   if (mid) {
-    const int ft = (int)tile / 64;
+    const int ft = (int)tile / 32;
     arks_mid_items(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
                    n_items, x.stride(0), 2 * I * H, (int)I, (int)H, (int)k,
-                   (int)expert_base, (int)max_items, ft, 1, stream);
+                   (int)expert_base, (int)max_items, ft, (int)qt_up, 1, stream);
     arks_mid_items(y.data_ptr(), h.data_ptr(), w2.data_ptr(), nullptr, items,
                    n_items, I, H * I, (int)H, (int)I, (int)k,
-                   (int)expert_base, (int)max_items, ft, 0, stream);
+                   (int)expert_base, (int)max_items, ft, (int)qt_down, 0, stream);
   } else {
     arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
                   n_items, claims, x.stride(0), 2 * I * H, H, (int)I, (int)H,
@@ -875,7 +880,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_silu", &tile_silu);
   m.def("mid_gemm", &mid_gemm);
   m.def("stage_rows", &stage_rows);
-  m.def("moe_experts", &moe_experts);
+  m.def("moe_experts", &moe_experts, pybind11::arg("out"), pybind11::arg("x"),
+        pybind11::arg("w13"), pybind11::arg("w2"), pybind11::arg("weights"),
+        pybind11::arg("ids"), pybind11::arg("expert_base"),
+        pybind11::arg("tile"), pybind11::arg("mid"), pybind11::arg("qt_up") = 4,
+        pybind11::arg("qt_down") = 4);
   m.def("mfma_probe", &mfma_probe);
   m.def("mfma_probe32", &mfma_probe32);
   m.def("tr16_probe", &tr16_probe);

@@ -115,10 +115,11 @@ __device__ __forceinline__ void mid_barrier() {
 // ITEMS: the experts that rows chose. Jobs are (item, tile), an item being up to
 // 32 * FT pairs of one expert, whose weights are so read once; workgroups go
 // through them in turn (64 rows of 128 experts of 2048 x 768, 8 per row: gate and
-// up 126 -> 123 us, down 71 -> 67 against the kernel before). With plan and mix, us, here (the best of moe_gemm.hip):
-// 128 experts of 2048 x 768, 8 per row: 16 rows 129 (133), 64 rows 197 (207),
-// 200 rows 211 (235), 600 rows 233 (250); 8 experts of 4096 x 14336, 2 per row:
-// 16 rows 425 (505), 200 rows 464 (591).
+// up 126 -> 123 us, down 71 -> 67 against the kernel before). Items of 32 are for
+// up to 32 rows, where no expert has more pairs and a ring of half the rows goes
+// round faster; their tiles may be of 32 * 2 weight rows, to fill the last round
+// of tiles (with plan and mix, 128 experts of 2048 x 768, 8 per row: 7 rows 91.6
+// us streamed, 93.3 in items of 64, 90.6 of 32, 86.1 with gate and up cut so).
 template <int QT, int FT, bool SILU, bool ITEMS>
 __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
     void* __restrict__ out, const bf16* __restrict__ a,
@@ -513,28 +514,35 @@ extern "C" void arks_mid_gemm(void* out, const void* a, const void* w,
 #undef ARKS_MID
 }
 
-// out [places, n]: the items' pairs (at most 64 * ft each) times their experts'
-// weights, silu: [2n, k] each; n_items of the max_items items are there. k % 64
-// == 0, n % 8 == 0; an expert's weights and (perm) all rows of a under 4 GiB; 7 ints
-// behind the last of perm are there.
+// out [places, n]: the items' pairs (at most 32 * ft each, ft 1, 2 or 4) times
+// their experts' weights, silu: [2n, k] each; n_items of the max_items items are
+// there. qt: 16 * qt weight rows a wave, 4, or (ft 1) 2. k % 64 == 0, n % 8 == 0;
+// an expert's weights and (perm) all rows of a under 4 GiB; 7 ints behind the
+// last of perm are there.
 extern "C" void arks_mid_items(void* out, const void* a, const void* w,
                                const void* perm, const void* items,
                                const void* n_items, int64_t a_stride,
                                int64_t w_expert, int n, int k, int top_k,
-                               int expert_base, int max_items, int ft, int silu,
-                               hipStream_t stream) {
+                               int expert_base, int max_items, int ft, int qt,
+                               int silu, hipStream_t stream) {
   const MidItems of{(const int4*)items, (const int*)n_items, (const int*)perm,
                     w_expert, top_k, expert_base};
-  const int cols = silu ? 64 : 128;
+  const int cols = silu ? 16 * qt : 32 * qt;
   const int64_t jobs = (int64_t)((n + cols - 1) / cols) * max_items;
   const int grid = (int)(jobs < 256 ? jobs : 256);
 #define ARKS_MID(QT, FT, SILU)                                                 \
   hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, true>), dim3(grid),        \
                      dim3(512), 0, stream, out, (const bf16*)a,                \
                      (const bf16*)w, nullptr, 0, n, k, a_stride, 1, 0, 1, of)
-  if (ft == 1 && silu) ARKS_MID(4, 2, true);
-  else if (ft == 1) ARKS_MID(4, 2, false);
-  else if (silu) ARKS_MID(4, 4, true);
-  else ARKS_MID(4, 4, false);
+#define ARKS_MID_S(QT, FT)                                                     \
+  do {                                                                         \
+    if (silu) ARKS_MID(QT, FT, true);                                          \
+    else ARKS_MID(QT, FT, false);                                              \
+  } while (0)
+  if (ft == 1 && qt == 2) ARKS_MID_S(2, 1);
+  else if (ft == 1) ARKS_MID_S(4, 1);
+  else if (ft == 2) ARKS_MID_S(4, 2);
+  else ARKS_MID_S(4, 4);
+#undef ARKS_MID_S
 #undef ARKS_MID
 }

@@ -885,6 +885,41 @@ def test_moe_items(T, E, k, H, I, base, El, tile, skew):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("up,down", [(2, 2), (2, 4), (4, 2), (4, 4)])
+@pytest.mark.parametrize("T,E,k,H,I,base,El,skew", [
+    (1, 4, 2, 64, 64, 0, 4, False), (7, 128, 8, 256, 192, 0, 128, False),
+    (3, 8, 2, 64, 64, 6, 2, True),              # none of this rank's
+    (17, 64, 8, 1024, 704, 16, 16, False),      # another rank's pairs
+    # ends of items: one, one and a pair, two and a half
+    (32, 4, 2, 320, 576, 0, 4, True), (33, 4, 2, 384, 128, 0, 4, True),
+    (80, 4, 2, 128, 1088, 0, 4, True),
+    # more tiles than workgroups: of one step, and of more than there are stages
+    (32, 64, 8, 1088, 64, 0, 64, False), (32, 64, 8, 64, 1088, 0, 64, False),
+    (32, 64, 8, 576, 512, 0, 64, False),
+])
+def test_moe_items_of_32(T, E, k, H, I, base, El, skew, up, down):
+    """Items of 32 pairs, tiles of 64 and 128 weight rows, vs fp64."""
+    assert_native()
+    torch.manual_seed(T + E)
+    x = torch.randn(T, 2 * H, device=DEV).bfloat16()[:, :H]
+    w13 = (torch.randn(El, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(El, H, I, device=DEV) * I ** -0.5).bfloat16()
+    ids = torch.rand(T, E, device=DEV).topk(k).indices.int()
+    if skew:
+        ids = torch.arange(k, device=DEV, dtype=torch.int32).expand(T, k).contiguous()
+    w = torch.rand(T, k, device=DEV)
+    out = torch.empty(T, H, device=DEV, dtype=torch.bfloat16)
+    ops._native().moe_experts(out, x, w13, w2, w, ids, base, 32, True, up, down)
+    expect = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for e in range(El):
+        t, j = (ids == e + base).nonzero(as_tuple=True)
+        gu = x[t].double() @ w13[e].double().t()
+        h = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+        expect.index_add_(0, t, h @ w2[e].double().t() * w[t, j, None].double())
+    # as in test_moe_experts
+    assert (out.double() - expect).norm() <= 3 * 2 ** -8 * expect.norm()
+
+
 @pytest.mark.parametrize("rows", [1, 17, 64])
 @pytest.mark.parametrize("qt", [2, 4, 5])
 def test_mid_gemm_short_chains(rows, qt):

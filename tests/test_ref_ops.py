@@ -320,3 +320,18 @@ def test_moe_way():
         (128, False), (128, False), (256, False)]
     # no whole steps of 32: tiles of 128
     assert ops._moe_way(7, 4, 16, 16, 2056, 1416, False) == (128, False)
+
+
+def test_moe_few():
+    """Items of 32 pairs where their tiles fill the rounds, streamed else."""
+    from arks_amd import ops
+
+    assert ops._moe_few(7, 8, 128, 128, 2048, 768, True) == (2, 4)
+    assert ops._moe_few(1, 2, 8, 8, 4096, 14336, True) == (4, 2)
+    assert ops._moe_few(1, 2, 16, 16, 4096, 2048, True) is None
+    # never streamed where that is not the other choice
+    for rows in range(1, 33):
+        cut = ops._moe_few(rows, 2, 16, 16, 4096, 2048, False)
+        assert cut is None or set(cut) <= {2, 4}
+    # a rank's 16 of 128 experts: less than one of them per row
+    assert ops._moe_few(1, 8, 16, 128, 2048, 768, True) in (None, (2, 2))
