@@ -262,11 +262,16 @@ class MoEMLP(nn.Module):
     # need no host read of the routing at any size)
     DENSE_TOKENS = 256
 
-    def forward(self, x):
+    def forward(self, x, parts: bool = False):
+        """parts: the caller takes ops.Mixed too (one rank, no shared expert)."""
         from ..parallel.comm import tp_all_reduce
 
         weights, selected = ops.moe_route(x, self.gate, self.top_k,
                                           self.norm_topk)
+        if parts and self.shared is None and get_tp_world_size() == 1:
+            return ops.moe_experts_parts(
+                x, self.w_up, self.w_down, weights, selected, self.expert_base,
+                self.num_experts)
         out = ops.moe_experts(x, self.w_up, self.w_down, weights, selected,
                               self.expert_base, self.num_experts)
         out = tp_all_reduce(out)
@@ -291,7 +296,7 @@ class DecoderLayer(nn.Module):
 
     def forward(self, x, residual, batch: ForwardBatch, kv_cache,
                 parts: bool = False):
-        """parts: the caller takes ops.Parts too."""
+        """parts: the caller takes ops.Parts and ops.Mixed too."""
         if residual is None:
             residual = x
             x = self.input_layernorm(x)
@@ -306,7 +311,9 @@ class DecoderLayer(nn.Module):
         else:
             x = self.self_attn(x, batch, kv_cache)
         x, residual = self.post_attention_layernorm(x, residual)
-        if (parts and passable(self.mlp, MLP)
+        if parts and passable(self.mlp, MoEMLP):
+            return self.mlp(x, parts=True), residual
+        if (parts and not batch.is_prefill and passable(self.mlp, MLP)
                 and passable(self.mlp.down_proj, RowParallelLinear)):
             return self.mlp(x, parts=True), residual
         return self.mlp(x), residual
@@ -389,7 +396,7 @@ class LlamaFamilyForCausalLM(nn.Module):
         residual = None
         last = len(self.layers) - 1
         for i, layer in enumerate(self.layers):
-            parts = not batch.is_prefill and passable(layer, DecoderLayer)
+            parts = passable(layer, DecoderLayer)
             if parts and i < last:
                 after = self.layers[i + 1]
                 parts = (passable(after, DecoderLayer)

@@ -60,6 +60,11 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.T
 
 def fused_add_rmsnorm(x, residual, weight, eps: float = 1e-6):
     """In-place on GPU: residual += x (written to residual), out = norm(residual)."""
+    if isinstance(x, Mixed):
+        out = torch.empty_like(residual)
+        _native().fused_add_rmsnorm_mix(out, x.y, x.weights, x.rows, residual,
+                                        weight, eps)
+        return out, residual
     if isinstance(x, Parts):
         assert x.bias is None
         out = torch.empty_like(residual)
@@ -774,6 +779,14 @@ class Parts:
         self.sums, self.bias = sums, bias
 
 
+class Mixed:
+    """Experts' rows y [pairs, H] that are not mixed yet: row t of the result
+    is the sum over j of weights[t, j] * y[rows[t, j]]."""
+
+    def __init__(self, y, weights, rows):
+        self.y, self.weights, self.rows = y, weights, rows
+
+
 def _stream_parts(x, weight):
     """Split sums; as many splits as give every CU a workgroup of 128 weight
     rows (3584 x 3584, 64 rows, us without the sums: 4 splits 14.9, 8 11.4, 12
@@ -787,7 +800,10 @@ def _stream_parts(x, weight):
 
 
 def parts_sum(x):
-    """The bf16 tensor that x, a Parts or already a tensor, stands for."""
+    """The bf16 tensor that x, a Parts, a Mixed or already a tensor, stands
+    for."""
+    if isinstance(x, Mixed):
+        return moe_mix_rows(x.y, x.weights, x.rows)
     if not isinstance(x, Parts):
         return x
     out = torch.empty(x.sums.shape[1:], dtype=torch.bfloat16,
@@ -1171,24 +1187,45 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
     w13 [El, 2I, H] (gate rows, then up rows), w2 [El, H, I]; experts outside
     [expert_base, expert_base + El) contribute nothing (another rank's).
     experts: the number on all ranks (None: El)."""
-    El, H, I = w13.shape[0], w13.shape[2], w2.shape[2]
-    k = ids.shape[1]
-    if (x.is_cuda and x.dtype == torch.bfloat16 and H % 8 == 0
-            and I % 8 == 0 and El <= 1024 and k <= 16):
-        out = torch.empty((x.shape[0], H), dtype=x.dtype, device=x.device)
-        x = _rows_16b(x)
-        rows = x.shape[0]
-        whole = _moe_whole(x, H, I, rows * k)
-        way = _moe_way(rows, k, El, experts or El, H, I, whole)
-        # experts of 2 MB and more: below, launches are what counts
-        if (rows <= 32 and whole and way in ((16, False), (64, True))
-                and H * I >= 1 << 19):
-            cut = _moe_few(rows, k, El, experts or El, H, I, way[0] == 16)
-            if cut is not None:
-                way = (32, True, *cut)
+    if _moe_native(x, w13, w2, ids):
+        x, way = _moe_cut(x, w13, w2, ids, experts)
+        out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, *way)
         return out
     return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
+
+
+def moe_experts_parts(x, w13, w2, weights, ids, expert_base: int = 0,
+                      experts: int | None = None):
+    """moe_experts for a consumer that takes Mixed."""
+    if not (_moe_native(x, w13, w2, ids) and x.shape[0]):
+        return moe_experts(x, w13, w2, weights, ids, expert_base, experts)
+    x, way = _moe_cut(x, w13, w2, ids, experts)
+    return Mixed(*_native().moe_expert_rows(
+        x, w13, w2, weights, ids, expert_base, *(*way, 4, 4)[:4]))
+
+
+def _moe_native(x, w13, w2, ids) -> bool:
+    return (x.is_cuda and x.dtype == torch.bfloat16 and w13.shape[2] % 8 == 0
+            and w2.shape[2] % 8 == 0 and w13.shape[0] <= 1024
+            and ids.shape[1] <= 16)
+
+
+def _moe_cut(x, w13, w2, ids, experts):
+    """x with rows on 16 bytes, and (pairs of an item, whether mid_gemm.hip
+    takes them[, tiles of items of 32])."""
+    El, H, I = w13.shape[0], w13.shape[2], w2.shape[2]
+    rows, k = ids.shape
+    x = _rows_16b(x)
+    whole = _moe_whole(x, H, I, rows * k)
+    way = _moe_way(rows, k, El, experts or El, H, I, whole)
+    # experts of 2 MB and more: below, launches are what counts
+    if (rows <= 32 and whole and way in ((16, False), (64, True))
+            and H * I >= 1 << 19):
+        cut = _moe_few(rows, k, El, experts or El, H, I, way[0] == 16)
+        if cut is not None:
+            way = (32, True, *cut)
+    return x, way
 
 
 def moe_mix(y, weights, ids, expert_base: int = 0):

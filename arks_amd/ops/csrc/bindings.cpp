@@ -23,6 +23,11 @@ void arks_fused_add_rmsnorm(void* out, const void* input, void* residual,
 void arks_fused_add_rmsnorm_parts(void* out, const void* part, int splits,
                                   void* residual, const void* weight, float eps,
                                   int rows, int hidden, hipStream_t stream);
+void arks_fused_add_rmsnorm_mix(void* out, const void* input,
+                                const void* mix_weights, const void* mix_rows,
+                                int k, void* residual, const void* weight,
+                                float eps, int rows, int hidden,
+                                hipStream_t stream);
 void arks_rope_and_cache_parts(const void* positions, void* q, const void* part,
                                const void* bias, int splits, void* k_cache,
                                void* v_cache, const void* slot_mapping,
@@ -172,6 +177,35 @@ void fused_add_rmsnorm_parts(torch::Tensor out, torch::Tensor part,
                                (int)part.size(0), residual.data_ptr(),
                                weight.data_ptr(), (float)eps, (int)rows,
                                (int)hidden, current_stream());
+}
+
+// fused_add_rmsnorm of the mix (moe_mix_rows) of the rows y of experts
+void fused_add_rmsnorm_mix(torch::Tensor out, torch::Tensor y,
+                           torch::Tensor mix_weights, torch::Tensor mix_rows,
+                           torch::Tensor residual, torch::Tensor weight,
+                           double eps) {
+  check_bf16_contig(out, "out");
+  check_bf16_contig(y, "y");
+  check_bf16_contig(residual, "residual");
+  check_bf16_contig(weight, "weight");
+  check_rows_16b(y, "y");
+  TORCH_CHECK(y.dim() == 2 && mix_weights.dim() == 2 &&
+              mix_rows.sizes() == mix_weights.sizes() &&
+              mix_weights.is_cuda() && mix_rows.is_cuda() &&
+              mix_weights.scalar_type() == torch::kFloat32 &&
+              mix_rows.scalar_type() == torch::kInt32 &&
+              mix_weights.is_contiguous() && mix_rows.is_contiguous());
+  const int64_t hidden = y.size(1), rows = mix_weights.size(0);
+  const int64_t k = mix_weights.size(1);
+  TORCH_CHECK(hidden % 8 == 0 && out.numel() == rows * hidden &&
+              residual.numel() == rows * hidden && weight.numel() == hidden &&
+              k >= 1 && k <= 16 && (y.size(0) > 0 || rows == 0));
+  if (rows == 0) return;
+  arks_fused_add_rmsnorm_mix(out.data_ptr(), y.data_ptr(),
+                             mix_weights.data_ptr(), mix_rows.data_ptr(),
+                             (int)k, residual.data_ptr(), weight.data_ptr(),
+                             (float)eps, (int)rows, (int)hidden,
+                             current_stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor gate_up) {
@@ -748,16 +782,15 @@ void stage_rows(pybind11::list prompts, pybind11::list outputs,
   }
 }
 
-// The routed experts of x [T, H]: w13 [El, 2I, H], w2 [El, H, I], pairs
-// beyond this rank's El experts from expert_base on count as zero. tile: pairs
-// of a work item; mid: of 32, 64 or 128 pairs in mid_gemm.hip (32: qt_up and
-// qt_down, weight rows a wave / 16, may be 2), else in moe_gemm.hip (16, 128 or
-// 256).
-void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
-                 torch::Tensor w2, torch::Tensor weights, torch::Tensor ids,
-                 int64_t expert_base, int64_t tile, bool mid, int64_t qt_up,
-                 int64_t qt_down) {
-  check_bf16_contig(out, "out");
+// The experts' rows of x [T, H] and their mix: (y [T * k, H], weights and rows
+// [T, k]); w13 [El, 2I, H], w2 [El, H, I], pairs beyond this rank's El experts
+// from expert_base on weigh zero. tile: pairs of a work item; mid: of 32, 64 or
+// 128 pairs in mid_gemm.hip (32: qt_up and qt_down, weight rows a wave / 16, may
+// be 2), else in moe_gemm.hip (16, 128 or 256).
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
+    torch::Tensor x, torch::Tensor w13, torch::Tensor w2, torch::Tensor weights,
+    torch::Tensor ids, int64_t expert_base, int64_t tile, bool mid,
+    int64_t qt_up, int64_t qt_down) {
   check_bf16_rowstrided(x, "x");
   check_bf16_contig(w13, "w13");
   check_bf16_contig(w2, "w2");
@@ -766,7 +799,7 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
   check_rows_16b(w2, "w2");
   const int64_t T = x.size(0), H = x.size(1), El = w13.size(0);
   const int64_t I = w2.size(2), k = weights.size(1), P = T * k;
-  TORCH_CHECK(x.dim() == 2 && out.size(0) == T && out.size(1) == H);
+  TORCH_CHECK(x.dim() == 2);
   TORCH_CHECK(w13.size(1) == 2 * I && w13.size(2) == H && w2.size(0) == El &&
                   w2.size(1) == H,
               "expert weights do not fit");
@@ -788,7 +821,7 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
               weights.is_contiguous() && ids.scalar_type() == torch::kInt32 &&
               ids.is_contiguous() && ids.size(0) == T && ids.size(1) == k &&
               weights.size(0) == T);
-  if (T == 0) return;
+  if (T == 0) return {torch::empty({0, H}, x.options()), weights, ids};
   const int64_t max_items = std::min(P, El) + P / tile;
   TORCH_CHECK(max_items <= 65535 || tile != 16, "too many rows for this tile");
   auto ints = x.options().dtype(torch::kInt32);
@@ -828,8 +861,23 @@ void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
                   n_items, claims, I, H * I, I, (int)H, (int)I, (int)k,
                   (int)max_items, (int)tile, 0, stream);
   }
-  arks_moe_mix_rows(out.data_ptr(), y.data_ptr(), w_pair.data_ptr(), rows,
-                    (int)T, (int)H, (int)k, stream);
+  return {y, w_pair, plan.narrow(0, 4 * max_items + P, P).view({T, k})};
+}
+
+// The routed experts of x: the mix of moe_expert_rows
+void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
+                 torch::Tensor w2, torch::Tensor weights, torch::Tensor ids,
+                 int64_t expert_base, int64_t tile, bool mid, int64_t qt_up,
+                 int64_t qt_down) {
+  check_bf16_contig(out, "out");
+  TORCH_CHECK(x.dim() == 2 && out.size(0) == x.size(0) &&
+              out.size(1) == x.size(1));
+  const auto [y, w, rows] = moe_expert_rows(x, w13, w2, weights, ids,
+                                            expert_base, tile, mid, qt_up, qt_down);
+  if (x.size(0) == 0) return;
+  arks_moe_mix_rows(out.data_ptr(), y.data_ptr(), w.data_ptr(), rows.data_ptr(),
+                    (int)x.size(0), (int)x.size(1), (int)weights.size(1),
+                    current_stream());
 }
 
 void mfma_probe(torch::Tensor d, torch::Tensor a, torch::Tensor b) {
@@ -880,6 +928,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_silu", &tile_silu);
   m.def("mid_gemm", &mid_gemm);
   m.def("stage_rows", &stage_rows);
+  m.def("moe_expert_rows", &moe_expert_rows);
+  m.def("fused_add_rmsnorm_mix", &fused_add_rmsnorm_mix);
   m.def("moe_experts", &moe_experts, pybind11::arg("out"), pybind11::arg("x"),
         pybind11::arg("w13"), pybind11::arg("w2"), pybind11::arg("weights"),
         pybind11::arg("ids"), pybind11::arg("expert_base"),

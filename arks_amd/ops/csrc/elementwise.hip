@@ -11,21 +11,30 @@ namespace arks {
 // RMSNorm: one workgroup per row, of 4 waves (8 where it adds split sums: such
 // rows are few, and a row is one pass then).
 // hidden must be a multiple of 8 (bf16x8 vector loads).
-// PARTS: the input is the sum of fp32 splits [splits, rows, hidden] of the
+// IN_PARTS: the input is the sum of fp32 splits [splits, rows, hidden] of the
 // product before it; adding 8 of them here takes 0.5 us at 64 x 3584, a launch
 // of its own 5.
+// IN_MIX: the input is the mix of the experts' rows that a token chose, rounded
+// as moe_mix_rows stores it (behind 4 layers of 128 experts, 8 per row, one
+// step of 64 rows 1289 -> 1282 us, of 7 rows 724 -> 719, a prompt pass 3810 ->
+// 3792: a launch and, for many rows, one write and read of the mix less).
 // NV: vectors of a thread that stay in registers, with the weights loaded
 // beside them: few rows are bound by the chain of loads, sum and store, many
 // by the bytes. Rows that are longer (NV 0) are read again from L2 behind the
 // sum, as all were before: 64 x 3584 and 4 splits 5.3 us, held 4.9.
 // ---------------------------------------------------------------------------
-template <bool FUSED_ADD, bool PARTS, int NV>
+enum NormInput { IN_ROWS, IN_PARTS, IN_MIX };
+template <bool FUSED_ADD, NormInput IN, int NV>
 __global__ void rmsnorm_kernel(bf16* __restrict__ out,
                                const void* __restrict__ input,
                                bf16* __restrict__ residual,  // null unless FUSED_ADD
                                const bf16* __restrict__ weight,
                                const float eps, const int hidden,
-                               const int splits) {
+                               const int splits,
+                               const float* __restrict__ mix_weights,  // [rows, k]
+                               const int* __restrict__ mix_rows,       // [rows, k]
+                               const int mix_k) {
+  constexpr bool PARTS = IN == IN_PARTS;
   constexpr int BLOCK = PARTS ? 512 : 256;
   const int row = blockIdx.x;
   const bf16* in_row =
@@ -50,7 +59,12 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = j < 4 ? lo[j % 4] : hi[j % 4];
     } else {
-      s = *reinterpret_cast<const ushort8*>(in_row + i * 8);
+      if constexpr (IN == IN_MIX)
+        s = mix_rows8(reinterpret_cast<const bf16*>(input),
+                      mix_weights + (int64_t)row * mix_k,
+                      mix_rows + (int64_t)row * mix_k, mix_k, hidden, i * 8);
+      else
+        s = *reinterpret_cast<const ushort8*>(in_row + i * 8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = bf16_bits_to_float(s[j]);
     }
@@ -183,37 +197,54 @@ using namespace arks;
 
 extern "C" {
 
-#define ARKS_NORM(FUSED, PARTS, NV)                                            \
-  hipLaunchKernelGGL((rmsnorm_kernel<FUSED, PARTS, NV>), dim3(rows),           \
-                     dim3(PARTS ? 512 : 256), 0, stream, (bf16*)out, input,    \
-                     (bf16*)residual, (const bf16*)weight, eps, hidden, splits)
-#define ARKS_NORM_V(FUSED, PARTS)                                              \
+#define ARKS_NORM(FUSED, IN, NV)                                               \
+  hipLaunchKernelGGL((rmsnorm_kernel<FUSED, IN, NV>), dim3(rows),              \
+                     dim3(IN == IN_PARTS ? 512 : 256), 0, stream, (bf16*)out,  \
+                     input, (bf16*)residual, (const bf16*)weight, eps, hidden, \
+                     splits, (const float*)mix_weights, (const int*)mix_rows, k)
+#define ARKS_NORM_V(FUSED, IN)                                                 \
   do {                                                                         \
-    const int per = (hidden / 8 + (PARTS ? 511 : 255)) / (PARTS ? 512 : 256);  \
-    if (per <= 1) ARKS_NORM(FUSED, PARTS, 1);                                  \
-    else if (per <= 2) ARKS_NORM(FUSED, PARTS, 2);                             \
-    else if (per <= 4) ARKS_NORM(FUSED, PARTS, 4);                             \
-    else ARKS_NORM(FUSED, PARTS, 0);                                           \
+    const int block = IN == IN_PARTS ? 512 : 256;                              \
+    const int per = (hidden / 8 + block - 1) / block;                          \
+    if (per <= 1) ARKS_NORM(FUSED, IN, 1);                                     \
+    else if (per <= 2) ARKS_NORM(FUSED, IN, 2);                                \
+    else if (per <= 4) ARKS_NORM(FUSED, IN, 4);                                \
+    else ARKS_NORM(FUSED, IN, 0);                                              \
   } while (0)
 
 void arks_rmsnorm(void* out, const void* input, const void* weight, float eps,
                   int rows, int hidden, hipStream_t stream) {
   void* const residual = nullptr;
-  const int splits = 0;
-  ARKS_NORM_V(false, false);
+  const int splits = 0, k = 0;
+  const void *const mix_weights = nullptr, *const mix_rows = nullptr;
+  ARKS_NORM_V(false, IN_ROWS);
 }
 
 void arks_fused_add_rmsnorm(void* out, const void* input, void* residual,
                             const void* weight, float eps, int rows, int hidden,
                             hipStream_t stream) {
-  const int splits = 0;
-  ARKS_NORM_V(true, false);
+  const int splits = 0, k = 0;
+  const void *const mix_weights = nullptr, *const mix_rows = nullptr;
+  ARKS_NORM_V(true, IN_ROWS);
 }
 
 void arks_fused_add_rmsnorm_parts(void* out, const void* input, int splits,
                                   void* residual, const void* weight, float eps,
                                   int rows, int hidden, hipStream_t stream) {
-  ARKS_NORM_V(true, true);
+  const int k = 0;
+  const void *const mix_weights = nullptr, *const mix_rows = nullptr;
+  ARKS_NORM_V(true, IN_PARTS);
+}
+
+// input [any, hidden]: row r gets the k (at most 16) rows mix_rows[r] of it,
+// times mix_weights[r]
+void arks_fused_add_rmsnorm_mix(void* out, const void* input,
+                                const void* mix_weights, const void* mix_rows,
+                                int k, void* residual, const void* weight,
+                                float eps, int rows, int hidden,
+                                hipStream_t stream) {
+  const int splits = 0;
+  ARKS_NORM_V(true, IN_MIX);
 }
 #undef ARKS_NORM_V
 #undef ARKS_NORM

@@ -11,6 +11,7 @@
 // The reference delegates MoE serving to external images; these kernels are
 // internals of its runtime slot.
 #include "common.h"
+#include "parts.h"
 
 #include <cfloat>
 
@@ -89,46 +90,22 @@ __global__ __launch_bounds__(256) void moe_mix_rows_kernel(
     const int* __restrict__ rows,       // [T, k]
     const int T, const int H, const int k) {
   const int t = blockIdx.x;
-  __shared__ float w[16];
-  __shared__ int64_t base[16];
-  if (threadIdx.x < 16) {
-    const int j = min((int)threadIdx.x, k - 1);
-    w[threadIdx.x] = (int)threadIdx.x < k ? weights[(int64_t)t * k + j] : 0.f;
-    base[threadIdx.x] = (int64_t)rows[(int64_t)t * k + j] * H;
-  }
-  __syncthreads();
-  // 8 rows' loads at a time, of 16 bytes where rows start there; rows of
-  // weight 0 count as nothing (they may hold anything)
+  weights += (int64_t)t * k;
+  rows += (int64_t)t * k;
+  // loads of 16 bytes where rows start there
   if (H % 8 == 0 &&
       (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out)) % 16 == 0) {
-    for (int h = threadIdx.x * 8; h < H; h += 256 * 8) {
-      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (int j0 = 0; j0 < k; j0 += 8) {
-        ushort8 u[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          u[j] = *reinterpret_cast<const ushort8*>(y + base[j0 + j] + h);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float f = w[j0 + j];
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            acc[e] += f == 0.f ? 0.f : f * bf16_bits_to_float(u[j][e]);
-        }
-      }
-      ushort8 o;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = float_to_bf16_bits(acc[e]);
-      *reinterpret_cast<ushort8*>(out + (int64_t)t * H + h) = o;
-    }
+    for (int h = threadIdx.x * 8; h < H; h += 256 * 8)
+      *reinterpret_cast<ushort8*>(out + (int64_t)t * H + h) =
+          mix_rows8(y, weights, rows, k, H, h);
     return;
   }
   for (int h = threadIdx.x * 2; h < H; h += 256 * 2) {
     float a0 = 0.f, a1 = 0.f;
     for (int j = 0; j < k; ++j) {
-      const uint32_t u = *reinterpret_cast<const uint32_t*>(y + base[j] + h);
-      a0 += w[j] == 0.f ? 0.f : w[j] * bf16_bits_to_float((uint16_t)u);
-      a1 += w[j] == 0.f ? 0.f : w[j] * bf16_bits_to_float((uint16_t)(u >> 16));
+      const uint32_t u = *reinterpret_cast<const uint32_t*>(y + (int64_t)rows[j] * H + h);
+      a0 += weights[j] == 0.f ? 0.f : weights[j] * bf16_bits_to_float((uint16_t)u);
+      a1 += weights[j] == 0.f ? 0.f : weights[j] * bf16_bits_to_float((uint16_t)(u >> 16));
     }
     uint32_t packed = (uint32_t)float_to_bf16_bits(a0) |
                       ((uint32_t)float_to_bf16_bits(a1) << 16);

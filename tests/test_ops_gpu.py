@@ -885,6 +885,61 @@ def test_moe_items(T, E, k, H, I, base, El, tile, skew):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("T,k,H", [
+    (1, 1, 8), (3, 8, 2048), (5, 9, 2056), (70, 2, 4104), (33, 16, 8200),
+    (600, 8, 2048)])
+def test_norm_of_mix(T, k, H):
+    """Experts' rows mixed inside the norm behind them: the bits of a mix of its
+    own; rows of weight 0 hold anything."""
+    assert_native()
+    torch.manual_seed(T)
+    y = torch.randn(T * k, H, device=DEV).bfloat16()
+    rows = torch.randperm(T * k, device=DEV).int().view(T, k)
+    w = torch.rand(T, k, device=DEV)
+    w[::2, k - 1] = 0
+    y[rows[::2, k - 1].long()] = float("nan")
+    res = torch.randn(T, H, device=DEV).bfloat16()
+    nw = torch.rand(H, device=DEV).bfloat16()
+    want = ops.fused_add_rmsnorm(ops.moe_mix_rows(y, w, rows), res.clone(), nw, 1e-6)
+    mixed = ops.Mixed(y, w, rows)
+    assert torch.equal(ops.parts_sum(mixed), ops.moe_mix_rows(y, w, rows))
+    got = ops.fused_add_rmsnorm(mixed, res.clone(), nw, 1e-6)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert not want[0].isnan().any()
+
+
+@pytest.mark.parametrize("T", [7, 40, 300])
+def test_moe_layers_pass_rows_on(T):
+    """Layers of experts hand the norm their rows, at any number of rows, and a
+    tensor where a hook looks on: the same bits. Replays of a captured step too."""
+    assert_native()
+    from arks_amd.config import PRESET_CONFIGS
+    from arks_amd.models import llama_family as lf
+
+    torch.manual_seed(T)
+    cfg = PRESET_CONFIGS["tiny-moe"]
+    mlp = lf.MoEMLP(cfg).to(DEV)
+    for p in mlp.parameters():
+        p.data.normal_(std=cfg.hidden_size ** -0.5)
+    norm = lf.RMSNorm(cfg.hidden_size, 1e-6).to(DEV)
+    x = torch.randn(T, cfg.hidden_size, device=DEV).bfloat16()
+    res = torch.randn_like(x)
+    want = norm(mlp(x), res.clone())
+    assert isinstance(mlp(x, parts=True), ops.Mixed)
+    got = norm(mlp(x, parts=True), res.clone())
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    torch.cuda.synchronize()
+    graph, into = torch.cuda.CUDAGraph(), res.clone()
+    with torch.cuda.graph(graph):
+        out, _ = norm(mlp(x, parts=True), into)
+    for _ in range(3):
+        x.normal_()
+        into.copy_(res)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, norm(mlp(x), res.clone())[0])
+
+
 @pytest.mark.parametrize("up,down", [(2, 2), (2, 4), (4, 2), (4, 4)])
 @pytest.mark.parametrize("T,E,k,H,I,base,El,skew", [
     (1, 4, 2, 64, 64, 0, 4, False), (7, 128, 8, 256, 192, 0, 128, False),
