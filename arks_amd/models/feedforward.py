@@ -266,18 +266,12 @@ class RoutedMoE(nn.Module):
                 self.shared_limit, self.alpha, self.shared_gate), self.w_down)
         weights, ids = ops.moe_route_grouped(z, k, self.groups, self.keep,
                                              **route)
-        xs, place, counts = sort_by_expert(h, ids, E)
-        gu = expert_products(
-            xs, counts, lambda e: self.w_gu[e * 2 * ff:(e + 1) * 2 * ff].t())
-        row_scale = None
-        if self.weigh_input:
-            row_scale = torch.zeros(gu.shape[0], dtype=torch.float32,
-                                    device=h.device)
-            row_scale[place.reshape(-1).long()] = weights.reshape(-1)
-        a = ops.glu_act(gu, self.act, self.limit, self.alpha,
-                        row_scale=row_scale)
-        y = expert_products(
-            a, counts, lambda e: self.w_down[:, e * ff:(e + 1) * ff].t())
+        if (self.act == "swiglu"
+                and ops.moe_wide_takes(h, self.w_gu, self.w_down, E, ff, k)):
+            y, place = ops.moe_wide_rows(h, self.w_gu, self.w_down, weights,
+                                         ids, E, ff, self.weigh_input)
+        else:
+            y, place = self._expert_rows(h, weights, ids)
         shared = None
         if sff:
             su = linear(h, self.w_gu[E * 2 * ff:])
@@ -291,6 +285,23 @@ class RoutedMoE(nn.Module):
         return ops.moe_mix_rows_seq(y, torch.ones_like(weights)
                                     if self.weigh_input else weights,
                                     place, shared)
+
+    def _expert_rows(self, h, weights, ids):
+        """The experts' rows of h, and each pair's place there [T, top]."""
+        E, ff = self.E, self.ff
+        xs, place, counts = sort_by_expert(h, ids, E)
+        gu = expert_products(
+            xs, counts, lambda e: self.w_gu[e * 2 * ff:(e + 1) * 2 * ff].t())
+        row_scale = None
+        if self.weigh_input:
+            row_scale = torch.zeros(gu.shape[0], dtype=torch.float32,
+                                    device=h.device)
+            row_scale[place.reshape(-1).long()] = weights.reshape(-1)
+        a = ops.glu_act(gu, self.act, self.limit, self.alpha,
+                        row_scale=row_scale)
+        y = expert_products(
+            a, counts, lambda e: self.w_down[:, e * ff:(e + 1) * ff].t())
+        return y, place
 
 
 def build_feedforward(mlp: dict, width: int, dtype, arch: str = "") -> nn.Module:

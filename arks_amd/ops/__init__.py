@@ -2065,6 +2065,48 @@ def routed_experts(h, w_gu, w_down, scale, scale_input=True, act="swiglu",
     return y
 
 
+def moe_wide_takes(h, w_gu, w_down, experts: int, ff: int, top: int) -> bool:
+    """Whether moe_wide_rows takes these rows and weights: whole steps of 64
+    columns, and what 32-bit row offsets reach; more experts than 2, whose many
+    rows fill the chip one by one. For the rows of prompts. us with plan or sort and
+    mix, moe_wide_rows (a library product per expert and matrix, behind a gather
+    and a host read of their counts): 16 experts of 4096 x 3584, 4 per row: 257
+    rows 274 (742), 1000 rows 522 (1103), 3500 rows 1098 (1736), 8000 rows 2387
+    (2727); 64 of 2048 x 1408, 6 per row: 1000 rows 284 (2610), 16384 rows 1551
+    (3394); 4 of 4096 x 14336, 2 per row: 257 rows 485 (703), 8192 rows 4742
+    (5085); 2 of these, 2 per row: 257 rows 468 (374), 8192 rows 4583 (4157). The
+    same bits as the library's where an expert has more than 64 rows and at most
+    about 3000, whose products there are one chain of sums too."""
+    T, W = h.shape
+    return (_USE_SKINNY and h.is_cuda and T >= 1
+            and h.dtype == w_gu.dtype == w_down.dtype == torch.bfloat16
+            and 2 < experts <= 1024 and top <= 16 and ff > 0 and W > 0
+            and (W | ff) % 64 == 0 and T * W < 1 << 31
+            and T * top < (1 << 23) - 255 and 2 * ff * W < 1 << 31
+            and w_gu.shape[0] >= 2 * experts * ff and w_gu.shape[1] == W
+            and w_down.shape[0] == W and w_down.shape[1] >= experts * ff
+            and w_down.shape[1] % 8 == 0 and w_down.numel() < 1 << 31
+            and all(w.is_contiguous() and w.data_ptr() % 16 == 0
+                    for w in (w_gu, w_down))
+            and _plain(h, w_gu, w_down))
+
+
+def moe_wide_rows(h, w_gu, w_down, weights, ids, experts: int, ff: int,
+                  scale_input: bool = False):
+    """The silu-GLU experts' rows of h, in any order, and each (row, choice)
+    pair's place there [T, top]: w_gu [>= E * 2 ff, W], w_down [W, >= E * ff],
+    ids [T, top] int32 below E. Projections, activation and result are each
+    rounded to h's dtype; scale_input: the weights scale the experts' input (the
+    caller adds the rows up as they are)."""
+    x = h if (h.stride(-1) == 1 and h.stride(0) % 8 == 0
+              and h.data_ptr() % 16 == 0
+              and h.shape[0] * h.stride(0) < 1 << 31) else h.clone(
+                  memory_format=torch.contiguous_format)
+    return _native().moe_wide_rows(x, w_gu, w_down, weights.contiguous(),
+                                   ids.contiguous(), experts, ff,
+                                   bool(scale_input))
+
+
 # ----------------------------------------------------------------------
 # Sandwich-norm blocks, per-head output gate, capped logits, channel-decay
 # delta rule (same extension, same rule).

@@ -107,7 +107,7 @@ void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    const void* weights, int pairs, int expert_base, int n_local,
                    int tile, int max_items, int groups, hipStream_t stream);
 void arks_moe_gemm(void* out, const void* a, const void* w, const void* perm,
-                   const void* items, const void* n_items, void* claims,
+                   const void* items, const void* n_items, void* claims, const void* scale,
                    int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out, int k_total,
                    int top_k, int max_items, int tile, int up,
                    hipStream_t stream);
@@ -855,13 +855,74 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
                    (int)expert_base, (int)max_items, ft, (int)qt_down, 0, stream);
   } else {
     arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
-                  n_items, claims, x.stride(0), 2 * I * H, H, (int)I, (int)H,
+                  n_items, claims, nullptr, x.stride(0), 2 * I * H, H, (int)I, (int)H,
                   (int)k, (int)max_items, (int)tile, 1, stream);
     arks_moe_gemm(y.data_ptr(), h.data_ptr(), w2.data_ptr(), perm, items,
-                  n_items, claims, I, H * I, I, (int)H, (int)I, (int)k,
+                  n_items, claims, nullptr, I, H * I, I, (int)H, (int)I, (int)k,
                   (int)max_items, (int)tile, 0, stream);
   }
   return {y, w_pair, plan.narrow(0, 4 * max_items + P, P).view({T, k})};
+}
+
+// The experts' rows of x [T, W] in whole tiles: (y [T * k, W], rows [T, k]).
+// w_gu: from its first row on each expert's ff gate rows, then its up rows;
+// w_down [W, ..]: from its first column on ff columns an expert. All pairs are
+// of these experts; scaled: a pair's weight is a factor of its gate and up.
+std::tuple<torch::Tensor, torch::Tensor> moe_wide_rows(
+    torch::Tensor x, torch::Tensor w_gu, torch::Tensor w_down,
+    torch::Tensor weights, torch::Tensor ids, int64_t experts, int64_t ff,
+    bool scaled) {
+  check_bf16_rowstrided(x, "x");
+  check_bf16_contig(w_gu, "w_gu");
+  check_bf16_contig(w_down, "w_down");
+  check_rows_16b(x, "x");
+  check_rows_16b(w_gu, "w_gu");
+  check_rows_16b(w_down, "w_down");
+  TORCH_CHECK(x.dim() == 2 && w_gu.dim() == 2 && w_down.dim() == 2 &&
+              weights.dim() == 2);
+  const int64_t T = x.size(0), W = x.size(1), k = weights.size(1), P = T * k;
+  const int64_t down = w_down.size(1);
+  TORCH_CHECK(w_gu.size(1) == W && w_down.size(0) == W && experts >= 1 &&
+                  ff >= 64 && w_gu.size(0) >= experts * 2 * ff &&
+                  down >= experts * ff,
+              "expert weights do not fit");
+  TORCH_CHECK((W | ff) % 64 == 0 && W >= 64 && experts <= 1024 && k >= 1 &&
+                  k <= 16 && T * x.stride(0) < (1ll << 31) &&
+                  2 * ff * W < (1ll << 31) && W * down < (1ll << 31) &&
+                  P < (1 << 23) - 255,
+              "sizes that tiles of 256 do not take");
+  TORCH_CHECK(weights.is_cuda() && ids.is_cuda() &&
+              weights.scalar_type() == torch::kFloat32 &&
+              weights.is_contiguous() && ids.scalar_type() == torch::kInt32 &&
+              ids.is_contiguous() && ids.sizes() == weights.sizes() &&
+              weights.size(0) == T);
+  torch::Tensor y = torch::empty({P, W}, x.options());
+  if (T == 0) return {y, ids};
+  const int64_t max_items = std::min(P, experts) + P / 256;
+  const int64_t groups = P <= 8192 ? 1 : std::min<int64_t>(64, (P + 2047) / 2048);
+  // as in moe_expert_rows
+  torch::Tensor plan = torch::empty(
+      {4 * max_items + 2 * P + 17 + (groups > 1 ? groups * experts : 0)},
+      x.options().dtype(torch::kInt32));
+  int* items = plan.data_ptr<int>();
+  int* perm = items + 4 * max_items;
+  int* rows = perm + P;
+  int* n_items = rows + P;
+  int* claims = n_items + 1;
+  torch::Tensor w_pair = torch::empty_like(weights);
+  torch::Tensor h = torch::empty({P, ff}, x.options());
+  auto stream = current_stream();
+  arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
+                claims + 16, ids.data_ptr(), weights.data_ptr(), (int)P, 0,
+                (int)experts, 256, (int)max_items, (int)groups, stream);
+  arks_moe_gemm(h.data_ptr(), x.data_ptr(), w_gu.data_ptr(), perm, items,
+                n_items, claims, scaled ? w_pair.data_ptr() : nullptr,
+                x.stride(0), 2 * ff * W, W, (int)ff, (int)W, (int)k,
+                (int)max_items, 256, 2, stream);
+  arks_moe_gemm(y.data_ptr(), h.data_ptr(), w_down.data_ptr(), perm, items,
+                n_items, claims, nullptr, ff, ff, down, (int)W, (int)ff, (int)k,
+                (int)max_items, 256, 0, stream);
+  return {y, plan.narrow(0, 4 * max_items + P, P).view({T, k})};
 }
 
 // The routed experts of x: the mix of moe_expert_rows
@@ -929,6 +990,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mid_gemm", &mid_gemm);
   m.def("stage_rows", &stage_rows);
   m.def("moe_expert_rows", &moe_expert_rows);
+  m.def("moe_wide_rows", &moe_wide_rows);
   m.def("fused_add_rmsnorm_mix", &fused_add_rmsnorm_mix);
   m.def("moe_experts", &moe_experts, pybind11::arg("out"), pybind11::arg("x"),
         pybind11::arg("w13"), pybind11::arg("w2"), pybind11::arg("weights"),

@@ -28,6 +28,7 @@
 // [expert, out, in]: a lane reads 16 bytes along K, as the MFMA operands
 // want them. Items past the last one are empty, so grids depend on the shapes
 // alone and a decode step can be captured.
+#include "seq_common.h"
 #include "tile_engine.h"
 
 namespace arks {
@@ -36,6 +37,10 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int MOE_MAX_E = 1024;
+
+__device__ __forceinline__ float moe_bf16(const float v) {
+  return bf16_bits_to_float(float_to_bf16_bits(v));
+}
 
 __device__ __forceinline__ f32x4 moe_mfma(const ushort8& a, const ushort8& b,
                                           f32x4 c) {
@@ -419,12 +424,16 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
 // neither it nor the pairs' rows are waited for. Its place in LDS belongs to the
 // tiles' array: a second one made the compiler drain the loads before every
 // read of the first.
-template <bool UP>
+// GLU: gate and up are rounded to bf16 before they meet, as rows of a product in
+// memory would be, and scale [pairs] (or null) is a factor of both; it is loaded
+// in front of the next tile's first loads, so as not to be waited for behind them.
+template <bool UP, bool GLU>
 __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ a,
     const bf16* __restrict__ w, const int* __restrict__ perm,
     const int4* __restrict__ items, const int* __restrict__ n_items,
-    int* __restrict__ claims, const int64_t a_stride, const int64_t w_expert,
+    int* __restrict__ claims, const float* __restrict__ scale,
+    const int64_t a_stride, const int64_t w_expert, const int64_t w_stride,
     const int n_out, const int k_total, const int top_k, const int row_tiles) {
   __shared__ __attribute__((aligned(1024))) char lds[TILE_LDS + 16];
   int& claimed = *reinterpret_cast<int*>(lds + TILE_LDS);
@@ -460,7 +469,7 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     t.a = tile_buffer(a + (UP ? 0 : b.first * a_stride));
     const bf16* we = w + b.expert * w_expert;
     t.w[0] = tile_buffer(we);
-    t.w[1] = tile_buffer(we + (UP ? (int64_t)n_out * k_total : 0));
+    t.w[1] = tile_buffer(we + (UP ? n_out * w_stride : 0));
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -471,7 +480,7 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
                      tile_piece_a(r, tile.lane());
         t.wo[h][j] =
             (uint32_t)min(b.n0 + (UP ? 0 : h * 128) + r, n_out - 1) *
-                (uint32_t)(k_total * 2) +
+                (uint32_t)(w_stride * 2) +
             tile_piece_w(r, tile.lane());
       }
     return t;
@@ -491,6 +500,11 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     const Job next = more ? job(i) : now;
     if (more) places(next, p);
     tile.run(t, steps, now.pairs <= TILE_HALF);
+    float by[GLU ? 8 : 1];
+    if constexpr (GLU)
+      tile.each([&](int x, int m, int, const float(&)[8], const float(&)[8]) {
+        by[x] = scale ? scale[perm[now.first + min(m, now.pairs - 1)]] : 1.f;
+      });
     int c;
     if (more) {
       if (threadIdx.x == 0) c = atomicAdd(&claims[xcd], 1);
@@ -503,7 +517,9 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
       if constexpr (UP) {
         float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = tile_silu_mul(g[j], u[j]);
+        for (int j = 0; j < 8; ++j)
+          v[j] = GLU ? silu_f(by[x] * moe_bf16(g[j])) * (by[x] * moe_bf16(u[j]))
+                     : tile_silu_mul(g[j], u[j]);
         o[x] = tile_round(v);
       } else {
         o[2 * x] = tile_round(g);
@@ -562,15 +578,16 @@ extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
 
 // tile: pairs of an item, 16 (streamed; n_out % 32 == k_total % 32 == 0) or 128
 // (tiles through LDS; n_out % 8 == k_total % 8 == 0) or 256 (the engine;
-// n_out % 8 == k_total % 64 == 0, w_stride == k_total, an expert's weights and
-// (up) all rows of a under 4 GiB).
+// n_out % 8 == k_total % 64 == 0, an expert's weights and (up) all rows of a
+// under 4 GiB; up: 1, or 2 for GLU, with scale [pairs] or null).
 extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
                               const void* perm, const void* items,
                               const void* n_items, void* claims,
-                              int64_t a_stride, int64_t w_expert,
+                              const void* scale, int64_t a_stride, int64_t w_expert,
                               int64_t w_stride, int n_out, int k_total,
                               int top_k, int max_items, int tile, int up,
                               hipStream_t stream) {
+  const bool glu = up == 2;
 #define ARKS_STREAM(NF, WV, UP)                                               \
   hipLaunchKernelGGL((moe_stream_kernel<NF, WV, UP>),                         \
                      dim3(n_out / (UP ? 16 : 16 * NF), max_items),            \
@@ -590,14 +607,16 @@ extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
     const int row_tiles = (n_out + (up ? 127 : 255)) / (up ? 128 : 256);
     const int64_t jobs = (int64_t)max_items * row_tiles;
     const dim3 grid(jobs < 256 ? (jobs + 7) / 8 * 8 : 256), block(512);
-#define ARKS_ENGINE(UP)                                                       \
-  hipLaunchKernelGGL((moe_engine_kernel<UP>), grid, block, 0, stream,         \
+#define ARKS_ENGINE(UP, GLU)                                                  \
+  hipLaunchKernelGGL((moe_engine_kernel<UP, GLU>), grid, block, 0, stream,    \
                      (bf16*)out, (const bf16*)a, (const bf16*)w,              \
                      (const int*)perm, (const int4*)items,                    \
                      (const int*)n_items, (int*)claims + (up ? 0 : 8),        \
-                     a_stride, w_expert, n_out, k_total, top_k, row_tiles)
-    if (up) ARKS_ENGINE(true);
-    else ARKS_ENGINE(false);
+                     (const float*)scale, a_stride, w_expert, w_stride, n_out, \
+                     k_total, top_k, row_tiles)
+    if (up && glu) ARKS_ENGINE(true, true);
+    else if (up) ARKS_ENGINE(true, false);
+    else ARKS_ENGINE(false, false);
 #undef ARKS_ENGINE
   } else {
     const int cols = up ? MT_BN / 2 : MT_BN;

@@ -611,3 +611,65 @@ def test_routed_experts_read_the_chosen_alone(rows, E, top, ff, W, act):
     scale.zero_()
     w_gu.nan_to_num_(0.5), w_down.nan_to_num_(0.5)
     assert not ops.routed_experts(h, w_gu, w_down, scale).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("T,E,top,W,ff,extra", [
+    (1, 3, 1, 64, 64, 0), (300, 16, 4, 128, 192, 0), (257, 3, 2, 192, 64, 64),
+    (700, 5, 1, 320, 576, 128), (33, 64, 16, 64, 320, 0), (2100, 9, 4, 64, 128, 8)])
+def test_moe_wide_rows(T, E, top, W, ff, extra, scaled):
+    """Experts in whole tiles against float64: strided rows, weights that hold
+    more behind them, experts with 0, 1, 255, 256 and 257 rows, ends of the
+    tiles. Projections, activation and result are each rounded to bf16."""
+    torch.manual_seed(T)
+    dev = "cuda"
+    h = torch.randn(T, 2 * W, device=dev).bfloat16()[:, :W]
+    w_gu = (torch.randn(2 * E * ff + 2 * extra, W, device=dev) * W ** -0.5).bfloat16()
+    w_down = (torch.randn(W, E * ff + extra, device=dev) * ff ** -0.5).bfloat16()
+    ids = torch.rand(T, E, device=dev).topk(top).indices.int()
+    if E == 9:  # every row takes expert 8; the first choices are as below
+        near = torch.repeat_interleave(
+            torch.arange(4, device=dev), torch.tensor([1, 255, 256, 257], device=dev))
+        ids[:] = torch.tensor([4, 5, 6, 8], device=dev)
+        ids[:near.numel(), 0] = near.int()
+    weights = torch.rand(T, top, device=dev) + 0.1
+    assert ops.moe_wide_takes(h, w_gu, w_down, E, ff, top)
+    y, place = ops.moe_wide_rows(h, w_gu, w_down, weights, ids, E, ff, scaled)
+    assert sorted(place.flatten().tolist()) == list(range(T * top))
+    for e in range(E):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        s = weights[t, j].double()[:, None] if scaled else 1.0
+        g, u = (h[t].double() @ w_gu[2 * e * ff:2 * (e + 1) * ff].double().t()
+                ).split(ff, 1)
+        a = torch.nn.functional.silu(s * g) * s * u
+        d = w_down[:, e * ff:(e + 1) * ff].double()
+        # a gate's or up's rounding (2^-9 of it; silu's slope is at most 1.1)
+        # and the activation's own
+        near = 2 ** -9 * ((1.1 * s * g.abs() + a.abs() / (s * u).abs().clamp(1e-9))
+                          * (s * u).abs() + a.abs()) + 1e-6
+        err = (y[place[t, j].long()].double() - a @ d.t()).abs()
+        assert bool((err <= near @ d.abs().t() + 2 ** -8 * (a @ d.t()).abs() + 1e-6).all())
+
+
+@pytest.mark.gpu
+def test_moe_wide_rows_are_the_layers():
+    """A layer's prompt rows through the tiles and through one product per
+    expert: the same sums up to their order."""
+    from arks_amd.models.feedforward import RoutedMoE
+
+    torch.manual_seed(1)
+    for weigh, shared in (("input", 0), ("output", 0), ("output", 64)):
+        m = RoutedMoE(256, 8, 192, 2, torch.bfloat16, shared_ff=shared,
+                      weigh=weigh).to("cuda")
+        for p in m.parameters():
+            torch.nn.init.normal_(p, std=256 ** -0.5)
+        h = torch.randn(400, 256, device="cuda").bfloat16()
+        with torch.no_grad():
+            out, takes = m(h).double(), ops.moe_wide_takes
+            ops.moe_wide_takes = lambda *a: False
+            try:
+                other = m(h).double()
+            finally:
+                ops.moe_wide_takes = takes
+        assert (out - other).norm() <= 2 ** -8 * other.norm()
