@@ -455,15 +455,15 @@ def step_decode_plan(seq_lens, num_kv_heads: int, window: int, kv_fp8: bool,
 def decode_waves(num_seqs: int, num_kv_heads: int, kv_fp8: bool = False,
                  num_partitions: int | None = None) -> int:
     """Runs per key/value head that the decode kernel cuts all sequences'
-    pages into (attn_decode.hip). One workgroup of 4 waves per CU where a run
-    holds few sequences (64 x 1024: 31.4 us, with two 33.2; 16 x 8000: 55 and
-    64), two where waves often start on a new sequence and wait for its first
-    rows (256 sequences of 1..4000: 86 and 74 us) or where the rows are half
-    as long (48 fp8 ones: 36 and 33). num_partitions: that many runs per
-    sequence on average instead."""
+    pages into (attn_decode.hip). One workgroup of 4 waves per CU (us at 28/4
+    heads x 128: 200 sequences of 20..4000 59.0, with two 60.0; 256 of 100 17.1
+    and 19.9; 256 of 1..4000 178 and 182; 64 x 1024 28.2 and 28.9; counts between
+    6 to 25 % more), two where the rows are half as long (48 fp8 sequences of
+    900..5000 38.9 and 36.3). num_partitions: that many runs per sequence on
+    average instead."""
     if num_partitions is not None:
         return max(1, num_partitions * num_seqs)
-    waves = 2048 if kv_fp8 or num_seqs > 64 else 1024
+    waves = 2048 if kv_fp8 else 1024
     return max(1, waves // num_kv_heads)
 
 

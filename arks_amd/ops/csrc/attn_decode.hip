@@ -6,8 +6,8 @@
 // of very different lengths, and a decode graph fixes the grid before they
 // are known. So the work is cut by what it is and not by the grid: a unit is
 // 32 tokens (2 pages) of one sequence; the units of all sequences are one
-// line, cut into runs of equal length, one run per WAVE, 4 or 8 waves per CU. A
-// run that covers a whole sequence writes its rows of the output, any other
+// line, cut into runs of equal length (where runs hold many short sequences,
+// the start of each counts too), one run per WAVE, 4 or 8 waves per CU. A run that covers a whole sequence writes its rows of the output, any other
 // an f32 partial (acc, m, l), and attn_decode_combine merges a sequence's
 // partials. Waves share nothing: no barrier. The runs depend on the lengths
 // alone, so attn_decode_plan finds them once for all layers of a step:
@@ -30,7 +30,8 @@
 // 2 workgroups per CU, and less at counts between. 28/4 heads x 128, kernel
 // and merge, with a workgroup per (sequence, head, part of the grid) before:
 //   64 x 1024, bf16            34.4 -> 31.4 us
-//   256 of 1..4000, bf16      108.9 -> 74.2 us
+//   256 of 1..4000, bf16      108.9 -> 74.2 us (two workgroups per CU, all
+//                              units alike; starts counted, one: 3 % less)
 //   48 x 900..5000, fp8       140.8 -> 33.3 us (its bytes were converted one
 //                              by one, in front of the wait for the next)
 //
@@ -115,46 +116,97 @@ __global__ __launch_bounds__(1024) void attn_decode_plan_kernel(
     int* __restrict__ plan, const int* __restrict__ lens, const int n,
     const int window, const int waves) {
   constexpr int NW = 1024 / WAVE_SIZE;
-  __shared__ int sums[NW], tops[NW];
+  __shared__ int sums[NW], tops[NW], seqs_in[NW], shorter;
   const int tid = threadIdx.x, lane = tid % WAVE_SIZE, wave = tid / WAVE_SIZE;
   const int per = (n + 1023) / 1024;
   const int s0 = min(n, tid * per), s1 = min(n, s0 + per);
-  int mine = 0, longest = 0;
+  int mine = 0, longest = 0, some = 0;
   for (int s = s0; s < s1; ++s) {
     const int u = dec_units(lens[s], window);
     mine += u;
+    some += u > 0;
     longest = max(longest, u);
   }
-  int scan = mine;
+  int scan = mine, scan_s = some;
 #pragma unroll
   for (int off = 1; off < WAVE_SIZE; off <<= 1) {
     const int v = __shfl_up(scan, off, WAVE_SIZE);
-    if (lane >= off) scan += v;
+    const int vs = __shfl_up(scan_s, off, WAVE_SIZE);
+    if (lane >= off) {
+      scan += v;
+      scan_s += vs;
+    }
     longest = max(longest, __shfl_xor(longest, off, WAVE_SIZE));
   }
-  if (lane == WAVE_SIZE - 1) sums[wave] = scan;
+  if (lane == WAVE_SIZE - 1) {
+    sums[wave] = scan;
+    seqs_in[wave] = scan_s;
+  }
   if (lane == 0) tops[wave] = longest;
+  if (tid == 0) shorter = 0;
   __syncthreads();
-  int at = scan - mine, total = 0;
+  int units = scan - mine, seqs_before = scan_s - some, total = 0, held = 0;
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    if (w < wave) at += sums[w];
+    if (w < wave) {
+      units += sums[w];
+      seqs_before += seqs_in[w];
+    }
     total += sums[w];
+    held += seqs_in[w];
     longest = max(longest, tops[w]);
   }
-  const int run = dec_run_length(total, longest, waves);
+  // Equal runs of units, unless some would hold whole sequences: a run waits for
+  // a chain of loads (page ids, then rows) at each sequence that it starts, which
+  // counts as one unit more then. 28/4 heads x 128, us with the merge, so (equal
+  // units): 200 of 20..4000 (even over the logarithm) 60.6 (64.6), fp8 36.1
+  // (40.5); 64 of them 24.8 (26.8); 256 of 20..500 23.1 (24.3); 256 of 1..4000
+  // 180 (182). Half a unit gives half of it, two no more.
+  const int even = dec_run_length(total, longest, waves);
+  int less = 0;
+  for (int s = s0; s < s1; ++s) {
+    const int u = dec_units(lens[s], window);
+    less |= u > 0 && u < even;
+  }
+  if (less) shorter = 1;
+  __syncthreads();
+  const int front = shorter;
+  const int line = total + held * front;
+  const int run = shorter ? max(dec_run_length(0, longest, waves),
+                                (line + waves - 1) / waves)
+                          : even;
+  int at = units + seqs_before * front;
   int4* runs = reinterpret_cast<int4*>(plan);
   int2* seqs = reinterpret_cast<int2*>(plan + 4 * waves);
+  // unit j of a sequence lies at `at` + front + j. A run (of 2 places at least)
+  // holds a unit, and its length is found from the first units of its neighbours.
   for (int s = s0; s < s1; ++s) {
-    const int L = lens[s], u = dec_units(L, window);
-    const int w0 = at / run;
-    seqs[s] = make_int2(w0, u > 0 ? (at + u - 1) / run - w0 + 1 : 0);
-    for (int w = (at + run - 1) / run; w * run < at + u; ++w)
-      runs[w] = make_int4(s, w * run - at, L, min(run, total - w * run));
-    at += u;
+    const int L = lens[s], u = dec_units(L, window), b = at + front;
+    if (u == 0) {
+      seqs[s] = make_int2(0, 0);
+      continue;
+    }
+    const int w0 = b / run, w1 = (b + u - 1) / run;
+    seqs[s] = make_int2(w0, w1 - w0 + 1);
+    // (the unit in front of this sequence lies at `at` - 1)
+    for (int w = at == 0 || at - 1 < w0 * run ? w0 : w0 + 1; w <= w1; ++w) {
+      const int j = max(0, w * run - b);
+      runs[w] = make_int4(s, j, L, units + j);
+    }
+    at = b + u;
+    units += u;
   }
-  for (int w = (total + run - 1) / run + tid; w < waves; w += 1024)
-    runs[w] = make_int4(0, 0, 0, 0);
+  const int used = (line + run - 1) / run;
+  __threadfence_block();
+  __syncthreads();
+  for (int w0 = 0; w0 < waves; w0 += 1024) {
+    const int w = w0 + tid;
+    const int first = w < used ? runs[w].w : 0;
+    const int next = w + 1 < used ? runs[w + 1].w : total;
+    __syncthreads();
+    if (w < used) runs[w].w = next - first;
+    else if (w < waves) runs[w] = make_int4(0, 0, 0, 0);
+  }
 }
 
 template <int HEAD_DIM, int GQ, bool KV_FP8>

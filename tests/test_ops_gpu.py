@@ -305,6 +305,46 @@ def test_attention_decode_plan_size():
             ops.attention_decode_paged(q, kc, kc, bt, lens, 1.0, plan=plan)
 
 
+@pytest.mark.parametrize("waves", [1, 5, 256, 1024, 3000])
+@pytest.mark.parametrize("n,high", [(1, 1), (3, 30000), (64, 40), (200, 4000),
+                                    (1500, 300)])
+def test_attention_decode_plan_runs(n, high, waves):
+    """Every unit of 32 visible tokens belongs to one run, in order, runs are
+    about as long as each other (with a unit for each sequence that they start),
+    and a sequence's runs are those that hold its units."""
+    assert_native()
+    g = torch.Generator().manual_seed(n + waves)
+    for window in (0, 100):
+        lens = torch.exp(torch.rand(n, generator=g) * math.log(high + 1)).int()
+        lens[torch.rand(n, generator=g) < 0.1] = 0
+        plan = torch.full((4 * waves + 2 * n,), -7, dtype=torch.int32, device=DEV)
+        ops._native().attention_decode_plan(plan, lens.to(DEV), waves, window)
+        plan, lens = plan.tolist(), lens.tolist()
+        units = [-(-L // 32) - (max(0, (L - window) // 32) if window else 0)
+                 for L in lens]
+        line = [(s, u) for s in range(n) for u in range(units[s])]
+        at, seen, longest = 0, [set() for _ in lens], 0
+        for w in range(waves):
+            s, first, L, count = plan[4 * w:4 * w + 4]
+            if count == 0:
+                assert at == len(line)
+                continue
+            assert (s, first) == line[at] and L == lens[s]
+            mine = line[at:at + count]
+            assert len(mine) == count
+            longest = max(longest, count + len({s for s, _ in mine}))
+            for s, _ in mine:
+                seen[s].add(w)
+            at += count
+        assert at == len(line)
+        for s in range(n):
+            w0, count = plan[4 * waves + 2 * s:4 * waves + 2 * s + 2]
+            assert seen[s] == set(range(w0, w0 + count))
+        # a run's share and the units it is rounded by, or that merging asks for
+        merge = math.ceil(math.sqrt(0.15 * max(units)))
+        assert longest <= max(2, merge, -(-(len(line) + n) // waves)) + 2
+
+
 def test_attention_decode_fp8_codes():
     """Every e4m3 code reads as its own value."""
     assert_native()
