@@ -684,10 +684,10 @@ def _mid(x, weight, bias=None, silu: bool = False, summed: bool = False):
     else None. summed: the consumer adds the sums of splits. It takes up to 256
     rows, but for what the streamed product (few rows of small weights, which
     has no sums to add) or the library does as fast (_mid_sizes). us, here
-    (other): 37888 x 3584 with the activation, 1 row 42.2 (48.1), 32 rows 42.9
-    (57.6), 128 rows 51.0 (71.2), 200 rows 65 (85); 152064 x 3584, 1 row 168
-    (182), 64 rows 201 (209), 200 rows 284 (325); 3584 x 18944, 1 row 23.0 and
-    0.3 of sums (27.4), 100 rows 30.3 and 3 (96.5)."""
+    (other): 37888 x 3584 with the activation, 1 row 44.7 (48.1), 32 rows 45.1
+    (57.6), 128 rows 52.9 (71.2), 200 rows 61.6 (85); 152064 x 3584, 1 row 168
+    (182), 64 rows 189 (209), 200 rows 264 (325); 3584 x 18944 with a launch for
+    the sums, 1 row 26.3 (27.4), 100 rows 36.1 (96.5)."""
     if not _mid_takes(x, weight, bias):
         return None
     N, K = weight.shape
@@ -1098,12 +1098,13 @@ def moe_tile(rows: int, top_k: int, experts: int, whole: bool = False) -> int:
     sizes are whole steps (mid_gemm.hip, whose items of 128 take over at 32 on
     the mean, as some experts have twice the mean), 128 or more beyond
     (moe_experts). Other sizes are streamed up to 8 on the mean. us, 16 (64;
-    128 of mid_gemm; 256): 128 experts of 2048 x 768, 8 per row: 7 rows 83 (86),
-    16 rows 142 (142), 64 rows 208 (196; 215), 200 rows 268 (210; 228; 234), 600
-    rows (233; 251; 252), 1000 rows (346; 265; 269), 1300 rows (461; 280; 281);
-    8 experts of 4096 x 14336, 2 per row: 1 row 137 (169), 16 rows 509 (424;
-    429), 200 rows (463; 476; 590), 600 rows (1384; 1099; 726). experts: those
-    that the rows choose from, of all ranks."""
+    128 of mid_gemm; 256): 128 experts of 2048 x 768, 8 per row: 7 rows 91 (91),
+    16 rows 147 (139), 64 rows 208 (190; 207), 200 rows 254 (208; 223; 238), 600
+    rows (226; 245; 254), 1000 rows (346; 265; 269), 1300 rows (461; 280; 281);
+    8 experts of 4096 x 14336, 2 per row: 1 row 133 (162), 16 rows 505 (437;
+    446), 200 rows (474; 478; 566), 600 rows (1384; 1099; 726). Up to 32 rows
+    items of 32 may take their place (_moe_few). experts: those that the rows
+    choose from, of all ranks."""
     if whole and experts <= rows * top_k <= 64 * experts:
         return 64
     return 16 if rows * top_k <= 8 * experts else 128
@@ -1219,7 +1220,7 @@ def _moe_cut(x, w13, w2, ids, experts):
     x = _rows_16b(x)
     whole = _moe_whole(x, H, I, rows * k)
     way = _moe_way(rows, k, El, experts or El, H, I, whole)
-    # experts of 2 MB and more: below, launches are what counts
+    # matrices of 2^19 weights and more: below, launches are what counts
     if (rows <= 32 and whole and way in ((16, False), (64, True))
             and H * I >= 1 << 19):
         cut = _moe_few(rows, k, El, experts or El, H, I, way[0] == 16)
