@@ -35,11 +35,11 @@ constants as constructor parameters:
   projections, an activation whose factor is 0 for the experts a row does
   not use (so their columns are exactly 0), and ONE down GEMM over all
   columns, which sums the chosen experts and the shared one (up to 16 rows
-  without a shared expert ops.routed_experts gives the same, and reads the
-  chosen experts alone). Above it the
-  (row, expert) pairs are sorted by expert as in GroupedMoE. Experts may also
-  be chosen in groups, by scores with a correction per expert that the
-  weights do not see, and a group ranked by its best or its two best;
+  without a shared expert, for weights of more than 34 million elements,
+  ops.routed_experts gives the same, and reads the chosen experts alone).
+  Above it the (row, expert) pairs are sorted by expert as in GroupedMoE.
+  Experts may also be chosen in groups, by scores with a correction per expert
+  that the weights do not see, and a group ranked by its best or its two best;
   the activation may be ClampedGLU's (limit, and shared_limit for the shared
   expert); and the shared expert may be weighed by sigmoid(W_sg h), a row of
   the router's matrix.
@@ -256,7 +256,10 @@ class RoutedMoE(nn.Module):
         if T <= self.DENSE_TOKENS:
             _, _, scale = ops.moe_route_grouped(
                 z, k, self.groups, self.keep, matrix=True, **route)
-            if not sff and ops.routed_takes(h, self.w_gu, self.w_down, E, ff):
+            # (weights that linear_fixed takes keep the order of sums that they
+            # have at 17 rows and more)
+            if (not sff and ops.routed_takes(h, self.w_gu, self.w_down, E, ff)
+                    and not ops.sums_fixed(T, self.w_gu, self.w_down)):
                 return ops.routed_experts(h, self.w_gu, self.w_down, scale,
                                           self.weigh_input, self.act,
                                           self.limit, self.alpha)

@@ -872,6 +872,12 @@ def fix_sums(weights) -> None:
         w.fixed_sums = True
 
 
+def sums_fixed(M: int, *weights) -> bool:
+    """Whether linear_fixed has an order of its own for any of these weights at
+    M rows (up to 64)."""
+    return any(_fixed_run(M, *w.shape) for w in weights)
+
+
 def linear_fixed(x, weight, bias=None):
     """x weight^T (+ bias) whose order of sums follows from the weight alone up
     to 48 rows, for models that choose experts. Near a tie between two of them
@@ -2037,32 +2043,22 @@ def routed_takes(h, w_gu, w_down, experts: int, ff: int) -> bool:
             and _plain(h, w_gu, w_down) and seq_native_available())
 
 
-def routed_chunk(rows: int, down: bool) -> int:
-    """Columns of K after which the 4 chains of sums of a routed product move on
-    together. Which rows take which follows the library's products, whose places
-    these took and whose sums they are, bit for bit: 114688 x 4096 and 4096 x
-    57344 at 1 to 16 rows."""
-    if rows in (1, 8):
-        return 1024 if down else 512
-    return 512 if down else 128
-
-
 def routed_experts(h, w_gu, w_down, scale, scale_input=True, act="swiglu",
                    limit=0.0, alpha=1.0):
     """The weighted sum of the experts that rows chose (scale [T, E] fp32: their
     weights, 0 elsewhere), for what routed_takes takes: linear, moe_glu_scaled and
-    linear over all experts, without those that nobody chose. us, here (those
-    three), 16 experts of ff 3584 on 4096 columns, 4 per row, weights cold: 1 row
-    (4 of them chosen) 67 (244), 2 rows (8) 124 (287), 8 rows (11) 167 (245), 16
-    rows (all) 248 (308)."""
+    linear over all experts, without those that nobody chose, in one order of sums
+    for any number of rows. us, here (those three), 16 experts of ff 3584 on 4096
+    columns, 4 per row, weights cold: 1 row (4 of them chosen) 67 (244), 2 rows
+    (8) 124 (287), 8 rows (11) 167 (245), 16 rows (all) 248 (308)."""
     T, E = scale.shape
     C = _native_seq()
     x = _rows_16b(h)
     a = torch.empty((T, w_down.shape[1]), dtype=h.dtype, device=h.device)
-    C.routed_up(a, x, w_gu, scale, routed_chunk(T, False), bool(scale_input),
-                act == "clamped", float(limit), float(alpha))
+    C.routed_up(a, x, w_gu, scale, bool(scale_input), act == "clamped",
+                float(limit), float(alpha))
     y = torch.empty((T, w_down.shape[0]), dtype=h.dtype, device=h.device)
-    C.routed_down(y, a, w_down, scale, routed_chunk(T, True))
+    C.routed_down(y, a, w_down, scale)
     return y
 
 

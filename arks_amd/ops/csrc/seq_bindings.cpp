@@ -199,13 +199,13 @@ int arks_seq_diff_head_norm_gate(void* out, int64_t ldo, const void* a,
                                  int V, int act_f32, hipStream_t stream);
 void arks_seq_routed_up(void* out, const void* x, int64_t x_stride,
                         const void* w, const void* scale, int64_t scale_stride,
-                        int m, int k, int chunk, int experts, int ff,
-                        int scale_in, int clamped, float limit, float alpha,
+                        int m, int k, int experts, int ff, int scale_in,
+                        int clamped, float limit, float alpha,
                         hipStream_t stream);
 void arks_seq_routed_down(void* out, const void* x, int64_t x_stride,
                           const void* w, const void* scale,
-                          int64_t scale_stride, int m, int n, int chunk,
-                          int experts, int ff, hipStream_t stream);
+                          int64_t scale_stride, int m, int n, int experts,
+                          int ff, hipStream_t stream);
 void arks_seq_moe_glu_scaled(void* out, const void* gu, int64_t ldg,
                              const void* scale, int64_t lds, int64_t T, int E,
                              int ff, int sff, int scale_in, int clamped,
@@ -1228,38 +1228,37 @@ void check_routed(const Tensor& x, const Tensor& w, const Tensor& scale,
   TORCH_CHECK(M >= 1 && M <= 16 && out.size(0) == M && scale.size(1) >= 1 &&
                   scale.size(1) <= 64 && w.size(1) == K && ff % 16 == 0 && ff > 0,
               "at most 16 rows and 64 experts");
-  TORCH_CHECK((chunk == 128 || (chunk > 0 && chunk % 256 == 0)) &&
-                  K % chunk == 0 && K % 256 == 0 && K < (1 << 22),
-              "K must be whole chunks");
+  TORCH_CHECK(K % chunk == 0 && K < (1 << 22), "K must be whole chunks");
 }
 
 // Activated gate and up products of the experts that rows chose (scale [M, E]:
 // not 0), 0 for those that only others chose; what nobody chose stays as it was.
-void routed_up(Tensor out, Tensor x, Tensor w, Tensor scale, int64_t chunk,
-               bool scale_input, bool clamped, double limit, double alpha) {
+void routed_up(Tensor out, Tensor x, Tensor w, Tensor scale, bool scale_input,
+               bool clamped, double limit, double alpha) {
+  TORCH_CHECK(w.dim() == 2 && scale.dim() == 2 && scale.size(1) >= 1);
   const int64_t E = scale.size(1), ff = w.size(0) / (2 * E);
-  check_routed(x, w, scale, out, chunk, ff);
+  check_routed(x, w, scale, out, 512, ff);
   TORCH_CHECK(w.size(0) == E * 2 * ff && out.size(1) == E * ff &&
               2 * ff * w.size(1) * 2 < (1ll << 32));
   arks_seq_routed_up(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(),
                      scale.data_ptr(), scale.stride(0), (int)x.size(0),
-                     (int)x.size(1), (int)chunk, (int)E, (int)ff,
-                     scale_input ? 1 : 0, clamped ? 1 : 0, (float)limit,
-                     (float)alpha, current_stream());
+                     (int)x.size(1), (int)E, (int)ff, scale_input ? 1 : 0,
+                     clamped ? 1 : 0, (float)limit, (float)alpha,
+                     current_stream());
 }
 
 // x [M, E * ff] . w [N, E * ff]^T over the columns of the experts that rows chose.
-void routed_down(Tensor out, Tensor x, Tensor w, Tensor scale, int64_t chunk) {
+void routed_down(Tensor out, Tensor x, Tensor w, Tensor scale) {
+  TORCH_CHECK(w.dim() == 2 && scale.dim() == 2 && scale.size(1) >= 1);
   const int64_t E = scale.size(1), ff = w.size(1) / E;
-  check_routed(x, w, scale, out, chunk, ff);
+  check_routed(x, w, scale, out, 1024, ff);
   TORCH_CHECK(w.size(1) == E * ff && out.size(1) == w.size(0) &&
                   w.size(0) % 16 == 0 && w.size(0) < (1 << 24) &&
-                  chunk % 256 == 0 && ff % (chunk / 4) == 0,
+                  ff % 256 == 0,
               "an expert's columns must be whole quarters of chunks");
   arks_seq_routed_down(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(),
                        scale.data_ptr(), scale.stride(0), (int)x.size(0),
-                       (int)w.size(0), (int)chunk, (int)E, (int)ff,
-                       current_stream());
+                       (int)w.size(0), (int)E, (int)ff, current_stream());
 }
 
 void moe_glu_scaled(Tensor out, Tensor gu, Tensor scale, int64_t experts,

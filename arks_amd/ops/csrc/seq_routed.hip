@@ -6,20 +6,20 @@
 // in mid_gemm.hip, whose stages, waits and barriers these are: rows go from
 // memory straight into LDS, NS steps ahead.
 //
-// The order of sums is fixed by `chunk`: K is cut into chunks, a chunk into 4
-// parts, and wave p adds up part p of every chunk in one chain; the 4 sums are
-// added in order. That is how the library's products of these rows add up (chunk:
-// ops.routed_chunk), which took these places before: near a tie the last bits of
-// a row decide between two experts, and no choice may turn with the kernel. The
-// columns of experts that nobody chose are products with 0, so that leaving them
-// out changes nothing.
+// The order of sums is the same for any number of rows: K is cut into chunks of
+// CHUNK columns, a chunk into 4 parts, and wave p adds up part p of every chunk in
+// one chain; the 4 sums are added in order. Near a tie the last bits of a row
+// decide between two experts, and no choice may turn with the rows that share a
+// step. The columns of experts that nobody chose are products with 0, so that
+// leaving them out changes nothing. (The chunks are those in which the library's
+// products of 1 and of 8 rows, which were here before, were seen to add up with
+// weights of 114688 x 4096 and 4096 x 57344: such steps kept their bits.)
 //
 // 16 experts of ff 3584 on 4096 columns, 4 per row, weights cold, us (the
 // library's products over all experts): gate and up with the activation, 1 row
 // (4 experts chosen) 42.7 (157 and 4.6 for the activation), 8 rows (11) 111 (158
 // and 4.3), 16 rows (16) 161 (190 and 4.5), 5.5 to 6.1 TB/s; down 23.8 (82), 56
-// (82), 87 (114). Parts of 32 columns (chunk 128) loaded by the wave that takes
-// them, half lines of 64 bytes, 16 rows 187.
+// (82), 87 (114).
 #include <type_traits>
 
 #include "seq_common.h"
@@ -68,18 +68,18 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ x, const int64_t x_stride,
     const bf16* __restrict__ w, const float* __restrict__ scale,
     const int64_t scale_stride, const int m_rows, const int n_total,
-    const int k_total, const int chunk, const int experts, const int ff,
-    const RoutedAct act) {
+    const int k_total, const int experts, const int ff, const RoutedAct act) {
   constexpr int NS = routed_stages(QT);
   constexpr int PART = (QT + 1) * 2048, STAGE = 4 * PART;  // of wave p; of all
   constexpr int LOADS = 2 * QT + 2;
   constexpr int COLS = UP ? 8 * QT : 16 * QT;
+  constexpr int CHUNK = UP ? 512 : 1024, OWN = CHUNK / 4;  // columns; of a wave
   static_assert(NS >= 3 && (NS - 1) * LOADS < 64 && (!UP || QT % 2 == 0));
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
   __shared__ tile_f32x4 sums[4][QT][WAVE_SIZE];
   const int lane = threadIdx.x % WAVE_SIZE, lq = lane % 16, la = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
-  const int p = wave % 4, part = chunk / 4;
+  const int p = wave % 4;
 
   // the experts that somebody chose (none: all rows of the first one's are 0)
   bool mine = false;
@@ -89,10 +89,10 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
   if (chosen == 0) chosen = 1;
 
   // which chunks' part of a wave is a chosen expert's, 64 of them from `first`
-  const int chunks = k_total / chunk;
+  const int chunks = k_total / CHUNK;
   auto active = [&](const int first, const int of) -> uint64_t {
     const int c = first + lane;
-    const int e = (c * chunk + of * part) / ff;
+    const int e = (c * CHUNK + of * OWN) / ff;
     return __ballot(c < chunks && (chosen >> min(e, 63) & 1));
   };
   const int per = UP ? k_total / 256 : 1;  // steps of a job
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
     for (int of = 0; of < 4; ++of) {
       int n = 0;
       for (int c = 0; c < chunks; c += 64) n += __popcll(active(c, of));
-      n *= part / 64;
+      n *= OWN / 64;
       steps = max(steps, n);
       if (of == p) own_steps = n;
     }
@@ -166,10 +166,10 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
       int col;  // of this wave's step s
       if constexpr (UP) {
         const int i = s * 64;
-        col = part == 32 ? s * 256 + p * 64 : i / part * chunk + p * part + i % part;
+        col = i / OWN * CHUNK + p * OWN + i % OWN;
       } else {
-        col = c * chunk + p * part + sub * 64;
-        if (++sub == part / 64) {
+        col = c * CHUNK + p * OWN + sub * 64;
+        if (++sub == OWN / 64) {
           sub = 0;
           next_chunk();
         }
@@ -223,15 +223,8 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
     return;
   }
 
-  // where half h of a step's operands lie: 16 rows of 128 B, pieces permuted. Of
-  // parts of 32 columns a step of whole lines holds all 4, in two lines, of two
-  // chunks.
+  // where a step's operands lie: 16 rows of 128 B, pieces permuted
   const int frag = lq * 128 + ((la ^ (lq & 7)) * 16);
-  int from[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-    from[h] = part == 32 ? (2 * h + p / 2) * PART + (frag ^ (p % 2 * 64))
-                         : p * PART + (frag ^ (h * 64));
   int at = 0;  // the stage that is read
   routed_barrier();
   for (int j = blockIdx.x; j < jobs; j += gridDim.x) {
@@ -243,7 +236,7 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
       ushort8 wf[2][QT], xf[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const char* rows = lds + at * STAGE + from[h];
+        const char* rows = lds + at * STAGE + p * PART + (frag ^ (h * 64));
         xf[h] = *reinterpret_cast<const ushort8*>(rows + QT * 2048);
 #pragma unroll
         for (int q = 0; q < QT; ++q)
@@ -314,12 +307,11 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
 
 using namespace arks;
 
-// m <= 16, experts <= 64, ff % 16 == 0, k % 256 == 0 and % chunk == 0, chunk 128
-// or a multiple of 256; an expert's rows and all of x under 4 GiB, rows of x and
-// w on 16 bytes.
+// m <= 16, experts <= 64, ff % 16 == 0, k % 512 == 0; an expert's rows and all of
+// x under 4 GiB, rows of x and w on 16 bytes.
 extern "C" void arks_seq_routed_up(void* out, const void* x, int64_t x_stride,
                                    const void* w, const void* scale,
-                                   int64_t scale_stride, int m, int k, int chunk,
+                                   int64_t scale_stride, int m, int k,
                                    int experts, int ff, int scale_in,
                                    int clamped, float limit, float alpha,
                                    hipStream_t stream) {
@@ -328,21 +320,19 @@ extern "C" void arks_seq_routed_up(void* out, const void* x, int64_t x_stride,
   hipLaunchKernelGGL((routed_gemm_kernel<4, true>),
                      dim3((unsigned)(jobs < 256 ? jobs : 256)), dim3(512), 0,
                      stream, (bf16*)out, (const bf16*)x, x_stride, (const bf16*)w,
-                     (const float*)scale, scale_stride, m, 0, k, chunk, experts,
-                     ff, act);
+                     (const float*)scale, scale_stride, m, 0, k, experts, ff, act);
 }
 
-// x [m, experts * ff], w [n, experts * ff], n % 16 == 0, chunk a multiple of 256
-// whose quarter divides ff, chunks whole; 16 rows of w and all of x under 4 GiB.
+// x [m, experts * ff], w [n, experts * ff], n % 16 == 0, ff % 256 == 0, experts *
+// ff % 1024 == 0; 16 rows of w and all of x under 4 GiB.
 extern "C" void arks_seq_routed_down(void* out, const void* x, int64_t x_stride,
                                      const void* w, const void* scale,
                                      int64_t scale_stride, int m, int n,
-                                     int chunk, int experts, int ff,
-                                     hipStream_t stream) {
+                                     int experts, int ff, hipStream_t stream) {
   const int jobs = n / 16;
   hipLaunchKernelGGL((routed_gemm_kernel<1, false>),
                      dim3(jobs < 256 ? jobs : 256), dim3(512), 0, stream,
                      (bf16*)out, (const bf16*)x, x_stride, (const bf16*)w,
-                     (const float*)scale, scale_stride, m, n, experts * ff, chunk,
+                     (const float*)scale, scale_stride, m, n, experts * ff,
                      experts, ff, RoutedAct{});
 }

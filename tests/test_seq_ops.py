@@ -614,6 +614,37 @@ def test_routed_experts_read_the_chosen_alone(rows, E, top, ff, W, act):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("E,top,ff,W,most", [
+    (4, 2, 512, 1024, 48),     # weights of linear_fixed
+    (16, 4, 1024, 2560, 16)])  # routed_experts takes them
+def test_routed_layer_order_of_sums(E, top, ff, W, most, monkeypatch):
+    """A row's experts add up to the same bits whatever rows share its step."""
+    from arks_amd.models.feedforward import RoutedMoE
+
+    torch.manual_seed(E)
+    m = RoutedMoE(W, E, ff, top, torch.bfloat16, weigh="output").to("cuda")
+    for p in m.parameters():
+        torch.nn.init.normal_(p, std=p.shape[-1] ** -0.5)
+    ops.fix_sums(m.parameters())
+    h = torch.randn(most, W, device="cuda").bfloat16()
+    scale = torch.zeros(most, E, device="cuda")
+    scale.scatter_(1, torch.randn(most, E, device="cuda").topk(top).indices,
+                   torch.rand(most, top, device="cuda") + 0.1)
+    monkeypatch.setattr(ops, "moe_route_grouped", lambda z, *a, **k: (
+        None, None, scale[:z.shape[0]]))
+    routed = ops.routed_experts
+    took = []
+    monkeypatch.setattr(ops, "routed_experts", lambda h, *a: (
+        took.append(h.shape[0]), routed(h, *a))[1])
+    with torch.no_grad():
+        whole = m(h)
+        for T in (1, 2, 7, 8, 9, 15, 16, 17, 33):
+            if T <= most:
+                assert torch.equal(m(h[:T]), whole[:T]), T
+    assert took == ([] if E == 4 else [16, 1, 2, 7, 8, 9, 15, 16])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("scaled", [False, True])
 @pytest.mark.parametrize("T,E,top,W,ff,extra", [
     (1, 3, 1, 64, 64, 0), (300, 16, 4, 128, 192, 0), (257, 3, 2, 192, 64, 64),
