@@ -158,8 +158,10 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   // first): workgroups that read the same columns of rows a power of two apart
   // would all meet on a few memory channels (16 rows x 151936 x 2048 127 -> 102
   // us, x 57344 x 8192 164 -> 147). An expert's follows from its number and
-  // the tile alone, not from the item: which item a pair is in depends on the
-  // other rows of the step, and its order of sums must not.
+  // the column alone, in units of a tile of QT 4: not from the item, nor from the
+  // tiles, which both depend on the other rows of the step. So a pair's sums are
+  // the same bits in items of 32 and of 64, with tiles of any height (items of 128
+  // and the streamed kernel of moe_gemm.hip add up in other chains).
   struct Job {
     int n0, split, s0, steps, turn;
     int expert, first, rows;
@@ -167,9 +169,10 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   auto job = [&](const int j) {
     if constexpr (ITEMS) {
       const int4 it = of.items[j / tiles];
-      const unsigned tile = j % tiles;
-      const unsigned at = (unsigned)(of.expert_base + it.x) * tiles + tile;
-      return Job{(int)tile * COLS, 0, 0, all_steps,
+      constexpr unsigned UNIT = SILU ? 64 : 128;
+      const unsigned n0 = j % tiles * COLS, units = (n_total + UNIT - 1) / UNIT;
+      const unsigned at = (unsigned)(of.expert_base + it.x) * units + n0 / UNIT;
+      return Job{(int)n0, 0, 0, all_steps,
                  rotate ? (int)(at % (unsigned)all_steps) : 0,
                  it.x, it.y, it.z};
     }

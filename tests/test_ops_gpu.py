@@ -1461,6 +1461,42 @@ def test_stream_gemm(M, N, K, bias):
     assert ((out - expect).abs() <= 2 * slack + 2 ** -8 * expect.abs()).all()
 
 
+def test_moe_items_order_of_sums_by_rows():
+    """A row's experts give the same bits in items of 32 with tiles of either
+    height and in items of 64, as a tensor and as rows to mix, whatever rows
+    share the step."""
+    assert_native()
+    torch.manual_seed(5)
+    E, k, H, I = 16, 2, 1024, 576
+    sizes = (8, 16, 20, 32, 33, 64)
+    cuts = [ops._moe_few(T, k, E, E, H, I, False) for T in sizes if T <= 32]
+    assert set(cuts) == {(2, 2), (4, 2)}
+    assert all(ops._moe_way(T, k, E, E, H, I, True) == (64, True) for T in sizes)
+    x = torch.randn(64, H, device=DEV).bfloat16()
+    w13 = (torch.randn(E, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(E, H, I, device=DEV) * I ** -0.5).bfloat16()
+    ids = torch.rand(64, E, device=DEV).topk(k).indices.int()
+    w = torch.rand(64, k, device=DEV)
+    whole = ops.moe_experts(x, w13, w2, w, ids)
+    for T in sizes:
+        args = x[:T], w13, w2, w[:T], ids[:T]
+        out = ops.moe_experts(*args)
+        assert torch.equal(out, whole[:T]), T
+        assert torch.equal(ops.parts_sum(ops.moe_experts_parts(*args)), out)
+    for up, down in ((2, 2), (2, 4), (4, 2), (4, 4)):
+        out = torch.empty_like(x)
+        ops._native().moe_experts(out, x, w13, w2, w, ids, 0, 32, True, up, down)
+        assert torch.equal(out, whole), (up, down)
+    expect = torch.zeros(64, H, dtype=torch.float64, device=DEV)
+    for e in range(E):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        gu = x[t].double() @ w13[e].double().t()
+        h = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+        expect.index_add_(0, t, h @ w2[e].double().t() * w[t, j, None].double())
+    # as in test_moe_experts
+    assert (whole.double() - expect).norm() <= 3 * 2 ** -8 * expect.norm()
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 64])
 @pytest.mark.parametrize("N", [13320, 32000])
 def test_linear_f32_tiles(M, N):
