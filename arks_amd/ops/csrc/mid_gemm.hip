@@ -276,14 +276,22 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   const int frag = lq * 128 + ((la ^ (lq & 7)) * 16);
   const int w_at = wm * QT * 2048 + frag;
   const int a_at = W_STAGE + wn * FT * 2048 + frag;
-  // Up to 64 rows a chain of sums is 4 steps long, and those of 4 steps are added
-  // up apart: the streamed products, which are the other choice there, add up
-  // the shorter chains of several waves. 64 rows of 4608 x 3584 in 3 runs of K
-  // err by 1.0e-7, in a chain per run by 2.0e-7 (streamed, 7 runs: 1.4e-7); it
-  // takes 1.4 % longer over 60 sizes, in front of the multiplications (2.2 %
-  // behind them). Library products, the other choice beyond, are one chain too.
-  constexpr bool SETTLE = FT <= 2;
-  f32x4 acc[QT][FT], settled[SETTLE ? QT : 1][FT];
+  // Up to 64 rows a chain of sums is 4 steps long, those of 4 steps are added up
+  // apart, and those of 16 steps again (far): the streamed products, which are the
+  // other choice there, add up the shorter chains of several waves, and the error
+  // must not grow with the run of K that a cut gives. Relative to 64 bits, 8 rows,
+  // chains of 4 steps in one chain -> in chains of 16: 5120 x 27648 in 3 runs
+  // 1.45e-7 -> 1.17e-7 (in 8 runs 1.25e-7 before), 3584 x 18944 in 4 1.28e-7 ->
+  // 1.12e-7 (in 8 1.20e-7 before), 10240 x 2048 in one 1.03e-7 -> 1.00e-7 (streamed
+  // 0.98e-7); 64 rows of 4608 x 3584 in 3 runs err by 1.0e-7, in a chain per run by
+  // 2.0e-7.
+  // Chains of 4 steps take 1.4 % longer over 60 sizes with the kernel before this
+  // one, in front of the multiplications (2.2 % behind them); far nothing (45 sizes
+  // at 1 to 48 rows 0.999; as values that are chosen and not as a branch 3 %).
+  // Library products, the other choice beyond, are one chain; there
+  // ops._mid_cut keeps runs short. An expert's items have one run each, as before.
+  constexpr bool SETTLE = FT <= 2, FAR = SETTLE && !ITEMS;
+  f32x4 acc[QT][FT], settled[SETTLE ? QT : 1][FT], far[FAR ? QT : 1][FT];
   // The fragments of the next half step are read while this one's are
   // multiplied: those of w and the last two of a into a second set of
   // registers, the others into the same once they have been used.
@@ -334,6 +342,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
       for (int f = 0; f < FT; ++f) {
         acc[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
         if constexpr (SETTLE) settled[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (FAR) far[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
     for (int s = 0; s < now.steps; ++s) {
       if constexpr (SETTLE) {
@@ -345,6 +354,18 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
               settled[q][f] += acc[q][f];
               acc[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
+          if constexpr (FAR) {
+            if ((s & 15) == 0 && s > 0) {
+              asm volatile("");  // a branch
+#pragma unroll
+              for (int q = 0; q < QT; ++q)
+#pragma unroll
+                for (int f = 0; f < FT; ++f) {
+                  far[q][f] += settled[q][f];
+                  settled[q][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+          }
         }
       }
       half_step(std::integral_constant<int, 0>{});
@@ -360,7 +381,10 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
 #pragma unroll
       for (int q = 0; q < QT; ++q)
 #pragma unroll
-        for (int f = 0; f < FT; ++f) acc[q][f] += settled[q][f];
+        for (int f = 0; f < FT; ++f) {
+          acc[q][f] += settled[q][f];
+          if constexpr (FAR) acc[q][f] += far[q][f];
+        }
     }
     const int n0 = now.n0 + wm * (COLS / 2);
 #pragma unroll

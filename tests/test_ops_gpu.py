@@ -1497,6 +1497,28 @@ def test_moe_items_order_of_sums_by_rows():
     assert (whole.double() - expect).norm() <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("M", [5, 64])
+@pytest.mark.parametrize("qt", [2, 4, 5])
+def test_mid_gemm_error_of_long_runs(M, qt):
+    """Up to 64 rows the error of sums hardly grows with the run of K: 2 runs of
+    130 steps against 8 of 32 or 33, the runs added in 64 bits. A chain of n sums
+    leaves a squared error in proportion to n: 8 products, 4 chains of those and
+    all of these 8 or 2, so sqrt((8 + 4 + 8) / (8 + 4 + 2)) = 1.2 times as much
+    (chains of 8 products and of all of those: 1.6)."""
+    assert_native()
+    torch.manual_seed(M + qt)
+    N, K = 640, 64 * 260
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    expect = x.double() @ w.double().t()
+    err = []
+    for runs in (2, 8):
+        sums = torch.empty(runs, M, N, device=DEV)
+        ops._native().mid_gemm(sums, x, w, None, qt, False)
+        err.append((sums.double().sum(0) - expect).norm().item())
+    assert err[0] <= 1.2 * err[1]
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 64])
 @pytest.mark.parametrize("N", [13320, 32000])
 def test_linear_f32_tiles(M, N):
