@@ -322,6 +322,19 @@ def test_moe_way():
     assert ops._moe_way(7, 4, 16, 16, 2056, 1416, False) == (128, False)
 
 
+def test_mid_cut_runs():
+    """Beyond 64 rows, where a run of K is one chain of sums, the most runs that
+    cost next to nothing; up to 64 rows the least time alone."""
+    from arks_amd import ops
+
+    assert ops._mid_cut(96, 2048, 2048, False, True) == (2, 8)
+    assert ops._mid_cut(96, 5120, 27648, False, True) == (5, 8)
+    assert ops._mid_cut(32, 3584, 18944, False, True) == (2, 4)
+    # not where it costs: one run for tiles that fill the CUs
+    assert ops._mid_cut(96, 32000, 4096, False, False)[1] == 1
+    assert ops._mid_cut(96, 18944, 3584, True, False)[1] == 1
+
+
 def test_moe_few():
     """Items of 32 pairs where their tiles fill the rounds, streamed else."""
     from arks_amd import ops
