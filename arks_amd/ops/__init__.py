@@ -746,7 +746,10 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
             return None
     else:
         few = splits > 1 or fill <= 0.5
-        if (small and few and N <= 8192
+        # (the streamed product takes K beyond 4096 from 2048 columns on; below,
+        # its splits are slower: 896 x 4864, 4 rows 7.3 us here, 8.5, 1536 x 8192
+        # 9.2 and 11.8)
+        if (small and few and N <= 8192 and _stream_sizes(M, N, K)
                 and M <= (16 if K <= 256 and N > 2048 else 64)
                 and (K <= 1536 or M * K <= (65536 if N > 2048 else 32768))):
             return None

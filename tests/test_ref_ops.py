@@ -335,6 +335,22 @@ def test_mid_cut_runs():
     assert ops._mid_cut(96, 18944, 3584, True, False)[1] == 1
 
 
+def test_mid_sizes_leave_to_streamed():
+    """Small weights at up to 64 rows are left to the streamed product only where
+    it takes them."""
+    from arks_amd import ops
+
+    left = 0
+    for M in (1, 2, 4, 6, 8, 16, 32, 64):
+        for N in (128, 512, 896, 1536, 2040, 2048, 4096, 8192):
+            for K in (256, 896, 2048, 4096, 4160, 4864, 8192, 14336):
+                if (N * K <= ops._SKINNY_MAX_ELEMS
+                        and ops._mid_sizes(M, N, K, False, False) is None):
+                    left += 1
+                    assert ops._stream_sizes(M, N, K), (M, N, K)
+    assert left > 50
+
+
 def test_moe_few():
     """Items of 32 pairs where their tiles fill the rounds, streamed else."""
     from arks_amd import ops
