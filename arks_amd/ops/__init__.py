@@ -712,10 +712,11 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
       rows 0.82, 8192 x 2048, 16 rows 1.11, 48 rows 0.71; with the activation
       1920 x 1088 (60 tiles), 5 rows 6.0 (5.6), 4096 x 5120 (half of the CUs)
       the same;
-    - library, sums: 4096 x 2048, 208 rows 1.13 of it; 3584 x 3584, 256 rows
-      1.05, 224 rows 22.3 (23.8); 1152 x 896, 208 rows 1.07; without a consumer 8192 x 2048, 96 rows
-      1.07, 208 rows 1.29, 64 rows 0.85, 4096 x 4096, 208 rows 1.02, 2192 x 896
-      (35 tiles), 100 rows 9.4 (8.3); with the activation 2256 x 2048 (71 tiles),
+    - library, sums: 4096 x 2048, 208 rows 1.13 of it; 193 to 224 rows of
+      3072..3840 x 3072..4096 0.55 to 1.00 (3584 x 3584, 224 rows 22.4 (23.7)), 256
+      rows 0.87 to 1.03, 4096 x 3072, 193 to 224 rows 1.02 to 1.03; 1152 x 896, 208
+      rows 1.07; without a consumer 8192 x 2048, 96 rows 1.07, 208 rows 1.29, 64 rows
+      0.85, 4096 x 4096, 208 rows 1.02, 2192 x 896 (35 tiles), 100 rows 9.4 (8.3); with the activation 2256 x 2048 (71 tiles),
       250 rows 24.5 (19.4);
     - library, whole: 50304 x 2560, whose tiles fill the second round of CUs by
       a quarter, 96 rows 1.15, 64 rows 1.04; gate and up 55296 x 5120, 0.84 full,
@@ -735,7 +736,7 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
             return None
         if N * K < 13_000_000 and K <= 4096 and M > (
                 128 if K <= 1024 or (K <= 2048 and M % 32)
-                else 224 if min(N, K) >= 3072 else 192):
+                else 224 if K >= 3072 and 3072 <= N < 4096 else 192):
             return None
     elif silu:
         if (fill < 0.6 and K >= 4096 and M <= 64

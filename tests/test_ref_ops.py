@@ -351,6 +351,18 @@ def test_mid_sizes_leave_to_streamed():
     assert left > 50
 
 
+def test_mid_sizes_up_to_224_rows():
+    """Sums of up to 224 rows of squares from 3072 on; 4096 columns of 3072 are
+    the library's beyond 192 rows."""
+    from arks_amd import ops
+
+    takes = lambda *size: ops._mid_sizes(*size, False, True) is not None
+    for M in (193, 208, 224):
+        for N, K in ((3072, 3072), (3584, 3584), (3840, 3328), (3072, 4096)):
+            assert takes(M, N, K) and not takes(225, N, K)
+        assert takes(192, 4096, 3072) and not takes(M, 4096, 3072)
+
+
 def test_moe_few():
     """Items of 32 pairs where their tiles fill the rounds, streamed else."""
     from arks_amd import ops
