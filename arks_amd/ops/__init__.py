@@ -455,15 +455,25 @@ def step_decode_plan(seq_lens, num_kv_heads: int, window: int, kv_fp8: bool,
 def decode_waves(num_seqs: int, num_kv_heads: int, kv_fp8: bool = False,
                  num_partitions: int | None = None) -> int:
     """Runs per key/value head that the decode kernel cuts all sequences'
-    pages into (attn_decode.hip). One workgroup of 4 waves per CU (us at 28/4
-    heads x 128: 200 sequences of 20..4000 59.0, with two 60.0; 256 of 100 17.1
-    and 19.9; 256 of 1..4000 178 and 182; 64 x 1024 28.2 and 28.9; counts between
-    6 to 25 % more), two where the rows are half as long (48 fp8 sequences of
-    900..5000 38.9 and 36.3). num_partitions: that many runs per sequence on
-    average instead."""
+    pages into (attn_decode.hip). One workgroup of 4 waves per CU, two where the
+    rows are half as long (fp8) or where there are more sequences than runs, so
+    that a run would hold several short ones. us, kernel and merge, one workgroup
+    per CU (two), lengths even over the logarithm unless said:
+    - up to 1024 (sequence, head) pairs: 28/4 heads x 128: 64 of 1024 30.5 (31.2),
+      200 of 20..4000 60.8 (63.9), 256 of 100 17.0 (20.0); 14/2 x 64: 128 of
+      20..4000 18.4 (20.5), 256 of 1..4000, even, 52.0 (52.4); 32/8 x 64: 100 of
+      20..4000 36.1 (34.2), 128 of 100 11.3 (12.7);
+    - more of them: 32/8 x 128: 256 of 100 31.1 (27.5), 256 of 20..4000 141.5
+      (145.9); 32/8 x 64: 200 of 20..4000 62.1 (59.7), 256 of 20..500 24.6 (21.8);
+      16/16 x 64: 256 of 100 33.1 (27.3);
+    - fp8, 28/4 x 128: 200 of 20..4000 45.9 (42.9), 256 of 1..4000, even, 121.5
+      (108.1).
+    Counts between are 6 to 25 % slower. num_partitions: that many runs per
+    sequence on average instead."""
     if num_partitions is not None:
         return max(1, num_partitions * num_seqs)
-    waves = 2048 if kv_fp8 else 1024
+    many = kv_fp8 or num_seqs * num_kv_heads > 1024
+    waves = 2048 if many else 1024
     return max(1, waves // num_kv_heads)
 
 
@@ -646,10 +656,11 @@ def _mid_cut(M: int, N: int, K: int, silu: bool, summed: bool,
     and read at 5 TB/s, and added by a launch of their own unless the consumer
     does (summed). At most 8 runs, as the consumer's time grows with them. Beyond
     64 rows a run is one chain of sums, whose error grows with it: where K is cut,
-    of the cuts within 4 % of the least time the one with the most runs (error against 64 bits
-    and us, so, and with the least time by the fit: 2048 x 2048, 96 rows, 1.02e-7
-    in 8 runs, 11.3, and 1.32e-7 in 4, 10.8; 5120 x 27648 3.64e-7 in 8, 58.8, and
-    4.24e-7 in 6, 59.7; 288 sizes and numbers of rows take 1.0009 of the time).
+    of the cuts within 4 % of the least time the one with the most runs (error
+    against 64 bits and us, so, and with the least time by the fit: 2048 x 2048, 96
+    rows, 1.02e-7 in 8 runs, 11.3, and 1.32e-7 in 4, 10.8; 5120 x 27648 3.64e-7 in
+    8, 58.8, and 4.24e-7 in 6, 59.7; 288 sizes and numbers of rows take 1.0009 of
+    the time).
     whole: one run."""
     steps, groups = K // 64, -(-M // 32)
     cuts = []
@@ -716,8 +727,8 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
       3072..3840 x 3072..4096 0.55 to 1.00 (3584 x 3584, 224 rows 22.4 (23.7)), 256
       rows 0.87 to 1.03, 4096 x 3072, 193 to 224 rows 1.02 to 1.03; 1152 x 896, 208
       rows 1.07; without a consumer 8192 x 2048, 96 rows 1.07, 208 rows 1.29, 64 rows
-      0.85, 4096 x 4096, 208 rows 1.02, 2192 x 896 (35 tiles), 100 rows 9.4 (8.3); with the activation 2256 x 2048 (71 tiles),
-      250 rows 24.5 (19.4);
+      0.85, 4096 x 4096, 208 rows 1.02, 2192 x 896 (35 tiles), 100 rows 9.4 (8.3);
+      with the activation 2256 x 2048 (71 tiles), 250 rows 24.5 (19.4);
     - library, whole: 50304 x 2560, whose tiles fill the second round of CUs by
       a quarter, 96 rows 1.15, 64 rows 1.04; gate and up 55296 x 5120, 0.84 full,
       96 rows 1.06, 57344 x 8192, 0.875 full, 0.86."""

@@ -322,6 +322,18 @@ def test_moe_way():
     assert ops._moe_way(7, 4, 16, 16, 2056, 1416, False) == (128, False)
 
 
+def test_decode_waves():
+    """Two workgroups per CU for fp8 rows, and where sequences outnumber runs."""
+    from arks_amd import ops
+
+    assert ops.decode_waves(64, 4) == ops.decode_waves(256, 4) == 256
+    assert ops.decode_waves(257, 4) == 512
+    assert ops.decode_waves(128, 8) == 128 and ops.decode_waves(256, 8) == 256
+    assert ops.decode_waves(256, 2) == 512 and ops.decode_waves(80, 16) == 128
+    assert ops.decode_waves(1, 4, True) == 512
+    assert ops.decode_waves(3, 4, False, 5) == 15
+
+
 def test_mid_cut_runs():
     """Beyond 64 rows, where a run of K is one chain of sums, the most runs that
     cost next to nothing; up to 64 rows the least time alone."""
