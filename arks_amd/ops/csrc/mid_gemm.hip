@@ -423,10 +423,17 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
         constexpr uint32_t none = 1u << 31;
         // Past the caches beside the loads of other jobs, from 17 rows on: the
         // output's lines do not push out those of a (152064 x 3584, 64 rows 197
-        // -> 178 us, 32 rows 179 -> 171; 8 rows 163 -> 166). Not sums: whoever
-        // adds them would read them from memory (64 rows x 3584 and their norm
-        // 5.0 -> 5.4 us, 200 rows 7.4 -> 8.5).
-        const bool once = jobs > (int)gridDim.x && now.rows > 16;
+        // -> 178 us, 32 rows 179 -> 171; 8 rows 163 -> 166; 128256 x 2048, 256
+        // rows 152 -> 145). Waves of 80 columns (QT 5) store parts of lines, which
+        // is slower past the caches, so there only as long as the output is little
+        // beside the weights: us, past the caches (not), 151936 x 896, 48 rows 56.9
+        // (56.6), 64 rows 61.6 (59.2), 192 rows 95.2 (86.0); x 2048, 96 rows 124
+        // (129), 192 rows 158 (154); 100352 x 2560, 128 rows 124.7 (125.1), 192
+        // rows 143.7 (139.0); 152064 x 3584, 160 rows 241.7 (240.5), 224 rows 274
+        // (261). Not sums: whoever adds them would read them from memory (64 rows x
+        // 3584 and their norm 5.0 -> 5.4 us, 200 rows 7.4 -> 8.5).
+        const bool once = jobs > (int)gridDim.x && now.rows > 16 &&
+                          (QT % 4 == 0 || now.rows * 19 < k_total);
         const uint32_t size = parts ? 4 : 2;
         const uint32_t even = m0 + (lq & ~1) < now.rows
                                   ? (lq & ~1) * n_total * size : none;
