@@ -730,7 +730,9 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
       0.85, 4096 x 4096, 208 rows 1.02, 2192 x 896 (35 tiles), 100 rows 9.4 (8.3);
       with the activation 2256 x 2048 (71 tiles), 250 rows 24.5 (19.4);
     - library, whole: 50304 x 2560, whose tiles fill the second round of CUs by
-      a quarter, 96 rows 1.15, 64 rows 1.04; gate and up 55296 x 5120, 0.84 full,
+      a quarter, 96 rows 1.15, 64 rows 1.04; 55296 x 5120, 0.84 full, 160 to 224
+      rows 1.10 to 1.14, 50304 x 4096, 0.77 full, 1.06 to 1.10, 128 rows 0.96, 102400
+      x 4096, three rounds 0.83 full, 0.90 to 0.94; gate and up 55296 x 5120, 0.84 full,
       96 rows 1.06, 57344 x 8192, 0.875 full, 0.86."""
     if (K % 64 or N % 8 or not 64 <= K < 1 << 22 or not 0 < N < 1 << 24
             or (silu and 2 * N * K >= 1 << 31)):
@@ -775,7 +777,8 @@ def _mid_sizes(M: int, N: int, K: int, silu: bool, summed: bool):
         if splits == 1 and tiles > 256 and (
                 (fill < 0.8 and M > 64 and (
                     K <= 1024 or (K <= 2048 and M > 192) or 2048 < K <= 3072))
-                or (M > 128 and K >= 8192)):
+                or (M > 128 and (K >= 8192 or (
+                    tiles <= 512 and fill < 0.9 and N * K > 1 << 27)))):
             return None
     return qt, splits
 

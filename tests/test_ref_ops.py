@@ -375,6 +375,20 @@ def test_mid_sizes_up_to_224_rows():
         assert takes(192, 4096, 3072) and not takes(M, 4096, 3072)
 
 
+def test_mid_sizes_of_a_second_round():
+    """Beyond 128 rows large weights whose tiles leave much of a second round of
+    CUs empty are the library's."""
+    from arks_amd import ops
+
+    takes = lambda *size: ops._mid_sizes(*size, False, False) is not None
+    for M in (129, 160, 224):
+        for N, K in ((55296, 5120), (50304, 4096), (43008, 5120)):
+            assert not takes(M, N, K), (M, N, K)
+        for N, K in ((102400, 4096), (36864, 5120), (152064, 3584), (32064, 4096)):
+            assert takes(M, N, K), (M, N, K)
+    assert takes(128, 50304, 4096)
+
+
 def test_moe_few():
     """Items of 32 pairs where their tiles fill the rounds, streamed else."""
     from arks_amd import ops
