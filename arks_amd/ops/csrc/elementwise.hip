@@ -22,6 +22,9 @@ namespace arks {
 // beside them: few rows are bound by the chain of loads, sum and store, many
 // by the bytes. Rows that are longer (NV 0) are read again from L2 behind the
 // sum, as all were before: 64 x 3584 and 4 splits 5.3 us, held 4.9.
+// The arguments fill one line of 64 bytes: a dimension of the grid, which lies
+// behind them, would be one more load in front of the sums' addresses (64 x 3584
+// and 4 splits 3.84 us back to back, with the rows as an argument 3.69).
 // ---------------------------------------------------------------------------
 enum NormInput { IN_ROWS, IN_PARTS, IN_MIX };
 template <bool FUSED_ADD, NormInput IN, int NV>
@@ -30,10 +33,10 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
                                bf16* __restrict__ residual,  // null unless FUSED_ADD
                                const bf16* __restrict__ weight,
                                const float eps, const int hidden,
-                               const int splits,
+                               const int rows,
+                               const int n_in,  // splits, or k of a mix
                                const float* __restrict__ mix_weights,  // [rows, k]
-                               const int* __restrict__ mix_rows,       // [rows, k]
-                               const int mix_k) {
+                               const int* __restrict__ mix_rows) {     // [rows, k]
   constexpr bool PARTS = IN == IN_PARTS;
   constexpr int BLOCK = PARTS ? 512 : 256;
   const int row = blockIdx.x;
@@ -41,7 +44,7 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
       reinterpret_cast<const bf16*>(input) + (int64_t)row * hidden;
   const float* part_row =
       reinterpret_cast<const float*>(input) + (int64_t)row * hidden;
-  const int64_t part_stride = (int64_t)gridDim.x * hidden;
+  const int64_t part_stride = (int64_t)rows * hidden;
   bf16* res_row = FUSED_ADD ? residual + (int64_t)row * hidden : nullptr;
   bf16* out_row = out + (int64_t)row * hidden;
 
@@ -55,14 +58,14 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
     if constexpr (PARTS) {
       f32x4 lo, hi;
       sum_parts_pair(part_row + i * 8, part_row + i * 8 + 4, part_stride,
-                     splits, lo, hi);
+                     n_in, lo, hi);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = j < 4 ? lo[j % 4] : hi[j % 4];
     } else {
       if constexpr (IN == IN_MIX)
         s = mix_rows8(reinterpret_cast<const bf16*>(input),
-                      mix_weights + (int64_t)row * mix_k,
-                      mix_rows + (int64_t)row * mix_k, mix_k, hidden, i * 8);
+                      mix_weights + (int64_t)row * n_in,
+                      mix_rows + (int64_t)row * n_in, n_in, hidden, i * 8);
       else
         s = *reinterpret_cast<const ushort8*>(in_row + i * 8);
 #pragma unroll
@@ -201,7 +204,7 @@ extern "C" {
   hipLaunchKernelGGL((rmsnorm_kernel<FUSED, IN, NV>), dim3(rows),              \
                      dim3(IN == IN_PARTS ? 512 : 256), 0, stream, (bf16*)out,  \
                      input, (bf16*)residual, (const bf16*)weight, eps, hidden, \
-                     splits, (const float*)mix_weights, (const int*)mix_rows, k)
+                     rows, n_in, (const float*)mix_weights, (const int*)mix_rows)
 #define ARKS_NORM_V(FUSED, IN)                                                 \
   do {                                                                         \
     const int block = IN == IN_PARTS ? 512 : 256;                              \
@@ -215,7 +218,7 @@ extern "C" {
 void arks_rmsnorm(void* out, const void* input, const void* weight, float eps,
                   int rows, int hidden, hipStream_t stream) {
   void* const residual = nullptr;
-  const int splits = 0, k = 0;
+  const int n_in = 0;
   const void *const mix_weights = nullptr, *const mix_rows = nullptr;
   ARKS_NORM_V(false, IN_ROWS);
 }
@@ -223,7 +226,7 @@ void arks_rmsnorm(void* out, const void* input, const void* weight, float eps,
 void arks_fused_add_rmsnorm(void* out, const void* input, void* residual,
                             const void* weight, float eps, int rows, int hidden,
                             hipStream_t stream) {
-  const int splits = 0, k = 0;
+  const int n_in = 0;
   const void *const mix_weights = nullptr, *const mix_rows = nullptr;
   ARKS_NORM_V(true, IN_ROWS);
 }
@@ -231,7 +234,7 @@ void arks_fused_add_rmsnorm(void* out, const void* input, void* residual,
 void arks_fused_add_rmsnorm_parts(void* out, const void* input, int splits,
                                   void* residual, const void* weight, float eps,
                                   int rows, int hidden, hipStream_t stream) {
-  const int k = 0;
+  const int n_in = splits;
   const void *const mix_weights = nullptr, *const mix_rows = nullptr;
   ARKS_NORM_V(true, IN_PARTS);
 }
@@ -243,7 +246,7 @@ void arks_fused_add_rmsnorm_mix(void* out, const void* input,
                                 int k, void* residual, const void* weight,
                                 float eps, int rows, int hidden,
                                 hipStream_t stream) {
-  const int splits = 0;
+  const int n_in = k;
   ARKS_NORM_V(true, IN_MIX);
 }
 #undef ARKS_NORM_V
