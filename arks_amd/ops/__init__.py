@@ -1186,15 +1186,17 @@ def _moe_few(rows: int, top_k: int, El: int, experts: int, H: int, I: int,
     kernel is expected to take less (streamed: it is the other choice, else items
     of 64 are). Counted are the tiles of the experts that so many rows touch if
     they choose evenly, in rounds over 256 CUs, a step as in _mid_cut, 1.5 us a
-    round; the streamed kernel at 4 us and 5 TB/s. us with plan and mix, items of 32 as
-    cut here (streamed; items of 64): 128 experts of 2048 x 768, 8 per row: 1 row
-    23.2 (25.7; 30.7), 7 rows 86 (92; 93), 16 rows 142 (146; 146); 8 of 4096 x
+    round; the streamed kernel at 1.5 us and 5.2 TB/s. us with plan and mix, items of
+    32 as cut here (streamed; items of 64): 128 experts of 2048 x 768, 8 per row: 1
+    row 23.2 (25.7; 30.7), 7 rows 86 (92; 93), 16 rows 142 (146; 146); 8 of 4096 x
     14336, 2 per row: 1 row 132 (132; 164), 4 rows 285 (333; 303), 8 rows 381
     (435; 383); 16 of 4096 x 2048, 2 per row: 1 row 34.6 (30.9; 49), 8 rows 106
-    (100; 112). Over 6 sizes at 1 to 32 rows this choice is 1.7 % from the best,
-    streaming 9.2 %."""
+    (100; 112); 32 of 1536 x 512, 4 per row, 6 rows 27.0 (23.9; 28.8), 16 rows 36.8
+    (36.6; 38.6). Over 21 sizes at 1 to 32 rows this choice takes 0.94 of the time
+    without items of 32 and 1.5 % more than the best; 5 of 294 are more than 2 %
+    slower than without (16 of 4096 x 2048, 5 rows 105 (97))."""
     n = max(1, round(El * (1 - (1 - top_k / experts) ** rows)))
-    best = [4 + 6 * H * I * n / 5e6] if streamed else [math.inf]
+    best = [1.5 + 6 * H * I * n / 5.2e6] if streamed else [math.inf]
     best.append(None)
     cost = {}
     for up in (True, False):

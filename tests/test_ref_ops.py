@@ -396,6 +396,9 @@ def test_moe_few():
     assert ops._moe_few(7, 8, 128, 128, 2048, 768, True) == (2, 4)
     assert ops._moe_few(1, 2, 8, 8, 4096, 14336, True) == (4, 2)
     assert ops._moe_few(1, 2, 16, 16, 4096, 2048, True) is None
+    # short columns: what the items win does not pay for their rounds
+    assert ops._moe_few(3, 4, 32, 32, 1536, 512, True) is None
+    assert ops._moe_few(6, 4, 32, 32, 1536, 512, True) is None
     # never streamed where that is not the other choice
     for rows in range(1, 33):
         cut = ops._moe_few(rows, 2, 16, 16, 4096, 2048, False)
