@@ -62,12 +62,17 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = j < 4 ? lo[j % 4] : hi[j % 4];
     } else {
-      if constexpr (IN == IN_MIX)
-        s = mix_rows8(reinterpret_cast<const bf16*>(input),
-                      mix_weights + (int64_t)row * n_in,
-                      mix_rows + (int64_t)row * n_in, n_in, hidden, i * 8);
-      else
+      if constexpr (IN == IN_MIX) {
+        // weights and rows are the same in all lanes: scalar loads, no barrier
+        const float* w = mix_weights + (int64_t)row * n_in;
+        const int* rows_in = mix_rows + (int64_t)row * n_in;
+        s = mix_rows8(
+            reinterpret_cast<const bf16*>(input), n_in, i * 8,
+            [&](int j) { return (int64_t)rows_in[min(j, n_in - 1)] * hidden; },
+            [&](int j) { return j < n_in ? w[min(j, n_in - 1)] : 0.f; });
+      } else {
         s = *reinterpret_cast<const ushort8*>(in_row + i * 8);
+      }
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = bf16_bits_to_float(s[j]);
     }

@@ -50,28 +50,27 @@ __device__ __forceinline__ void sum_parts_pair(const float* p, const float* q,
   }
 }
 
-// The weighted mix of a token's k rows of y [any, H]: weights and rows are the
-// token's own, the same in all lanes (so they come as scalars, without a
-// barrier). 8 columns from h on, in the rows' order, 8 rows' loads in flight;
-// rows of weight 0 count as nothing (they may hold anything).
-__device__ __forceinline__ ushort8 mix_rows8(const bf16* y, const float* weights,
-                                             const int* rows, const int k,
-                                             const int64_t H, const int h) {
+// The weighted mix of a token's k rows of y: 8 columns from h on, in the rows'
+// order, 8 rows' loads in flight. start(j), weight(j) for j up to the next multiple
+// of 8: where row j begins in y, and its weight, 0 from k on; rows of weight 0 count
+// as nothing (they may hold anything).
+template <typename Start, typename Weight>
+__device__ __forceinline__ ushort8 mix_rows8(const bf16* y, const int k, const int h,
+                                             Start start, Weight weight) {
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (int j0 = 0; j0 < k; j0 += 8) {
     ushort8 u[8];
-    float w[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int at = min(j0 + j, k - 1);
-      u[j] = *reinterpret_cast<const ushort8*>(y + rows[at] * H + h);
-      w[j] = j0 + j < k ? weights[at] : 0.f;
-    }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
+      u[j] = *reinterpret_cast<const ushort8*>(y + start(j0 + j) + h);
+    __builtin_amdgcn_sched_barrier(0);  // all 8 are asked for first
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float w = weight(j0 + j);
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        acc[e] += w[j] == 0.f ? 0.f : w[j] * bf16_bits_to_float(u[j][e]);
+        acc[e] += w == 0.f ? 0.f : w * bf16_bits_to_float(u[j][e]);
+    }
   }
   ushort8 o;
 #pragma unroll
