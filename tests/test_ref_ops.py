@@ -403,5 +403,8 @@ def test_moe_few():
     for rows in range(1, 33):
         cut = ops._moe_few(rows, 2, 16, 16, 4096, 2048, False)
         assert cut is None or set(cut) <= {2, 4}
+        assert cut is not None
     # a rank's 16 of 128 experts: less than one of them per row
     assert ops._moe_few(1, 8, 16, 128, 2048, 768, True) in (None, (2, 2))
+    assert ops._moe_few(1, 8, 16, 128, 2048, 768, True) is None
+    assert ops._moe_few(16, 8, 16, 128, 2048, 768, True) == (2, 4)

@@ -684,6 +684,24 @@ def test_moe_wide_rows(T, E, top, W, ff, extra, scaled):
 
 
 @pytest.mark.gpu
+def test_moe_wide_rows_order_of_sums():
+    """A pair's row has the same bits whatever rows share the prompt, in tiles of
+    128 pairs and of 256."""
+    torch.manual_seed(2)
+    E, top, W, ff = 5, 2, 1024, 576
+    h = torch.randn(2000, W, device="cuda").bfloat16()
+    w_gu = (torch.randn(2 * E * ff, W, device="cuda") * W ** -0.5).bfloat16()
+    w_down = (torch.randn(W, E * ff, device="cuda") * ff ** -0.5).bfloat16()
+    ids = torch.rand(2000, E, device="cuda").topk(top).indices.int()
+    weights = torch.rand(2000, top, device="cuda")
+    rows = {}
+    for T in (60, 257, 700, 2000):  # 24, 103, 280 and 800 pairs an expert
+        y, place = ops.moe_wide_rows(h[:T], w_gu, w_down, weights[:T], ids[:T], E, ff)
+        rows[T] = y[place[:60].long()]
+        assert torch.equal(rows[T], rows[60]), T
+
+
+@pytest.mark.gpu
 def test_moe_wide_rows_are_the_layers():
     """A layer's prompt rows through the tiles and through one product per
     expert: the same sums up to their order."""
@@ -697,6 +715,7 @@ def test_moe_wide_rows_are_the_layers():
             torch.nn.init.normal_(p, std=256 ** -0.5)
         h = torch.randn(400, 256, device="cuda").bfloat16()
         with torch.no_grad():
+            assert ops.moe_wide_takes(h, m.w_gu, m.w_down, m.E, m.ff, m.top)
             out, takes = m(h).double(), ops.moe_wide_takes
             ops.moe_wide_takes = lambda *a: False
             try:
