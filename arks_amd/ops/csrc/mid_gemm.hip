@@ -21,10 +21,7 @@
 // 61.8 -> 58.5 us), and 4 waves' loads are faster than 8 waves' (loads of 32 KB
 // of a and 24 KB of weights a step, nothing else: 58 and 70 us in 56 steps).
 //
-// One barrier a step. In front of the barrier of step s the waves that load wait
-// for their loads of step s + 1, and the others for their reads of step s:
-// behind it step s + 1 may be read and the stage of step s be loaded anew (with
-// step s + NS).
+// The ring and its waits: ring.h.
 //
 // us against the kernel before this one (8 waves that load and multiply in
 // turns), weights cold: 37888 x 3584 with the activation, 8 rows 43.4 -> 42.3,
@@ -33,7 +30,7 @@
 // 152064 x 3584, 64 rows 201 -> 180, 208 rows 270 -> 251.
 #include <type_traits>
 #include "parts.h"
-#include "tile_engine.h"
+#include "ring.h"
 
 namespace arks {
 
@@ -60,17 +57,6 @@ struct MidItems {
   int expert_base;  // number of the first of these experts among all ranks'
 };
 
-// 1 KB of 8 rows into LDS, 16 B a lane, from step s of its offset. The weights
-// are read once and pass the caches by (non-temporal): 64 rows x 37888 x 3584
-// 51 -> 45 us, the rows of a stay there.
-template <bool ONCE>
-__device__ __forceinline__ void mid_load(const __amdgpu_buffer_rsrc_t& b,
-                                         char* to, const uint32_t offset,
-                                         const int s) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      b, (__attribute__((address_space(3))) char*)to, 16, offset,
-      s * (TILE_K * 2), 0, ONCE ? 2 : 0);
-}
 // Lanes of neighbouring rows swap x of the odd row against y of the even one:
 // a store then covers twice the columns of half the rows, whole lines.
 template <typename V>
@@ -102,16 +88,6 @@ __device__ __forceinline__ void mid_store(const __amdgpu_buffer_rsrc_t& to,
   else __builtin_amdgcn_raw_buffer_store_b64(v, to, offset, 0, 0);
 }
 
-template <int N>
-__device__ __forceinline__ void mid_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void mid_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // ITEMS: the experts that rows chose. Jobs are (item, tile), an item being up to
 // 32 * FT pairs of one expert, whose weights are so read once; workgroups go
 // through them in turn (64 rows of 128 experts of 2048 x 768, 8 per row: gate and
@@ -131,7 +107,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   constexpr int W_ROWS = 32 * QT, COLS = SILU ? W_ROWS / 2 : W_ROWS;
   constexpr int W_STAGE = W_ROWS * 128, STAGE = W_STAGE + 32 * FT * 128;
   constexpr int LOADS = QT + FT;  // of a step, of a wave that loads
-  static_assert(NS >= 3 && (NS - 1) * LOADS < 64, "waits count to 63");
+  static_assert(NS >= 3);
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
   const int lane = threadIdx.x % WAVE_SIZE, lq = lane % 16, la = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
@@ -232,9 +208,10 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
       char* to = lds + stage * STAGE + own * 1024;
 #pragma unroll
       for (int i = 0; i < FT; ++i)
-        mid_load<false>(ab, to + W_STAGE + i * 4096, ao[i], at);
+        ring_load<false>(ab, to + W_STAGE + i * 4096, ao[i], at * (TILE_K * 2));
 #pragma unroll
-      for (int i = 0; i < QT; ++i) mid_load<true>(wb, to + i * 4096, wo[i], at);
+      for (int i = 0; i < QT; ++i)
+        ring_load<true>(wb, to + i * 4096, wo[i], at * (TILE_K * 2));
       stage = stage == NS - 1 ? 0 : stage + 1;
       if (++s == b.steps) {
         s = 0;
@@ -245,29 +222,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
         }
       }
     };
-    // the loads of all but the newest n steps are there
-    auto wait = [&](const int n) {
-      if (n >= NS - 1) mid_wait<(NS - 1) * LOADS>();
-      else if (n == 4) mid_wait<(NS > 5 ? 4 : 0) * LOADS>();
-      else if (n == 3) mid_wait<(NS > 4 ? 3 : 0) * LOADS>();
-      else if (n == 2) mid_wait<(NS > 3 ? 2 : 0) * LOADS>();
-      else if (n == 1) mid_wait<LOADS>();
-      else mid_wait<0>();
-    };
-    const int first = min(NS, total);
-    for (int t = 0; t < first; ++t) load();
-    wait(first - 1);
-    mid_barrier();
-    int t = 0;
-    for (; t + NS < total; ++t) {
-      mid_wait<(NS - 2) * LOADS>();
-      mid_barrier();
-      load();
-    }
-    for (; t < total; ++t) {
-      wait(max(0, total - 2 - t));
-      mid_barrier();
-    }
+    ring_feed<NS, LOADS>(total, load, [](int) {});
     return;
   }
 
@@ -330,7 +285,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   };
   int j = blockIdx.x;  // grid <= jobs
   Job now = job(j);
-  mid_barrier();
+  ring_barrier();
   for (;;) {
 #pragma unroll
   for (int q = 0; q < QT; ++q) read_w(0, q);
@@ -371,7 +326,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
       half_step(std::integral_constant<int, 0>{});
       // this step has been read, the next one is there
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      mid_barrier();
+      ring_barrier();
       at = at == NS - 1 ? 0 : at + 1;
       half_step(std::integral_constant<int, 1>{});
     }

@@ -2,9 +2,8 @@
 // experts that rows chose, with their activation, and the down product over
 // those experts' columns. Experts that no row chose are not read.
 //
-// What bounds them is the weights' stream. 4 waves multiply and 4 only load, as
-// in mid_gemm.hip, whose stages, waits and barriers these are: rows go from
-// memory straight into LDS, NS steps ahead.
+// What bounds them is the weights' stream. 4 waves multiply and 4 only load, NS
+// steps ahead (ring.h).
 //
 // The order of sums is the same for any number of rows: K is cut into chunks of
 // CHUNK columns, a chunk into 4 parts, and wave p adds up part p of every chunk in
@@ -22,8 +21,8 @@
 // (82), 87 (114).
 #include <type_traits>
 
+#include "ring.h"
 #include "seq_common.h"
-#include "tile_engine.h"
 
 namespace arks {
 
@@ -32,26 +31,6 @@ struct RoutedAct {
   int clamped;   // min(g, l) sigmoid(alpha g) (clamp(u, -l, l) + 1)
   float limit, alpha;
 };
-
-// 1 KB of 8 rows into LDS, 16 B a lane, `at` bytes behind its offset; weights are
-// read once and pass the caches by.
-template <bool ONCE>
-__device__ __forceinline__ void routed_load(const __amdgpu_buffer_rsrc_t& b,
-                                            char* to, const uint32_t offset,
-                                            const int at) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      b, (__attribute__((address_space(3))) char*)to, 16, offset, at, 0,
-      ONCE ? 2 : 0);
-}
-template <int N>
-__device__ __forceinline__ void routed_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void routed_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
 
 // Stages of LDS: what fits beside the sums that waves hand over, at most 8.
 constexpr int routed_stages(int qt) {
@@ -74,7 +53,7 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
   constexpr int LOADS = 2 * QT + 2;
   constexpr int COLS = UP ? 8 * QT : 16 * QT;
   constexpr int CHUNK = UP ? 512 : 1024, OWN = CHUNK / 4;  // columns; of a wave
-  static_assert(NS >= 3 && (NS - 1) * LOADS < 64 && (!UP || QT % 2 == 0));
+  static_assert(NS >= 3 && (!UP || QT % 2 == 0));
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE];
   __shared__ tile_f32x4 sums[4][QT][WAVE_SIZE];
   const int lane = threadIdx.x % WAVE_SIZE, lq = lane % 16, la = lane / 16;
@@ -177,10 +156,10 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
       char* to = lds + stage * STAGE + p * PART;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        routed_load<false>(xb, to + QT * 2048 + i * 1024, xo[i], col * 2);
+        ring_load<false>(xb, to + QT * 2048 + i * 1024, xo[i], col * 2);
 #pragma unroll
       for (int i = 0; i < 2 * QT; ++i)
-        routed_load<true>(wb, to + i * 1024, wo[i], col * 2);
+        ring_load<true>(wb, to + i * 1024, wo[i], col * 2);
       stage = stage == NS - 1 ? 0 : stage + 1;
       if (++s == steps) {
         s = 0;
@@ -194,39 +173,20 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
         }
       }
     };
-    // the loads of all but the newest n steps are there
-    auto wait = [&](const int n) {
-      if (n >= NS - 1) routed_wait<(NS - 1) * LOADS>();
-      else if (n == 6) routed_wait<(NS > 7 ? 6 : 0) * LOADS>();
-      else if (n == 5) routed_wait<(NS > 6 ? 5 : 0) * LOADS>();
-      else if (n == 4) routed_wait<(NS > 5 ? 4 : 0) * LOADS>();
-      else if (n == 3) routed_wait<(NS > 4 ? 3 : 0) * LOADS>();
-      else if (n == 2) routed_wait<(NS > 3 ? 2 : 0) * LOADS>();
-      else if (n == 1) routed_wait<LOADS>();
-      else routed_wait<0>();
-    };
-    const int first = min(NS, total);
-    for (int t = 0; t < first; ++t) load();
-    wait(first - 1);
-    routed_barrier();
     int end = steps;  // of the job that is multiplied
-    for (int t = 0; t < total; ++t) {
-      if (t + NS < total) routed_wait<(NS - 2) * LOADS>();
-      else wait(max(0, total - 2 - t));
-      routed_barrier();
-      if (t + NS < total) load();
+    ring_feed<NS, LOADS>(total, load, [&](const int t) {
       if (t + 1 == end) {  // the sums are handed over
-        routed_barrier();
+        ring_barrier();
         end += steps;
       }
-    }
+    });
     return;
   }
 
   // where a step's operands lie: 16 rows of 128 B, pieces permuted
   const int frag = lq * 128 + ((la ^ (lq & 7)) * 16);
   int at = 0;  // the stage that is read
-  routed_barrier();
+  ring_barrier();
   for (int j = blockIdx.x; j < jobs; j += gridDim.x) {
     const Job b = job(j);
     tile_f32x4 acc[QT];
@@ -244,7 +204,7 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
       }
       // this step has been read, the next one is there
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      routed_barrier();
+      ring_barrier();
       at = at == NS - 1 ? 0 : at + 1;
       if (UP || s < own_steps) {
 #pragma unroll
@@ -257,7 +217,7 @@ __global__ __launch_bounds__(512, 2) void routed_gemm_kernel(
 #pragma unroll
     for (int q = 0; q < QT; ++q) sums[p][q][lane] = acc[q];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    routed_barrier();
+    ring_barrier();
     auto sum = [&](const int q) {
       tile_f32x4 v = sums[0][q][lane];
 #pragma unroll
