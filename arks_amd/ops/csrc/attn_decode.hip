@@ -30,8 +30,8 @@
 // 2 workgroups per CU, and less at counts between. 28/4 heads x 128, kernel
 // and merge, with a workgroup per (sequence, head, part of the grid) before:
 //   64 x 1024, bf16            34.4 -> 31.4 us
-//   256 of 1..4000, bf16      108.9 -> 74.2 us (two workgroups per CU, all
-//                              units alike; starts counted, one: 3 % less)
+//   256 of 1..4000, even, bf16   176 us (5.7 TB/s; units all alike and two
+//                              workgroups per CU 183)
 //   48 x 900..5000, fp8       140.8 -> 33.3 us (its bytes were converted one
 //                              by one, in front of the wait for the next)
 //

@@ -27,7 +27,7 @@
 // turns), weights cold: 37888 x 3584 with the activation, 8 rows 43.4 -> 42.3,
 // 200 rows 63.5 -> 59.5; 3584 x 18944 in 8 runs of K, 64 rows 26.1 -> 25.3, 200
 // rows 41.2 -> 37.5; 4608 x 3584 in 4, 8 rows 12.7 -> 9.7, 64 rows 14.5 -> 13.1;
-// 152064 x 3584, 64 rows 201 -> 180, 208 rows 270 -> 251.
+// 152064 x 3584, 64 rows 201 -> 180, 200 rows 264 -> 247.
 #include <type_traits>
 #include "parts.h"
 #include "ring.h"
@@ -240,9 +240,8 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   // 1.12e-7 (in 8 1.20e-7 before), 10240 x 2048 in one 1.03e-7 -> 1.00e-7 (streamed
   // 0.98e-7); 64 rows of 4608 x 3584 in 3 runs err by 1.0e-7, in a chain per run by
   // 2.0e-7.
-  // Chains of 4 steps take 1.4 % longer over 60 sizes with the kernel before this
-  // one, in front of the multiplications (2.2 % behind them); far nothing (45 sizes
-  // at 1 to 48 rows 0.999; as values that are chosen and not as a branch 3 %).
+  // Both together take 0.3 % longer than one chain over 100 sizes and numbers of rows
+  // (far as values that are chosen, and not as a branch, 3 %).
   // Library products, the other choice beyond, are one chain; there
   // ops._mid_cut keeps runs short. An expert's items have one run each, as before.
   constexpr bool SETTLE = FT <= 2, FAR = SETTLE && !ITEMS;
