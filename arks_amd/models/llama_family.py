@@ -108,7 +108,8 @@ class Attention(nn.Module):
             q = ops.rope_and_cache_parts(
                 batch.positions, qkv, kv_cache[0], kv_cache[1],
                 batch.slot_mapping, self._cos_sin, self.head_dim, **norms)
-            return self._out(self._decode(q, batch, kv_cache).view(T, -1), parts)
+            return self._out(self._decode(q, batch, kv_cache).view(T, -1), batch,
+                             parts)
         # Strided views into the fused QKV buffer — RoPE/cache/attention
         # kernels take row strides, so no .contiguous() copies on the hot path.
         q, k, v = self.qkv_proj.split_qkv(qkv)
@@ -157,10 +158,12 @@ class Attention(nn.Module):
                 )
         else:
             out = self._decode(q, batch, kv_cache)
-        return self._out(out.view(T, -1), parts)
+        return self._out(out.view(T, -1), batch, parts)
 
-    def _out(self, x, parts: bool):
-        return self.o_proj(x, parts=True) if parts else self.o_proj(x)
+    def _out(self, x, batch: ForwardBatch, parts: bool):
+        if not parts:
+            return self.o_proj(x)
+        return self.o_proj(x, parts=True, own_cut=not batch.is_prefill)
 
     def _decode(self, q, batch: ForwardBatch, kv_cache):
         k_cache, v_cache = kv_cache
@@ -185,7 +188,8 @@ class MLP(nn.Module):
 
     fp8 = False
 
-    def forward(self, x, parts: bool = False):
+    def forward(self, x, parts: bool = False, own_cut: bool = True):
+        """parts: the caller takes ops.Parts too (own_cut as ops.linear_parts)."""
         if self.fp8:
             return self.down_proj(ops.silu_mul_fp8(self.gate_up_proj(x)))
         if (isinstance(x, tuple) or self.gate_up_proj.fp8
@@ -193,7 +197,9 @@ class MLP(nn.Module):
             h = ops.silu_mul(self.gate_up_proj(x))
         else:
             h = ops.linear_silu_mul(x, self.gate_up_proj.weight)
-        return self.down_proj(h, parts=True) if parts else self.down_proj(h)
+        if not parts:
+            return self.down_proj(h)
+        return self.down_proj(h, parts=True, own_cut=own_cut)
 
 
 class MoEMLP(nn.Module):
@@ -302,9 +308,9 @@ class DecoderLayer(nn.Module):
             x = self.input_layernorm(x)
         else:
             x, residual = self.input_layernorm(x, residual)
-        # the norm behind a row-parallel product of a decode step can add its
-        # split sums; what a hook may look at stays a tensor
-        if (not batch.is_prefill and passable(self.self_attn, Attention)
+        # the norm behind a row-parallel product can add its split sums; what a
+        # hook may look at stays a tensor
+        if (passable(self.self_attn, Attention)
                 and passable(self.self_attn.o_proj, RowParallelLinear)
                 and passable(self.post_attention_layernorm, RMSNorm)):
             x = self.self_attn(x, batch, kv_cache, parts=True)
@@ -313,9 +319,10 @@ class DecoderLayer(nn.Module):
         x, residual = self.post_attention_layernorm(x, residual)
         if parts and passable(self.mlp, MoEMLP):
             return self.mlp(x, parts=True), residual
-        if (parts and not batch.is_prefill and passable(self.mlp, MLP)
+        if (parts and passable(self.mlp, MLP)
                 and passable(self.mlp.down_proj, RowParallelLinear)):
-            return self.mlp(x, parts=True), residual
+            return (self.mlp(x, parts=True, own_cut=not batch.is_prefill),
+                    residual)
         return self.mlp(x), residual
 
 

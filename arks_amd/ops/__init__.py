@@ -848,14 +848,122 @@ def _stream_gemm(x, weight, bias=None, dtype=None, silu: bool = False):
     return out
 
 
-def linear_parts(x, weight, bias=None):
-    """linear_bf16 for a consumer that takes Parts."""
-    cut = _mid(x, weight, bias, summed=True)
+# Tiles of wide_gemm.hip (rows of a x rows of w): us of a step of 64 columns
+# where all CUs are busy. Other combinations of 128, 192, 256 and 320 give less
+# than 0.1 % over 1500 sizes.
+_WIDE_STEP = {(128, 256): 0.92, (192, 256): 1.16, (256, 128): 0.89,
+              (256, 192): 1.11, (256, 256): 1.33, (256, 320): 1.59,
+              (320, 128): 1.03, (320, 256): 1.56}
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_cut(M: int, N: int, K: int, split: bool, summed: bool):
+    """(rows of a, rows of w, runs of K, workgroups) of a wide_gemm, w [N, K]:
+    the tiles and runs that finish first by a fit of what 15 sizes took at 257 to
+    8192 rows with every tile and cut (the chosen ones are 0.7 % from the best on
+    average). A round over the CUs takes its steps and the end of a tile; the
+    last, when fewer CUs run, somewhat less. fp32 sums are written (0.12 us / MB)
+    and read again (0.15), by a launch of their own unless the consumer adds them
+    (summed). split: K may be cut."""
+    best, steps = None, K // 64
+    for (tm, tw), step in _WIDE_STEP.items():
+        tiles = -(-M // tm) * -(-N // tw)
+        for splits in range(1, max(1, min(16, steps // 4) if split else 1) + 1):
+            jobs = tiles * splits
+            if splits > 1 and splits * M * N > 1 << 25:
+                break  # 128 MB of sums
+            most = max(jobs * (x + 1) // 8 - jobs * x // 8 for x in range(8))
+            rounds, last = -(-most // 32), ((most - 1) % 32 + 1) / 32
+            one = -(-steps // splits) * step + 6.0 * tm * tw / 65536
+            us = 3.2 + one * (rounds - 0.22 * (1.0 - last))
+            if splits > 1:
+                us += splits * M * N * 1.08e-6 + (0.0 if summed else 4.0)
+            if best is None or us < best[0]:
+                best = us, tm, tw, splits, jobs
+    return best[1:]
+
+
+def _wide_takes(x, weight, bias=None) -> bool:
+    """Whether wide_gemm can take these tensors, of more rows than mid_gemm."""
+    return (_USE_SKINNY and x.is_cuda and x.dim() == 2
+            and 256 < x.shape[0] < 1 << 24
+            and x.dtype == weight.dtype == torch.bfloat16
+            and weight.shape[1] % 64 == 0 and weight.shape[0] % 16 == 0
+            and 64 <= weight.shape[1] < 1 << 22
+            and 0 < weight.shape[0] < 1 << 24
+            and x.stride(0) < 1 << 22 and _plain(x, weight, bias)
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == x.dtype
+                                  and bias.shape == weight.shape[:1]
+                                  and bias.is_contiguous()))
+            and native_available())
+
+
+def _wide(x, weight, bias=None, summed: bool = False):
+    """(rows of a, rows of w, runs of K) if x weight^T takes wide_gemm, else
+    None: more than 256 rows of long weights. The library's kernels there turn
+    with the row count, and do not cut K as finely as a few hundred rows need. us,
+    here with a launch for the sums (library): 3584 x 18944, 300 rows 60 (101),
+    432 rows 75 (198), 700 rows 97 (165), 1309 rows 164 (256), 1691 rows 201
+    (228), 2314 rows 267 (485), 3344 rows 367 (328), 4666 rows 456 (876); 4096 x
+    14336, 300 rows 55 (76), 1549 rows 151 (329), 1972 rows 196 (188); 4096 x
+    8192, 300 rows 39 (47), 763 rows 60 (59), 1594 rows 101 (100), 4949 rows 225
+    (256); 1024 x 16384, 450 rows 31 (46). Many whole tiles of rows are what the
+    library does best: 3584 x 18944, 8192 rows 806 (740). With K up to 4096 a run
+    has few steps: 4096 x 4096, 491 rows 32 (30), 1159 rows 51 (44)."""
+    if not _wide_takes(x, weight, bias):
+        return None
+    M, (N, K) = x.shape[0], weight.shape
+    if K < 8192 or N < 1024 or (M >= 4096 and M % 256 == 0):
+        return None
+    return _wide_cut(M, N, K, True, summed)[:3]
+
+
+def _wide_silu(x, weight):
+    """(rows of a, rows of w) if silu_mul(x weight^T) takes wide_gemm, the
+    activation inside, else None: more than 256 rows, where at least half of the
+    CUs get a tile (fewer: 4096 x 2048, 600 rows 31 us, library and activation
+    23). us, here (library and activation; tiles of 256 alone): 37888 x 3584, 300
+    rows 97 (121; 131), 400 rows 104 (144; 157), 600 rows 154 (168; 162), 1000
+    rows 194 (316; 236), 2048 rows 384 (416; 396), 3150 rows 607 (809; 677), 8192
+    rows 1520 (1663; 1599); 28672 x 4096, 600 rows 109 (136; 151); 12288 x 2048,
+    1280 rows 50 (61; 60)."""
+    if not _wide_takes(x, weight):
+        return None
+    N, K = weight.shape
+    if (N // 2 + 320) * K >= 1 << 31:  # a tile's rows lie 4 GiB apart
+        return None
+    tm, tw, _, jobs = _wide_cut(x.shape[0], N, K, False, False)
+    return (tm, tw) if jobs >= 128 else None
+
+
+def _wide_gemm(x, weight, bias, cut, summed: bool = False):
+    """A product by wide_gemm: a tensor, or Parts where K is cut or the consumer
+    adds sums (summed)."""
+    (tm, tw, splits), M, N = cut, x.shape[0], weight.shape[0]
+    if splits > 1:
+        sums = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
+        _native().wide_gemm(sums, _rows_16b(x), weight, None, tm, tw, False)
+        parts = Parts(sums, bias)
+        return parts if summed else parts_sum(parts)
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    _native().wide_gemm(out, _rows_16b(x), weight, bias, tm, tw, False)
+    return out
+
+
+def linear_parts(x, weight, bias=None, own_cut: bool = True):
+    """linear_bf16 for a consumer that takes Parts. own_cut: up to 256 rows K is
+    cut with that in mind; else as linear_bf16 does, so that a prompt's rows have
+    the order of sums that they have without a consumer."""
+    cut = _mid(x, weight, bias, summed=own_cut)
     if cut is not None:
-        return _mid_gemm(x, weight, bias, cut, summed=True)
-    if (x.dim() == 2 and not _streams(x, weight, bias=bias)
-            and _splits(x, weight, bias)):
+        return _mid_gemm(x, weight, bias, cut, summed=own_cut or cut[1] > 1)
+    if own_cut and (x.dim() == 2 and not _streams(x, weight, bias=bias)
+                    and _splits(x, weight, bias)):
         return Parts(_stream_parts(x, weight), bias)
+    cut = _wide(x, weight, bias, summed=True)
+    if cut is not None:
+        return _wide_gemm(x, weight, bias, cut, summed=True)
     return linear_bf16(x, weight, bias)
 
 
@@ -870,6 +978,9 @@ def linear_bf16(x, weight, bias=None):
         return _stream_gemm(x, weight, bias)
     if x.dim() == 2 and _splits(x, weight, bias):
         return parts_sum(Parts(_stream_parts(x, weight), bias))
+    cut = _wide(x, weight, bias)
+    if cut is not None:
+        return _wide_gemm(x, weight, bias, cut)
     import torch.nn.functional as F
 
     return F.linear(x, weight, bias)
@@ -1033,6 +1144,11 @@ def linear_silu_mul(x, weight):
             return _mid_gemm(x, weight, None, cut, silu=True)
         if _streams(x, weight, True):
             return _stream_gemm(x, weight, silu=True)
+        tile = _wide_silu(x, weight)
+        if tile is not None:
+            out = x.new_empty((x.shape[0], weight.shape[0] // 2))
+            _native().wide_gemm(out, _rows_16b(x), weight, None, *tile, True)
+            return out
         if _tiles(x, weight):
             out = x.new_empty((x.shape[0], weight.shape[0] // 2))
             _native().tile_silu(out, _rows_16b(x), weight)

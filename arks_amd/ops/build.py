@@ -32,6 +32,7 @@ SOURCES = [
     os.path.join(CSRC, "moe_gemm.hip"),
     os.path.join(CSRC, "stream_gemm.hip"),
     os.path.join(CSRC, "tile_gemm.hip"),
+    os.path.join(CSRC, "wide_gemm.hip"),
     os.path.join(CSRC, "mid_gemm.hip"),
     os.path.join(CSRC, "allreduce.hip"),
 ]

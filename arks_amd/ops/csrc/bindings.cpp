@@ -94,6 +94,9 @@ void arks_stream_sum(void* out, const void* part, const void* bias, int64_t m,
                      int n, int splits, hipStream_t stream);
 void arks_tile_silu(void* out, const void* a, const void* w, int m, int n,
                     int k, int64_t a_stride, hipStream_t stream);
+int arks_wide_gemm(void* out, const void* a, const void* w, const void* bias,
+                   int m, int n, int k, int64_t a_stride, int tm, int tw,
+                   int splits, int kind, hipStream_t stream);
 void arks_mid_gemm(void* out, const void* a, const void* w, const void* bias,
                    int m, int n, int k, int64_t a_stride, int qt, int splits,
                    int parts, int silu, hipStream_t stream);
@@ -669,6 +672,43 @@ void tile_silu(torch::Tensor out, torch::Tensor a, torch::Tensor w) {
                  (int)K, a.stride(0), current_stream());
 }
 
+// out [M, N] = a w^T (+ bias), bf16, or fp32 [splits, M, N] its sums over runs of
+// K; silu: silu(gate) * up of w [2N, K]; tiles of tm rows of a x tw of w
+// (wide_gemm.hip)
+void wide_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
+               c10::optional<torch::Tensor> bias, int64_t tm, int64_t tw,
+               bool silu) {
+  const bool parts = out.dim() == 3;
+  check_bf16_rowstrided(a, "a");
+  check_bf16_contig(w, "w");
+  if (parts) check_parts(out);
+  else check_bf16_contig(out, "out");
+  TORCH_CHECK((parts || out.dim() == 2) && a.dim() == 2 && w.dim() == 2);
+  check_rows_16b(out, "out");
+  check_rows_16b(a, "a");
+  check_rows_16b(w, "w");
+  const int64_t M = a.size(0), K = a.size(1), splits = parts ? out.size(0) : 1;
+  const int64_t N = silu ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(w.size(1) == K && w.size(0) == (silu ? 2 * N : N) &&
+              out.size(out.dim() - 2) == M && out.size(out.dim() - 1) == N);
+  TORCH_CHECK(K >= 64 && K % 64 == 0 && N % 8 == 0 && M < (1 << 24) &&
+                  N < (1 << 24) && K < (1 << 22) && a.stride(0) < (1 << 22) &&
+                  (!silu || (N + 320) * K < ((int64_t)1 << 31)),
+              "need K % 64 == 0, N % 8 == 0");
+  TORCH_CHECK(splits >= 1 && splits <= K / 64 && splits <= 64 && !(parts && silu));
+  if (bias.has_value()) {
+    check_bf16_contig(*bias, "bias");
+    TORCH_CHECK(bias->numel() == N && !silu && !parts);
+  }
+  if (M == 0 || N == 0) return;
+  TORCH_CHECK(arks_wide_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(),
+                             bias.has_value() ? bias->data_ptr() : nullptr,
+                             (int)M, (int)N, (int)K, a.stride(0), (int)tm,
+                             (int)tw, (int)splits, parts ? 1 : silu ? 2 : 0,
+                             current_stream()),
+              "no tile of this size");
+}
+
 // out [M, N] = a w^T (+ bias), bf16, or fp32 [splits, M, N] its sums over runs
 // of K; silu: silu(gate) * up of w [2N, K] (mid_gemm.hip)
 void mid_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
@@ -987,6 +1027,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("a"), pybind11::arg("w"), pybind11::arg("per") = 0);
   m.def("stream_sum", &stream_sum);
   m.def("tile_silu", &tile_silu);
+  m.def("wide_gemm", &wide_gemm);
   m.def("mid_gemm", &mid_gemm);
   m.def("stage_rows", &stage_rows);
   m.def("moe_expert_rows", &moe_expert_rows);

@@ -1,5 +1,6 @@
 // out[M, N] = silu(a w_gate^T) * (a w_up^T) for many rows, w [2N, K] the gate
-// rows, then the up rows: the product of tile_engine.h with a tile's two
+// rows, then the up rows, where these lie beyond the 32-bit offsets of
+// wide_gemm.hip (from 2^31 gate elements on; it is faster below): the product of tile_engine.h with a tile's two
 // halves of w as 128 gate rows and their up rows, so that the activation is
 // taken on the fp32 sums and neither product travels through memory. 18944 x
 // 3584: 8192 rows 1511 us (1473 TFLOP/s; a library product and the activation

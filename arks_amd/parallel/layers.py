@@ -203,8 +203,9 @@ class RowParallelLinear(nn.Module):
 
     fp8 = False
 
-    def forward(self, x, parts: bool = False):
-        """parts: the caller takes ops.Parts too (one rank, no bias)."""
+    def forward(self, x, parts: bool = False, own_cut: bool = True):
+        """parts: the caller takes ops.Parts too (one rank, no bias; own_cut as
+        ops.linear_parts)."""
         if isinstance(x, tuple) or self.fp8:
             bias = self.bias
             self.bias = None  # bias must be applied post-reduce, once
@@ -217,7 +218,7 @@ class RowParallelLinear(nn.Module):
             from .. import ops
 
             if parts and get_tp_world_size() == 1 and self.bias is None:
-                return ops.linear_parts(x, self.weight)
+                return ops.linear_parts(x, self.weight, own_cut=own_cut)
             y = ops.linear_bf16(x, self.weight)
         y = tp_all_reduce(y)
         if self.bias is not None:

@@ -1633,6 +1633,83 @@ def test_mid_gemm(M, N, K, qt, splits, kind):
             <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("M,N,K,splits", [
+    (1, 8, 64, 1), (129, 136, 128, 2), (257, 328, 192, 3), (320, 72, 320, 2),
+    # workgroups that go from tile to tile, of one step and of several
+    (2404, 8200, 64, 1), (2570, 4104, 192, 2), (700, 8000, 448, 3),
+])
+@pytest.mark.parametrize("tm,tw", sorted(ops._WIDE_STEP))
+@pytest.mark.parametrize("kind", ["bias", "sums", "silu"])
+def test_wide_gemm(M, N, K, splits, tm, tw, kind):
+    """Every tile vs fp64: ends of tiles in both directions, one step of K to
+    seven, runs of K, strided rows, nothing behind the last row."""
+    assert_native()
+    torch.manual_seed(M + N + K)
+    silu = kind == "silu"
+    x = torch.randn(M, 2 * K, dtype=torch.bfloat16, device=DEV)[:, :K]
+    w = (torch.randn(2 * N if silu else N, K, device=DEV) * K ** -0.5).bfloat16()
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV) if kind == "bias" else None
+    if kind == "sums":
+        buf = torch.full((splits + 1, M, N), 7.0, device=DEV)
+        out = buf[:splits]
+    else:
+        buf = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
+        out = buf[:M]
+    ops._native().wide_gemm(out, x, w, b, tm, tw, silu)
+    assert (buf[-1] == 7.0).all()
+    xd, wd = x.double(), w.double()
+    expect = xd @ wd.t()
+    # as in test_mid_gemm: fp32 sums within K * 2^-24 of sum |x w|
+    slack = K * 2 ** -24 * (xd.abs() @ wd.abs().t())
+    if kind == "sums":
+        ends = [K // 64 * i // splits * 64 for i in range(splits + 1)]
+        for i, (lo, hi) in enumerate(zip(ends, ends[1:])):
+            run = xd[:, lo:hi] @ wd[:, lo:hi].t()
+            assert ((out[i].double() - run).abs() <= slack).all()
+        return
+    if silu:
+        g, u, sg, su = expect[:, :N], expect[:, N:], slack[:, :N], slack[:, N:]
+        expect = torch.nn.functional.silu(g) * u
+        slack = 1.1 * sg * u.abs() + g.abs() * su + 2 ** -19 * expect.abs()
+    else:
+        expect = expect + b.double()
+    assert ((out.double() - expect).abs()
+            <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
+
+
+def test_wide_rule():
+    """More than 256 rows of long weights, and gate and up products of any K that
+    give half of the CUs a tile; what it cannot take goes on to the library, and
+    the sums reach a norm as they are."""
+    assert_native()
+    w = torch.randn(2048, 8192, device=DEV).mul_(8192 ** -0.5).bfloat16()
+    x = torch.randn(700, 8192, device=DEV).bfloat16()
+    assert ops._wide(x[:257], w) and not ops._wide(x[:256], w)
+    assert not ops._wide(x[:, :4096], w[:, :4096].contiguous())
+    assert not ops._wide(x.float(), w) and not ops._wide(x, w.clone().requires_grad_())
+    assert not ops._wide(x, w, torch.ones(1, dtype=torch.bfloat16, device=DEV))
+    many = x[:1].expand(4097, -1)
+    assert ops._wide(many, w) and not ops._wide(many[:4096], w)
+    gated = torch.empty(16384, 64, dtype=torch.bfloat16, device=DEV)
+    assert ops._wide_silu(x[:300, :64], gated)
+    assert ops._wide_silu(x[:300, :64], gated[:4096]) is None  # few tiles
+    bias = torch.randn(2048, device=DEV).bfloat16()
+    wide = torch.randn(700, 8200, device=DEV).bfloat16()[:, 3:8195]  # copied: 6 bytes off
+    for rows, b in ((x[::2], bias), (x, None), (wide, bias), (x[:1].expand(300, -1), None)):
+        out = ops.linear_bf16(rows, w, b)
+        torch.testing.assert_close(
+            out.float(), torch.nn.functional.linear(rows, w, b).float(),
+            atol=2e-2, rtol=2e-2)
+        parts = ops.linear_parts(rows, w, b)
+        assert isinstance(parts, ops.Parts)
+        torch.testing.assert_close(ops.parts_sum(parts), out, atol=2e-2, rtol=2e-2)
+    norm = torch.randn(2048, device=DEV).bfloat16()
+    res = torch.randn(700, 2048, device=DEV).bfloat16()
+    y, r = ops.fused_add_rmsnorm(ops.linear_parts(x, w), res.clone(), norm)
+    want = res.double() + x.double() @ w.double().t()
+    assert (r.double() - want).norm() <= 2 ** -8 * want.norm()
+
+
 @pytest.mark.parametrize("M", [16, 17, 32, 33, 96, 97, 160, 161, 224, 225])
 @pytest.mark.parametrize("qt", [2, 4, 5])
 @pytest.mark.parametrize("N", [88, 42008])

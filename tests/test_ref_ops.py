@@ -283,6 +283,24 @@ def test_mid_sizes_leave_what_others_do_faster():
         assert not takes(*left, silu=True) and takes(*taken, silu=True)
 
 
+def test_wide_cut():
+    """Tiles that wide_gemm has, runs of at least four steps, at most 128 MB of
+    sums, and no cut where none is asked for; a few hundred rows of long weights
+    fill the CUs."""
+    from arks_amd import ops
+
+    for M in (257, 300, 511, 700, 1400, 2049, 5000, 16385):
+        for N, K in ((2048, 8192), (3584, 18944), (8192, 28672), (37888, 64), (16, 64)):
+            for split in (False, True):
+                tm, tw, splits, jobs = ops._wide_cut(M, N, K, split, True)
+                assert (tm, tw) in ops._WIDE_STEP
+                assert jobs == -(-M // tm) * -(-N // tw) * splits
+                assert splits == 1 or split and (
+                    K // 64 // splits >= 4 and splits * M * N * 4 <= 1 << 27)
+    assert all(ops._wide_cut(M, 3584, 18944, True, True)[3] >= 200
+               for M in range(257, 2049, 64))
+
+
 def test_tile_fill_is_what_the_schedule_takes():
     """The share against the schedule walked out: every workgroup's tiles of its
     XCD in turn, 1 for a whole one and 0.55 for those of the last 128 rows."""
