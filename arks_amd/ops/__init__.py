@@ -908,13 +908,18 @@ def _wide(x, weight, bias=None, summed: bool = False):
     (228), 2314 rows 267 (485), 3344 rows 367 (328), 4666 rows 456 (876); 4096 x
     14336, 300 rows 55 (76), 1549 rows 151 (329), 1972 rows 196 (188); 4096 x
     8192, 300 rows 39 (47), 763 rows 60 (59), 1594 rows 101 (100), 4949 rows 225
-    (256); 1024 x 16384, 450 rows 31 (46). Many whole tiles of rows are what the
-    library does best: 3584 x 18944, 8192 rows 806 (740). With K up to 4096 a run
-    has few steps: 4096 x 4096, 491 rows 32 (30), 1159 rows 51 (44)."""
+    (256); 1024 x 16384, 450 rows 31 (46). What the library does best are many
+    whole tiles of rows, and weights of up to 80 million elements where tiles of 256
+    x 256 make one round over the CUs, at least 5/8 full: 3584 x 18944, 8192 rows 806
+    (740), 3102 rows 369 (355); 4096 x 14336, 2837 rows 279 (249), 3394 rows 299
+    (285). With K up to 4096 a run has few steps: 4096 x 4096, 491 rows 32 (30),
+    1159 rows 51 (44)."""
     if not _wide_takes(x, weight, bias):
         return None
     M, (N, K) = x.shape[0], weight.shape
     if K < 8192 or N < 1024 or (M >= 4096 and M % 256 == 0):
+        return None
+    if N * K <= 80_000_000 and 160 <= -(-M // 256) * -(-N // 256) <= 256:
         return None
     return _wide_cut(M, N, K, True, summed)[:3]
 

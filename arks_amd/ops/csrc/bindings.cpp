@@ -113,7 +113,7 @@ void arks_moe_gemm(void* out, const void* a, const void* w, const void* perm,
                    const void* items, const void* n_items, void* claims, const void* scale,
                    int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out, int k_total,
                    int top_k, int max_items, int tile, int up,
-                   hipStream_t stream);
+                   int once, hipStream_t stream);
 void arks_mfma_probe(void* d, const void* a, const void* b, hipStream_t stream);
 void arks_mfma_probe32(void* d, const void* a, const void* b, hipStream_t stream);
 void arks_tr16_probe(void* out, int stride_bytes, hipStream_t stream);
@@ -826,7 +826,7 @@ void stage_rows(pybind11::list prompts, pybind11::list outputs,
 // [T, k]); w13 [El, 2I, H], w2 [El, H, I], pairs beyond this rank's El experts
 // from expert_base on weigh zero. tile: pairs of a work item; mid: of 32, 64 or
 // 128 pairs in mid_gemm.hip (32: qt_up and qt_down, weight rows a wave / 16, may
-// be 2), else in moe_gemm.hip (16, 128 or 256).
+// be 2), else in moe_gemm.hip (16, 128 or, 256, its engine's up to 320).
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
     torch::Tensor x, torch::Tensor w13, torch::Tensor w2, torch::Tensor weights,
     torch::Tensor ids, int64_t expert_base, int64_t tile, bool mid,
@@ -862,7 +862,7 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
               ids.is_contiguous() && ids.size(0) == T && ids.size(1) == k &&
               weights.size(0) == T);
   if (T == 0) return {torch::empty({0, H}, x.options()), weights, ids};
-  const int64_t max_items = std::min(P, El) + P / tile;
+  const int64_t max_items = std::min(P, El) + P / (tile == 256 ? 320 : tile);
   TORCH_CHECK(max_items <= 65535 || tile != 16, "too many rows for this tile");
   auto ints = x.options().dtype(torch::kInt32);
   // one workgroup plans 8192 pairs in 9 us and 16384 in 20; two launches of a
@@ -883,8 +883,8 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
   int* claims = n_items + 1;
   arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
                 claims + 16, ids.data_ptr(), weights.data_ptr(), (int)P,
-                (int)expert_base, (int)El, (int)tile, (int)max_items,
-                (int)groups, stream);
+                (int)expert_base, (int)El, tile == 256 ? 320 : (int)tile,
+                (int)max_items, (int)groups, stream);
   if (mid) {
     const int ft = (int)tile / 32;
     arks_mid_items(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
@@ -894,12 +894,14 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
                    n_items, I, H * I, (int)H, (int)I, (int)k,
                    (int)expert_base, (int)max_items, ft, (int)qt_down, 0, stream);
   } else {
+    // (moe_gemm.hip: experts that mostly have one item)
+    const int once = P <= 160 * El ? 2 : 0;
     arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
                   n_items, claims, nullptr, x.stride(0), 2 * I * H, H, (int)I, (int)H,
-                  (int)k, (int)max_items, (int)tile, 1, stream);
+                  (int)k, (int)max_items, (int)tile, 1, once, stream);
     arks_moe_gemm(y.data_ptr(), h.data_ptr(), w2.data_ptr(), perm, items,
                   n_items, claims, nullptr, I, H * I, I, (int)H, (int)I, (int)k,
-                  (int)max_items, (int)tile, 0, stream);
+                  (int)max_items, (int)tile, 0, once, stream);
   }
   return {y, w_pair, plan.narrow(0, 4 * max_items + P, P).view({T, k})};
 }
@@ -938,7 +940,7 @@ std::tuple<torch::Tensor, torch::Tensor> moe_wide_rows(
               weights.size(0) == T);
   torch::Tensor y = torch::empty({P, W}, x.options());
   if (T == 0) return {y, ids};
-  const int64_t max_items = std::min(P, experts) + P / 256;
+  const int64_t max_items = std::min(P, experts) + P / 320;
   const int64_t groups = P <= 8192 ? 1 : std::min<int64_t>(64, (P + 2047) / 2048);
   // as in moe_expert_rows
   torch::Tensor plan = torch::empty(
@@ -954,14 +956,16 @@ std::tuple<torch::Tensor, torch::Tensor> moe_wide_rows(
   auto stream = current_stream();
   arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
                 claims + 16, ids.data_ptr(), weights.data_ptr(), (int)P, 0,
-                (int)experts, 256, (int)max_items, (int)groups, stream);
+                (int)experts, 320, (int)max_items, (int)groups, stream);
+  // not rotated: an expert's row adds up in the same order at any number of rows
+  const int once = P <= 160 * experts ? 1 : 0;
   arks_moe_gemm(h.data_ptr(), x.data_ptr(), w_gu.data_ptr(), perm, items,
                 n_items, claims, scaled ? w_pair.data_ptr() : nullptr,
                 x.stride(0), 2 * ff * W, W, (int)ff, (int)W, (int)k,
-                (int)max_items, 256, 2, stream);
+                (int)max_items, 256, 2, once, stream);
   arks_moe_gemm(y.data_ptr(), h.data_ptr(), w_down.data_ptr(), perm, items,
                 n_items, claims, nullptr, ff, ff, down, (int)W, (int)ff, (int)k,
-                (int)max_items, 256, 0, stream);
+                (int)max_items, 256, 0, once, stream);
   return {y, plan.narrow(0, 4 * max_items + P, P).view({T, k})};
 }
 

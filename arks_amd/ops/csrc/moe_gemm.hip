@@ -13,11 +13,10 @@
 //              (4.8 TB/s); every expert as a batched product took 210 us.
 //   moe_engine more than 64 pairs per expert on the mean: bound by the matrix
 //              cores, and by the weights' one read while experts have few. Up
-//              to 256 pairs x 256 weight rows per workgroup (tile_engine.h).
-//              128 experts of 2048 x 768, 8 per row, with plan and mix: 5012
-//              rows 545 us (tiles of 128: 742), 512 rows 251 us for 1.2 GB of
-//              weights (270); 8 experts of 4096 x 14336, 2 per row, 8192 rows
-//              4.5 ms (9.4).
+//              to 320 pairs x 256 weight rows per workgroup (wide_engine.h).
+//              128 experts of 2048 x 768, 8 per row, with plan: 5012 rows 452
+//              us, 520 rows 225 us for 1.2 GB of weights; 8 experts of 4096 x
+//              14336, 2 per row, 8192 rows 4.6 ms.
 //   moe_tile   the same for sizes that are no multiple of 64, or leave the
 //              engine without work for the chip: 128 pairs x 128 weight rows, 64
 //              of K per step through double-buffered LDS and registers, 560
@@ -28,8 +27,9 @@
 // [expert, out, in]: a lane reads 16 bytes along K, as the MFMA operands
 // want them. Items past the last one are empty, so grids depend on the shapes
 // alone and a decode step can be captured.
+#include <type_traits>
 #include "seq_common.h"
-#include "tile_engine.h"
+#include "wide_engine.h"
 
 namespace arks {
 
@@ -145,9 +145,12 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
     for (int e = tid; e < n_local; e += 1024) {
       const int c = count[e];
       const int n = (c + tile - 1) / tile;
+      // (8 experts of 4096 x 14336, 2 per row, 2048 rows 1529 us with items of 320
+      // and what is left, even 1448)
+      const int per = tile > 256 && n ? ((c + n - 1) / n + 63) / 64 * 64 : tile;
       for (int i = 0; i < n; ++i)
         items[first_item[e] + i] = make_int4(
-            e, start[e] + i * tile, min(tile, c - i * tile), i | n << 16);
+            e, start[e] + i * per, min(per, c - i * per), i | n << 16);
     }
     for (int i = total_items + tid; i < max_items; i += 1024)
       items[i] = make_int4(0, 0, 0, 0);
@@ -415,28 +418,58 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
   }
 }
 
-// Up to 256 pairs of one expert x 256 weight rows (UP: 128 gate rows and their
-// 128 up rows) in the product engine of tile_engine.h. Each XCD takes a
-// contiguous stretch of (expert, row tile, item), so that an expert's items meet
-// the same weights in its L2; its workgroups claim tiles one by one, since
-// those of at most 128 pairs take about 0.55 of the others' time (dealt out in
-// turn, 5012 rows: 591 us, claimed 545). The claim is made a tile ahead, so that
-// neither it nor the pairs' rows are waited for. Its place in LDS belongs to the
-// tiles' array: a second one made the compiler drain the loads before every
-// read of the first.
+// Up to 320 pairs of one expert x 256 weight rows (UP: 128 gate rows and their up
+// rows) in the loop of wide_engine.h, whose waves take 1 to 5 fragments of 16 pairs
+// each: a tile's time is a fixed part of 0.5 and 0.21 for each 64 of its pairs.
+// 5012 rows of 128 experts of 2048 x 768, 8 per row, read 1.5 GB through the caches
+// in 276 us of gate and up, so that weights and rows bound them as much as the
+// matrix cores do (busy for 60 % of the CUs' time).
+// ONCE: for experts that have one item each, mostly (up to 160 pairs on the mean):
+// their weights pass the caches by, where the rows stay then, and (rotate) the tiles
+// of an expert begin at different steps, so that reads of columns a power of two
+// apart meet on more of the memory's channels. us with plan, as they are (past the
+// caches; and rotated): 128 experts of 2048 x 768, 8 per row, 300 rows 247 (226;
+// 213), 1000 rows 276 (258; 251), 2048 rows 329 (319; 312), 4096 rows 409 (425;
+// 432); 16 experts of 4096 x 3584, 4 per row, 500 rows 303 (290; 284), 2000 rows 740
+// (763; 771). In tiles of 256 and 128 pairs (tile_engine.h) before: 251, 276, 331,
+// 412; 325, 720.
+// Each XCD takes a contiguous stretch of (expert, row tile, item), so that an
+// expert's items meet the same weights in its L2; its workgroups claim tiles one by
+// one, as they take different times (dealt out in turn, 5012 rows: 591 us, claimed
+// 545). The claim is made a tile ahead, so that neither it nor the pairs' rows are
+// waited for. Its place in LDS belongs to the tiles' array: a second one made the
+// compiler drain the loads before every read of the first.
 // GLU: gate and up are rounded to bf16 before they meet, as rows of a product in
 // memory would be, and scale [pairs] (or null) is a factor of both; it is loaded
 // in front of the next tile's first loads, so as not to be waited for behind them.
-template <bool UP, bool GLU>
+template <bool ONCE>
+using MoeTileOf = WideTile<4, 4, 5, false, ONCE ? 2 : 0>;
+
+// f(fragments a wave that `pairs` pairs take), as a constant
+template <typename F>
+__device__ __forceinline__ void moe_frags(const int pairs, F f) {
+  switch ((pairs + 63) / 64) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    default: f(std::integral_constant<int, 5>{});
+  }
+}
+
+template <bool UP, bool GLU, bool ONCE>
 __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ a,
     const bf16* __restrict__ w, const int* __restrict__ perm,
     const int4* __restrict__ items, const int* __restrict__ n_items,
     int* __restrict__ claims, const float* __restrict__ scale,
     const int64_t a_stride, const int64_t w_expert, const int64_t w_stride,
-    const int n_out, const int k_total, const int top_k, const int row_tiles) {
-  __shared__ __attribute__((aligned(1024))) char lds[TILE_LDS + 16];
-  int& claimed = *reinterpret_cast<int*>(lds + TILE_LDS);
+    const int n_out, const int k_total, const int top_k, const int row_tiles,
+    const int rotate) {
+  using MoeTile = MoeTileOf<ONCE>;
+  constexpr int FY = 5, COLS = UP ? 128 : 256;
+  __shared__ __attribute__((aligned(1024))) char lds[MoeTile::LDS + 16];
+  int& claimed = *reinterpret_cast<int*>(lds + MoeTile::LDS);
   const int total = *n_items * row_tiles;
   const int xcd = blockIdx.x % 8, slots = gridDim.x / 8;
   const int j0 = (int)((int64_t)total * xcd / 8);
@@ -444,107 +477,120 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
   int i = blockIdx.x / 8;
   if (i >= jn) return;
   const int steps = k_total / TILE_K;
-  Tile tile(lds);
+  MoeTile tile(lds);
+  const int lq = tile.lane() % 16, la = tile.lane() / 16;
   struct Job {
     int expert, first, pairs, n0;
+    typename MoeTile::Span k;
   };
   auto job = [&](int i) {
     const int j = j0 + i, q = j / row_tiles, w4 = items[q].w;
     const int i0 = q - (w4 & 0xffff), r = j - i0 * row_tiles, n = w4 >> 16;
     const int4 it = items[i0 + r % n];
-    return Job{it.x, it.y, it.z, r / n * (UP ? 128 : 256)};
+    const int turn = rotate ? (it.x * row_tiles + r / n) % steps : 0;
+    return Job{it.x, it.y, it.z, r / n * COLS, {0, steps, turn}};
   };
-  auto places = [&](const Job& b, int (&p)[2][2]) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r = min(h * 128 + tile_row(tile.wave(), tile.lane(), j),
-                          b.pairs - 1);
-        p[h][j] = UP ? perm[b.first + r] : r;
-      }
+  // The rows of a that this wave loads, each in a lane of its own (so they are one
+  // register beside a tile's sums).
+  auto places = [&](const Job& b) {
+    const int f = (b.pairs + 63) / 64;
+    const int r = min(tile.wave() * f * 8 + tile.lane(), b.pairs - 1);
+    return UP ? perm[b.first + r] : r;
   };
-  auto rows = [&](const Job& b, const int (&p)[2][2]) {
-    TileRows t;
-    t.a = tile_buffer(a + (UP ? 0 : b.first * a_stride));
-    const bf16* we = w + b.expert * w_expert;
-    t.w[0] = tile_buffer(we);
-    t.w[1] = tile_buffer(we + (UP ? n_out * w_stride : 0));
+  auto rows = [&](const Job& b, const int p) {
+    typename MoeTile::Rows t;
+    t.x = tile_buffer(w + b.expert * w_expert);
+    t.y = tile_buffer(a + (UP ? 0 : b.first * a_stride));
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int j = 0; j < MoeTile::LX; ++j) {
+      // A wave's 64 weight rows: as in wide_gemm.hip, 8 neighbouring columns of a
+      // lane are 2 fragments, or (UP) 4, with a column's gate and up row in turns.
+      const int row = tile.row_x(j), q = row / 16 % 4, g = row % 16 / 4, r = row % 4;
+      const int base = row / 64 * (UP ? 32 : 64);
+      const int col = base + (UP ? 8 * g + 2 * q + r / 2
+                                 : q / 2 * 32 + 8 * g + 4 * (q & 1) + r);
+      t.xo[j] = (uint32_t)(min(b.n0 + col, n_out - 1) + (UP && (r & 1) ? n_out : 0)) *
+                    (uint32_t)(w_stride * 2) +
+                tile.piece();
+    }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r = tile_row(tile.wave(), tile.lane(), j);
-        const uint32_t row = UP ? p[h][j] / top_k : p[h][j];
-        t.ao[h][j] = row * (uint32_t)(a_stride * 2) +
-                     tile_piece_a(r, tile.lane());
-        t.wo[h][j] =
-            (uint32_t)min(b.n0 + (UP ? 0 : h * 128) + r, n_out - 1) *
-                (uint32_t)(w_stride * 2) +
-            tile_piece_w(r, tile.lane());
-      }
+    for (int j = 0; j < FY; ++j)
+      t.yo[j] = (uint32_t)__shfl(UP ? p / top_k : p, j * 8 + tile.lane() / 8) *
+                    (uint32_t)(a_stride * 2) +
+                tile.piece();
     return t;
   };
   Job now = job(i);
-  int p[2][2];
-  places(now, p);
-  TileRows t = rows(now, p);
-  tile.prologue(t, steps, now.pairs <= TILE_HALF);
+  int p = places(now);
+  typename MoeTile::Rows t = rows(now, p);
+  moe_frags(now.pairs, [&](auto f) { tile.template prologue<f>(t, now.k); });
   // workgroups' first tiles are theirs, the others are claimed
   if (threadIdx.x == 0) claimed = slots + atomicAdd(&claims[xcd], 1);
-  Tile::sync();
+  MoeTile::sync();
   i = __builtin_amdgcn_readfirstlane(claimed);
-  tile.prologue_wait(steps, now.pairs <= TILE_HALF);
+  moe_frags(now.pairs, [&](auto f) { tile.template prologue_wait<f>(steps); });
   for (;;) {
     const bool more = i < jn;
     const Job next = more ? job(i) : now;
-    if (more) places(next, p);
-    tile.run(t, steps, now.pairs <= TILE_HALF);
-    float by[GLU ? 8 : 1];
-    if constexpr (GLU)
-      tile.each([&](int x, int m, int, const float(&)[8], const float(&)[8]) {
-        by[x] = scale ? scale[perm[now.first + min(m, now.pairs - 1)]] : 1.f;
-      });
+    if (more) p = places(next);
+    moe_frags(now.pairs, [&](auto f) { tile.template run<f>(t, now.k); });
+    float by[GLU ? FY : 1];
+    if constexpr (GLU) {
+#pragma unroll
+      for (int y = 0; y < FY; ++y)
+        by[y] = scale ? scale[perm[now.first + min(tile.frag_y(y) + lq,
+                                                   now.pairs - 1)]]
+                      : 1.f;
+    }
     int c;
     if (more) {
       if (threadIdx.x == 0) c = atomicAdd(&claims[xcd], 1);
       // its loads travel while this tile is stored
       t = rows(next, p);
-      tile.prologue(t, steps, next.pairs <= TILE_HALF);
+      moe_frags(next.pairs, [&](auto f) { tile.template prologue<f>(t, next.k); });
     }
-    ushort8 o[UP ? 8 : 16];
-    tile.each([&](int x, int, int, const float(&g)[8], const float(&u)[8]) {
-      if constexpr (UP) {
-        float v[8];
+    // the sums' columns: 8 of each half (UP), 8 of each half's two pairs of fragments
+    constexpr int P = UP ? 1 : 2;
+    ushort8 o[FY][2 * P];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          v[j] = GLU ? silu_f(by[x] * moe_bf16(g[j])) * (by[x] * moe_bf16(u[j]))
-                     : tile_silu_mul(g[j], u[j]);
-        o[x] = tile_round(v);
-      } else {
-        o[2 * x] = tile_round(g);
-        o[2 * x + 1] = tile_round(u);
-      }
-    });
+    for (int y = 0; y < FY; ++y)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+          float v[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            if constexpr (UP) {
+              const float g = tile.acc[4 * h + e / 2][y][e % 2 * 2];
+              const float u = tile.acc[4 * h + e / 2][y][e % 2 * 2 + 1];
+              v[e] = GLU ? silu_f(by[y] * moe_bf16(g)) * (by[y] * moe_bf16(u))
+                         : tile_silu_mul(g, u);
+            } else {
+              v[e] = tile.acc[4 * h + 2 * q + e / 4][y][e % 4];
+            }
+          }
+          o[y][h * P + q] = tile_round(v);
+        }
     if (more) {
       if (threadIdx.x == 0) claimed = slots + c;
-      tile.prologue_wait(steps, next.pairs <= TILE_HALF);
+      moe_frags(next.pairs, [&](auto f) { tile.template prologue_wait<f>(steps); });
     }
-    tile.each([&](int x, int m, int n, const float(&)[8], const float(&)[8]) {
-      bf16* row = out + (int64_t)(now.first + m) * n_out;
-      const int col = now.n0 + n;  // n_out % 8 == 0
-      if (m >= now.pairs) return;
-      if constexpr (UP) {
-        if (col < n_out) *reinterpret_cast<ushort8*>(row + col) = o[x];
-      } else {
-        if (col < n_out) *reinterpret_cast<ushort8*>(row + col) = o[2 * x];
-        if (col + 128 < n_out)
-          *reinterpret_cast<ushort8*>(row + col + 128) = o[2 * x + 1];
+#pragma unroll
+    for (int y = 0; y < FY; ++y) {
+      const int m = tile.frag_y(y) + lq;
+      if (m >= now.pairs) break;  // fragments are in the rows' order
+      bf16* row = out + (int64_t)(now.first + m) * n_out + now.n0;
+#pragma unroll
+      for (int x = 0; x < 2 * P; ++x) {
+        const int col = x / P * (COLS / 2) + tile.wm() * (UP ? 32 : 64) +
+                        x % P * 32 + 8 * la;
+        if (now.n0 + col < n_out) *reinterpret_cast<ushort8*>(row + col) = o[y][x];
       }
-    });
+    }
     if (!more) return;
     now = next;
-    Tile::sync();
+    MoeTile::sync();
     i = __builtin_amdgcn_readfirstlane(claimed);
   }
 }
@@ -554,7 +600,8 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
 using namespace arks;
 
 // groups: workgroups that the pairs are spread over; more than one need
-// counts [groups, n_local].
+// counts [groups, n_local]. tile above 256 (moe_engine's): an expert's items are
+// even, in whole 64 pairs.
 extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
                               void* items, void* n_items, void* claims,
                               void* counts, const void* ids,
@@ -577,16 +624,17 @@ extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
 }
 
 // tile: pairs of an item, 16 (streamed; n_out % 32 == k_total % 32 == 0) or 128
-// (tiles through LDS; n_out % 8 == k_total % 8 == 0) or 256 (the engine;
-// n_out % 8 == k_total % 64 == 0, an expert's weights and (up) all rows of a
-// under 4 GiB; up: 1, or 2 for GLU, with scale [pairs] or null).
+// (tiles through LDS; n_out % 8 == k_total % 8 == 0) or 256 (the engine, whose items
+// have up to 320; n_out % 8 == k_total % 64 == 0, an expert's weights and (up) all
+// rows of a under 4 GiB; up: 1, or 2 for GLU, with scale [pairs] or null; once: 0,
+// 1, or 2 for rotated columns).
 extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
                               const void* perm, const void* items,
                               const void* n_items, void* claims,
                               const void* scale, int64_t a_stride, int64_t w_expert,
                               int64_t w_stride, int n_out, int k_total,
                               int top_k, int max_items, int tile, int up,
-                              hipStream_t stream) {
+                              int once, hipStream_t stream) {
   const bool glu = up == 2;
 #define ARKS_STREAM(NF, WV, UP)                                               \
   hipLaunchKernelGGL((moe_stream_kernel<NF, WV, UP>),                         \
@@ -607,17 +655,23 @@ extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
     const int row_tiles = (n_out + (up ? 127 : 255)) / (up ? 128 : 256);
     const int64_t jobs = (int64_t)max_items * row_tiles;
     const dim3 grid(jobs < 256 ? (jobs + 7) / 8 * 8 : 256), block(512);
-#define ARKS_ENGINE(UP, GLU)                                                  \
-  hipLaunchKernelGGL((moe_engine_kernel<UP, GLU>), grid, block, 0, stream,    \
+#define ARKS_ENGINE_O(UP, GLU, ONCE)                                          \
+  hipLaunchKernelGGL((moe_engine_kernel<UP, GLU, ONCE>), grid, block, 0, stream, \
                      (bf16*)out, (const bf16*)a, (const bf16*)w,              \
                      (const int*)perm, (const int4*)items,                    \
                      (const int*)n_items, (int*)claims + (up ? 0 : 8),        \
                      (const float*)scale, a_stride, w_expert, w_stride, n_out, \
-                     k_total, top_k, row_tiles)
+                     k_total, top_k, row_tiles, (int)(once == 2))
+#define ARKS_ENGINE(UP, GLU)                                                  \
+  do {                                                                        \
+    if (once) ARKS_ENGINE_O(UP, GLU, true);                                   \
+    else ARKS_ENGINE_O(UP, GLU, false);                                       \
+  } while (0)
     if (up && glu) ARKS_ENGINE(true, true);
     else if (up) ARKS_ENGINE(true, false);
     else ARKS_ENGINE(false, false);
 #undef ARKS_ENGINE
+#undef ARKS_ENGINE_O
   } else {
     const int cols = up ? MT_BN / 2 : MT_BN;
     const int row_tiles = (n_out + cols - 1) / cols;

@@ -44,7 +44,8 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(
   const int all = k_total / TILE_K;
 
   struct Job {
-    int m0, n0, split, s0, steps;
+    int m0, n0, split;
+    typename T::Span k;
   };
   auto job = [&](int i) {
     constexpr int G = 8;
@@ -52,8 +53,8 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(
     const int g = at / (G * tn), r = at % (G * tn);
     const int gm = min(G, tm - g * G);
     const int s0 = (int)((int64_t)all * split / splits);
-    return Job{(g * G + r % gm) * TM, r / gm * COLS, split, s0,
-               (int)((int64_t)all * (split + 1) / splits) - s0};
+    return Job{(g * G + r % gm) * TM, r / gm * COLS, split,
+               {s0, (int)((int64_t)all * (split + 1) / splits) - s0, 0}};
   };
   // The column (of those of a wave's f fragments) whose weights stand at row `at`
   // of them, so that a lane's sums are neighbours in the output: 8 columns of two
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(
       return (uint32_t)weight(r, b.n0) * (uint32_t)(k_total * 2) + tile.piece();
     };
 #pragma unroll
-    for (int j = 0; j < T::LX0 + T::LX1; ++j)
+    for (int j = 0; j < T::LX; ++j)
       t.xo[j] = AX ? of_a(tile.row_x(j)) : of_w(tile.row_x(j));
 #pragma unroll
     for (int j = 0; j < FY; ++j)
@@ -108,16 +109,16 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(
   };
   Job now = job(i);
   typename T::Rows t = rows(now);
-  tile.prologue(t, now.s0, now.steps);
-  tile.prologue_wait(now.steps);
+  tile.prologue(t, now.k);
+  tile.prologue_wait(now.k.steps);
   for (;;) {
-    tile.run(t, now.s0, now.steps);
+    tile.run(t, now.k);
     i += slots;
     const bool more = i < jn;
     const Job next = more ? job(i) : now;
     if (more) {
       t = rows(next);
-      tile.prologue(t, next.s0, next.steps);
+      tile.prologue(t, next.k);
     }
     const int lq = tile.lane() % 16, la = tile.lane() / 16;
     // a row's sums, of the fragments of weights from column n on
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(
     } else {
 #pragma unroll
       for (int y = 0; y < FY; ++y) {
-        const int m = (tile.wn() * FY + y) * 16 + lq;
+        const int m = tile.frag_y(y) + lq;
         store(m, tile.wm() * FX0 * 16 / S, std::integral_constant<int, FX0>{},
               [&](int q) { return tile.acc[q][y]; });
         store(m, (T::X0 + tile.wm() * FX1 * 16) / S,
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(
       }
     }
     if (!more) return;
-    tile.prologue_wait(next.steps);
+    tile.prologue_wait(next.k.steps);
     now = next;
   }
 }

@@ -888,6 +888,32 @@ def test_moe_experts(T, E, k, H, I, base, El, tile, skew, monkeypatch):
     assert err <= 3 * 2 ** -8 * expect.norm()
 
 
+@pytest.mark.parametrize("T", [1, 64, 65, 128, 129, 193, 257, 320, 321, 641, 1281, 1601])
+@pytest.mark.parametrize("El", [2, 24])
+def test_moe_engine_items(T, El):
+    """Items of the engine vs fp64: each number of fragments a wave, full and with
+    one pair more, an expert's items even; weights past the caches (24 experts, of
+    which two are chosen) and not; sums that begin at another step."""
+    assert_native()
+    torch.manual_seed(T)
+    H, I, k = 320, 192, 2
+    x = torch.randn(T, 2 * H, device=DEV).bfloat16()[:, :H]
+    w13 = (torch.randn(El, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(El, H, I, device=DEV) * I ** -0.5).bfloat16()
+    ids = torch.arange(k, device=DEV, dtype=torch.int32).expand(T, k).contiguous()
+    w = torch.rand(T, k, device=DEV)
+    out = torch.empty(T, H, device=DEV, dtype=torch.bfloat16)
+    ops._native().moe_experts(out, x, w13, w2, w, ids, 0, 256, False, 4, 4)
+    expect = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for e in range(k):
+        gu = x.double() @ w13[e].double().t()
+        h = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+        expect += (h @ w2[e].double().t()) * w[:, e:e + 1].double()
+    # as in test_moe_experts, and no row far off
+    err = (out.double() - expect).norm(dim=1)
+    assert (err <= 3 * 2 ** -8 * expect.norm(dim=1)).all()
+
+
 @pytest.mark.parametrize("T,E,k,H,I,base,El,tile,skew", [
     (1, 4, 2, 64, 64, 0, 4, 64, False), (7, 128, 8, 256, 192, 0, 128, 64, False),
     (33, 64, 8, 2048, 768, 16, 16, 64, False),  # another rank's pairs
@@ -1690,6 +1716,8 @@ def test_wide_rule():
     assert not ops._wide(x, w, torch.ones(1, dtype=torch.bfloat16, device=DEV))
     many = x[:1].expand(4097, -1)
     assert ops._wide(many, w) and not ops._wide(many[:4096], w)
+    more = x[:1].expand(5000, -1)  # 160 tiles of 256 x 256
+    assert ops._wide(more[:4800], w) and not ops._wide(more, w)
     gated = torch.empty(16384, 64, dtype=torch.bfloat16, device=DEV)
     assert ops._wide_silu(x[:300, :64], gated)
     assert ops._wide_silu(x[:300, :64], gated[:4096]) is None  # few tiles
