@@ -1367,6 +1367,20 @@ def _moe_native(x, w13, w2, ids) -> bool:
             and ids.shape[1] <= 16)
 
 
+def _moe_engine(pairs: int, El: int, experts: int, H: int, I: int, way) -> bool:
+    """Whether the engine takes over from items in mid_gemm.hip: from 32 pairs an
+    expert on, where both products have a tile for every CU. us with plan, engine
+    (the better of items of 64 and 128): 128 experts of 2048 x 768, 8 per row, 144
+    rows 203 (202), 528 rows 222 (246), 1008 rows 253 (297); 64 of 2048 x 1408, 6
+    per row, 352 rows 203 (218), 672 rows 227 (259); 16 of 4096 x 2048, 2 per row,
+    264 rows 139 (152), 504 rows 160 (197); with fewer tiles, 8 of 4096 x 14336, 2
+    per row, 252 rows 583 (526), 32 of 1536 x 512, 4 per row, 416 rows 60 (58). With
+    20 to 30 pairs it is the choice of experts that decides: a prompt of 400 rows
+    through 4 layers of the first 1608 us (1584)."""
+    return (way[1] and pairs >= 32 * experts
+            and El * min(-(-H // 256), -(-I // 128)) >= 256)
+
+
 def _moe_cut(x, w13, w2, ids, experts):
     """x with rows on 16 bytes, and (pairs of an item, whether mid_gemm.hip
     takes them[, tiles of items of 32])."""
@@ -1375,6 +1389,8 @@ def _moe_cut(x, w13, w2, ids, experts):
     x = _rows_16b(x)
     whole = _moe_whole(x, H, I, rows * k)
     way = _moe_way(rows, k, El, experts or El, H, I, whole)
+    if _moe_engine(rows * k, El, experts or El, H, I, way):
+        way = (256, False)
     # matrices of 2^19 weights and more: below, launches are what counts
     if (rows <= 32 and whole and way in ((16, False), (64, True))
             and H * I >= 1 << 19):

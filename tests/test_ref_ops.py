@@ -340,6 +340,20 @@ def test_moe_way():
     assert ops._moe_way(7, 4, 16, 16, 2056, 1416, False) == (128, False)
 
 
+def test_moe_engine_takes_over():
+    """Items of mid_gemm give way to the engine from 32 pairs an expert on, with a
+    tile for every CU in both products."""
+    from arks_amd import ops
+
+    takes = lambda rows, k, E, H, I, El=None: ops._moe_engine(
+        rows * k, El or E, E, H, I, ops._moe_way(rows, k, El or E, E, H, I, True))
+    assert not takes(511, 8, 128, 2048, 768) and takes(512, 8, 128, 2048, 768)
+    assert takes(256, 2, 16, 4096, 2048) and not takes(252, 2, 8, 4096, 14336)
+    assert not takes(416, 4, 32, 1536, 512)
+    assert not takes(512, 8, 128, 2048, 768, 16)  # a rank's 16 experts
+    assert not ops._moe_engine(1 << 20, 128, 128, 2048, 768, (128, False))
+
+
 def test_decode_waves():
     """Two workgroups per CU for fp8 rows, and where sequences outnumber runs."""
     from arks_amd import ops
