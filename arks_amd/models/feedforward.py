@@ -178,8 +178,11 @@ class GroupedMoE(nn.Module):
     def forward(self, h, batch=None, cache=None) -> torch.Tensor:
         T = h.shape[0]
         E, ff, W, k = self.E, self.ff, self.width, self.top
-        z = linear_f32(h, self.router)  # fp32 logits
-        weights, ids = ops.moe_route_grouped(z, k, self.groups, self.keep)
+        if ops.route_rows_takes(h, self.router, self.groups):
+            weights, ids = ops.moe_route_rows(h, self.router, k)
+        else:
+            z = linear_f32(h, self.router)  # fp32 logits
+            weights, ids = ops.moe_route_grouped(z, k, self.groups, self.keep)
         if T <= self.DENSE_TOKENS:
             gu = linear(h, self.w13)  # [T, E * 2ff]
             a = ops.glu_act(gu.view(T * E, 2 * ff), "swiglu")
@@ -249,13 +252,16 @@ class RoutedMoE(nn.Module):
     def forward(self, h, batch=None, cache=None) -> torch.Tensor:
         T = h.shape[0]
         E, ff, sff, k = self.E, self.ff, self.sff, self.top
-        z = linear_f32(h, self.router)  # fp32 logits
         route = dict(score=self.score, renorm=self.renorm, bias=self.router_b,
-                     correction=self.correction, group_top=self.group_top,
-                     shared_gate=self.shared_gate)
+                     correction=self.correction, shared_gate=self.shared_gate)
         if T <= self.DENSE_TOKENS:
-            _, _, scale = ops.moe_route_grouped(
-                z, k, self.groups, self.keep, matrix=True, **route)
+            if ops.route_rows_takes(h, self.router, self.groups):
+                _, _, scale = ops.moe_route_rows(h, self.router, k, matrix=True,
+                                                 **route)
+            else:
+                _, _, scale = ops.moe_route_grouped(
+                    linear_f32(h, self.router), k, self.groups, self.keep,
+                    matrix=True, group_top=self.group_top, **route)
             # (weights that linear_fixed takes keep the order of sums that they
             # have at 17 rows and more)
             if (not sff and ops.routed_takes(h, self.w_gu, self.w_down, E, ff)
@@ -267,8 +273,9 @@ class RoutedMoE(nn.Module):
             return linear(ops.moe_glu_scaled(
                 gu, scale, E, ff, sff, self.weigh_input, self.act, self.limit,
                 self.shared_limit, self.alpha, self.shared_gate), self.w_down)
+        z = linear_f32(h, self.router)  # fp32 logits
         weights, ids = ops.moe_route_grouped(z, k, self.groups, self.keep,
-                                             **route)
+                                             group_top=self.group_top, **route)
         if (self.act == "swiglu"
                 and ops.moe_wide_takes(h, self.w_gu, self.w_down, E, ff, k)):
             y, place = ops.moe_wide_rows(h, self.w_gu, self.w_down, weights,

@@ -100,8 +100,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T with fp32 OUTPUT from rows of the model's dtype (bf16 inputs,
     fp32 accumulate, no rounding of the result)."""
-    if x.dtype != torch.float32 and not getattr(w, "fixed_sums", False):
-        out = ops.linear_f32_rows(x, w)
+    if x.dtype != torch.float32:
+        rows = (ops.linear_f32_fixed if getattr(w, "fixed_sums", False)
+                else ops.linear_f32_rows)
+        out = rows(x, w)
         if out is not None:
             return out
     return ops.linear_f32_lib(x, w)

@@ -1020,13 +1020,37 @@ def sums_fixed(M: int, *weights) -> bool:
     return any(_fixed_run(M, *w.shape) for w in weights)
 
 
+@functools.lru_cache(maxsize=1024)
+def _fixed_cut(N: int, K: int, f32: bool):
+    """(qt, splits) of a fixed product of more than _SKINNY_MAX_ELEMS weights
+    (f32: with an fp32 result, one run), or None: mid_gemm's sums of up to 64 rows
+    are the same for a cut, as long as tiles begin at the same steps (K up to 16384,
+    arks_mid_gemm), and the cut is that of 16 rows at any number of them. us, 1 to
+    16 rows (library): 12608 x 4096 18.5 (26), 16640 x 4096 27 (67), 10240 x 5120
+    21.5 (24), 20480 x 2560 23.5 (48), 114688 x 4096 148 (160 to 198); in fp32 32000
+    x 4096 45 (59), 64 rows 46 (51)."""
+    if (N * K <= _SKINNY_MAX_ELEMS or K % 64 or N % 8
+            or not 2048 <= K <= 16384 or N >= 1 << 24):
+        return None
+    return _mid_cut(16, N, K, False, False, whole=f32)
+
+
+def _fixed_mid(x, weight, bias=None, f32: bool = False):
+    """The cut, if x weight^T takes a fixed product of mid_gemm: up to 64 rows, with
+    K below 4096 32 (50304 x 2560, 48 rows 57 us, library 53)."""
+    N, K = weight.shape
+    if not _mid_takes(x, weight, bias) or x.shape[0] > (64 if K >= 4096 else 32):
+        return None
+    return _fixed_cut(N, K, f32)
+
+
 def linear_fixed(x, weight, bias=None):
     """x weight^T (+ bias) whose order of sums follows from the weight alone up
-    to 48 rows, for models that choose experts. Near a tie between two of them
-    the last bits of a row decide, and with the expert its logits move (up to
-    0.2 of their norm in 3 layers of 16 experts): the choice must not turn with
-    the number of rows that share a step. linear_bf16 picks its kernel, and so
-    the order, by the rows."""
+    to 48 rows (large weights with K below 4096: 32), for models that choose
+    experts. Near a tie between two of them the last bits of a row decide, and with
+    the expert its logits move (up to 0.2 of their norm in 3 layers of 16 experts):
+    the choice must not turn with the number of rows that share a step. linear_bf16
+    picks its kernel, and so the order, by the rows."""
     M, (N, K) = x.shape[0], weight.shape
     per = _fixed_run(M, N, K) if _few_rows(x, weight, bias) else 0
     if per:
@@ -1034,9 +1058,21 @@ def linear_fixed(x, weight, bias=None):
                            device=x.device)
         _native().stream_split(sums, _rows_16b(x), weight, per)
         return parts_sum(Parts(sums, bias))
+    cut = _fixed_mid(x, weight, bias)
+    if cut is not None:
+        return parts_sum(_mid_gemm(x, weight, bias, cut))
     import torch.nn.functional as F
 
     return F.linear(x, weight, bias)
+
+
+def linear_f32_fixed(x, weight):
+    """x weight^T in fp32, as linear_fixed, where mid_gemm has a fixed product
+    with an fp32 result, else None."""
+    cut = _fixed_mid(x, weight, f32=True)
+    if cut is None:
+        return None
+    return _mid_gemm(x, weight, None, cut, summed=True).sums[0]
 
 
 def _mid_f32_tile(M: int, N: int, K: int):
@@ -1974,6 +2010,35 @@ def moe_route_grouped(logits, top, groups=1, keep=1, score="softmax",
             mat = torch.cat([mat, torch.sigmoid(logits[:, -1:].float())], 1)
         return w, ids, mat
     return w, ids
+
+
+def route_rows_takes(h, router, groups: int = 1) -> bool:
+    """Whether moe_route_rows takes these rows: steps of few, whose launches count,
+    and a lane an expert, no groups. us in a replayed graph, here (the library's
+    product and moe_route_grouped): 16 experts of 4096 columns, 1 row 6.4 (12.0), 64
+    rows 6.9 (12.8); 64 of 2048, 64 rows 10.2 (12.6), 256 rows 16.3 (12.4)."""
+    T, W = h.shape
+    return (_USE_SKINNY and h.is_cuda and 1 <= T <= 64 and groups == 1
+            and h.dtype == router.dtype == torch.bfloat16
+            and 8 <= W and W % 8 == 0 and router.shape[0] <= 64
+            and h.stride(-1) == 1 and h.stride(0) % 8 == 0
+            and h.data_ptr() % 16 == 0 and router.is_contiguous()
+            and router.data_ptr() % 16 == 0 and _plain(h, router))
+
+
+def moe_route_rows(h, router, top, score="softmax", renorm=True, matrix=False,
+                   bias=None, correction=None, shared_gate=False):
+    """moe_route_grouped of the fp32 logits h router^T without groups, where
+    route_rows_takes."""
+    T, E = h.shape[0], router.shape[0]
+    w = torch.empty((T, top), dtype=torch.float32, device=h.device)
+    ids = torch.empty((T, top), dtype=torch.int32, device=h.device)
+    mat = (torch.empty((T, E), dtype=torch.float32, device=h.device)
+           if matrix else None)
+    _native_seq().moe_route_rows(w, ids, h, router, top, score == "sigmoid",
+                                 bool(renorm), mat, bias, correction,
+                                 bool(shared_gate))
+    return (w, ids, mat) if matrix else (w, ids)
 
 
 def moe_sort_pairs(ids, experts, pad=0):

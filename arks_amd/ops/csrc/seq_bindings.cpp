@@ -172,6 +172,11 @@ int arks_seq_moe_route_grouped(void* weights, void* ids, const void* logits,
                                const void* bias, const void* correction,
                                int group_top, int shared_gate,
                                hipStream_t stream);
+int arks_seq_moe_route_rows(void* weights, void* ids, void* logits, const void* x,
+                            int64_t x_stride, const void* router, int W, int T,
+                            int E, int top, int sigmoid, int renorm, void* matrix,
+                            const void* bias, const void* correction,
+                            int shared_gate, hipStream_t stream);
 int arks_seq_moe_sort_pairs(void* row_of_place, void* place, void* counts,
                             const void* ids, int n, int k, int E, int pad,
                             hipStream_t stream);
@@ -1038,6 +1043,47 @@ void moe_route_grouped(Tensor weights, Tensor ids, Tensor logits, int64_t top,
   TORCH_CHECK(rc == 0, "routing sizes the kernel does not hold");
 }
 
+// moe_route_grouped of the logits x [T, W] . router [E (+ 1), W]^T, both bf16, without
+// groups
+void moe_route_rows(Tensor weights, Tensor ids, Tensor x, Tensor router,
+                    int64_t top, bool sigmoid, bool renorm, OptTensor matrix,
+                    OptTensor bias, OptTensor correction, bool shared_gate) {
+  TORCH_CHECK(x.is_cuda() && router.is_cuda() && x.dim() == 2 &&
+              router.dim() == 2 && x.scalar_type() == torch::kBFloat16 &&
+              router.scalar_type() == torch::kBFloat16 && router.is_contiguous() &&
+              x.size(1) == router.size(1) && x.stride(1) == 1);
+  TORCH_CHECK(x.stride(0) % 8 == 0 && x.size(1) % 8 == 0 &&
+                  reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(router.data_ptr()) % 16 == 0,
+              "rows must start on 16 bytes");
+  check_f32(weights, "weights");
+  check_i32(ids, "ids");
+  const int T = x.size(0), E = router.size(0) - (shared_gate ? 1 : 0);
+  TORCH_CHECK(weights.size(0) == T && weights.size(1) == top &&
+              ids.size(0) == T && ids.size(1) == top);
+  void* mat_p = nullptr;
+  if (matrix.has_value()) {
+    check_f32(*matrix, "scale matrix");
+    TORCH_CHECK(matrix->dim() == 2 && matrix->size(0) == T &&
+                matrix->size(1) == router.size(0));
+    mat_p = matrix->data_ptr();
+  }
+  for (const OptTensor* v : {&bias, &correction})
+    if (v->has_value()) {
+      check_f32(**v, "router bias or correction");
+      TORCH_CHECK((*v)->numel() == E);
+    }
+  Tensor logits = torch::empty({T, router.size(0)}, weights.options());
+  const int rc = arks_seq_moe_route_rows(
+      weights.data_ptr(), ids.data_ptr(), logits.data_ptr(), x.data_ptr(), x.stride(0),
+      router.data_ptr(), (int)x.size(1), T, E, (int)top, sigmoid ? 1 : 0,
+      renorm ? 1 : 0, mat_p,
+      bias.has_value() ? bias->data_ptr() : nullptr,
+      correction.has_value() ? correction->data_ptr() : nullptr,
+      shared_gate ? 1 : 0, current_stream());
+  TORCH_CHECK(rc == 0, "routing sizes the kernel does not hold");
+}
+
 // False: more experts than the kernel holds.
 bool moe_sort_pairs(Tensor row_of_place, Tensor place, Tensor counts,
                     Tensor ids) {
@@ -1823,6 +1869,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_write_pooled", &kv_write_pooled);
   m.def("attention_window_pool", &attention_window_pool);
   m.def("attention_window_pool_mfma", &attention_window_pool_mfma);
+  m.def("moe_route_rows", &moe_route_rows);
   m.def("moe_route_grouped", &moe_route_grouped);
   m.def("moe_sort_pairs", &moe_sort_pairs);
   m.def("moe_mix", &moe_mix);

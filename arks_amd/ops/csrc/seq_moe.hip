@@ -14,6 +14,7 @@
 //       matrix (optional, [T, E]): the row's weights at the experts it uses,
 //       0 elsewhere; with shared_gate the logits have a column E more, whose
 //       sigmoid is the matrix's column E.
+//   moe_route_rows  the same, without groups, from the rows and the router's weights
 //   moe_sort_pairs  (row, expert) pairs in expert order, stable: the row of
 //       every sorted place, every pair's place, the pairs per expert
 //   moe_mix_rows  out[t] = sum_j w[t][j] * y[row(t, j)], row given, or
@@ -21,6 +22,7 @@
 #include "seq_common.h"
 
 #include <cfloat>
+#include <climits>
 
 namespace arks {
 
@@ -102,9 +104,8 @@ __global__ __launch_bounds__(64) void moe_route_grouped_kernel(
       if (g_s[e / per] != INFINITY) s_s[e] = -INFINITY;
     __syncthreads();
   }
-  float wsum = 0.f;
-  float wk[ROUTE_MAX_K];
-  int ik[ROUTE_MAX_K];
+  float wsum = 0.f, mine = 0.f;  // lane r keeps choice r
+  int mine_id = 0;
   for (int r = 0; r < top; ++r) {
     float best = -INFINITY;
     int bi = E;
@@ -123,22 +124,110 @@ __global__ __launch_bounds__(64) void moe_route_grouped_kernel(
     const float sc = !correction ? best
                      : sigmoid   ? sigmoid_f(row[bi] + (bias ? bias[bi] : 0.f))
                                  : best - correction[bi];
-    wk[r] = sc;
-    ik[r] = bi;
+    if (lane == r) {
+      mine = sc;
+      mine_id = bi;
+    }
     wsum += sc;
     __syncthreads();
     if (lane == 0) s_s[bi] = -INFINITY;
     __syncthreads();
   }
-  if (lane == 0) {
-    const float d = wsum + 1e-20f;
-    for (int r = 0; r < top; ++r) {
-      const float w = renorm ? wk[r] / d : wk[r];
-      weights[(int64_t)t * top + r] = w;
-      ids[(int64_t)t * top + r] = ik[r];
-      if (matrix) matrix[(int64_t)t * ldm + ik[r]] = w;
+  if (lane < top) {
+    const float w = renorm ? mine / (wsum + 1e-20f) : mine;
+    weights[(int64_t)t * top + lane] = w;
+    ids[(int64_t)t * top + lane] = mine_id;
+    if (matrix) matrix[(int64_t)t * ldm + mine_id] = w;
+  }
+}
+
+// The router's product and the routing of steps of few rows, up to 64 experts
+// without groups, in two launches that latency bounds. A wave per logit: a lane adds
+// up its 16-byte pieces of the row in turn, then the lanes are added, so that a
+// logit is the same bits at any number of rows. Then a wave per row, whose scores
+// are a lane each. us for 16 experts of 4096 columns in a replayed graph (the
+// library's product, of one workgroup, and moe_route_grouped): 1 row 6.4 (12.0), 64
+// rows 6.9 (12.8); 64 experts of 2048, 8 rows 8.5 (12.4). In one launch, a workgroup
+// per row, 8.7: one CU reads the router alone.
+constexpr int ROUTE_LANES = 64;
+
+// A float's order as an integer's; NaN below all others.
+__device__ __forceinline__ int route_key(const float v) {
+  const int b = __float_as_int(v);
+  return v != v ? INT_MIN : b < 0 ? b ^ 0x7fffffff : b;
+}
+
+__global__ __launch_bounds__(256) void moe_router_kernel(
+    float* __restrict__ logits, const bf16* __restrict__ x,
+    const int64_t x_stride, const bf16* __restrict__ router, const int W,
+    const int all) {
+  const int lane = threadIdx.x % WAVE_SIZE, t = blockIdx.y;
+  const int e = blockIdx.x * 4 + threadIdx.x / WAVE_SIZE;
+  if (e >= all) return;
+  const bf16* row = x + t * x_stride;
+  const bf16* w = router + (int64_t)e * W;
+  float sum = 0.f;
+  for (int i0 = lane * 8; i0 < W; i0 += 8 * 512) {
+    ushort8 a[8], b[8];  // 16 loads under way
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int i = min(i0 + j * 512, W - 8);
+      a[j] = *reinterpret_cast<const ushort8*>(row + i);
+      b[j] = *reinterpret_cast<const ushort8*>(w + i);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float part = 0.f;
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        part += bf16_bits_to_float(a[j][c]) * bf16_bits_to_float(b[j][c]);
+      sum += i0 + j * 512 < W ? part : 0.f;
     }
   }
+  sum = wave_reduce_sum(sum);
+  if (lane == 0) logits[t * all + e] = sum;
+}
+
+__global__ __launch_bounds__(64) void moe_route_lanes_kernel(
+    float* __restrict__ weights, int* __restrict__ ids,
+    const float* __restrict__ logits, const int E, const int top,
+    const int sigmoid, const int renorm, float* __restrict__ matrix,
+    const float* __restrict__ bias, const float* __restrict__ correction,
+    const int shared_gate) {
+  const int lane = threadIdx.x, t = blockIdx.x, all = E + shared_gate;
+  const float z = lane < all ? logits[t * all + lane] : 0.f;
+  const bool on = lane < E;
+  const float zb = z + (bias && on ? bias[lane] : 0.f);
+  float s;
+  if (sigmoid) {
+    s = sigmoid_f(zb);
+  } else {
+    const float m = wave_reduce_max(on ? zb : -FLT_MAX);
+    const float p = on ? expf(zb - m) : 0.f;
+    s = p * (1.f / wave_reduce_sum(p));
+  }
+  const float add = correction && on ? correction[lane] : 0.f;
+  const float choice = correction ? s + add : s;
+  const int key = route_key(choice);
+  int rank = 0;
+  for (int e = 0; e < E; ++e) {
+    const int k = __builtin_amdgcn_readlane(key, e);
+    rank += k > key || (k == key && e < lane) ? 1 : 0;
+  }
+  // the score itself
+  const float sc = !correction ? choice : sigmoid ? s : choice - add;
+  float wsum = 0.f;
+  for (int r = 0; r < top; ++r) {
+    const int at = __ffsll((unsigned long long)__ballot(on && rank == r)) - 1;
+    wsum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), at));
+  }
+  const float w = renorm ? sc / (wsum + 1e-20f) : sc;
+  if (on && rank < top) {
+    weights[(int64_t)t * top + rank] = w;
+    ids[(int64_t)t * top + rank] = lane;
+  }
+  if (matrix && lane < all)
+    matrix[(int64_t)t * all + lane] = !on ? sigmoid_f(z) : rank < top ? w : 0.f;
 }
 
 // Stable counting sort in one block. Wave w owns the w-th run of pairs; its
@@ -282,6 +371,30 @@ extern "C" int arks_seq_moe_route_grouped(void* weights, void* ids,
                      top, groups, keep, sigmoid, renorm, (float*)matrix,
                      (const float*)bias, (const float*)correction, group_top,
                      shared_gate);
+  return 0;
+}
+
+// x [T, W] and router [E + shared_gate, W] bf16, rows on 16 bytes, W % 8 == 0;
+// logits [T, E + shared_gate]: scratch.
+extern "C" int arks_seq_moe_route_rows(void* weights, void* ids, void* logits,
+                                       const void* x, int64_t x_stride,
+                                       const void* router, int W, int T, int E,
+                                       int top, int sigmoid, int renorm,
+                                       void* matrix, const void* bias,
+                                       const void* correction, int shared_gate,
+                                       hipStream_t stream) {
+  const int all = E + shared_gate;
+  if (E < 1 || all > ROUTE_LANES || top > E || top > ROUTE_MAX_K || W < 8 || W % 8 ||
+      T > 65535)
+    return 1;
+  if (T == 0) return 0;
+  hipLaunchKernelGGL(moe_router_kernel, dim3((all + 3) / 4, T), dim3(256), 0,
+                     stream, (float*)logits, (const bf16*)x, x_stride,
+                     (const bf16*)router, W, all);
+  hipLaunchKernelGGL(moe_route_lanes_kernel, dim3(T), dim3(64), 0, stream,
+                     (float*)weights, (int*)ids, (const float*)logits, E, top,
+                     sigmoid, renorm, (float*)matrix, (const float*)bias,
+                     (const float*)correction, shared_gate);
   return 0;
 }
 

@@ -2217,6 +2217,29 @@ def test_fixed_products(N, K):
             assert torch.equal(ops.linear_fixed(x[:m], w, b), want[:m]), m
 
 
+@pytest.mark.parametrize("N,K", [(12608, 4096), (16640, 2560), (2400, 16384)])
+def test_fixed_large_products(N, K):
+    """Weights beyond those that test_fixed_products has: the same bits for any
+    number of rows up to 64 (32 where K is short), in bf16 and fp32."""
+    assert_native()
+    torch.manual_seed(N)
+    x = torch.randn(64, K, dtype=torch.bfloat16, device=DEV)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    b = torch.randn(N, dtype=torch.bfloat16, device=DEV)
+    most = 64 if K >= 4096 else 32
+    assert ops._fixed_mid(x[:most], w, b) and not ops._fixed_mid(x[:1], w[:1024])
+    want, whole = ops.linear_fixed(x[:most], w, b), ops.linear_f32_fixed(x[:most], w)
+    for m in (1, 2, 15, 16, 17, 31, 32, 33, 63):
+        if m < most:
+            assert torch.equal(ops.linear_fixed(x[:m], w, b), want[:m]), m
+            assert torch.equal(ops.linear_f32_fixed(x[:m], w), whole[:m]), m
+    exact = x[:most].double() @ w.double().t()
+    slack = K * 2 ** -24 * (x[:most].double().abs() @ w.double().abs().t())
+    assert ((whole.double() - exact).abs() <= slack).all()
+    exact += b.double()
+    assert ((want.double() - exact).abs() <= 2 * slack + 2 ** -8 * exact.abs()).all()
+
+
 def test_host_tensors_are_refused():
     """Tensors on the host never reach a kernel."""
     assert_native()

@@ -614,6 +614,48 @@ def test_routed_experts_read_the_chosen_alone(rows, E, top, ff, W, act):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,W,gate", [
+    (1, 16, 4, 4096, False), (64, 64, 8, 2048, False), (5, 63, 32, 4104, True),
+    (3, 1, 1, 8, False), (7, 5, 2, 520, True)])
+@pytest.mark.parametrize("score", ["softmax", "sigmoid"])
+def test_route_rows(T, E, top, W, gate, score):
+    """Router product and routing against moe_route_grouped of logits in float64:
+    ends of a row's pieces, every lane an expert, ties, a correction that decides;
+    a row's choice does not turn with the rows beside it."""
+    torch.manual_seed(E + W)
+    dev = "cuda"
+    h = torch.randn(T, 2 * W, device=dev).bfloat16()[:, :W]
+    router = (torch.randn(E + gate, W, device=dev) * W ** -0.5).bfloat16()
+    if E > 2:
+        router[1] = router[0]  # equal scores: the lower index first
+    bias = torch.randn(E, device=dev) * 0.1
+    bias[:2] = 0.2
+    corr = torch.randn(E, device=dev) * 0.05
+    corr[:2] = 0.1
+    assert ops.route_rows_takes(h, router) and not ops.route_rows_takes(h, router, 2)
+    assert not ops.route_rows_takes(h.float(), router.float())
+    z = (h.double() @ router.double().t()).float()
+    for kw in ({}, dict(bias=bias), dict(bias=bias, correction=corr)):
+        kw.update(score=score, shared_gate=gate)
+        out = ops.moe_route_rows(h, router, top, matrix=True, **kw)
+        want = ops.moe_route_grouped(z, top, matrix=True, **kw)
+        # logits within W 2^-24 sum |x w|: scores apart by less may swap
+        slack = 4 * W * 2 ** -24 * (h.double().abs() @ router.double().abs().t()).max().item()
+        for a, b in ((out[0], want[0]), (out[2], want[2])):
+            assert (a - b).abs().max().item() <= slack + 1e-6
+        assert torch.equal(out[1], want[1])
+        for n in {1, T // 2} - {0}:
+            for a, b in zip(ops.moe_route_rows(h[:n], router, top, matrix=True, **kw), out):
+                assert torch.equal(a, b[:n])
+    # rows that hold no numbers stay in bounds
+    h = h.clone()
+    h[0, 0] = float("nan")
+    ids = ops.moe_route_rows(h, router, top)[1]
+    assert ids.min() >= 0 and ids.max() < E + gate
+    assert all(len(set(r)) == top for r in ids.tolist())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,top,ff,W,most", [
     (4, 2, 512, 1024, 48),     # weights of linear_fixed
     (16, 4, 1024, 2560, 16)])  # routed_experts takes them
