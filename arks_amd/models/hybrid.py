@@ -115,8 +115,9 @@ from .. import ops
 from ..config import HybridModelConfig
 from ..engine.forward_batch import ForwardBatch
 from ..parallel.comm import get_tp_world_size
+from ..parallel.layers import passable
 from .feedforward import GLU, build_feedforward
-from .mixers import build_mixer, linear, linear_f32, _param
+from .mixers import build_mixer, linear, linear_f32, linear_parts, _param
 
 
 @dataclass(frozen=True)
@@ -151,6 +152,19 @@ ARRANGEMENTS = {
     "Fuzelorn": BlockArrangement(token_shift=False, gated_residual=False,
                                  norm_place="pre"),
 }
+
+
+def _heads(mixer) -> bool:
+    """Whether a block may multiply mixer.heads() by mixer.o itself."""
+    own = next((c for c in type(mixer).__mro__ if "heads" in c.__dict__), None)
+    return own is not None and passable(mixer, own)
+
+
+def _columns(p, first: int, end: int):
+    """Columns of a tensor or Parts."""
+    if isinstance(p, ops.Parts):
+        return p.columns(first, end)
+    return p[:, first:end]
 
 
 class HybridBlock(nn.Module):
@@ -205,15 +219,20 @@ class HybridBlock(nn.Module):
                 batch.seq_lens, batch.state_slots, batch.token_seq, dtype)
         else:
             xs = xa = x.to(dtype)
-        y = self.mixer(xs, batch, cache)
-        g = linear(xa, self.rg1) if self.rg1 is not None else None
+        if self.rg1 is not None and dtype == torch.bfloat16 and _heads(self.mixer):
+            h = self.mixer.heads(xs, batch, cache)
+            y, g = (ops.linear_pair(h, self.mixer.o, xa, self.rg1)
+                    or (linear_parts(h, self.mixer.o), linear_parts(xa, self.rg1)))
+        else:
+            y = self.mixer(xs, batch, cache)
+            g = linear(xa, self.rg1) if self.rg1 is not None else None
         xa = ops.gated_norm_residual(x, y, g, self.rg1_b, self.norm1, self.eps,
                                      dtype if self.ff else None)
         if self.ff:
-            ug = linear(xa, self.up_gate)
-            h = ops.gelu_tanh(ug[:, :self.ff])
-            y = linear(h, self.down)
-            g = ug[:, self.ff:] if self.arr.gated_residual else None
+            ug = linear_parts(xa, self.up_gate)
+            y = linear_parts(ops.gelu_tanh(_columns(ug, 0, self.ff)), self.down)
+            g = (_columns(ug, self.ff, self.ff + self.width)
+                 if self.arr.gated_residual else None)
             ops.gated_norm_residual(x, y, g, self.rg2_b, self.norm2, self.eps, None)
 
 

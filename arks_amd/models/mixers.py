@@ -97,6 +97,16 @@ def linear(x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
     return F.linear(x, w, b)
 
 
+def linear_parts(x: torch.Tensor, w: torch.Tensor):
+    """linear, for a consumer that takes ops.Parts too. Below 2^20 weights a product
+    is one launch without sums to add (8 rows of 1024 x 1024 and the norm behind it
+    the same either way)."""
+    if (x.dtype == torch.bfloat16 and w.numel() >= 1 << 20
+            and not getattr(w, "fixed_sums", False)):
+        return ops.linear_parts(x, w)
+    return linear(x, w)
+
+
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T with fp32 OUTPUT from rows of the model's dtype (bf16 inputs,
     fp32 accumulate, no rounding of the result)."""
@@ -295,14 +305,15 @@ class SinkRotaryAttention(nn.Module):
             res = res * out_scale
         out.copy_(res.view(p.shape[0], H * V))
 
-    def forward(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+    def heads(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+        """The rows that the out-projection takes."""
         T = xs.shape[0]
         H, G, D, V = self.H, self.G, self.D, self.V
         qkv = linear(xs, self.qkv)
         if self.masked:
             out = torch.empty((T, H * V), dtype=xs.dtype, device=xs.device)
             self.core(qkv, batch, cache, out, 1.0)
-            return linear(out, self.o)
+            return out
         q, k, v = self._split(qkv)
         q = self._prepare(q, k, v, batch, cache)
         out = ops.attention_sink_paged(
@@ -311,7 +322,10 @@ class SinkRotaryAttention(nn.Module):
             self.inv_freq_v, self.interleaved, batch.max_q_len,
             batch.positions, self._tiles(batch, q),
             step_cache=batch.step_cache)
-        return linear(out.view(T, H * V), self.o)
+        return out.view(T, H * V)
+
+    def forward(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+        return linear(self.heads(xs, batch, cache), self.o)
 
 
 class LightningMixer(nn.Module):
@@ -336,7 +350,8 @@ class LightningMixer(nn.Module):
     def cache_layout(self, block_size: int, dtype) -> dict:
         return {"S": ("slot", (self.H, self.D, self.V), torch.float32)}
 
-    def forward(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+    def heads(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+        """The rows that the out-projection takes."""
         T = xs.shape[0]
         H, D, V = self.H, self.D, self.V
         p = linear(xs, self.qkvg)
@@ -348,8 +363,11 @@ class LightningMixer(nn.Module):
                                batch.cu_seqlens, batch.seq_lens,
                                batch.state_slots, batch.max_q_len,
                                step_chunks(batch, xs.device))
-        y = ops.gated_rmsnorm(o.view(T, H * V), self.norm, g, self.eps, xs.dtype)
-        return linear(y, self.o)
+        return ops.gated_rmsnorm(o.view(T, H * V), self.norm, g, self.eps,
+                                 xs.dtype)
+
+    def forward(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+        return linear(self.heads(xs, batch, cache), self.o)
 
 
 class Mamba1Mixer(nn.Module):
@@ -393,7 +411,8 @@ class Mamba1Mixer(nn.Module):
             out["conv"] = ("slot", (self.taps - 1, self.C), torch.float32)
         return out
 
-    def forward(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+    def heads(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+        """The rows that the out-projection takes."""
         C = self.C
         xz = linear(xs, self.w_in)
         u = ops.causal_conv_silu(
@@ -404,11 +423,13 @@ class Mamba1Mixer(nn.Module):
         dt_pre = None
         if xs.is_cuda and self.R >= 8:
             dt_pre = linear_f32(dbc[:, :self.R], self.dt_w_mm)
-        y = ops.selective_scan(
+        return ops.selective_scan(
             u, dbc, xz[:, C:], self.dt_w, self.dt_b, self.A, self.D,
             cache["ssm"], batch.cu_seqlens, batch.seq_lens, batch.state_slots,
             batch.max_q_len, dt_pre, step_chunks(batch, xs.device))
-        return linear(y, self.o)
+
+    def forward(self, xs, batch: ForwardBatch, cache: dict) -> torch.Tensor:
+        return linear(self.heads(xs, batch, cache), self.o)
 
 
 class SplitMixer(nn.Module):

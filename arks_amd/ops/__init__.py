@@ -556,6 +556,10 @@ _USE_SKINNY = os.environ.get("ARKS_SKINNY_GEMM", "1") == "1"
 _SKINNY_MAX_ELEMS = 34_000_000
 
 
+# weights of two products that go in one launch, together
+_PAIR_ELEMS = 100_000_000
+
+
 def _rows_16b(x):
     """x, or a copy whose rows start on 16 bytes."""
     if x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
@@ -804,6 +808,11 @@ class Parts:
     def __init__(self, sums, bias=None):
         self.sums, self.bias = sums, bias
 
+    def columns(self, first: int, end: int):
+        """Those of columns [first, end)."""
+        return Parts(self.sums[:, :, first:end],
+                     None if self.bias is None else self.bias[first:end])
+
 
 class Mixed:
     """Experts' rows y [pairs, H] that are not mixed yet: row t of the result
@@ -834,7 +843,7 @@ def parts_sum(x):
         return x
     out = torch.empty(x.sums.shape[1:], dtype=torch.bfloat16,
                       device=x.sums.device)
-    _native().stream_sum(out, x.sums, x.bias)
+    _native().stream_sum(out, x.sums.contiguous(), x.bias)
     return out
 
 
@@ -970,6 +979,54 @@ def linear_parts(x, weight, bias=None, own_cut: bool = True):
     if cut is not None:
         return _wide_gemm(x, weight, bias, cut, summed=True)
     return linear_bf16(x, weight, bias)
+
+
+@functools.lru_cache(maxsize=1024)
+def _pair_cut(M: int, N: int, K: int, K2: int):
+    """(qt, runs of K, runs of K2) of a pair of products of N columns, by the fit
+    of _mid_cut: a workgroup's time is that of the longest run, and the sums of all
+    runs are written and read. At most 8 runs of each."""
+    steps, groups = (K // 64, K2 // 64), -(-M // 32)
+    best = None
+    for qt in (4, 5, 2):
+        tiles = -(-N // (32 * qt))
+        alone = 0.02 + 0.095 * qt + 0.06 * groups
+        for run in range(1, max(steps) + 1):
+            splits = [-(-s // run) for s in steps]
+            if max(splits) > 8:
+                continue
+            rounds, last = divmod(tiles * sum(splits), 256)
+            us = rounds * (0.6 + run * max(alone, 0.15 * qt))
+            if last:
+                us += 0.6 + run * max(alone, 0.15 * qt * last / 256)
+            us += sum(splits) * (0.1 + M * N * 1.6e-6)
+            if best is None or us < best[0]:
+                best = us, qt, splits
+    return best[1], *best[2]
+
+
+def linear_pair(x, weight, x2, weight2):
+    """(x weight^T, x2 weight2^T), both Parts, or None: one launch for up to 64
+    rows of two products of as many columns, as long as the start and the end of a
+    launch weigh beside the weights' stream (up to _PAIR_ELEMS). us with the norm
+    behind both, cold weights (linear_parts of each; linear_bf16): 4096 x 4096 twice,
+    1 row 18.3 (20.4; 20.7), 8 rows 18.7 (22.9; 22.8), 64 rows 21.4 (27.0; 31.6);
+    4096 x (8192 and 4096), 8 rows 23.9 (27.9; 30.3); 1024 x 1024, 8 rows 8.6 (11.1;
+    11.2); 5120 x 5120 27.1 (30.0; 40.6); 8192 x 8192 56.8 (57.3; 60.0), 6144 x (12288
+    and 6144) 49.0 (49.0; 51.2)."""
+    if (x.dim() == x2.dim() == 2 and 1 <= x.shape[0] == x2.shape[0] <= 64
+            and weight.shape[0] == weight2.shape[0] and weight.shape[0] % 8 == 0
+            and weight.shape[1] % 64 == weight2.shape[1] % 64 == 0
+            and 1024 <= min(weight.shape[1], weight2.shape[1])
+            and weight.numel() + weight2.numel() <= _PAIR_ELEMS
+            and _mid_takes(x, weight) and _mid_takes(x2, weight2)):
+        M, N = x.shape[0], weight.shape[0]
+        qt, n, n2 = _pair_cut(M, N, weight.shape[1], weight2.shape[1])
+        sums = torch.empty((n + n2, M, N), dtype=torch.float32, device=x.device)
+        _native().mid_pair(sums, _rows_16b(x), weight, _rows_16b(x2), weight2, qt,
+                           n)
+        return Parts(sums[:n]), Parts(sums[n:])
+    return None
 
 
 def linear_bf16(x, weight, bias=None):
@@ -1543,7 +1600,21 @@ def token_shift(x, shift_w, prev_state, cu_seqlens, seq_lens, state_slots,
 
 def gated_norm_residual(x, y, gate, gate_bias, weight, eps, out_dtype=None):
     """x (fp32, in place) += rmsnorm(y * sigmoid(gate + bias)) * weight.
-    Returns the new x cast to out_dtype when one is asked for."""
+    Returns the new x cast to out_dtype when one is asked for. y and gate may
+    be Parts."""
+    if isinstance(y, Parts) or isinstance(gate, Parts):
+        W = x.shape[1]
+        if (out_dtype in (None, torch.bfloat16) and W % 8 == 0 and W <= 8192
+                and all(not isinstance(p, Parts) or p.bias is None
+                        for p in (y, gate))):
+            xa = (torch.empty(x.shape, dtype=out_dtype, device=x.device)
+                  if out_dtype is not None else None)
+            _native_seq().gated_norm_sums(
+                x, xa, *(p.sums if isinstance(p, Parts)
+                         else p if p is None else _rows_16b(p)
+                         for p in (y, gate)), gate_bias, weight, eps)
+            return xa
+        y, gate = parts_sum(y), parts_sum(gate)
     if x.is_cuda:
         if out_dtype == torch.float32:
             out_dtype = None  # x itself is the fp32 copy
@@ -1823,7 +1894,14 @@ def selective_scan(u, dbc, z, dt_w, dt_b, A, Dp, state, cu_seqlens, seq_lens,
 
 
 def gelu_tanh(x):
-    """tanh-form GELU; x may be a column slice of a wider GEMM output."""
+    """tanh-form GELU; x may be a column slice of a wider GEMM output, or Parts."""
+    if isinstance(x, Parts):
+        if x.bias is None and x.sums.shape[2] % 8 == 0:
+            out = torch.empty(x.sums.shape[1:], dtype=torch.bfloat16,
+                              device=x.sums.device)
+            _native_seq().gelu_tanh_sums(out, x.sums)
+            return out
+        x = parts_sum(x)
     if x.is_cuda:
         out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         _native_seq().gelu_tanh(out, x)

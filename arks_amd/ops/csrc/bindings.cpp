@@ -100,6 +100,10 @@ int arks_wide_gemm(void* out, const void* a, const void* w, const void* bias,
 void arks_mid_gemm(void* out, const void* a, const void* w, const void* bias,
                    int m, int n, int k, int64_t a_stride, int qt, int splits,
                    int parts, int silu, hipStream_t stream);
+void arks_mid_pair(void* out, const void* a, const void* w, int k,
+                   int64_t a_stride, int splits, const void* a2, const void* w2,
+                   int k2, int64_t a_stride2, int splits2, int m, int n, int qt,
+                   hipStream_t stream);
 void arks_mid_items(void* out, const void* a, const void* w, const void* perm,
                     const void* items, const void* n_items, int64_t a_stride,
                     int64_t w_expert, int n, int k, int top_k, int expert_base,
@@ -749,6 +753,41 @@ void mid_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
                 current_stream());
 }
 
+// out [splits + splits2, M, N]: the sums of a . w^T in `splits` runs of K, then
+// those of a2 . w2^T (mid_gemm.hip)
+void mid_pair(torch::Tensor out, torch::Tensor a, torch::Tensor w,
+              torch::Tensor a2, torch::Tensor w2, int64_t qt, int64_t splits) {
+  TORCH_CHECK(out.is_cuda() && out.dim() == 3 && out.is_contiguous() &&
+                  out.scalar_type() == torch::kFloat32 &&
+                  reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0,
+              "sums are contiguous fp32 on the GPU");
+  const int64_t M = out.size(1), N = out.size(2), splits2 = out.size(0) - splits;
+  TORCH_CHECK(M <= 64 && N % 8 == 0 && N < (1 << 24) && splits >= 1 &&
+                  splits2 >= 1 && (qt == 2 || qt == 4 || qt == 5),
+              "need M <= 64, N % 8 == 0");
+  auto check = [&](const torch::Tensor& x, const torch::Tensor& weight,
+                   int64_t runs) {
+    check_bf16_rowstrided(x, "a");
+    check_bf16_contig(weight, "w");
+    TORCH_CHECK(x.dim() == 2 && weight.dim() == 2);
+    check_rows_16b(x, "a");
+    check_rows_16b(weight, "w");
+    const int64_t K = x.size(1);
+    TORCH_CHECK(x.size(0) == M && weight.size(0) == N && weight.size(1) == K &&
+                    x.device() == out.device() && weight.device() == out.device() &&
+                    K % 64 == 0 && runs <= K / 64 && K < (1 << 22) &&
+                    x.stride(0) < (1 << 22),
+                "need rows of K % 64 == 0 columns, a run of 64 at least");
+  };
+  check(a, w, splits);
+  check(a2, w2, splits2);
+  if (M == 0 || N == 0) return;
+  arks_mid_pair(out.data_ptr(), a.data_ptr(), w.data_ptr(), (int)a.size(1),
+                a.stride(0), (int)splits, a2.data_ptr(), w2.data_ptr(),
+                (int)a2.size(1), a2.stride(0), (int)splits2, (int)M, (int)N,
+                (int)qt, current_stream());
+}
+
 // What a step's rows read, into host tensors: sequence i's tokens (prompt, then
 // output) from starts[i] on, counts[i] of them (none given: its last one), their
 // positions and cache slots, packed; its length behind them into lens[i], its
@@ -1033,6 +1072,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_silu", &tile_silu);
   m.def("wide_gemm", &wide_gemm);
   m.def("mid_gemm", &mid_gemm);
+  m.def("mid_pair", &mid_pair);
   m.def("stage_rows", &stage_rows);
   m.def("moe_expert_rows", &moe_expert_rows);
   m.def("moe_wide_rows", &moe_wide_rows);

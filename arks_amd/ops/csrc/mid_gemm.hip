@@ -57,6 +57,16 @@ struct MidItems {
   int expert_base;  // number of the first of these experts among all ranks'
 };
 
+// The second of two products in one launch: a, w [n_total, k] of rows of its own,
+// whose runs of K come behind the first one's `splits`.
+struct MidPair {
+  const bf16* __restrict__ a;
+  const bf16* __restrict__ w;
+  int64_t a_stride;
+  int k_total;
+  int splits;  // of the first product
+};
+
 // Lanes of neighbouring rows swap x of the odd row against y of the even one:
 // a store then covers twice the columns of half the rows, whole lines.
 template <typename V>
@@ -96,13 +106,20 @@ __device__ __forceinline__ void mid_store(const __amdgpu_buffer_rsrc_t& to,
 // round faster; their tiles may be of 32 * 2 weight rows, to fill the last round
 // of tiles (with plan and mix, 128 experts of 2048 x 768, 8 per row: 7 rows 91.6
 // us streamed, 93.3 in items of 64, 90.6 of 32, 86.1 with gate and up cut so).
-template <int QT, int FT, bool SILU, bool ITEMS>
+//
+// PAIR: two products a . w^T of different rows and K, with as many columns each, for
+// a consumer that adds the sums of both: few rows of 16 to 34 million weights are
+// over before the loads have come up to speed (8 rows of 4096 x 4096 take 8.6 us, at
+// 3.9 TB/s), and two of them do so once (ops._pair_cut).
+enum MidKind { MID_ONE, MID_ITEMS, MID_PAIR };
+template <int QT, int FT, bool SILU, MidKind KIND>
 __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
     void* __restrict__ out, const bf16* __restrict__ a,
     const bf16* __restrict__ w, const bf16* __restrict__ bias,
     const int m_rows, const int n_total, const int k_total,
     const int64_t a_stride, const int splits, const int parts,
-    const int rotate, const MidItems of) {
+    const int rotate, const MidItems of, const MidPair second) {
+  constexpr bool ITEMS = KIND == MID_ITEMS, PAIR = KIND == MID_PAIR;
   constexpr int NS = mid_stages(QT, FT);
   constexpr int W_ROWS = 32 * QT, COLS = SILU ? W_ROWS / 2 : W_ROWS;
   constexpr int W_STAGE = W_ROWS * 128, STAGE = W_STAGE + 32 * FT * 128;
@@ -141,6 +158,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
   struct Job {
     int n0, split, s0, steps, turn;
     int expert, first, rows;
+    bool other;  // of the second product
   };
   auto job = [&](const int j) {
     if constexpr (ITEMS) {
@@ -150,31 +168,45 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
       const unsigned at = (unsigned)(of.expert_base + it.x) * units + n0 / UNIT;
       return Job{(int)n0, 0, 0, all_steps,
                  rotate ? (int)(at % (unsigned)all_steps) : 0,
-                 it.x, it.y, it.z};
+                 it.x, it.y, it.z, false};
+    }
+    if constexpr (PAIR) {
+      const unsigned run = j / tiles;
+      const bool other = run >= (unsigned)second.splits;
+      const unsigned at = other ? run - second.splits : run;
+      const unsigned n = other ? splits - second.splits : second.splits;
+      const unsigned all = other ? second.k_total / TILE_K : all_steps;
+      const int s0 = all * at / n, steps = all * (at + 1) / n - s0;
+      return Job{(int)(j % tiles) * COLS, (int)run, s0, steps,
+                 rotate ? (int)((unsigned)j % (unsigned)steps) : 0,
+                 0, 0, m_rows, other};
     }
     const unsigned split = j / tiles, n = splits;  // all_steps * n < 2^32
     const int s0 = all_steps * split / n;
     const int steps = all_steps * (split + 1) / n - s0;
     return Job{(int)(j % tiles) * COLS, (int)split, s0, steps,
                rotate ? (int)((unsigned)j % (unsigned)steps) : 0,
-               0, 0, m_rows};
+               0, 0, m_rows, false};
   };
   if (wave >= 4) {
     const int own = wave % 4;
     __amdgpu_buffer_rsrc_t wb, ab;
     uint32_t wo[QT], ao[FT];
     auto aim = [&](const Job& b) {
-      wb = tile_buffer(w + (ITEMS ? b.expert * of.w_expert : 0) +
-                       (int64_t)b.n0 * k_total + b.s0 * TILE_K);
-      ab = tile_buffer(a + b.s0 * TILE_K +
-                       (ITEMS && !of.perm ? b.first * a_stride : 0));
+      const int k = PAIR && b.other ? second.k_total : k_total;
+      const int64_t stride = PAIR && b.other ? second.a_stride : a_stride;
+      wb = tile_buffer((PAIR && b.other ? second.w : w) +
+                       (ITEMS ? b.expert * of.w_expert : 0) +
+                       (int64_t)b.n0 * k + b.s0 * TILE_K);
+      ab = tile_buffer((PAIR && b.other ? second.a : a) + b.s0 * TILE_K +
+                       (ITEMS && !of.perm ? b.first * stride : 0));
 #pragma unroll
       for (int i = 0; i < QT; ++i) {
         const int row = (own + 4 * i) * 8 + lane / 8;
         const int side = row / (16 * QT), at = row % (16 * QT);
         const int col = min(side * (COLS / 2) + column(at), n_total - 1 - b.n0);
         wo[i] = (uint32_t)(col + (SILU && (at & 1) ? n_total : 0)) *
-                    (uint32_t)(k_total * 2) +
+                    (uint32_t)(k * 2) +
                 tile_piece_a(row, lane);
       }
 #pragma unroll
@@ -192,7 +224,7 @@ __global__ __launch_bounds__(512, 2) void mid_gemm_kernel(
           for (int k = 1; k < 8; ++k) pair = (int)r - base == k ? at[k] : pair;
           r = (uint32_t)pair / (uint32_t)of.top_k;
         }
-        ao[i] = r * (uint32_t)(a_stride * 2) + tile_piece_a(row, lane);
+        ao[i] = r * (uint32_t)(stride * 2) + tile_piece_a(row, lane);
       }
     };
     int total = 0;  // steps of all of this workgroup's jobs
@@ -474,10 +506,11 @@ extern "C" void arks_mid_gemm(void* out, const void* a, const void* w,
   // 3584 x 18944 39 -> 48 us)
   const int rotate = (int64_t)m * k <= 1 << 20;
 #define ARKS_MID(QT, FT, SILU)                                                 \
-  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, false>),                   \
+  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, MID_ONE>),                 \
                      dim3(jobs < 256 ? jobs : 256), dim3(512), 0, stream, out, \
                      (const bf16*)a, (const bf16*)w, (const bf16*)bias, m, n,  \
-                     k, a_stride, splits, parts, rotate, MidItems{})
+                     k, a_stride, splits, parts, rotate, MidItems{},           \
+                     MidPair{})
 #define ARKS_MID_S(QT, FT)                                                     \
   do {                                                                         \
     if (silu) ARKS_MID(QT, FT, true);                                          \
@@ -502,6 +535,34 @@ extern "C" void arks_mid_gemm(void* out, const void* a, const void* w,
 #undef ARKS_MID
 }
 
+// out: fp32 [splits + splits2, m, n], the sums of a . w^T in runs of k and behind
+// them those of a2 . w2^T in runs of k2; m <= 64, the other conditions of
+// arks_mid_gemm for both.
+extern "C" void arks_mid_pair(void* out, const void* a, const void* w, int k,
+                              int64_t a_stride, int splits, const void* a2,
+                              const void* w2, int k2, int64_t a_stride2,
+                              int splits2, int m, int n, int qt,
+                              hipStream_t stream) {
+  const int jobs = (n + 32 * qt - 1) / (32 * qt) * (splits + splits2);
+  const int rotate = (int64_t)m * (k + k2) <= 1 << 20;
+  const MidPair second{(const bf16*)a2, (const bf16*)w2, a_stride2, k2, splits};
+#define ARKS_MID(QT, FT)                                                       \
+  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, false, MID_PAIR>),               \
+                     dim3(jobs < 256 ? jobs : 256), dim3(512), 0, stream, out, \
+                     (const bf16*)a, (const bf16*)w, nullptr, m, n, k,         \
+                     a_stride, splits + splits2, 1, rotate, MidItems{}, second)
+#define ARKS_MID_M(QT)                                                         \
+  do {                                                                         \
+    if (m <= 32) ARKS_MID(QT, 1);                                              \
+    else ARKS_MID(QT, 2);                                                      \
+  } while (0)
+  if (qt == 2) ARKS_MID_M(2);
+  else if (qt == 4) ARKS_MID_M(4);
+  else ARKS_MID_M(5);
+#undef ARKS_MID_M
+#undef ARKS_MID
+}
+
 // out [places, n]: the items' pairs (at most 32 * ft each, ft 1, 2 or 4) times
 // their experts' weights, silu: [2n, k] each; n_items of the max_items items are
 // there. qt: 16 * qt weight rows a wave, 4, or (ft 1) 2. k % 64 == 0, n % 8 == 0;
@@ -519,9 +580,10 @@ extern "C" void arks_mid_items(void* out, const void* a, const void* w,
   const int64_t jobs = (int64_t)((n + cols - 1) / cols) * max_items;
   const int grid = (int)(jobs < 256 ? jobs : 256);
 #define ARKS_MID(QT, FT, SILU)                                                 \
-  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, true>), dim3(grid),        \
+  hipLaunchKernelGGL((mid_gemm_kernel<QT, FT, SILU, MID_ITEMS>), dim3(grid),   \
                      dim3(512), 0, stream, out, (const bf16*)a,                \
-                     (const bf16*)w, nullptr, 0, n, k, a_stride, 1, 0, 1, of)
+                     (const bf16*)w, nullptr, 0, n, k, a_stride, 1, 0, 1, of,  \
+                     MidPair{})
 #define ARKS_MID_S(QT, FT)                                                     \
   do {                                                                         \
     if (silu) ARKS_MID(QT, FT, true);                                          \

@@ -19,6 +19,14 @@ void arks_seq_gated_norm_residual(void* x, void* xa, const void* y,
 void arks_seq_rms_norm_f32(void* out, const void* x, const void* w,
                            const void* gate, int64_t ldg, float eps, int T,
                            int W, int act_f32, hipStream_t stream);
+void arks_seq_gated_norm_sums(void* x, void* xa, const void* y, int64_t ldy,
+                              int64_t part_y, int splits_y, const void* g,
+                              int64_t ldg, int64_t part_g, int splits_g,
+                              const void* gb, const void* w, float eps, int T,
+                              int W, hipStream_t stream);
+void arks_seq_gelu_tanh_sums(void* out, const void* x, int64_t ldx, int64_t part,
+                             int splits, int64_t rows, int n,
+                             hipStream_t stream);
 void arks_seq_gelu_tanh(void* out, const void* x, int64_t ldx, int64_t rows,
                         int n, int act_f32, hipStream_t stream);
 int arks_seq_qk_norm_rope_cache(
@@ -403,6 +411,62 @@ void gated_norm_residual(Tensor x, OptTensor xa, Tensor y, OptTensor gate,
   arks_seq_gated_norm_residual(x.data_ptr(), xa_p, y.data_ptr(), g_p, ldg, gb_p,
                                w.data_ptr(), (float)eps, T, W, f32,
                                current_stream());
+}
+
+// Rows [T, W] of a product: bf16 (rows on 16 bytes), or fp32 sums [splits, T, W].
+struct ProductRows {
+  const void* p = nullptr;
+  int64_t ld = 0, part = 0;
+  int splits = 0;
+};
+ProductRows product_rows(const Tensor& t, int64_t T, int64_t W, const char* name) {
+  const bool sums = t.dim() == 3;
+  TORCH_CHECK(t.is_cuda() && (sums || t.dim() == 2) &&
+                  t.scalar_type() == (sums ? torch::kFloat32 : torch::kBFloat16) &&
+                  t.size(-2) == T && t.size(-1) == W && t.stride(-1) == 1 &&
+                  W % 8 == 0 && t.stride(-2) % (sums ? 4 : 8) == 0 &&
+                  (!sums || (t.size(0) >= 1 && t.stride(0) % 4 == 0)) &&
+                  reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+              name, " must be bf16 rows or fp32 sums of them on 16 bytes");
+  return {t.data_ptr(), t.stride(-2), sums ? t.stride(0) : 0,
+          sums ? (int)t.size(0) : 0};
+}
+
+// gated_norm_residual (bf16 rows) where y or the gate are sums
+void gated_norm_sums(Tensor x, OptTensor xa, Tensor y, OptTensor gate,
+                     OptTensor gate_bias, Tensor w, double eps) {
+  check_f32(x, "x");
+  check_f32(w, "norm weight");
+  TORCH_CHECK(x.dim() == 2);
+  const int64_t T = x.size(0), W = x.size(1);
+  TORCH_CHECK(w.numel() == W && W <= 8192);
+  const ProductRows yr = product_rows(y, T, W, "y");
+  ProductRows gr;
+  const void* gb_p = nullptr;
+  if (gate.has_value()) {
+    gr = product_rows(*gate, T, W, "gate");
+    TORCH_CHECK(gate_bias.has_value());
+    check_f32(*gate_bias, "gate bias");
+    TORCH_CHECK(gate_bias->numel() == W);
+    gb_p = gate_bias->data_ptr();
+  }
+  void* xa_p = nullptr;
+  if (xa.has_value()) {
+    TORCH_CHECK(xa->is_cuda() && xa->scalar_type() == torch::kBFloat16 &&
+                xa->is_contiguous() && xa->sizes() == x.sizes());
+    xa_p = xa->data_ptr();
+  }
+  arks_seq_gated_norm_sums(x.data_ptr(), xa_p, yr.p, yr.ld, yr.part, yr.splits,
+                           gr.p, gr.ld, gr.part, gr.splits, gb_p, w.data_ptr(),
+                           (float)eps, (int)T, (int)W, current_stream());
+}
+
+void gelu_tanh_sums(Tensor out, Tensor sums) {
+  TORCH_CHECK(sums.dim() == 3 && out.is_cuda() && out.dim() == 2 &&
+              out.scalar_type() == torch::kBFloat16 && out.is_contiguous());
+  const ProductRows r = product_rows(sums, out.size(0), out.size(1), "sums");
+  arks_seq_gelu_tanh_sums(out.data_ptr(), r.p, r.ld, r.part, r.splits,
+                          out.size(0), (int)out.size(1), current_stream());
 }
 
 void rms_norm_f32(Tensor out, Tensor x, Tensor w, double eps) {
@@ -1878,6 +1942,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("unrotate_rows", &unrotate_rows);
   m.def("token_shift", &token_shift);
   m.def("gated_norm_residual", &gated_norm_residual);
+  m.def("gated_norm_sums", &gated_norm_sums);
+  m.def("gelu_tanh_sums", &gelu_tanh_sums);
   m.def("rms_norm_f32", &rms_norm_f32);
   m.def("gated_rmsnorm", &gated_rmsnorm);
   m.def("gelu_tanh", &gelu_tanh);

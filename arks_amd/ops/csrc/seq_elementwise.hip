@@ -2,6 +2,7 @@
 // decoders: token shift, gated output norm + residual add, final norm,
 // gated RMS norm, tanh-GELU, and the attention front end (per-head q/k RMS
 // norm, rotary, position-turned values, paged cache write).
+#include "parts.h"
 #include "seq_common.h"
 
 namespace arks {
@@ -122,6 +123,86 @@ __global__ __launch_bounds__(256) void gated_norm_residual_vec8_kernel(
         }
         *reinterpret_cast<ushort8*>(xa + (int64_t)t * W + i) = o;
       }
+    }
+  }
+}
+
+// Rows of a product: bf16, or (splits > 0) fp32 sums of its runs of K that are still
+// to be added, `part` floats apart.
+struct SumRows {
+  const void* p;
+  int64_t ld, part;
+  int splits;
+};
+
+// 8 values from column i of row t on
+__device__ __forceinline__ void sum_rows8(const SumRows& in, const int t,
+                                          const int i, float (&v)[8]) {
+  if (in.splits > 0) {
+    const float* p = reinterpret_cast<const float*>(in.p) + t * in.ld + i;
+    f32x4 lo, hi;
+    sum_parts_pair(p, p + 4, in.part, in.splits, lo, hi);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = e < 4 ? lo[e % 4] : hi[e % 4];
+  } else {
+    const ushort8 u = *reinterpret_cast<const ushort8*>(
+        reinterpret_cast<const bf16*>(in.p) + t * in.ld + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = bf16_bits_to_float(u[e]);
+  }
+}
+
+// gated_norm_residual_vec8 of products whose sums are not added yet: a row is a
+// chain of loads, so its threads have 8 columns each up to W 4096 and ask for all
+// sums of both products at once.
+__global__ __launch_bounds__(512) void gated_norm_sums_kernel(
+    float* __restrict__ x, bf16* __restrict__ xa, const SumRows y,
+    const SumRows g, const float* __restrict__ gb, const float* __restrict__ w,
+    const float eps, const int W) {
+  __shared__ float scratch[8];
+  constexpr int VPT = 2;  // W <= 8 * 512 * VPT
+  const int t = blockIdx.x;
+  float* xr = x + (int64_t)t * W;
+  float z[VPT][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int i = (k * 512 + threadIdx.x) * 8;
+    if (i < W) {
+      sum_rows8(y, t, i, z[k]);
+      if (g.p) {
+        float gv[8];
+        sum_rows8(g, t, i, gv);
+        const float4v b0 = *reinterpret_cast<const float4v*>(gb + i);
+        const float4v b1 = *reinterpret_cast<const float4v*>(gb + i + 4);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          z[k][e] *= sigmoid_f(gv[e] + (e < 4 ? b0[e % 4] : b1[e % 4]));
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += z[k][e] * z[k][e];
+    }
+  }
+  ss = block_reduce_sum<512>(ss, scratch);
+  const float rstd = 1.f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int i = (k * 512 + threadIdx.x) * 8;
+    if (i < W) {
+      ushort8 o;
+#pragma unroll
+      for (int hlf = 0; hlf < 2; ++hlf) {
+        const int j = i + 4 * hlf;
+        float4v xv = *reinterpret_cast<const float4v*>(xr + j);
+        const float4v wv = *reinterpret_cast<const float4v*>(w + j);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          xv[e] += z[k][4 * hlf + e] * rstd * wv[e];
+          o[4 * hlf + e] = float_to_bf16_bits(xv[e]);
+        }
+        *reinterpret_cast<float4v*>(xr + j) = xv;
+      }
+      if (xa) *reinterpret_cast<ushort8*>(xa + (int64_t)t * W + i) = o;
     }
   }
 }
@@ -268,17 +349,17 @@ __global__ __launch_bounds__(256) void gelu_tanh_kernel(
 // bf16, 8 elements per thread; tanh(u) = 1 - 2 / (1 + e^(2u)) with the
 // hardware exponential (saturates cleanly at both ends)
 __global__ __launch_bounds__(256) void gelu_tanh_vec8_kernel(
-    bf16* __restrict__ out, const bf16* __restrict__ x, int64_t ldx,
-    int64_t rows, int n8) {
+    bf16* __restrict__ out, const SumRows x, int64_t rows, int n8) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= rows * n8) return;
   const int64_t r = idx / n8;
   const int c = (int)(idx - r * n8) * 8;
-  const ushort8 v = *reinterpret_cast<const ushort8*>(x + r * ldx + c);
+  float v[8];
+  sum_rows8(x, (int)r, c, v);
   ushort8 o;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float z = bf16_bits_to_float(v[e]);
+    const float z = v[e];
     const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
     const float th = 1.f - 2.f / (1.f + __expf(2.f * u));
     o[e] = float_to_bf16_bits(0.5f * z * (1.f + th));
@@ -620,6 +701,31 @@ extern "C" void arks_seq_gated_norm_residual(void* x, void* xa, const void* y,
       (const float*)w, eps, W));
 }
 
+// y and g (null: no gate): bf16 rows, or sums (splits > 0) on 16 bytes; W % 8 == 0,
+// W <= 8192
+extern "C" void arks_seq_gated_norm_sums(
+    void* x, void* xa, const void* y, int64_t ldy, int64_t part_y, int splits_y,
+    const void* g, int64_t ldg, int64_t part_g, int splits_g, const void* gb,
+    const void* w, float eps, int T, int W, hipStream_t stream) {
+  if (T == 0) return;
+  hipLaunchKernelGGL(gated_norm_sums_kernel, dim3(T), dim3(512), 0, stream,
+                     (float*)x, (bf16*)xa, SumRows{y, ldy, part_y, splits_y},
+                     SumRows{g, ldg, part_g, splits_g}, (const float*)gb,
+                     (const float*)w, eps, W);
+}
+
+// x: sums on 16 bytes, n % 8 == 0
+extern "C" void arks_seq_gelu_tanh_sums(void* out, const void* x, int64_t ldx,
+                                        int64_t part, int splits, int64_t rows,
+                                        int n, hipStream_t stream) {
+  const int64_t total = rows * n;
+  if (total == 0) return;
+  hipLaunchKernelGGL(gelu_tanh_vec8_kernel,
+                     dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0,
+                     stream, (bf16*)out, SumRows{x, ldx, part, splits}, rows,
+                     n / 8);
+}
+
 extern "C" void arks_seq_rms_norm_f32(void* out, const void* x, const void* w,
                                       const void* gate, int64_t ldg, float eps,
                                       int T, int W, int act_f32,
@@ -652,7 +758,7 @@ extern "C" void arks_seq_gelu_tanh(void* out, const void* x, int64_t ldx,
   if (!act_f32 && n % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0) {
     hipLaunchKernelGGL(gelu_tanh_vec8_kernel,
                        dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0,
-                       stream, (bf16*)out, (const bf16*)x, ldx, rows, n / 8);
+                       stream, (bf16*)out, SumRows{x, ldx, 0, 0}, rows, n / 8);
     return;
   }
   SEQ_DISPATCH_ACT(act_f32, hipLaunchKernelGGL(

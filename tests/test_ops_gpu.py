@@ -1659,6 +1659,69 @@ def test_mid_gemm(M, N, K, qt, splits, kind):
             <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("M,N,K,K2,qt,splits,splits2", [
+    (1, 8, 64, 128, 2, 1, 2), (16, 72, 128, 64, 5, 2, 1), (33, 168, 192, 576, 4, 3, 5),
+    (64, 320, 1088, 448, 5, 5, 2), (32, 4104, 320, 640, 2, 2, 4),
+    # workgroups that go from a job of one product to one of the other
+    (3, 20000, 64, 192, 5, 1, 1), (64, 9000, 384, 128, 2, 3, 1),
+])
+def test_mid_pair(M, N, K, K2, qt, splits, splits2):
+    """Two products in one launch vs fp64: ends of tiles, one step of K to many, runs
+    of both, strided rows, nothing behind the sums."""
+    assert_native()
+    torch.manual_seed(M + N + K)
+    pairs = [(torch.randn(M, 2 * k, dtype=torch.bfloat16, device=DEV)[:, :k],
+              (torch.randn(N, k, device=DEV) * k ** -0.5).bfloat16(), n)
+             for k, n in ((K, splits), (K2, splits2))]
+    buf = torch.full((splits + splits2 + 1, M, N), 7.0, device=DEV)
+    ops._native().mid_pair(buf[:-1], *pairs[0][:2], *pairs[1][:2], qt, splits)
+    assert (buf[-1] == 7.0).all()
+    at = 0
+    for x, w, n in pairs:
+        xd, wd, k = x.double(), w.double(), x.shape[1]
+        slack = k * 2 ** -24 * (xd.abs() @ wd.abs().t())  # as in test_mid_gemm
+        ends = [k // 64 * i // n * 64 for i in range(n + 1)]
+        for lo, hi in zip(ends, ends[1:]):
+            run = xd[:, lo:hi] @ wd[:, lo:hi].t()
+            assert ((buf[at].double() - run).abs() <= slack).all()
+            at += 1
+
+
+@pytest.mark.parametrize("T,W,sy,sg", [
+    (1, 8, 1, 0), (3, 4096, 4, 2), (5, 4104, 0, 8), (2, 8192, 3, 9), (70, 136, 8, 1),
+])
+def test_gated_norm_of_sums(T, W, sy, sg):
+    """The residual's norm and the activation from products whose sums are not added
+    yet (s* of them; 0: bf16 rows), columns of wider ones among them, vs the same in
+    fp64."""
+    assert_native()
+    torch.manual_seed(T + W)
+
+    def product(splits, pad):
+        if not splits:
+            t = torch.randn(T, W + pad, dtype=torch.bfloat16, device=DEV)[:, pad:]
+            return t, t.double()
+        p = ops.Parts(torch.randn(splits, T, W + pad, device=DEV)).columns(pad, pad + W)
+        return p, p.sums.double().sum(0)
+
+    y, yd = product(sy, 0)
+    g, gd = product(sg, 24)
+    x, gb, w = (torch.randn(s, device=DEV) for s in ((T, W), (W,), (W,)))
+    z = yd * torch.sigmoid(gd + gb.double())
+    expect = x.double() + z * torch.rsqrt(
+        z.square().mean(1, keepdim=True) + 1e-6) * w.double()
+    xa = ops.gated_norm_residual(x, y, g, gb, w, 1e-6, torch.bfloat16)
+    # a dozen fp32 steps, the sums' and the reciprocals' among them
+    slack = 2 ** -19 * (expect.abs() + 8 * w.double().abs() + 1)
+    assert ((x.double() - expect).abs() <= slack).all()
+    assert torch.equal(xa, x.bfloat16())
+    for p, pd in ((y, yd), (g, gd)):
+        if isinstance(p, ops.Parts):
+            out = ops.gelu_tanh(p).double()
+            e = torch.nn.functional.gelu(pd, approximate="tanh")
+            assert ((out - e).abs() <= 2 ** -8 * e.abs() + 2 ** -18 * (1 + pd.abs())).all()
+
+
 @pytest.mark.parametrize("M,N,K,splits", [
     (1, 8, 64, 1), (129, 136, 128, 2), (257, 328, 192, 3), (320, 72, 320, 2),
     # workgroups that go from tile to tile, of one step and of several
