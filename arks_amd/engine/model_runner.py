@@ -123,6 +123,8 @@ class ModelRunner:
         # every reachable position (OOB table reads fault on GPU)
         if hasattr(self.model, "extend_rope_table"):
             self.model.extend_rope_table(self.cfg.max_model_len)
+        if self.cfg.kv_cache_dtype == "fp8":
+            ops.plain_prompts(self.model.parameters())
         self._weights_loaded = True
 
     def profile_num_blocks(self) -> int:

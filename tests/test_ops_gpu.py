@@ -1659,6 +1659,23 @@ def test_mid_gemm(M, N, K, qt, splits, kind):
             <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(93, 512, 4096), (300, 1024, 8192)])
+def test_plain_prompts(M, N, K):
+    """Prompts' products of weights beside fp8 pages reach their norm as the rounded
+    rows that linear_bf16 without wide_gemm gives, those of other weights as sums."""
+    assert_native()
+    torch.manual_seed(M)
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = torch.nn.Parameter((torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16(),
+                           requires_grad=False)
+    assert isinstance(ops.linear_parts(x, w, own_cut=False), ops.Parts)
+    ops.plain_prompts([w])
+    y = ops.linear_parts(x, w, own_cut=False)
+    assert not ops._wide_takes(x, w)
+    assert torch.equal(y, ops.linear_bf16(x, w) if M <= 256
+                       else torch.nn.functional.linear(x, w))
+
+
 @pytest.mark.parametrize("M,N,K,K2,qt,splits,splits2", [
     (1, 8, 64, 128, 2, 1, 2), (16, 72, 128, 64, 5, 2, 1), (33, 168, 192, 576, 4, 3, 5),
     (64, 320, 1088, 448, 5, 5, 2), (32, 4104, 320, 640, 2, 2, 4),
