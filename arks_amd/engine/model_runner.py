@@ -299,12 +299,14 @@ class ModelRunner:
                 )
             t64, t256, singles, ctab, ws_rows = (
                 ext_tiles or (None, None, (None, None), None, 0))
+            state = self._state_fields(sb.seqs, q_lens)
             (input_ids, positions, slot_mapping, cu_seqlens, seq_lens, bt,
-             logits_indices, t64, t256, ctab, drows, dseqs) = ops.upload(
+             logits_indices, t64, t256, ctab, drows, dseqs,
+             *values) = ops.upload(
                 [input_ids, positions, slot_mapping,
                  torch.tensor(cu, dtype=torch.int32), seq_lens, bt,
                  torch.tensor(logits_idx, dtype=torch.int64), t64, t256, ctab,
-                 *singles], self.device)
+                 *singles, *state.values()], self.device)
             return ForwardBatch(
                 is_prefill=True,
                 input_ids=input_ids,
@@ -317,7 +319,7 @@ class ModelRunner:
                 ext_tiles=(ext_tiles and
                            (t64, t256, (drows, dseqs), ctab, ws_rows)),
                 logits_indices=logits_indices,
-                **self._state_fields(sb.seqs, q_lens),
+                **dict(zip(state, values)),
             )
         # decode
         input_ids = [s.last_token() for s in sb.seqs]
@@ -335,6 +337,7 @@ class ModelRunner:
             )
             seq.num_cached_tokens = seq.num_tokens
         dev = self.device
+        state = self._state_fields(sb.seqs, [1] * len(sb.seqs))
         return ForwardBatch(
             is_prefill=False,
             input_ids=torch.tensor(input_ids, dtype=torch.int64, device=dev),
@@ -345,7 +348,7 @@ class ModelRunner:
             **(dict(cu_seqlens=torch.arange(len(sb.seqs) + 1, dtype=torch.int32,
                                             device=dev),
                     seq_lens_list=[1] * len(sb.seqs),
-                    **self._state_fields(sb.seqs, [1] * len(sb.seqs)))
+                    **dict(zip(state, ops.upload(list(state.values()), dev))))
                if self.seq_state else {}),
         )
 
@@ -370,17 +373,16 @@ class ModelRunner:
             at += n
 
     def _state_fields(self, seqs: list[Sequence], q_lens: list[int]) -> dict:
-        """ForwardBatch fields of models with per-sequence state."""
+        """ForwardBatch fields of models with per-sequence state, on the host."""
         if not self.seq_state:
             return {}
         import numpy as np
 
-        dev = self.device
         return dict(
             state_slots=torch.tensor([s.state_slot for s in seqs],
-                                     dtype=torch.int32, device=dev),
+                                     dtype=torch.int32),
             token_seq=torch.from_numpy(np.repeat(
-                np.arange(len(seqs), dtype=np.int32), q_lens)).to(dev),
+                np.arange(len(seqs), dtype=np.int32), q_lens)),
             max_q_len=max(q_lens),
             kv_lens_list=[s.num_cached_tokens for s in seqs],
         )
@@ -473,29 +475,24 @@ class ModelRunner:
             self._staging_event = torch.cuda.Event()
         else:
             self._staging_event.synchronize()
-        ops.stage_rows([s.prompt_token_ids for s in sb.seqs],
-                       [s.output_token_ids for s in sb.seqs],
-                       [s.block_table for s in sb.seqs], None, None,
-                       b["h_input_ids"], b["h_positions"], b["h_slot_mapping"],
-                       b["h_seq_lens"], b["h_block_tables"],
-                       self.cfg.block_size)
-        for seq in sb.seqs:
-            seq.num_cached_tokens = seq.num_tokens
+        prompts = [s.prompt_token_ids for s in sb.seqs]
+        outputs = [s.output_token_ids for s in sb.seqs]
+        ops.stage_rows(prompts, outputs, [s.block_table for s in sb.seqs], None,
+                       None, b["h_input_ids"], b["h_positions"],
+                       b["h_slot_mapping"], b["h_seq_lens"],
+                       b["h_block_tables"], self.cfg.block_size, bs)
         if self.seq_state:
-            b["h_state_slots"][:B] = torch.tensor(
-                [s.state_slot for s in sb.seqs], dtype=torch.int32)
-            b["h_state_slots"][B:bs] = -1
-        if B < bs:  # neutralize padding rows
-            b["h_input_ids"][B:bs] = 0
-            b["h_positions"][B:bs] = 0
-            b["h_slot_mapping"][B:bs] = -1
-            b["h_seq_lens"][B:bs] = 1
-            b["h_block_tables"][B:bs, 0] = 0
+            b["h_state_slots"][:bs] = torch.tensor(
+                [s.state_slot for s in sb.seqs] + [-1] * (bs - B),
+                dtype=torch.int32)
         n = b["small"] + bs * b["row"]
         b["all"][:n].copy_(b["h_all"][:n], non_blocking=True)
         self._staging_event.record()
         gr = self._graphs[bs]
         gr.graph.replay()
+        # (while the step runs)
+        for seq, p, o in zip(sb.seqs, prompts, outputs):
+            seq.num_cached_tokens = len(p) + len(o)
         return gr.logits[:B]
 
     # ---------------- execution ----------------
@@ -688,8 +685,10 @@ class ModelRunner:
                         device=logits.device, generator=gen,
                     )
             ids = ops.sample_tokens(logits.contiguous(), t, u)
-        out = ids.tolist()
-        self._last_logprobs = self._gather_logprobs(logits, seqs, out)
+        scored = any(s.sampling.logprobs is not None for s in seqs)
+        out = ids.tolist()  # waits for the step
+        self._last_logprobs = (self._gather_logprobs(logits, seqs, out)
+                               if scored else None)
         return out
 
     _last_logprobs: dict | None = None

@@ -248,13 +248,19 @@ class Scheduler:
         # Ensure each running sequence has a slot for its next token;
         # preempt from the back (most recent) on exhaustion.
         scheduled: list[Sequence] = []
+        bs = self.allocator.block_size
         i = 0
         while i < len(self.running):
             seq = self.running[i]
-            need = BlockAllocator.blocks_needed(
-                seq.num_tokens, self.allocator.block_size
-            ) - len(seq.block_table)
-            if need > 0 and not self.allocator.can_allocate(need):
+            # (spelled out: a step of 200 sequences waits for this loop)
+            if (len(seq.prompt_token_ids) + len(seq.output_token_ids)
+                    <= len(seq.block_table) * bs):
+                scheduled.append(seq)
+                i += 1
+                continue
+            need = (BlockAllocator.blocks_needed(seq.num_tokens, bs)
+                    - len(seq.block_table))
+            if not self.allocator.can_allocate(need):
                 # Victims must be unvisited (not already in this batch).
                 if not self._preempt_last(exclude=seq, protected=scheduled):
                     # nothing left to preempt but this seq itself
@@ -262,8 +268,7 @@ class Scheduler:
                     self.running.remove(seq)
                     continue
                 continue  # retry same seq
-            if need > 0:
-                seq.block_table.extend(self.allocator.allocate(need))
+            seq.block_table.extend(self.allocator.allocate(need))
             scheduled.append(seq)
             i += 1
         if not scheduled:

@@ -172,10 +172,11 @@ def attention_prefill_varlen(q, k, v, cu_seqlens, seq_lens: list[int],
 
 
 def stage_rows(prompts: list, outputs: list, tables: list, starts, counts, ids,
-               pos, slots, lens, block_tables, block_size: int) -> None:
+               pos, slots, lens, block_tables, block_size: int,
+               rows: int = 0) -> None:
     """What a step's rows read, into host tensors (see bindings.cpp)."""
     _native().stage_rows(prompts, outputs, tables, starts, counts, ids, pos,
-                         slots, lens, block_tables, block_size)
+                         slots, lens, block_tables, block_size, rows)
 
 
 def upload(tensors: list, device) -> list:
@@ -1799,13 +1800,14 @@ def scan_chunks(q_lens: list[int], device, chunk: int = SCAN_CHUNK) -> dict:
     for n in q_lens:
         rows += [min(chunk, n - j) for j in range(0, n, chunk)]
         off.append(len(rows))
-    t = lambda x: torch.tensor(x, dtype=torch.int32, device=device)
     cu = [0]
     for r in rows:
         cu.append(cu[-1] + r)
-    return {"n": len(rows), "cu": t(cu), "lens0": t(rows),
-            "lens1": t([r + 1 for r in rows]), "rows": t(rows),
-            "slots": t(list(range(len(rows)))), "off": t(off)}
+    cu, lens0, lens1, slots, off = upload(
+        [torch.tensor(x, dtype=torch.int32) for x in (
+            cu, rows, [r + 1 for r in rows], list(range(len(rows))), off)], device)
+    return {"n": len(rows), "cu": cu, "lens0": lens0, "lens1": lens1,
+            "rows": lens0, "slots": slots, "off": off}
 
 
 # the lightning kernels' input convention without positions: rows pass

@@ -793,12 +793,13 @@ void mid_pair(torch::Tensor out, torch::Tensor a, torch::Tensor w,
 // positions and cache slots, packed; its length behind them into lens[i], its
 // page numbers into row i of block_tables (what stands behind them stays). Lists
 // are walked here because a step waits for it: 200 requests with 8700 pages take
-// 400 us in Python, 30 here.
+// 400 us in Python, 30 here. rows (one token each): those behind the sequences' are
+// padding up to there, without a cache slot, of length 1.
 void stage_rows(pybind11::list prompts, pybind11::list outputs,
                 pybind11::list tables, pybind11::object starts,
                 pybind11::object counts, torch::Tensor ids, torch::Tensor pos,
                 torch::Tensor slots, torch::Tensor lens,
-                torch::Tensor block_tables, int64_t block_size) {
+                torch::Tensor block_tables, int64_t block_size, int64_t rows) {
   const Py_ssize_t n = PyList_GET_SIZE(prompts.ptr());
   auto host = [](const torch::Tensor& t, torch::ScalarType type, int64_t least) {
     TORCH_CHECK(!t.is_cuda() && t.scalar_type() == type && t.is_contiguous() &&
@@ -813,12 +814,15 @@ void stage_rows(pybind11::list prompts, pybind11::list outputs,
               PyList_GET_SIZE(tables.ptr()) == n &&
               (last || (PyList_GET_SIZE(from.ptr()) == n &&
                         PyList_GET_SIZE(many.ptr()) == n)));
-  host(lens, torch::kInt32, n);
+  TORCH_CHECK(rows <= n || last, "stage_rows: padding is of rows of one token");
+  const int64_t most = std::max<int64_t>(n, rows);
+  host(lens, torch::kInt32, most);
   host(block_tables, torch::kInt32, 0);
-  TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) >= n);
-  host(ids, torch::kInt64, last ? n : 0);
-  host(pos, torch::kInt64, last ? n : 0);
-  host(slots, torch::kInt64, last ? n : 0);
+  TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) >= most &&
+              (rows <= n || block_tables.size(1) >= 1));
+  host(ids, torch::kInt64, last ? most : 0);
+  host(pos, torch::kInt64, last ? most : 0);
+  host(slots, torch::kInt64, last ? most : 0);
   const int64_t room =
       std::min({ids.numel(), pos.numel(), slots.numel()});
   const int64_t width = block_tables.size(1);
@@ -858,6 +862,12 @@ void stage_rows(pybind11::list prompts, pybind11::list outputs,
       to_slots[at] = (int64_t)row[j / block_size] * block_size + j % block_size;
     }
     to_lens[i] = (int32_t)(s + c);
+  }
+  for (int64_t i = n; i < rows; ++i) {
+    to_ids[i] = to_pos[i] = 0;
+    to_slots[i] = -1;
+    to_lens[i] = 1;
+    to_table[i * width] = 0;
   }
 }
 

@@ -3,6 +3,7 @@ tested against) — internal consistency checks that run without a GPU."""
 
 import math
 
+import pytest
 import torch
 
 from arks_amd.ops import ref
@@ -206,6 +207,33 @@ def test_stage_rows():
         with pytest.raises((RuntimeError, TypeError)):
             ops.stage_rows(prompts, a["outputs"], a["tables"], a["starts"],
                            a["counts"], *a["bufs"], bs)
+
+
+@pytest.mark.parametrize("rows", [0, 1, 2, 5])
+def test_stage_rows_pads(rows):
+    """Rows behind the sequences': no cache slot, length 1, page 0; nothing beyond."""
+    import arks_amd.ops as ops
+
+    if not ops.native_available():
+        pytest.skip("needs the built extension")
+    ids, pos, slots = torch.full((3, 6), -7).unbind()
+    lens = torch.full((6,), -7, dtype=torch.int32)
+    bt = torch.full((6, 3), -7, dtype=torch.int32)
+    ops.stage_rows([[4, 5, 6], [7]], [[], [8]], [[2], [9]], None, None, ids, pos,
+                   slots, lens, bt, 16, rows)
+    pad = max(0, rows - 2)
+    rest = [-7] * (4 - pad)
+    assert ids.tolist() == [6, 8] + [0] * pad + rest
+    assert pos.tolist() == [2, 1] + [0] * pad + rest
+    assert slots.tolist() == [34, 145] + [-1] * pad + rest
+    assert lens.tolist() == [3, 2] + [1] * pad + rest
+    assert bt[:, 0].tolist() == [2, 9] + [0] * pad + rest
+    for bad in (7, dict(starts=[0, 0], counts=[1, 1])):  # no room; not one token each
+        a = dict(starts=None, counts=None) | (bad if isinstance(bad, dict) else {})
+        with pytest.raises(RuntimeError):
+            ops.stage_rows([[4], [7]], [[], []], [[2], [9]], a["starts"], a["counts"],
+                           ids, pos, slots, lens, bt, 16,
+                           bad if isinstance(bad, int) else 3)
 
 
 def test_objects_older_than_a_header_are_built_again(tmp_path):
