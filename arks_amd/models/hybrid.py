@@ -211,9 +211,23 @@ class HybridBlock(nn.Module):
             out["shift"] = ("slot", (self.width,), torch.float32)
         return out
 
-    def forward(self, x, batch: ForwardBatch, cache: dict, dtype) -> None:
-        """x: fp32 residual rows [T, width], updated in place."""
-        if self.shift is not None:
+    def forward(self, x, batch: ForwardBatch, cache: dict, dtype, shifted=None,
+                after=None):
+        """x: fp32 residual rows [T, width], updated in place. shifted: this
+        layer's token shift of them, if the layer in front has made it; after: the
+        layer behind and its cache, if this one is to make that layer's
+        (ops.norm_shift_takes), which is returned."""
+        def end(*args):
+            if after is None:
+                return ops.gated_norm_residual(x, *args, self.eps, None)
+            layer, held = after
+            return ops.gated_norm_shift(x, *args, self.eps, layer.shift,
+                                        held["shift"], batch.seq_lens,
+                                        batch.state_slots)
+
+        if shifted is not None:
+            xs, xa = shifted
+        elif self.shift is not None:
             xs, xa = ops.token_shift(
                 x, self.shift, cache["shift"], batch.cu_seqlens,
                 batch.seq_lens, batch.state_slots, batch.token_seq, dtype)
@@ -226,14 +240,17 @@ class HybridBlock(nn.Module):
         else:
             y = self.mixer(xs, batch, cache)
             g = linear(xa, self.rg1) if self.rg1 is not None else None
-        xa = ops.gated_norm_residual(x, y, g, self.rg1_b, self.norm1, self.eps,
-                                     dtype if self.ff else None)
-        if self.ff:
+        if not self.ff:
+            shifted = end(y, g, self.rg1_b, self.norm1)
+        else:
+            xa = ops.gated_norm_residual(x, y, g, self.rg1_b, self.norm1, self.eps,
+                                         dtype)
             ug = linear_parts(xa, self.up_gate)
             y = linear_parts(ops.gelu_tanh(_columns(ug, 0, self.ff)), self.down)
             g = (_columns(ug, self.ff, self.ff + self.width)
                  if self.arr.gated_residual else None)
-            ops.gated_norm_residual(x, y, g, self.rg2_b, self.norm2, self.eps, None)
+            shifted = end(y, g, self.rg2_b, self.norm2)
+        return shifted if after is not None else None
 
 
 class StreamBlock(nn.Module):
@@ -602,8 +619,17 @@ class HybridForCausalLM(nn.Module):
         if self.arr.norm_place in ("sandwich", "pre"):
             return self._forward_sandwich(batch, caches)
         x = self.embed[batch.input_ids].float()
+        fuse = self.arr.token_shift and ops.norm_shift_takes(x, batch, self.dtype)
+        shifted = None
         for i, layer in enumerate(self.layers):
-            layer(x, batch, caches[i], self.dtype)
+            if fuse and all(passable(b, HybridBlock) for b in self.layers[i:i + 2]):
+                after = ((self.layers[i + 1], caches[i + 1])
+                         if i + 1 < len(self.layers) else None)
+                shifted = layer(x, batch, caches[i], self.dtype, shifted, after)
+            elif shifted is not None:
+                shifted = layer(x, batch, caches[i], self.dtype, shifted)
+            else:
+                layer(x, batch, caches[i], self.dtype)
             if self.residual_tap is not None:
                 self.residual_tap(i, x)
         if batch.logits_indices is not None:

@@ -1625,9 +1625,8 @@ def gated_norm_residual(x, y, gate, gate_bias, weight, eps, out_dtype=None):
             xa = (torch.empty(x.shape, dtype=out_dtype, device=x.device)
                   if out_dtype is not None else None)
             _native_seq().gated_norm_sums(
-                x, xa, *(p.sums if isinstance(p, Parts)
-                         else p if p is None else _rows_16b(p)
-                         for p in (y, gate)), gate_bias, weight, eps)
+                x, xa, *map(_sums_or_rows, (y, gate)), gate_bias, weight, eps,
+                None, None, None, None, None)
             return xa
         y, gate = parts_sum(y), parts_sum(gate)
     if x.is_cuda:
@@ -1641,6 +1640,29 @@ def gated_norm_residual(x, y, gate, gate_bias, weight, eps, out_dtype=None):
         _native_seq().gated_norm_residual(x, xa, y, gate, gate_bias, weight, eps)
         return x if ret_x else xa
     return ref.gated_norm_residual(x, y, gate, gate_bias, weight, eps, out_dtype)
+
+
+def _sums_or_rows(p):
+    return p.sums if isinstance(p, Parts) else p if p is None else _rows_16b(p)
+
+
+def norm_shift_takes(x, batch, out_dtype) -> bool:
+    """Whether gated_norm_shift takes a step's residual rows: one a sequence."""
+    return (x.is_cuda and out_dtype == torch.bfloat16 and batch.max_q_len == 1
+            and batch.seq_lens.shape[0] == x.shape[0] and x.shape[1] % 8 == 0
+            and x.shape[1] <= 8192)
+
+
+def gated_norm_shift(x, y, gate, gate_bias, weight, eps, shift_w, prev_state,
+                     seq_lens, state_slots):
+    """gated_norm_residual, then token_shift of its rows (in bf16, one a sequence:
+    norm_shift_takes) for the layer behind, from one launch."""
+    xs, xa = (torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
+              for _ in range(2))
+    _native_seq().gated_norm_sums(
+        x, xa, *map(_sums_or_rows, (y, gate)), gate_bias, weight, eps, xs, shift_w,
+        prev_state, seq_lens, state_slots)
+    return xs, xa
 
 
 def rms_norm_f32(x, weight, eps, out_dtype):

@@ -23,7 +23,9 @@ void arks_seq_gated_norm_sums(void* x, void* xa, const void* y, int64_t ldy,
                               int64_t part_y, int splits_y, const void* g,
                               int64_t ldg, int64_t part_g, int splits_g,
                               const void* gb, const void* w, float eps, int T,
-                              int W, hipStream_t stream);
+                              int W, void* xs, const void* shift_w, void* state,
+                              const void* seq_lens, const void* slots,
+                              hipStream_t stream);
 void arks_seq_gelu_tanh_sums(void* out, const void* x, int64_t ldx, int64_t part,
                              int splits, int64_t rows, int n,
                              hipStream_t stream);
@@ -432,9 +434,12 @@ ProductRows product_rows(const Tensor& t, int64_t T, int64_t W, const char* name
           sums ? (int)t.size(0) : 0};
 }
 
-// gated_norm_residual (bf16 rows) where y or the gate are sums
+// gated_norm_residual (bf16 rows) where y or the gate may be sums; with xs, the token
+// shift of rows that are a sequence each behind it
 void gated_norm_sums(Tensor x, OptTensor xa, Tensor y, OptTensor gate,
-                     OptTensor gate_bias, Tensor w, double eps) {
+                     OptTensor gate_bias, Tensor w, double eps, OptTensor xs,
+                     OptTensor shift_w, OptTensor state, OptTensor seq_lens,
+                     OptTensor slots) {
   check_f32(x, "x");
   check_f32(w, "norm weight");
   TORCH_CHECK(x.dim() == 2);
@@ -456,9 +461,29 @@ void gated_norm_sums(Tensor x, OptTensor xa, Tensor y, OptTensor gate,
                 xa->is_contiguous() && xa->sizes() == x.sizes());
     xa_p = xa->data_ptr();
   }
+  void* shift[5] = {};
+  if (xs.has_value()) {
+    TORCH_CHECK(shift_w.has_value() && state.has_value() && seq_lens.has_value() &&
+                slots.has_value());
+    TORCH_CHECK(xs->is_cuda() && xs->scalar_type() == torch::kBFloat16 &&
+                xs->is_contiguous() && xs->sizes() == x.sizes());
+    check_f32(*shift_w, "shift weight");
+    check_f32(*state, "shift state");
+    check_i32(*seq_lens, "seq_lens");
+    check_i32(*slots, "state_slots");
+    TORCH_CHECK(shift_w->numel() == W && state->dim() == 2 && state->size(1) == W &&
+                seq_lens->numel() == T && slots->numel() == T,
+                "the shift is of one row a sequence");
+    shift[0] = xs->data_ptr();
+    shift[1] = shift_w->data_ptr();
+    shift[2] = state->data_ptr();
+    shift[3] = seq_lens->data_ptr();
+    shift[4] = slots->data_ptr();
+  }
   arks_seq_gated_norm_sums(x.data_ptr(), xa_p, yr.p, yr.ld, yr.part, yr.splits,
                            gr.p, gr.ld, gr.part, gr.splits, gb_p, w.data_ptr(),
-                           (float)eps, (int)T, (int)W, current_stream());
+                           (float)eps, (int)T, (int)W, shift[0], shift[1],
+                           shift[2], shift[3], shift[4], current_stream());
 }
 
 void gelu_tanh_sums(Tensor out, Tensor sums) {

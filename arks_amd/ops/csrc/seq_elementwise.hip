@@ -152,27 +152,103 @@ __device__ __forceinline__ void sum_rows8(const SumRows& in, const int t,
   }
 }
 
+// The same of two products, U runs of both in flight (loads of runs that are not
+// there repeat the last one, and take as long as others).
+template <int U>
+__device__ __forceinline__ void sum_rows8_two(const SumRows& a, const SumRows& b,
+                                              const int t, const int i,
+                                              float (&va)[8], float (&vb)[8]) {
+  if (a.splits == 0 || b.splits == 0) {
+    sum_rows8(a, t, i, va);
+    sum_rows8(b, t, i, vb);
+    return;
+  }
+  const float* pa = reinterpret_cast<const float*>(a.p) + t * a.ld + i;
+  const float* pb = reinterpret_cast<const float*>(b.p) + t * b.ld + i;
+  f32x4 sum[4] = {};
+  for (int s0 = 0; s0 < max(a.splits, b.splits); s0 += U) {
+    f32x4 v[U][4];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const float* qa = pa + min(s0 + j, a.splits - 1) * a.part;
+      const float* qb = pb + min(s0 + j, b.splits - 1) * b.part;
+      v[j][0] = *reinterpret_cast<const f32x4*>(qa);
+      v[j][1] = *reinterpret_cast<const f32x4*>(qa + 4);
+      v[j][2] = *reinterpret_cast<const f32x4*>(qb);
+      v[j][3] = *reinterpret_cast<const f32x4*>(qb + 4);
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      if (s0 + j < a.splits) {
+        sum[0] += v[j][0];
+        sum[1] += v[j][1];
+      }
+      if (s0 + j < b.splits) {
+        sum[2] += v[j][2];
+        sum[3] += v[j][3];
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    va[e] = sum[e / 4][e % 4];
+    vb[e] = sum[2 + e / 4][e % 4];
+  }
+}
+
+// The token shift of the layer behind, of rows that are a sequence each (as
+// token_shift_vec8_kernel; no w: none).
+struct ShiftRows {
+  bf16* __restrict__ xs;
+  const float* __restrict__ w;
+  float* __restrict__ state;
+  const int* __restrict__ seq_lens;
+  const int* __restrict__ slots;
+};
+
 // gated_norm_residual_vec8 of products whose sums are not added yet: a row is a
 // chain of loads, so its threads have 8 columns each up to W 4096 and ask for all
-// sums of both products at once.
+// sums of both products at once, U runs of each (loads that repeat take as long
+// as others). A step of one row a sequence shifts the row
+// for the layer behind it on the way. us, 8 rows of 4096, both apart -> here: 2 + 2
+// sums 7.4 -> 5.0, 4 + 2 7.9 -> 5.5, 8 + 4 9.0 -> 6.7; 1 row 7.0 -> 4.9.
+template <int U>
 __global__ __launch_bounds__(512) void gated_norm_sums_kernel(
     float* __restrict__ x, bf16* __restrict__ xa, const SumRows y,
     const SumRows g, const float* __restrict__ gb, const float* __restrict__ w,
-    const float eps, const int W) {
+    const float eps, const int W, const ShiftRows shift) {
   __shared__ float scratch[8];
   constexpr int VPT = 2;  // W <= 8 * 512 * VPT
   const int t = blockIdx.x;
   float* xr = x + (int64_t)t * W;
+  const int slot = shift.w ? shift.slots[t] : -1;
+  const bool held = slot >= 0 && shift.seq_lens[t] > 1;
+  float* prev = shift.state + (int64_t)max(slot, 0) * W;
+  // what the end of the row takes is asked for here too: behind the reduction it
+  // would be another wait
   float z[VPT][8];
+  float4v xv[VPT][2], wv[VPT][2], pv[VPT][2], sv[VPT][2];
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int i = (k * 512 + threadIdx.x) * 8;
     if (i < W) {
-      sum_rows8(y, t, i, z[k]);
-      if (g.p) {
+#pragma unroll
+      for (int hlf = 0; hlf < 2; ++hlf) {
+        const int j = i + 4 * hlf;
+        xv[k][hlf] = *reinterpret_cast<const float4v*>(xr + j);
+        wv[k][hlf] = *reinterpret_cast<const float4v*>(w + j);
+        if (shift.w) {
+          pv[k][hlf] = float4v{0.f, 0.f, 0.f, 0.f};
+          if (held) pv[k][hlf] = *reinterpret_cast<const float4v*>(prev + j);
+          sv[k][hlf] = *reinterpret_cast<const float4v*>(shift.w + j);
+        }
+      }
+      if (!g.p) {
+        sum_rows8(y, t, i, z[k]);
+      } else {
         float gv[8];
-        sum_rows8(g, t, i, gv);
+        sum_rows8_two<U>(y, g, t, i, z[k], gv);
         const float4v b0 = *reinterpret_cast<const float4v*>(gb + i);
         const float4v b1 = *reinterpret_cast<const float4v*>(gb + i + 4);
 #pragma unroll
@@ -189,20 +265,27 @@ __global__ __launch_bounds__(512) void gated_norm_sums_kernel(
   for (int k = 0; k < VPT; ++k) {
     const int i = (k * 512 + threadIdx.x) * 8;
     if (i < W) {
-      ushort8 o;
+      ushort8 o, os;
 #pragma unroll
       for (int hlf = 0; hlf < 2; ++hlf) {
         const int j = i + 4 * hlf;
-        float4v xv = *reinterpret_cast<const float4v*>(xr + j);
-        const float4v wv = *reinterpret_cast<const float4v*>(w + j);
+        float4v nx = xv[k][hlf];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          xv[e] += z[k][4 * hlf + e] * rstd * wv[e];
-          o[4 * hlf + e] = float_to_bf16_bits(xv[e]);
+          nx[e] += z[k][4 * hlf + e] * rstd * wv[k][hlf][e];
+          o[4 * hlf + e] = float_to_bf16_bits(nx[e]);
         }
-        *reinterpret_cast<float4v*>(xr + j) = xv;
+        *reinterpret_cast<float4v*>(xr + j) = nx;
+        if (shift.w) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            os[4 * hlf + e] = float_to_bf16_bits(
+                nx[e] + (pv[k][hlf][e] - nx[e]) * sv[k][hlf][e]);
+          if (slot >= 0) *reinterpret_cast<float4v*>(prev + j) = nx;
+        }
       }
       if (xa) *reinterpret_cast<ushort8*>(xa + (int64_t)t * W + i) = o;
+      if (shift.w) *reinterpret_cast<ushort8*>(shift.xs + (int64_t)t * W + i) = os;
     }
   }
 }
@@ -702,16 +785,25 @@ extern "C" void arks_seq_gated_norm_residual(void* x, void* xa, const void* y,
 }
 
 // y and g (null: no gate): bf16 rows, or sums (splits > 0) on 16 bytes; W % 8 == 0,
-// W <= 8192
+// W <= 8192; shift_w (null: no shift): xs takes the shifted rows, one a sequence
 extern "C" void arks_seq_gated_norm_sums(
     void* x, void* xa, const void* y, int64_t ldy, int64_t part_y, int splits_y,
     const void* g, int64_t ldg, int64_t part_g, int splits_g, const void* gb,
-    const void* w, float eps, int T, int W, hipStream_t stream) {
+    const void* w, float eps, int T, int W, void* xs, const void* shift_w,
+    void* state, const void* seq_lens, const void* slots, hipStream_t stream) {
   if (T == 0) return;
-  hipLaunchKernelGGL(gated_norm_sums_kernel, dim3(T), dim3(512), 0, stream,
-                     (float*)x, (bf16*)xa, SumRows{y, ldy, part_y, splits_y},
-                     SumRows{g, ldg, part_g, splits_g}, (const float*)gb,
-                     (const float*)w, eps, W);
+  const int most = splits_y > splits_g ? splits_y : splits_g;
+#define ARKS_GN(U)                                                             \
+  hipLaunchKernelGGL((gated_norm_sums_kernel<U>), dim3(T), dim3(512), 0, stream, \
+                     (float*)x, (bf16*)xa, SumRows{y, ldy, part_y, splits_y},  \
+                     SumRows{g, ldg, part_g, splits_g}, (const float*)gb,      \
+                     (const float*)w, eps, W,                                  \
+                     ShiftRows{(bf16*)xs, (const float*)shift_w, (float*)state, \
+                               (const int*)seq_lens, (const int*)slots})
+  if (most <= 2) ARKS_GN(2);
+  else if (most <= 4) ARKS_GN(4);
+  else ARKS_GN(8);
+#undef ARKS_GN
 }
 
 // x: sums on 16 bytes, n % 8 == 0

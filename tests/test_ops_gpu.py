@@ -1727,7 +1727,18 @@ def test_gated_norm_of_sums(T, W, sy, sg):
     z = yd * torch.sigmoid(gd + gb.double())
     expect = x.double() + z * torch.rsqrt(
         z.square().mean(1, keepdim=True) + 1e-6) * w.double()
+    x0, sw, state = x.clone(), torch.rand(W, device=DEV), torch.randn(9, W, device=DEV)
     xa = ops.gated_norm_residual(x, y, g, gb, w, 1e-6, torch.bfloat16)
+    # with the shift behind it: rows that hold a state, begin, or have no slot
+    if T <= 5:
+        lens, slots = (torch.tensor(v[:T], dtype=torch.int32, device=DEV)
+                       for v in ([7, 1, 2, 5, 1], [3, 0, 8, -1, -1]))
+        seqs = torch.arange(T + 1, dtype=torch.int32, device=DEV)
+        s2 = state.clone()
+        got = ops.gated_norm_shift(x0, y, g, gb, w, 1e-6, sw, state, lens, slots)
+        want = ops.token_shift(x, sw, s2, seqs, lens, slots, seqs[:T], torch.bfloat16)
+        assert torch.equal(x0, x) and torch.equal(state, s2)
+        assert all(map(torch.equal, got, want))
     # a dozen fp32 steps, the sums' and the reciprocals' among them
     slack = 2 ** -19 * (expect.abs() + 8 * w.double().abs() + 1)
     assert ((x.double() - expect).abs() <= slack).all()
