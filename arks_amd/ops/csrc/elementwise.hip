@@ -27,7 +27,7 @@ namespace arks {
 // and 4 splits 3.84 us back to back, with the rows as an argument 3.69).
 // ---------------------------------------------------------------------------
 enum NormInput { IN_ROWS, IN_PARTS, IN_MIX };
-template <bool FUSED_ADD, NormInput IN, int NV>
+template <bool FUSED_ADD, NormInput IN, int NV, int U = 8>
 __global__ void rmsnorm_kernel(bf16* __restrict__ out,
                                const void* __restrict__ input,
                                bf16* __restrict__ residual,  // null unless FUSED_ADD
@@ -57,8 +57,8 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
     if constexpr (FUSED_ADD) r = *reinterpret_cast<const ushort8*>(res_row + i * 8);
     if constexpr (PARTS) {
       f32x4 lo, hi;
-      sum_parts_pair(part_row + i * 8, part_row + i * 8 + 4, part_stride,
-                     n_in, lo, hi);
+      sum_parts_pair<U>(part_row + i * 8, part_row + i * 8 + 4, part_stride,
+                        n_in, lo, hi);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = j < 4 ? lo[j % 4] : hi[j % 4];
     } else {
@@ -205,11 +205,19 @@ using namespace arks;
 
 extern "C" {
 
-#define ARKS_NORM(FUSED, IN, NV)                                               \
-  hipLaunchKernelGGL((rmsnorm_kernel<FUSED, IN, NV>), dim3(rows),              \
+#define ARKS_NORM_U(FUSED, IN, NV, U)                                          \
+  hipLaunchKernelGGL((rmsnorm_kernel<FUSED, IN, NV, U>), dim3(rows),           \
                      dim3(IN == IN_PARTS ? 512 : 256), 0, stream, (bf16*)out,  \
                      input, (bf16*)residual, (const bf16*)weight, eps, hidden, \
                      rows, n_in, (const float*)mix_weights, (const int*)mix_rows)
+#define ARKS_NORM(FUSED, IN, NV)                                               \
+  do {                                                                         \
+    constexpr bool P = IN == IN_PARTS;                                         \
+    const int u = P ? parts_flight(n_in) : 8;                                  \
+    if (u == 2) ARKS_NORM_U(FUSED, IN, NV, (P ? 2 : 8));                       \
+    else if (u == 4) ARKS_NORM_U(FUSED, IN, NV, (P ? 4 : 8));                  \
+    else ARKS_NORM_U(FUSED, IN, NV, 8);                                        \
+  } while (0)
 #define ARKS_NORM_V(FUSED, IN)                                                 \
   do {                                                                         \
     const int block = IN == IN_PARTS ? 512 : 256;                              \
@@ -256,6 +264,7 @@ void arks_fused_add_rmsnorm_mix(void* out, const void* input,
 }
 #undef ARKS_NORM_V
 #undef ARKS_NORM
+#undef ARKS_NORM_U
 
 void arks_silu_mul(void* out, const void* gate_up, int64_t rows, int d,
                    hipStream_t stream) {

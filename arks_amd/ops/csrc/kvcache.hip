@@ -128,7 +128,7 @@ namespace arks {
 // Few tokens and split sums keep 2: a thread's chain of loads is what they wait
 // for.
 // ---------------------------------------------------------------------------
-template <bool FP8, bool NORM, bool PARTS, int W>
+template <bool FP8, bool NORM, bool PARTS, int W, int U = 8>
 __global__ void rope_cache_kernel(
     const int64_t* __restrict__ positions,
     bf16* __restrict__ q,        // [T, Hq*D] rows strided
@@ -186,8 +186,8 @@ __global__ void rope_cache_kernel(
       static_assert(W == 2);
       const int c = h * head_dim + p2;
       f32x2 f1, f2;
-      sum_parts_pair(part_row + c, part_row + c + half, part_stride, splits, f1,
-                     f2);
+      sum_parts_pair<U>(part_row + c, part_row + c + half, part_stride, splits,
+                        f1, f2);
       a2[0] = f1.x, a2[1] = f1.y, b2[0] = f2.x, b2[1] = f2.y;
       if (bias) {
 #pragma unroll
@@ -272,8 +272,8 @@ __global__ void rope_cache_kernel(
     if constexpr (PARTS) {
       const int c = (num_q_heads + num_kv_heads) * head_dim + i * 8;
       f32x4 lo, hi;
-      sum_parts_pair(part_row + c, part_row + c + 4, part_stride, splits, lo,
-                     hi);
+      sum_parts_pair<U>(part_row + c, part_row + c + 4, part_stride, splits, lo,
+                        hi);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float b = bias ? bf16_bits_to_float(bias[c + e]) : 0.f;
@@ -356,8 +356,15 @@ extern "C" void arks_rope_and_cache_parts(
             rope_groups(num_tokens, num_q_heads + num_kv_heads, head_dim)),
       block(256);
 #define ARKS_ROPE(FP8, NORM)                                                   \
-  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, true, 2>), grid, block, 0,  \
-                     stream, (const int64_t*)positions, (bf16*)q, nullptr,     \
+  do {                                                                         \
+    const int u = parts_flight(splits);                                        \
+    if (u == 2) ARKS_ROPE_U(FP8, NORM, 2);                                     \
+    else if (u == 4) ARKS_ROPE_U(FP8, NORM, 4);                                \
+    else ARKS_ROPE_U(FP8, NORM, 8);                                            \
+  } while (0)
+#define ARKS_ROPE_U(FP8, NORM, U)                                              \
+  hipLaunchKernelGGL((rope_cache_kernel<FP8, NORM, true, 2, U>), grid, block,  \
+                     0, stream, (const int64_t*)positions, (bf16*)q, nullptr,     \
                      nullptr, k_cache, v_cache, (const int64_t*)slot_mapping,  \
                      (const float*)cos_sin, head_dim, num_q_heads,             \
                      num_kv_heads, block_size,                                 \
@@ -370,4 +377,5 @@ extern "C" void arks_rope_and_cache_parts(
     if (q_norm) ARKS_ROPE(false, true); else ARKS_ROPE(false, false);
   }
 #undef ARKS_ROPE
+#undef ARKS_ROPE_U
 }

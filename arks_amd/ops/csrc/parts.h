@@ -8,41 +8,50 @@ namespace arks {
 using f32x2 = __attribute__((ext_vector_type(2))) float;
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 
-// 4 columns of all splits, `stride` floats apart; 8 loads in flight
+// How many splits' loads are asked for at once (U below). Loads of splits that are not
+// there repeat the last one and take as long as others: us, always 8 -> so, 64 rows of
+// 3584 and their norm, 2 splits 3.43 -> 2.78, 4 splits 3.44 -> 2.99; 4608 columns to
+// be rotated, 3 splits 4.43 -> 3.90; 200 rows, 3 splits 5.23 -> 4.41.
+inline int parts_flight(const int splits) {
+  return splits <= 2 ? 2 : splits <= 4 ? 4 : 8;
+}
+
+// 4 columns of all splits, `stride` floats apart; U loads in flight
+template <int U>
 __device__ __forceinline__ f32x4 sum_parts4(const float* p,
                                             const int64_t stride,
                                             const int splits) {
   f32x4 s{0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < splits; s0 += 8) {
-    f32x4 v[8];
+  for (int s0 = 0; s0 < splits; s0 += U) {
+    f32x4 v[U];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < U; ++j)
       v[j] = *reinterpret_cast<const f32x4*>(
           p + (int64_t)min(s0 + j, splits - 1) * stride);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < U; ++j)
       if (s0 + j < splits) s += v[j];
   }
   return s;
 }
 
-// The same at two places, 16 loads in flight (1 x 3584, 8 splits and their
+// The same at two places, 2 * U loads in flight (1 x 3584, 8 splits and their
 // norm 4.6 us; one place after the other 5.4).
-template <typename T>
+template <int U, typename T>
 __device__ __forceinline__ void sum_parts_pair(const float* p, const float* q,
                                                const int64_t stride,
                                                const int splits, T& a, T& b) {
   a = b = T{};
-  for (int s0 = 0; s0 < splits; s0 += 8) {
-    T v[8], w[8];
+  for (int s0 = 0; s0 < splits; s0 += U) {
+    T v[U], w[U];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < U; ++j) {
       const int64_t at = (int64_t)min(s0 + j, splits - 1) * stride;
       v[j] = *reinterpret_cast<const T*>(p + at);
       w[j] = *reinterpret_cast<const T*>(q + at);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < U; ++j)
       if (s0 + j < splits) {
         a += v[j];
         b += w[j];

@@ -136,12 +136,13 @@ struct SumRows {
 };
 
 // 8 values from column i of row t on
+template <int U>
 __device__ __forceinline__ void sum_rows8(const SumRows& in, const int t,
                                           const int i, float (&v)[8]) {
   if (in.splits > 0) {
     const float* p = reinterpret_cast<const float*>(in.p) + t * in.ld + i;
     f32x4 lo, hi;
-    sum_parts_pair(p, p + 4, in.part, in.splits, lo, hi);
+    sum_parts_pair<U>(p, p + 4, in.part, in.splits, lo, hi);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = e < 4 ? lo[e % 4] : hi[e % 4];
   } else {
@@ -152,15 +153,14 @@ __device__ __forceinline__ void sum_rows8(const SumRows& in, const int t,
   }
 }
 
-// The same of two products, U runs of both in flight (loads of runs that are not
-// there repeat the last one, and take as long as others).
+// The same of two products, U runs of both in flight.
 template <int U>
 __device__ __forceinline__ void sum_rows8_two(const SumRows& a, const SumRows& b,
                                               const int t, const int i,
                                               float (&va)[8], float (&vb)[8]) {
   if (a.splits == 0 || b.splits == 0) {
-    sum_rows8(a, t, i, va);
-    sum_rows8(b, t, i, vb);
+    sum_rows8<U>(a, t, i, va);
+    sum_rows8<U>(b, t, i, vb);
     return;
   }
   const float* pa = reinterpret_cast<const float*>(a.p) + t * a.ld + i;
@@ -208,8 +208,7 @@ struct ShiftRows {
 
 // gated_norm_residual_vec8 of products whose sums are not added yet: a row is a
 // chain of loads, so its threads have 8 columns each up to W 4096 and ask for all
-// sums of both products at once, U runs of each (loads that repeat take as long
-// as others). A step of one row a sequence shifts the row
+// sums of both products at once, U runs of each (parts_flight). A step of one row a sequence shifts the row
 // for the layer behind it on the way. us, 8 rows of 4096, both apart -> here: 2 + 2
 // sums 7.4 -> 5.0, 4 + 2 7.9 -> 5.5, 8 + 4 9.0 -> 6.7; 1 row 7.0 -> 4.9.
 template <int U>
@@ -245,7 +244,7 @@ __global__ __launch_bounds__(512) void gated_norm_sums_kernel(
         }
       }
       if (!g.p) {
-        sum_rows8(y, t, i, z[k]);
+        sum_rows8<U>(y, t, i, z[k]);
       } else {
         float gv[8];
         sum_rows8_two<U>(y, g, t, i, z[k], gv);
@@ -431,6 +430,7 @@ __global__ __launch_bounds__(256) void gelu_tanh_kernel(
 
 // bf16, 8 elements per thread; tanh(u) = 1 - 2 / (1 + e^(2u)) with the
 // hardware exponential (saturates cleanly at both ends)
+template <int U>
 __global__ __launch_bounds__(256) void gelu_tanh_vec8_kernel(
     bf16* __restrict__ out, const SumRows x, int64_t rows, int n8) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(256) void gelu_tanh_vec8_kernel(
   const int64_t r = idx / n8;
   const int c = (int)(idx - r * n8) * 8;
   float v[8];
-  sum_rows8(x, (int)r, c, v);
+  sum_rows8<U>(x, (int)r, c, v);
   ushort8 o;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -792,7 +792,7 @@ extern "C" void arks_seq_gated_norm_sums(
     const void* w, float eps, int T, int W, void* xs, const void* shift_w,
     void* state, const void* seq_lens, const void* slots, hipStream_t stream) {
   if (T == 0) return;
-  const int most = splits_y > splits_g ? splits_y : splits_g;
+  const int u = parts_flight(splits_y > splits_g ? splits_y : splits_g);
 #define ARKS_GN(U)                                                             \
   hipLaunchKernelGGL((gated_norm_sums_kernel<U>), dim3(T), dim3(512), 0, stream, \
                      (float*)x, (bf16*)xa, SumRows{y, ldy, part_y, splits_y},  \
@@ -800,8 +800,8 @@ extern "C" void arks_seq_gated_norm_sums(
                      (const float*)w, eps, W,                                  \
                      ShiftRows{(bf16*)xs, (const float*)shift_w, (float*)state, \
                                (const int*)seq_lens, (const int*)slots})
-  if (most <= 2) ARKS_GN(2);
-  else if (most <= 4) ARKS_GN(4);
+  if (u == 2) ARKS_GN(2);
+  else if (u == 4) ARKS_GN(4);
   else ARKS_GN(8);
 #undef ARKS_GN
 }
@@ -812,10 +812,16 @@ extern "C" void arks_seq_gelu_tanh_sums(void* out, const void* x, int64_t ldx,
                                         int n, hipStream_t stream) {
   const int64_t total = rows * n;
   if (total == 0) return;
-  hipLaunchKernelGGL(gelu_tanh_vec8_kernel,
-                     dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0,
-                     stream, (bf16*)out, SumRows{x, ldx, part, splits}, rows,
-                     n / 8);
+#define ARKS_GELU(U)                                                           \
+  hipLaunchKernelGGL((gelu_tanh_vec8_kernel<U>),                               \
+                     dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0,  \
+                     stream, (bf16*)out, SumRows{x, ldx, part, splits}, rows,  \
+                     n / 8)
+  const int u = parts_flight(splits);
+  if (u == 2) ARKS_GELU(2);
+  else if (u == 4) ARKS_GELU(4);
+  else ARKS_GELU(8);
+#undef ARKS_GELU
 }
 
 extern "C" void arks_seq_rms_norm_f32(void* out, const void* x, const void* w,
@@ -848,7 +854,7 @@ extern "C" void arks_seq_gelu_tanh(void* out, const void* x, int64_t ldx,
   const int64_t total = rows * n;
   if (total == 0) return;
   if (!act_f32 && n % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0) {
-    hipLaunchKernelGGL(gelu_tanh_vec8_kernel,
+    hipLaunchKernelGGL((gelu_tanh_vec8_kernel<2>),
                        dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0,
                        stream, (bf16*)out, SumRows{x, ldx, 0, 0}, rows, n / 8);
     return;

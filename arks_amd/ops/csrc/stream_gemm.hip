@@ -275,13 +275,14 @@ __global__ __launch_bounds__(512) void stream_split_kernel(
 }
 
 // out = the sum of the splits (+ bias), 4 columns a thread.
+template <int U>
 __global__ __launch_bounds__(256) void stream_sum_kernel(
     bf16* __restrict__ out, const float* __restrict__ part,
     const bf16* __restrict__ bias, const int64_t total, const int n_total,
     const int splits) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= total) return;
-  f32x4 s = sum_parts4(part + i, total, splits);
+  f32x4 s = sum_parts4<U>(part + i, total, splits);
   ushort4v o;
 #pragma unroll
   for (int r = 0; r < 4; ++r)
@@ -376,7 +377,13 @@ extern "C" void arks_stream_sum(void* out, const void* part, const void* bias,
                                 int64_t m, int n, int splits,
                                 hipStream_t stream) {
   const int64_t total = m * n;
-  hipLaunchKernelGGL(stream_sum_kernel, dim3((total / 4 + 255) / 256),
-                     dim3(256), 0, stream, (bf16*)out, (const float*)part,
-                     (const bf16*)bias, total, n, splits);
+#define ARKS_SUM(U)                                                            \
+  hipLaunchKernelGGL((stream_sum_kernel<U>), dim3((total / 4 + 255) / 256),    \
+                     dim3(256), 0, stream, (bf16*)out, (const float*)part,     \
+                     (const bf16*)bias, total, n, splits)
+  const int u = parts_flight(splits);
+  if (u == 2) ARKS_SUM(2);
+  else if (u == 4) ARKS_SUM(4);
+  else ARKS_SUM(8);
+#undef ARKS_SUM
 }
