@@ -272,9 +272,15 @@ class MoEMLP(nn.Module):
         """parts: the caller takes ops.Mixed too (one rank, no shared expert)."""
         from ..parallel.comm import tp_all_reduce
 
+        mixed = parts and self.shared is None and get_tp_world_size() == 1
+        if mixed:
+            out = ops.moe_routed_parts(x, self.gate, self.top_k, self.norm_topk,
+                                       self.w_up, self.w_down, self.expert_base)
+            if out is not None:
+                return out
         weights, selected = ops.moe_route(x, self.gate, self.top_k,
                                           self.norm_topk)
-        if parts and self.shared is None and get_tp_world_size() == 1:
+        if mixed:
             return ops.moe_experts_parts(
                 x, self.w_up, self.w_down, weights, selected, self.expert_base,
                 self.num_experts)

@@ -1343,14 +1343,22 @@ def moe_route(x, gate, k: int, renorm: bool):
     """moe_topk of the router product x gate^T, its logits fp32 at any number
     of rows: rounded ones tie, and the choice of a row must not turn with the
     step that it runs in."""
-    if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= MOE_ROUTE_ROWS
-            and x.shape[1] % 32 == 0 and gate.is_contiguous()
-            and gate.data_ptr() % 16 == 0):
-        logits = torch.empty((x.shape[0], gate.shape[0]), dtype=torch.float32,
-                             device=x.device)
-        _native().stream_gemm(logits, _rows_16b(x), gate, None, 1, 1, 16, False)
-        return moe_topk(logits, k, renorm)
+    if _route_streams(x, gate):
+        return moe_topk(_route_logits(x, gate), k, renorm)
     return moe_topk(linear_f32_lib(x, gate), k, renorm)
+
+
+def _route_streams(x, gate) -> bool:
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= MOE_ROUTE_ROWS
+            and x.shape[1] % 32 == 0 and gate.is_contiguous()
+            and gate.data_ptr() % 16 == 0)
+
+
+def _route_logits(x, gate):
+    logits = torch.empty((x.shape[0], gate.shape[0]), dtype=torch.float32,
+                         device=x.device)
+    _native().stream_gemm(logits, _rows_16b(x), gate, None, 1, 1, 16, False)
+    return logits
 
 
 def moe_tile(rows: int, top_k: int, experts: int, whole: bool = False) -> int:
@@ -1466,7 +1474,33 @@ def moe_experts_parts(x, w13, w2, weights, ids, expert_base: int = 0,
         return moe_experts(x, w13, w2, weights, ids, expert_base, experts)
     x, way = _moe_cut(x, w13, w2, ids, experts)
     return Mixed(*_native().moe_expert_rows(
-        x, w13, w2, weights, ids, expert_base, *(*way, 4, 4)[:4]))
+        x, w13, w2, weights, ids, expert_base, *(*way, 4, 4)[:4], None, False))
+
+
+# Rows whose choice of experts the plan makes (moe_gemm.hip), a wave a row: beyond,
+# its one workgroup takes longer than the launch that it saves. us with small experts,
+# so (apart): 128 experts, 8 per row, 1 row 14.3 (15.4), 8 rows 16.8 (17.8), 16 rows
+# 24.6 (24.0), 32 rows 29.6 (24.8); 64, 6 per row, 8 rows 15.6 (16.6), 16 rows 20.7
+# (20.8); 8, 2 per row, 8 rows 12.5 (13.8), 24 rows 14.0 (14.3).
+_PLAN_ROWS = 8
+
+
+def moe_routed_parts(x, gate, k: int, renorm: bool, w13, w2, expert_base: int = 0):
+    """moe_experts_parts of what moe_route chooses among gate's experts, the choice
+    made by the kernel that plans the experts' rows, or None where that takes no such
+    rows: few, whose launches count."""
+    T, E = x.shape[0], gate.shape[0]
+    if not (1 <= T <= _PLAN_ROWS and E <= 128 and 1 <= k <= min(16, E) and T * k <= 512
+            and _route_streams(x, gate)):
+        return None
+    weights = torch.empty((T, k), dtype=torch.float32, device=x.device)
+    ids = torch.empty((T, k), dtype=torch.int32, device=x.device)
+    if not _moe_native(x, w13, w2, ids):
+        return None
+    x, way = _moe_cut(x, w13, w2, ids, E)
+    return Mixed(*_native().moe_expert_rows(
+        x, w13, w2, weights, ids, expert_base, *(*way, 4, 4)[:4],
+        _route_logits(x, gate), bool(renorm)))
 
 
 def _moe_native(x, w13, w2, ids) -> bool:

@@ -113,6 +113,10 @@ void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, void* claims, void* counts, const void* ids,
                    const void* weights, int pairs, int expert_base, int n_local,
                    int tile, int max_items, int groups, hipStream_t stream);
+void arks_moe_plan_topk(void* perm, void* rows, void* weights_out, void* items,
+                        void* n_items, void* claims, const void* logits,
+                        int experts, int k, int renorm, int pairs, int expert_base,
+                        int n_local, int tile, int max_items, hipStream_t stream);
 void arks_moe_gemm(void* out, const void* a, const void* w, const void* perm,
                    const void* items, const void* n_items, void* claims, const void* scale,
                    int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out, int k_total,
@@ -875,11 +879,13 @@ void stage_rows(pybind11::list prompts, pybind11::list outputs,
 // [T, k]); w13 [El, 2I, H], w2 [El, H, I], pairs beyond this rank's El experts
 // from expert_base on weigh zero. tile: pairs of a work item; mid: of 32, 64 or
 // 128 pairs in mid_gemm.hip (32: qt_up and qt_down, weight rows a wave / 16, may
-// be 2), else in moe_gemm.hip (16, 128 or, 256, its engine's up to 320).
+// be 2), else in moe_gemm.hip (16, 128 or, 256, its engine's up to 320). logits
+// [T, experts]: the plan finds ids and weights (only their sizes count then).
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
     torch::Tensor x, torch::Tensor w13, torch::Tensor w2, torch::Tensor weights,
     torch::Tensor ids, int64_t expert_base, int64_t tile, bool mid,
-    int64_t qt_up, int64_t qt_down) {
+    int64_t qt_up, int64_t qt_down,
+    c10::optional<torch::Tensor> logits = c10::nullopt, bool renorm = false) {
   check_bf16_rowstrided(x, "x");
   check_bf16_contig(w13, "w13");
   check_bf16_contig(w2, "w2");
@@ -910,6 +916,13 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
               weights.is_contiguous() && ids.scalar_type() == torch::kInt32 &&
               ids.is_contiguous() && ids.size(0) == T && ids.size(1) == k &&
               weights.size(0) == T);
+  if (logits.has_value())
+    TORCH_CHECK(logits->is_cuda() && logits->is_contiguous() &&
+                    logits->scalar_type() == torch::kFloat32 &&
+                    logits->dim() == 2 && logits->size(0) == T &&
+                    logits->size(1) <= 128 && logits->size(1) >= k && k >= 1 &&
+                    P <= 512,
+                "the plan takes fp32 logits of 128 experts, 512 pairs");
   if (T == 0) return {torch::empty({0, H}, x.options()), weights, ids};
   const int64_t max_items = std::min(P, El) + P / (tile == 256 ? 320 : tile);
   TORCH_CHECK(max_items <= 65535 || tile != 16, "too many rows for this tile");
@@ -930,10 +943,17 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
   torch::Tensor y = torch::empty({P, H}, x.options());
   auto stream = current_stream();
   int* claims = n_items + 1;
-  arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
-                claims + 16, ids.data_ptr(), weights.data_ptr(), (int)P,
-                (int)expert_base, (int)El, tile == 256 ? 320 : (int)tile,
-                (int)max_items, (int)groups, stream);
+  const int places = tile == 256 ? 320 : (int)tile;
+  if (logits.has_value())
+    arks_moe_plan_topk(perm, rows, w_pair.data_ptr(), items, n_items, claims,
+                       logits->data_ptr(), (int)logits->size(1), (int)k, renorm,
+                       (int)P, (int)expert_base, (int)El, places, (int)max_items,
+                       stream);
+  else
+    arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
+                  claims + 16, ids.data_ptr(), weights.data_ptr(), (int)P,
+                  (int)expert_base, (int)El, places, (int)max_items, (int)groups,
+                  stream);
   if (mid) {
     const int ft = (int)tile / 32;
     arks_mid_items(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,

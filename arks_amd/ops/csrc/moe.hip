@@ -11,17 +11,12 @@
 // The reference delegates MoE serving to external images; these kernels are
 // internals of its runtime slot.
 #include "common.h"
+#include "moe_topk.h"
 #include "parts.h"
-
-#include <cfloat>
 
 namespace arks {
 
-// One wave per token row: softmax over E (<= 64 * S) then k argmax passes over
-// the logits (same order as over probs), ties to the lower expert. The row
-// stays in registers and a pass moves one value over the lanes (their index
-// comes from a ballot); with the row read again for each pass and value and
-// index both moved it took 11 us for 64 rows of 128, k 8.
+// One wave per token row.
 template <int S>
 __global__ __launch_bounds__(64) void moe_topk_kernel(
     float* __restrict__ weights,    // [T, k]
@@ -30,53 +25,12 @@ __global__ __launch_bounds__(64) void moe_topk_kernel(
     const int E, const int k, const int renorm) {
   const int t = blockIdx.x;
   const int lane = threadIdx.x;
-  const float* row = logits + (int64_t)t * E;
-  float v[S];
-  uint32_t open = 0;  // this lane's entries e = 64 * i + lane not yet chosen
-#pragma unroll
-  for (int i = 0; i < S; ++i) {
-    const int e = 64 * i + lane;
-    v[i] = e < E ? row[e] : -INFINITY;
-    if (e < E) open |= 1u << i;
-  }
-  float m = -FLT_MAX;
-#pragma unroll
-  for (int i = 0; i < S; ++i) m = fmaxf(m, v[i]);
-  m = wave_reduce_max(m);
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < S; ++i) s += __expf(v[i] - m);
-  s = wave_reduce_sum(s);
-
-  float mine = 0.f, wsum = 0.f;  // lane j keeps choice j
-  int mine_id = 0;
-  for (int j = 0; j < k; ++j) {
-    float best = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < S; ++i)
-      if (open >> i & 1) best = fmaxf(best, v[i]);
-    best = wave_reduce_max(best);
-    int id = -1, first = -1;  // first: of rows of NaN
-#pragma unroll
-    for (int i = S - 1; i >= 0; --i) {
-      const bool is_open = open >> i & 1;
-      const uint64_t any = __ballot(is_open);
-      const uint64_t hit = __ballot(is_open && v[i] == best);
-      if (any) first = 64 * i + __ffsll((unsigned long long)any) - 1;
-      if (hit) id = 64 * i + __ffsll((unsigned long long)hit) - 1;
-    }
-    if (id < 0) id = first;
-    if (id % 64 == lane) open &= ~(1u << (id / 64));
-    const float w = __expf(best - m) / s;
-    if (lane == j) {
-      mine = w;
-      mine_id = id;
-    }
-    wsum += w;
-  }
+  float weight;
+  int id;
+  moe_topk_row<S>(logits + (int64_t)t * E, E, k, renorm, lane, weight, id);
   if (lane < k) {
-    weights[(int64_t)t * k + lane] = mine * (renorm ? 1.f / wsum : 1.f);
-    ids[(int64_t)t * k + lane] = mine_id;
+    weights[(int64_t)t * k + lane] = weight;
+    ids[(int64_t)t * k + lane] = id;
   }
 }
 

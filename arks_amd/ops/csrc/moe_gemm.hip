@@ -28,6 +28,7 @@
 // want them. Items past the last one are empty, so grids depend on the shapes
 // alone and a decode step can be captured.
 #include <type_traits>
+#include "moe_topk.h"
 #include "seq_common.h"
 #include "wide_engine.h"
 
@@ -59,14 +60,44 @@ __device__ __forceinline__ f32x4 moe_mfma(const ushort8& a, const ushort8& b,
 // STAGE 2 places it behind the runs before it. STAGE 0: one workgroup does
 // both. 40096 pairs of 128 experts 46.9 -> 10.6 us, 131072 of 512 experts 166
 // -> 16; the runs' length hardly matters (512 to 4096 pairs: 11.8 to 10.6).
-template <int STAGE>
+// TOPK (STAGE 0, of up to MOE_TOPK_PAIRS pairs): ids and weights are found here, from
+// the rows' logits [rows, experts <= 64 * TOPK], a wave a row: a launch less, while
+// rows are few (ops._PLAN_ROWS).
+struct MoeLogits {
+  const float* __restrict__ logits;
+  int experts, k, renorm;
+};
+constexpr int MOE_TOPK_PAIRS = 512;
+template <int STAGE, int TOPK = 0>
 __global__ __launch_bounds__(1024) void moe_plan_kernel(
     int* __restrict__ perm, int* __restrict__ rows,
     float* __restrict__ weights_out, int4* __restrict__ items,
     int* __restrict__ n_items, int* __restrict__ claims,
     int* __restrict__ counts, const int* __restrict__ ids,
     const float* __restrict__ weights, const int pairs, const int expert_base,
-    const int n_local, const int tile, const int max_items) {
+    const int n_local, const int tile, const int max_items,
+    const MoeLogits route) {
+  __shared__ int chosen[TOPK ? MOE_TOPK_PAIRS : 1];
+  __shared__ float chosen_w[TOPK ? MOE_TOPK_PAIRS : 1];
+  auto id_of = [&](const int p) { return TOPK ? chosen[TOPK ? p : 0] : ids[p]; };
+  auto weight_of = [&](const int p) {
+    return TOPK ? chosen_w[TOPK ? p : 0] : weights[p];
+  };
+  if constexpr (TOPK > 0) {
+    const int lane = threadIdx.x % WAVE_SIZE;
+    for (int t = threadIdx.x / WAVE_SIZE; t < pairs / route.k;
+         t += 1024 / WAVE_SIZE) {
+      float w;
+      int id;
+      moe_topk_row<TOPK>(route.logits + (int64_t)t * route.experts, route.experts,
+                         route.k, route.renorm, lane, w, id);
+      if (lane < route.k) {
+        chosen[t * route.k + lane] = id;
+        chosen_w[t * route.k + lane] = w;
+      }
+    }
+    // (the barrier behind the counters' clearing stands in front of their use)
+  }
   __shared__ int count[MOE_MAX_E], start[MOE_MAX_E], first_item[MOE_MAX_E];
   __shared__ int total_items;
   const int tid = threadIdx.x;
@@ -82,7 +113,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
       int e[PB];
 #pragma unroll
       for (int j = 0; j < PB; ++j)
-        e[j] = p0 + j * 1024 < end ? ids[p0 + j * 1024] - expert_base : -1;
+        e[j] = p0 + j * 1024 < end ? id_of(p0 + j * 1024) - expert_base : -1;
 #pragma unroll
       for (int j = 0; j < PB; ++j)
         if (e[j] >= 0 && e[j] < n_local) atomicAdd(&count[e[j]], 1);
@@ -165,8 +196,8 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
 #pragma unroll
     for (int j = 0; j < PB; ++j) {
       const int p = min(p0 + j * 1024, end - 1);
-      e[j] = ids[p] - expert_base;
-      w[j] = weights[p];
+      e[j] = id_of(p) - expert_base;
+      w[j] = weight_of(p);
     }
 #pragma unroll
     for (int j = 0; j < PB; ++j) {
@@ -613,7 +644,7 @@ extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
                      stream, (int*)perm, (int*)rows, (float*)weights_out,     \
                      (int4*)items, (int*)n_items, (int*)claims, (int*)counts, \
                      (const int*)ids, (const float*)weights, pairs,           \
-                     expert_base, n_local, tile, max_items)
+                     expert_base, n_local, tile, max_items, MoeLogits{})
   if (groups == 1) {
     ARKS_PLAN(0);
   } else {
@@ -621,6 +652,21 @@ extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
     ARKS_PLAN(2);
   }
 #undef ARKS_PLAN
+}
+
+// arks_moe_plan of one group whose ids and weights come from logits [pairs / k,
+// experts]: at most 512 pairs, 128 experts in all, k <= 64.
+extern "C" void arks_moe_plan_topk(void* perm, void* rows, void* weights_out,
+                                   void* items, void* n_items, void* claims,
+                                   const void* logits, int experts, int k,
+                                   int renorm, int pairs, int expert_base,
+                                   int n_local, int tile, int max_items,
+                                   hipStream_t stream) {
+  hipLaunchKernelGGL((moe_plan_kernel<0, 2>), dim3(1), dim3(1024), 0, stream,
+                     (int*)perm, (int*)rows, (float*)weights_out, (int4*)items,
+                     (int*)n_items, (int*)claims, nullptr, nullptr, nullptr, pairs,
+                     expert_base, n_local, tile, max_items,
+                     MoeLogits{(const float*)logits, experts, k, renorm});
 }
 
 // tile: pairs of an item, 16 (streamed; n_out % 32 == k_total % 32 == 0) or 128

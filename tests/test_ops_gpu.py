@@ -1659,6 +1659,33 @@ def test_mid_gemm(M, N, K, qt, splits, kind):
             <= 2 * slack + 2 ** -8 * expect.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("T", [1, 3, 8])
+@pytest.mark.parametrize("E,k,base,El", [
+    (128, 8, 0, 128), (100, 16, 0, 100), (64, 6, 16, 32), (1, 1, 0, 1), (65, 2, 0, 65),
+])
+def test_moe_routed_parts(T, E, k, base, El):
+    """Experts chosen by the kernel that plans their rows: the same rows, weights and
+    mix as from moe_route, ties and rows of NaN among them."""
+    assert_native()
+    torch.manual_seed(E + T)
+    H, I = 256, 64
+    x = torch.randn(T, H, dtype=torch.bfloat16, device=DEV)
+    gate = torch.randn(E, H, dtype=torch.bfloat16, device=DEV)
+    gate[E // 2:] = gate[:E - E // 2].clone()  # ties
+    if T == 3:
+        x[1] = float("nan")
+    w13 = (torch.randn(El, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(El, H, I, device=DEV) * I ** -0.5).bfloat16()
+    for renorm in (False, True):
+        weights, ids = ops.moe_route(x, gate, k, renorm)
+        want = ops.moe_experts_parts(x, w13, w2, weights, ids, base, E)
+        got = ops.moe_routed_parts(x, gate, k, renorm, w13, w2, base)
+        assert torch.equal(got.weights.nan_to_num(7.0), want.weights.nan_to_num(7.0))
+        a, b = (ops.parts_sum(m) for m in (got, want))
+        assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+    assert ops.moe_routed_parts(x.repeat(9, 1), gate, k, True, w13, w2, base) is None
+
+
 @pytest.mark.parametrize("M,N,K", [(93, 512, 4096), (300, 1024, 8192)])
 def test_plain_prompts(M, N, K):
     """Prompts' products of weights beside fp8 pages reach their norm as the rounded
