@@ -30,7 +30,10 @@ Kernel plan per block (bf16 serving; fp32 runs the same kernels on float
 rows): token_shift -> GEMM(mixer in) .. mixer kernels .. GEMM(mixer out),
 GEMM(gate) -> gated_norm_residual [-> GEMM(up|gate) -> gelu_tanh ->
 GEMM(down) -> gated_norm_residual]. The feed-forward's up projection and
-its residual gate read the same row, so they are one fused GEMM.
+its residual gate read the same row, so they are one fused GEMM. Few rows:
+GEMM(mixer out) and GEMM(gate) are one launch, the kernels behind products
+add their split sums, and steps of one row a sequence have the next block's
+token shift from the last norm.
 
 Legalix's is:
   - ONE norm per layer, a tanh norm without statistics,
