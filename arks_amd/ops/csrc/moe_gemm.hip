@@ -471,8 +471,13 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
 // waited for. Its place in LDS belongs to the tiles' array: a second one made the
 // compiler drain the loads before every read of the first.
 // GLU: gate and up are rounded to bf16 before they meet, as rows of a product in
-// memory would be, and scale [pairs] (or null) is a factor of both; it is loaded
-// in front of the next tile's first loads, so as not to be waited for behind them.
+// memory would be. SCALED: scale [pairs] is a factor of both; it is loaded in front
+// of the next tile's first loads, so as not to be waited for behind them, and named
+// again behind them: only rows that a tile has use it, so that the compiler took the
+// others' loads to be still under way, and drained all loads in every step of the
+// loop for 193 to 256 pairs, whose fragments lie in these registers. us with plan,
+// before (which asked at run time whether there is a scale) -> so: 16 experts of 4096
+// x 3584, 4 per row, no scale, 2000 rows 719 -> 703, 3000 rows 1039 -> 961.
 template <bool ONCE>
 using MoeTileOf = WideTile<4, 4, 5, false, ONCE ? 2 : 0>;
 
@@ -488,7 +493,7 @@ __device__ __forceinline__ void moe_frags(const int pairs, F f) {
   }
 }
 
-template <bool UP, bool GLU, bool ONCE>
+template <bool UP, bool GLU, bool SCALED, bool ONCE>
 __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ a,
     const bf16* __restrict__ w, const int* __restrict__ perm,
@@ -565,13 +570,14 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     const Job next = more ? job(i) : now;
     if (more) p = places(next);
     moe_frags(now.pairs, [&](auto f) { tile.template run<f>(t, now.k); });
-    float by[GLU ? FY : 1];
-    if constexpr (GLU) {
+    float by[SCALED ? FY : 1];
+    if constexpr (SCALED) {
+      int at[FY];
 #pragma unroll
       for (int y = 0; y < FY; ++y)
-        by[y] = scale ? scale[perm[now.first + min(tile.frag_y(y) + lq,
-                                                   now.pairs - 1)]]
-                      : 1.f;
+        at[y] = perm[now.first + min(tile.frag_y(y) + lq, now.pairs - 1)];
+#pragma unroll
+      for (int y = 0; y < FY; ++y) by[y] = scale[at[y]];
     }
     int c;
     if (more) {
@@ -595,14 +601,20 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
             if constexpr (UP) {
               const float g = tile.acc[4 * h + e / 2][y][e % 2 * 2];
               const float u = tile.acc[4 * h + e / 2][y][e % 2 * 2 + 1];
-              v[e] = GLU ? silu_f(by[y] * moe_bf16(g)) * (by[y] * moe_bf16(u))
-                         : tile_silu_mul(g, u);
+              if constexpr (SCALED)
+                v[e] = silu_f(by[y] * moe_bf16(g)) * (by[y] * moe_bf16(u));
+              else
+                v[e] = GLU ? silu_f(moe_bf16(g)) * moe_bf16(u) : tile_silu_mul(g, u);
             } else {
               v[e] = tile.acc[4 * h + 2 * q + e / 4][y][e % 4];
             }
           }
           o[y][h * P + q] = tile_round(v);
         }
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int y = 0; y < FY; ++y) asm volatile("" : "+v"(by[y]));
+    }
     if (more) {
       if (threadIdx.x == 0) claimed = slots + c;
       moe_frags(next.pairs, [&](auto f) { tile.template prologue_wait<f>(steps); });
@@ -701,21 +713,22 @@ extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
     const int row_tiles = (n_out + (up ? 127 : 255)) / (up ? 128 : 256);
     const int64_t jobs = (int64_t)max_items * row_tiles;
     const dim3 grid(jobs < 256 ? (jobs + 7) / 8 * 8 : 256), block(512);
-#define ARKS_ENGINE_O(UP, GLU, ONCE)                                          \
-  hipLaunchKernelGGL((moe_engine_kernel<UP, GLU, ONCE>), grid, block, 0, stream, \
-                     (bf16*)out, (const bf16*)a, (const bf16*)w,              \
+#define ARKS_ENGINE_O(UP, GLU, SCALED, ONCE)                                  \
+  hipLaunchKernelGGL((moe_engine_kernel<UP, GLU, SCALED, ONCE>), grid, block, 0, \
+                     stream, (bf16*)out, (const bf16*)a, (const bf16*)w,      \
                      (const int*)perm, (const int4*)items,                    \
                      (const int*)n_items, (int*)claims + (up ? 0 : 8),        \
                      (const float*)scale, a_stride, w_expert, w_stride, n_out, \
                      k_total, top_k, row_tiles, (int)(once == 2))
-#define ARKS_ENGINE(UP, GLU)                                                  \
+#define ARKS_ENGINE(UP, GLU, SCALED)                                          \
   do {                                                                        \
-    if (once) ARKS_ENGINE_O(UP, GLU, true);                                   \
-    else ARKS_ENGINE_O(UP, GLU, false);                                       \
+    if (once) ARKS_ENGINE_O(UP, GLU, SCALED, true);                           \
+    else ARKS_ENGINE_O(UP, GLU, SCALED, false);                               \
   } while (0)
-    if (up && glu) ARKS_ENGINE(true, true);
-    else if (up) ARKS_ENGINE(true, false);
-    else ARKS_ENGINE(false, false);
+    if (up && glu && scale) ARKS_ENGINE(true, true, true);
+    else if (up && glu) ARKS_ENGINE(true, true, false);
+    else if (up) ARKS_ENGINE(true, false, false);
+    else ARKS_ENGINE(false, false, false);
 #undef ARKS_ENGINE
 #undef ARKS_ENGINE_O
   } else {
