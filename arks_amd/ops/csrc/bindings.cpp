@@ -5,6 +5,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -112,11 +113,13 @@ void arks_mid_items(void* out, const void* a, const void* w, const void* perm,
 void arks_moe_plan(void* perm, void* rows, void* weights_out, void* items,
                    void* n_items, void* claims, void* counts, const void* ids,
                    const void* weights, int pairs, int expert_base, int n_local,
-                   int tile, int max_items, int groups, hipStream_t stream);
+                   int tile, int max_items, int groups, const int* rounds,
+                   hipStream_t stream);
 void arks_moe_plan_topk(void* perm, void* rows, void* weights_out, void* items,
                         void* n_items, void* claims, const void* logits,
                         int experts, int k, int renorm, int pairs, int expert_base,
-                        int n_local, int tile, int max_items, hipStream_t stream);
+                        int n_local, int tile, int max_items, const int* rounds,
+                        hipStream_t stream);
 void arks_moe_gemm(void* out, const void* a, const void* w, const void* perm,
                    const void* items, const void* n_items, void* claims, const void* scale,
                    int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out, int k_total,
@@ -875,6 +878,13 @@ void stage_rows(pybind11::list prompts, pybind11::list outputs,
   }
 }
 
+// Tiles of weight rows and steps of 64 columns of an expert's products in
+// moe_gemm.hip's engine: gate and up of 2I x H, then H x I.
+static std::array<int, 4> engine_rounds(int64_t H, int64_t I) {
+  return {(int)((I + 127) / 128), (int)((H + 255) / 256), (int)(H / 64),
+          (int)(I / 64)};
+}
+
 // The experts' rows of x [T, H] and their mix: (y [T * k, H], weights and rows
 // [T, k]); w13 [El, 2I, H], w2 [El, H, I], pairs beyond this rank's El experts
 // from expert_base on weigh zero. tile: pairs of a work item; mid: of 32, 64 or
@@ -924,7 +934,7 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
                     P <= 512,
                 "the plan takes fp32 logits of 128 experts, 512 pairs");
   if (T == 0) return {torch::empty({0, H}, x.options()), weights, ids};
-  const int64_t max_items = std::min(P, El) + P / (tile == 256 ? 320 : tile);
+  const int64_t max_items = std::min(P, El) + P / (tile == 256 ? 192 : tile);
   TORCH_CHECK(max_items <= 65535 || tile != 16, "too many rows for this tile");
   auto ints = x.options().dtype(torch::kInt32);
   // one workgroup plans 8192 pairs in 9 us and 16384 in 20; two launches of a
@@ -944,16 +954,17 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
   auto stream = current_stream();
   int* claims = n_items + 1;
   const int places = tile == 256 ? 320 : (int)tile;
+  const auto rounds = engine_rounds(H, I);
   if (logits.has_value())
     arks_moe_plan_topk(perm, rows, w_pair.data_ptr(), items, n_items, claims,
                        logits->data_ptr(), (int)logits->size(1), (int)k, renorm,
                        (int)P, (int)expert_base, (int)El, places, (int)max_items,
-                       stream);
+                       rounds.data(), stream);
   else
     arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
                   claims + 16, ids.data_ptr(), weights.data_ptr(), (int)P,
                   (int)expert_base, (int)El, places, (int)max_items, (int)groups,
-                  stream);
+                  rounds.data(), stream);
   if (mid) {
     const int ft = (int)tile / 32;
     arks_mid_items(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
@@ -1009,7 +1020,7 @@ std::tuple<torch::Tensor, torch::Tensor> moe_wide_rows(
               weights.size(0) == T);
   torch::Tensor y = torch::empty({P, W}, x.options());
   if (T == 0) return {y, ids};
-  const int64_t max_items = std::min(P, experts) + P / 320;
+  const int64_t max_items = std::min(P, experts) + P / 192;
   const int64_t groups = P <= 8192 ? 1 : std::min<int64_t>(64, (P + 2047) / 2048);
   // as in moe_expert_rows
   torch::Tensor plan = torch::empty(
@@ -1025,7 +1036,8 @@ std::tuple<torch::Tensor, torch::Tensor> moe_wide_rows(
   auto stream = current_stream();
   arks_moe_plan(perm, rows, w_pair.data_ptr(), items, n_items, claims,
                 claims + 16, ids.data_ptr(), weights.data_ptr(), (int)P, 0,
-                (int)experts, 320, (int)max_items, (int)groups, stream);
+                (int)experts, 320, (int)max_items, (int)groups,
+                engine_rounds(W, ff).data(), stream);
   // not rotated: an expert's row adds up in the same order at any number of rows
   const int once = P <= 160 * experts ? 1 : 0;
   arks_moe_gemm(h.data_ptr(), x.data_ptr(), w_gu.data_ptr(), perm, items,

@@ -68,6 +68,51 @@ struct MoeLogits {
   int experts, k, renorm;
 };
 constexpr int MOE_TOPK_PAIRS = 512;
+// Tiles of weight rows and steps of 64 columns of the experts' two products (the
+// engine's; moe_cut).
+struct MoeRounds {
+  int up_tiles, down_tiles, up_steps, down_steps;
+};
+// How many pairs the items of moe_engine may have, 320, 256 or 192, for the counts
+// that the plan finds (a wave's work): items are work for 256 CUs in rounds, and a tile
+// takes as long as on the mean (moe_engine: 0.5 and 0.21 for each 64 pairs). us, 320
+// (256; 192), 16 experts of 4096 x 2048, 2 per row: 2000 rows 247 (325; 268), 2250 rows
+// 331 (301; 354), 2500 rows 327 (314; 293); 16 of 4096 x 3584, 4 per row: 1000 rows 398
+// (493; 464), 1300 rows 583 (533; 565); 32 of 2048 x 1024, 4 per row, 1700 rows 198
+// (176; 166). Over 77 sizes the choice takes 1.004 of the best, always 320 1.026. It
+// is 0.7 us of the plan. Against tiles of 256 pairs and of 128 for what is left, in
+// tile_engine.h's loop, 79 sizes take 0.956, in the worst 8 experts of 4096 x 14336, 2
+// per row, 3000 rows 1801 (1684) and 16 of 4096 x 2048, 5000 rows 513 (469).
+__device__ __forceinline__ int moe_cut(const MoeRounds& r, const int* count,
+                                       const int n_local, const int pairs) {
+  int sum[4] = {};
+  for (int e = threadIdx.x; e < n_local; e += WAVE_SIZE) {
+    const int c = count[e];
+    sum[0] += (c + 319) / 320;
+    sum[1] += (c + 255) / 256;
+    sum[2] += (c + 191) / 192;
+    sum[3] += (c + 63) / 64;
+  }
+#pragma unroll
+  for (int off = 1; off < WAVE_SIZE; off <<= 1)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sum[j] += __shfl_xor(sum[j], off, WAVE_SIZE);
+  float best = INFINITY;
+  int cap = 320;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const float n = fmaxf((float)sum[j], 1.f);
+    const float time = (r.up_steps * ceilf(n * r.up_tiles / 256.f) +
+                        r.down_steps * ceilf(n * r.down_tiles / 256.f)) *
+                       (0.5f + 0.21f * sum[3] / n);
+    // (an item's number within its expert has 15 bits)
+    if (time < best && (j < 2 || pairs < 1 << 22)) {
+      best = time;
+      cap = 320 - 64 * j;
+    }
+  }
+  return cap;
+}
 template <int STAGE, int TOPK = 0>
 __global__ __launch_bounds__(1024) void moe_plan_kernel(
     int* __restrict__ perm, int* __restrict__ rows,
@@ -76,7 +121,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
     int* __restrict__ counts, const int* __restrict__ ids,
     const float* __restrict__ weights, const int pairs, const int expert_base,
     const int n_local, const int tile, const int max_items,
-    const MoeLogits route) {
+    const MoeLogits route, const MoeRounds rounds) {
   __shared__ int chosen[TOPK ? MOE_TOPK_PAIRS : 1];
   __shared__ float chosen_w[TOPK ? MOE_TOPK_PAIRS : 1];
   auto id_of = [&](const int p) { return TOPK ? chosen[TOPK ? p : 0] : ids[p]; };
@@ -99,7 +144,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
     // (the barrier behind the counters' clearing stands in front of their use)
   }
   __shared__ int count[MOE_MAX_E], start[MOE_MAX_E], first_item[MOE_MAX_E];
-  __shared__ int total_items;
+  __shared__ int total_items, item_cap;
   const int tid = threadIdx.x;
   const int group = STAGE == 0 ? 0 : (int)blockIdx.x;
   const int groups = STAGE == 0 ? 1 : (int)gridDim.x;
@@ -145,11 +190,13 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
     __syncthreads();
   }
   if (tid < WAVE_SIZE) {  // prefix sums, 64 experts at a time
-    int at = 0, item = 0;
+    int at = 0, item = 0, cap = tile;
+    if (tile > 256) cap = moe_cut(rounds, count, n_local, pairs);
+    if (tid == 0) item_cap = cap;
     for (int e0 = 0; e0 < n_local; e0 += WAVE_SIZE) {
       const int e = e0 + tid;
       const int c = e < n_local ? count[e] : 0;
-      const int n = (c + tile - 1) / tile;
+      const int n = (c + cap - 1) / cap;
       int sc = c, sn = n;
 #pragma unroll
       for (int off = 1; off < WAVE_SIZE; off <<= 1) {
@@ -173,9 +220,10 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(
   if (group == 0) {
     if (tid < 16) claims[tid] = 0;
     if (tid == 0) *n_items = total_items;
+    const int cap = item_cap;
     for (int e = tid; e < n_local; e += 1024) {
       const int c = count[e];
-      const int n = (c + tile - 1) / tile;
+      const int n = (c + cap - 1) / cap;
       // (8 experts of 4096 x 14336, 2 per row, 2048 rows 1529 us with items of 320
       // and what is left, even 1448)
       const int per = tile > 256 && n ? ((c + n - 1) / n + 63) / 64 * 64 : tile;
@@ -643,20 +691,22 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
 using namespace arks;
 
 // groups: workgroups that the pairs are spread over; more than one need
-// counts [groups, n_local]. tile above 256 (moe_engine's): an expert's items are
-// even, in whole 64 pairs.
+// counts [groups, n_local]. tile above 256 (moe_engine's): items of the
+// size that moe_cut finds for products of these MoeRounds, an expert's even, in whole
+// 64 pairs; max_items holds those of up to 192.
 extern "C" void arks_moe_plan(void* perm, void* rows, void* weights_out,
                               void* items, void* n_items, void* claims,
                               void* counts, const void* ids,
                               const void* weights, int pairs, int expert_base,
                               int n_local, int tile, int max_items, int groups,
-                              hipStream_t stream) {
+                              const int* rounds, hipStream_t stream) {
+  const MoeRounds rounds_of{rounds[0], rounds[1], rounds[2], rounds[3]};
 #define ARKS_PLAN(STAGE)                                                      \
   hipLaunchKernelGGL((moe_plan_kernel<STAGE>), dim3(groups), dim3(1024), 0,   \
                      stream, (int*)perm, (int*)rows, (float*)weights_out,     \
                      (int4*)items, (int*)n_items, (int*)claims, (int*)counts, \
                      (const int*)ids, (const float*)weights, pairs,           \
-                     expert_base, n_local, tile, max_items, MoeLogits{})
+                     expert_base, n_local, tile, max_items, MoeLogits{}, rounds_of)
   if (groups == 1) {
     ARKS_PLAN(0);
   } else {
@@ -673,12 +723,13 @@ extern "C" void arks_moe_plan_topk(void* perm, void* rows, void* weights_out,
                                    const void* logits, int experts, int k,
                                    int renorm, int pairs, int expert_base,
                                    int n_local, int tile, int max_items,
-                                   hipStream_t stream) {
+                                   const int* rounds, hipStream_t stream) {
   hipLaunchKernelGGL((moe_plan_kernel<0, 2>), dim3(1), dim3(1024), 0, stream,
                      (int*)perm, (int*)rows, (float*)weights_out, (int4*)items,
                      (int*)n_items, (int*)claims, nullptr, nullptr, nullptr, pairs,
                      expert_base, n_local, tile, max_items,
-                     MoeLogits{(const float*)logits, experts, k, renorm});
+                     MoeLogits{(const float*)logits, experts, k, renorm},
+                     MoeRounds{rounds[0], rounds[1], rounds[2], rounds[3]});
 }
 
 // tile: pairs of an item, 16 (streamed; n_out % 32 == k_total % 32 == 0) or 128

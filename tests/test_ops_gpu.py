@@ -914,6 +914,75 @@ def test_moe_engine_items(T, El):
     assert (err <= 3 * 2 ** -8 * expect.norm(dim=1)).all()
 
 
+@pytest.mark.parametrize("T,E,k,H,I,skew,cap", [
+    # one item an expert where two are a round more, and where they are not
+    (193, 16, 16, 2304, 1152, 0, 320), (256, 16, 16, 2304, 1152, 0, 320),
+    (257, 16, 16, 2304, 1152, 0, 320), (320, 16, 16, 2304, 1152, 0, 320),
+    (320, 4, 4, 512, 256, 0, 256), (900, 16, 8, 2304, 1152, 0, 192),
+    (641, 16, 16, 2304, 1152, 0, 320), (500, 16, 8, 2304, 1152, 0, 256),
+    (1200, 8, 2, 2304, 4096, 0, 256), (700, 8, 2, 2304, 4096, 1, 192),
+    # many pairs, in runs of their own; experts that none chooses
+    (2300, 24, 4, 512, 1152, 2, 192), (640, 8, 4, 2304, 2304, 1, 256),
+])
+@pytest.mark.parametrize("kind", ["plain", "rounded", "scaled"])
+def test_moe_engine_cut(T, E, k, H, I, skew, cap, kind):
+    """The items that the engine's plan cuts: all pairs once, evenly, of the size whose
+    rounds over the CUs take least, and the rows' products in them vs fp64."""
+    assert_native()
+    torch.manual_seed(T + E)
+    likes = torch.arange(E, 0, -1) * (0.1 * skew)
+    ids = (torch.rand(T, E) + likes).topk(k).indices.int().to(DEV)
+    x = torch.randn(T, H, device=DEV).bfloat16()
+    if kind == "plain":
+        w13 = (torch.randn(E, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+        w2 = (torch.randn(E, H, I, device=DEV) * I ** -0.5).bfloat16()
+    else:
+        w13 = (torch.randn(E * 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+        w2 = (torch.randn(H, E * I, device=DEV) * I ** -0.5).bfloat16()
+    w = torch.rand(T, k, device=DEV) + 0.5
+    if kind == "plain":
+        y, _, place = ops._native().moe_expert_rows(
+            x, w13, w2, w, ids, 0, 256, False, 4, 4, None, False)
+    else:
+        y, place = ops._native().moe_wide_rows(x, w13, w2, w, ids, E, I,
+                                               kind == "scaled")
+    # (the items stand in front of the rows in one buffer)
+    most = (place.storage_offset() - T * k) // 4
+    items = torch.as_strided(place, (most, 4), (4, 1), 0).cpu()
+    counts = ids.flatten().bincount(minlength=E).cpu()
+
+    def cut(size):
+        return [-(-c // size) for c in counts.tolist()]
+
+    def per(c, n):
+        return -(-(-(-c // n)) // 64) * 64
+
+    def cost(size):
+        n = sum(cut(size))
+        frags = sum(n and (n - 1) * per(c, n) // 64 + -(-(c - (n - 1) * per(c, n)) // 64)
+                    for c, n in zip(counts.tolist(), cut(size)))
+        return ((H // 64 * -(-n * -(-I // 128) // 256)
+                 + I // 64 * -(-n * -(-H // 256) // 256)) * (0.5 + 0.21 * frags / n))
+
+    assert min((320, 256, 192), key=cost) == cap
+    want, start = [], 0
+    for e, (c, n) in enumerate(zip(counts.tolist(), cut(cap))):
+        want += [[e, start + i * per(c, n), min(per(c, n), c - i * per(c, n)), i | n << 16]
+                 for i in range(n)]
+        start += c
+    assert items[:len(want)].tolist() == want and not items[len(want):, 2].any()
+    for e in range(E):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        s = w[t, j].double()[:, None] if kind == "scaled" else 1.0
+        gu = w13[e] if kind == "plain" else w13[2 * e * I:2 * (e + 1) * I]
+        d = (w2[e] if kind == "plain" else w2[:, e * I:(e + 1) * I]).double()
+        g, u = (x[t].double() @ gu.double().t()).split(I, 1)
+        expect = (torch.nn.functional.silu(s * g) * s * u) @ d.t()
+        # as in test_moe_experts, and no row far off
+        err = (y[place[t, j].long()].double() - expect).norm(dim=1)
+        assert (err <= 3 * 2 ** -8 * expect.norm(dim=1)).all(), e
+
+
 @pytest.mark.parametrize("T,E,k,H,I,base,El,tile,skew", [
     (1, 4, 2, 64, 64, 0, 4, 64, False), (7, 128, 8, 256, 192, 0, 128, 64, False),
     (33, 64, 8, 2048, 768, 16, 16, 64, False),  # another rank's pairs
