@@ -1462,7 +1462,8 @@ def moe_experts(x, w13, w2, weights, ids, expert_base: int = 0,
     if _moe_native(x, w13, w2, ids):
         x, way = _moe_cut(x, w13, w2, ids, experts)
         out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-        _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, *way)
+        _native().moe_experts(out, x, w13, w2, weights, ids, expert_base, *way,
+                              experts=experts or 0)
         return out
     return ref.moe_experts(x, w13, w2, weights, ids, expert_base)
 
@@ -1474,7 +1475,8 @@ def moe_experts_parts(x, w13, w2, weights, ids, expert_base: int = 0,
         return moe_experts(x, w13, w2, weights, ids, expert_base, experts)
     x, way = _moe_cut(x, w13, w2, ids, experts)
     return Mixed(*_native().moe_expert_rows(
-        x, w13, w2, weights, ids, expert_base, *(*way, 4, 4)[:4], None, False))
+        x, w13, w2, weights, ids, expert_base, *(*way, 4, 4)[:4], None, False,
+        experts or 0))
 
 
 # Rows whose choice of experts the plan makes (moe_gemm.hip), a wave a row: beyond,
@@ -1500,7 +1502,7 @@ def moe_routed_parts(x, gate, k: int, renorm: bool, w13, w2, expert_base: int = 
     x, way = _moe_cut(x, w13, w2, ids, E)
     return Mixed(*_native().moe_expert_rows(
         x, w13, w2, weights, ids, expert_base, *(*way, 4, 4)[:4],
-        _route_logits(x, gate), bool(renorm)))
+        _route_logits(x, gate), bool(renorm), E))
 
 
 def _moe_native(x, w13, w2, ids) -> bool:

@@ -124,7 +124,7 @@ void arks_moe_gemm(void* out, const void* a, const void* w, const void* perm,
                    const void* items, const void* n_items, void* claims, const void* scale,
                    int64_t a_stride, int64_t w_expert, int64_t w_stride, int n_out, int k_total,
                    int top_k, int max_items, int tile, int up,
-                   int once, hipStream_t stream);
+                   int once, int expert_base, hipStream_t stream);
 void arks_mfma_probe(void* d, const void* a, const void* b, hipStream_t stream);
 void arks_mfma_probe32(void* d, const void* a, const void* b, hipStream_t stream);
 void arks_tr16_probe(void* out, int stride_bytes, hipStream_t stream);
@@ -891,11 +891,13 @@ static std::array<int, 4> engine_rounds(int64_t H, int64_t I) {
 // 128 pairs in mid_gemm.hip (32: qt_up and qt_down, weight rows a wave / 16, may
 // be 2), else in moe_gemm.hip (16, 128 or, 256, its engine's up to 320). logits
 // [T, experts]: the plan finds ids and weights (only their sizes count then).
+// experts: the number on all ranks (at least El).
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
     torch::Tensor x, torch::Tensor w13, torch::Tensor w2, torch::Tensor weights,
     torch::Tensor ids, int64_t expert_base, int64_t tile, bool mid,
     int64_t qt_up, int64_t qt_down,
-    c10::optional<torch::Tensor> logits = c10::nullopt, bool renorm = false) {
+    c10::optional<torch::Tensor> logits = c10::nullopt, bool renorm = false,
+    int64_t experts = 0) {
   check_bf16_rowstrided(x, "x");
   check_bf16_contig(w13, "w13");
   check_bf16_contig(w2, "w2");
@@ -975,13 +977,14 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> moe_expert_rows(
                    (int)expert_base, (int)max_items, ft, (int)qt_down, 0, stream);
   } else {
     // (moe_gemm.hip: experts that mostly have one item)
-    const int once = P <= 160 * El ? 2 : 0;
+    const int once = P <= 160 * std::max(experts, El) ? 2 : 0;
     arks_moe_gemm(h.data_ptr(), x.data_ptr(), w13.data_ptr(), perm, items,
                   n_items, claims, nullptr, x.stride(0), 2 * I * H, H, (int)I, (int)H,
-                  (int)k, (int)max_items, (int)tile, 1, once, stream);
+                  (int)k, (int)max_items, (int)tile, 1, once, (int)expert_base,
+                  stream);
     arks_moe_gemm(y.data_ptr(), h.data_ptr(), w2.data_ptr(), perm, items,
                   n_items, claims, nullptr, I, H * I, I, (int)H, (int)I, (int)k,
-                  (int)max_items, (int)tile, 0, once, stream);
+                  (int)max_items, (int)tile, 0, once, (int)expert_base, stream);
   }
   return {y, w_pair, plan.narrow(0, 4 * max_items + P, P).view({T, k})};
 }
@@ -1043,10 +1046,10 @@ std::tuple<torch::Tensor, torch::Tensor> moe_wide_rows(
   arks_moe_gemm(h.data_ptr(), x.data_ptr(), w_gu.data_ptr(), perm, items,
                 n_items, claims, scaled ? w_pair.data_ptr() : nullptr,
                 x.stride(0), 2 * ff * W, W, (int)ff, (int)W, (int)k,
-                (int)max_items, 256, 2, once, stream);
+                (int)max_items, 256, 2, once, 0, stream);
   arks_moe_gemm(y.data_ptr(), h.data_ptr(), w_down.data_ptr(), perm, items,
                 n_items, claims, nullptr, ff, ff, down, (int)W, (int)ff, (int)k,
-                (int)max_items, 256, 0, once, stream);
+                (int)max_items, 256, 0, once, 0, stream);
   return {y, plan.narrow(0, 4 * max_items + P, P).view({T, k})};
 }
 
@@ -1054,12 +1057,13 @@ std::tuple<torch::Tensor, torch::Tensor> moe_wide_rows(
 void moe_experts(torch::Tensor out, torch::Tensor x, torch::Tensor w13,
                  torch::Tensor w2, torch::Tensor weights, torch::Tensor ids,
                  int64_t expert_base, int64_t tile, bool mid, int64_t qt_up,
-                 int64_t qt_down) {
+                 int64_t qt_down, int64_t experts) {
   check_bf16_contig(out, "out");
   TORCH_CHECK(x.dim() == 2 && out.size(0) == x.size(0) &&
               out.size(1) == x.size(1));
   const auto [y, w, rows] = moe_expert_rows(x, w13, w2, weights, ids,
-                                            expert_base, tile, mid, qt_up, qt_down);
+                                            expert_base, tile, mid, qt_up, qt_down,
+                                            c10::nullopt, false, experts);
   if (x.size(0) == 0) return;
   arks_moe_mix_rows(out.data_ptr(), y.data_ptr(), w.data_ptr(), rows.data_ptr(),
                     (int)x.size(0), (int)x.size(1), (int)weights.size(1),
@@ -1116,14 +1120,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mid_gemm", &mid_gemm);
   m.def("mid_pair", &mid_pair);
   m.def("stage_rows", &stage_rows);
-  m.def("moe_expert_rows", &moe_expert_rows);
+  m.def("moe_expert_rows", &moe_expert_rows, pybind11::arg("x"),
+        pybind11::arg("w13"), pybind11::arg("w2"), pybind11::arg("weights"),
+        pybind11::arg("ids"), pybind11::arg("expert_base"),
+        pybind11::arg("tile"), pybind11::arg("mid"), pybind11::arg("qt_up"),
+        pybind11::arg("qt_down"), pybind11::arg("logits"), pybind11::arg("renorm"),
+        pybind11::arg("experts") = 0);
   m.def("moe_wide_rows", &moe_wide_rows);
   m.def("fused_add_rmsnorm_mix", &fused_add_rmsnorm_mix);
   m.def("moe_experts", &moe_experts, pybind11::arg("out"), pybind11::arg("x"),
         pybind11::arg("w13"), pybind11::arg("w2"), pybind11::arg("weights"),
         pybind11::arg("ids"), pybind11::arg("expert_base"),
         pybind11::arg("tile"), pybind11::arg("mid"), pybind11::arg("qt_up") = 4,
-        pybind11::arg("qt_down") = 4);
+        pybind11::arg("qt_down") = 4, pybind11::arg("experts") = 0);
   m.def("mfma_probe", &mfma_probe);
   m.def("mfma_probe32", &mfma_probe32);
   m.def("tr16_probe", &tr16_probe);

@@ -506,7 +506,8 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
 // ONCE: for experts that have one item each, mostly (up to 160 pairs on the mean):
 // their weights pass the caches by, where the rows stay then, and (rotate) the tiles
 // of an expert begin at different steps, so that reads of columns a power of two
-// apart meet on more of the memory's channels. us with plan, as they are (past the
+// apart meet on more of the memory's channels; which step follows from the expert's
+// number among all ranks', as its order of sums must. us with plan, as they are (past the
 // caches; and rotated): 128 experts of 2048 x 768, 8 per row, 300 rows 247 (226;
 // 213), 1000 rows 276 (258; 251), 2048 rows 329 (319; 312), 4096 rows 409 (425;
 // 432); 16 experts of 4096 x 3584, 4 per row, 500 rows 303 (290; 284), 2000 rows 740
@@ -549,7 +550,7 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     int* __restrict__ claims, const float* __restrict__ scale,
     const int64_t a_stride, const int64_t w_expert, const int64_t w_stride,
     const int n_out, const int k_total, const int top_k, const int row_tiles,
-    const int rotate) {
+    const int rotate, const int expert_base) {
   using MoeTile = MoeTileOf<ONCE>;
   constexpr int FY = 5, COLS = UP ? 128 : 256;
   __shared__ __attribute__((aligned(1024))) char lds[MoeTile::LDS + 16];
@@ -571,7 +572,7 @@ __global__ __launch_bounds__(512, 2) void moe_engine_kernel(
     const int j = j0 + i, q = j / row_tiles, w4 = items[q].w;
     const int i0 = q - (w4 & 0xffff), r = j - i0 * row_tiles, n = w4 >> 16;
     const int4 it = items[i0 + r % n];
-    const int turn = rotate ? (it.x * row_tiles + r / n) % steps : 0;
+    const int turn = rotate ? ((expert_base + it.x) * row_tiles + r / n) % steps : 0;
     return Job{it.x, it.y, it.z, r / n * COLS, {0, steps, turn}};
   };
   // The rows of a that this wave loads, each in a lane of its own (so they are one
@@ -736,14 +737,14 @@ extern "C" void arks_moe_plan_topk(void* perm, void* rows, void* weights_out,
 // (tiles through LDS; n_out % 8 == k_total % 8 == 0) or 256 (the engine, whose items
 // have up to 320; n_out % 8 == k_total % 64 == 0, an expert's weights and (up) all
 // rows of a under 4 GiB; up: 1, or 2 for GLU, with scale [pairs] or null; once: 0,
-// 1, or 2 for rotated columns).
+// 1, or 2 for rotated columns, by an expert's number from expert_base on).
 extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
                               const void* perm, const void* items,
                               const void* n_items, void* claims,
                               const void* scale, int64_t a_stride, int64_t w_expert,
                               int64_t w_stride, int n_out, int k_total,
                               int top_k, int max_items, int tile, int up,
-                              int once, hipStream_t stream) {
+                              int once, int expert_base, hipStream_t stream) {
   const bool glu = up == 2;
 #define ARKS_STREAM(NF, WV, UP)                                               \
   hipLaunchKernelGGL((moe_stream_kernel<NF, WV, UP>),                         \
@@ -770,7 +771,7 @@ extern "C" void arks_moe_gemm(void* out, const void* a, const void* w,
                      (const int*)perm, (const int4*)items,                    \
                      (const int*)n_items, (int*)claims + (up ? 0 : 8),        \
                      (const float*)scale, a_stride, w_expert, w_stride, n_out, \
-                     k_total, top_k, row_tiles, (int)(once == 2))
+                     k_total, top_k, row_tiles, (int)(once == 2), expert_base)
 #define ARKS_ENGINE(UP, GLU, SCALED)                                          \
   do {                                                                        \
     if (once) ARKS_ENGINE_O(UP, GLU, SCALED, true);                           \

@@ -983,6 +983,32 @@ def test_moe_engine_cut(T, E, k, H, I, skew, cap, kind):
         assert (err <= 3 * 2 ** -8 * expect.norm(dim=1)).all(), e
 
 
+@pytest.mark.parametrize("T", [40, 300, 700, 1300])  # 10, 75, 175 and 325 pairs each
+def test_moe_engine_order_of_sums(T):
+    """A pair's row has the same bits whichever rank has its expert."""
+    assert_native()
+    torch.manual_seed(T)
+    E, k, H, I = 8, 2, 1024, 576
+    x = torch.randn(T, H, device=DEV).bfloat16()
+    w13 = (torch.randn(E, 2 * I, H, device=DEV) * H ** -0.5).bfloat16()
+    w2 = (torch.randn(E, H, I, device=DEV) * I ** -0.5).bfloat16()
+    ids = torch.rand(T, E, device=DEV).topk(k).indices.int()
+    w = torch.rand(T, k, device=DEV) + 0.5
+
+    def rows(base, n):
+        y, weights, place = ops._native().moe_expert_rows(
+            x, w13[base:base + n], w2[base:base + n], w, ids, base, 256, False, 4, 4,
+            None, False, E)
+        return y[place.long()], weights > 0
+
+    whole, mine = rows(0, E)
+    assert mine.all()
+    for base, n in ((0, 3), (3, 4), (7, 1)):
+        part, mine = rows(base, n)
+        assert torch.equal(mine, (ids >= base) & (ids < base + n))
+        assert torch.equal(part[mine], whole[mine]), base
+
+
 @pytest.mark.parametrize("T,E,k,H,I,base,El,tile,skew", [
     (1, 4, 2, 64, 64, 0, 4, 64, False), (7, 128, 8, 256, 192, 0, 128, 64, False),
     (33, 64, 8, 2048, 768, 16, 16, 64, False),  # another rank's pairs
