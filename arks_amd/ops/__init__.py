@@ -867,8 +867,8 @@ _WIDE_STEP = {(128, 256): 0.92, (192, 256): 1.16, (256, 128): 0.89,
 
 
 @functools.lru_cache(maxsize=4096)
-def _wide_cut(M: int, N: int, K: int, split: bool, summed: bool):
-    """(rows of a, rows of w, runs of K, workgroups) of a wide_gemm, w [N, K]:
+def _wide_fit(M: int, N: int, K: int, split: bool, summed: bool):
+    """(us, rows of a, rows of w, runs of K, workgroups) of a wide_gemm, w [N, K]:
     the tiles and runs that finish first by a fit of what 15 sizes took at 257 to
     8192 rows with every tile and cut (the chosen ones are 0.7 % from the best on
     average). A round over the CUs takes its steps and the end of a tile; the
@@ -890,7 +890,12 @@ def _wide_cut(M: int, N: int, K: int, split: bool, summed: bool):
                 us += splits * M * N * 1.08e-6 + (0.0 if summed else 4.0)
             if best is None or us < best[0]:
                 best = us, tm, tw, splits, jobs
-    return best[1:]
+    return best
+
+
+def _wide_cut(M: int, N: int, K: int, split: bool, summed: bool):
+    """_wide_fit without its time."""
+    return _wide_fit(M, N, K, split, summed)[1:]
 
 
 def _wide_takes(x, weight, bias=None) -> bool:
@@ -912,27 +917,32 @@ def _wide_takes(x, weight, bias=None) -> bool:
 
 def _wide(x, weight, bias=None, summed: bool = False):
     """(rows of a, rows of w, runs of K) if x weight^T takes wide_gemm, else
-    None: more than 256 rows of long weights. The library's kernels there turn
-    with the row count, and do not cut K as finely as a few hundred rows need. us,
-    here with a launch for the sums (library): 3584 x 18944, 300 rows 60 (101),
-    432 rows 75 (198), 700 rows 97 (165), 1309 rows 164 (256), 1691 rows 201
-    (228), 2314 rows 267 (485), 3344 rows 367 (328), 4666 rows 456 (876); 4096 x
-    14336, 300 rows 55 (76), 1549 rows 151 (329), 1972 rows 196 (188); 4096 x
-    8192, 300 rows 39 (47), 763 rows 60 (59), 1594 rows 101 (100), 4949 rows 225
-    (256); 1024 x 16384, 450 rows 31 (46). What the library does best are many
-    whole tiles of rows, and weights of up to 80 million elements where tiles of 256
-    x 256 make one round over the CUs, at least 5/8 full: 3584 x 18944, 8192 rows 806
-    (740), 3102 rows 369 (355); 4096 x 14336, 2837 rows 279 (249), 3394 rows 299
-    (285). With K up to 4096 a run has few steps: 4096 x 4096, 491 rows 32 (30),
+    None: more than 256 rows of long weights, where that is expected to finish in
+    front of the library. At its best a library kernel of 256 x 256 tiles does a step
+    of 64 columns in 1.06 us in whole rounds over the CUs, here it is 1.33: so the
+    library keeps what fills its rounds, and sums that have a launch of their own
+    (not summed) count 2e-6 us each beyond the fit. Of a few hundred rows it often
+    has slower kernels, which turn with the row count. us in front of a norm
+    (library), 3584 x 18944: 300 rows 64 (108), 450 rows 77 (207), 700 rows 101 (176),
+    1309 rows 175 (267), 2314 rows 275 (499), 4666 rows 479 (908), left to it 3344 rows
+    412 (357), 8192 rows 873 (807); 4096 x 14336: 300 rows 57 (84), 1536 rows 174
+    (188), left 3344 rows 336 (314); 4096 x 8192: 300 rows 42 (53), 5000 rows 268 (295),
+    left 3344 rows 214 (194). Over 18 weights of 13 to 235 million
+    elements (N 1024 to 12288, K 8192 to 28672) at 37 numbers of rows 0.825 of the
+    library's time, the better of the two 0.804, 11 sizes more than 3 % slower, the
+    worst 1.12 (3072 x 24576, 3344 rows); with a launch for the sums 0.840 (0.816), 25
+    and 1.12. With K up to 4096 a run has few steps: 4096 x 4096, 491 rows 32 (30),
     1159 rows 51 (44)."""
     if not _wide_takes(x, weight, bias):
         return None
     M, (N, K) = x.shape[0], weight.shape
-    if K < 8192 or N < 1024 or (M >= 4096 and M % 256 == 0):
+    if K < 8192 or N < 1024:
         return None
-    if N * K <= 80_000_000 and 160 <= -(-M // 256) * -(-N // 256) <= 256:
-        return None
-    return _wide_cut(M, N, K, True, summed)[:3]
+    us, *cut, _ = _wide_fit(M, N, K, True, summed)
+    if cut[2] > 1 and not summed:
+        us += 2e-6 * cut[2] * M * N
+    rounds = -(-(-(-M // 256) * -(-N // 256)) // 256)
+    return cut if us < 3.0 + rounds * (5.0 + 1.06 * K / 64) else None
 
 
 def _wide_silu(x, weight):

@@ -1927,10 +1927,9 @@ def test_wide_rule():
     assert not ops._wide(x[:, :4096], w[:, :4096].contiguous())
     assert not ops._wide(x.float(), w) and not ops._wide(x, w.clone().requires_grad_())
     assert not ops._wide(x, w, torch.ones(1, dtype=torch.bfloat16, device=DEV))
-    many = x[:1].expand(4097, -1)
-    assert ops._wide(many, w) and not ops._wide(many[:4096], w)
-    more = x[:1].expand(5000, -1)  # 160 tiles of 256 x 256
-    assert ops._wide(more[:4800], w) and not ops._wide(more, w)
+    many = x[:1].expand(5121, -1)  # 20 x 8 tiles of 256 x 256 fill a round well enough
+    assert ops._wide(many[:5120], w, summed=True) and not ops._wide(many, w, summed=True)
+    assert ops._wide(many[:3694], w) and not ops._wide(many[:3695], w)
     gated = torch.empty(16384, 64, dtype=torch.bfloat16, device=DEV)
     assert ops._wide_silu(x[:300, :64], gated)
     assert ops._wide_silu(x[:300, :64], gated[:4096]) is None  # few tiles

@@ -329,6 +329,33 @@ def test_wide_cut():
                for M in range(257, 2049, 64))
 
 
+@pytest.mark.parametrize("N,K,takes,leaves", [
+    (3584, 18944, (300, 1309, 2314, 4666), (3344, 4352, 8192)),
+    (4096, 14336, (300, 1536, 4352), (2837, 3344, 6144, 8192)),
+    (6144, 16384, (600, 1309, 2837, 6000), (1800, 2048, 3344, 4096)),
+    (8192, 22016, (700, 2314, 4666), (1536, 2048, 3344, 8192)),
+    (5120, 27648, (400, 1691, 3344, 7000), (2837, 4666)),
+    (2048, 8192, (700, 1280), (6000, 8192)),
+    (3584, 8128, (), (300, 2314)), (1008, 16384, (), (300, 2314)),
+])
+def test_wide_leaves_full_rounds_to_the_library(N, K, takes, leaves, monkeypatch):
+    """Sizes at which the library's tiles of 256 x 256 fill their rounds over the CUs
+    stay with it (measured 3 to 24 % behind here), whatever the row count is divisible
+    by; those of part rounds are taken (4 % to three times as fast)."""
+    from types import SimpleNamespace as S
+
+    from arks_amd import ops
+
+    monkeypatch.setattr(ops, "_wide_takes", lambda *a: True)
+    for rows in (takes, leaves):
+        for M in rows:
+            for summed in (False, True):
+                cut = ops._wide(S(shape=(M, K)), S(shape=(N, K)), None, summed)
+                assert bool(cut) == (rows is takes), (M, summed)
+                if cut:
+                    assert tuple(cut) == ops._wide_cut(M, N, K, True, summed)[:3]
+
+
 def test_tile_fill_is_what_the_schedule_takes():
     """The share against the schedule walked out: every workgroup's tiles of its
     XCD in turn, 1 for a whole one and 0.55 for those of the last 128 rows."""
