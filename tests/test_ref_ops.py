@@ -356,6 +356,20 @@ def test_wide_leaves_full_rounds_to_the_library(N, K, takes, leaves, monkeypatch
                     assert tuple(cut) == ops._wide_cut(M, N, K, True, summed)[:3]
 
 
+def test_wide_leaves_full_rounds_to_tiles_of_256(monkeypatch):
+    """Gate and up products whose tiles of 256 rows fill their rounds stay in them."""
+    from types import SimpleNamespace as S
+
+    from arks_amd import ops
+
+    monkeypatch.setattr(ops, "_wide_takes", lambda *a: True)
+    wide = lambda M, N, K: ops._wide_silu(S(shape=(M, K)), S(shape=(N, K)))
+    for M, N, K in ((4096, 28672, 4096), (8192, 28672, 4096), (8192, 55296, 5120),
+                    (8192, 36864, 6144)):
+        assert wide(M, N, K) is None and wide(M - 512 + 20, N, K)
+    assert wide(512, 32768, 4096) and wide(8192, 37888, 3584)
+
+
 def test_tile_fill_is_what_the_schedule_takes():
     """The share against the schedule walked out: every workgroup's tiles of its
     XCD in turn, 1 for a whole one and 0.55 for those of the last 128 rows."""
