@@ -2187,9 +2187,9 @@ def route_rows_takes(h, router, groups: int = 1) -> bool:
     return (_USE_SKINNY and h.is_cuda and 1 <= T <= 64 and groups == 1
             and h.dtype == router.dtype == torch.bfloat16
             and 8 <= W and W % 8 == 0 and router.shape[0] <= 64
-            and h.stride(-1) == 1 and h.stride(0) % 8 == 0
+            and _plain(h, router) and h.stride(-1) == 1 and h.stride(0) % 8 == 0
             and h.data_ptr() % 16 == 0 and router.is_contiguous()
-            and router.data_ptr() % 16 == 0 and _plain(h, router))
+            and router.data_ptr() % 16 == 0 and seq_native_available())
 
 
 def moe_route_rows(h, router, top, score="softmax", renorm=True, matrix=False,

@@ -656,6 +656,24 @@ def test_route_rows(T, E, top, W, gate, score):
 
 
 @pytest.mark.gpu
+def test_route_rows_steps_aside(monkeypatch):
+    """Rows under a transform, with gradients or tangents, or without the kernels, are
+    left to the products that follow them."""
+    h = torch.randn(3, 5, 256, device="cuda").bfloat16()
+    router = torch.randn(16, 256, device="cuda").bfloat16()
+    takes = []
+    torch.vmap(lambda x: (takes.append(ops.route_rows_takes(x, router)), x)[1])(h)
+    torch.vmap(lambda r: (takes.append(ops.route_rows_takes(h[0], r)), r)[1])(
+        router.expand(3, -1, -1))
+    takes.append(ops.route_rows_takes(h[0], router.clone().requires_grad_()))
+    with torch.autograd.forward_ad.dual_level():
+        takes.append(ops.route_rows_takes(h[0], router))
+    assert takes == [False] * 4 and ops.route_rows_takes(h[0], router)
+    monkeypatch.setattr(ops, "seq_native_available", lambda: False)
+    assert not ops.route_rows_takes(h[0], router)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,top,ff,W,most", [
     (4, 2, 512, 1024, 48),     # weights of linear_fixed
     (16, 4, 1024, 2560, 16)])  # routed_experts takes them
