@@ -622,7 +622,9 @@ class HybridForCausalLM(nn.Module):
         if self.arr.norm_place in ("sandwich", "pre"):
             return self._forward_sandwich(batch, caches)
         x = self.embed[batch.input_ids].float()
-        fuse = self.arr.token_shift and ops.norm_shift_takes(x, batch, self.dtype)
+        # (a tap may change x in front of the next layer's shift)
+        fuse = (self.arr.token_shift and self.residual_tap is None
+                and ops.norm_shift_takes(x, batch, self.dtype))
         shifted = None
         for i, layer in enumerate(self.layers):
             if fuse and all(passable(b, HybridBlock) for b in self.layers[i:i + 2]):

@@ -219,6 +219,40 @@ def test_other_sizes(tmp_path, device, dtype, which):
     assert rel_err(got["b"], orc.run(tb)) < TOL[dtype]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tap", [False, True])
+def test_token_shift_of_the_layer_behind(tmp_path, monkeypatch, tap):
+    """Steps of one row a sequence have the next layer's token shift from a layer's
+    last norm: the same bits with a hook on a layer, which is then called as it is, and
+    with a tap that changes the rows between two layers."""
+    from arks_amd import ops
+
+    cfg = model_cfg([attn(mlp=FF), lightning(), mamba(mlp=FF), attn(), mamba()])
+    write_checkpoint(tmp_path / "m", cfg, seed=5)
+    ta, tb = toks(12, seed=3), toks(9, seed=4)
+    steps = ([[("a", ta[:6], False)], [("a", ta[6:7], False), ("b", tb[:4], False)]]
+             + [[("a", ta[k:k + 1], k == 11), ("b", tb[k - 3:k - 2], k == 11)]
+                for k in range(7, 12)])
+    fused, calls = ops.gated_norm_shift, []
+    monkeypatch.setattr(ops, "gated_norm_shift",
+                        lambda *a: (calls.append(1), fused(*a))[1])
+    got = {}
+    for name, hooked in (("none", ()), ("one", (2,)), ("all", range(5))):
+        eng = make_engine(tmp_path / "m", "cuda", "bfloat16", enforce_eager=True)
+        model = eng.runner.model
+        for i in hooked:
+            model.layers[i].register_forward_hook(lambda *a: None)
+        if tap:
+            model.residual_tap = lambda i, x: x.mul_(0.5) if i in (1, 3) else None
+        calls.clear()
+        out = replay(eng, tmp_path, steps)
+        got[name] = np.concatenate([out["a"], out["b"]])
+        # 4 of 5 layers have one behind them; a hook takes two pairs away
+        assert len(calls) == (0 if tap else 5 * {"none": 4, "one": 2, "all": 0}[name])
+    assert np.array_equal(got["none"], got["all"])
+    assert np.array_equal(got["one"], got["all"])
+
+
 @pytest.mark.parametrize("device,dtype", CASES)
 def test_greedy_generation_through_the_scheduler(tmp_path, device, dtype):
     from arks_amd.engine import SamplingParams
