@@ -1826,6 +1826,48 @@ def test_mid_pair(M, N, K, K2, qt, splits, splits2):
             at += 1
 
 
+@pytest.mark.parametrize("M", [1, 33, 64])
+@pytest.mark.parametrize("N,K,K2", [(1024, 1024, 2048), (520, 4096, 1024), (8, 1088, 1024)])
+def test_linear_pair(M, N, K, K2):
+    """Two products of unlike K in one launch vs fp64: which sums are whose, in the
+    runs that _pair_cut chooses; rows that start off 16 bytes are copied."""
+    assert_native()
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K + 8, dtype=torch.bfloat16, device=DEV)[:, 3:K + 3]
+    x2 = torch.randn(M, 2 * K2, dtype=torch.bfloat16, device=DEV)[:, :K2]
+    w, w2 = ((torch.randn(N, k, device=DEV) * k ** -0.5).bfloat16() for k in (K, K2))
+    pair = ops.linear_pair(x, w, x2, w2)
+    _, n, n2 = ops._pair_cut(M, N, K, K2)
+    assert [p.sums.shape[0] for p in pair] == [n, n2]
+    for p, a, b in zip(pair, (x, x2), (w, w2)):
+        ad, bd = a.double(), b.double()
+        slack = a.shape[1] * 2 ** -24 * (ad.abs() @ bd.abs().t())  # as in test_mid_gemm
+        assert ((p.sums.double().sum(0) - ad @ bd.t()).abs() <= slack).all()
+
+
+def test_linear_pair_takes():
+    """Up to 64 rows of two products of as many columns, of whole steps and K of 1024
+    and more; others are left to linear_parts."""
+    assert_native()
+    x = torch.randn(65, 2048, dtype=torch.bfloat16, device=DEV)
+    w, w2 = (torch.randn(n, 2048, dtype=torch.bfloat16, device=DEV) for n in (512, 504))
+    takes = lambda *a: ops.linear_pair(*a) is not None
+    assert takes(x[:64], w, x[:64], w)
+    assert not takes(x, w, x, w)                   # 65 rows
+    assert not takes(x[:0], w, x[:0], w)
+    assert not takes(x[:2], w, x[:3], w)           # other rows
+    assert not takes(x[:2], w, x[:2], w2)          # other columns
+    for k in (960, 1056):                          # a short K, no whole steps
+        assert not takes(x[:2], w, x[:2, :k], w[:, :k].contiguous())
+    assert not takes(x[:2], w, x[:2], w.t().contiguous().t())
+    assert not takes(x[:2], w, x[:2], w.clone().requires_grad_())
+    assert not takes(x[:2].float(), w.float(), x[:2], w)
+    assert not takes(x[0], w, x[0], w)
+    big = torch.empty(ops._PAIR_ELEMS // 4096 + 8 & ~7, 2048, dtype=torch.bfloat16,
+                      device=DEV)
+    assert not takes(x[:1], big, x[:1], big)
+
+
 @pytest.mark.parametrize("T,W,sy,sg", [
     (1, 8, 1, 0), (3, 4096, 4, 2), (5, 4104, 0, 8), (2, 8192, 3, 9), (70, 136, 8, 1),
 ])

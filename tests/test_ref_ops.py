@@ -370,6 +370,24 @@ def test_wide_leaves_full_rounds_to_tiles_of_256(monkeypatch):
     assert wide(512, 32768, 4096) and wide(8192, 37888, 3584)
 
 
+def test_pair_cut():
+    """Tiles that mid_gemm has, and 1 to 8 runs of a step or more of each product,
+    whichever comes first."""
+    import random
+
+    from arks_amd import ops
+
+    rng = random.Random(3)
+    for _ in range(300):
+        M, N = rng.randint(1, 64), 8 * int(2 ** rng.uniform(0, 11))
+        K, K2 = (64 * int(16 * 2 ** rng.uniform(0, 5)) for _ in range(2))
+        qt, *runs = ops._pair_cut(M, N, K, K2)
+        assert qt in (2, 4, 5)
+        for n, k in zip(runs, (K, K2)):
+            assert 1 <= n <= min(8, k // 64)
+        assert ops._pair_cut(M, N, K2, K) == (qt, *runs[::-1])
+
+
 def test_tile_fill_is_what_the_schedule_takes():
     """The share against the schedule walked out: every workgroup's tiles of its
     XCD in turn, 1 for a whole one and 0.55 for those of the last 128 rows."""
