@@ -262,8 +262,9 @@ class RoutedMoE(nn.Module):
                 _, _, scale = ops.moe_route_grouped(
                     linear_f32(h, self.router), k, self.groups, self.keep,
                     matrix=True, group_top=self.group_top, **route)
-            # (weights that linear_fixed takes keep the order of sums that they
-            # have at 17 rows and more)
+            # (weights of ops._fixed_run keep the order of sums that they have at 17
+            # rows and more; larger ones have one up to 16 rows and another, that of
+            # linear_fixed's cut, from 17 on)
             if (not sff and ops.routed_takes(h, self.w_gu, self.w_down, E, ff)
                     and not ops.sums_fixed(T, self.w_gu, self.w_down)):
                 return ops.routed_experts(h, self.w_gu, self.w_down, scale,

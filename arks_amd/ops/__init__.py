@@ -1101,8 +1101,9 @@ def fix_sums(weights) -> None:
 
 
 def sums_fixed(M: int, *weights) -> bool:
-    """Whether linear_fixed has an order of its own for any of these weights at
-    M rows (up to 64)."""
+    """Whether linear_fixed adds any of these weights up in runs of _fixed_run at M
+    rows (up to 64). Larger weights, whose order there is that of _fixed_cut, do not
+    count: where routed_experts takes them, up to 16 rows, theirs is its own."""
     return any(_fixed_run(M, *w.shape) for w in weights)
 
 
