@@ -1067,7 +1067,8 @@ def linear_pair(x, weight, x2, weight2):
 def linear_bf16(x, weight, bias=None):
     """Linear dispatch: the streamed product for few rows of small weights, the
     tiles of mid_gemm.hip for up to 256 rows, K split over workgroups for sizes
-    that those do not take, hipBLASLt (F.linear) otherwise."""
+    that those do not take, the tiles of wide_gemm.hip for more rows of long weights
+    (_wide), hipBLASLt (F.linear) otherwise."""
     cut = _mid(x, weight, bias)
     if cut is not None:
         return parts_sum(_mid_gemm(x, weight, bias, cut))
@@ -1402,11 +1403,11 @@ def moe_tile(rows: int, top_k: int, experts: int, whole: bool = False) -> int:
 
 def _moe_whole(x, H: int, I: int, pairs: int) -> bool:
     """Whether experts can run in items of 64 and more pairs that load rows
-    straight into LDS (mid_gemm.hip, tile_engine.h): whole steps of 64 columns,
+    straight into LDS (mid_gemm.hip, wide_engine.h): whole steps of 64 columns,
     and what their 32-bit row offsets reach. Tiles of 128 take the rest, and
-    were never the faster ones: 128 experts of 2048 x 768, 8 per row, us, 256
-    (128): 200 rows 242 (265), 5012 rows 545 (742); 8 of 4096 x 14336, 2 per
-    row: 200 rows 565 (611), 8192 rows 4527 (9434)."""
+    were never the faster ones: 128 experts of 2048 x 768, 8 per row, us, engine
+    (128): 5012 rows 452 (742); 8 of 4096 x 14336, 2 per row, 8192 rows 4550
+    (9434)."""
     return (_USE_SKINNY and (H | I) % 64 == 0
             and x.shape[0] * x.stride(0) < 1 << 31
             and 2 * I * H < 1 << 31 and pairs < (1 << 23) - 255)
@@ -1415,8 +1416,8 @@ def _moe_whole(x, H: int, I: int, pairs: int) -> bool:
 def _moe_way(rows: int, top_k: int, El: int, experts: int, H: int, I: int,
              whole: bool):
     """(pairs of an item, whether in mid_gemm.hip) for El experts here of
-    `experts` in all: moe_tile's, and 256 (tile_engine.h) in place of 128 where
-    whole. Experts whose columns leave most CUs without a tile keep the kernels
+    `experts` in all: moe_tile's, and 256 (the engine, wide_engine.h, whose items
+    have up to 320) in place of 128 where whole. Experts whose columns leave most CUs without a tile keep the kernels
     with more of them, us, 16 (64 of mid_gemm), 128 (256): 4 experts of 512 x
     256, 2 per row, 16 rows 13 (21), 64 rows 24 (21) in tiles of 128, 1000 rows
     29 (36), 5000 rows 47 (45); 16 experts of 4096 x 1024, 4 per row, 256 tiles
@@ -1430,6 +1431,7 @@ def _moe_way(rows: int, top_k: int, El: int, experts: int, H: int, I: int,
             if (H | I) % 32 == 0 else 128)
     if tile == 64:
         return (128 if pairs > 32 * experts else 64), True
+    # (the engine's items are of 192 to 320 pairs: about this many)
     if (tile == 128 and whole
             and (El + pairs // 256) * -(-I // 128) >= 64):
         tile = 256

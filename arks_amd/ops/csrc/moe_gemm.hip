@@ -11,12 +11,13 @@
 //              LDS and no barrier before the final sum over the waves. 7 rows,
 //              8 of 128 experts each (2048 x 768): 90 us for 46 experts' 434 MB
 //              (4.8 TB/s); every expert as a batched product took 210 us.
-//   moe_engine more than 64 pairs per expert on the mean: bound by the matrix
-//              cores, and by the weights' one read while experts have few. Up
-//              to 320 pairs x 256 weight rows per workgroup (wide_engine.h).
-//              128 experts of 2048 x 768, 8 per row, with plan: 5012 rows 452
-//              us, 520 rows 225 us for 1.2 GB of weights; 8 experts of 4096 x
-//              14336, 2 per row, 8192 rows 4.6 ms.
+//   moe_engine 32 and more pairs per expert on the mean (fewer tiles than CUs:
+//              more than 64, ops._moe_engine): bound by the matrix cores, and by
+//              the weights' one read while experts have few. Up to 320, 256 or
+//              192 pairs (moe_cut) x 256 weight rows per workgroup
+//              (wide_engine.h). 128 experts of 2048 x 768, 8 per row, with
+//              plan: 5012 rows 452 us, 520 rows 218 us for 1.2 GB of weights; 8
+//              experts of 4096 x 14336, 2 per row, 8192 rows 4.55 ms.
 //   moe_tile   the same for sizes that are no multiple of 64, or leave the
 //              engine without work for the chip: 128 pairs x 128 weight rows, 64
 //              of K per step through double-buffered LDS and registers, 560
@@ -507,18 +508,17 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(
 // their weights pass the caches by, where the rows stay then, and (rotate) the tiles
 // of an expert begin at different steps, so that reads of columns a power of two
 // apart meet on more of the memory's channels; which step follows from the expert's
-// number among all ranks', as its order of sums must. us with plan, as they are (past the
-// caches; and rotated): 128 experts of 2048 x 768, 8 per row, 300 rows 247 (226;
-// 213), 1000 rows 276 (258; 251), 2048 rows 329 (319; 312), 4096 rows 409 (425;
-// 432); 16 experts of 4096 x 3584, 4 per row, 500 rows 303 (290; 284), 2000 rows 740
-// (763; 771). In tiles of 256 and 128 pairs (tile_engine.h) before: 251, 276, 331,
-// 412; 325, 720.
+// number among all ranks', as its order of sums must. us with plan, items of up to 320,
+// as they are (past the caches; and rotated): 128 experts of 2048 x 768, 8 per row, 1000
+// rows 268 (251; 239), 2048 rows 309 (295; 298), 4096 rows 449 (456; 454); 16 experts of
+// 4096 x 3584, 4 per row, 500 rows 319 (306; 299), 2000 rows 690 (706; 716). The line
+// could lie a little higher: 200 pairs, 128 experts 346 (326; 310).
 // Each XCD takes a contiguous stretch of (expert, row tile, item), so that an
 // expert's items meet the same weights in its L2; its workgroups claim tiles one by
-// one, as they take different times (dealt out in turn, 5012 rows: 591 us, claimed
-// 545). The claim is made a tile ahead, so that neither it nor the pairs' rows are
-// waited for. Its place in LDS belongs to the tiles' array: a second one made the
-// compiler drain the loads before every read of the first.
+// one, as they take different times (5012 rows in tile_engine.h's tiles, dealt out in
+// turn 591 us, claimed 545). The claim is made a tile ahead, so that neither it nor the
+// pairs' rows are waited for. Its place in LDS belongs to the tiles' array: a second one
+// made the compiler drain the loads before every read of the first.
 // GLU: gate and up are rounded to bf16 before they meet, as rows of a product in
 // memory would be. SCALED: scale [pairs] is a factor of both; it is loaded in front
 // of the next tile's first loads, so as not to be waited for behind them, and named

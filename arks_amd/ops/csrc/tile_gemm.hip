@@ -1,8 +1,10 @@
 // out[M, N] = silu(a w_gate^T) * (a w_up^T) for many rows, w [2N, K] the gate
-// rows, then the up rows, where these lie beyond the 32-bit offsets of
-// wide_gemm.hip (from 2^31 gate elements on; it is faster below): the product of tile_engine.h with a tile's two
-// halves of w as 128 gate rows and their up rows, so that the activation is
-// taken on the fp32 sums and neither product travels through memory. 18944 x
+// rows, then the up rows: the product of tile_engine.h with a tile's two halves of w
+// as 128 gate rows and their up rows, so that the activation is taken on the fp32
+// sums and neither product travels through memory. It has what fills 0.98 of its
+// rounds (28672 x 4096, 8192 rows 1303 us, wide_gemm.hip 1381), weights that stay out
+// of wide_gemm.hip (ops.plain_prompts) and those beyond its 32-bit offsets (from 2^31
+// gate elements on). 18944 x
 // 3584: 8192 rows 1511 us (1473 TFLOP/s; a library product and the activation
 // behind it 1633), 3150 rows 612 us (1398 TFLOP/s; 798), 2048 rows 397 us
 // (420). One workgroup per CU goes from tile to tile, the next one's first
